@@ -29,6 +29,8 @@ SYMBOLS = (
     "gd_expand_rgb24",
     "gd_pack_actors",
     "gd_pack_weapon",
+    "gd_ray_tables",
+    "gd_sprite_depth",
 )
 
 _LIBRARY = None
@@ -84,6 +86,10 @@ def library() -> C.CDLL:
     lib.gd_pack_actors.argtypes = [C.POINTER(_abi.ActorDesc), C.c_void_p]
     lib.gd_pack_weapon.restype = C.c_int
     lib.gd_pack_weapon.argtypes = [C.POINTER(_abi.WeaponDesc), C.c_void_p]
+    lib.gd_ray_tables.restype = C.c_int
+    lib.gd_ray_tables.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]
+    lib.gd_sprite_depth.restype = C.c_int
+    lib.gd_sprite_depth.argtypes = [C.c_void_p] * 5 + [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p]
     _LIBRARY = lib
     return lib
 

@@ -12,6 +12,9 @@ the lane tensors live on:
 * ``sprite depth       = clamp_min(sqrt(dx²+dy²),1) * cos(wrap(atan2(dy,dx) - angle))``
   (``engine.py:14684-14688``)
 * retained view angle ``bam.float() * (2π / 2³²)``      (``engine.py:10651``)
+
+Tensors on a ROCm device take one kernel of the library for the ray tables and one for the sprite depths, which
+give the Torch expressions' bits (``gd_ray_tables``, ``gd_sprite_depth``); everything else takes the expressions.
 """
 
 from __future__ import annotations
@@ -33,7 +36,23 @@ def cosine_correction(device) -> torch.Tensor:
     return torch.cos(native_ray_offsets(device))
 
 
+def _on_device(*tensors: torch.Tensor) -> bool:
+    """Are these contiguous float32 tensors of one ROCm device, as the library's kernels read them?"""
+
+    device = tensors[0].device
+    return device.type == "cuda" and all(t.dtype is torch.float32 and t.device == device and t.is_contiguous() for t in tensors)
+
+
 def ray_tables(angle: torch.Tensor, offsets: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    if _on_device(angle, offsets) and angle.dim() == 1 and offsets.shape == (SCREEN_WIDTH,):
+        from . import _lib  # noqa: PLC0415
+
+        tables = torch.empty((2, angle.shape[0], SCREEN_WIDTH), dtype=torch.float32, device=angle.device)
+        ray_cos, ray_sin = tables[0], tables[1]
+        with torch.cuda.device(angle.device):
+            _lib.check(_lib.library().gd_ray_tables(angle.data_ptr(), offsets.data_ptr(), angle.shape[0], ray_cos.data_ptr(), ray_sin.data_ptr(),
+                                                    torch.cuda.current_stream(angle.device).cuda_stream))
+        return ray_cos, ray_sin
     ray_angles = angle[:, None] + offsets[None, :]
     return torch.cos(ray_angles).contiguous(), torch.sin(ray_angles).contiguous()
 
@@ -43,6 +62,14 @@ def angle_from_bam(angle_bam: torch.Tensor) -> torch.Tensor:
 
 
 def sprite_depth(x, y, angle, sprite_x, sprite_y) -> torch.Tensor:
+    if _on_device(x, y, angle, sprite_x, sprite_y) and x.shape == y.shape == angle.shape == sprite_x.shape[:1] and sprite_x.shape == sprite_y.shape and sprite_x.dim() == 2:
+        from . import _lib  # noqa: PLC0415
+
+        depth = torch.empty_like(sprite_x)
+        with torch.cuda.device(x.device):
+            _lib.check(_lib.library().gd_sprite_depth(x.data_ptr(), y.data_ptr(), angle.data_ptr(), sprite_x.data_ptr(), sprite_y.data_ptr(), sprite_x.shape[0],
+                                                      sprite_x.shape[1], depth.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream))
+        return depth
     dx = sprite_x - x[:, None]
     dy = sprite_y - y[:, None]
     distance = torch.sqrt(dx * dx + dy * dy).clamp_min(1)

@@ -495,6 +495,18 @@ typedef struct gd_weapon_desc {
 int gd_pack_weapon(const gd_weapon_desc *weapon, void *stream);
 
 /*
+ * The float32 inputs of gd_lanes_desc that the reference evaluates with Torch, in one kernel each; bit for bit what the Torch
+ * expressions give on this device (each operation is rounded on its own, cos / sin / atan2 / fmod are the device library's).
+ *   gd_ray_tables:    ray_cos / ray_sin [N,320] = cos / sin(angle[n] + ray_offsets[x])                 (engine.py:10966-10974)
+ *   gd_sprite_depth:  depth [N,A] = max(|d|, 1) * cos(remainder(atan2(dy, dx) - angle + pi, 2 pi) - pi), d = sprite - camera
+ *                     (engine.py:14684-14688)
+ * All pointers are device pointers to contiguous arrays.  Returns GD_E_ARG for a null pointer or a negative count.
+ */
+int gd_ray_tables(const float *angle, const float *ray_offsets, int32_t lane_count, float *ray_cos, float *ray_sin, void *stream);
+int gd_sprite_depth(const float *x, const float *y, const float *angle, const float *sprite_x, const float *sprite_y,
+                    int32_t lane_count, int32_t sprite_slots, float *depth, void *stream);
+
+/*
  * Time `launches` back-to-back gd_render launches with HIP events on `stream`
  * and return the average milliseconds per launch of each kernel stage in
  * ms[0..stage_count).  Measurement helper for the benchmark; replaces nothing.
