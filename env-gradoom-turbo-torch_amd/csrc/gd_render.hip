@@ -12,10 +12,10 @@
 //   wall_raster     1 wave / strip            the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
 //   plane_shade     1 thread / 12 pixels      flat texel + light for every pixel a plane of the wall pass shows,
 //                                             the wall tiers' palette indices
-//   flat_list       128 threads / lane        per-pixel plane rays (fine point raster) for the listed gap pixels
-//   flat_span_select, flat_tail, flat_span_finish
+//   flat_gap        4 waves / gap column      per-pixel plane rays (fine point raster) for the gap pixels, vertical repair
+//   flat_rows, flat_span_select, flat_tail, flat_span_finish
 //                                             visplane repair of the rows where a gap pixel stayed unresolved
-//   flat_shade      128 threads / lane        the gap pixels' flats
+//   flat_shade      1 wave / gap column       the gap pixels' flats
 //   decal           320 threads / lane        bullet chips on the wall tiers they hit (frames that carry decals
 //                                             also keep a per-pixel scene depth: wall_raster<true>, plane_shade<true>)
 //   sprite_columns  320 threads / lane        billboards far -> near, opaque / additive / translucent
@@ -160,6 +160,7 @@ struct DeviceMap {  // device copy of gd_map_desc (device pointers) + fixed tabl
     // (x0, y0, x1, y1) per sector outside which no point tests inside that sector.
     const int *level_box_ofs;
     const float4 *level_boxes;
+    const float4 *level_box;             // [levels] one box around all sectors of the level: no probe point outside it lands in one
     // The coarse grid repacked for the crossing test of flat selection: per cell its item range, per
     // item one 16-byte record, per item edge a copy of the linedef's endpoints, so that a test is
     // three dependent loads (range, record, edges) instead of six.
@@ -192,22 +193,19 @@ struct Scratch {    // per-chunk working memory, sized at create
     int spill_slots;       // pool slots of this chunk (a multiple of 320)
     unsigned short *flat_sector;// [L,208,320]
     unsigned char *flat_flags;  // [L,208,320] bit0 unresolved
-    int *flat_list;        // [L,FLAT_LIST_MAX] view pixels no wall tier, plane or masked texture covers: they show the
-                           // flat pass's picture.  Listed by wall_raster_kernel, column by column.
-    int *flat_list_count;  // [L] how many there are (more than FLAT_LIST_MAX: the lane is handled pixel by pixel)
+    int2 *gap_columns;     // [L*320] the screen columns that hold view pixels no wall tier, plane or masked texture covers (they
+                           // show the flat pass's picture), of every lane, as one work list: lane << 9 | column, and the rows
+                           // they lie in, first | one past the last << 8.  Listed by wall_raster_kernel.
+    int *gap_column_count; // [1] its length (cleared by lane_setup_kernel)
     int *flat_tail;        // [L,2,320] per screen half and column: the sector of the first resolved pixel below the
                            // half's noted rows, -1 if the column was not looking for one or found none
     int *flat_span;        // [L,4] first / last row of the ceiling half, then of the floor half, that holds a shown
                            // pixel the flat pass could not resolve and whose repair reads its row (208, -1 = none):
                            // the rows the row repairs work on
+    int *flat_spans;       // [L*2] the (lane << 1 | half) with such rows, as one work list
+    int *flat_span_count;  // [1] its length (cleared by lane_setup_kernel)
     int *flat_rows;        // [L*208] the noted rows of every lane as one work list, entry = lane << 8 | row
     int *flat_row_count;   // [1] its length (cleared by lane_setup_kernel, filled by flat_rows_kernel)
-    int *gap_columns;      // [L*2*320] the screen columns (of any lane, either half) that hold a shown pixel the flat pass
-                           // could not resolve, as one work list: lane << 18 | half << 17 | topmost such row << 9 | column
-    int *gap_column_count; // [1] its length (cleared by lane_setup_kernel, filled by flat_gap_column_kernel)
-    int *flat_col_top;     // [L,2,320] per screen half and column: the topmost shown pixel the flat pass could not
-                           // resolve (any value >= 208: none).  lane_tables_kernel sets "none", flat_gap_column_kernel
-                           // lowers it while it selects the gap pixels.
     int pass_slots;        // passes a column can record in this chunk
     PassRec *pass_rec;     // [L,pass_slots,320] the drawsegs of each column's passes, in pass order
     float *pass_path_distance;  // [L,pass_slots,320] distance of the portal path of a pass that carries PB_PS_KEEPS (written for those only)
@@ -232,7 +230,6 @@ struct Scratch {    // per-chunk working memory, sized at create
     i64 *step_scale;       // [L, 3, 2, 16] per log2 texture size (widths, then heights): the flat texture step per
                            // column, the fraction at screen column 0, the camera's offset
 };
-#define FLAT_LIST_MAX 1024 // listed gap pixels per lane (a gap is typically one column wide)
 #define PLANE_LEVELS 32    // the per-lane plane tables of level lists up to this long (each) are staged in LDS by the
                            // shading kernels; longer lists are read where lane_tables_kernel left them
 
@@ -250,10 +247,11 @@ struct Scratch {    // per-chunk working memory, sized at create
 #define META_SECTOR_MASK 0x1FFFu  // plane sector + 1
 #define META_WALL_MASK 0xFFFFu    // sprite-clip linedef + 1
 
+// Does the view pixel with this word show the flat pass's picture: no wall tier, no plane, no masked texture?
+__device__ __forceinline__ bool gap_pixel(unsigned int word) { return !(word & (META_FILLED | META_MASKED)) && ((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) == 0; }
+
 #define STATUS_CAND_OVERFLOW 1
 #define STATUS_PASS_OVERFLOW 2
-#define SPAN_SELECT_BLOCKS 6144   // flat_span_select_kernel's grid: four times what 256 compute units hold at eight wavefronts per
-                                  // SIMD, so that rows of unequal cost even out
 #define STEP_TABLE 96   // int64 entries per lane of Scratch::step_scale
 
 __device__ __forceinline__ i64 mul64(i64 a, i64 b) { return (i64)((u64)a * (u64)b); }
@@ -430,8 +428,6 @@ __device__ __forceinline__ int grid_cell_of(const gd_map_desc *m, float px, floa
 #define FINE_MIXED 2u
 #define FINE_UNKNOWN 3u
 #define FINE_MASK_LEVELS 15
-#define FLAT_BATCH 2       // plane levels probed together in flat_select
-#define FLAT_BATCH_MASKED 3   // ... on maps with bit sets of reachable levels, where a batch holds levels that are looked at
 
 // Fine raster lookup.  Points outside the raster (or not finite) report FINE_UNKNOWN with a
 // negative cell, and the caller locates them with grid_cell_of.  The coarse cell of a point
@@ -507,8 +503,6 @@ __global__ void lane_tables_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_b
     const LaneCtx &c = sc.ctx[local];
     // the lane's per-column lists start empty
     for (int x = threadIdx.x; x < SW; x += blockDim.x) { sc.cand_count[(size_t)local * SW + x] = 0; sc.block_hit[(size_t)local * SW + x] = ~0ULL; }
-    // and no column holds an unresolved gap pixel yet
-    for (int k = threadIdx.x; k < 2 * SW; k += blockDim.x) sc.flat_col_top[(size_t)local * 2 * SW + k] = VH;
     {   // does a live billboard of the lane blend with what lies under it?
         bool blends = false;
         if (lanes.sprite_style && lanes.sprite_alive)
@@ -612,8 +606,7 @@ __global__ void lane_setup_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_ba
     sc.ctx[local] = c;
     int *span = sc.flat_span + (size_t)local * 4;
     span[0] = VH; span[1] = -1; span[2] = VH; span[3] = -1;
-    sc.flat_list_count[local] = 0;
-    if (local == 0) { *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
+    if (local == 0) { *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
 }
 
 __device__ __forceinline__ void ray_direction(const LaneCtx &c, int x, float *rx, float *ry) {
@@ -1089,29 +1082,207 @@ __device__ bool flat_ray_resolves(const DeviceMap &dm, const LaneCtx &c, float r
     return false;
 }
 //
-// flat_select_pixel is called by whole wavefronts whose 64 lanes look at 64 pixels of ONE row of one lane's
-// screen (wanted or not: every lane takes part in the level broadcasts); it returns the sector, -1 if no
-// level's probe point lies in a sector of that level.
-// MASKS: the map has enough plane levels for the per-bucket bit sets (level_mask_words() > 0).
-template <bool MASKS>
-__device__ __forceinline__ int flat_select_pixel(const DeviceMap &dm, const Scratch &sc, const gd_lanes_desc &lanes, int local, int n,
-                                                 int x, int y, bool wanted) {
+// The plane levels of one half of the screen (floors or ceilings) as one lane sees them.
+struct LevelSide {
+    const float *level, *reach, *far;   // plane height, and the bounds of the distance to the sectors of that level
+    const float4 *box;                  // the box around them
+    const unsigned int *masks;          // the lane's bit sets by bucket (level_bucket), null without
+    int count, first, mask_words;       // levels of this half, the first one's bit
+    int index_shift, mask_shift;        // where a raster entry keeps the sector's level index and the mask of undecided cells
+};
+__device__ __forceinline__ LevelSide level_side(const DeviceMap &dm, const Scratch &sc, int local, bool is_floor) {
+    const gd_map_desc *m = &dm.d;
+    LevelSide side;
+    const int total = m->floor_level_count + m->ceil_level_count;
+    side.count = is_floor ? m->floor_level_count : m->ceil_level_count;
+    side.first = is_floor ? 0 : m->floor_level_count;
+    side.level = is_floor ? m->floor_levels : m->ceil_levels;
+    side.reach = sc.level_reach + (size_t)local * total + side.first;
+    side.far = sc.level_far + (size_t)local * total + side.first;
+    side.box = dm.level_box + side.first;
+    side.mask_words = level_mask_words(m);
+    side.masks = sc.level_masks + (size_t)local * LEVEL_BUCKETS * side.mask_words;
+    side.index_shift = is_floor ? 16 : 20;
+    side.mask_shift = is_floor ? 0 : FINE_MASK_LEVELS;
+    return side;
+}
+
+// A hit of a flat probe as one number: distances are positive, so the smallest key is the nearest hit, the lowest sector on ties.
+#define PROBE_NONE 0xFFFFFFFFFFFFFFFFULL
+__device__ __forceinline__ u64 probe_key(float cd, int sector) { return ((u64)__float_as_uint(cd) << 32) | (unsigned)sector; }
+__device__ __forceinline__ float probe_distance(u64 key) { return key == PROBE_NONE ? GD_INF : __uint_as_float((unsigned)(key >> 32)); }
+__device__ __forceinline__ int probe_sector(u64 key) { return key == PROBE_NONE ? -1 : (int)(unsigned)key; }
+
+// The sector of plane level k that holds a point, from the coarse grid's cell (-1: located here), -1 if none does: what the
+// raster leaves undecided (engine.py:10994-11015).
+__device__ __forceinline__ int cell_sector(const DeviceMap &dm, bool is_floor, int k, float level, int cell, float px, float py) {
+    const gd_map_desc *m = &dm.d;
+    if (cell < 0) cell = grid_cell_of(m, px, py);
+    if (cell < 0) return -1;
+    const int2 range = dm.cell_range[cell];
+    int found = -1;
+    for (int it = range.x; it < range.y; ++it) {
+        const int4 item = dm.cell_item[it];
+        const int s = item.x & ~GRID_ALWAYS_INSIDE;
+        const bool same_level = item.y >= 0 ? ((is_floor ? (item.y & 0xFFFF) : (item.y >> 16)) == k)
+                                            : (m->sector_heights[2 * s + (is_floor ? 0 : 1)] == level);
+        if (!same_level || (found >= 0 && s > found)) continue;
+        if ((item.x & GRID_ALWAYS_INSIDE) || inside_edge_copies(dm.cell_edge, item.z, item.w, px, py)) found = s;
+    }
+    return found;
+}
+
+// Lanes of one wavefront leave words in LDS for one another: the order is the program's, the compiler has to keep it.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One pixel's flat ray, tested by PROBE_LANES lanes of a wavefront (a wavefront takes four pixels, of any lanes): the sector of the
+// nearest plane level whose probe point lies in a sector of that level, -1 if there is none (engine.py:10981-11024).  Sectors that
+// share a plane height share the probe point.  The lanes list the half's levels that the pixel's bucket names, then
+// keep those whose probe point lies in the box around the level's sectors, then look the kept ones up, each step for all of them at
+// once: a pixel costs a few rounds of loads, where one thread walking the levels of a map with a level per sector waited
+// for some forty, one after the other (98 us a pixel; the flat pass of 512 lanes with 800 plane levels took 1.0 ms, its chain of
+// kernels being as long as the slowest pixel of each).
+#define PROBE_LANES 16
+#define PROBE_GROUPS (64 / PROBE_LANES)
+#define PROBE_LEVELS 96     // levels a group can list by their bits; a pixel whose bucket names more tests the bits level by level
+#define PROBE_KEPT 32       // kept levels waiting to be looked up: one round and one more
+struct ProbeLds {
+    unsigned short level[PROBE_GROUPS][PROBE_LEVELS];
+    float kept_cd[PROBE_GROUPS][PROBE_KEPT]; unsigned short kept_level[PROBE_GROUPS][PROBE_KEPT];
+};
+__device__ __forceinline__ int flat_probe_group(const DeviceMap &dm, const Scratch &sc, const gd_lanes_desc &lanes, int local, int n, int x, int y, bool live, ProbeLds *lds) {
     const gd_map_desc *m = &dm.d;
     const LaneCtx &c = sc.ctx[local];
+    const int lane_id = threadIdx.x & 63, group = lane_id / PROBE_LANES, slot = lane_id - group * PROBE_LANES;
     const float delta = (float)y - flat_center(c);
     const bool is_floor = delta > 0;
-    float denom = fmaxf(fabsf(delta), 0.5f);
-    float cc = dm.cosine_correction[x];
-    float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x];
-    // A wavefront covers 64 pixels of one row (320 = 5 * 64), so the plane side and everything
-    // that depends only on (row, level) is the same in all its lanes.
-    const bool floor_uniform = __builtin_amdgcn_readfirstlane((int)is_floor) != 0;
-    const float *levels = floor_uniform ? m->floor_levels : m->ceil_levels;
-    const int level_count = floor_uniform ? m->floor_level_count : m->ceil_level_count;
-    const int mask_shift = floor_uniform ? 0 : FINE_MASK_LEVELS;
-    const int index_shift = floor_uniform ? 16 : 20;
-    const float *reach = sc.level_reach + (size_t)local * (m->floor_level_count + m->ceil_level_count) + (floor_uniform ? 0 : m->floor_level_count);
-    const float *far = sc.level_far + (size_t)local * (m->floor_level_count + m->ceil_level_count) + (floor_uniform ? 0 : m->floor_level_count);
+    const float denom = fmaxf(fabsf(delta), 0.5f), cc = dm.cosine_correction[x];
+    const float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x];
+    const LevelSide side = level_side(dm, sc, local, is_floor);
+    const unsigned int *row = side.mask_words > 0 ? side.masks + level_bucket((192.0f / denom) / cc) * side.mask_words : nullptr;
+    const u64 group_mask = ((1ULL << PROBE_LANES) - 1) << (group * PROBE_LANES), lower_lanes = (1ULL << lane_id) - 1;
+    // the levels the bucket names, listed: each lane takes whole words of the bit set
+    int named = live ? side.count : 0;
+    bool listed = false;
+    if (row) {
+        unsigned int bits[2] = {0u, 0u};
+        static_assert(LEVEL_MASK_WORDS_MAX <= 2 * PROBE_LANES, "flat_probe_group: two words of a bucket's bit set a lane");
+        const int end = side.first + side.count;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int word = slot * 2 + j, base = word * 32;
+            if (live && word < side.mask_words) bits[j] = row[word];
+            if (base < side.first) bits[j] = base + 32 <= side.first ? 0u : bits[j] & (~0u << (side.first - base));
+            if (base + 32 > end) bits[j] = base >= end ? 0u : bits[j] & ((1u << (end - base)) - 1u);
+        }
+        int at = __popc(bits[0]) + __popc(bits[1]);
+        const int own = at;
+#pragma unroll
+        for (int step = 1; step < PROBE_LANES; step <<= 1) { const int left = __shfl_up(at, step, PROBE_LANES); at += slot >= step ? left : 0; }
+        const int total = __shfl(at, PROBE_LANES - 1, PROBE_LANES);
+        at -= own;
+        listed = total <= PROBE_LEVELS;
+        if (listed) {
+            named = total;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                for (unsigned int rest = bits[j]; rest; rest &= rest - 1u) lds->level[group][at++] = (unsigned short)(slot * 64 + j * 32 + __ffs((int)rest) - 1 - side.first);
+        }
+        wave_lds_fence();
+    }
+    u64 best = PROBE_NONE;
+    int kept = 0;
+    auto look_up = [&]() {
+        wave_lds_fence();
+        for (int base = 0; __ballot(base < kept) != 0; base += PROBE_LANES) {
+            u64 key = PROBE_NONE;
+            if (base + slot < kept) {
+                const float cd = lds->kept_cd[group][base + slot];
+                const int k = lds->kept_level[group][base + slot];
+                const float px = c.x + rc * cd, py = c.y + rs * cd;
+                int cell;
+                const unsigned fine = fine_lookup(m, dm.fine_inverse, px, py, &cell);
+                const unsigned kind = FINE_KIND(fine);
+                int s = -1;
+                if (kind == FINE_DECIDED) {
+                    const int decided = (int)(fine & 0xFFFFu);
+                    const unsigned index = (fine >> side.index_shift) & 15u;   // the sector's level index, 15 = not recorded
+                    if (index == 15u ? m->sector_heights[2 * decided + (is_floor ? 0 : 1)] == side.level[k] : index == (unsigned)k) s = decided;
+                } else if (kind == FINE_UNKNOWN || (kind == FINE_MIXED && ((fine >> (side.mask_shift + k)) & 1u))) {
+                    s = cell_sector(dm, is_floor, k, side.level[k], cell, px, py);
+                }
+                if (s >= 0) key = probe_key(cd, s);
+            }
+#pragma unroll
+            for (int step = 1; step < PROBE_LANES; step <<= 1) {
+                const u64 other = ((u64)(unsigned)__shfl_xor((int)(key >> 32), step) << 32) | (unsigned)__shfl_xor((int)(unsigned)key, step);
+                key = other < key ? other : key;
+            }
+            best = key < best ? key : best;
+        }
+        kept = 0;
+        wave_lds_fence();
+    };
+    for (int base = 0; __ballot(base < named) != 0; base += PROBE_LANES) {
+        bool wanted = base + slot < named;
+        int k = base + slot;
+        if (wanted && listed) k = lds->level[group][base + slot];
+        if (wanted && row && !listed) { const int bit = side.first + k; wanted = (row[bit >> 5] >> (bit & 31)) & 1u; }
+        float cd = 0.0f;
+        if (wanted) {
+            const float height = is_floor ? (c.view_z - side.level[k]) : (side.level[k] - c.view_z);
+            const float4 box = side.box[k];
+            cd = (height * 192.0f / denom) / cc;
+            const float px = c.x + rc * cd, py = c.y + rs * cd;
+            wanted = height > 0 && finitef(cd) && cd > 0 && px >= box.x && px <= box.z && py >= box.y && py <= box.w && !(cd > probe_distance(best));
+        }
+        const u64 bits = __ballot(wanted) & group_mask;
+        if (wanted) {
+            const int at = kept + __popcll(bits & lower_lanes);
+            lds->kept_cd[group][at] = cd; lds->kept_level[group][at] = (unsigned short)k;
+        }
+        kept += __popcll(bits);
+        if (__ballot(kept > PROBE_KEPT - PROBE_LANES) != 0) look_up();
+    }
+    look_up();
+    return probe_sector(best);
+}
+
+// 64 neighbouring pixels of ONE row of one lane's screen, a wavefront's lane each (wanted or not: every lane takes part);
+// the sector of each as in flat_probe_group.  The 64 rays share the row, so a level's perpendicular distance is worked out once
+// (by the lane whose turn it is), and the levels none of the 64 can reach are never listed: those whose sectors lie nearer or
+// farther than any of their probe points, or beside the wedge the 64 rays span (with a level per sector that leaves a few of
+// forty).  The listed ones are looked up in the raster one after the other, ROW_BATCH loads in flight; what the raster leaves
+// undecided (a point near a linedef) waits in a queue in LDS and is settled at the end by all lanes together, unless a nearer
+// level has been found by then.  (Settled where it came up, a single undecided pixel held up its whole wavefront for
+// the three dependent loads of the coarse grid, at nearly every level.)
+#define ROW_LIST 96         // levels listed at a time: 32 and one more round of 64
+#define ROW_BATCH 4         // levels looked up together
+#define ROW_QUEUE (64 + 64 * ROW_BATCH)   // undecided probes waiting: at most 64 before a batch of levels
+#define ROW_NAMED 256       // levels listed by their bits; where the buckets name more, the bits are tested level by level
+struct RowLds {
+    float4 level[ROW_LIST];                                    // perpendicular distance, least distance to a sector, greatest, bits(index)
+    float queue_cd[ROW_QUEUE]; unsigned queue_who[ROW_QUEUE];   // lane << 16 | level index
+    unsigned short named[ROW_NAMED];
+    u64 best[64];
+};
+// MASKS: the map has enough plane levels for the per-bucket bit sets (level_mask_words() > 0).
+template <bool MASKS>
+__device__ __forceinline__ int flat_select_row(const DeviceMap &dm, const Scratch &sc, const gd_lanes_desc &lanes, int local, int n, int x, int y, bool wanted, RowLds *lds) {
+    const gd_map_desc *m = &dm.d;
+    const LaneCtx &c = sc.ctx[local];
+    const int lane_id = threadIdx.x & 63;
+    const u64 lower_lanes = (1ULL << lane_id) - 1;
+    const float delta = (float)y - flat_center(c);
+    const bool is_floor = __builtin_amdgcn_readfirstlane((int)(delta > 0)) != 0;   // the same in every lane, like the row
+    const float denom = fmaxf(fabsf(delta), 0.5f);
+    const float cc = dm.cosine_correction[x];
+    const float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x];
+    const LevelSide side = level_side(dm, sc, local, is_floor);
     // cd = perpendicular / cc below is the hot division.  With y = RN(1 / cc), q = RN(p * y) is within
     // one ulp of p / cc, and RN(q + RN(p - cc * q) * y) is then the correctly rounded quotient
     // (Markstein's theorem; the inner product is exact in an FMA) as long as nothing over- or
@@ -1122,75 +1293,47 @@ __device__ __forceinline__ int flat_select_pixel(const DeviceMap &dm, const Scra
     // the probe point camera + ray * cd in raster cell units, as one multiply-add per axis
     const float cell_x0 = (c.x - m->grid_min_x) * inv_fine, cell_y0 = (c.y - m->grid_min_y) * inv_fine;
     const float cell_dx = rc * inv_fine, cell_dy = rs * inv_fine;
-    const int slot_in_wave = threadIdx.x & 63;
-    // cd <= perpendicular / (smallest cc of the wavefront): with it a level whose every sector is
-    // farther than that from the camera is dropped for the whole wavefront at once
+    // perpendicular / (smallest cc of the 64) bounds every cd from above, perpendicular / (largest cc) from below
     const float reach_scale = dm.strip_reach_scale[__builtin_amdgcn_readfirstlane(x >> 6)];
-    // and cd >= perpendicular / (largest cc of the wavefront): a level whose every sector ends nearer than that
     const float far_scale = dm.strip_far_scale[__builtin_amdgcn_readfirstlane(x >> 6)];
-    float best = GD_INF; int best_sector = -1;
-    const bool camera_in_grid = grid_cell_of(m, c.x, c.y) >= 0;
+    // the wedge's leftmost and rightmost ray; rays turn clockwise from left to right
+    const float left_c = bcast(rc, 0), left_s = bcast(rs, 0), right_c = bcast(rc, 63), right_s = bcast(rs, 63);
+    u64 best = PROBE_NONE;
     bool done = !wanted;
-    // The levels some pixel of the wavefront can reach at all (level_bucket): the bit sets of the buckets its 64 scales
-    // fall into, joined; lane j holds word j.  Levels outside them are skipped by the whole wavefront at once.
-    const int mask_words = MASKS ? level_mask_words(m) : 0;
-    constexpr int BATCH = MASKS ? FLAT_BATCH_MASKED : FLAT_BATCH;
-    unsigned int joined_word = 0u;
-    if (MASKS) {
-        const int bucket = level_bucket((192.0f / denom) / cc);
-        int lowest = bucket, highest = bucket;
-#pragma unroll
-        for (int step = 1; step < 64; step <<= 1) { lowest = min(lowest, __shfl_xor(lowest, step)); highest = max(highest, __shfl_xor(highest, step)); }
-        const unsigned int *masks = sc.level_masks + (size_t)local * LEVEL_BUCKETS * mask_words;
-        if (slot_in_wave < mask_words) for (int b = lowest; b <= highest; ++b) joined_word |= masks[b * mask_words + slot_in_wave];
-    }
-    const int first_bit = floor_uniform ? 0 : m->floor_level_count;
-    for (int base = 0; base < level_count; base += 64) {
-        if (__ballot(!done) == 0) break;   // every lane takes part in the level broadcasts below, wanted or not
-        u64 chunk_levels = ~0ULL;          // bit k: level base + k is worth a look
-        if (MASKS) {
-            const int at = first_bit + base, word = at >> 5, shift = at & 31;
-            const u64 w0 = (unsigned)bcast((int)joined_word, word), w1 = (unsigned)bcast((int)joined_word, (word + 1) & 63), w2 = (unsigned)bcast((int)joined_word, (word + 2) & 63);
-            chunk_levels = ((w0 | (w1 << 32)) >> shift) | (shift ? w2 << (64 - shift) : 0ULL);   // lanes past the last word hold zeros
-            if (chunk_levels == 0ULL) continue;    // the same in every lane
-        }
-        // lane k works out level base+k: its height and perpendicular distance (one division for
-        // the wavefront instead of one per level per lane); a level the plane cannot show gets -1
-        const int mine = base + slot_in_wave;
-        const float my_level = mine < level_count ? levels[mine] : 0.0f;
-        const float my_reach = mine < level_count ? reach[mine] : 0.0f;
-        const float my_far = mine < level_count ? far[mine] : GD_INF;
-        const float my_height = floor_uniform ? (c.view_z - my_level) : (my_level - c.view_z);
-        const float my_perpendicular = (mine < level_count && my_height > 0) ? my_height * 192.0f / denom : -1.0f;
-        const int chunk = level_count - base < 64 ? level_count - base : 64;
-        // Levels are taken BATCH at a time: first the probe points and raster loads of the whole
-        // batch (independent, so their memory latencies overlap), then the decisions in level order.
-        // A load for a level past the one that ends the scan is wasted, never wrong.
-        // Only the levels whose bit is set are walked (with bit sets: the few that some pixel here can reach), so a
-        // batch holds BATCH levels that are looked at, not BATCH list positions.  `rest` is the same in every lane.
-        if (chunk < 64) chunk_levels &= (1ULL << chunk) - 1ULL;
-        u64 rest = ((u64)(unsigned)__builtin_amdgcn_readfirstlane((int)(chunk_levels >> 32)) << 32) | (u64)(unsigned)__builtin_amdgcn_readfirstlane((int)chunk_levels);
-        while (rest != 0ULL) {
-            if (__ballot(!done) == 0) break;
-            float cdv[BATCH];
-            unsigned finev[BATCH];
-            int cellv[BATCH];
-            int kv[BATCH];
-#pragma unroll
-            for (int j = 0; j < BATCH; ++j) {
-                kv[j] = rest ? __ffsll((long long)rest) - 1 : -1;
-                rest &= rest - 1ULL;
+    int listed = 0, queued = 0;                   // the same in every lane
+    auto settle_queue = [&]() {
+        if (queued == 0) return;
+        lds->best[lane_id] = best;
+        wave_lds_fence();
+        for (int base = 0; base < queued; base += 64) {
+            const int e = base + lane_id;
+            const bool live = e < queued;
+            const unsigned who = live ? lds->queue_who[e] : 0u;
+            const int owner = (int)(who >> 16), k = (int)(who & 0xFFFFu);
+            const float cd = live ? lds->queue_cd[e] : 0.0f;
+            const float o_rc = __shfl(rc, owner), o_rs = __shfl(rs, owner);
+            if (live && !(cd > probe_distance(lds->best[owner]))) {
+                const int s = cell_sector(dm, is_floor, k, side.level[k], -1, c.x + o_rc * cd, c.y + o_rs * cd);
+                if (s >= 0) atomicMin(&lds->best[owner], probe_key(cd, s));
             }
+        }
+        wave_lds_fence();
+        best = lds->best[lane_id];
+        queued = 0;
+    };
+    auto probe_listed = [&]() {
+        wave_lds_fence();
+        for (int j0 = 0; j0 < listed; j0 += ROW_BATCH) {
+            if (__ballot(!done) == 0) break;
+            if (queued > 64) settle_queue();
+            float cdv[ROW_BATCH]; unsigned finev[ROW_BATCH]; int kv[ROW_BATCH];
 #pragma unroll
-            for (int j = 0; j < BATCH; ++j) {
-                const int k = kv[j];
-                cdv[j] = -1.0f; finev[j] = 0x40000000u; cellv[j] = -1;
-                if (k < 0) continue;                             // the same in every lane
-                const float perpendicular = bcast(my_perpendicular, k);
-                const float nearest = bcast(my_reach, k);
-                if (!(perpendicular > 0)) continue;              // the same in every lane
-                if (perpendicular * reach_scale < nearest) continue;   // the same in every lane: no lane can reach the level
-                if (perpendicular * far_scale > bcast(my_far, k)) continue;   // the same in every lane: every lane looks past the level
+            for (int j = 0; j < ROW_BATCH; ++j) {
+                cdv[j] = -1.0f; finev[j] = 0x40000000u; kv[j] = 0;                    // empty: nothing there
+                if (j0 + j >= listed) continue;                                       // the same in every lane
+                const float4 entry = lds->level[j0 + j];
+                kv[j] = __float_as_int(entry.w);
+                const float perpendicular = entry.x;
                 float cd;
                 if (cc_plain && perpendicular >= 1e-18f && perpendicular <= 1e18f) {
                     const float q = perpendicular * inv_cc;
@@ -1199,288 +1342,180 @@ __device__ __forceinline__ int flat_select_pixel(const DeviceMap &dm, const Scra
                     cd = perpendicular / cc;
                 }
                 cdv[j] = cd;
-                if (done || !(finitef(cd) && cd > 0) || cd > best || cd < nearest) continue;   // cd < nearest: every sector at this level is farther away
-                finev[j] = fine_lookup_cells(m, __builtin_fmaf(cd, cell_dx, cell_x0), __builtin_fmaf(cd, cell_dy, cell_y0), &cellv[j]);
+                if (cd > probe_distance(best)) done = true;      // later levels are at least this far
+                if (done || !(finitef(cd) && cd > 0) || cd < entry.y || cd > entry.z) continue;
+                int cell;
+                finev[j] = fine_lookup_cells(m, __builtin_fmaf(cd, cell_dx, cell_x0), __builtin_fmaf(cd, cell_dy, cell_y0), &cell);
             }
 #pragma unroll
-            for (int j = 0; j < BATCH; ++j) {
+            for (int j = 0; j < ROW_BATCH; ++j) {
+                const unsigned fine = finev[j], kind = FINE_KIND(fine);
                 const int k = kv[j];
-                if (k < 0 || done) continue;
-                const float cd = cdv[j];
-                if (!(finitef(cd) && cd > 0)) continue;
-                if (cd > best) { done = true; continue; }        // later levels are at least this far
-                const unsigned fine = finev[j];
-                const unsigned kind = FINE_KIND(fine);
-                if (kind == FINE_EMPTY) continue;                // also levels skipped above
-                const float level = bcast(my_level, k);
+                bool undecided = false;
                 if (kind == FINE_DECIDED) {
                     const int s = (int)(fine & 0xFFFFu);
-                    const unsigned listed = (fine >> index_shift) & 15u;   // the sector's level index, 15 = not recorded
-                    bool same_level = listed == (unsigned)(base + k);
-                    if (listed == 15u) same_level = m->sector_heights[2 * s + (floor_uniform ? 0 : 1)] == level;
-                    if (same_level && (cd < best || (cd == best && s < best_sector))) { best = cd; best_sector = s; }
-                    continue;
-                }
-                if (kind == FINE_MIXED && !((fine >> (mask_shift + base + k)) & 1u)) continue;   // no sector here has this level
-                const float px = c.x + rc * cd, py = c.y + rs * cd;
-                int cell = cellv[j];
-                if (cell < 0) cell = grid_cell_of(m, px, py);
-                // Outside the grid (above, below or right of every linedef) no sector holds the point.  Seen from a
-                // camera inside that convex region, the probe points of the levels still to come lie farther
-                // along the same ray, which has left the region for good.
-                if (cell < 0) { done = camera_in_grid; continue; }
-                const int2 range = dm.cell_range[cell];
-                for (int it = range.x; it < range.y; ++it) {
-                    const int4 item = dm.cell_item[it];
-                    const int s = item.x & ~GRID_ALWAYS_INSIDE;
-                    const bool same_level = item.y >= 0 ? ((floor_uniform ? (item.y & 0xFFFF) : (item.y >> 16)) == base + k)
-                                                        : (m->sector_heights[2 * s + (floor_uniform ? 0 : 1)] == level);
-                    if (!same_level) continue;
-                    if (cd < best || (cd == best && s < best_sector)) {
-                        if ((item.x & GRID_ALWAYS_INSIDE) || inside_edge_copies(dm.cell_edge, item.z, item.w, px, py)) { best = cd; best_sector = s; }
+                    const unsigned index = (fine >> side.index_shift) & 15u;   // the sector's level index, 15 = not recorded
+                    if (index == 15u ? m->sector_heights[2 * s + (is_floor ? 0 : 1)] == side.level[k] : index == (unsigned)k) {
+                        const u64 key = probe_key(cdv[j], s);
+                        best = key < best ? key : best;
                     }
+                } else if (kind == FINE_UNKNOWN || (kind == FINE_MIXED && ((fine >> (side.mask_shift + k)) & 1u))) {
+                    undecided = true;
                 }
+                const u64 waiting = __ballot(undecided);
+                if (undecided) {
+                    const int at = queued + __popcll(waiting & lower_lanes);
+                    lds->queue_cd[at] = cdv[j]; lds->queue_who[at] = ((unsigned)lane_id << 16) | (unsigned)k;
+                }
+                queued += __popcll(waiting);
             }
         }
-    }
-    return best_sector;
-}
-
-// One pixel's flat ray on its own (flat_select_pixel shares work between the 64 pixels of a row): the sector of
-// the nearest plane level whose probe point lies in a sector of that level, -1 if there is none
-// (engine.py:10981-11024).
-// The plane levels of the map and, per lane and level, bounds of the distance from the camera to the sectors of that
-// level: floors first, then ceilings, in all three lists.  A pixel's scan reads them level after level, each read
-// waiting for the one before (the scan may end at any level), so a block that works on one lane copies them to LDS
-// first: with a plane level per sector (several hundred) the scans otherwise spend their time waiting for device memory.
-#define FLAT_LDS_LEVELS (32 * LEVEL_MASK_WORDS_MAX)
-struct LevelLists { const float *level, *reach, *far; const unsigned int *masks; int floors, ceilings, mask_words; };
-struct LevelLds { float lists[3 * FLAT_LDS_LEVELS]; };
-__device__ __forceinline__ LevelLists stage_level_lists(const DeviceMap &dm, const Scratch &sc, int local, LevelLds *lds) {
-    const gd_map_desc *m = &dm.d;
-    LevelLists lists;
-    lists.floors = m->floor_level_count; lists.ceilings = m->ceil_level_count;
-    lists.mask_words = level_mask_words(m);
-    const int total = lists.floors + lists.ceilings;
-    const float *reach = sc.level_reach + (size_t)local * total, *far = sc.level_far + (size_t)local * total;
-    if (total > FLAT_LDS_LEVELS) {        // read where they are; `level` then only serves the floors (see flat_probe_pixel)
-        lists.level = nullptr; lists.reach = reach; lists.far = far; lists.masks = nullptr;   // more levels than the bit sets cover
-        return lists;
-    }
-    for (int k = threadIdx.x; k < total; k += blockDim.x) {
-        lds->lists[k] = k < lists.floors ? m->floor_levels[k] : m->ceil_levels[k - lists.floors];
-        lds->lists[FLAT_LDS_LEVELS + k] = reach[k];
-        lds->lists[2 * FLAT_LDS_LEVELS + k] = far[k];
-    }
-    const unsigned int *masks = sc.level_masks + (size_t)local * LEVEL_BUCKETS * lists.mask_words;
-    lists.level = lds->lists; lists.reach = lds->lists + FLAT_LDS_LEVELS; lists.far = lds->lists + 2 * FLAT_LDS_LEVELS;
-    lists.masks = masks;   // one row of a few words per pixel: read where it is
-    return lists;   // the caller synchronises the block before the first scan
-}
-
-__device__ int flat_probe_pixel(const DeviceMap &dm, const Scratch &sc, const LevelLists &lists, int local, float rc, float rs, float cc, int y) {
-    const LaneCtx &c = sc.ctx[local];
-    const gd_map_desc *m = &dm.d;
-    const float delta = (float)y - flat_center(c);
-    const bool is_floor = delta > 0;
-    const float denom = fmaxf(fabsf(delta), 0.5f);
-    const int first = is_floor ? 0 : lists.floors;
-    const float *levels = lists.level ? lists.level + first : (is_floor ? m->floor_levels : m->ceil_levels);
-    const int level_count = is_floor ? lists.floors : lists.ceilings;
-    const float *reach = lists.reach + first, *far = lists.far + first;
-    float best = GD_INF; int best_sector = -1;
-    const bool camera_in_grid = grid_cell_of(m, c.x, c.y) >= 0;
-    // one level of the scan; true ends it
-    auto visit = [&](int k) -> bool {
-        const float level = levels[k];
-        const float height = is_floor ? (c.view_z - level) : (level - c.view_z);
-        if (!(height > 0)) return false;
-        const float cd = (height * 192.0f / denom) / cc;
-        if (!(finitef(cd) && cd > 0)) return false;
-        if (cd > best) return true;                                 // later levels are at least this far
-        if (cd < reach[k] || cd > far[k]) return false;            // no sector of this level lies at that distance
-        const float px = c.x + rc * cd, py = c.y + rs * cd;
-        int cell;
-        const unsigned fine = fine_lookup(m, dm.fine_inverse, px, py, &cell);
-        const unsigned kind = FINE_KIND(fine);
-        if (kind == FINE_EMPTY) return false;
-        if (kind == FINE_DECIDED) {
-            const int s = (int)(fine & 0xFFFFu);
-            if (m->sector_heights[2 * s + (is_floor ? 0 : 1)] == level && (cd < best || (cd == best && s < best_sector))) { best = cd; best_sector = s; }
-            return false;
-        }
-        if (cell < 0) cell = grid_cell_of(m, px, py);
-        if (cell < 0) return camera_in_grid;   // outside the grid no sector holds the point; seen from inside it, the ray has left that convex region for good
-        const int2 range = dm.cell_range[cell];
-        for (int it = range.x; it < range.y; ++it) {
-            const int4 item = dm.cell_item[it];
-            const int s = item.x & ~GRID_ALWAYS_INSIDE;
-            if (m->sector_heights[2 * s + (is_floor ? 0 : 1)] != level) continue;
-            if (cd < best || (cd == best && s < best_sector)) {
-                if ((item.x & GRID_ALWAYS_INSIDE) || inside_edge_copies(dm.cell_edge, item.z, item.w, px, py)) { best = cd; best_sector = s; }
-            }
-        }
-        return false;
+        listed = 0;
+        wave_lds_fence();
     };
-    // With bit sets: only the levels whose distance bounds can hold a probe of this pixel's scale at all (level_bucket),
-    // in level order; bits [first, end) of the bucket's row are this half's levels.  Without: every level.
-    const bool masked = lists.mask_words > 0 && lists.masks;
-    const unsigned int *row = masked ? lists.masks + level_bucket((192.0f / denom) / cc) * lists.mask_words : nullptr;
-    const int end = first + level_count;
-    int word = (first >> 5) - 1, k = -1;
-    unsigned int bits = 0u;
-    for (;;) {
-        if (masked) {
-            while (!bits && word < ((end - 1) >> 5)) {
-                ++word;
-                bits = row[word];
-                if (word == first >> 5) bits &= ~0u << (first & 31);
-                if (word == (end - 1) >> 5 && (end & 31)) bits &= (1u << (end & 31)) - 1u;
-            }
-            if (!bits) break;
-            k = (word << 5) + __ffs((int)bits) - 1 - first;
-            bits &= bits - 1;
-        } else if (++k >= level_count) {
-            break;
+    // The levels the buckets of the 64 scales name: lane j joins word j of their bit sets.
+    int named = side.count;
+    bool by_bits = false;
+    unsigned int joined_word = 0u;
+    if (MASKS) {
+        const int bucket = level_bucket((192.0f / denom) / cc);
+        int lowest = bucket, highest = bucket;
+#pragma unroll
+        for (int step = 1; step < 64; step <<= 1) { lowest = min(lowest, __shfl_xor(lowest, step)); highest = max(highest, __shfl_xor(highest, step)); }
+        if (lane_id < side.mask_words) for (int b = lowest; b <= highest; ++b) joined_word |= side.masks[b * side.mask_words + lane_id];
+        unsigned int bits = joined_word;
+        const int base = lane_id * 32, end = side.first + side.count;
+        if (base < side.first) bits = base + 32 <= side.first ? 0u : bits & (~0u << (side.first - base));
+        if (base + 32 > end) bits = base >= end ? 0u : bits & ((1u << (end - base)) - 1u);
+        int at = __popc(bits);
+        const int own = at;
+#pragma unroll
+        for (int step = 1; step < LEVEL_MASK_WORDS_MAX; step <<= 1) { const int left = __shfl_up(at, step); at += lane_id >= step ? left : 0; }
+        const int total = bcast(at, LEVEL_MASK_WORDS_MAX - 1);
+        at -= own;
+        by_bits = total <= ROW_NAMED;
+        if (by_bits) {
+            named = total;
+            for (; bits; bits &= bits - 1u) lds->named[at++] = (unsigned short)(base + __ffs((int)bits) - 1 - side.first);
         }
-        if (visit(k)) break;
+        wave_lds_fence();
     }
-    return best_sector;
+    for (int base = 0; base < named; base += 64) {
+        if (__ballot(!done) == 0) break;
+        bool reachable = base + lane_id < named;
+        int k = base + lane_id;
+        if (MASKS) {
+            if (by_bits) { if (reachable) k = lds->named[base + lane_id]; }
+            else {
+                const int bit = side.first + k;
+                const unsigned int word = (unsigned)__shfl((int)joined_word, (bit >> 5) & 63);   // lanes past the last word hold zeros
+                reachable = reachable && ((word >> (bit & 31)) & 1u);
+            }
+        }
+        float4 entry = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(k));
+        if (reachable) {
+            const float height = is_floor ? (c.view_z - side.level[k]) : (side.level[k] - c.view_z);
+            const float4 box = side.box[k];
+            entry.x = height * 192.0f / denom; entry.y = side.reach[k]; entry.z = side.far[k];
+            // the box's corner farthest to the right of the leftmost ray, farthest to the left of the rightmost one, and farthest ahead
+            // (a map unit to spare: the rays are unit vectors, the coordinates below 2^15)
+            const float x0 = box.x - c.x, x1 = box.z - c.x, y0 = box.y - c.y, y1 = box.w - c.y;
+            const float beyond_left = fminf(left_c * y0, left_c * y1) - fmaxf(left_s * x0, left_s * x1);
+            const float beyond_right = fmaxf(right_c * y0, right_c * y1) - fminf(right_s * x0, right_s * x1);
+            reachable = height > 0 && entry.x > 0 && !(entry.x * reach_scale < entry.y) && !(entry.x * far_scale > entry.z) &&
+                        !(beyond_left > 1.0f) && !(beyond_right < -1.0f);
+        }
+        const u64 bits = __ballot(reachable);
+        if (reachable) lds->level[listed + __popcll(bits & lower_lanes)] = entry;
+        listed += __popcll(bits);
+        if (listed > ROW_LIST - 64) probe_listed();
+    }
+    probe_listed();
+    settle_queue();
+    return probe_sector(best);
 }
 
 // The flat pass runs after the walls and only where its result can matter.  A pixel a wall tier filled never
 // shows it; a pixel a plane of the wall pass claimed only asks whether the flat ray resolved at all, and only
 // where a sprite stands behind the plane with no sprite clip recorded, which the sprite pass finds out for
 // itself (flat_ray_resolves); the few pixels left (columns whose traversal left a gap) show the flat pass's
-// picture.  wall_raster_kernel lists those.  flat_gap_column_kernel, one block per lane, first selects them, one
-// thread per listed pixel, and notes per screen half and column the topmost one that stayed unresolved.
+// picture.  wall_raster_kernel lists their columns, of all lanes together: most lanes have none, some have hundreds.
+// flat_gap_kernel, a work-group per listed column, selects them.
 //
-// Then the vertical repair (engine.py:11026-11083) of the listed pixels, column by column.  An unresolved pixel takes
-// the sector of the next resolved pixel below it in its half of the screen; when that sector is not the camera's,
+// Then, column by column, the vertical repair (engine.py:11026-11083).  An unresolved
+// pixel takes the sector of the next resolved pixel below it in its half of the screen; when that sector is not the camera's,
 // the pixel is its own left and right anchor in the horizontal repair (engine.py:11085-11135), which then leaves
 // it as it is: such a pixel is settled here and its row needs no further work.  Only the rows of the others (no
 // resolved pixel below, or the camera's own sector) are noted for the row kernels (flat_span_select_kernel,
-// flat_tail_kernel, flat_span_finish_kernel).  A wavefront takes one column that holds an unresolved listed pixel
-// after another, its lanes probing 64 rows of the column at a time, from the bottom of the half up to the column's
-// topmost unresolved listed pixel.
-// GAP_THREADS: three wavefronts a lane.  Most lanes have a few dozen listed pixels and one or two columns to repair, and a
-// launch lasts as many rounds of blocks as the chip needs to hold them all: with five wavefronts a block (one thread a
-// column) it took 0.05 ms longer, with one or two the lanes with many columns hold it up.
-#define GAP_THREADS 192
-__global__ void __launch_bounds__(GAP_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) flat_gap_column_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
-    const int local = blockIdx.x;
-    if (local >= lane_count) return;
-    const int listed = sc.flat_list_count[local];
-    if (listed == 0) return;                         // the same in every thread: a lane without gap pixels has no flat pass
-    const LaneCtx &c = sc.ctx[local];
-    const int n = lane_base + local;
-    const int lane_id = threadIdx.x & 63;
-    int *span = sc.flat_span + (size_t)local * 4;
-    const int last_ceiling_row = c.last_ceiling_row;
-    const unsigned int *meta = sc.meta + (size_t)local * VH * SW;
-    __shared__ LevelLds level_lds;
-    const LevelLists lists = stage_level_lists(dm, sc, local, &level_lds);
-    __syncthreads();
-    if (listed > FLAT_LIST_MAX) {
-        // too many to list (a camera outside the map, say): every row of both halves is selected and repaired
-        if (threadIdx.x == 0) {
-            if (last_ceiling_row >= 0) { span[0] = 0; span[1] = last_ceiling_row; }
-            if (last_ceiling_row + 1 < VH) { span[2] = last_ceiling_row + 1; span[3] = VH - 1; }
-        }
-    } else {
-        for (int slot = threadIdx.x; slot < listed; slot += blockDim.x) {
-            const int pixel = sc.flat_list[(size_t)local * FLAT_LIST_MAX + slot];
-            const int y = pixel / SW, x = pixel - y * SW;
-            const int s = flat_probe_pixel(dm, sc, lists, local, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x], dm.cosine_correction[x], y);
-            const size_t i = (size_t)local * VH * SW + pixel;
-            sc.flat_sector[i] = (unsigned short)(s < 0 ? c.sector : s);
-            sc.flat_flags[i] = s < 0 ? 1 : 0;
-            if (s < 0) {
-                const bool floor_row = ((float)y - flat_center(c)) > 0;
-                atomicMin(&sc.flat_col_top[((size_t)local * 2 + (floor_row ? 1 : 0)) * SW + x], y);
-            }
-        }
-    }
-    __threadfence_block();   // what the selection wrote (column tops, row ranges) is read below by other threads of the block
-    __syncthreads();
-    // the lane's columns with work, both halves together, join one work list that flat_gap_repair_kernel deals out to
-    // wavefronts evenly, whichever lanes they come from
-    __shared__ int column_list[2 * SW];
-    __shared__ int column_count, list_base;
-    if (threadIdx.x == 0) column_count = 0;
-    __syncthreads();
-    for (int half = 0; half < 2; ++half) for (int x = threadIdx.x; x < SW; x += blockDim.x) {
-        int *top_at = sc.flat_col_top + ((size_t)local * 2 + half) * SW + x;
-        const int top = __hip_atomic_load(top_at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // where the atomics above wrote, not a cached copy
-        if (top < VH) {
-            column_list[atomicAdd(&column_count, 1)] = x | (top << 9) | (half << 17) | (local << 18);
-        }
-    }
-    __syncthreads();
-    const int columns = column_count;
-    if (columns == 0) return;                        // the same in every thread
-    if (threadIdx.x == 0) list_base = atomicAdd(sc.gap_column_count, columns);
-    __syncthreads();
-    for (int k = threadIdx.x; k < columns; k += blockDim.x) sc.gap_columns[list_base + k] = column_list[k];
+// flat_tail_kernel, flat_span_finish_kernel).
+
+// A lane's half of the screen gets rows to repair: it joins the work list of the row kernels when it gets its first.
+__device__ __forceinline__ void note_row(const Scratch &sc, int local, int half, int y) {
+    int *span = sc.flat_span + (size_t)local * 4 + 2 * half;
+    atomicMax(&span[1], y);
+    if (atomicMin(&span[0], y) == VH) sc.flat_spans[atomicAdd(sc.flat_span_count, 1)] = (local << 1) | half;
 }
 
-// The vertical repair (engine.py:11026-11083) of the listed gap pixels, column by column: one work-group per listed column
-// (flat_gap_column_kernel's work list), one wavefront per chunk of 64 rows between the column's topmost unresolved listed
-// pixel and the bottom of its half, all chunks probed at once.  What a chunk needs from the chunks below it (the sector of
-// the next resolved pixel down) goes through LDS once every chunk has probed: a column lasts as long as its slowest
-// pixel's walk over the plane levels, not as long as one such walk per chunk.
-#define GAP_REPAIR_BLOCKS 8192
-#define GAP_REPAIR_CHUNKS ((VH + 63) / 64)
-__global__ void __launch_bounds__(64 * GAP_REPAIR_CHUNKS) __attribute__((amdgpu_waves_per_eu(8, 8))) flat_gap_repair_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
-    __shared__ LevelLds level_lds;
-    __shared__ int chunk_found[GAP_REPAIR_CHUNKS], chunk_sector[GAP_REPAIR_CHUNKS];
+// GAP_WAVES wavefronts a column, which probe 16 of its rows at a time: first the gap pixels', then the others' from the topmost
+// unresolved gap pixel down, until the lowest one is past and a resolved pixel below it is found (or the half ends).
+#define GAP_WAVES 4
+#define ROW_UNPROBED -2
+__global__ void __launch_bounds__(64 * GAP_WAVES) flat_gap_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
+    __shared__ ProbeLds probe_lds[GAP_WAVES];
+    __shared__ short row_sector[VH];                  // the sector of each row's pixel, -1 unresolved, ROW_UNPROBED
+    __shared__ int unresolved_first, unresolved_last;
     const int total = *sc.gap_column_count;
-    const int lane_id = threadIdx.x & 63, chunk = threadIdx.x >> 6;
-    int staged = -1;
-    LevelLists lists;
+    const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63, group = wave * PROBE_GROUPS + lane_id / PROBE_LANES;
+    const bool speaks = (lane_id & (PROBE_LANES - 1)) == 0;
+    constexpr int ROWS = GAP_WAVES * PROBE_GROUPS;
     for (int entry = blockIdx.x; entry < total; entry += gridDim.x) {
-        const int packed = sc.gap_columns[entry];
-        const int x = packed & 511, first = (packed >> 9) & 255, half = (packed >> 17) & 1, local = packed >> 18;
-        __syncthreads();         // nobody reads the previous column's chunk results or the previous lane's lists any more
-        if (local != staged) {   // the same in every thread
-            lists = stage_level_lists(dm, sc, local, &level_lds);
-            staged = local;
-        }
-        __syncthreads();
+        const int2 packed = sc.gap_columns[entry];
+        const int x = packed.x & 511, local = packed.x >> 9;
         const LaneCtx &c = sc.ctx[local];
-        const int n = lane_base + local;
-        int *span = sc.flat_span + (size_t)local * 4;
-        const unsigned int *meta = sc.meta + (size_t)local * VH * SW;
-        const int half_end = half ? VH - 1 : c.last_ceiling_row;
-        const float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x], cc = dm.cosine_correction[x];
-        const int chunks = (half_end - first) / 64 + 1;   // at most GAP_REPAIR_CHUNKS
-        const int y = first + chunk * 64 + lane_id;
-        const bool live = chunk < chunks && y <= half_end;
-        const int s = live ? flat_probe_pixel(dm, sc, lists, local, rc, rs, cc, y) : -1;
-        const u64 resolved = __ballot(live && s >= 0);
-        const int first_sector = __shfl(s, resolved ? __ffsll((long long)resolved) - 1 : 0);
-        if (lane_id == 0) { chunk_found[chunk] = resolved != 0; chunk_sector[chunk] = first_sector; }
-        __syncthreads();
-        // the next resolved pixel below: in this chunk, else the topmost one of the nearest chunk below that has any
-        bool below_found = false; int below_sector = 0;
-        for (int lower_chunk = chunk + 1; lower_chunk < chunks && !below_found; ++lower_chunk)
-            if (chunk_found[lower_chunk]) { below_found = true; below_sector = chunk_sector[lower_chunk]; }
-        const u64 lower = resolved & ~((2ULL << lane_id) - 1);   // resolved rows of this chunk below this one (none for lane 63)
-        const int from = lower ? __ffsll((long long)lower) - 1 : lane_id;
-        const int taken = __shfl(s, from);
-        const bool found = lower ? true : below_found;
-        const int sector = lower ? taken : below_sector;
-        if (live && s < 0) {
-            const size_t i = (size_t)y * SW + x;
-            const unsigned int word = meta[i];
-            const bool listed = !(word & (META_FILLED | META_MASKED)) && ((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) == 0;
-            if (listed) {
-                if (found && sector != c.sector) {
-                    sc.flat_sector[(size_t)local * VH * SW + i] = (unsigned short)sector;
-                    sc.flat_flags[(size_t)local * VH * SW + i] = (unsigned char)(1 | 2 | 4 | 8);
+        const int n = lane_base + local, last_ceiling_row = c.last_ceiling_row;
+        const unsigned int *meta = sc.meta + (size_t)local * VH * SW + x;
+        unsigned short *sector = sc.flat_sector + (size_t)local * VH * SW + x;
+        unsigned char *flags = sc.flat_flags + (size_t)local * VH * SW + x;
+        for (int half = 0; half < 2; ++half) {
+            const int half_end = half ? VH - 1 : last_ceiling_row;
+            const int lo = max(packed.y & 255, half ? last_ceiling_row + 1 : 0), hi = min((packed.y >> 8) - 1, half_end);
+            if (lo > hi) continue;                    // the same in the whole block, like everything that steers it here
+            __syncthreads();                          // nobody reads the previous column's rows any more
+            if (threadIdx.x == 0) { unresolved_first = VH; unresolved_last = -1; }
+            __syncthreads();
+            for (int y0 = lo; y0 <= hi; y0 += ROWS) {
+                const int y = y0 + group;
+                const bool shown = y <= hi && gap_pixel(meta[(size_t)y * SW]);
+                const int s = flat_probe_group(dm, sc, lanes, local, n, x, y <= hi ? y : lo, shown, &probe_lds[wave]);
+                if (y > hi || !speaks) continue;
+                row_sector[y] = shown ? (short)s : (short)ROW_UNPROBED;
+                if (!shown) continue;
+                sector[(size_t)y * SW] = (unsigned short)(s < 0 ? c.sector : s);
+                flags[(size_t)y * SW] = s < 0 ? 1 : 0;
+                if (s < 0) { atomicMin(&unresolved_first, y); atomicMax(&unresolved_last, y); }
+            }
+            __syncthreads();
+            const int first = unresolved_first, last = unresolved_last;
+            if (last < 0) continue;
+            int rows_end = hi + 1;                    // rows below it are known or were found not to matter
+            for (int y0 = first + 1; y0 <= half_end; y0 += ROWS) {
+                const int y = y0 + group;
+                const bool live = y <= half_end && (y > hi || row_sector[y] == ROW_UNPROBED);
+                const int s = flat_probe_group(dm, sc, lanes, local, n, x, y <= half_end ? y : lo, live, &probe_lds[wave]);
+                if (live && speaks) row_sector[y] = (short)s;
+                rows_end = max(rows_end, min(y0 + ROWS, half_end + 1));
+                if (__syncthreads_or(y <= half_end && y > last && (live ? s : (int)row_sector[y]) >= 0)) break;
+            }
+            __syncthreads();
+            for (int y = first + (int)threadIdx.x; y <= last; y += blockDim.x) {
+                if (row_sector[y] != -1 || !gap_pixel(meta[(size_t)y * SW])) continue;
+                int below = -1;
+                for (int j = y + 1; j < rows_end && below < 0; ++j) below = row_sector[j];
+                if (below >= 0 && below != c.sector) {
+                    sector[(size_t)y * SW] = (unsigned short)below;
+                    flags[(size_t)y * SW] = (unsigned char)(1 | 2 | 4 | 8);
                 } else {
-                    atomicMin(&span[half ? 2 : 0], y);
-                    atomicMax(&span[half ? 3 : 1], y);
+                    note_row(sc, local, half, y);
                 }
             }
         }
@@ -1675,23 +1710,22 @@ __device__ __forceinline__ unsigned plane_span_texel(const PlaneSpan &s, int k) 
     return (s.texture_row0 + v) * s.atlas_width + u;   // the atlas is below 4 GiB (checked at create)
 }
 
-// Visplane repair (engine.py:11026-11135) of the row ranges flat_select_kernel noted, one block per lane, one
-// wavefront per 64 columns.  Every pixel of those rows is selected first (the repairs read whole rows and
-// columns).  Vertical: an unresolved pixel takes the sector of the next resolved pixel below it in its half of
-// the screen; rows below the noted range are selected one at a time until every column that still looks for
-// one has found it.  Horizontal: an unresolved pixel between a left and a right anchor of one sector takes
-// that sector.  Pixels outside the noted rows need none of this: no shown pixel there is unresolved, and
-// resolved pixels are never repaired.
-// Every pixel of the noted rows: the blocks take the rows of the work list in turn, so that lanes with many rows
-// and lanes with none load the chip alike.  One block per row at a time, one wavefront per 64 columns.
+// Visplane repair (engine.py:11026-11135) of the noted row ranges.  Every pixel of those rows is selected first (the repairs
+// read whole rows and columns).  Vertical: an unresolved pixel takes the sector of the next resolved pixel below it in its
+// half of the screen; rows below the noted range are selected until every column that still looks for one has found it.
+// Horizontal: an unresolved pixel between a left and a right anchor of one sector takes that sector.  Pixels outside the
+// noted rows need none of this: no shown pixel there is unresolved, and resolved pixels are never repaired.
+// Every pixel of the noted rows: a wavefront takes 64 columns of a row of the work list at a time, so that lanes with many rows
+// and lanes with none load the chip alike.
 template <bool MASKS>
-__global__ void __launch_bounds__(SW) __attribute__((amdgpu_waves_per_eu(8, 8))) flat_span_select_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
-    const int total = *sc.flat_row_count;
-    const int x = threadIdx.x;
-    for (int entry = blockIdx.x; entry < total; entry += gridDim.x) {
-        const int packed = sc.flat_rows[entry];
-        const int local = packed >> 8, y = packed & 255;
-        const int s = flat_select_pixel<MASKS>(dm, sc, lanes, local, lane_base + local, x, y, true);
+__global__ void __launch_bounds__(256) flat_span_select_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
+    __shared__ RowLds row_lds[4];
+    const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63;
+    const int total = *sc.flat_row_count * (SW / 64);
+    for (int task = blockIdx.x * 4 + wave; task < total; task += gridDim.x * 4) {
+        const int entry = task / (SW / 64), x = (task - entry * (SW / 64)) * 64 + lane_id;
+        const int packed = sc.flat_rows[entry], local = packed >> 8, y = packed & 255;
+        const int s = flat_select_row<MASKS>(dm, sc, lanes, local, lane_base + local, x, y, true, &row_lds[wave]);
         const size_t i = (size_t)local * VH * SW + (size_t)y * SW + x;
         sc.flat_sector[i] = (unsigned short)(s < 0 ? sc.ctx[local].sector : s);
         sc.flat_flags[i] = s < 0 ? 1 : 0;
@@ -1699,33 +1733,27 @@ __global__ void __launch_bounds__(SW) __attribute__((amdgpu_waves_per_eu(8, 8)))
 }
 
 // A column whose pixel in the last noted row of a half is unresolved looks further down for a resolved one
-// (engine.py:11026-11083).  One block per (lane, 64-column strip); its tail_rows() wavefronts select that many rows
-// at a time, while any of the strip's columns is still looking.  Eight rows a step suit maps with few plane levels, where
-// a resolved row is usually near; with a level per sector a search runs further and sixteen are quicker.
-constexpr int tail_rows(bool masks) { return masks ? 16 : 8; }
+// (engine.py:11026-11083).  One block per 64 columns of a half with noted rows; its TAIL_ROWS wavefronts select that many rows
+// at a time, while any of the columns is still looking.
+#define TAIL_ROWS 16
 template <bool MASKS>
-__global__ void __launch_bounds__(64 * tail_rows(MASKS)) flat_tail_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
-    constexpr int TAIL_ROWS = tail_rows(MASKS);
+__global__ void __launch_bounds__(64 * TAIL_ROWS) flat_tail_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
+    __shared__ RowLds row_lds[TAIL_ROWS];
     __shared__ int found_lds[TAIL_ROWS][64];
-    const int local = blockIdx.y;
-    if (local >= lane_count) return;
-    const int *span = sc.flat_span + (size_t)local * 4;
-    const int lo[2] = {span[0], span[2]}, hi[2] = {span[1], span[3]};
-    if (hi[0] < lo[0] && hi[1] < lo[1]) return;      // the same in every thread
-    const int n = lane_base + local;
     const int slot = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int x = blockIdx.x * 64 + slot;
-    const int last_ceiling_row = sc.ctx[local].last_ceiling_row;
-    for (int half = 0; half < 2; ++half) {
-        if (hi[half] < lo[half]) continue;           // the same in every thread
-        const int half_end = half ? VH - 1 : last_ceiling_row;
-        bool looking = sc.flat_flags[(size_t)local * VH * SW + (size_t)hi[half] * SW + x] & 1;
+    const int total = *sc.flat_span_count * (SW / 64);
+    for (int task = blockIdx.x; task < total; task += gridDim.x) {
+        const int entry = task / (SW / 64), x = (task - entry * (SW / 64)) * 64 + slot;
+        const int packed = sc.flat_spans[entry], local = packed >> 1, half = packed & 1;
+        const int last = sc.flat_span[(size_t)local * 4 + 2 * half + 1];
+        const int half_end = half ? VH - 1 : sc.ctx[local].last_ceiling_row;
+        bool looking = sc.flat_flags[(size_t)local * VH * SW + (size_t)last * SW + x] & 1;
         int found = -1;
-        for (int y0 = hi[half] + 1; y0 <= half_end; y0 += TAIL_ROWS) {
+        for (int y0 = last + 1; y0 <= half_end; y0 += TAIL_ROWS) {
             if (!__syncthreads_or(looking)) break;   // also keeps the rows of the previous step apart from this one's
             const int y = y0 + wave;
             int s = -1;
-            if (y <= half_end) s = flat_select_pixel<MASKS>(dm, sc, lanes, local, n, x, y, looking);   // the same in a whole wavefront
+            if (y <= half_end) s = flat_select_row<MASKS>(dm, sc, lanes, local, lane_base + local, x, y, looking, &row_lds[wave]);   // the same in a whole wavefront
             found_lds[wave][slot] = s;
             __syncthreads();
             if (looking) {
@@ -1740,85 +1768,79 @@ __global__ void __launch_bounds__(64 * tail_rows(MASKS)) flat_tail_kernel(Device
     }
 }
 
-__global__ void __launch_bounds__(SW) flat_span_finish_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
-    const int local = blockIdx.x;
-    if (local >= lane_count) return;
-    const int *span = sc.flat_span + (size_t)local * 4;
-    const int lo[2] = {span[0], span[2]}, hi[2] = {span[1], span[3]};
-    if (hi[0] < lo[0] && hi[1] < lo[1]) return;      // the same in every thread
-    const LaneCtx c = sc.ctx[local];
-    const int n = lane_base + local;
-    unsigned short *sector = sc.flat_sector + (size_t)local * VH * SW;
-    unsigned char *flags = sc.flat_flags + (size_t)local * VH * SW;
-    const int x = threadIdx.x;
-    const int last_ceiling_row = c.last_ceiling_row;
-    // --- vertical (engine.py:11026-11083): floors and ceilings alike look downwards, within their own half
-    for (int half = 0; half < 2; ++half) {
-        if (hi[half] < lo[half]) continue;           // the same in every thread
-        const int half_end = half ? VH - 1 : last_ceiling_row;
-        // what flat_tail_kernel found below the range for a column whose pixel in the range's last row is unresolved
-        const int below = sc.flat_tail[((size_t)local * 2 + half) * SW + x];
-        bool found = below >= 0;
-        int span_sector = found ? below : 0;
-        // eight rows at a time, their loads first: a column's rows are its own, so no store of the loop touches them
-        for (int y0 = hi[half]; y0 >= lo[half]; y0 -= 8) {
-            unsigned char row_flags[8]; unsigned short row_sector[8];
+// The repairs of one half of a lane's screen, one thread per column, one block per entry of the work list.
+__global__ void __launch_bounds__(SW) flat_span_finish_kernel(Scratch sc) {
+    __shared__ u64 anchors[VH][SW / 64];              // per noted row and 64 columns: the pixels that are anchors
+    const int x = threadIdx.x, wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63;
+    const int total = *sc.flat_span_count;
+    for (int entry = blockIdx.x; entry < total; entry += gridDim.x) {
+        const int packed = sc.flat_spans[entry], local = packed >> 1, half = packed & 1;
+        const int lo = sc.flat_span[(size_t)local * 4 + 2 * half], hi = sc.flat_span[(size_t)local * 4 + 2 * half + 1];
+        const int camera_sector = sc.ctx[local].sector;
+        unsigned short *sector = sc.flat_sector + (size_t)local * VH * SW;
+        unsigned char *flags = sc.flat_flags + (size_t)local * VH * SW;
+        const unsigned int *meta = sc.meta + (size_t)local * VH * SW;
+        __syncthreads();                              // nobody reads the previous entry's anchors any more
+        // --- vertical (engine.py:11026-11083): floors and ceilings alike look downwards, within their own half
+        {
+            // what flat_tail_kernel found below the range for a column whose pixel in the range's last row is unresolved
+            const int below = sc.flat_tail[((size_t)local * 2 + half) * SW + x];
+            bool found = below >= 0;
+            int span_sector = found ? below : 0;
+            // eight rows at a time, their loads first: a column's rows are its own, so no store of the loop touches them
+            for (int y0 = hi; y0 >= lo; y0 -= 8) {
+                unsigned char row_flags[8]; unsigned short row_sector[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int y = y0 - j < lo[half] ? lo[half] : y0 - j;
-                row_flags[j] = flags[(size_t)y * SW + x]; row_sector[j] = sector[(size_t)y * SW + x];
-            }
+                for (int j = 0; j < 8; ++j) {
+                    const int y = y0 - j < lo ? lo : y0 - j;
+                    row_flags[j] = flags[(size_t)y * SW + x]; row_sector[j] = sector[(size_t)y * SW + x];
+                }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int y = y0 - j;
-                if (y < lo[half]) break;
-                const size_t i = (size_t)y * SW + x;
-                if (!(row_flags[j] & 1)) { found = true; span_sector = row_sector[j]; }
-                else if (found) {
-                    sector[i] = (unsigned short)span_sector;
-                    // bit1: vertical span; bit2: its sector differs from the camera's (anchor)
-                    flags[i] = (unsigned char)(1 | 2 | ((span_sector != c.sector) ? 4 : 0));
+                for (int j = 0; j < 8; ++j) {
+                    const int y = y0 - j;
+                    if (y < lo) break;
+                    const size_t i = (size_t)y * SW + x;
+                    const bool resolved = !(row_flags[j] & 1);
+                    if (resolved) { found = true; span_sector = row_sector[j]; }
+                    const bool anchor = resolved || (found && span_sector != camera_sector);
+                    if (!resolved && found) {
+                        sector[i] = (unsigned short)span_sector;
+                        // bit1: vertical span; bit2: its sector differs from the camera's (anchor)
+                        flags[i] = (unsigned char)(1 | 2 | (anchor ? 4 : 0));
+                    }
+                    const u64 row_anchors = __ballot(anchor);
+                    if (lane_id == 0) anchors[y][wave] = row_anchors;
                 }
             }
         }
-    }
-    __syncthreads();
-    // --- horizontal (engine.py:11085-11135): between a left and a right anchor of one sector
-    {
-        const int lane_id = threadIdx.x & 63;
-        const int wave = threadIdx.x >> 6;
-        const int rows0 = hi[0] < lo[0] ? 0 : hi[0] - lo[0] + 1, rows1 = hi[1] < lo[1] ? 0 : hi[1] - lo[1] + 1;
-        for (int r = wave; r < rows0 + rows1; r += SW / 64) {
-            const int y = r < rows0 ? lo[0] + r : lo[1] + (r - rows0);
-            unsigned short *row_sector = sector + (size_t)y * SW;
-            unsigned char *row_flags = flags + (size_t)y * SW;
-            u64 anchors[5];
-            unsigned char f[5];
+        __syncthreads();
+        // --- horizontal (engine.py:11085-11135): a shown pixel between a left and a right anchor of one sector.  (An anchor is
+        // its own on either side; what is not shown needs no repair.)
+        for (int y0 = lo; y0 <= hi; y0 += 8) {
+            unsigned int word[8]; unsigned char row_flags[8];
 #pragma unroll
-            for (int k = 0; k < 5; ++k) f[k] = row_flags[k * 64 + lane_id];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) {
-                bool anchor = !(f[k] & 1) || (f[k] & 4);
-                anchors[k] = __ballot(anchor);
+            for (int j = 0; j < 8; ++j) {
+                const size_t i = (size_t)min(y0 + j, hi) * SW + x;
+                word[j] = meta[i]; row_flags[j] = flags[i];
             }
-            for (int k = 0; k < 5; ++k) {
-                if (!(f[k] & 1)) continue;
-                int col = k * 64 + lane_id;
-                // nearest anchor at or left of col
-                int left = -1;
-                u64 below = anchors[k] & ((lane_id == 63) ? ~0ULL : ((1ULL << (lane_id + 1)) - 1));
-                if (below) left = k * 64 + 63 - __clzll(below);
-                else for (int j = k - 1; j >= 0 && left < 0; --j) if (anchors[j]) left = j * 64 + 63 - __clzll(anchors[j]);
-                int right = SW;
-                u64 above = anchors[k] & ~((1ULL << lane_id) - 1);
-                if (above) right = k * 64 + __ffsll((long long)above) - 1;
-                else for (int j = k + 1; j < 5 && right >= SW; ++j) if (anchors[j]) right = j * 64 + __ffsll((long long)anchors[j]) - 1;
-                if (left >= 0 && right < SW) {
-                    int ls = row_sector[left], rs_ = row_sector[right];
-                    // anchors are never rewritten by this pass, so reading them while other
-                    // lanes write their own unresolved pixels is race free
-                    if (ls == rs_) { row_sector[col] = (unsigned short)ls; row_flags[col] = (unsigned char)(f[k] | 8); }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int y = y0 + j;
+                if (y > hi || !(row_flags[j] & 1) || (row_flags[j] & 4)) continue;
+                if (!gap_pixel(word[j])) continue;
+                int left = -1, right = SW;            // this pixel is no anchor: the nearest ones on either side
+                for (int k = wave; k >= 0 && left < 0; --k) {
+                    const u64 bits = anchors[y][k] & (k == wave ? (1ULL << lane_id) - 1 : ~0ULL);
+                    if (bits) left = k * 64 + 63 - __clzll((long long)bits);
                 }
+                for (int k = wave; k < SW / 64 && right >= SW; ++k) {
+                    const u64 bits = anchors[y][k] & (k == wave ? ~(((1ULL << lane_id) - 1) | (1ULL << lane_id)) : ~0ULL);
+                    if (bits) right = k * 64 + __ffsll((long long)bits) - 1;
+                }
+                if (left < 0 || right >= SW) continue;
+                // anchors are not rewritten here, so reading them while other threads write their own pixels is race free
+                const int left_sector = sector[(size_t)y * SW + left], right_sector = sector[(size_t)y * SW + right];
+                if (left_sector == right_sector) { sector[(size_t)y * SW + x] = (unsigned short)left_sector; flags[(size_t)y * SW + x] = (unsigned char)(row_flags[j] | 8); }
             }
         }
     }
@@ -3405,14 +3427,16 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     // what is left of a window no one-sided drawseg closed shows the flat pass's picture
     if (!window_dirty) zero_rows(pb, gaps, x, st.ceiling_clip <= 0.0f ? 0 : (int)st.ceiling_clip, st.floor_clip >= (float)VH ? VH : (int)st.floor_clip);
     masked_midtexture<DEPTH, SPLIT>(cc, st, pb, colormap_lds);
-    // The view pixels no wall tier, plane or masked texture covers: the flat pass selects them (flat_gap_column_kernel) and
-    // flat_shade_kernel paints them.  More than the list holds: the lane is handled pixel by pixel.
-    for (int y = gaps.lo(), gap_end = gaps.hi(); y < gap_end; ++y) {
-        const unsigned int word = pb.m(y);
-        if ((word & (META_FILLED | META_MASKED)) || ((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) != 0) continue;
-        const int slot = atomicAdd(&sc.flat_list_count[local], 1);
-        if (slot < FLAT_LIST_MAX) sc.flat_list[(size_t)local * FLAT_LIST_MAX + slot] = y * SW + x;
-    }
+    // The columns with view pixels that no wall tier, plane or masked texture covers join the flat pass's work list, those of a
+    // wavefront in one piece (flat_gap_kernel selects the pixels, flat_shade_kernel paints them).
+    bool holds_gap = false;
+    for (int y = gaps.lo(), gap_end = gaps.hi(); y < gap_end && !holds_gap; ++y) holds_gap = gap_pixel(pb.m(y));
+    const u64 holders = __ballot(holds_gap);
+    if (holders == 0) return;
+    int list_base = 0;
+    if (lane_id == 0) list_base = atomicAdd(sc.gap_column_count, __popcll(holders));
+    list_base = __builtin_amdgcn_readfirstlane(list_base);
+    if (holds_gap) sc.gap_columns[list_base + __popcll(holders & ((1ULL << lane_id) - 1))] = make_int2((local << 9) | x, gaps.lo() | (gaps.hi() << 8));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -3586,27 +3610,18 @@ __device__ void flat_shade_pixel(const DeviceMap &dm, const Scratch &sc, const L
 
 // lane_pick: LANES_ALL, or one half of launch_chunk's split: LANES_PLAIN for the lanes whose billboards were painted first and
 // marked the gap pixels they took, LANES_BLENDING for the others, whose billboards come after this.
-__global__ void __launch_bounds__(128) flat_shade_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride, int lane_pick) {
-    const int local = blockIdx.x;
-    if (local >= lane_count) return;
-    if (lane_pick != LANES_ALL && (sc.lane_blends[local] != 0) != (lane_pick == LANES_BLENDING)) return;   // the same in the whole block
+__global__ void __launch_bounds__(64) flat_shade_kernel(DeviceMap dm, Scratch sc, unsigned char *frame_base, size_t frame_stride, int lane_pick) {
     const bool after_billboards = lane_pick == LANES_PLAIN;
-    const int listed = sc.flat_list_count[local];
-    const LaneCtx &c = sc.ctx[local];
-    unsigned char *frame = frame_base + (size_t)local * frame_stride;
-    if (listed <= FLAT_LIST_MAX) {
-        for (int slot = threadIdx.x; slot < listed; slot += blockDim.x) {
-            const int pixel = sc.flat_list[(size_t)local * FLAT_LIST_MAX + slot];
-            if (after_billboards && (sc.meta[(size_t)local * VH * SW + pixel] & META_GAP_COVERED)) continue;
-            flat_shade_pixel(dm, sc, c, local, pixel, frame);
+    const int total = *sc.gap_column_count;
+    for (int entry = blockIdx.x; entry < total; entry += gridDim.x) {
+        const int2 packed = sc.gap_columns[entry];
+        const int local = packed.x >> 9, x = packed.x & 511, last = packed.y >> 8;
+        if (lane_pick != LANES_ALL && (sc.lane_blends[local] != 0) != (lane_pick == LANES_BLENDING)) continue;   // the same in the whole block
+        for (int y = (packed.y & 255) + (int)threadIdx.x; y < last; y += 64) {
+            const unsigned int word = sc.meta[(size_t)local * VH * SW + (size_t)y * SW + x];
+            if (gap_pixel(word) && !(after_billboards && (word & META_GAP_COVERED)))
+                flat_shade_pixel(dm, sc, sc.ctx[local], local, y * SW + x, frame_base + (size_t)local * frame_stride);
         }
-        return;
-    }
-    // a lane with more gap pixels than the list holds: every pixel is looked at
-    for (int pixel = threadIdx.x; pixel < VH * SW; pixel += blockDim.x) {
-        const unsigned int meta = sc.meta[(size_t)local * VH * SW + pixel];
-        if (!(meta & (META_FILLED | META_MASKED)) && ((meta >> META_SECTOR_SHIFT) & META_SECTOR_MASK) == 0 && !(after_billboards && (meta & META_GAP_COVERED)))
-            flat_shade_pixel(dm, sc, c, local, pixel, frame);
     }
 }
 
@@ -4861,13 +4876,12 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.flat_flags, L * PX);
     take(&sc.flat_span, L * 4);
     take(&sc.flat_tail, L * 2 * SW);
+    take(&sc.flat_spans, L * 2);
+    take(&sc.flat_span_count, 1);
     take(&sc.flat_rows, L * (size_t)VH);
     take(&sc.flat_row_count, 1);
-    take(&sc.gap_columns, L * 2 * SW);
+    take(&sc.gap_columns, L * SW);
     take(&sc.gap_column_count, 1);
-    take(&sc.flat_col_top, L * 2 * SW);
-    take(&sc.flat_list, L * FLAT_LIST_MAX);
-    take(&sc.flat_list_count, L);
     sc.pass_slots = h.sector_count < 16 ? 16 : (h.sector_count > PASS_MAX ? PASS_MAX : h.sector_count);
     take(&sc.pass_rec, L * (size_t)sc.pass_slots * SW);
     take(&sc.pass_path_distance, L * (size_t)sc.pass_slots * SW);
@@ -5117,15 +5131,16 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     if (!beside) shade_planes();
     mark();
     // the flat pass, where the walls left it something to decide
-    hipLaunchKernelGGL(flat_gap_column_kernel, dim3(count), dim3(GAP_THREADS), 0, stream, r->dm, *lanes, base, count, sc);
-    hipLaunchKernelGGL(flat_gap_repair_kernel, dim3(GAP_REPAIR_BLOCKS), dim3(64 * GAP_REPAIR_CHUNKS), 0, stream, r->dm, *lanes, base, sc);
-    hipLaunchKernelGGL(flat_rows_kernel, dim3(count), dim3(64), 0, stream, count, sc);
+    // The sizes of its work lists are known on the device only: each kernel's grid follows the lanes, a block takes one entry after another.
+    auto flat_grid = [count](int per_lane, int most) { return dim3((unsigned)(count >= most / per_lane ? most : (count * per_lane < 32 ? 32 : count * per_lane))); };
     const int plane_levels = m.floor_level_count + m.ceil_level_count;
     const bool level_masks = plane_levels > LEVEL_MASK_MIN_LEVELS && plane_levels <= 32 * LEVEL_MASK_WORDS_MAX;   // level_mask_words() > 0
-    hipLaunchKernelGGL(level_masks ? flat_span_select_kernel<true> : flat_span_select_kernel<false>, dim3(SPAN_SELECT_BLOCKS), dim3(SW), 0, stream, r->dm, *lanes, base, count, sc);
+    hipLaunchKernelGGL(flat_gap_kernel, flat_grid(4, 2048), dim3(64 * GAP_WAVES), 0, stream, r->dm, *lanes, base, sc);
+    hipLaunchKernelGGL(flat_rows_kernel, dim3(count), dim3(64), 0, stream, count, sc);
+    hipLaunchKernelGGL(level_masks ? flat_span_select_kernel<true> : flat_span_select_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, sc);
     mark();
-    hipLaunchKernelGGL(level_masks ? flat_tail_kernel<true> : flat_tail_kernel<false>, dim3(SW / 64, count), dim3(64 * tail_rows(level_masks)), 0, stream, r->dm, *lanes, base, count, sc);
-    hipLaunchKernelGGL(flat_span_finish_kernel, dim3(count), dim3(SW), 0, stream, r->dm, *lanes, base, count, sc);
+    hipLaunchKernelGGL(level_masks ? flat_tail_kernel<true> : flat_tail_kernel<false>, flat_grid(4, 1024), dim3(64 * TAIL_ROWS), 0, stream, r->dm, *lanes, base, sc);
+    hipLaunchKernelGGL(flat_span_finish_kernel, flat_grid(2, 1024), dim3(SW), 0, stream, sc);
     // Billboards that simply cover what lies under them need not wait for the flat pass's pixels: the lanes that hold no other
     // kind (lane_blends, decided on the device) have theirs painted right after the shading, on the side stream, where they
     // mark the gap pixels they take; the flat pass's pixels of those lanes are painted after the join, around the marks.  The
@@ -5139,13 +5154,13 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         const size_t shared = (size_t)lanes->sprite_slots * (sizeof(SpriteRec) + sizeof(unsigned short));
         hipLaunchKernelGGL(sprite_columns_kernel, dim3((SW + SPRITE_COLUMNS - 1) / SPRITE_COLUMNS, count), dim3(SPRITE_COLUMNS * SPRITE_ROW_PARTS), shared, on, r->dm, *lanes, base, count, sc, frame_base, frame_stride, lane_pick);
     };
-    if (!fused && !(billboards_split && !may_blend)) hipLaunchKernelGGL(flat_shade_kernel, dim3(count), dim3(128), 0, stream, r->dm, count, sc, frame_base, frame_stride, billboards_split ? LANES_BLENDING : LANES_ALL);
+    if (!fused && !(billboards_split && !may_blend)) hipLaunchKernelGGL(flat_shade_kernel, flat_grid(4, 4096), dim3(64), 0, stream, r->dm, sc, frame_base, frame_stride, billboards_split ? LANES_BLENDING : LANES_ALL);
     if (beside) {
         shade_planes();
         if (billboards_split) paint_billboards(r->side_stream, LANES_PLAIN);
         HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
         HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
-        if (billboards_split) hipLaunchKernelGGL(flat_shade_kernel, dim3(count), dim3(128), 0, stream, r->dm, count, sc, frame_base, frame_stride, LANES_PLAIN);
+        if (billboards_split) hipLaunchKernelGGL(flat_shade_kernel, flat_grid(4, 4096), dim3(64), 0, stream, r->dm, sc, frame_base, frame_stride, LANES_PLAIN);
     }
     mark();
     const float *blend = lanes->screen_blend ? lanes->screen_blend + 2 * (size_t)base : nullptr;
@@ -5296,6 +5311,13 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
         build_level_boxes(h, box_ofs, boxes);
         if (rc == GD_OK) rc = upload(r, box_ofs.data(), box_ofs.size(), &r->dm.level_box_ofs);
         if (rc == GD_OK) rc = upload(r, boxes.data(), boxes.size(), &r->dm.level_boxes);
+        std::vector<float4> around(box_ofs.size() - 1, make_float4(GD_INF, GD_INF, -GD_INF, -GD_INF));   // a level without a sector: no point
+        for (size_t l = 0; l + 1 < box_ofs.size(); ++l)
+            for (int k = box_ofs[l]; k < box_ofs[l + 1]; ++k) {
+                const float4 box = boxes[k];
+                around[l] = make_float4(std::fmin(around[l].x, box.x), std::fmin(around[l].y, box.y), std::fmax(around[l].z, box.z), std::fmax(around[l].w, box.w));
+            }
+        if (rc == GD_OK) rc = upload(r, around.data(), around.size(), &r->dm.level_box);
         std::vector<int> blocking_slot(W, -1);
         for (int b = 0; b < h->blocking_count; ++b) {
             const int w = h->blocking_walls[b];
