@@ -9,6 +9,7 @@
 //                                             nearest blocking hit of every column (64-bit atomicMin)
 //   strip_key/order 1 thread / 64-col strip   longest strip first (counting sort on the blocking distance)
 //   wall_select     1 wave / strip            portal traversal: which drawseg every column pass selects, one record each
+//   wall_geometry   1 block / lane            the linedefs those passes draw, as lines over the columns: every division of the drawing
 //   wall_raster     1 wave / strip            the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
 //   plane_shade     1 thread / 12 pixels      flat texel + light for every pixel a plane of the wall pass shows,
 //                                             the wall tiers' palette indices
@@ -79,7 +80,6 @@ static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and it
 #define CF_LEDGE 4
 #define CF_ALONG_HI 8   // along > 0.5: the ray is nearer the linedef's end vertex
 #define CF_FF 16        // camera on the front side of the linedef (float32 test)
-#define CF_MASKED 32    // candidate entries only: the side facing the camera carries a masked mid-texture
 
 // wall record flags
 #define WF_HC 1        // owns at least one column after every span test
@@ -111,12 +111,52 @@ struct WallRec {   // one linedef seen from one lane
 struct __align__(16) PassRec {
     unsigned short wall, render_current, bits, ps_path;
     short ps_other;
-    unsigned short spare;
+    unsigned short marks;     // REC_*
     float distance;
 };
+#define REC_SIDE1 1       // the pass draws the back side
+#define REC_OWN_ROWS 2    // the pass draws from a sector that is not the one its side faces, or through a BSP fragment: its rows are not
+                          // the linedef's lines but its own (Scratch::pass_rows, written by wall_geometry_kernel)
 #define PASS_MAX 255  // most column passes recorded per screen column (the count is a byte).  A chunk keeps room for as many as the
                       // map has sectors (a column runs at most that many passes), at least 16, at most PASS_MAX: Scratch::pass_slots.
                       // A column that needs more sets STATUS_PASS_OVERFLOW.
+
+// What the drawing half of the traversal asks of a linedef seen from one lane, as straight lines over the screen columns: every
+// division of it (OWallMost's of its four heights, the wallscan light's) depends on the linedef alone, not on the column.
+struct __align__(16) ColumnLine {    // base + x * step
+    i64 base, step;
+    __device__ __forceinline__ i64 at(int x) const { return (i64)((u64)base + (u64)(i64)x * (u64)step); }
+};
+// A height's row is clamp(line >> 16) (engine.py:12294-12605).  A height that the view frustum cuts, or that lies beyond it, bends: it
+// then shows row 0 over the columns [top0, top1) and row 208 over [bottom0, bottom1) (but not at column `collapsed`), and in the
+// columns outside the linedef's own screen span the line `outside`.
+struct HeightBend {
+    unsigned int top;      // top0 | top1 << 10 | (collapsed + 1) << 20
+    unsigned int bottom;   // bottom0 | bottom1 << 10 | bends << 31
+};
+struct __align__(16) WallGeo {
+    ColumnLine line[4];        // front ceiling, front floor, back floor, back ceiling
+    HeightBend bend[4];
+    ColumnLine visibility[2];  // wallscan light of side 0 and 1 (engine.py:11217-11291)
+    int tx0, tx1, ty0, ty1;    // as in WallRec
+    int span0, span1;          // the linedef's screen span within [0, 320] (empty: span0 == span1)
+    int past_left, spare;      // does the span start right of column 0?
+    ColumnLine outside[4];     // of heights that bend
+};
+struct __align__(16) MaskedGeo {   // the same of a linedef's masked mid-texture (engine.py:13424-13744): its upper and lower edge
+    ColumnLine line[2];
+    ColumnLine scale;              // the column's sprite scale
+    ColumnLine outside[2];
+    HeightBend bend[2];
+};
+// What a linedef's side adds that no camera changes
+struct __align__(16) WallSide {
+    int tex[3];              // mid, lower, upper
+    short other, spare;      // the sector behind the side (-1 = none)
+    float offset_y, contrast;// vertical texture offset; +16 on vertical linedefs, -16 on horizontal ones (engine.py:12853-12861)
+    i64 offset_x, repeat;    // 16.16 texture offset and linedef length
+    i64 spare2;
+};
 
 struct RecSpan {   // what a ray test of one linedef needs (eval_segment), kept for every linedef of the map; the full record
                    // above exists only for the linedefs the camera can see at all
@@ -168,6 +208,9 @@ struct DeviceMap {  // device copy of gd_map_desc (device pointers) + fixed tabl
     const int4 *cell_item;               // [items] sector | GRID_ALWAYS_INSIDE, floor level index | ceiling level
                                          // index << 8 (or -1 when not recorded), first edge, one past the last
     const float4 *cell_edge;             // [item edges] x1, y1, x2, y2
+    const WallSide *wall_side;           // [W,2]
+    const int *masked_slot;              // [W] number of the linedef among those with a mid-texture on a two-sided side, else -1
+    int masked_count;                    // how many there are
     const int *wall_blocking_slot;       // [W] position of the linedef in blocking_walls, -1 when it does not block
     const unsigned int *sector_level;    // [S] index of the floor in floor_levels | index of the ceiling in ceil_levels << 16;
                                          // null when some sector's height is missing from the level lists
@@ -181,6 +224,16 @@ struct Scratch {    // per-chunk working memory, sized at create
     LaneCtx *ctx;          // [L]
     WallRec *rec;          // [L,W] written for the linedefs wall_setup_kernel does not cull; never read for the others
     RecSpan *span;         // [L,W] every linedef
+    WallGeo *geo;          // [L*W] the linedefs some column pass draws, those of a lane in a run of their own (wall_geometry_kernel)
+    int *geo_count;        // [1] how many there are (cleared by lane_setup_kernel)
+    unsigned int *geo_slot;// [L,W] where in geo (written for those linedefs only)
+    unsigned int *named;   // [L,(W+31)/32] a bit per linedef some column pass draws (cleared by lane_tables_kernel, set by wall_select_kernel)
+    unsigned int *own_rows;// [L] bit k: strip k holds a pass with REC_OWN_ROWS (the same)
+    int lane_stride;       // lanes of the chunk's planes
+    MaskedGeo *masked_geo; // [L,masked_count] those whose masked mid-texture is some column's nearest
+    u64 *masked_hit;       // [L,320] cand_key of the nearest candidate with a masked mid-texture on the side facing the camera and a
+                           // projection that owns the column, CAND_KEY_NONE if none (engine.py:13436-13460)
+    uint2 *pass_rows;      // [pass_slots,L,320] the eight projected rows of a pass whose record carries REC_OWN_ROWS (written for those only)
     WallRec *frag_rec;     // [L,split_count,fragment_slots] FWallCoords of the BSP fragments of split linedefs
     float *scene_depth;    // [L,208,320] depth of the surface each pixel shows (engine.py:11553, 12700, 13411, 13740),
                            // kept only for frames that draw wall decals, else null
@@ -207,11 +260,13 @@ struct Scratch {    // per-chunk working memory, sized at create
     int *flat_rows;        // [L*208] the noted rows of every lane as one work list, entry = lane << 8 | row
     int *flat_row_count;   // [1] its length (cleared by lane_setup_kernel, filled by flat_rows_kernel)
     int pass_slots;        // passes a column can record in this chunk
-    PassRec *pass_rec;     // [L,pass_slots,320] the drawsegs of each column's passes, in pass order
-    float *pass_path_distance;  // [L,pass_slots,320] distance of the portal path of a pass that carries PB_PS_KEEPS (written for those only)
+    // where pass `pass` of a column lies in the three planes below: the passes that most columns make lie close together
+    __device__ __forceinline__ size_t pass_at(int pass, int local, int x) const { return ((size_t)pass * (size_t)lane_stride + (size_t)local) * SW + (size_t)x; }
+    PassRec *pass_rec;     // [pass_slots,L,320] the drawsegs of each column's passes, in pass order
+    float *pass_path_distance;  // [pass_slots,L,320] distance of the portal path of a pass that carries PB_PS_KEEPS (written for those only)
     unsigned char *pass_count;  // [L,320] passes recorded for the column: up to its last pass that draws or moves a clip
     unsigned int *meta;    // [L,208,320] filled | floor | plane_sector+1 | clip_wall+1
-    float *clip_depth;     // [L,208,320]
+    unsigned char *masked_texel; // [L,208,320] palette indices of masked mid-textures, where no frame takes them (band_finish_kernel)
     unsigned char *frame;  // [L,240,320] when the caller wants no indexed output
     u64 *block_hit;        // [L,320] nearest blocking linedef of the column ray: float bits of the distance << 32 |
                            // slot in blocking_walls, all ones when no ray hits (engine.py:10534-10557)
@@ -252,6 +307,7 @@ __device__ __forceinline__ bool gap_pixel(unsigned int word) { return !(word & (
 
 #define STATUS_CAND_OVERFLOW 1
 #define STATUS_PASS_OVERFLOW 2
+__device__ __forceinline__ int named_words(const gd_map_desc *m) { return (m->wall_count + 31) / 32; }
 #define STEP_TABLE 96   // int64 entries per lane of Scratch::step_scale
 
 __device__ __forceinline__ i64 mul64(i64 a, i64 b) { return (i64)((u64)a * (u64)b); }
@@ -502,7 +558,9 @@ __global__ void lane_tables_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_b
     if (local >= lane_count) return;
     const LaneCtx &c = sc.ctx[local];
     // the lane's per-column lists start empty
-    for (int x = threadIdx.x; x < SW; x += blockDim.x) { sc.cand_count[(size_t)local * SW + x] = 0; sc.block_hit[(size_t)local * SW + x] = ~0ULL; }
+    for (int x = threadIdx.x; x < SW; x += blockDim.x) { sc.cand_count[(size_t)local * SW + x] = 0; sc.block_hit[(size_t)local * SW + x] = ~0ULL; sc.masked_hit[(size_t)local * SW + x] = CAND_KEY_NONE; }
+    for (int k = threadIdx.x; k < named_words(&dm.d); k += blockDim.x) sc.named[(size_t)local * named_words(&dm.d) + k] = 0u;
+    if (threadIdx.x == 0) sc.own_rows[local] = 0u;
     {   // does a live billboard of the lane blend with what lies under it?
         bool blends = false;
         if (lanes.sprite_style && lanes.sprite_alive)
@@ -606,7 +664,7 @@ __global__ void lane_setup_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_ba
     sc.ctx[local] = c;
     int *span = sc.flat_span + (size_t)local * 4;
     span[0] = VH; span[1] = -1; span[2] = VH; span[3] = -1;
-    if (local == 0) { *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
+    if (local == 0) { *sc.geo_count = 0; *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
 }
 
 __device__ __forceinline__ void ray_direction(const LaneCtx &c, int x, float *rx, float *ry) {
@@ -916,6 +974,9 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
     const int rec_pl = r.pl, rec_pr = r.pr;
     // Most linedefs cover a few columns only, so several of them share a turn: eight with eight lanes each, then
     // four with sixteen, then two with thirty-two; a wider one has the wavefront to itself.
+    auto note_masked = [&](int wall, int x, const Eval &e) {
+        atomicMin(&sc.masked_hit[(size_t)local * SW + x], ((u64)__float_as_uint(e.dist) << 32) | ((u64)wall << 16) | (u64)e.flags);
+    };
     const bool listed = a_lo < a_hi;
     const bool narrow = listed && (a_hi - a_lo <= 32);
     auto shared_turns = [&](bool member, int lanes_each) {
@@ -942,13 +1003,14 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
             float rx, ry; ray_direction(c, x, &rx, &ry);
             const Eval e = eval_segment(b_wl, b_span & 0xFF, b_pl, b_pr, (b_span & 0x100) != 0, c, x, rx, ry);
             if (!finitef(e.dist)) continue;
+            if ((b_span & 0x200) && (e.flags & CF_PROJ)) note_masked(b_wall, x, e);
             const int slot = atomicAdd(&counts[x], 1);
             if (slot < CAND_MAX) {
                 Cand entry;
                 entry.wall = (unsigned short)b_wall;
                 entry.s0 = (short)(b_sectors & 0xFFFF); entry.s1 = (short)(b_sectors >> 16);
                 entry.v0 = (unsigned short)(b_vertices & 0xFFFF); entry.v1 = (unsigned short)((unsigned)b_vertices >> 16);
-                entry.flags = (unsigned short)(e.flags | ((b_span & 0x200) ? CF_MASKED : 0));
+                entry.flags = (unsigned short)e.flags;
                 entry.dist = e.dist;
                 list[(size_t)slot * SW + x] = entry;
             }   // else: the count says so, and the column is listed afresh in the spill pool (strip_key_kernel, cand_spill_kernel)
@@ -972,9 +1034,10 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
             float rx, ry; ray_direction(c, x, &rx, &ry);
             Eval e = eval_segment(b_wl, b_span & 0xFF, b_pl, b_pr, (b_span & 0x100) != 0, c, x, rx, ry);
             if (finitef(e.dist)) {
+                if ((b_span & 0x200) && (e.flags & CF_PROJ)) note_masked(entry.wall, x, e);
                 int slot = atomicAdd(&counts[x], 1);
                 if (slot < CAND_MAX) {
-                    entry.flags = (unsigned short)(e.flags | ((b_span & 0x200) ? CF_MASKED : 0));
+                    entry.flags = (unsigned short)e.flags;
                     entry.dist = e.dist;
                     list[(size_t)slot * SW + x] = entry;
                 }
@@ -1009,12 +1072,10 @@ __global__ void __launch_bounds__(64) cand_spill_kernel(DeviceMap dm, Scratch sc
                 const Eval e = eval_wall(m, c, spans, x, w, rx, ry);
                 keep = finitef(e.dist);
                 const int s1 = m->wall_sectors[2 * w + 1];
-                const bool front_facing = (spans[w].flags & WF_FF) != 0;
-                const bool masked_side = s1 >= 0 && m->side_tex[(w * 2 + (front_facing ? 0 : 1)) * 3] >= 0;
                 entry.wall = (unsigned short)w;
                 entry.s0 = (short)m->wall_sectors[2 * w]; entry.s1 = (short)s1;
                 entry.v0 = (unsigned short)m->wall_vertex[2 * w]; entry.v1 = (unsigned short)m->wall_vertex[2 * w + 1];
-                entry.flags = (unsigned short)(e.flags | (masked_side ? CF_MASKED : 0));
+                entry.flags = (unsigned short)e.flags;
                 entry.dist = e.dist;
             }
             const u64 keeps = __ballot(keep);
@@ -1547,17 +1608,18 @@ struct Tables {
     const unsigned char *tex_bits; // floor(log2 width) | floor(log2 height) << 4
     const unsigned int *tex_odd;   // bit t: the width of texture t is no power of two
     int sector_cached, tex_cached;
-    __device__ __forceinline__ float floor_h(int s) const { return s < sector_cached ? sector[s].x : m->sector_heights[2 * s]; }
-    __device__ __forceinline__ float ceil_h(int s) const { return s < sector_cached ? sector[s].y : m->sector_heights[2 * s + 1]; }
-    __device__ __forceinline__ float light(int s) const { return s < sector_cached ? sector[s].z : m->sector_lights[s]; }
-    __device__ __forceinline__ int floor_tex(int s) const { return s < sector_cached ? (int)(__float_as_uint(sector[s].w) & 0xFFFFu) : m->sector_floor_tex[s]; }
-    __device__ __forceinline__ int ceil_tex(int s) const { return s < sector_cached ? (int)(__float_as_uint(sector[s].w) >> 16) : m->sector_ceil_tex[s]; }
-    __device__ __forceinline__ int width_bits(int t) const { return t < tex_cached ? (tex_bits[t] & 15) : ilog2(m->tex_w[t]); }
-    __device__ __forceinline__ int height_bits(int t) const { return t < tex_cached ? (tex_bits[t] >> 4) : ilog2(m->tex_h[t]); }
+    bool all_cached = false;       // a kernel's constant: every sector and texture of the map is staged
+    __device__ __forceinline__ float floor_h(int s) const { return all_cached || s < sector_cached ? sector[s].x : m->sector_heights[2 * s]; }
+    __device__ __forceinline__ float ceil_h(int s) const { return all_cached || s < sector_cached ? sector[s].y : m->sector_heights[2 * s + 1]; }
+    __device__ __forceinline__ float light(int s) const { return all_cached || s < sector_cached ? sector[s].z : m->sector_lights[s]; }
+    __device__ __forceinline__ int floor_tex(int s) const { return all_cached || s < sector_cached ? (int)(__float_as_uint(sector[s].w) & 0xFFFFu) : m->sector_floor_tex[s]; }
+    __device__ __forceinline__ int ceil_tex(int s) const { return all_cached || s < sector_cached ? (int)(__float_as_uint(sector[s].w) >> 16) : m->sector_ceil_tex[s]; }
+    __device__ __forceinline__ int width_bits(int t) const { return all_cached || t < tex_cached ? (tex_bits[t] & 15) : ilog2(m->tex_w[t]); }
+    __device__ __forceinline__ int height_bits(int t) const { return all_cached || t < tex_cached ? (tex_bits[t] >> 4) : ilog2(m->tex_h[t]); }
     // Texture column of a wall: torch.remainder(u, width) (engine.py:12792-12798).  Widths are powers of two
     // on most maps, where the remainder is a mask; WAD textures of other widths take the division.
     __device__ __forceinline__ i64 wrap_column(int t, i64 u) const {
-        const bool odd = t < tex_cached ? ((tex_odd[t >> 5] >> (t & 31)) & 1u) != 0 : (m->tex_w[t] & (m->tex_w[t] - 1)) != 0;
+        const bool odd = all_cached || t < tex_cached ? ((tex_odd[t >> 5] >> (t & 31)) & 1u) != 0 : (m->tex_w[t] & (m->tex_w[t] - 1)) != 0;
         if (!odd) return u & (i64)((1 << width_bits(t)) - 1);
         const i64 width = m->tex_w[t];
         const i64 r = u - tdiv(u, width) * width;
@@ -1969,9 +2031,11 @@ __device__ i64 wall_visibility(const WallRec &r, int side, int x) {
 }
 
 // engine.py:10672-10739 (PrepWall) for one (linedef, column)
-__device__ void texture_mapping(const gd_map_desc *m, const WallRec &r, int w, int x, i64 *hoff, i64 *vstep) {
+// `ends`: anything with the linedef's view-space endpoints (WallRec, WallGeo)
+template <typename Ends>
+__device__ __forceinline__ void texture_mapping(const Ends &ends, i64 linedef_repeat, int x, i64 *hoff, i64 *vstep) {
     const float wall_map_scale = (float)((320 * 200.0 / 320.0 / 240) * 64.0 / (320 / 2.0));
-    i64 tx1 = r.tx0, tx2 = r.tx1, ty1 = r.ty0, ty2 = r.ty1;
+    i64 tx1 = ends.tx0, tx2 = ends.tx1, ty1 = ends.ty0, ty2 = ends.ty1;
     double u_over_z_origin = (double)((float)tx1 * 160.0f);
     float u_over_z_step_f = -(float)ty1;
     double u_over_z_step = (double)u_over_z_step_f;
@@ -1980,7 +2044,7 @@ __device__ void texture_mapping(const gd_map_desc *m, const WallRec &r, int w, i
     double inv_z_step = (double)inv_z_step_float;
     double depth_scale = (double)(inv_z_step_float * wall_map_scale);
     double depth_origin = (double)(-u_over_z_step_f * wall_map_scale);
-    double repeat = (double)round_to_i64(m->wall_len[w] * 65536.0f);
+    double repeat = (double)linedef_repeat;
     double column = (double)x - 160.0;
     double top = u_over_z_origin + u_over_z_step * column;
     double bottom = inv_z_origin + inv_z_step * column;
@@ -2136,11 +2200,10 @@ struct PassColumn {
     int side_tex[3];
     int ps_path_index, ps_other, no_path_other, sel_vertex, fb_idx;
     float ps_path_distance, no_path_distance;
-    int bits;
+    int bits, marks;       // PB_*, REC_*
     // what the drawing half adds (pass_geometry, pass_clip)
     int render_other;       // the sector behind the drawn side, -1 for none
     float one_top, one_bottom, lower_top, upper_bottom;              // the four heights' projected rows, not yet clipped
-    float path_top, path_bottom, path_lower_top, path_upper_bottom;  // the same of the portal path of a PB_PS_KEEPS pass
     i64 u_base, swall;      // texture column before wrapping, texture step (engine.py:12762-12807)
     float offset_y;         // the side's vertical texture offset
     float fake_contrast;    // +16 on vertical linedefs, -16 on horizontal ones (engine.py:12853-12861)
@@ -2167,75 +2230,88 @@ __device__ __forceinline__ void take_min(float v, int w, float &best, int &best_
     if (v < best || (v == best && w < best_w && finitef(v))) { best = v; best_w = w; }
 }
 
-// engine.py:12240-12620, 12762-12861, 12969-13010: what one column draws of the drawseg a pass selected, as far as it
-// depends on the selection alone (r.wall, r.render_current, r.ps_path_index, r.ps_other, PB_RASTER / PB_ONE_SIDED /
-// PB_PS_KEEPS / PB_PS_FROM_FRONT in r.bits) and not on the column's clips: the side and sectors drawn from, the wallscan
-// light, the four heights' projected rows, the texture column and step, and the projected rows of a portal path behind a
-// projected solid.  Every division of the drawing half is in here.
-template <bool SPLIT>
-__device__ __forceinline__ void pass_geometry(const ColumnCtx &cc, PassColumn &r) {
-    const gd_map_desc *m = cc.m;
-    const MapView &mv = cc.mv;
-    const LaneCtx &L = *cc.c;
-    const int x = cc.x, wi = r.wall, render_current = r.render_current;
-    const bool one_sided = r.bits & PB_ONE_SIDED;
-    // h. sides (engine.py:12240-12292)
-    const int front = mv.sec(wi, 0), back = mv.sec(wi, 1);
-    const bool render_from_front = render_current == front;
-    const int render_other = render_from_front ? back : front;
-    const int side = render_from_front ? 0 : 1;
-    const int safe_other = render_other < 0 ? 0 : render_other;
-    r.side = side; r.render_other = render_other;
-    const WallRec &wr = cc.rec(wi);
-    const FragmentChoice wr_fragment = choose_fragment<SPLIT>(m, cc.frags, wr, wi, x);
-    r.visibility = wall_visibility(wr_fragment.lights ? *wr_fragment.rec : wr, side, x);
-    const float view_floor = m->sector_heights[2 * render_current], view_ceiling = m->sector_heights[2 * render_current + 1];
-    const float other_floor = m->sector_heights[2 * safe_other], other_ceiling = m->sector_heights[2 * safe_other + 1];
-    for (int t = 0; t < 3; ++t) r.side_tex[t] = m->side_tex[(wi * 2 + side) * 3 + t];
-    // j. projection (engine.py:12607-12620): one copy of the projection code, four heights; the back sector's two only
-    // matter across a two-sided linedef (every use of them is behind !one_sided)
-    r.one_top = 0; r.one_bottom = 0; r.lower_top = 0; r.upper_bottom = 0;
-    const int heights = one_sided ? 2 : 4;
-#pragma unroll 1
-    for (int k = 0; k < heights; ++k) {
-        float z = k == 0 ? view_ceiling : (k == 1 ? view_floor : (k == 2 ? other_floor : other_ceiling));
-        float v = project(L, wr, wr_fragment, z, x);
-        if (k == 0) r.one_top = v; else if (k == 1) r.one_bottom = v; else if (k == 2) r.lower_top = v; else r.upper_bottom = v;
+__device__ __forceinline__ float height_row(const ColumnLine &line, int x) { return (float)(int)clampi(line.at(x) >> 16, 0, VH); }
+__device__ __forceinline__ float bent_row(float row, const HeightBend &b, int x) {
+    const int top0 = b.top & 1023u, top1 = (b.top >> 10) & 1023u, collapsed = (int)(b.top >> 20) - 1;
+    const int bottom0 = b.bottom & 1023u, bottom1 = (b.bottom >> 10) & 1023u;
+    if (x >= bottom0 && x < bottom1 && x != collapsed) row = (float)VH;
+    if (x >= top0 && x < top1 && x != collapsed) row = 0.0f;
+    return row;
+}
+__device__ __forceinline__ bool bends(const HeightBend &b) { return (b.bottom >> 31) != 0; }
+
+// The rows of a linedef's four heights at column x: ceiling and floor of the sector its front (`back`: its back) side faces, floor
+// and ceiling of the other one.  Nothing here waits for a load before the next is asked for, except in columns
+// outside the span of a linedef with a height that bends, which are few.
+struct WallRows { float ceiling, floor, other_floor, other_ceiling; };
+__device__ __forceinline__ WallRows wall_rows(const WallGeo &geo, bool back, int x) {
+    const int first = back ? 3 : 0, next = back ? -1 : 1;
+    const ColumnLine l0 = geo.line[first], l1 = geo.line[first + next], l2 = geo.line[first + 2 * next], l3 = geo.line[first + 3 * next];
+    const HeightBend b0 = geo.bend[first], b1 = geo.bend[first + next], b2 = geo.bend[first + 2 * next], b3 = geo.bend[first + 3 * next];
+    const int span0 = geo.span0, span1 = geo.span1;
+    WallRows r;
+    r.ceiling = bent_row(height_row(l0, x), b0, x); r.floor = bent_row(height_row(l1, x), b1, x);
+    r.other_floor = bent_row(height_row(l2, x), b2, x); r.other_ceiling = bent_row(height_row(l3, x), b3, x);
+    if ((x < span0 || x >= span1) && ((b0.bottom | b1.bottom | b2.bottom | b3.bottom) >> 31)) {
+        if (bends(b0)) r.ceiling = height_row(geo.outside[first], x);
+        if (bends(b1)) r.floor = height_row(geo.outside[first + next], x);
+        if (bends(b2)) r.other_floor = height_row(geo.outside[first + 2 * next], x);
+        if (bends(b3)) r.other_ceiling = height_row(geo.outside[first + 3 * next], x);
     }
-    // texture column and step (engine.py:12762-12807), fake contrast (engine.py:12853-12861): only tiers use them
-    r.u_base = 0; r.swall = 0; r.offset_y = 0.0f; r.fake_contrast = 0.0f;
-    if (r.bits & PB_RASTER) {
-        const float *toff = m->side_off + (wi * 2 + side) * 2;
-        i64 h, swall;
-        texture_mapping(m, wr, wi, x, &h, &swall);
-        i64 repeat = round_to_i64(m->wall_len[wi] * 65536.0f);
-        if (side != 0) h = repeat - h;
-        if (wr.sl > 0 && h < 0) h = 0;
-        if (h >= repeat) h = repeat - 1;
-        i64 offx_fixed = round_to_i64(toff[0] * 65536.0f);
-        r.u_base = (h + offx_fixed) >> 16;
-        r.swall = swall;
-        r.offset_y = toff[1];
-        const float4 wl = *reinterpret_cast<const float4 *>(m->walls + 4 * wi);
-        bool horizontal = fabsf(wl.w - wl.y) < 1e-6f, vertical = fabsf(wl.z - wl.x) < 1e-6f;
-        r.fake_contrast = vertical ? 16.0f : (horizontal ? -16.0f : 0.0f);
+    return r;
+}
+
+// engine.py:10672-10739 (PrepWall) and 12762-12807: texture column before wrapping, texture step
+template <typename Ends>
+__device__ __forceinline__ void texture_column(const Ends &ends, bool past_left, const WallSide &ws, int side, int x, i64 *u_base, i64 *swall) {
+    i64 h;
+    texture_mapping(ends, ws.repeat, x, &h, swall);
+    if (side != 0) h = ws.repeat - h;
+    if (past_left && h < 0) h = 0;
+    if (h >= ws.repeat) h = ws.repeat - 1;
+    *u_base = (h + ws.offset_x) >> 16;
+}
+
+// engine.py:12240-12620, 12969-13010: what one column draws of the drawseg a pass selected, as far as it depends on the selection alone
+// and not on the column's clips: the side and sectors drawn from, the wallscan light, the four heights' projected rows, and
+// those of a portal path behind a projected solid.  All of it is read off the lines wall_geometry_kernel left for the linedef
+// (a pass marked REC_OWN_ROWS has its rows in Scratch::pass_rows); `at` is the record's place in the chunk's planes.
+struct WallEnds { int tx0, tx1, ty0, ty1; };
+struct PassTexture { WallEnds ends; bool past_left; WallSide side; };   // what the texture columns of the pass's tiers come from
+template <bool GENERAL>
+__device__ __forceinline__ void pass_geometry(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, const WallGeo &geo, size_t at, int marks, PassColumn &r, PassTexture &texture) {
+    const int x = cc.x, wi = r.wall, side = (marks & REC_SIDE1) ? 1 : 0;
+    texture.side = dm.wall_side[2 * wi + side];
+    texture.ends.tx0 = geo.tx0; texture.ends.tx1 = geo.tx1; texture.ends.ty0 = geo.ty0; texture.ends.ty1 = geo.ty1;
+    texture.past_left = geo.past_left != 0;
+    const ColumnLine visibility = geo.visibility[side];
+    const WallRows rows = wall_rows(geo, side != 0, x);
+    r.side = side; r.render_other = texture.side.other;
+    r.side_tex[0] = texture.side.tex[0]; r.side_tex[1] = texture.side.tex[1]; r.side_tex[2] = texture.side.tex[2];
+    r.visibility = visibility.at(x);
+    if (GENERAL) {   // wallscan light interpolates over the fragment where a linedef has several
+        const WallRec &wr = cc.rec(wi);
+        const FragmentChoice fragment = choose_fragment<true>(cc.m, cc.frags, wr, wi, x);
+        if (fragment.lights) r.visibility = wall_visibility(*fragment.rec, side, x);
     }
-    // the portal path behind a projected solid (engine.py:12969-13010): the view sector's two heights and the path's other
-    // sector's two, projected through the path linedef
-    r.path_top = 0; r.path_bottom = 0; r.path_lower_top = 0; r.path_upper_bottom = 0;
-    if (r.bits & PB_PS_KEEPS) {
-        const int path = r.ps_path_index;
-        const WallRec &pr = cc.rec(path);
-        const FragmentChoice pr_fragment = choose_fragment<SPLIT>(m, cc.frags, pr, path, x);
-        const int path_safe_other = r.ps_other < 0 ? 0 : r.ps_other;
-        const float pof = m->sector_heights[2 * path_safe_other], poc = m->sector_heights[2 * path_safe_other + 1];
-#pragma unroll 1
-        for (int k = 0; k < 4; ++k) {
-            float z = k == 0 ? view_ceiling : (k == 1 ? view_floor : (k == 2 ? pof : poc));
-            float v = project(L, pr, pr_fragment, z, x);
-            if (k == 0) r.path_top = v; else if (k == 1) r.path_bottom = v; else if (k == 2) r.path_lower_top = v; else r.path_upper_bottom = v;
-        }
+    r.one_top = rows.ceiling; r.one_bottom = rows.floor;
+    // the sector behind only matters across a two-sided linedef (every use of its heights is behind !one_sided)
+    r.lower_top = rows.other_floor; r.upper_bottom = rows.other_ceiling;
+    if (marks & REC_OWN_ROWS) {
+        const unsigned int own = sc.pass_rows[at].x;
+        r.one_top = (float)(own & 255u); r.one_bottom = (float)((own >> 8) & 255u);
+        r.lower_top = (float)((own >> 16) & 255u); r.upper_bottom = (float)(own >> 24);
     }
+}
+
+// The rows of the portal path behind a projected solid (PB_PS_KEEPS, one pass in a thousand).
+__device__ __forceinline__ WallRows path_rows(const ColumnCtx &cc, const Scratch &sc, size_t at, int marks, const PassColumn &r) {
+    if (!(marks & REC_OWN_ROWS)) return wall_rows(sc.geo[sc.geo_slot[cc.rec_base + (unsigned)r.ps_path_index]], !(r.bits & PB_PS_FROM_FRONT), cc.x);
+    const unsigned int own = sc.pass_rows[at].y;
+    WallRows rows;
+    rows.ceiling = (float)(own & 255u); rows.floor = (float)((own >> 8) & 255u);
+    rows.other_floor = (float)((own >> 16) & 255u); rows.other_ceiling = (float)(own >> 24);
+    return rows;
 }
 
 // engine.py:12607-12636: the projected rows of pass_geometry against the column's clips, the plane marks and the tiers.
@@ -2445,6 +2521,12 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
     bool ps_keeps = has_ps && ps_path_geo && (ps_other >= 0);
     bool one_sided = other_sector < 0;
 
+    // Can the rows of the pass be read off its linedefs' lines (WallGeo)?  Not through BSP fragments, and only where the sector
+    // drawn from is the one its side (and its portal path's side) faces.
+    bool own_rows = render_current != (render_from_front ? front : back) || (!one_sided && back < 0) ||
+                    (ps_keeps && render_current != (ps_from_front ? cs : mv.sec(ps_path_index, 1)));
+    if (SPLIT) own_rows = own_rows || m->wall_split_slot[wi] >= 0 || (ps_keeps && m->wall_split_slot[ps_path_index] >= 0);
+    r.marks = (side ? REC_SIDE1 : 0) | (own_rows ? REC_OWN_ROWS : 0);
     r.wall = wi; r.side = side; r.render_current = render_current; r.other_sector = other_sector;
     r.distance = distance;
     r.ps_path_index = ps_path_index; r.ps_other = ps_other; r.no_path_other = no_path_other; r.sel_vertex = sel_vertex; r.fb_idx = fb_idx;
@@ -2458,15 +2540,26 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
 // The per-pixel planes of a chunk of lanes and one column's place in them.  The wavefronts of the traversal hold columns of
 // several lanes, so the planes' base pointers are the same for all of them and each column keeps byte offsets: a chunk
 // is at most 4096 lanes, which keeps every offset below 4 GiB.
+//
+// The runs of rows are stored through buffer descriptors (put): a column that has nothing to store in a row the wavefront walks stores
+// beyond the descriptor's end, which the hardware drops.  With a branch around the store instead, the compiler no longer knows how
+// many stores are under way, so that the next use of a loaded texel waits for all of them to reach memory: every row
+// waited for the row before (wall_raster_kernel, 4096 lanes on the 4000-linedef map: 69 % of its wavefront cycles).
+#define BUFFER_WORDS 0x00027000   // descriptor word 3: 32-bit elements
+#define BUFFER_NOWHERE 0x80000000u   // an offset beyond every plane: 4096 lanes are 1.1 GB
 struct PixelBuffers {
     unsigned char *frame;   // [L][240][320] or null
     unsigned int *meta;     // [L][208][320]
-    float *clip_depth;      // [L][208][320], only meaningful where the meta word names a clip linedef
+    unsigned char *masked_texel;   // [L][208][320], used where there is no frame
     float *scene_depth;     // [L][208][320] or null
+    __amdgpu_buffer_rsrc_t words, depths;   // meta and scene_depth once more, as buffers: see put()
     unsigned word_column;   // byte offset of (lane, row 0, column) in the four-byte planes
     unsigned frame_column;  // and in the frame
     __device__ __forceinline__ unsigned int &m(int y) const { return *reinterpret_cast<unsigned int *>(reinterpret_cast<char *>(meta) + (word_column + (unsigned)y * (SW * 4u))); }
-    __device__ __forceinline__ float &d(int y) const { return *reinterpret_cast<float *>(reinterpret_cast<char *>(clip_depth) + (word_column + (unsigned)y * (SW * 4u))); }
+    // `y` is the same in the whole wavefront
+    __device__ __forceinline__ void put(bool active, int y, unsigned int word) const { __builtin_amdgcn_raw_buffer_store_b32(word, words, active ? word_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
+    __device__ __forceinline__ void put_depth(bool active, int y, float depth) const { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(depth), depths, active ? word_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
+    __device__ __forceinline__ unsigned char &t(int y) const { return masked_texel[(word_column >> 2) + (unsigned)y * (unsigned)SW]; }
     __device__ __forceinline__ float &s(int y) const { return *reinterpret_cast<float *>(reinterpret_cast<char *>(scene_depth) + (word_column + (unsigned)y * (SW * 4u))); }
     __device__ __forceinline__ unsigned char &f(int y) const { return frame[frame_column + (unsigned)y * (unsigned)SW]; }
 };
@@ -2479,50 +2572,48 @@ struct SilhouetteBounds {
     float bot_depth, top_depth;
 };
 
+// The ray distance of a linedef at this column: what the sprite clip of a row whose word names the linedef is at.  (Every clip is
+// recorded with the distance the ray test of that linedef gives at that column, eval_segment's, so the word need not carry it.)
+__device__ __forceinline__ float clip_distance(const ColumnCtx &cc, int w) {
+    const float4 wl = *reinterpret_cast<const float4 *>(cc.m->walls + 4 * w);
+    const float segx = wl.z - wl.x, segy = wl.w - wl.y, offx = wl.x - cc.c->x, offy = wl.y - cc.c->y;
+    return (offx * segy - offy * segx) / (cc.rx * segy - cc.ry * segx);
+}
+
 // Rows [first, last) of one column take `distance` / `wall` as their sprite clip where it is nearer
 // than what they hold.  WALL_ROWS rows at a time, loads first, so the rows' memory latencies overlap.
-__device__ __forceinline__ void clip_rows(PixelBuffers &pb, int x, int first, int last, float distance, int wall) {
-    // one batch ahead: the next rows are asked for before this batch's stores (the rows of two batches are distinct)
-    auto load_rows = [&](int y0, float (&held)[WALL_ROWS], unsigned int (&meta)[WALL_ROWS]) {
-#pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) {
-            const int y = y0 + j < last ? y0 + j : last - 1;
-            held[j] = pb.d(y); meta[j] = pb.m(y);
-        }
-    };
-    float held[WALL_ROWS]; unsigned int meta[WALL_ROWS];
-    if (first < last) load_rows(first, held, meta);
+__device__ __forceinline__ void clip_rows(const ColumnCtx &cc, PixelBuffers &pb, int first, int last, float distance, int wall) {
+    unsigned int held_wall = 0;           // linedef + 1 of the row before and its distance: rows of one clip are neighbours
+    float held = GD_INF;                  // no clip recorded yet: infinite
     for (int y0 = first; y0 < last; y0 += WALL_ROWS) {
-        float next_held[WALL_ROWS]; unsigned int next_meta[WALL_ROWS];
+        unsigned int meta[WALL_ROWS];
 #pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) { next_held[j] = 0.0f; next_meta[j] = 0u; }
-        if (y0 + WALL_ROWS < last) load_rows(y0 + WALL_ROWS, next_held, next_meta);
+        for (int j = 0; j < WALL_ROWS; ++j) meta[j] = pb.m(y0 + j < last ? y0 + j : last - 1);
 #pragma unroll
         for (int j = 0; j < WALL_ROWS; ++j) {
-            const float depth = (meta[j] & META_WALL_MASK) ? held[j] : GD_INF;   // no clip recorded yet: infinite
-            if (y0 + j >= last || !(distance < depth)) continue;
-            pb.d(y0 + j) = distance; pb.m(y0 + j) = (meta[j] & ~META_WALL_MASK) | (unsigned)(wall + 1);
+            if (y0 + j >= last) break;
+            const unsigned int row_wall = meta[j] & META_WALL_MASK;
+            if (row_wall != held_wall) { held_wall = row_wall; held = row_wall ? clip_distance(cc, (int)row_wall - 1) : GD_INF; }
+            if (distance < held) pb.m(y0 + j) = (meta[j] & ~META_WALL_MASK) | (unsigned)(wall + 1);
         }
-#pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) { held[j] = next_held[j]; meta[j] = next_meta[j]; }
     }
 }
 
 // `done_from` / `done_to`: rows [done_from, done_to) already carry this silhouette (pass_paint wrote it with
 // the rows the pass took out of a window nothing had touched); an empty range otherwise.
-__device__ __forceinline__ void apply_silhouette(PixelBuffers &pb, SilhouetteBounds &sb, int x, bool bottom, bool top, float floor_clip, float ceiling_clip, float distance, int wall,
+__device__ __forceinline__ void apply_silhouette(const ColumnCtx &cc, PixelBuffers &pb, SilhouetteBounds &sb, bool bottom, bool top, float floor_clip, float ceiling_clip, float distance, int wall,
                                                  int done_from, int done_to) {
     if (bottom) {
         int first = floor_clip <= 0.0f ? 0 : (floor_clip >= (float)VH ? VH : (int)floor_clip);   // clips hold integers
         int last = (distance >= sb.bot_depth) ? (sb.bot_row < VH ? sb.bot_row : VH) : VH;
-        clip_rows(pb, x, (done_to > first && done_from <= first) ? done_to : first, last, distance, wall);
+        clip_rows(cc, pb, (done_to > first && done_from <= first) ? done_to : first, last, distance, wall);
         sb.bot_row = first < sb.bot_row ? first : sb.bot_row;
         sb.bot_depth = fmaxf(sb.bot_depth, distance);
     }
     if (top) {
         int end = ceiling_clip <= 0.0f ? 0 : (ceiling_clip >= (float)VH ? VH : (int)ceiling_clip);
         int start = (distance >= sb.top_depth) ? (sb.top_row > 0 ? sb.top_row : 0) : 0;
-        clip_rows(pb, x, start, (done_from < end && done_to >= end) ? done_from : end, distance, wall);
+        clip_rows(cc, pb, start, (done_from < end && done_to >= end) ? done_from : end, distance, wall);
         sb.top_row = end > sb.top_row ? end : sb.top_row;
         sb.top_depth = fmaxf(sb.top_depth, distance);
     }
@@ -2576,19 +2667,16 @@ __device__ __forceinline__ float quad_min(float v) {
     return fminf(v, __int_as_float(quad_move<0x4E>(__float_as_int(v))));
 }
 
-// Smallest / largest of a small value (0..255) over the lanes that execute the call, found by ballots: usable inside
-// divergent code, where a lane exchange would read lanes that are switched off.  The result is uniform.
-__device__ __forceinline__ int wave_min_byte(int v) {
-    u64 candidates = __ballot(true);
-    int result = 0;
-#pragma unroll
-    for (int bit = 7; bit >= 0; --bit) {
-        const u64 clear = __ballot(!((v >> bit) & 1)) & candidates;
-        if (clear) candidates = clear; else result |= 1 << bit;
-    }
-    return result;
+// Smallest / largest value of the wavefront, by lane moves (all lanes executing; the result is uniform).
+template <int CONTROL, int ROWS> __device__ __forceinline__ int wave_move(int other, int v) { return __builtin_amdgcn_update_dpp(other, v, CONTROL, ROWS, 0xF, false); }
+__device__ __forceinline__ int wave_min(int v) {
+    const int none = 0x7fffffff;
+    v = min(v, wave_move<0x111, 0xF>(none, v)); v = min(v, wave_move<0x112, 0xF>(none, v));   // row_shr:1, 2, 4, 8: the last lane of
+    v = min(v, wave_move<0x114, 0xF>(none, v)); v = min(v, wave_move<0x118, 0xF>(none, v));   // every sixteen holds their smallest
+    v = min(v, wave_move<0x142, 0xA>(none, v)); v = min(v, wave_move<0x143, 0xC>(none, v));   // row_bcast:15, 31: lane 63 that of all
+    return __builtin_amdgcn_readlane(v, 63);
 }
-__device__ __forceinline__ int wave_max_byte(int v) { return 255 - wave_min_byte(255 - v); }
+__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
 
 // engine.py:12637-12884
 // `window_dirty` says whether some pixel inside the open window [ceiling_clip, floor_clip) may
@@ -2600,7 +2688,8 @@ template <bool DEPTH>
 __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnState &c, const PassColumn &r, PixelBuffers &pb,
                            const bool group_valid[3], const float group_bottom[3], i64 first_group_visibility,
                            const unsigned char *colormap, bool &window_dirty, GapRange &gaps) {
-    if (!(r.bits & PB_RASTER)) return;
+    // The whole wavefront comes here together, columns with nothing to draw as well: they take part in the walks over the rows.
+    const bool active = (r.bits & PB_RASTER) != 0;
     const gd_map_desc *m = cc.m;
     const LaneCtx &L = *cc.c;
     const int x = cc.x, wi = r.wall, side = r.side;
@@ -2617,7 +2706,8 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
     int y1 = c.floor_clip >= (float)VH ? VH : (int)c.floor_clip;
     const bool lower_on = !one_sided && (r.view_floor < r.other_floor);
     const bool upper_on = !one_sided && (r.view_ceiling > r.other_ceiling);
-    if (!window_dirty) {
+    const bool fresh = active && !window_dirty;
+    if (__any(fresh)) {
         // clips and projections hold integers in [0, 208]
         const unsigned claim = (unsigned)(r.render_current + 1) << META_SECTOR_SHIFT;
         // The sprite silhouettes of a two-sided drawseg (engine.py:12943-12964) give every row that this pass
@@ -2632,34 +2722,29 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
         const bool sil_top = folds && ((r.view_ceiling < r.other_ceiling) || (L.view_z > r.other_ceiling) || masked_texture);
         const unsigned clip_word = (unsigned)(wi + 1);
         int ceiling_rows_end = 0; bool ceiling_claims = false;
+        auto walk = [&](int first, int last, unsigned int word) {
+            const unsigned rows = (unsigned)max(last - first, 0);
+            for (int y = wave_min(first), wave_last = wave_max(last); y < wave_last; ++y) pb.put((unsigned)(y - first) < rows, y, word);
+        };
         {
             const bool claims = r.bits & PB_MARK_CEILING;
             const bool bare = !claims && sil_top && upper_on && (r.side_tex[2] >= 0);   // the upper tier lowers the clip past these rows
             // The wavefront walks the rows together, each column writing where its own range has the row: neighbouring
             // columns then store to neighbouring words, where loops that start at each column's own first row would
             // scatter every store over as many rows as the edges' slopes spread them.
-            const bool writes = claims || bare;
+            const bool writes = fresh && (claims || bare);
             const int first = writes ? (y0 < 0 ? 0 : y0) : VH, last = writes ? min((int)ceiling_plane_bottom, VH) : 0;
             const unsigned word = (claims ? claim : 0u) | (sil_top ? clip_word : 0u);
-            for (int y = wave_min_byte(first), wave_last = wave_max_byte(last); y < wave_last; ++y) {
-                if (y < first || y >= last) continue;
-                pb.m(y) = word;
-                if (sil_top) pb.d(y) = r.distance;
-                ceiling_rows_end = last; ceiling_claims = claims;
-        }
+            walk(first, last, word);
             ceiling_rows_end = last; ceiling_claims = claims;
         }
         {
             const bool claims = r.bits & PB_MARK_FLOOR;
             const bool bare = !claims && sil_bottom && lower_on && (r.side_tex[1] >= 0);   // the lower tier raises the clip past these rows
-            const bool writes = claims || bare;
+            const bool writes = fresh && (claims || bare);
             const int first = writes ? max((int)floor_plane_top, 0) : VH, last = writes ? y1 : 0;
             const unsigned word = (claims ? (claim | META_FLOOR) : 0u) | (sil_bottom ? clip_word : 0u);
-            for (int y = wave_min_byte(min(first, VH)), wave_last = wave_max_byte(last); y < wave_last; ++y) {
-                if (y < first || y >= last) continue;
-                pb.m(y) = word;
-                if (sil_bottom) pb.d(y) = r.distance;
-            }
+            walk(first, last, word);
             // A sector whose ceiling lies below its floor: the rows from its floor's row down to its ceiling's row
             // belong to both runs.  There the floor's claim has the say, the ceiling's stands where the floor makes none,
             // and the clip is recorded if either silhouette asks for it.
@@ -2668,15 +2753,14 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 const unsigned both = (claims ? (claim | META_FLOOR) : (ceiling_claims ? claim : 0u)) | ((sil_top || sil_bottom) ? clip_word : 0u);
                 for (int y = first; y < both_end; ++y) {
                     pb.m(y) = both;
-                    if (sil_top || sil_bottom) pb.d(y) = r.distance;
                 }
             }
         }
         // Rows that leave the window without being written: those the upper tier covers but that belong to a lower
         // tier without a texture (the lower tier has the say there), and a one-sided drawseg's own rows when it has none.
-        if (lower_on && upper_on && r.side_tex[1] < 0 && r.side_tex[2] >= 0)
+        if (fresh && lower_on && upper_on && r.side_tex[1] < 0 && r.side_tex[2] >= 0)
             zero_rows(pb, gaps, x, max((int)r.clipped_top, (int)r.clipped_lower_top), min((int)r.clipped_upper_bottom, (int)r.clipped_bottom));
-        if (one_sided && r.side_tex[0] < 0) zero_rows(pb, gaps, x, max((int)r.clipped_top, y0), min((int)r.clipped_bottom, y1));
+        if (fresh && one_sided && r.side_tex[0] < 0) zero_rows(pb, gaps, x, max((int)r.clipped_top, y0), min((int)r.clipped_bottom, y1));
         int t0 = VH, t1 = 0;
         if (one_sided) { t0 = (int)r.clipped_top; t1 = (int)r.clipped_bottom; }
         if (lower_on) { t0 = min(t0, (int)r.clipped_lower_top); t1 = max(t1, (int)r.clipped_bottom); }
@@ -2689,60 +2773,65 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
         const unsigned atlas_w = (unsigned)m->tex_max_w;
         const int side_tex0 = r.side_tex[0], side_tex1 = r.side_tex[1], side_tex2 = r.side_tex[2];
         const bool tiers_overlap = lower_on && upper_on && r.clipped_lower_top < r.clipped_upper_bottom;
-        if (!tiers_overlap) {
+        {
             // The usual case: the rows of a tier are one run, [top, bottom) of a one-sided drawseg, or the upper tier
             // above the lower one.  Each run is painted by a loop that knows its texture, so a row costs an add, a
             // shift, a texel, a colormap entry and the stores.  WALL_ROWS rows at a time, one batch ahead: the texels
             // of the next batch are asked for before the rows of this one are stored, so that a step waits for memory
             // once, not for its stores and then for its loads.
-            auto paint_run = [&](int first, int last, int texture, float origin, bool has_tail, float tail_from) {
-                if (texture < 0 || first >= last) return;
-                const int bits = tb.height_bits(texture);
+            // The wavefront walks the rows together (as above): neighbouring columns then read neighbouring texels and store
+            // neighbouring words.  Each column starting at its own first row, every load and store touched 64 cache lines
+            // (338 million cache accesses for 4096 lanes on the 4000-linedef map, 0.55 ms of every compute unit's time).
+            // First run: a one-sided drawseg's rows, or the upper tier; second run: the lower tier.
+            const bool runs = fresh && !tiers_overlap;
+#pragma unroll 1
+            for (int run = 0; run < 2; ++run) {   // one copy of the loop: the kernel is larger than the instruction cache as it is
+                const bool second = run != 0;
+                const int texture = second ? side_tex1 : (one_sided ? side_tex0 : side_tex2);
+                int first = (int)(second ? r.clipped_lower_top : r.clipped_top), last = (int)(second || one_sided ? r.clipped_bottom : r.clipped_upper_bottom);
+                const bool paints = runs && (second ? lower_on : one_sided || upper_on) && texture >= 0 && first < last;
+                if (!__any(paints)) continue;
+                first = paints ? first : VH; last = paints ? last : 0;
+                const float origin = second ? r.other_floor : (one_sided ? r.view_ceiling : r.other_ceiling);
+                const bool has_tail = second ? group_valid[1] : (one_sided ? group_valid[0] : group_valid[2]);
+                const float tail_from = second ? group_bottom[1] : (one_sided ? group_bottom[0] : group_bottom[2]);
+                const int id = paints ? texture : 0;
+                const int bits = tb.height_bits(id);
                 const i64 step64 = mul64(swall, shl64(1, 14 - bits));
                 const i64 base = shl64(round_to_i64((origin - L.view_z) * 65536.0f + toff_y), 16 - bits);
                 const unsigned shift = (unsigned)(31 - bits);   // a one-row texture (bits == 0) must shift everything out: two shifts
                 const unsigned step = (unsigned)step64;
-                unsigned frac = (unsigned)(base + (mul64(step64, FIXED_UNIT - L.center_fixed) >> 16)) + step * (unsigned)first;
-                const unsigned char *column = m->tex_atlas + ((size_t)texture * m->tex_max_h * m->tex_max_w + (size_t)tb.wrap_column(texture, u_base));
+                const int wave_first = wave_min(first), wave_last = wave_max(last);
+                unsigned frac = (unsigned)base + mul64_bits_16_47(step64, FIXED_UNIT - L.center_fixed) + step * (unsigned)wave_first;
+                // every texel asked for is the texture's own, whatever the row: the loads need no branch either
+                const unsigned column = (unsigned)id * (unsigned)(m->tex_max_h * m->tex_max_w) + (unsigned)(paints ? tb.wrap_column(id, u_base) : 0);   // the atlas is below 4 GiB
                 // rows from tail_row on take the group's shade: (float)y >= tail_from, which no row meets if that is not a number
                 const int tail_row = !has_tail || !(tail_from < (float)VH) ? VH : (tail_from <= 0.0f ? 0 : (int)ceilf(tail_from));
-                const unsigned meta_word = META_FILLED | (unsigned)(wi + 1);
-                auto load_rows = [&](int yb, unsigned char (&texel)[WALL_ROWS]) {
+                const unsigned meta_word = META_FILLED | (unsigned)(wi + 1), rows = (unsigned)max(last - first, 0);
+                const unsigned char *own_shades = colormap + shade_own * 256, *group_shades = colormap + shade_group * 256;
+                auto load_rows = [&](unsigned char (&texel)[WALL_ROWS]) {
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) {
-                        texel[j] = 0;
-                        if (yb + j < last) texel[j] = column[__umul24((frac >> shift) >> 1, atlas_w)];
-                        frac += step;
-                    }
+                    for (int j = 0; j < WALL_ROWS; ++j) { texel[j] = m->tex_atlas[column + __umul24((frac >> shift) >> 1, atlas_w)]; frac += step; }
                 };
                 unsigned char texel[WALL_ROWS];
-                load_rows(first, texel);
-                for (int yb = first; yb < last; yb += WALL_ROWS) {
-                    unsigned char next_texel[WALL_ROWS];
+                load_rows(texel);
+                for (int yb = wave_first; yb < wave_last; yb += WALL_ROWS) {
+                    unsigned char next_texel[WALL_ROWS]; unsigned colour[WALL_ROWS];
+                    load_rows(next_texel);
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) next_texel[j] = 0;
-                    if (yb + WALL_ROWS < last) load_rows(yb + WALL_ROWS, next_texel);
+                    for (int j = 0; j < WALL_ROWS; ++j) colour[j] = (yb + j >= tail_row ? group_shades : own_shades)[texel[j]];
 #pragma unroll
                     for (int j = 0; j < WALL_ROWS; ++j) {
-                        const int y = yb + j;
-                        if (y >= last) break;
-                        const unsigned colour = colormap[(y >= tail_row ? shade_group : shade_own) * 256 + texel[j]];
-                        pb.d(y) = r.distance;
-                        if (DEPTH) pb.s(y) = r.distance;
-                        pb.m(y) = meta_word | (colour << META_SECTOR_SHIFT);
+                        const bool own = (unsigned)(yb + j - first) < rows;
+                        if (DEPTH) pb.put_depth(own, yb + j, r.distance);
+                        pb.put(own, yb + j, meta_word | (colour[j] << META_SECTOR_SHIFT));
                     }
 #pragma unroll
                     for (int j = 0; j < WALL_ROWS; ++j) texel[j] = next_texel[j];
                 }
-            };
-            // first run: a one-sided drawseg's rows, or the upper tier; second run: the lower tier
-            const bool first_run = one_sided || upper_on;
-            paint_run(first_run ? (int)r.clipped_top : 0, first_run ? (int)(one_sided ? r.clipped_bottom : r.clipped_upper_bottom) : 0,
-                      one_sided ? side_tex0 : side_tex2, one_sided ? r.view_ceiling : r.other_ceiling,
-                      one_sided ? group_valid[0] : group_valid[2], one_sided ? group_bottom[0] : group_bottom[2]);
-            paint_run(lower_on ? (int)r.clipped_lower_top : 0, lower_on ? (int)r.clipped_bottom : 0, side_tex1, r.other_floor,
-                      group_valid[1], group_bottom[1]);
-        } else {
+            }
+        }
+        if (fresh && tiers_overlap) {
             // The lower and the upper tier share rows (a closed door, say): the lower tier has the say there, row by row.
                 int tier_tex[3]; unsigned tier_frac[3], tier_step[3], tier_shift[3]; size_t tier_texel[3];
             const float tier_origin[3] = {r.view_ceiling, r.other_floor, r.other_ceiling};
@@ -2795,7 +2884,6 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 for (int j = 0; j < WALL_ROWS; ++j) {
                     if (!(draw & (1u << j))) continue;
                     const unsigned colour = colormap[((tail & (1u << j)) ? shade_group : shade_own) * 256 + texel[j]];
-                    pb.d(yb + j) = r.distance;
                     if (DEPTH) pb.s(yb + j) = r.distance;
                     pb.m(yb + j) = META_FILLED | (colour << META_SECTOR_SHIFT) | (unsigned)(wi + 1);
                 }
@@ -2804,12 +2892,12 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 draw = next_draw; tail = next_tail;
             }
         }
-        if (one_sided) {
+        if (fresh && one_sided) {
             window_dirty = true;
             if (r.side_tex[0] >= 0 && t0 < t1) gaps.set_filled(max(t0, 0), min(t1, VH));   // every row of [t0, t1) was drawn just now
         }
-        return;
     }
+    if (!active || fresh) return;
     // A one-sided drawseg has painted this window.  Every row of it has been written since (GapRange), so what a later pass
     // can still change is narrow: a tier pixel where no tier was drawn yet, which can only lie in this pass's own tier rows
     // and outside the rows that drawseg filled, and a plane claim on a row nobody owns, which can only be one of the rows
@@ -2859,8 +2947,8 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 unsigned char texel = m->tex_atlas[((size_t)texture_id * m->tex_max_h + tv) * m->tex_max_w + tu];
                 const unsigned colour = colormap[(bottom_tail ? shade_group : shade_own) * 256 + texel];
                 if (DEPTH) pb.s(y) = r.distance;
-                const float held = (meta & META_WALL_MASK) ? pb.d(y) : GD_INF;   // no clip recorded yet
-                if (r.distance < held) { pb.d(y) = r.distance; meta = (meta & ~META_WALL_MASK) | (unsigned)(wi + 1); }
+                const float held = (meta & META_WALL_MASK) ? clip_distance(cc, (int)(meta & META_WALL_MASK) - 1) : GD_INF;   // no clip recorded yet
+                if (r.distance < held) { meta = (meta & ~META_WALL_MASK) | (unsigned)(wi + 1); }
                 meta = (meta & ~(META_SECTOR_MASK << META_SECTOR_SHIFT)) | (colour << META_SECTOR_SHIFT) | META_FILLED;
                 meta_dirty = true;
             }
@@ -2876,7 +2964,8 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
 #define ADVANCE_STATE 1
 #define ADVANCE_CLIPS 2
 template <bool SPLIT, int PART>
-__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c, const PassColumn &r, PixelBuffers &pb, SilhouetteBounds &sb, bool window_untouched, GapRange &gaps) {
+__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c, const PassColumn &r, PixelBuffers &pb, SilhouetteBounds &sb, bool window_untouched, GapRange &gaps,
+                             const Scratch *sc = nullptr, size_t at = 0) {   // the pass's place in the chunk's planes, for the clips
     const gd_map_desc *m = cc.m;
     const MapView &mv = cc.mv;
     const LaneCtx &L = *cc.c;
@@ -2911,10 +3000,10 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c
             // one call per side: the rows already done differ.  pass_paint stays inside the old window, and a sector whose
             // ceiling lies below its floor can carry a clip past the window's other end: then the rows beyond that end
             // are not done, and the range is cut there (apply_silhouette then takes no short cut and visits them all).
-            apply_silhouette(pb, sb, x, bottom_sil, false, c.floor_clip, c.ceiling_clip, distance, wi, max(row_of(c.floor_clip), old_ceiling), old_floor);
-            apply_silhouette(pb, sb, x, false, top_sil, c.floor_clip, c.ceiling_clip, distance, wi, old_ceiling, min(row_of(c.ceiling_clip), old_floor));
+            apply_silhouette(cc, pb, sb, bottom_sil, false, c.floor_clip, c.ceiling_clip, distance, wi, max(row_of(c.floor_clip), old_ceiling), old_floor);
+            apply_silhouette(cc, pb, sb, false, top_sil, c.floor_clip, c.ceiling_clip, distance, wi, old_ceiling, min(row_of(c.ceiling_clip), old_floor));
         } else {
-            apply_silhouette(pb, sb, x, bottom_sil, top_sil, c.floor_clip, c.ceiling_clip, distance, wi, 0, 0);
+            apply_silhouette(cc, pb, sb, bottom_sil, top_sil, c.floor_clip, c.ceiling_clip, distance, wi, 0, 0);
         }
     }
     // r. clips of the geometric portal behind a projected solid (engine.py:12969-13069)
@@ -2925,11 +3014,12 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c
         float pof = tb.floor_h(path_safe_other), poc = tb.ceil_h(path_safe_other);
         int pside = (r.bits & PB_PS_FROM_FRONT) ? 0 : 1;
         const int *ptex = m->side_tex + (path * 2 + pside) * 3;
-        const float path_top = r.path_top, path_bottom = r.path_bottom, path_lower_top = r.path_lower_top, path_upper_bottom = r.path_upper_bottom;
-        float pct = fmaxf(path_top, c.ceiling_clip);
-        float pcb = fminf(path_bottom, c.floor_clip);
-        float pcub = fmaxf(fminf(path_upper_bottom, c.floor_clip), pct);
-        float pclt = fminf(fmaxf(path_lower_top, c.ceiling_clip), pcb);
+        const WallRows rows = path_rows(cc, *sc, at, r.marks, r);
+        const float path_distance = sc->pass_path_distance[at];
+        float pct = fmaxf(rows.ceiling, c.ceiling_clip);
+        float pcb = fminf(rows.floor, c.floor_clip);
+        float pcub = fmaxf(fminf(rows.other_ceiling, c.floor_clip), pct);
+        float pclt = fminf(fmaxf(rows.other_floor, c.ceiling_clip), pcb);
         bool light_differs = tb.light(r.render_current) != tb.light(path_safe_other);
         bool p_draws_upper = (r.view_ceiling > poc) && (ptex[2] >= 0);
         bool p_marks_ceiling = (r.view_ceiling != poc) || (tb.ceil_tex(r.render_current) != tb.ceil_tex(path_safe_other)) || light_differs;
@@ -2950,7 +3040,7 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c
         bool pmasked = ptex[0] >= 0;
         bool pbottom = (r.view_floor > pof) || (L.view_z < pof) || pmasked;
         bool ptop = (r.view_ceiling < poc) || (L.view_z > poc) || pmasked;
-        apply_silhouette(pb, sb, x, pbottom, ptop, c.floor_clip, c.ceiling_clip, r.ps_path_distance, path, 0, 0);
+        apply_silhouette(cc, pb, sb, pbottom, ptop, c.floor_clip, c.ceiling_clip, path_distance, path, 0, 0);
     }
   }
     if (PART == ADVANCE_CLIPS) return false;
@@ -3058,79 +3148,60 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c
 }
 
 // engine.py:13424-13744 for one column
-template <bool DEPTH, bool SPLIT>
-__device__ __forceinline__ void masked_midtexture(const ColumnCtx &cc, const ColumnState &c, PixelBuffers &pb, const unsigned char *colormap) {
+template <bool DEPTH, bool GENERAL>
+__device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, int local, const ColumnState &c, PixelBuffers &pb, const unsigned char *colormap) {
     const gd_map_desc *m = cc.m;
-    const MapView &mv = cc.mv;
     const LaneCtx &L = *cc.c;
     const int x = cc.x;
-    float md = GD_INF; int mw = 0x7fffffff; int mside = 0; int cand_flags = 0;
-    for (int k0 = 0; k0 < cc.count; k0 += CAND_BATCH) {
-        Cand batch[CAND_BATCH];
-        cc.cand_batch(k0, batch);
-#pragma unroll
-        for (int j = 0; j < CAND_BATCH; ++j) {
-            if (k0 + j >= cc.count) continue;
-            const Cand q = batch[j];
-            int w = q.wall;
-            if (!(q.flags & CF_PROJ) || (q.s1 < 0)) continue;
-            int sidew = (q.flags & CF_FF) ? 0 : 1;   // engine.py:13436-13444, the float32 facing test
-            if (!(q.flags & CF_MASKED)) continue;     // no mid-texture on that side
-            if (q.dist < md || (q.dist == md && w < mw)) { md = q.dist; mw = w; mside = sidew; cand_flags = q.flags; }
-        }
-    }
-    if (!finitef(md)) return;
-    int texture_id = m->side_tex[(mw * 2 + mside) * 3];
-    if (texture_id < 0) texture_id = 0;
+    const u64 hit = sc.masked_hit[(size_t)local * SW + x];
+    if (hit == CAND_KEY_NONE) return;
+    const int mw = cand_key_wall(hit), cand_flags = cand_key_flags(hit);
+    const float md = cand_key_distance(hit);
+    const int mside = (cand_flags & CF_FF) ? 0 : 1;   // engine.py:13436-13444, the float32 facing test
     bool left_edge = cand_flags & CF_LEDGE;
     bool has_saved = c.masked_wall == mw;
     if (!(has_saved || left_edge)) return;
-    const WallRec &wr = cc.rec(mw);
-    const FragmentChoice wr_fragment = choose_fragment<SPLIT>(m, cc.frags, wr, mw, x);
-    int front_sector = mv.sec(mw, 0), back_sector = mv.sec(mw, 1) < 0 ? 0 : mv.sec(mw, 1);
-    int light_sector = mside == 0 ? front_sector : back_sector;
+    const WallSide &ws = dm.wall_side[2 * mw + mside];
+    const WallGeo &geo = sc.geo[sc.geo_slot[cc.rec_base + (unsigned)mw]];
+    const MaskedGeo &masked = sc.masked_geo[(size_t)local * dm.masked_count + dm.masked_slot[mw]];
+    const int texture_id = ws.tex[0];
     const Tables &tb = *cc.tb;
-    float world_top = fminf(tb.ceil_h(front_sector), tb.ceil_h(back_sector));
+    const int front_sector = cc.mv.sec(mw, 0), back_sector = cc.mv.sec(mw, 1);
+    const int light_sector = mside == 0 ? front_sector : back_sector;
+    const float world_top = fminf(tb.ceil_h(front_sector), tb.ceil_h(back_sector));
     const int th = m->tex_h[texture_id];   // the texture's own height, whatever its row mask (engine.py:13480-13483)
-    float owall_top = 0, owall_bottom = 0;
+    float owall_top, owall_bottom;
+    i64 visibility = geo.visibility[mside].at(x);
+    bool split = false;
+    if (GENERAL) {
+        const WallRec &wr = cc.rec(mw);
+        split = (wr.flags & WF_SPLIT) != 0;
+        if (split) {
+            const FragmentChoice fragment = choose_fragment<true>(m, cc.frags, wr, mw, x);
 #pragma unroll 1
-    for (int k = 0; k < 2; ++k) {
-        float v = project(L, wr, wr_fragment, k == 0 ? world_top : world_top - (float)th, x);
-        if (k == 0) owall_top = v; else owall_bottom = v;
+            for (int k = 0; k < 2; ++k) {
+                float v = project(L, wr, fragment, k == 0 ? world_top : world_top - (float)th, x);
+                if (k == 0) owall_top = v; else owall_bottom = v;
+            }
+            if (fragment.lights) visibility = wall_visibility(*fragment.rec, mside, x);
+        }
+    }
+    if (!split) {
+        const bool in_span = x >= geo.span0 && x < geo.span1;
+        const HeightBend top_bend = masked.bend[0], bottom_bend = masked.bend[1];
+        owall_top = !in_span && bends(top_bend) ? height_row(masked.outside[0], x) : bent_row(height_row(masked.line[0], x), top_bend, x);
+        owall_bottom = !in_span && bends(bottom_bend) ? height_row(masked.outside[1], x) : bent_row(height_row(masked.line[1], x), bottom_bend, x);
     }
     float mceil = fmaxf(owall_top, has_saved ? c.masked_ceiling_clip : 0.0f);
     float mfloor = fminf(owall_bottom, has_saved ? c.masked_floor_clip : (float)VH);
-    const float *toff = m->side_off + (mw * 2 + mside) * 2;
-    i64 h, swall_cur;
-    texture_mapping(m, wr, mw, x, &h, &swall_cur);
-    i64 repeat = round_to_i64(m->wall_len[mw] * 65536.0f);
-    if (mside != 0) h = repeat - h;
-    i64 msl = wr.sl, msr = wr.sr;
-    if (msl > 0 && h < 0) h = 0;
-    if (h >= repeat) h = repeat - 1;
-    i64 offx = round_to_i64(toff[0] * 65536.0f);
-    i64 mu = tb.wrap_column(texture_id, (h + offx) >> 16);
+    i64 u_base, swall_cur;
+    texture_column(geo, geo.past_left != 0, ws, mside, x, &u_base, &swall_cur);
+    const i64 mu = tb.wrap_column(texture_id, u_base);
     int height_bits = ilog2(th);
     i64 vertical_step = mul64(swall_cur, shl64(1, 14 - height_bits));
     i64 center_fixed = L.center_fixed;
-    i64 texture_mid = round_to_i64((world_top - L.view_z) * 65536.0f + toff[1] * 65536.0f);
-    int safe_left = (int)clampi(msl, 0, SW - 1), safe_last = (int)clampi(msr - 1, 0, SW - 1);
-    i64 dummy_h, start_swall = 0, end_swall = 0;
-#pragma unroll 1
-    for (int k = 0; k < 2; ++k) {
-        i64 sw;
-        texture_mapping(m, wr, mw, k == 0 ? safe_left : safe_last, &dummy_h, &sw);
-        if (k == 0) start_swall = sw; else end_swall = sw;
-    }
-    auto iscale_of = [](i64 swall) {
-        i64 s = mul64(swall, FIXED_UNIT) >> 18;
-        if (s >= 0 && s < 3) return (i64)3;
-        if (s > -3 && s < 0) return (i64)-3;
-        return s;
-    };
-    i64 start_scale = tdiv(1LL << 32, iscale_of(start_swall)), end_scale = tdiv(1LL << 32, iscale_of(end_swall));
-    i64 scale_step = tdiv(end_scale - start_scale, max64(msr - msl, 1));
-    i64 sprite_scale = start_scale + mul64(scale_step, (i64)x - msl);
+    i64 texture_mid = round_to_i64((world_top - L.view_z) * 65536.0f + ws.offset_y * 65536.0f);
+    const i64 sprite_scale = masked.scale.at(x);
     i64 top_screen = center_fixed - (mul64(texture_mid, sprite_scale) >> 16);
     i64 post_top = top_screen >> 16;
     i64 post_bottom = ((top_screen + mul64(sprite_scale, th) - FIXED_UNIT) >> 16) + 1;
@@ -3142,11 +3213,8 @@ __device__ __forceinline__ void masked_midtexture(const ColumnCtx &cc, const Col
     i64 frac_end = frac_start + mul64(clipped_bottom - clipped_top - 1, dc_iscale);
     bool extends = initial_post && ((float)clipped_bottom < mfloor) && (frac_end < (i64)th * FIXED_UNIT - dc_iscale);
     clipped_bottom += extends ? 1 : 0;
-    const float4 wl = *reinterpret_cast<const float4 *>(m->walls + 4 * mw);
-    bool horizontal = fabsf(wl.w - wl.y) < 1e-6f, vertical = fabsf(wl.z - wl.x) < 1e-6f;
-    float contrast = vertical ? 16.0f : (horizontal ? -16.0f : 0.0f);
-    float light = (tb.light(light_sector) + (float)(L.flash_light * 16)) + contrast;
-    i64 shade = wall_shade(light, wall_visibility(wr_fragment.lights ? *wr_fragment.rec : wr, mside, x));
+    float light = (tb.light(light_sector) + (float)(L.flash_light * 16)) + ws.contrast;
+    i64 shade = wall_shade(light, visibility);
     int y0 = (int)clampi(clipped_top, 0, VH), y1 = (int)clampi(clipped_bottom, 0, VH);
     // WALL_ROWS rows at a time: texels and meta words are asked for together, then the stores
     // as in pass_paint: only the low 32 bits of the row fraction matter, and they advance by the step's low 32 bits
@@ -3168,14 +3236,215 @@ __device__ __forceinline__ void masked_midtexture(const ColumnCtx &cc, const Col
         for (int j = 0; j < WALL_ROWS; ++j) {
             const int y = yb + j;
             if (y >= y1) continue;
-            // the texel goes to the frame where there is one; otherwise it waits in the sprite clip plane, which nothing
-            // reads any more once a column's traversal is over, for the kernel that assembles the frame
+            // the texel goes to the frame where there is one; otherwise it waits for the kernel that assembles the frame
             const unsigned char colour = colormap[shade * 256 + texel[j]];
             if (pb.frame) pb.f(y) = colour;
-            else pb.d(y) = __uint_as_float((unsigned)colour);
+            else pb.t(y) = colour;
             pb.m(y) = word[j] | META_MASKED;
             if (DEPTH) pb.s(y) = md;
         }
+    }
+}
+
+// One height of a linedef as a line over the columns: OWallMost (engine.py:12294-12605, project() above) with the column left open.
+struct HeightLine { ColumnLine line, outside; HeightBend bend; };
+__device__ __forceinline__ HeightLine height_line(const LaneCtx &c, const WallRec &g, float world_z) {
+    HeightLine out;
+    const i64 depth_left = max64(g.dl, 1), depth_right = max64(g.dr, 1);
+    const i64 pz = -(round_to_i64((world_z - c.view_z) * 65536.0f) >> 4);
+    auto line_of = [&](i64 left, i64 right, i64 dl, i64 dr) {
+        const i64 pl = tdiv(mul64(pz, FOCAL_Y_FIXED), max64(dl, 1)), pr = tdiv(mul64(pz, FOCAL_Y_FIXED), max64(dr, 1));
+        ColumnLine line;
+        line.step = tdiv(pr - pl, max64(right - left, 1));
+        line.base = (i64)((u64)(c.center_fixed + pl) - (u64)left * (u64)line.step);
+        return line;
+    };
+    out.outside = line_of(g.sl, g.sr, depth_left, depth_right);
+    out.line = out.outside;
+    out.bend.top = 0u; out.bend.bottom = 0u;
+    if (!(g.sr > g.sl)) return out;
+    const i64 upper_left = mul64(c.upper_clip, depth_left) >> 16, upper_right = mul64(c.upper_clip, depth_right) >> 16;
+    const i64 lower_left = mul64(c.lower_clip, depth_left) >> 16, lower_right = mul64(c.lower_clip, depth_right) >> 16;
+    const bool above_left = pz < upper_left, above_right = pz < upper_right;
+    const bool below_left = pz > lower_left, below_right = pz > lower_right;
+    const bool entirely_above = above_left && above_right, entirely_below = below_left && below_right;
+    const bool crosses_top = above_left != above_right, crosses_bottom = below_left != below_right;
+    if (!(entirely_above || entirely_below || crosses_top || crosses_bottom)) return out;
+    out.bend.bottom = 0x80000000u;
+    i64 clipped_left = g.sl, clipped_right = g.sr, clipped_dl = depth_left, clipped_dr = depth_right;
+    i64 top0 = 0, top1 = 0, bottom0 = 0, bottom1 = 0;
+#pragma unroll 1
+    for (int edge = 0; edge < 2; ++edge) {   // the top of the view, then its bottom: one copy of the divisions
+        if (!(edge ? crosses_bottom : crosses_top)) continue;
+        const i64 at_left = edge ? lower_left : upper_left, at_right = edge ? lower_right : upper_right;
+        const bool beyond_left = edge ? below_left : above_left, beyond_right = edge ? below_right : above_right;
+        const i64 fraction = tdiv(shl64(pz - at_left, 30), at_right != at_left ? at_right - at_left : 1);
+        const i64 depth = depth_left + (mul64(depth_right - depth_left, fraction) >> 30);
+        const i64 cross = g.sl + tdiv(mul64(mul64(depth_right, fraction) >> 30, g.sr - g.sl), max64(depth, 1));
+        if (beyond_right && g.sl <= cross) { clipped_right = cross; clipped_dr = depth; }
+        if (beyond_left && cross <= g.sr) { clipped_left = cross; clipped_dl = depth; }
+        const i64 from = beyond_right ? cross : g.sl, to = beyond_right ? g.sr : cross;   // the columns beyond the edge
+        if (edge) { bottom0 = from; bottom1 = to; } else { top0 = from; top1 = to; }
+    }
+    auto column = [](i64 v) { return (unsigned int)clampi(v, 0, SW); };
+    if (entirely_above) {
+        out.line.base = 0; out.line.step = 0;
+        return out;
+    }
+    out.bend.top = column(top0) | (column(top1) << 10);
+    if (entirely_below) {
+        out.line.base = (i64)VH << 16; out.line.step = 0;
+        return out;
+    }
+    out.bend.bottom |= column(bottom0) | (column(bottom1) << 10);
+    if (clipped_right == clipped_left && clipped_left >= 0 && clipped_left < SW) out.bend.top |= (unsigned int)(clipped_left + 1) << 20;
+    out.line = line_of(clipped_left, clipped_right, clipped_dl, clipped_dr);
+    return out;
+}
+
+// The same for a linedef's masked mid-texture, by four threads: its upper and lower edge, and the two ends of the sprite scale
+// (engine.py:13480-13560).  `r` faces the camera with the side that carries the texture.
+__device__ __forceinline__ void masked_lines(const DeviceMap &dm, const LaneCtx &c, const WallRec &r, int w, int k, MaskedGeo &out) {
+    const gd_map_desc *m = &dm.d;
+    const WallSide &ws = dm.wall_side[2 * w + ((r.flags & WF_FF) ? 0 : 1)];
+    const float world_top = fminf(m->sector_heights[2 * m->wall_sectors[2 * w] + 1], m->sector_heights[2 * m->wall_sectors[2 * w + 1] + 1]);
+    const HeightLine edge = height_line(c, r, (k & 1) ? world_top - (float)m->tex_h[ws.tex[0]] : world_top);
+    i64 hoff, swall;
+    texture_mapping(r, ws.repeat, (int)clampi((k & 1) ? r.sr - 1 : r.sl, 0, SW - 1), &hoff, &swall);
+    i64 iscale = mul64(swall, FIXED_UNIT) >> 18;
+    if (iscale >= 0 && iscale < 3) iscale = 3;
+    else if (iscale > -3 && iscale < 0) iscale = -3;
+    const i64 scale = tdiv(1LL << 32, iscale);
+    const i64 other = (i64)(((u64)(unsigned)quad_move<0xB1>((int)(scale >> 32)) << 32) | (u64)(unsigned)quad_move<0xB1>((int)scale));
+    if (k >= 2) return;
+    out.line[k] = edge.line; out.bend[k] = edge.bend;
+    if (bends(edge.bend)) out.outside[k] = edge.outside;
+    if (k == 0) {
+        out.scale.step = tdiv(other - scale, max64(r.sr - r.sl, 1));
+        out.scale.base = (i64)((u64)scale - (u64)r.sl * (u64)out.scale.step);
+    }
+}
+
+// A linedef's WallGeo by four threads of a quad: thread k takes height k.
+__device__ __forceinline__ void wall_lines(const DeviceMap &dm, const LaneCtx &c, const WallRec &r, int w, int k, WallGeo &geo) {
+    const gd_map_desc *m = &dm.d;
+    const int sector = m->wall_sectors[2 * w + (k >> 1)];
+    const float height = m->sector_heights[2 * (sector < 0 ? 0 : sector) + ((k == 0 || k == 3) ? 1 : 0)];
+    const HeightLine line = height_line(c, r, height);
+    geo.line[k] = line.line; geo.bend[k] = line.bend;
+    if (bends(line.bend)) geo.outside[k] = line.outside;
+    // the wallscan light (engine.py:11217-11291): thread k takes end k & 1 of side k >> 1
+    const int side = k >> 1, end = k & 1;
+    const i64 tx1 = side ? r.tx1 : r.tx0, tx2 = side ? r.tx0 : r.tx1, ty1 = side ? r.ty1 : r.ty0, ty2 = side ? r.ty0 : r.ty1;
+    const i64 center = 160 * FIXED_UNIT;
+    const i64 tx = end ? tx2 : tx1, ty = end ? ty2 : ty1;
+    const bool inside = end ? tx2 <= ty2 : tx1 >= -ty1;
+    const i64 projected = ((center + tdiv(tx * center, ty == 0 ? 1 : ty)) >> 16) + (tx >= 0);
+    const i64 den = end ? ty2 - ty1 - tx2 + tx1 : tx1 - tx2 - ty2 + ty1;
+    const i64 column = inside ? projected : (end ? SW : 0);
+    const i64 depth = inside ? ty : ty1 + tdiv((ty2 - ty1) * (end ? tx1 - ty1 : tx1 + ty1), den == 0 ? 1 : den);
+    const i64 light = tdiv(WALL_VISIBILITY_FIXED << 12, max64(depth, 1));
+    auto other_end = [](i64 v) { return (i64)(((u64)(unsigned)quad_move<0xB1>((int)(v >> 32)) << 32) | (u64)(unsigned)quad_move<0xB1>((int)v)); };
+    const i64 other_light = other_end(light), other_column = other_end(column);
+    const i64 light_left = end ? other_light : light, light_right = end ? light : other_light;
+    const i64 left = end ? other_column : column, right = end ? column : other_column;
+    ColumnLine visibility;
+    visibility.step = tdiv(light_right - light_left, max64(right - left, 1));
+    visibility.base = (i64)((u64)light_left - (u64)left * (u64)visibility.step);
+    if (end == 0) geo.visibility[side] = visibility;
+    if (k == 0) {
+        const bool spans = r.sr > r.sl;
+        geo.tx0 = r.tx0; geo.tx1 = r.tx1; geo.ty0 = r.ty0; geo.ty1 = r.ty1;
+        geo.span0 = (int)(spans ? clampi(r.sl, 0, SW) : 0); geo.span1 = (int)(spans ? clampi(r.sr, 0, SW) : 0);
+        geo.past_left = r.sl > 0 ? 1 : 0;
+    }
+}
+
+// The linedefs that the recorded passes of a lane draw, each worked out once (WallGeo) for all the columns and passes that draw it.
+// The drawing half used to do this per column and pass: some 25 64-bit divisions, two thirds of its instructions, for what is
+// the same in every column of a linedef.  One work-group per lane: it turns the bits wall_select_kernel left into a list, takes as many
+// slots of geo, and gives four threads to a linedef (one a height; the wallscan light's four ends likewise).
+#define GEO_LIST 1024                            // linedefs listed at a time
+template <bool SPLIT>
+__global__ void __launch_bounds__(SW) wall_geometry_kernel(DeviceMap dm, int lane_count, Scratch sc) {
+    const gd_map_desc *m = &dm.d;
+    __shared__ unsigned short list[GEO_LIST];
+    __shared__ int listed, list_end, first_slot, masked_listed;
+    __shared__ unsigned short masked_list[SW];
+    const int local = blockIdx.x;
+    if (local >= lane_count) return;              // uniform over the block
+    const int x = threadIdx.x, k = threadIdx.x & 3;
+    const LaneCtx &c = sc.ctx[local];
+    const WallRec *recs = sc.rec + (size_t)local * m->wall_count;
+    unsigned int *slots = sc.geo_slot + (size_t)local * m->wall_count;
+    unsigned int *named = sc.named + (size_t)local * named_words(m);
+    if (threadIdx.x == 0) { listed = 0; list_end = GEO_LIST; masked_listed = 0; }
+    __syncthreads();
+    if (dm.masked_count > 0) {
+        // masked mid-textures: the linedef of every column's nearest one (its light and its texture mapping are WallGeo's)
+        const u64 hit = sc.masked_hit[(size_t)local * SW + x];
+        const int w = cand_key_wall(hit);
+        if (hit != CAND_KEY_NONE) atomicOr(&named[w >> 5], 1u << (w & 31));
+        // runs of columns share theirs: the first of a run (within its 16 columns) lists it
+        if (hit != CAND_KEY_NONE && __builtin_amdgcn_update_dpp(-1, w, 0x111 /* row_shr:1 */, 0xF, 0xF, false) != w) masked_list[atomicAdd(&masked_listed, 1)] = (unsigned short)w;
+        __syncthreads();                          // the bits are in place too: the barrier orders the block's memory
+        MaskedGeo *masked = sc.masked_geo + (size_t)local * dm.masked_count;
+        for (int task = threadIdx.x; task < 4 * masked_listed; task += SW) {
+            const int w = masked_list[task >> 2];
+            masked_lines(dm, c, recs[w], w, k, masked[dm.masked_slot[w]]);
+        }
+    }
+    const int words = named_words(m);
+    for (int word0 = 0; word0 < words; word0 += SW) {
+        // the bits of SW words at a time: a thread a word, as many of them as the list holds
+        unsigned int bits = word0 + x < words ? __hip_atomic_load(&named[word0 + x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+        for (;;) {
+            if (bits) {
+                const int mine = __popc(bits);
+                int at = atomicAdd(&listed, mine);
+                if (at + mine <= GEO_LIST) {
+                    for (; bits; bits &= bits - 1u) list[at++] = (unsigned short)((word0 + x) * 32 + __ffs((int)bits) - 1);
+                } else {
+                    atomicMin(&list_end, at);     // full: the first to find it so ends the list, everybody after it finds it so too
+                }
+            }
+            const int waiting = __syncthreads_or(bits != 0u);
+            const int count = min(listed, list_end);
+            if (threadIdx.x == 0 && count > 0) first_slot = atomicAdd(sc.geo_count, count);
+            __syncthreads();
+            for (int task = threadIdx.x; task < 4 * count; task += SW) {   // the four threads of a linedef are one DPP quad
+                const int w = list[task >> 2], slot = first_slot + (task >> 2);
+                wall_lines(dm, c, recs[w], w, k, sc.geo[slot]);
+                if (k == 0) slots[w] = (unsigned int)slot;
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) { listed = 0; list_end = GEO_LIST; }
+            __syncthreads();
+            if (!waiting) break;                  // the same in the whole block
+        }
+    }
+    // the few passes whose rows are their own, column by column
+    if (!((sc.own_rows[local] >> (x >> 6)) & 1u)) return;
+    const WallRec *frags = sc.frag_rec + (size_t)local * m->split_count * m->fragment_slots;
+    const int passes = sc.pass_count[(size_t)local * SW + x];
+    for (int pass = 0; pass < passes; ++pass) {
+        const size_t at = sc.pass_at(pass, local, x);
+        const PassRec rec = sc.pass_rec[at];
+        if (!(rec.bits & (PB_RASTER | PB_PS_KEEPS)) || !(rec.marks & REC_OWN_ROWS)) continue;
+        const int other = m->wall_sectors[2 * rec.wall + ((rec.marks & REC_SIDE1) ? 0 : 1)];
+        unsigned int rows[2] = {0u, 0u};
+#pragma unroll 1
+        for (int h = 0; h < 8; ++h) {
+            if (h < 4 ? (h >= 2 && (rec.bits & PB_ONE_SIDED)) : !(rec.bits & PB_PS_KEEPS)) continue;
+            const int w = h < 4 ? rec.wall : rec.ps_path;
+            const int behind = h < 4 ? other : (int)rec.ps_other;
+            const int sector = (h & 2) ? (behind < 0 ? 0 : behind) : (int)rec.render_current;
+            const float z = m->sector_heights[2 * sector + ((h & 3) == 0 || (h & 3) == 3 ? 1 : 0)];
+            const FragmentChoice fragment = choose_fragment<SPLIT>(m, frags, recs[w], w, x);
+            const unsigned int row = (unsigned int)project(c, recs[w], fragment, z, x);
+            rows[h >> 2] |= row << (8 * (h & 3));
+        }
+        sc.pass_rows[at] = make_uint2(rows[0], rows[1]);
     }
 }
 
@@ -3291,8 +3560,12 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
     bool boundary_has_po = false;
     for (int k = 0; k < cc.count; ++k) if (cc.cand(k).flags & CF_LEDGE) { boundary_has_po = true; break; }
-    PassRec *records = sc.pass_rec + ((size_t)local * sc.pass_slots * SW + x);
-    float *path_distances = sc.pass_path_distance + ((size_t)local * sc.pass_slots * SW + x);
+    PassRec *records = sc.pass_rec + sc.pass_at(0, local, x);
+    float *path_distances = sc.pass_path_distance + sc.pass_at(0, local, x);
+    const size_t pass_stride = (size_t)sc.lane_stride * SW;
+    // the linedefs the recorded passes draw get a bit each; columns that draw what the column before them draws leave it to that one
+    unsigned int *named = sc.named + (size_t)local * named_words(m);
+    int last_named = -1;
     PixelBuffers no_pixels; SilhouetteBounds no_bounds; GapRange no_gaps;   // the state part of pass_advance touches none of them
     PassColumn pc;
     bool done = false;
@@ -3306,11 +3579,20 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
                     PassRec rec;
                     rec.wall = (unsigned short)pc.wall; rec.render_current = (unsigned short)pc.render_current;
                     rec.bits = (unsigned short)pc.bits; rec.ps_path = (unsigned short)pc.ps_path_index;
-                    rec.ps_other = (short)pc.ps_other; rec.spare = 0; rec.distance = pc.distance;
+                    rec.ps_other = (short)pc.ps_other; rec.marks = (unsigned short)pc.marks; rec.distance = pc.distance;
                     // passes between two recorded ones keep whatever the slot held: the drawing half skips them by their bits
-                    for (int skipped = recorded; skipped < pass; ++skipped) records[(size_t)skipped * SW].bits = 0;
-                    records[(size_t)pass * SW] = rec;
-                    if (pc.bits & PB_PS_KEEPS) path_distances[(size_t)pass * SW] = pc.ps_path_distance;
+                    for (int skipped = recorded; skipped < pass; ++skipped) records[(size_t)skipped * pass_stride].bits = 0;
+                    records[(size_t)pass * pass_stride] = rec;
+                    const bool repeats = last_named == pc.wall;
+                    last_named = pc.wall;
+                    // a neighbour that does not take part in this pass shows the linedef it named last
+                    if (!repeats && __builtin_amdgcn_update_dpp(-1, last_named, 0x111 /* row_shr:1 */, 0xF, 0xF, false) != last_named)
+                        atomicOr(&named[pc.wall >> 5], 1u << (pc.wall & 31));
+                    if (pc.bits & PB_PS_KEEPS) {
+                        path_distances[(size_t)pass * pass_stride] = pc.ps_path_distance;
+                        atomicOr(&named[pc.ps_path_index >> 5], 1u << (pc.ps_path_index & 31));
+                    }
+                    if (pc.marks & REC_OWN_ROWS) atomicOr(&sc.own_rows[local], 1u << (x >> 6));
                     recorded = pass + 1;
                 } else {
                     atomicOr(sc.status, STATUS_PASS_OVERFLOW);
@@ -3330,10 +3612,12 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
 // those tables, 16.7 KB, are held once per group rather than once per wavefront (a CU has 160 KB of LDS and room for
 // sixteen of these wavefronts at 128 registers).  After the staging barrier the wavefronts never meet again.
 #define WALL_STRIPS_PER_GROUP 2
-// DEPTH: also keep the depth of every wall pixel (frames that draw decals).  SPLIT: the map has linedefs with
-// BSP projection fragments.
-template <bool DEPTH, bool SPLIT>
-__global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(4, 4))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
+#define RASTER_WAVES 4
+// DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
+// BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
+// behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
+template <bool DEPTH, bool GENERAL>
+__global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(RASTER_WAVES, RASTER_WAVES))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
     __shared__ LaneCtx lane_ctxs[WALL_STRIPS_PER_GROUP][64 / SEG_COLS];
     __shared__ unsigned char colormap_lds[32 * 256];   // shade rows 0..31 are the only ones indexed
@@ -3348,6 +3632,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     const int local = segment / SEGS_PER_LANE;
     Tables tb;
     stage_tables(m, sector_lds, &tex_lds, tb);
+    tb.all_cached = !GENERAL;
     if ((lane_id & (SEG_COLS - 1)) == 0 && live) lane_ctxs[wave_in_group][segment_in_wave] = sc.ctx[local];
     for (int k = threadIdx.x; k < 32 * 256 / 4; k += blockDim.x) reinterpret_cast<unsigned int *>(colormap_lds)[k] = reinterpret_cast<const unsigned int *>(m->colormap)[k];
     __syncthreads();
@@ -3361,14 +3646,15 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     cc.recs = sc.rec; cc.spans = sc.span;
     cc.rec_base = (unsigned)local * (unsigned)m->wall_count;
     cc.frags = sc.frag_rec + (size_t)local * m->split_count * m->fragment_slots;
-    cc.set_list(sc, local, x);
     cc.x = x;
     ray_direction(lane_ctx, x, &cc.rx, &cc.ry);
     PixelBuffers pb;
     pb.frame = frame_base;
-    pb.meta = sc.meta; pb.clip_depth = sc.clip_depth;
+    pb.meta = sc.meta; pb.masked_texel = sc.masked_texel;
     pb.scene_depth = DEPTH ? sc.scene_depth : nullptr;
     pb.word_column = ((unsigned)local * (VH * SW) + (unsigned)x) * 4u;
+    pb.words = __builtin_amdgcn_make_buffer_rsrc(sc.meta, 0, lane_count * (VH * SW * 4), BUFFER_WORDS);
+    pb.depths = __builtin_amdgcn_make_buffer_rsrc(pb.scene_depth, 0, DEPTH ? lane_count * (VH * SW * 4) : 0, BUFFER_WORDS);
     pb.frame_column = (unsigned)local * (unsigned)frame_stride + (unsigned)x;
     // the meta plane arrives with whatever the last frame left: see GapRange for how every row gets written
     ColumnState st;   // only the clips and the masked-drawseg snapshot live here; the traversal state stayed in wall_select_kernel
@@ -3380,27 +3666,42 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
     SilhouetteBounds sb; sb.bot_row = VH; sb.top_row = 0; sb.bot_depth = -GD_INF; sb.top_depth = -GD_INF;
     const int passes = sc.pass_count[(size_t)local * SW + x];
-    const PassRec *records = sc.pass_rec + ((size_t)local * sc.pass_slots * SW + x);
-    const float *path_distances = sc.pass_path_distance + ((size_t)local * sc.pass_slots * SW + x);
-    PassColumn pc;
-    pc.wall = 0; pc.side = 0; pc.bits = 0; pc.visibility = 0;
-    pc.clipped_top = 0.0f; pc.clipped_bottom = 0.0f; pc.clipped_upper_bottom = 0.0f; pc.clipped_lower_top = 0.0f;
+    const size_t first_record = sc.pass_at(0, local, x), pass_stride = (size_t)sc.lane_stride * SW;
+    const unsigned int *geo_slots = sc.geo_slot + cc.rec_base;
+    // A pass's record names its linedef, the linedef's slot where it lies in geo: the next pass's slot and the record after it
+    // are asked for a pass ahead.  (Columns past their last pass keep asking for their first one.)
+    PassRec record = {}, next_record = {};
+    unsigned int slot = 0u, slot_wall = 0u;      // a pass that draws nothing names no linedef: the slot of the last one asked for will do
+    if (passes > 0) {
+        record = sc.pass_rec[first_record]; next_record = sc.pass_rec[first_record + (passes > 1 ? pass_stride : (size_t)0)];
+        slot_wall = record.bits ? record.wall : 0u;
+        slot = geo_slots[slot_wall];
+    }
     for (int pass = 0; __ballot(pass < passes) != 0; ++pass) {
         const bool mine = pass < passes;
         bool draws = false;
+        PassColumn pc = {};   // a finished column, or one whose pass draws nothing, paints no row and draws no tier: its group of four has no common tail
         if (mine) {
-            const PassRec rec = records[(size_t)pass * SW];
+            const PassRec rec = record;
+            const unsigned int geo_at = slot;
+            const size_t at = first_record + (size_t)pass * pass_stride;
+            record = next_record;
+            slot_wall = record.bits ? record.wall : slot_wall;
+            slot = geo_slots[slot_wall];
+            next_record = sc.pass_rec[pass + 2 < passes ? at + 2 * pass_stride : first_record];
             draws = (rec.bits & (PB_RASTER | PB_PS_KEEPS)) != 0;
             pc.bits = draws ? (int)rec.bits : 0;
             if (draws) {
                 pc.wall = rec.wall; pc.render_current = rec.render_current; pc.distance = rec.distance;
-                pc.ps_path_index = rec.ps_path; pc.ps_other = rec.ps_other;
-                pc.ps_path_distance = (rec.bits & PB_PS_KEEPS) ? path_distances[(size_t)pass * SW] : 0.0f;
-                pass_geometry<SPLIT>(cc, pc);
+                pc.ps_path_index = rec.ps_path; pc.ps_other = rec.ps_other; pc.marks = rec.marks;
+                PassTexture texture;
+                pass_geometry<GENERAL>(dm, cc, sc, sc.geo[geo_at], at, rec.marks, pc, texture);
                 pass_clip(cc, st.ceiling_clip, st.floor_clip, pc);
+                if (pc.bits & (PB_TIER0 | PB_TIER1 | PB_TIER2)) {
+                    texture_column(texture.ends, texture.past_left, texture.side, pc.side, x, &pc.u_base, &pc.swall);
+                    pc.offset_y = texture.side.offset_y; pc.fake_contrast = texture.side.contrast;
+                }
             }
-        } else {
-            pc.bits = 0;   // a finished column draws no tier: its group of four has no common tail
         }
         // 4-column wallscan groups (engine.py:12688-12761): the aligned group of four columns agrees on its drawseg, on
         // which tiers all four draw and on the rows all four share.  The four lanes of a group are one DPP quad, so every
@@ -3419,14 +3720,14 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
         group_valid[0] = same_group && (agreed & PB_TIER0) && (shared_top < shared_bottom);
         group_valid[1] = same_group && (agreed & PB_TIER1) && (shared_lower_top < shared_bottom);
         group_valid[2] = same_group && (agreed & PB_TIER2) && (shared_top < shared_upper_bottom);
+        pass_paint<DEPTH>(cc, st, pc, pb, group_valid, common_bottom, first_group_visibility, colormap_lds, window_dirty, gaps);
         if (draws) {
-            pass_paint<DEPTH>(cc, st, pc, pb, group_valid, common_bottom, first_group_visibility, colormap_lds, window_dirty, gaps);
-            pass_advance<SPLIT, ADVANCE_CLIPS>(cc, st, pc, pb, sb, !window_dirty, gaps);
+            pass_advance<GENERAL, ADVANCE_CLIPS>(cc, st, pc, pb, sb, !window_dirty, gaps, &sc, first_record + (size_t)pass * pass_stride);
         }
     }
     // what is left of a window no one-sided drawseg closed shows the flat pass's picture
     if (!window_dirty) zero_rows(pb, gaps, x, st.ceiling_clip <= 0.0f ? 0 : (int)st.ceiling_clip, st.floor_clip >= (float)VH ? VH : (int)st.floor_clip);
-    masked_midtexture<DEPTH, SPLIT>(cc, st, pb, colormap_lds);
+    if (dm.masked_count > 0) masked_midtexture<DEPTH, GENERAL>(dm, cc, sc, local, st, pb, colormap_lds);
     // The columns with view pixels that no wall tier, plane or masked texture covers join the flat pass's work list, those of a
     // wavefront in one piece (flat_gap_kernel selects the pixels, flat_shade_kernel paints them).
     bool holds_gap = false;
@@ -4424,7 +4725,7 @@ __global__ void __launch_bounds__(BAND_THREADS) __attribute__((amdgpu_waves_per_
             const int x = j * 64 + lane_id;
             const int ps = (int)((meta[j] >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1;
             unsigned char colour;
-            if (meta[j] & META_MASKED) colour = (unsigned char)__float_as_uint(sc.clip_depth[row_at + x]);   // left there by masked_midtexture
+            if (meta[j] & META_MASKED) colour = sc.masked_texel[row_at + x];   // left there by masked_midtexture
             else if (meta[j] & META_FILLED) colour = (unsigned char)(meta[j] >> META_SECTOR_SHIFT);
             else if (shade[j]) colour = colormap_lds[colormap_row[j] * 256 + texel[j]];
             else if (ps >= 0) colour = flat_pixel(tb, colormap_lds, L, ps, (meta[j] & META_FLOOR) != 0, x, y);
@@ -4853,7 +5154,7 @@ size_t spill_pool_blocks(int lanes) {
 // 256-byte aligned) and return the bytes the layout takes; with a null `base` nothing is assigned and the call
 // only measures.  `status` is not part of the block: the renderer keeps it.  `depth`: also the scene depth plane
 // of frames that draw decals.
-size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_desc &h, bool depth, size_t spill_blocks) {
+size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_desc &h, int masked_count, bool depth, size_t spill_blocks) {
     // `depth`: frames that draw decals also need a scene depth plane
     size_t used = 0;
     auto take = [&](auto **field, size_t count) {
@@ -4866,6 +5167,14 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.ctx, L);
     take(&sc.rec, L * W);
     take(&sc.span, L * W);
+    take(&sc.geo, L * W);
+    take(&sc.geo_count, 1);
+    take(&sc.geo_slot, L * W);
+    take(&sc.named, L * ((W + 31) / 32));
+    take(&sc.own_rows, L);
+    sc.lane_stride = (int)L;
+    take(&sc.masked_geo, L * (size_t)masked_count);
+    take(&sc.masked_hit, L * SW);
     take(&sc.frag_rec, L * (size_t)(h.split_count > 0 ? h.split_count * h.fragment_slots : 1));
     take(&sc.cand, L * CAND_MAX * SW + spill_blocks * SPILL_DEPTH * SW);   // byte offsets into it are 32 bits wide: L <= 4096, spill_blocks <= 512
     sc.spill_base = (unsigned)(L * CAND_MAX * SW); sc.spill_slots = (int)(spill_blocks * SW);
@@ -4885,9 +5194,10 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     sc.pass_slots = h.sector_count < 16 ? 16 : (h.sector_count > PASS_MAX ? PASS_MAX : h.sector_count);
     take(&sc.pass_rec, L * (size_t)sc.pass_slots * SW);
     take(&sc.pass_path_distance, L * (size_t)sc.pass_slots * SW);
+    take(&sc.pass_rows, L * (size_t)sc.pass_slots * SW);
     take(&sc.pass_count, L * SW);
     take(&sc.meta, L * PX);
-    take(&sc.clip_depth, L * PX);
+    take(&sc.masked_texel, L * PX);
     take(&sc.level_reach, L * levels);
     take(&sc.level_far, L * levels);
     take(&sc.level_masks, L * LEVEL_BUCKETS * (size_t)(levels <= 32 * LEVEL_MASK_WORDS_MAX ? (levels + 31) / 32 : 1));
@@ -5100,9 +5410,11 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
             hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0);
         }
         mark();
+        hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(count), dim3(SW), 0, stream, r->dm, count, sc);
         const dim3 grid((wavefronts + WALL_STRIPS_PER_GROUP - 1) / WALL_STRIPS_PER_GROUP), block(64 * WALL_STRIPS_PER_GROUP);
-        auto kernel = decals ? (split ? wall_raster_kernel<true, true> : wall_raster_kernel<true, false>)
-                             : (split ? wall_raster_kernel<false, true> : wall_raster_kernel<false, false>);
+        const bool general = split || m.sector_count > LDS_SECTORS || m.texture_count > LDS_TEXTURES;
+        auto kernel = decals ? (general ? wall_raster_kernel<true, true> : wall_raster_kernel<true, false>)
+                             : (general ? wall_raster_kernel<false, true> : wall_raster_kernel<false, false>);
         hipLaunchKernelGGL(kernel, grid, block, 0, stream, r->dm, count, sc, frame_base, frame_stride);
     }
     mark();
@@ -5325,6 +5637,26 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
             if (blocking_slot[w] < 0) blocking_slot[w] = b;   // the first slot wins ties, like the scan it replaces
         }
         if (rc == GD_OK) rc = upload(r, blocking_slot.data(), blocking_slot.size(), &r->dm.wall_blocking_slot);
+        std::vector<WallSide> sides(W * 2);
+        std::vector<int> masked_slot(W, -1);
+        r->dm.masked_count = 0;
+        for (size_t w = 0; w < W; ++w) {
+            const float *l = h->walls + 4 * w;
+            const bool horizontal = std::fabs(l[3] - l[1]) < 1e-6f, vertical = std::fabs(l[2] - l[0]) < 1e-6f;
+            for (int side = 0; side < 2; ++side) {
+                WallSide &ws = sides[w * 2 + side];
+                std::memset(&ws, 0, sizeof(ws));
+                for (int t = 0; t < 3; ++t) ws.tex[t] = h->side_tex[(w * 2 + side) * 3 + t];
+                ws.other = (short)h->wall_sectors[2 * w + (side == 0 ? 1 : 0)];
+                ws.offset_x = (i64)std::rint(h->side_off[(w * 2 + side) * 2] * 65536.0f);
+                ws.offset_y = h->side_off[(w * 2 + side) * 2 + 1];
+                ws.contrast = vertical ? 16.0f : (horizontal ? -16.0f : 0.0f);
+                ws.repeat = (i64)std::rint(h->wall_len[w] * 65536.0f);
+                if (h->wall_sectors[2 * w + 1] >= 0 && ws.tex[0] >= 0 && masked_slot[w] < 0) masked_slot[w] = r->dm.masked_count++;
+            }
+        }
+        if (rc == GD_OK) rc = upload(r, sides.data(), sides.size(), &r->dm.wall_side);
+        if (rc == GD_OK) rc = upload(r, masked_slot.data(), masked_slot.size(), &r->dm.masked_slot);
         r->dm.sector_level = nullptr;
         std::vector<unsigned int> pairs(S, 0);
         bool listed = h->floor_level_count <= 65535 && h->ceil_level_count <= 65535;
@@ -5368,10 +5700,10 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
     Scratch &sc = r->sc;
     if (rc == GD_OK && chunk > 0) {
         unsigned char *block = nullptr;
-        const size_t bytes = carve_scratch(sc, nullptr, (size_t)chunk, *h, false, spill_pool_blocks(chunk));
+        const size_t bytes = carve_scratch(sc, nullptr, (size_t)chunk, *h, r->dm.masked_count, false, spill_pool_blocks(chunk));
         rc = scratch_alloc(r, bytes, &block);
         if (rc == GD_OK) {
-            carve_scratch(sc, block, (size_t)chunk, *h, false, spill_pool_blocks(chunk));
+            carve_scratch(sc, block, (size_t)chunk, *h, r->dm.masked_count, false, spill_pool_blocks(chunk));
             r->scratch_block = block; r->scratch_bytes = bytes;
         }
     }
@@ -5448,17 +5780,17 @@ int gd_render_static(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_
     const gd_map_desc &m = r->dm.d;
     const bool decals = lanes->decal_slots > 0 && lanes->decal_state && lanes->decal_geom && r->overlays.d.decal_variant_count > 0;
     Scratch sc = r->sc;   // keeps the renderer's status word
-    const size_t one = carve_scratch(sc, nullptr, 1, m, decals, STATIC_SPILL_BLOCKS), two = carve_scratch(sc, nullptr, 2, m, decals, STATIC_SPILL_BLOCKS);
+    const size_t one = carve_scratch(sc, nullptr, 1, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS), two = carve_scratch(sc, nullptr, 2, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS);
     if (one > STATIC_SCRATCH_BYTES)
         return fail(GD_E_ARG, "map too large for gd_render_static: one lane needs " + std::to_string(one) + " bytes of working memory, the static block holds " +
                                   std::to_string(STATIC_SCRATCH_BYTES));
     // the layout grows by a fixed amount per lane, up to the padding between its buffers
     size_t fit = 1 + (STATIC_SCRATCH_BYTES - one) / (two - one);
-    while (fit > 1 && carve_scratch(sc, nullptr, fit, m, decals, STATIC_SPILL_BLOCKS) > STATIC_SCRATCH_BYTES) --fit;
+    while (fit > 1 && carve_scratch(sc, nullptr, fit, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS) > STATIC_SCRATCH_BYTES) --fit;
     const int chunk = fit > 4096 ? 4096 : (int)fit;
     if (lanes->lane_count > GD_STATIC_MAX_LANES)
         return fail(GD_E_ARG, "gd_render_static renders at most " + std::to_string(GD_STATIC_MAX_LANES) + " lanes per call");
-    carve_scratch(sc, block, (size_t)chunk, m, decals, STATIC_SPILL_BLOCKS);
+    carve_scratch(sc, block, (size_t)chunk, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS);
     hipStream_t caller = static_cast<hipStream_t>(stream);
     // the block keeps whatever the last call left: the kernels expect nothing of it
     for (int base = 0; base < lanes->lane_count; base += chunk) {
