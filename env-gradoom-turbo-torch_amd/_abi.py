@@ -391,3 +391,18 @@ class WeaponDesc(_Sized):
         + [(name, _P) for name in WEAPON_INPUTS + WEAPON_TABLES]
         + [("weapon_state", _P), ("flash_light", _P)]
     )
+
+
+POSE_LANE_FIELDS = ("x", "y", "angle", "view_z", "x_fixed", "y_fixed", "angle_bam", "pitch_bam", "flash_light")
+POSE_SPRITE_FIELDS = ("sprite_x", "sprite_y", "sprite_z", "sprite_id", "sprite_alive", "sprite_fullbright")
+POSE_POOL_FIELDS = ("x", "y", "view_z", "angle_bam", "pitch_bam", "flash_light") + POSE_SPRITE_FIELDS
+
+
+class PoseDesc(_Sized):
+    """``gd_pose_desc``: a pool of poses, which of them each lane shows, and the lane tensors ``gd_pose_lanes`` writes."""
+
+    _fields_ = (
+        [("struct_size", C.c_uint32), ("lane_count", C.c_int32), ("sprite_slots", C.c_int32), ("pool_size", C.c_int32), ("phase", _P), ("rows", _P)]
+        + [("pool_" + name, _P) for name in POSE_POOL_FIELDS]
+        + [(name, _P) for name in POSE_LANE_FIELDS + POSE_SPRITE_FIELDS]
+    )

@@ -6,7 +6,7 @@ import os
 import subprocess
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = [os.path.join(HERE, "csrc", "gd_render.hip")]
+SOURCES = [os.path.join(HERE, "csrc", name) for name in ("gd_render.hip", "gd_env.hip")]
 LIBRARY = os.path.join(HERE, "libgradoom_amd.so")
 
 # -ffp-contract=off: the reference evaluates float32 expressions one rounded op at a time.
@@ -28,8 +28,8 @@ def needs_build() -> bool:
     if not os.path.exists(LIBRARY):
         return True
     built = os.path.getmtime(LIBRARY)
-    header = os.path.join(os.path.dirname(HERE), "include", "gradoom_amd.h")
-    return any(os.path.getmtime(path) > built for path in SOURCES + [header])
+    headers = [os.path.join(os.path.dirname(HERE), "include", "gradoom_amd.h"), os.path.join(HERE, "csrc", "gd_internal.h")]
+    return any(os.path.getmtime(path) > built for path in SOURCES + headers)
 
 
 def build_library(force: bool = False) -> str:

@@ -31,6 +31,13 @@ SYMBOLS = (
     "gd_pack_weapon",
     "gd_ray_tables",
     "gd_sprite_depth",
+    "gd_pose_lanes",
+    "gd_pose_step",
+    "gd_pose_reset",
+    "gd_env_step",
+    "gd_env_reset",
+    "gd_env_check",
+    "gd_fill_stacks",
 )
 
 _LIBRARY = None
@@ -90,6 +97,17 @@ def library() -> C.CDLL:
     lib.gd_ray_tables.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.gd_sprite_depth.restype = C.c_int
     lib.gd_sprite_depth.argtypes = [C.c_void_p] * 5 + [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p]
+    for name, arguments in (
+        ("gd_pose_lanes", [C.POINTER(_abi.PoseDesc), C.c_void_p]),
+        ("gd_pose_step", [C.c_void_p] * 3 + [C.c_int32, C.c_int64, C.c_int64] + [C.c_void_p] * 4),
+        ("gd_pose_reset", [C.c_void_p] * 4 + [C.c_int32, C.c_int64, C.c_void_p]),
+        ("gd_env_step", [C.c_void_p] * 3 + [C.c_int32] + [C.c_void_p] * 5),
+        ("gd_env_reset", [C.c_void_p] * 3 + [C.c_int32] + [C.c_void_p] * 5),
+        ("gd_env_check", [C.c_void_p] * 3 + [C.c_int32, C.c_int32] + [C.c_void_p] * 2),
+        ("gd_fill_stacks", [C.c_void_p] * 2 + [C.c_int32] + [C.c_void_p] * 2),
+    ):
+        function = getattr(lib, name)
+        function.restype, function.argtypes = C.c_int, arguments
     _LIBRARY = lib
     return lib
 

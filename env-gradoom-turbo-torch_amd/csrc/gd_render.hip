@@ -42,6 +42,10 @@
 #include <vector>
 
 #include "../../include/gradoom_amd.h"
+#include "gd_internal.h"
+
+thread_local std::string g_error;
+int gd_fail(int code, const std::string &message) { g_error = message; return code; }
 
 namespace {
 
@@ -274,7 +278,7 @@ struct Scratch {    // per-chunk working memory, sized at create
                            // lane_tables_kernel says; launch_chunk's two billboard launches split the lanes by it
     unsigned char *strip_key;  // [L*SEGS_PER_LANE] expected traversal length of each (lane, segment of SEG_COLS columns)
     int *strip_order;      // [L*SEGS_PER_LANE] segments, longest expected traversal first
-    int *status;           // [1] sticky overflow flags
+    volatile unsigned char *status;   // [2] sticky flags in pinned host memory: a candidate list, a list of passes was cut short
     float *level_reach;    // [L, floor levels + ceiling levels] lower bound of the distance from the
                            // camera to any point inside a sector with that plane level
     float *level_far;      // [L, floor levels + ceiling levels] upper bound of that distance
@@ -305,8 +309,8 @@ struct Scratch {    // per-chunk working memory, sized at create
 // Does the view pixel with this word show the flat pass's picture: no wall tier, no plane, no masked texture?
 __device__ __forceinline__ bool gap_pixel(unsigned int word) { return !(word & (META_FILLED | META_MASKED)) && ((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) == 0; }
 
-#define STATUS_CAND_OVERFLOW 1
-#define STATUS_PASS_OVERFLOW 2
+#define STATUS_CAND_OVERFLOW 0
+#define STATUS_PASS_OVERFLOW 1
 __device__ __forceinline__ int named_words(const gd_map_desc *m) { return (m->wall_count + 31) / 32; }
 #define STEP_TABLE 96   // int64 entries per lane of Scratch::step_scale
 
@@ -758,7 +762,7 @@ __global__ void fragment_setup_kernel(DeviceMap dm, int lane_count, Scratch sc) 
 __device__ __forceinline__ void request_spill_slot(const Scratch &sc, int column) {
     const int slot = atomicAdd(sc.spill_count, 1);
     if (slot < sc.spill_slots) sc.spill_columns[slot] = column;
-    else atomicOr(sc.status, STATUS_CAND_OVERFLOW);
+    else sc.status[STATUS_CAND_OVERFLOW] = 1;
 }
 
 // One thread owns one linedef for the per-linedef arithmetic.  The two per-column loops have
@@ -1082,7 +1086,7 @@ __global__ void __launch_bounds__(64) cand_spill_kernel(DeviceMap dm, Scratch sc
             const int position = listed + __popcll(keeps & ((1ULL << threadIdx.x) - 1ULL));
             if (keep) {
                 if (position < SPILL_DEPTH) list[(size_t)position * SW] = entry;
-                else atomicOr(sc.status, STATUS_CAND_OVERFLOW);
+                else sc.status[STATUS_CAND_OVERFLOW] = 1;
             }
             listed += __popcll(keeps);
         }
@@ -3363,7 +3367,8 @@ __device__ __forceinline__ void wall_lines(const DeviceMap &dm, const LaneCtx &c
 // The linedefs that the recorded passes of a lane draw, each worked out once (WallGeo) for all the columns and passes that draw it.
 // The drawing half used to do this per column and pass: some 25 64-bit divisions, two thirds of its instructions, for what is
 // the same in every column of a linedef.  One work-group per lane: it turns the bits wall_select_kernel left into a list, takes as many
-// slots of geo, and gives four threads to a linedef (one a height; the wallscan light's four ends likewise).
+// slots of geo, and gives four threads to a linedef (one a height; the wallscan light's four ends likewise).  4096 lanes on the
+// 4000-linedef map draw 1.3 million linedefs: 0.33 ms here, 0.3 ms off wall_raster_kernel.
 #define GEO_LIST 1024                            // linedefs listed at a time
 template <bool SPLIT>
 __global__ void __launch_bounds__(SW) wall_geometry_kernel(DeviceMap dm, int lane_count, Scratch sc) {
@@ -3595,7 +3600,7 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
                     if (pc.marks & REC_OWN_ROWS) atomicOr(&sc.own_rows[local], 1u << (x >> 6));
                     recorded = pass + 1;
                 } else {
-                    atomicOr(sc.status, STATUS_PASS_OVERFLOW);
+                    sc.status[STATUS_PASS_OVERFLOW] = 1;
                 }
             }
             const bool changed = pass_advance<SPLIT, ADVANCE_STATE>(cc, st, pc, no_pixels, no_bounds, false, no_gaps);
@@ -3616,6 +3621,9 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
 // DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
 // BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
+// 4096 lanes on the 4000-linedef map: 1.78 -> 1.00 ms (with wall_geometry_kernel 1.33): the linedefs' lines 1.53, no sprite clip plane
+// and the rows walked together 1.33, no branch around a load or a store 1.03.  It is left at four wavefronts a SIMD (128 registers, four
+// of them spilled; at 96 registers the spills in the row loops make it 1.6 ms), 55 % of their cycles waiting.
 template <bool DEPTH, bool GENERAL>
 __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(RASTER_WAVES, RASTER_WAVES))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
@@ -4431,17 +4439,6 @@ __device__ __forceinline__ unsigned char blended_channel(unsigned char value, in
     return (unsigned char)fminf(fmaxf(v, 0.0f), 255.0f);
 }
 
-// `blend` points at the first lane's (bonus, damage) alphas, or is null for plain PLAYPAL colours.
-__device__ __forceinline__ void stage_palette(unsigned char *pal, const unsigned char *playpal, const float *blend, int lane) {
-    if (blend) {
-        const float bonus = blend[2 * lane], flash = blend[2 * lane + 1];
-        for (int k = threadIdx.x; k < 768; k += blockDim.x) pal[k] = blended_channel(playpal[k], k % 3, bonus, flash);
-    } else {
-        for (int k = threadIdx.x; k < 768; k += blockDim.x) pal[k] = playpal[k];
-    }
-    __syncthreads();
-}
-
 // The frame stack of one lane, four pixels (one word per stacked observation) at a time: what the stack holds after
 // this call goes to `stack` (when it changes) and to the caller's copy, which is laid out either like the stack
 // ([4][84][84]) or with the four stacked values of a pixel next to each other ([84][84][4]).
@@ -4598,16 +4595,54 @@ __global__ void __launch_bounds__(256) observe_kernel(const unsigned char *index
                                  final_hwc, stack_aligned, word, kept, grays, resets, stack_mode);
 }
 
-// engine.py:15381-15384
-// A block of 256 pixels never straddles two lanes when lane_pixels is a multiple of 256 (240 x 320 is).
-__global__ void expand_rgb_kernel(const unsigned char *indexed, const unsigned char *playpal, size_t pixels, unsigned char *rgb,
-                                  const float *blend, size_t lane_pixels) {
-    __shared__ unsigned char pal[768];
-    stage_palette(pal, playpal, blend, blend ? (int)(((size_t)blockIdx.x * blockDim.x) / lane_pixels) : 0);
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= pixels) return;
-    int p = indexed[i] * 3;
-    rgb[i * 3] = pal[p]; rgb[i * 3 + 1] = pal[p + 1]; rgb[i * 3 + 2] = pal[p + 2];
+// engine.py:15381-15384: PLAYPAL expansion.  A thread takes sixteen pixels: one 16-byte load, sixteen palette words from LDS; the 48 bytes
+// they make go through LDS, so that every store of a wavefront is a kilobyte of one piece (which host memory over PCIe asks for
+// even more than device memory does: viewers have their frames expanded straight into pinned host memory).  512 lanes: bytes stored
+// three apart took 0.123 ms, four times what the copy of as many bytes takes.
+#define EXPAND_THREADS 192       // 3072 pixels: 25 blocks are exactly a lane's frame, so a block has one palette
+#define EXPAND_PIXELS (EXPAND_THREADS * 16)
+static_assert((GD_SCREEN_HEIGHT * SW) % EXPAND_PIXELS == 0, "expand_rgb_kernel: one lane per block");
+__global__ void __launch_bounds__(EXPAND_THREADS) expand_rgb_kernel(const unsigned char *indexed, const unsigned char *playpal, size_t pixels, unsigned char *rgb,
+                                                                    const float *blend, size_t lane_pixels) {
+    __shared__ unsigned int pal[256];
+    __shared__ __align__(16) unsigned int staged[EXPAND_THREADS / 64][64 * 12];
+    const size_t block_first = (size_t)blockIdx.x * EXPAND_PIXELS;
+    const int lane = blend ? (int)(block_first / lane_pixels) : 0;
+    for (int k = threadIdx.x; k < 256; k += EXPAND_THREADS) {
+        unsigned int r = playpal[3 * k], g = playpal[3 * k + 1], b = playpal[3 * k + 2];
+        if (blend) {
+            const float bonus = blend[2 * lane], flash = blend[2 * lane + 1];
+            r = blended_channel((unsigned char)r, 0, bonus, flash); g = blended_channel((unsigned char)g, 1, bonus, flash); b = blended_channel((unsigned char)b, 2, bonus, flash);
+        }
+        pal[k] = r | (g << 8) | (b << 16);
+    }
+    __syncthreads();
+    const size_t first = block_first + (size_t)threadIdx.x * 16;     // pixel counts are whole rows: a thread has all its sixteen or none
+    const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63;
+    const bool aligned = ((reinterpret_cast<size_t>(indexed) | reinterpret_cast<size_t>(rgb)) & 15) == 0;
+    if (!aligned) {
+        if (first < pixels) for (int k = 0; k < 16; ++k) {
+            const unsigned int c = pal[indexed[first + k]];
+            rgb[(first + k) * 3] = (unsigned char)c; rgb[(first + k) * 3 + 1] = (unsigned char)(c >> 8); rgb[(first + k) * 3 + 2] = (unsigned char)(c >> 16);
+        }
+        return;
+    }
+    uint4 four = make_uint4(0u, 0u, 0u, 0u);
+    if (first < pixels) four = *reinterpret_cast<const uint4 *>(indexed + first);
+    const unsigned int words[4] = {four.x, four.y, four.z, four.w};
+    unsigned int *mine = staged[wave] + lane_id * 12;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {   // four pixels, twelve bytes, three words
+        const unsigned int c0 = pal[words[j] & 255u], c1 = pal[(words[j] >> 8) & 255u], c2 = pal[(words[j] >> 16) & 255u], c3 = pal[words[j] >> 24];
+        mine[3 * j] = c0 | (c1 << 24); mine[3 * j + 1] = (c1 >> 8) | (c2 << 16); mine[3 * j + 2] = (c2 >> 16) | (c3 << 8);
+    }
+    wave_lds_fence();
+    const size_t wave_bytes = (block_first + (size_t)wave * 1024) * 3, end = pixels * 3;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int at = j * 64 + lane_id;
+        if (wave_bytes + (size_t)at * 16 < end) *reinterpret_cast<uint4 *>(rgb + wave_bytes + (size_t)at * 16) = reinterpret_cast<const uint4 *>(staged[wave])[at];
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -5006,9 +5041,7 @@ __global__ void __launch_bounds__(64) pack_actors_kernel(gd_actor_desc a, int wi
 // ---------------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------------
-thread_local std::string g_error;
-
-int fail(int code, const std::string &message) { g_error = message; return code; }
+int fail(int code, const std::string &message) { return gd_fail(code, message); }
 
 // gd_pack_weapon: one thread per lane.  Which patch the player's weapon shows and where (engine.py:14949-14967,
 // 15051-15092): the frame table is indexed by weapon, by a parity that alternates with every shot (an idling chainsaw
@@ -5045,19 +5078,8 @@ __global__ void __launch_bounds__(64) pack_weapon_kernel(gd_weapon_desc d) {
     if (d.flash_light) d.flash_light[lane] = d.weapon_flash_lights[entry];
 }
 
-#define HIP_TRY(expr)                                                                          \
-    do {                                                                                       \
-        hipError_t e_ = (expr);                                                                \
-        if (e_ != hipSuccess) return fail(GD_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
-    } while (0)
-
-// A descriptor filled in against another version of the header is refused before any of its fields is trusted.
-#define SIZE_CHECK(ptr, type)                                                                  \
-    do {                                                                                       \
-        if ((ptr)->struct_size != sizeof(type))                                                \
-            return fail(GD_E_ARG, #type ".struct_size is " + std::to_string((ptr)->struct_size) + ", this library expects " + \
-                                      std::to_string(sizeof(type)) + ": the caller was built against another gradoom_amd.h"); \
-    } while (0)
+#define HIP_TRY GD_HIP_TRY
+#define SIZE_CHECK GD_SIZE_CHECK
 
 }  // namespace
 
@@ -5516,8 +5538,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     }
     if (out->rgb) {
         size_t pixels = (size_t)count * frame_stride;
-        static_assert((GD_SCREEN_HEIGHT * SW) % 256 == 0, "expand_rgb_kernel: one lane per block");
-        hipLaunchKernelGGL(expand_rgb_kernel, dim3((unsigned)((pixels + 255) / 256)), dim3(256), 0, stream, frame_base, m.playpal, pixels,
+        hipLaunchKernelGGL(expand_rgb_kernel, dim3((unsigned)((pixels + EXPAND_PIXELS - 1) / EXPAND_PIXELS)), dim3(EXPAND_THREADS), 0, stream, frame_base, m.playpal, pixels,
                            out->rgb + (size_t)base * frame_stride * 3, blend, (size_t)GD_SCREEN_HEIGHT * SW);
     }
     mark();
@@ -5707,8 +5728,12 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
             r->scratch_block = block; r->scratch_bytes = bytes;
         }
     }
-    if (rc == GD_OK) rc = scratch_alloc(r, 1, &sc.status);
-    if (rc == GD_OK && hipMemset(sc.status, 0, sizeof(int)) != hipSuccess) rc = fail(GD_E_HIP, "hipMemset status");
+    if (rc == GD_OK) {
+        // in host memory: asking for it then is a wait for the device, not a copy behind the wait as well
+        void *words = nullptr;
+        if (hipHostMalloc(&words, 64) != hipSuccess) rc = fail(GD_E_HIP, "hipHostMalloc status");
+        else { sc.status = static_cast<unsigned char *>(words); sc.status[0] = 0; sc.status[1] = 0; }
+    }
     if (rc == GD_OK) rc = static_scratch_address(nullptr);   // looked up once per device, outside any stream capture
     if (rc == GD_OK) {
         for (int i = 0; i < 16; ++i) if (hipEventCreate(&r->events[i]) != hipSuccess) rc = fail(GD_E_HIP, "hipEventCreate");
@@ -5731,6 +5756,7 @@ void gd_renderer_destroy(gd_renderer *r) {
     if (!r) return;
     for (void *ptr : r->allocations) (void)hipFree(ptr);
     for (void *ptr : r->overlay_allocations) (void)hipFree(ptr);
+    if (r->sc.status) (void)hipHostFree(const_cast<unsigned char *>(r->sc.status));
     if (r->events_ready) for (int i = 0; i < 16; ++i) (void)hipEventDestroy(r->events[i]);
     if (r->side_ready) { (void)hipEventDestroy(r->fork_event); (void)hipEventDestroy(r->join_event); (void)hipStreamDestroy(r->side_stream); }
     delete r;
@@ -5829,9 +5855,8 @@ int gd_render_timed(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_o
    CAND_MAX candidate linedefs and its list was truncated. Replaces nothing in the reference. */
 int gd_renderer_status(gd_renderer *r, int32_t *status) {
     if (!r || !status) return fail(GD_E_ARG, "null argument");
-    int value = 0;
-    HIP_TRY(hipMemcpy(&value, r->sc.status, sizeof(int), hipMemcpyDeviceToHost));
-    *status = value;
+    HIP_TRY(hipDeviceSynchronize());
+    *status = (r->sc.status[STATUS_CAND_OVERFLOW] ? 1 : 0) | (r->sc.status[STATUS_PASS_OVERFLOW] ? 2 : 0);
     return GD_OK;
 }
 
@@ -5946,10 +5971,10 @@ int gd_expand_rgb24(const uint8_t *indexed, int32_t rows, const uint8_t *playpal
     size_t pixels = (size_t)lane_count * rows * SW;
     if (pixels == 0) return GD_OK;        // an empty batch: its tensors may have no address
     if (!indexed || !playpal || !rgb) return fail(GD_E_ARG, "null argument");
-    const size_t step = (size_t)1 << 30;
+    const size_t step = (size_t)320 << 22;   // whole rows
     for (size_t base = 0; base < pixels; base += step) {
         size_t count = pixels - base < step ? pixels - base : step;
-        hipLaunchKernelGGL(expand_rgb_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
+        hipLaunchKernelGGL(expand_rgb_kernel, dim3((unsigned)((count + EXPAND_PIXELS - 1) / EXPAND_PIXELS)), dim3(EXPAND_THREADS), 0, static_cast<hipStream_t>(stream),
                            indexed + base, playpal, count, rgb + base * 3, nullptr, (size_t)1);
     }
     HIP_TRY(hipGetLastError());

@@ -21,6 +21,7 @@ three methods on top of its own state tensors.
 
 from __future__ import annotations
 
+import ctypes as C
 import dataclasses
 import operator
 from collections.abc import Sequence
@@ -28,7 +29,7 @@ from collections.abc import Sequence
 import numpy as np
 import torch
 
-from . import hostmath, synthmap
+from . import _abi, _lib, hostmath, synthmap
 from .renderer import HipRenderer, LaneState
 
 SIGNAL_COUNT = 27  # len(DEVICE_SIGNAL_NAMES), engine.py:509-539
@@ -69,8 +70,22 @@ def _normalize_seed(seed, num_envs: int):  # env.py:101-113
     return [int(seed) + lane for lane in range(num_envs)]
 
 
+def _stream(device) -> int:
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+def _kernel_ready(tensor, dtype, count: int, device) -> bool:
+    """Can a kernel of the library take this tensor as it is: ``count`` contiguous elements of ``dtype`` on ``device``?"""
+
+    return isinstance(tensor, torch.Tensor) and tensor.dtype is dtype and tensor.shape == (count,) and tensor.device == device and tensor.is_contiguous()
+
+
 class PosePoolDynamics:
-    """Deterministic lane state source: lane ``i`` at time ``t`` shows pose ``(seed_i + t) mod pool``."""
+    """Deterministic lane state source: lane ``i`` at time ``t`` shows pose ``(seed_i + t) mod pool``.
+
+    On a ROCm device a step, a reset and the lane state are one kernel each (``gd_pose_step``, ``gd_pose_reset``,
+    ``gd_pose_lanes``); elsewhere they are the Torch expressions below.
+    """
 
     def __init__(self, smap, num_envs: int, device, *, pool: int = 64, sprites: int = 0, episode_timeout: int = 32, seed: int = 0):
         self.device = torch.device(device)
@@ -95,11 +110,32 @@ class PosePoolDynamics:
         self.phase = torch.zeros(num_envs, dtype=torch.int64, device=self.device)
         self.episode_time = torch.zeros(num_envs, dtype=torch.int64, device=self.device)
 
+    def _on_device(self, *tensors) -> bool:
+        """Do the kernels take this call: the pool's own two counters and the call's tensors, each where and what it should be?"""
+
+        if self.device.type != "cuda":
+            return False
+        device, count = self.phase.device, self.num_envs
+        return (_kernel_ready(self.phase, torch.int64, count, device) and _kernel_ready(self.episode_time, torch.int64, count, device)
+                and all(_kernel_ready(tensor, dtype, count, device) for tensor, dtype in tensors))
+
     def reset(self, mask: torch.Tensor, seeds: torch.Tensor) -> None:
+        if self._on_device((mask, torch.bool), (seeds, torch.int64)):
+            with torch.cuda.device(self.device):
+                _lib.check(_lib.library().gd_pose_reset(self.phase.data_ptr(), self.episode_time.data_ptr(), mask.data_ptr(), seeds.data_ptr(), self.num_envs,
+                                                        self._pool_size, _stream(self.device)))
+            return
         self.phase.copy_(torch.where(mask, torch.remainder(seeds, self._pool_size), self.phase))
         self.episode_time.copy_(torch.where(mask, torch.zeros_like(self.episode_time), self.episode_time))
 
     def step(self, actions: torch.Tensor):
+        if self._on_device((actions, torch.int64)):
+            rewards = torch.empty(self.num_envs, dtype=torch.float32, device=self.device)
+            terminated, truncated = torch.empty((2, self.num_envs), dtype=torch.bool, device=self.device).unbind(0)
+            with torch.cuda.device(self.device):
+                _lib.check(_lib.library().gd_pose_step(self.phase.data_ptr(), self.episode_time.data_ptr(), actions.data_ptr(), self.num_envs, self._pool_size,
+                                                       self.episode_timeout, rewards.data_ptr(), terminated.data_ptr(), truncated.data_ptr(), _stream(self.device)))
+            return rewards, terminated, truncated
         self.phase.copy_(torch.remainder(self.phase + 1 + actions, self._pool_size))
         self.episode_time.add_(1)
         rewards = torch.zeros(self.num_envs, dtype=torch.float32, device=self.device)
@@ -107,9 +143,13 @@ class PosePoolDynamics:
         truncated = self.episode_time >= self.episode_timeout
         return rewards, terminated, truncated
 
-    def lane_state(self) -> LaneState:
-        index = self.phase
+    def lane_state(self, rows: torch.Tensor | None = None) -> LaneState:
+        """The lane state of every lane, or of the lanes that ``rows`` (int64, on the device) names."""
+
         pool = self._pool
+        if self._on_device() and all(value.is_contiguous() for value in pool.values()):
+            return self._lane_state_kernel(rows)
+        index = self.phase if rows is None else self.phase[rows]
         x, y = pool["x"][index], pool["y"][index]
         bam = pool["angle_bam"][index]
         fields = dict(
@@ -120,6 +160,32 @@ class PosePoolDynamics:
         if self._sprites is not None:
             fields.update({name: value[index].contiguous() for name, value in self._sprites.items()})
         return LaneState(**{name: value.contiguous() for name, value in fields.items()})
+
+    def _lane_state_kernel(self, rows) -> LaneState:
+        count = self.num_envs if rows is None else int(rows.shape[0])
+        device = self.device
+        desc = _abi.PoseDesc()
+        desc.lane_count, desc.pool_size, desc.phase = count, self._pool_size, self.phase.data_ptr()
+        if rows is not None:
+            desc.rows = rows.data_ptr()
+        pool = self._pool
+        for name in ("x", "y", "view_z", "angle_bam", "pitch_bam", "flash_light"):
+            setattr(desc, "pool_" + name, pool[name].data_ptr())
+        fields = dict(zip(("x", "y", "angle", "view_z"), torch.empty((4, count), dtype=torch.float32, device=device).unbind(0)))
+        fields.update(zip(("x_fixed", "y_fixed", "angle_bam", "pitch_bam", "flash_light"), torch.empty((5, count), dtype=torch.int64, device=device).unbind(0)))
+        if self._sprites is not None:
+            slots = int(self._sprites["sprite_x"].shape[1])
+            desc.sprite_slots = slots
+            for name, value in self._sprites.items():
+                setattr(desc, "pool_" + name, value.data_ptr())
+            fields.update(zip(("sprite_x", "sprite_y", "sprite_z"), torch.empty((3, count, slots), dtype=torch.float32, device=device).unbind(0)))
+            fields["sprite_id"] = torch.empty((count, slots), dtype=torch.int32, device=device)
+            fields.update(zip(("sprite_alive", "sprite_fullbright"), torch.empty((2, count, slots), dtype=torch.uint8, device=device).unbind(0)))
+        for name, value in fields.items():
+            setattr(desc, name, value.data_ptr())
+        with torch.cuda.device(device):
+            _lib.check(_lib.library().gd_pose_lanes(C.byref(desc), _stream(device)))
+        return LaneState(**fields)
 
 
 class GraDoomVecEnv:
@@ -184,7 +250,15 @@ class GraDoomVecEnv:
             tuple(torch.empty(view_shape, dtype=torch.uint8, device=self.device) for _ in range(2)) if obs_copy == "safe_view" else ()
         )
         self._safe_obs_index = 0
+        # What the host wants to know of a step (gd_env_step, gd_env_check), in pinned memory: the kernels write it, a wait on the
+        # stream makes it readable.
+        self._native = self.device.type == "cuda"
+        self._words = torch.zeros(16, dtype=torch.int32, pin_memory=True) if self._native else None
+        self._words_read = self._words.numpy() if self._native else None
+        self._done_rows = torch.zeros(n, dtype=torch.int64, device=self.device) if self._native else None
+        self._rgb_staging = None        # pinned, at most RGB_STAGING_BYTES
         self._seed_values = [None] * n
+        self._done_listed = False       # did the last step's kernel list the lanes that ended?
         self._deferred_actions = None   # the one-element tuple step_async leaves for step_wait
         self._reset_rngs = [np.random.default_rng() for _ in range(n)]
 
@@ -203,6 +277,14 @@ class GraDoomVecEnv:
 
     def _device_observations(self, observations: torch.Tensor) -> torch.Tensor:  # env.py:690-691
         return observations.permute(0, 2, 3, 1) if self.obs_layout == "hwc" else observations
+
+    def _bookkeeping_ready(self) -> bool:
+        """Are the tensors of a step's bookkeeping what the kernels take?  (A dynamics object may keep its clock in another type.)"""
+
+        return self._native and _kernel_ready(self._dynamics.episode_time, torch.int64, self.num_envs, self.frames.device)
+
+    def _wait(self) -> None:
+        torch.cuda.current_stream(self.device).synchronize()
 
     def _update_signals(self) -> None:
         self.signal_buffer[:, 17].copy_(self._dynamics.episode_time)  # episode_time, engine.py:15469
@@ -223,23 +305,61 @@ class GraDoomVecEnv:
         # writing only under the mask.
         self._renderer.render(self._dynamics.lane_state(), frames=self.frames, reset_mask=device_mask, obs=None, stack_only_masked=True,
                               final_frames=view, final_layout=self.obs_layout)
+        self._after_reset(device_mask, device_seeds)
+        return self._device_observations(self.frames), self.signal_buffer
+
+    def _after_reset(self, device_mask: torch.Tensor, device_seeds: torch.Tensor) -> None:
+        if self._bookkeeping_ready() and device_mask.is_contiguous() and device_seeds.is_contiguous():
+            with torch.cuda.device(self.device):
+                _lib.check(_lib.library().gd_env_reset(device_mask.data_ptr(), device_seeds.data_ptr(), self._dynamics.episode_time.data_ptr(), self.num_envs,
+                                                       self._latest_reset_seeds.data_ptr(), self._initialized.data_ptr(), self.pending_reset.data_ptr(),
+                                                       self.signal_buffer.data_ptr(), _stream(self.device)))
+            return
         self._latest_reset_seeds.copy_(torch.where(device_mask, device_seeds, self._latest_reset_seeds))
         self._initialized |= device_mask
         self.pending_reset.masked_fill_(device_mask, False)   # engine.py:2409
         self._update_signals()
+
+    def _reset_rows(self, device_mask: torch.Tensor, seeds: torch.Tensor, count: int):
+        """``_reset`` of the ``count`` lanes that ``_done_rows`` lists: only they are rendered, four copies each into their stacks."""
+
+        device_seeds = self._require_device_tensor(seeds, "seeds", shape=(self.num_envs,), dtypes=INDEX_DTYPES).to(torch.int64).contiguous()
+        self._dynamics.reset(device_mask, device_seeds)
+        rows = self._done_rows[:count]
+        state = self._dynamics.lane_state(rows) if isinstance(self._dynamics, PosePoolDynamics) else self._dynamics.lane_state().select(rows)
+        obs = torch.empty((count, 84, 84), dtype=torch.uint8, device=self.device)
+        self._renderer.render(state, obs=obs)
+        with torch.cuda.device(self.device):
+            _lib.check(_lib.library().gd_fill_stacks(obs.data_ptr(), rows.data_ptr(), count, self.frames.data_ptr(), _stream(self.device)))
+        self._after_reset(device_mask, device_seeds)
         return self._device_observations(self.frames), self.signal_buffer
 
     def step_device(self, actions: torch.Tensor) -> DeviceTransition:
         return self._step(actions, None)
 
-    def _step(self, actions: torch.Tensor, final_frames, final_layout: str = "chw") -> DeviceTransition:
+    def _after_step(self, terminated, truncated, list_done: bool) -> bool:
+        """The bookkeeping of a step in one kernel; false where its tensors are not what the kernel takes."""
+
+        device, count = self.frames.device, self.num_envs
+        if not (self._bookkeeping_ready() and _kernel_ready(terminated, torch.bool, count, device) and _kernel_ready(truncated, torch.bool, count, device)):
+            return False
+        with torch.cuda.device(self.device):
+            _lib.check(_lib.library().gd_env_step(terminated.data_ptr(), truncated.data_ptr(), self._dynamics.episode_time.data_ptr(), count,
+                                                  self.pending_reset.data_ptr(), self.signal_buffer.data_ptr(), self._done_rows.data_ptr() if list_done else None,
+                                                  self._words.data_ptr() if list_done else None, _stream(self.device)))
+        return True
+
+    def _step(self, actions: torch.Tensor, final_frames, final_layout: str = "chw", list_done: bool = False) -> DeviceTransition:
         if self.closed:
             raise RuntimeError("cannot step a closed environment")
         indices = self._require_device_tensor(actions, "actions", shape=(self.num_envs,), dtypes=INDEX_DTYPES).to(torch.int64)
         rewards, terminated, truncated = self._dynamics.step(indices)
-        self.pending_reset.copy_(terminated | truncated)      # engine.py:9542
+        self._done_listed = self._after_step(terminated, truncated, list_done)
+        if not self._done_listed:
+            self.pending_reset.copy_(terminated | truncated)      # engine.py:9542
         self._renderer.render(self._dynamics.lane_state(), frames=self.frames, final_frames=final_frames, final_layout=final_layout)
-        self._update_signals()
+        if not self._done_listed:
+            self._update_signals()
         return DeviceTransition(
             observations=self._device_observations(self.frames), rewards=rewards, terminated=terminated, truncated=truncated,
             signals=self.signal_buffer, info_histories=self._info_history,
@@ -248,19 +368,28 @@ class GraDoomVecEnv:
     def step_and_reset_device(self, actions: torch.Tensor, reset_seeds: torch.Tensor) -> DeviceAutoResetTransition:
         # the final-observation clone (env.py:915) is written by the observation kernel of the step
         final_frames = torch.empty_like(self.frames)
-        transition = self._step(actions, final_frames)
+        transition = self._step(actions, final_frames, list_done=True)
         final_observations = self._device_observations(final_frames)
         final_signals = transition.signals.clone()
         final_info_histories = transition.info_histories.clone()
-        done = transition.terminated | transition.truncated
-        any_done = bool(torch.any(done))  # env.py:919: one host sync for the reference renderer
+        listed = self._done_listed
+        if listed:   # how many lanes ended came with the step: one wait on the stream
+            self._wait()
+            done_count = int(self._words_read[0])
+        else:
+            done = transition.terminated | transition.truncated
+            done_count = int(torch.count_nonzero(done))  # env.py:919: one host sync for the reference renderer
         self.check_renderer_status()      # the device is idle here anyway
-        if not any_done:
+        if not done_count:
             return DeviceAutoResetTransition(
                 transition.observations, transition.rewards, transition.terminated, transition.truncated,
                 transition.signals, transition.info_histories, final_observations, final_signals, final_info_histories,
             )
-        observations, signals = self.reset_device(done, reset_seeds)
+        if listed and done_count <= 65535:
+            observations, signals = self._reset_rows(self.pending_reset.clone(), reset_seeds, done_count)
+        else:
+            done = transition.terminated | transition.truncated
+            observations, signals = self.reset_device(done, reset_seeds)
         return DeviceAutoResetTransition(
             observations, transition.rewards, transition.terminated, transition.truncated, signals, self._info_history,
             final_observations, final_signals, final_info_histories,
@@ -332,18 +461,32 @@ class GraDoomVecEnv:
         observations, _ = self._reset(mask, seeds, view)
         return (observations if view is None else view), {}
 
+    def _check_step(self, actions):
+        """(some lane was never reset, some lane has ended, some action is out of range); the last None where that was not looked at."""
+
+        if not self._native:
+            return not bool(torch.all(self._initialized)), bool(torch.any(self.pending_reset)), None
+        looked_at = _kernel_ready(actions, torch.int64, self.num_envs, self.frames.device)
+        with torch.cuda.device(self.device):
+            _lib.check(_lib.library().gd_env_check(self._initialized.data_ptr(), self.pending_reset.data_ptr(), actions.data_ptr() if looked_at else None,
+                                                   self.num_envs, self.action_count, self._words.data_ptr() + 4, _stream(self.device)))
+        self._wait()
+        flags = int(self._words_read[1])
+        return bool(flags & 1), bool(flags & 2), bool(flags & 4) if looked_at else None
+
     def step(self, actions: torch.Tensor):
         if self.closed:
             raise RuntimeError("cannot step a closed environment")
-        if not bool(torch.all(self._initialized)):
+        uninitialized, pending, outside = self._check_step(actions)
+        if uninitialized:
             raise RuntimeError("all lanes must be reset before the first step")
-        if bool(torch.any(self.pending_reset)):   # env.py:819-821
+        if pending:   # env.py:819-821
             lanes = torch.nonzero(self.pending_reset).flatten().to("cpu").tolist()
             raise RuntimeError(f"terminal lanes must be reset before step: {lanes}")
         # every argument is checked before the observation buffer is taken: a refused call must not advance the
         # safe_view rotation, or the next step would write into the buffer the caller still holds (env.py:459-472)
         indices = self._require_device_tensor(actions, "actions", shape=(self.num_envs,), dtypes=INDEX_DTYPES).to(torch.int64)
-        if bool(torch.any((indices < 0) | (indices >= self.action_count))):   # env.py:828-829
+        if outside if outside is not None else bool(torch.any((indices < 0) | (indices >= self.action_count))):   # env.py:828-829
             raise ValueError("actions fall outside the declared action space")
         view = self._view_target()
         transition = self._step(indices, view, self.obs_layout)
@@ -363,13 +506,35 @@ class GraDoomVecEnv:
         return self.step(actions)
 
     # ------------------------------------------------------------------ RGB frames
-    def _rgb_frames(self, lane: int | None = None) -> torch.Tensor:
+    RGB_STAGING_BYTES = 64 << 20
+
+    def _rgb_frames(self, lane: int | None = None) -> np.ndarray:
+        """RGB frames of all lanes, or of one, as a host array of its own."""
+
         state = self._dynamics.lane_state()
-        if lane is not None:   # one lane's frame: only that lane is rendered
+        if lane is not None and self.num_envs > 1:   # one lane's frame: only that lane is rendered
             state = state.select(slice(lane, lane + 1))
-        rgb = torch.empty((state.x.shape[0], 240, 320, 3), dtype=torch.uint8, device=self.device)
-        self._renderer.render(state, rgb=rgb)
-        return rgb
+        count = int(state.x.shape[0])
+        render_to_host = getattr(self._renderer, "render_rgb_to_host", None)
+        if not self._native or render_to_host is None:
+            rgb = torch.empty((count, 240, 320, 3), dtype=torch.uint8, device=self.device)
+            self._renderer.render(state, rgb=rgb)
+            return rgb.detach().to("cpu").numpy()
+        # The expansion writes the frames into pinned host memory, over PCIe, as it makes them: no second copy of them on the device
+        # and no staging by the runtime.  The caller's array is filled from there by all cores (most of that is the first touch of its
+        # pages).
+        frame_bytes = 240 * 320 * 3
+        room = max(1, min(count, self.RGB_STAGING_BYTES // frame_bytes))
+        if self._rgb_staging is None or self._rgb_staging.shape[0] < room:
+            self._rgb_staging = torch.empty((room, 240, 320, 3), dtype=torch.uint8, pin_memory=True)
+        frames = torch.empty((count, 240, 320, 3), dtype=torch.uint8)
+        for base in range(0, count, room):
+            part = min(room, count - base)
+            staging = self._rgb_staging[:part]
+            render_to_host(state if part == count else state.select(slice(base, base + part)), staging)
+            self._wait()
+            frames[base : base + part].copy_(staging)
+        return frames.numpy()
 
     def render_lane(self, lane: int):  # env.py:1037-1053
         if self.closed:
@@ -381,7 +546,7 @@ class GraDoomVecEnv:
             raise IndexError(f"lane must be in [0, {self.num_envs - 1}]")
         if self.render_mode != "rgb_array":
             return None
-        frame = self._rgb_frames(lane_index)[0].detach().to("cpu").numpy().copy()
+        frame = self._rgb_frames(lane_index)[0]
         self.check_renderer_status()
         return frame
 
@@ -393,9 +558,9 @@ class GraDoomVecEnv:
             raise RuntimeError("cannot render a closed environment")
         if self.render_mode != "rgb_array":
             return [None for _ in range(self.num_envs)]
-        frames = self._rgb_frames().detach().to("cpu").numpy()
+        frames = self._rgb_frames()
         self.check_renderer_status()
-        return [frame.copy() for frame in frames]
+        return list(frames)
 
     def close(self) -> None:
         if not self.closed:

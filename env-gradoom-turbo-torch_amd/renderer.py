@@ -83,6 +83,8 @@ class LaneState:
 
 
 def _require(tensor: torch.Tensor, name: str, dtype, shape, device) -> torch.Tensor:
+    if isinstance(tensor, torch.Tensor) and tensor.dtype is dtype and tensor.shape == shape and tensor.device == device and tensor.is_contiguous():
+        return tensor
     # Same error classes as the reference's tensor validation (env.py:711-728).
     if not isinstance(tensor, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
@@ -294,6 +296,21 @@ class HipRenderer:
         stream = torch.cuda.current_stream(self.device).cuda_stream
         _lib.check(self._lib.gd_render(self._handle, C.byref(desc), C.byref(out), C.c_void_p(stream)))
         del keep_lanes, keep_out
+
+    def render_rgb_to_host(self, lanes: LaneState, rgb: torch.Tensor) -> None:
+        """One RGB frame per lane into ``rgb``, a pinned host tensor ``[N, 240, 320, 3]``: there once the stream has been waited for."""
+
+        if self._handle is None:
+            raise RuntimeError("renderer is closed")
+        desc, keep = self._lanes_desc(lanes)
+        if rgb.dtype != torch.uint8 or tuple(rgb.shape) != (desc.lane_count, 240, 320, 3) or not rgb.is_contiguous() or not rgb.is_pinned():
+            raise ValueError("rgb must be a contiguous pinned uint8 tensor of shape (lanes, 240, 320, 3)")
+        out = _abi.FrameOut()
+        out.stack_mode, out.obs_source_rows = _abi.STACK_STEP, 208
+        out.rgb = rgb.data_ptr()
+        stream = torch.cuda.current_stream(self.device).cuda_stream
+        _lib.check(self._lib.gd_render(self._handle, C.byref(desc), C.byref(out), C.c_void_p(stream)))
+        del keep
 
     def render_static(self, lanes: LaneState, *, indexed=None, obs=None, frames=None, reset_mask=None, rgb=None,
                       stack_only_masked: bool = False, final_frames=None, obs_source_rows: int = 208, final_layout: str = "chw") -> None:

@@ -507,6 +507,68 @@ int gd_sprite_depth(const float *x, const float *y, const float *angle, const fl
                     int32_t lane_count, int32_t sprite_slots, float *depth, void *stream);
 
 /*
+ * A vector environment's work around its frames (gradoom_amd/env.py), one kernel each on `stream`.  Pointers are device pointers, except
+ * done_count and flags, which may point into pinned host memory: a wait on the stream then makes them readable.  All return
+ * GD_E_ARG for a null pointer or a count out of range.
+ *
+ * gd_pose_lanes: the lane tensors of a pool of poses; lane i shows pose phase[rows ? rows[i] : i].  angle is the retained view angle
+ * (engine.py:10651), x_fixed / y_fixed the coordinates in 16.16.
+ */
+typedef struct gd_pose_desc {
+    uint32_t struct_size;    /* sizeof(gd_pose_desc) of the header the caller was built with */
+    int32_t lane_count, sprite_slots, pool_size;
+    const int64_t *phase;
+    const int64_t *rows;                 /* [lane_count], or null */
+    const float *pool_x;                 /* [pool_size] */
+    const float *pool_y;
+    const float *pool_view_z;
+    const int64_t *pool_angle_bam;
+    const int64_t *pool_pitch_bam;
+    const int64_t *pool_flash_light;
+    const float *pool_sprite_x;          /* [pool_size, sprite_slots]; null without billboards */
+    const float *pool_sprite_y;
+    const float *pool_sprite_z;
+    const int32_t *pool_sprite_id;
+    const uint8_t *pool_sprite_alive;
+    const uint8_t *pool_sprite_fullbright;
+    float *x;                            /* [lane_count] */
+    float *y;
+    float *angle;
+    float *view_z;
+    int64_t *x_fixed;
+    int64_t *y_fixed;
+    int64_t *angle_bam;
+    int64_t *pitch_bam;
+    int64_t *flash_light;
+    float *sprite_x;                     /* [lane_count, sprite_slots] */
+    float *sprite_y;
+    float *sprite_z;
+    int32_t *sprite_id;
+    uint8_t *sprite_alive;
+    uint8_t *sprite_fullbright;
+} gd_pose_desc;
+
+int gd_pose_lanes(const gd_pose_desc *desc, void *stream);
+
+/* phase = (phase + 1 + action) mod pool_size, episode_time + 1, truncated where it reaches episode_timeout; rewards and terminated zero. */
+int gd_pose_step(int64_t *phase, int64_t *episode_time, const int64_t *actions, int32_t lane_count, int64_t pool_size, int64_t episode_timeout,
+                 float *rewards, uint8_t *terminated, uint8_t *truncated, void *stream);
+/* Where mask is set: phase = seed mod pool_size, episode_time = 0. */
+int gd_pose_reset(int64_t *phase, int64_t *episode_time, const uint8_t *mask, const int64_t *seeds, int32_t lane_count, int64_t pool_size, void *stream);
+/* pending = terminated | truncated (engine.py:9542) and the two signals of [lane_count, 27] that follow it (engine.py:15469-15472); the lanes
+   that ended in done_rows, in lane order, and how many in done_count (both may be null). */
+int gd_env_step(const uint8_t *terminated, const uint8_t *truncated, const int64_t *episode_time, int32_t lane_count, uint8_t *pending, float *signals,
+                int64_t *done_rows, int32_t *done_count, void *stream);
+/* Where mask is set: latest_seeds = seeds, initialized = 1, pending = 0; then the two signals of every lane. */
+int gd_env_reset(const uint8_t *mask, const int64_t *seeds, const int64_t *episode_time, int32_t lane_count, int64_t *latest_seeds, uint8_t *initialized,
+                 uint8_t *pending, float *signals, void *stream);
+/* flags: 1 some lane is not initialized | 2 some lane is pending | 4 some action lies outside [0, action_count) (actions may be null). */
+int gd_env_check(const uint8_t *initialized, const uint8_t *pending, const int64_t *actions, int32_t lane_count, int32_t action_count, int32_t *flags,
+                 void *stream);
+/* frames [., 4, 84, 84]: the stacks of the lanes that rows names become four copies of obs [count, 84, 84] (engine.py:2443-2450). */
+int gd_fill_stacks(const uint8_t *obs, const int64_t *rows, int32_t count, uint8_t *frames, void *stream);
+
+/*
  * Time `launches` back-to-back gd_render launches with HIP events on `stream`
  * and return the average milliseconds per launch of each kernel stage in
  * ms[0..stage_count).  Measurement helper for the benchmark; replaces nothing.
