@@ -19,7 +19,7 @@
 //   flat_shade      1 wave / gap column       the gap pixels' flats
 //   decal           320 threads / lane        bullet chips on the wall tiers they hit (frames that carry decals
 //                                             also keep a per-pixel scene depth: wall_raster<true>, plane_shade<true>)
-//   sprite_columns  320 threads / lane        billboards far -> near, opaque / additive / translucent
+//   sprite_pixels   thread per view pixel     billboards, nearest visible one first, or blended far -> near
 //   weapon_overlay, hud                       player weapon, muzzle flash and status bar patches
 //   observe         1 thread / obs pixel      PLAYPAL + exact area pool + gray + 4-frame stack
 //   expand_rgb      1 thread / pixel          PLAYPAL expansion for callers that want RGB24 frames
@@ -3937,278 +3937,418 @@ __global__ void __launch_bounds__(64) flat_shade_kernel(DeviceMap dm, Scratch sc
 // ---------------------------------------------------------------------------------------------
 // sprites: engine.py:10534-10557 (blocking raycast) and 14684-14947
 // ---------------------------------------------------------------------------------------------
-#define SPRITE_ROWS 4   // rows of a sprite column in flight together
-// Columns per block.  A block lasts as long as its slowest column, so many small blocks pack the chip better than a few
-// wide ones, until the staging each block repeats for itself outweighs that; each lists only the billboards that reach its
-// own columns.  Measured on 4096 lanes with 128 billboards each, columns x row parts: 128x1 0.70 ms, 128x2 0.55, 64x2 0.49,
-// 64x4 0.51, 32x2 0.59, 32x4 0.45.
-#define SPRITE_COLUMNS 32
+#define SPRITE_ROWS 4   // rows of a sprite column in flight together (sprite_column)
+// One billboard seen from one lane.  Pixels of a wavefront read different records of an LDS array: 104 bytes, 26 words,
+// spread them over the banks (96 would put every eighth record on the same one).
 struct SpriteRec {
-    float x, y, depth, light;
+    float x, y, depth;
+    int height;
     i64 depth_fixed, left, right, hstep, yscale, top_fixed, fraction_base, iscale;
-    int id, flags;   // bit0 alive, bit1 fullbright, bits 8..15 style (signed: -1 opaque, -2 translucent, >= 0 additive),
-                     // bits 16..23 / 24..31 first / one past the last screen row the patch can reach
+    size_t texel_base;   // first texel of the patch in the atlas
+    int slot, flags;   // bits 0..4 colormap row, bits 8..15 style (signed: -1 opaque, -2 translucent, >= 0 additive),
+                       // bits 16..23 / 24..31 first / one past the last screen row the patch can reach
+    int width, spare;
 };
+static_assert(sizeof(SpriteRec) == 104, "SpriteRec: 26 words");
 
-// A frame some kernel paints into: all of a lane's 320x240 frame in device memory, or the rows a work-group keeps in LDS.
-struct GlobalFrame {
-    unsigned char *base;     // row 0, column 0 of the lane's frame
-    __device__ __forceinline__ unsigned char *at(int y, int x) const { return base + (size_t)y * SW + x; }
-};
-
-// The billboards of one lane, worked out once per work-group (engine.py:14684-14760): `sp[a]` for every slot, and in
-// `on_screen` the slots that can reach columns [x_first, x_end) at all (alive, in front, some column between left and
-// right): the per-column loops only walk these.  Their order in the list is irrelevant, ties go by slot number.
-__device__ __forceinline__ void stage_sprites(const DeviceMap &dm, const gd_lanes_desc &lanes, int n, const LaneCtx &L, int x_first, int x_end,
-                                              int row_first, int row_end, SpriteRec *sp, unsigned short *on_screen, int *on_screen_count) {
+// Slot `a` of lane `n` as a record (engine.py:14684-14760); false if it cannot reach columns [x_first, x_end) and rows
+// [row_first, row_end) at all (dead, not in front, none of its columns or rows in them).
+__device__ __forceinline__ bool sprite_record(const DeviceMap &dm, const gd_lanes_desc &lanes, int n, const LaneCtx &L, int a, int x_first, int x_end,
+                                              int row_first, int row_end, SpriteRec &s) {
     const gd_map_desc *m = &dm.d;
-    const int A = lanes.sprite_slots;
-    for (int a = threadIdx.x; a < A; a += blockDim.x) {
+    const size_t k = (size_t)n * lanes.sprite_slots + a;
+    const int id = lanes.sprite_id[k];
+    s.depth = lanes.sprite_depth[k];
+    if (!lanes.sprite_alive[k] || id < 0 || id >= m->sprite_count || !(s.depth > 0)) return false;   // an unknown patch id is never drawn
+    s.x = lanes.sprite_x[k]; s.y = lanes.sprite_y[k];
+    const float z = lanes.sprite_z[k];
+    const i64 ax = round_to_i64(s.x * 65536.0f), ay = round_to_i64(s.y * 65536.0f);
+    const i64 rx = ax - L.view_x_fixed, ry = ay - L.view_y_fixed;
+    s.depth_fixed = (rx * L.vcos + ry * L.vsin) >> 20;
+    const i64 side_fixed = (rx * L.vsin - ry * L.vcos) >> 16;
+    const i64 xscale = tdiv(FOCAL_X_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
+    const i64 left_fixed = side_fixed - (i64)m->spr_left[id] * FIXED_UNIT;
+    s.width = m->spr_w[id];
+    s.left = SW / 2 + (mul64(left_fixed, xscale) >> 32);
+    const i64 right_fixed = left_fixed + (i64)s.width * FIXED_UNIT;
+    s.right = SW / 2 + (mul64(right_fixed, xscale) >> 32);
+    if (!(s.right > x_first && s.left < x_end && s.right > s.left)) return false;
+    s.height = m->spr_h[id];
+    s.hstep = tdiv((i64)s.width << 16, max64(s.right - s.left, 1));
+    s.yscale = tdiv(FOCAL_Y_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
+    const i64 texmid = (i64)m->spr_top[id] * FIXED_UNIT - round_to_i64((L.view_z - z) * 65536.0f);
+    s.top_fixed = L.center_fixed - (mul64(texmid, s.yscale) >> 16);
+    s.iscale = tdiv(UINT32_MASK, max64(s.yscale, 1));
+    // Screen row y shows source row (fraction_base + y * iscale) >> 16 (engine.py:14830-14846).  The rows whose source
+    // row can fall inside the patch: a bracket from two divisions, a row too wide on either side; the exact test
+    // stays per row.
+    s.fraction_base = texmid - (mul64(L.center_fixed - FIXED_UNIT, s.iscale) >> 16);
+    int y_lo = 0, y_hi = VH;
+    if (s.iscale > 0) {
+        y_lo = (int)clampi(tdiv(-s.fraction_base, s.iscale) - 1, 0, VH);
+        y_hi = (int)clampi(tdiv(((i64)s.height << 16) - s.fraction_base, s.iscale) + 2, 0, VH);
+    }
+    if (!(y_hi > row_first && y_lo < row_end)) return false;
+    float light = m->sector_lights[sector_at(m, s.x, s.y)] + (float)(L.flash_light * 16);
+    if (lanes.sprite_fullbright && lanes.sprite_fullbright[k]) light = 255.0f;
+    const float base_shade = 61.0f - light / 4.0f;
+    // engine.py:10583 divides a Python number by a tensor, which Torch evaluates as reciprocal(distance) * 1280
+    // (Tensor.__rtruediv__): two roundings, not one division
+    const float visibility = fminf((1.0f / fmaxf(s.depth, 1.0f)) * 1280.0f, 24.0f);
+    const int shade = (int)clampi((i64)floorf(base_shade - visibility), 0, 31);
+    const int style = lanes.sprite_style ? (int)lanes.sprite_style[k] : -1;
+    s.flags = (int)((unsigned)shade | (((unsigned)style & 0xFFu) << 8) | ((unsigned)y_lo << 16) | ((unsigned)y_hi << 24));
+    s.texel_base = (size_t)id * m->spr_max_h * m->spr_max_w;
+    s.slot = a; s.spare = 0;
+    return true;
+}
+
+// A lane's billboards that reach the given part of the view, one record per entry in no particular order (there is room for
+// every slot): the loops over billboards only walk these.  `listed` starts at 0.
+__device__ __forceinline__ void stage_sprites(const DeviceMap &dm, const gd_lanes_desc &lanes, int n, const LaneCtx &L, int x_first, int x_end,
+                                              int row_first, int row_end, SpriteRec *sp, int *listed) {
+    for (int a = threadIdx.x; a < lanes.sprite_slots; a += blockDim.x) {
         SpriteRec s;
-        size_t k = (size_t)n * A + a;
-        s.x = lanes.sprite_x[k]; s.y = lanes.sprite_y[k];
-        float z = lanes.sprite_z[k];
-        s.depth = lanes.sprite_depth[k]; s.id = lanes.sprite_id[k];
-        const bool known_patch = s.id >= 0 && s.id < m->sprite_count;   // an unknown patch id is never drawn
-        if (!known_patch) s.id = 0;
-        s.flags = ((lanes.sprite_alive[k] && known_patch) ? 1 : 0) | ((lanes.sprite_fullbright && lanes.sprite_fullbright[k]) ? 2 : 0);
-        s.flags |= ((lanes.sprite_style ? (int)lanes.sprite_style[k] : -1) & 0xFF) << 8;
-        i64 ax = round_to_i64(s.x * 65536.0f), ay = round_to_i64(s.y * 65536.0f);
-        i64 rx = ax - L.view_x_fixed, ry = ay - L.view_y_fixed;
-        s.depth_fixed = (rx * L.vcos + ry * L.vsin) >> 20;
-        i64 side_fixed = (rx * L.vsin - ry * L.vcos) >> 16;
-        i64 xscale = tdiv(FOCAL_X_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
-        i64 left_fixed = side_fixed - (i64)m->spr_left[s.id] * FIXED_UNIT;
-        s.left = SW / 2 + (mul64(left_fixed, xscale) >> 32);
-        i64 right_fixed = left_fixed + (i64)m->spr_w[s.id] * FIXED_UNIT;
-        s.right = SW / 2 + (mul64(right_fixed, xscale) >> 32);
-        s.hstep = tdiv((i64)m->spr_w[s.id] << 16, max64(s.right - s.left, 1));
-        s.yscale = tdiv(FOCAL_Y_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
-        const i64 texmid = (i64)m->spr_top[s.id] * FIXED_UNIT - round_to_i64((L.view_z - z) * 65536.0f);
-        s.top_fixed = L.center_fixed - (mul64(texmid, s.yscale) >> 16);
-        s.iscale = tdiv(UINT32_MASK, max64(s.yscale, 1));
-        // Screen row y shows source row (fraction_base + y * iscale) >> 16 (engine.py:14830-14846).  The rows whose source
-        // row can fall inside the patch: a bracket from two divisions, a row too wide on either side; the exact test
-        // stays per row.
-        s.fraction_base = texmid - (mul64(L.center_fixed - FIXED_UNIT, s.iscale) >> 16);
-        int y_lo = 0, y_hi = VH;
-        if (s.iscale > 0) {
-            y_lo = (int)clampi(tdiv(-s.fraction_base, s.iscale) - 1, 0, VH);
-            y_hi = (int)clampi(tdiv(((i64)m->spr_h[s.id] << 16) - s.fraction_base, s.iscale) + 2, 0, VH);
-        }
-        s.flags |= (int)(((unsigned)y_lo << 16) | ((unsigned)y_hi << 24));
-        const bool reaches = (s.flags & 1) && (s.depth > 0) && (s.right > x_first) && (s.left < x_end) && (s.right > s.left) &&
-                             y_hi > row_first && y_lo < row_end;
-        s.light = reaches ? m->sector_lights[sector_at(m, s.x, s.y)] : 0.0f;
-        sp[a] = s;
-        if (reaches) on_screen[atomicAdd(on_screen_count, 1)] = (unsigned short)a;
+        if (sprite_record(dm, lanes, n, L, a, x_first, x_end, row_first, row_end, s)) sp[atomicAdd(listed, 1)] = s;
     }
 }
 
-// The billboards that can show in column x at all (alive, in front, horizontally covering it and not hidden by the
-// column's blocking linedef), as a bit set over `on_screen` (sprite_slots <= 512): the painter's loop runs once per
-// drawn billboard and would otherwise test every slot each time.  engine.py:10534-10557, 14762-14800
-struct SpriteCover { u64 bits[8]; };
-__device__ __forceinline__ SpriteCover sprite_cover(const DeviceMap &dm, const Scratch &sc, int local, const SpriteRec *sp,
-                                                    const unsigned short *on_screen, int listed, int x) {
+// The nearest blocking linedef of a column (engine.py:10534-10557), gathered by wall_setup_kernel: what hides a billboard there.
+struct ColumnBlocker {
+    float distance, dx, dy, ox, oy;
+    i64 near, far;
+    bool owns;
+    __device__ __forceinline__ ColumnBlocker(const DeviceMap &dm, const Scratch &sc, int local, int x) {
+        const gd_map_desc *m = &dm.d;
+        const u64 hit = sc.block_hit[(size_t)local * SW + x];
+        const float best = hit == ~0ULL ? GD_INF : __uint_as_float((unsigned)(hit >> 32));
+        const int slot = finitef(best) ? (int)(hit & 0xFFFFFFFFu) : 0;
+        distance = fminf(fmaxf(best, 1.0f), 4096.0f);
+        const int bw = m->blocking_count ? m->blocking_walls[slot] : 0;
+        const WallRec &bg = sc.rec[(size_t)local * m->wall_count + bw];
+        near = min64(bg.dl, bg.dr); far = max64(bg.dl, bg.dr);
+        const float4 bl = *reinterpret_cast<const float4 *>(m->walls + 4 * bw);
+        dx = bl.z - bl.x; dy = bl.w - bl.y; ox = bl.x; oy = bl.y;
+        owns = (x >= bg.sl) && (x < bg.sr);
+    }
+    // Does billboard `s` cover the column, in front of the blocking linedef?  engine.py:14762-14800
+    __device__ __forceinline__ bool shows(const SpriteRec &s, int x) const {
+        if (!((x >= s.left) && (x < s.right))) return false;
+        bool ray_visible = s.depth < distance;
+        if (!ray_visible) {
+            const float side = dx * (s.y - oy) - dy * (s.x - ox);
+            const bool behind = (near > s.depth_fixed) || ((far > s.depth_fixed) && (side <= 0));
+            ray_visible = !owns || behind;
+        }
+        const i64 su = mul64((i64)x - s.left, s.hstep) >> 16;
+        return ray_visible && su >= 0 && su < s.width;
+    }
+};
+
+// What clips billboards at one view pixel: the linedef of its word or, where there is none but a plane of the wall pass shows, the
+// plane's own depth, unless the flat ray resolves there (engine.py:13417-13422).
+struct PixelClip {
+    i64 near, far;
+    float4 line;
+    float plane_depth;   // infinite without a plane
+    int plane;
+    bool by_linedef;
+    __device__ __forceinline__ void set(const DeviceMap &dm, const Scratch &sc, int local, const LaneCtx &L, unsigned int word, int y) {
+        const gd_map_desc *m = &dm.d;
+        const int cw = (int)(word & META_WALL_MASK) - 1;
+        by_linedef = cw >= 0;
+        plane = -1; plane_depth = GD_INF;
+        if (by_linedef) {
+            const WallRec &cg = sc.rec[(size_t)local * m->wall_count + cw];
+            near = min64(cg.dl, cg.dr); far = max64(cg.dl, cg.dr);
+            line = *reinterpret_cast<const float4 *>(m->walls + 4 * cw);
+        } else {
+            plane = (word & META_FILLED) ? -1 : (int)((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1;
+            if (plane >= 0) {
+                const bool plane_floor = (word & META_FLOOR) != 0;
+                const float plane_height = plane_floor ? (L.view_z - m->sector_heights[2 * plane]) : (m->sector_heights[2 * plane + 1] - L.view_z);
+                plane_depth = plane_height * 192.0f / fmaxf(fabsf((float)y - ((103.0f + L.pitch_offset) + 0.5f)), 0.5f);
+            }
+        }
+    }
+    __device__ __forceinline__ bool linedef_shows(const SpriteRec &s) const {
+        const float side = (line.z - line.x) * (s.y - line.y) - (line.w - line.y) * (s.x - line.x);
+        return (near > s.depth_fixed) || ((far > s.depth_fixed) && (side <= 0));
+    }
+};
+
+// engine.py:14914-14939: opaque, additive table or translucent table over the pixel below
+__device__ __forceinline__ unsigned char sprite_blend(const gd_map_desc *m, int style, unsigned char lit, unsigned char below) {
+    if (style == -2) return m->translucent_lut[(size_t)below * 256 + lit];
+    if (style >= 0) return m->additive_luts[((size_t)(style > 1 ? 1 : style) * 256 + below) * 256 + lit];
+    return lit;
+}
+
+__device__ __forceinline__ bool sprite_blends(const SpriteRec &s) { const int style = (int)(signed char)(s.flags >> 8); return style == -2 || style >= 0; }
+
+// Every billboard of column x, rows [row_first, row_end), far -> near (engine.py:14762-14947): band_finish_kernel's way, one thread
+// a column and SPRITE_ROWS rows in flight, over a frame whose rows lie in LDS.
+template <typename Frame>
+__device__ __forceinline__ void sprite_column(const DeviceMap &dm, const gd_lanes_desc &lanes, const Scratch &sc, int local, int n, const LaneCtx &L,
+                                              const SpriteRec *sp, int listed, int x, int row_first, int row_end, const Frame &frame) {
     const gd_map_desc *m = &dm.d;
-    const WallRec *recs = sc.rec + (size_t)local * m->wall_count;
-    // nearest blocking linedef of this column (engine.py:10534-10557), gathered by wall_setup
-    const u64 hit = sc.block_hit[(size_t)local * SW + x];
-    float best = hit == ~0ULL ? GD_INF : __uint_as_float((unsigned)(hit >> 32));
-    int slot = finitef(best) ? (int)(hit & 0xFFFFFFFFu) : 0;
-    float wall_distance = fminf(fmaxf(best, 1.0f), 4096.0f);
-    int bw = m->blocking_count ? m->blocking_walls[slot] : 0;
-    const WallRec &bg = recs[bw];
-    i64 bnear = min64(bg.dl, bg.dr), bfar = max64(bg.dl, bg.dr);
-    const float4 bl = *reinterpret_cast<const float4 *>(m->walls + 4 * bw);
-    float bdx = bl.z - bl.x, bdy = bl.w - bl.y;
-    bool owns = (x >= bg.sl) && (x < bg.sr);
-    SpriteCover cover;
+    const unsigned int *meta = sc.meta + (size_t)local * VH * SW;
+    const ColumnBlocker blocker(dm, sc, local, x);
+    u64 cover[8];   // the billboards of the column, a bit an entry (sprite_slots <= 512)
 #pragma unroll
     for (int word = 0; word < 8; ++word) {
-        cover.bits[word] = 0;
+        cover[word] = 0;
         if (word * 64 >= listed) continue;     // the same in every thread
-        u64 bits = 0;
         const int end = listed - word * 64 < 64 ? listed - word * 64 : 64;
-        for (int b = 0; b < end; ++b) {
-            const SpriteRec &s = sp[on_screen[word * 64 + b]];
-            if (!((x >= s.left) && (x < s.right))) continue;
-            bool ray_visible = s.depth < wall_distance;
-            if (!ray_visible) {
-                float bside = bdx * (s.y - bl.y) - bdy * (s.x - bl.x);
-                bool behind = (bnear > s.depth_fixed) || ((bfar > s.depth_fixed) && (bside <= 0));
-                ray_visible = !owns || behind;
-            }
-            if (ray_visible) bits |= 1ULL << b;
-        }
-        cover.bits[word] = bits;
+        for (int b = 0; b < end; ++b) if (blocker.shows(sp[word * 64 + b], x)) cover[word] |= 1ULL << b;
     }
-    return cover;
-}
-
-// Every billboard of `cover` in column x, rows [row_first, row_end), far -> near (engine.py:14762-14947).
-template <typename Frame>
-__device__ __forceinline__ void sprite_paint(const DeviceMap &dm, const gd_lanes_desc &lanes, const Scratch &sc, int local, int n, const LaneCtx &L,
-                                             const SpriteRec *sp, const unsigned short *on_screen, const SpriteCover &cover, int x, int row_first,
-                                             int row_end, const Frame &frame, bool mark_gaps = false) {
-    const gd_map_desc *m = &dm.d;
-    const int A = lanes.sprite_slots;
-    const WallRec *recs = sc.rec + (size_t)local * m->wall_count;
-    unsigned int *meta = sc.meta + (size_t)local * VH * SW;
-    int clip_wall = -1; i64 clip_near = 0, clip_far = 0; float4 clip_line = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     // painter's order far -> near: repeatedly take the farthest candidate nearer than the last one
-    float last_depth = GD_INF; int last_slot = A;
+    float last_depth = GD_INF; int last_slot = lanes.sprite_slots;
     for (;;) {
-        float pick_depth = -GD_INF; int pick = -1;
+        float pick_depth = -GD_INF; int pick = -1, pick_slot = -1;
 #pragma unroll
         for (int word = 0; word < 8; ++word) {
-            for (u64 bits = cover.bits[word]; bits; bits &= bits - 1) {
-                const int a = on_screen[word * 64 + __ffsll((long long)bits) - 1];
-                const float depth = sp[a].depth;
+            for (u64 bits = cover[word]; bits; bits &= bits - 1) {
+                const int at = word * 64 + __ffsll((long long)bits) - 1;
+                const float depth = sp[at].depth; const int a = sp[at].slot;
                 // strictly before (last_depth, last_slot) in (depth, slot) order
                 if (!(depth < last_depth || (depth == last_depth && a < last_slot))) continue;
-                if (depth > pick_depth || (depth == pick_depth && a > pick)) { pick_depth = depth; pick = a; }
+                if (depth > pick_depth || (depth == pick_depth && a > pick_slot)) { pick_depth = depth; pick = at; pick_slot = a; }
             }
         }
         if (pick < 0) break;
-        last_depth = pick_depth; last_slot = pick;
+        last_depth = pick_depth; last_slot = pick_slot;
         const SpriteRec &s = sp[pick];
-        int width = m->spr_w[s.id], height = m->spr_h[s.id];
-        i64 su = mul64((i64)x - s.left, s.hstep) >> 16;
-        if (!(su >= 0 && su < width)) continue;
-        const int style = (int)(signed char)(s.flags >> 8);
-        float light = s.light + (float)(L.flash_light * 16);
-        if (s.flags & 2) light = 255.0f;
-        float base_shade = 61.0f - light / 4.0f;
-        // engine.py:10583 divides a Python number by a tensor, which Torch evaluates as reciprocal(distance) * 1280
-        // (Tensor.__rtruediv__): two roundings, not one division
-        float visibility = fminf((1.0f / fmaxf(s.depth, 1.0f)) * 1280.0f, 24.0f);
-        i64 shade = clampi((i64)floorf(base_shade - visibility), 0, 31);
-        const i64 fraction_base = s.fraction_base;
+        const i64 su = mul64((i64)x - s.left, s.hstep) >> 16;
+        const int style = (int)(signed char)(s.flags >> 8), shade = s.flags & 31;
         const int y_lo = max((int)((unsigned)s.flags >> 16) & 255, row_first), y_hi = min((int)((unsigned)s.flags >> 24), row_end);
         // SPRITE_ROWS rows per step, each stage's loads issued together so that their latencies overlap
         for (int yb = y_lo; yb < y_hi; yb += SPRITE_ROWS) {
-            i64 sv[SPRITE_ROWS]; bool live[SPRITE_ROWS]; unsigned int row_meta[SPRITE_ROWS];
-#pragma unroll
-            for (int j = 0; j < SPRITE_ROWS; ++j) {
-                const int y = yb + j;
-                sv[j] = (fraction_base + mul64((i64)y, s.iscale)) >> 16;
-                live[j] = y < y_hi && sv[j] >= 0 && sv[j] < height;
-                const size_t i = (size_t)(y < VH ? y : VH - 1) * SW + x;
-                row_meta[j] = meta[i];
-            }
-            // the patch texels do not wait for the clip test: asked for now, they arrive with the meta words
+            bool live[SPRITE_ROWS]; unsigned int row_meta[SPRITE_ROWS];
             unsigned char opaque[SPRITE_ROWS], post_top[SPRITE_ROWS], texel[SPRITE_ROWS];
 #pragma unroll
             for (int j = 0; j < SPRITE_ROWS; ++j) {
+                const int y = yb + j;
+                const i64 sv = (s.fraction_base + mul64((i64)y, s.iscale)) >> 16;
+                live[j] = y < y_hi && sv >= 0 && sv < s.height;
+                row_meta[j] = meta[(size_t)(y < VH ? y : VH - 1) * SW + x];
                 opaque[j] = 0; post_top[j] = 0; texel[j] = 0;
                 if (!live[j]) continue;
-                const size_t t = ((size_t)s.id * m->spr_max_h + sv[j]) * m->spr_max_w + su;
+                const size_t t = s.texel_base + (size_t)sv * m->spr_max_w + su;
                 opaque[j] = m->spr_opaque[t]; post_top[j] = m->spr_post_top[t]; texel[j] = m->spr_atlas[t];
             }
 #pragma unroll
             for (int j = 0; j < SPRITE_ROWS; ++j) {
                 if (!live[j]) continue;
-                const int cw = (int)(row_meta[j] & META_WALL_MASK) - 1;
-                bool visible;
-                if (cw >= 0) {
-                    // runs of rows share their clip linedef: its depths and line are kept from row to row
-                    if (cw != clip_wall) {
-                        const WallRec &cg = recs[cw];
-                        clip_near = min64(cg.dl, cg.dr); clip_far = max64(cg.dl, cg.dr);
-                        clip_line = *reinterpret_cast<const float4 *>(m->walls + 4 * cw);
-                        clip_wall = cw;
-                    }
-                    float side = (clip_line.z - clip_line.x) * (s.y - clip_line.y) - (clip_line.w - clip_line.y) * (s.x - clip_line.x);
-                    visible = (clip_near > s.depth_fixed) || ((clip_far > s.depth_fixed) && (side <= 0));
+                PixelClip clip;
+                clip.set(dm, sc, local, L, row_meta[j], yb + j);
+                if (clip.by_linedef) {
+                    live[j] = clip.linedef_shows(s);
                 } else {
-                    visible = s.depth < GD_INF;   // no clip linedef: the clip depth is infinite
-                    // No clip recorded, but a plane of the wall pass shows here: where the flat ray did not
-                    // resolve, the plane's own depth clips sprites (engine.py:13417-13422).  Only a sprite
-                    // standing behind the plane needs to know.
-                    const int plane = (int)((row_meta[j] >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1;
-                    if (visible && plane >= 0 && !(row_meta[j] & META_FILLED)) {
-                        const int y = yb + j;
-                        const bool plane_floor = (row_meta[j] & META_FLOOR) != 0;
-                        const float plane_height = plane_floor ? (L.view_z - m->sector_heights[2 * plane]) : (m->sector_heights[2 * plane + 1] - L.view_z);
-                        const float plane_depth = plane_height * 192.0f / fmaxf(fabsf((float)y - ((103.0f + L.pitch_offset) + 0.5f)), 0.5f);
-                        if (!(s.depth < plane_depth))
-                            visible = flat_ray_resolves(dm, L, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x],
-                                                        dm.cosine_correction[x], y, plane);
-                    }
+                    live[j] = s.depth < GD_INF;   // no clip linedef: the clip depth is infinite
+                    // only a billboard standing behind the plane needs to know whether the flat ray resolves
+                    if (live[j] && clip.plane >= 0 && !(s.depth < clip.plane_depth))
+                        live[j] = flat_ray_resolves(dm, L, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x],
+                                                    dm.cosine_correction[x], yb + j, clip.plane);
                 }
-                live[j] = visible;
             }
 #pragma unroll
             for (int j = 0; j < SPRITE_ROWS; ++j) {
                 if (!live[j] || !opaque[j]) continue;
                 const int y = yb + j;
-                i64 post_screen_top = (s.top_fixed + mul64(s.yscale, post_top[j])) >> 16;
-                if ((i64)y < post_screen_top) continue;
-                // engine.py:14914-14939: opaque, additive table or translucent table over the pixel below
-                unsigned char lit = m->colormap[shade * 256 + texel[j]];
+                if ((i64)y < ((s.top_fixed + mul64(s.yscale, post_top[j])) >> 16)) continue;
                 unsigned char *pixel = frame.at(y, x);
-                if (style == -2) lit = m->translucent_lut[(size_t)*pixel * 256 + lit];
-                else if (style >= 0) lit = m->additive_luts[((size_t)(style > 1 ? 1 : style) * 256 + *pixel) * 256 + lit];
-                *pixel = lit;
-                // painted ahead of the flat pass's pixels (launch_chunk): a gap pixel says that it is taken
-                if (mark_gaps && !(row_meta[j] & (META_FILLED | META_MASKED)) && ((row_meta[j] >> META_SECTOR_SHIFT) & META_SECTOR_MASK) == 0)
-                    meta[(size_t)y * SW + x] = row_meta[j] | META_GAP_COVERED;
+                *pixel = sprite_blend(m, style, m->colormap[shade * 256 + texel[j]], *pixel);
             }
         }
     }
 }
 
-template <typename Frame>
-__device__ __forceinline__ void sprite_column(const DeviceMap &dm, const gd_lanes_desc &lanes, const Scratch &sc, int local, int n, const LaneCtx &L,
-                                              const SpriteRec *sp, const unsigned short *on_screen, int listed, int x, int row_first, int row_end,
-                                              const Frame &frame) {
-    const SpriteCover cover = sprite_cover(dm, sc, local, sp, on_screen, listed, x);
-    sprite_paint(dm, lanes, sc, local, n, L, sp, on_screen, cover, x, row_first, row_end, frame);
-}
-
-// Each column's rows are shared out among SPRITE_ROW_PARTS threads (a column's time is a chain of memory round trips,
-// one row batch after another); the first of them finds the column's billboards and leaves the set in LDS for the others.
-#define SPRITE_ROW_PARTS 4
-static_assert(VH % (SPRITE_ROW_PARTS * SPRITE_ROWS) == 0, "sprite_columns_kernel: row parts hold whole row batches");
-__global__ void __launch_bounds__(SPRITE_COLUMNS * SPRITE_ROW_PARTS) __attribute__((amdgpu_waves_per_eu(4, 4))) sprite_columns_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
-                                                            unsigned char *frame_base, size_t frame_stride, int lane_pick) {
-    extern __shared__ unsigned char shared_raw[];
-    SpriteRec *sp = reinterpret_cast<SpriteRec *>(shared_raw);
+// A thread a view pixel.  A work-group takes SPRITE_COLUMNS columns of a lane and 1 / gridDim.z of its rows: it lists the
+// billboards that reach them, orders the list near to far, and notes as bit sets over that order which entries show in each
+// column and which have a source row in each row; a pixel then walks the entries in both sets and stops at the first that is
+// visible and opaque there (in a lane with billboards that blend it then goes back over those it passed).  What clips
+// billboards at the pixel is read once, not once per billboard: on the 4000-linedef map most of what a column ray passes is behind
+// walls, and a column's thread used to read word, linedef and patch for every row of every one of them (and the flat ray's
+// decision, which does not depend on the billboard, each time as well), waiting for one before the next.
+// A list longer than SPRITE_CHUNK, one word of bits, is painted in chunks of that many, the farthest first: the LDS a group
+// needs (13 KB) does not follow the slots a lane has.
+// Bound by the listing (six 64-bit divisions a billboard in front of the camera, in every work-group), then by the waits of
+// pixels that show something.  4096 lanes with 128 billboards, beside the flat pass: 2.71 ms a column and quarter of its rows a
+// thread, 1.38 a pixel a thread with tiles dealt out beforehand, 0.70 with tiles taken when a wavefront is free; 2048 lanes with an
+// engine's 512 slots 0.62 -> 0.35, 512 lanes 0.33 -> 0.18, 256 lanes with 32 billboards 0.086 -> 0.071.
+#define SPRITE_THREADS 256
+#define SPRITE_TILE_W 16      // columns of a wavefront's tile: 8 to 64 within 3 %
+#define SPRITE_TILE_H (64 / SPRITE_TILE_W)
+#define SPRITE_TILES 4        // tiles of a wavefront whose words are asked for together
+#define SPRITE_CHUNK 64
+#define SPRITE_SLOTS_MAX 512
+#define SPRITE_COLUMNS 64     // a work-group for the whole lane: 0.95 ms instead of 0.70 (4 wavefronts), 0.86 (8)
+#define SPRITE_ROW_PARTS 4    // of a small batch's work-groups
+// Lanes from which a work-group takes all rows of its columns: fewer listings, but the last work-groups last longer.  Whole columns /
+// quarters: 256 lanes 0.099 / 0.071 ms, 512 lanes 0.176 / 0.232, 1024 lanes 0.131 / 0.141, 4096 lanes 0.70 / 0.84.
+#define SPRITE_TALL_LANES 512
+static_assert(SPRITE_COLUMNS == 64 && SW % SPRITE_COLUMNS == 0 && VH % (SPRITE_ROW_PARTS * SPRITE_TILE_H) == 0 && VH <= SPRITE_THREADS, "sprite_pixels_kernel: whole tiles");
+static_assert(SPRITE_CHUNK == 64 && SPRITE_CHUNK <= SPRITE_THREADS, "sprite_pixels_kernel: a bit an entry");
+__global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
+                                                                          unsigned char *frame_base, size_t frame_stride, int lane_pick) {
+    __shared__ SpriteRec sp[SPRITE_CHUNK];         // the chunk's records, near to far
+    __shared__ u64 cover[SPRITE_COLUMNS], in_row[VH];
+    __shared__ float depth_of[SPRITE_SLOTS_MAX];   // the whole list, in no order
+    __shared__ unsigned short slot_of[SPRITE_SLOTS_MAX], by_rank[SPRITE_SLOTS_MAX];
+    __shared__ int listed_count, next_tile;
     const int local = blockIdx.y;
     if (local >= lane_count) return;
     // lane_pick: LANES_ALL, or one half of launch_chunk's split: LANES_PLAIN (lanes whose billboards all simply cover what is
     // under them: painted early, marking the gap pixels they take) or LANES_BLENDING (the others, after the flat pass)
-    if (lane_pick != LANES_ALL && (sc.lane_blends[local] != 0) != (lane_pick == LANES_BLENDING)) return;   // the same in the whole block
+    const bool blends = sc.lane_blends[local] != 0;
+    if (lane_pick != LANES_ALL && blends != (lane_pick == LANES_BLENDING)) return;   // the same in the whole block
     const bool mark_gaps = lane_pick == LANES_PLAIN;
-    const int n = lane_base + local;
-    const int A = lanes.sprite_slots;
-    const int x_first = blockIdx.x * SPRITE_COLUMNS, x_end = x_first + SPRITE_COLUMNS < SW ? x_first + SPRITE_COLUMNS : SW;
-    unsigned short *on_screen = reinterpret_cast<unsigned short *>(sp + A);
-    __shared__ int on_screen_count;
-    if (threadIdx.x == 0) on_screen_count = 0;
+    const gd_map_desc *m = &dm.d;
+    const int n = lane_base + local, tid = threadIdx.x;
+    const int rows = VH / gridDim.z;
+    const int x_first = blockIdx.x * SPRITE_COLUMNS, row_first = blockIdx.z * rows;
+    if (tid == 0) listed_count = 0;
     __syncthreads();
-    const LaneCtx L = sc.ctx[local];
-    stage_sprites(dm, lanes, n, L, x_first, x_end, 0, VH, sp, on_screen, &on_screen_count);
-    __syncthreads();
-    const int column = threadIdx.x % SPRITE_COLUMNS, part = threadIdx.x / SPRITE_COLUMNS;
-    const int x = x_first + column;
-    const int listed = on_screen_count;
-    if (listed == 0) return;                       // the same in the whole block
-    __shared__ u64 cover_bits[8][SPRITE_COLUMNS];
-    SpriteCover cover;
-    if (part == 0 && x < x_end) {
-        cover = sprite_cover(dm, sc, local, sp, on_screen, listed, x);
-#pragma unroll
-        for (int word = 0; word < 8; ++word) if (word * 64 < listed) cover_bits[word][column] = cover.bits[word];
+    const LaneCtx &L = sc.ctx[local];
+    for (int a = tid; a < lanes.sprite_slots; a += SPRITE_THREADS) {
+        SpriteRec s;
+        if (!sprite_record(dm, lanes, n, L, a, x_first, x_first + SPRITE_COLUMNS, row_first, row_first + rows, s)) continue;
+        const int at = atomicAdd(&listed_count, 1);
+        depth_of[at] = s.depth; slot_of[at] = (unsigned short)a;
+        if (at < SPRITE_CHUNK) sp[at] = s;
     }
     __syncthreads();
-    if (x >= x_end) return;
+    const int listed = listed_count;
+    if (listed == 0) return;                       // the same in the whole block
+    // near to far, equal depths by slot: an entry's place is the number of entries before it
+    for (int i = tid; i < listed; i += SPRITE_THREADS) {
+        const float depth = depth_of[i]; const int slot = slot_of[i];
+        int before = 0;
+        for (int j = 0; j < listed; ++j) before += depth_of[j] < depth || (depth_of[j] == depth && slot_of[j] < slot);
+        by_rank[before] = (unsigned short)(listed <= SPRITE_CHUNK ? i : slot);
+    }
+    __syncthreads();
+    unsigned int *meta = sc.meta + (size_t)local * VH * SW;
+    unsigned char *frame = frame_base + (size_t)local * frame_stride;
+    const int lane_id = tid & 63, wave = tid >> 6;
+    constexpr int WAVES = SPRITE_THREADS / 64;
+    constexpr int TILES_ACROSS = SPRITE_COLUMNS / SPRITE_TILE_W;
+    const int tiles = TILES_ACROSS * (rows / SPRITE_TILE_H);
+    const int tile_x = lane_id % SPRITE_TILE_W, tile_y = lane_id / SPRITE_TILE_W;
+    for (int first = (listed - 1) / SPRITE_CHUNK * SPRITE_CHUNK; first >= 0; first -= SPRITE_CHUNK) {
+        const int length = listed - first < SPRITE_CHUNK ? listed - first : SPRITE_CHUNK;
+        {   // the chunk's records into their places
+            SpriteRec s;
+            if (tid < length) {
+                if (listed <= SPRITE_CHUNK) s = sp[by_rank[tid]];
+                else (void)sprite_record(dm, lanes, n, L, by_rank[first + tid], x_first, x_first + SPRITE_COLUMNS, row_first, row_first + rows, s);
+            }
+            if (tid < SPRITE_COLUMNS) cover[tid] = 0;
+            __syncthreads();                       // (also: every pixel of the chunk before is painted)
+            if (tid < length) sp[tid] = s;
+            if (tid == 0) next_tile = 0;
+            __syncthreads();
+        }
+        {   // a column's entries are shared out over the wavefronts
+            const ColumnBlocker blocker(dm, sc, local, x_first + lane_id);
+            u64 bits = 0;
+            for (int b = wave; b < length; b += WAVES) if (blocker.shows(sp[b], x_first + lane_id)) bits |= 1ULL << b;
+            if (bits) atomicOr(&cover[lane_id], bits);
+        }
+        if (tid < rows) {
+            const int y = row_first + tid;
+            u64 bits = 0;
+            for (int b = 0; b < length; ++b) {
+                const SpriteRec &s = sp[b];
+                const i64 sv = (s.fraction_base + mul64((i64)y, s.iscale)) >> 16;
+                if (y >= (int)(((unsigned)s.flags >> 16) & 255) && y < (int)((unsigned)s.flags >> 24) && sv >= 0 && sv < s.height) bits |= 1ULL << b;
+            }
+            in_row[tid] = bits;
+        }
+        __syncthreads();
+        // Wavefronts take the next tiles when they are done with theirs: what a tile costs ranges from a look at two bit sets to
+        // several rounds of patch texels and the flat ray's decision.
+        for (;;) {
+            int t0 = 0;
+            if (lane_id == 0) t0 = atomicAdd(&next_tile, SPRITE_TILES);
+            t0 = __builtin_amdgcn_readfirstlane(t0);
+            if (t0 >= tiles) break;
+            unsigned int pixel_words[SPRITE_TILES];
+            u64 entries[SPRITE_TILES];
 #pragma unroll
-    for (int word = 0; word < 8; ++word) cover.bits[word] = word * 64 < listed ? cover_bits[word][column] : 0;
-    GlobalFrame frame; frame.base = frame_base + (size_t)local * frame_stride;
-    sprite_paint(dm, lanes, sc, local, n, L, sp, on_screen, cover, x, part * (VH / SPRITE_ROW_PARTS), (part + 1) * (VH / SPRITE_ROW_PARTS), frame, mark_gaps);
+            for (int j = 0; j < SPRITE_TILES; ++j) {
+                const int t = t0 + j;
+                entries[j] = 0; pixel_words[j] = 0;
+                if (t >= tiles) continue;              // the same in the whole wavefront
+                const int column = t % TILES_ACROSS * SPRITE_TILE_W + tile_x, row = t / TILES_ACROSS * SPRITE_TILE_H + tile_y;
+                entries[j] = cover[column] & in_row[row];
+                if (entries[j]) pixel_words[j] = meta[(size_t)(row_first + row) * SW + x_first + column];
+            }
+#pragma unroll
+            for (int j = 0; j < SPRITE_TILES; ++j) {
+                if (!entries[j]) continue;
+                const int t = t0 + j;
+                const int x = x_first + t % TILES_ACROSS * SPRITE_TILE_W + tile_x, y = row_first + t / TILES_ACROSS * SPRITE_TILE_H + tile_y;
+                const unsigned int pixel_word = pixel_words[j];
+                PixelClip clip;
+                clip.set(dm, sc, local, L, pixel_word, y);
+                unsigned char *pixel = frame + (size_t)y * SW + x;
+                int value = -1;                        // what the pixel shows, once a billboard does
+                int resolves = -1;                     // does the flat ray resolve here: not known, no, yes
+                // is the billboard in front of what clips it here: no, yes, -1 = ask the flat ray first
+                auto in_front = [&](const SpriteRec &s) -> int {
+                    if (clip.by_linedef) return clip.linedef_shows(s);
+                    if (!(s.depth < GD_INF)) return 0;                                       // no clip linedef: the clip depth is infinite
+                    return (clip.plane < 0 || s.depth < clip.plane_depth) ? 1 : resolves;    // only a billboard standing behind the plane needs to know
+                };
+                // its colour at the pixel after the colormap, -1 where the patch has none
+                auto colour = [&](const SpriteRec &s) -> int {
+                    const i64 su = mul64((i64)x - s.left, s.hstep) >> 16, sv = (s.fraction_base + mul64((i64)y, s.iscale)) >> 16;
+                    const size_t at = s.texel_base + (size_t)sv * m->spr_max_w + su;
+                    const unsigned char opaque = m->spr_opaque[at], post_top = m->spr_post_top[at], texel = m->spr_atlas[at];
+                    if (!opaque || (i64)y < ((s.top_fixed + mul64(s.yscale, post_top)) >> 16)) return -1;
+                    return m->colormap[(s.flags & 31) * 256 + texel];
+                };
+                u64 bits = entries[j], blended = 0;
+                bool undecided;
+                do {
+                    undecided = false;
+                    while (bits) {
+                        const int bit = __ffsll((long long)bits) - 1;
+                        const SpriteRec &s = sp[bit];
+                        const int front = in_front(s);
+                        if (front < 0) { undecided = true; break; }
+                        bits &= bits - 1;
+                        if (!front) continue;
+                        if (blends && sprite_blends(s)) { blended |= 1ULL << bit; continue; }
+                        value = colour(s);
+                        if (value >= 0) bits = 0;
+                    }
+                    // a pixel that has to know whether its flat ray resolves leaves the walk for it, once: those that do ask together
+                    if (undecided)
+                        resolves = flat_ray_resolves(dm, L, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x],
+                                                     dm.cosine_correction[x], y, clip.plane) ? 1 : 0;
+                } while (undecided);
+                if (blended) {                         // from the opaque entry back to the eye
+                    bool below_known = value >= 0;
+                    while (blended) {
+                        const int bit = 63 - __clzll((long long)blended);
+                        blended &= ~(1ULL << bit);
+                        const SpriteRec &s = sp[bit];
+                        const int lit = colour(s);
+                        if (lit < 0) continue;
+                        if (!below_known) { value = *pixel; below_known = true; }
+                        value = sprite_blend(m, (int)(signed char)(s.flags >> 8), (unsigned char)lit, (unsigned char)value);
+                    }
+                }
+                if (value < 0) continue;
+                *pixel = (unsigned char)value;
+                // painted ahead of the flat pass's pixels (launch_chunk): a gap pixel says that it is taken
+                if (mark_gaps && gap_pixel(pixel_word)) meta[(size_t)y * SW + x] = pixel_word | META_GAP_COVERED;
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -4771,12 +4911,11 @@ __global__ void __launch_bounds__(BAND_THREADS) __attribute__((amdgpu_waves_per_
     // --- billboards, one thread per screen column
     if (lanes.sprite_slots > 0 && lanes.sprite_x && view_rows > 0) {
         __syncthreads();                  // every shaded pixel is in place, and the shading tables are free
-        const bool fits = (size_t)lanes.sprite_slots * (sizeof(SpriteRec) + sizeof(unsigned short)) <= sizeof(shading_lds);
+        const bool fits = (size_t)lanes.sprite_slots * sizeof(SpriteRec) <= sizeof(shading_lds);
         SpriteRec *sp = reinterpret_cast<SpriteRec *>(fits ? reinterpret_cast<unsigned char *>(&shading_lds) : shared_raw);
-        unsigned short *on_screen = reinterpret_cast<unsigned short *>(sp + lanes.sprite_slots);
-        stage_sprites(dm, lanes, n, L, 0, SW, row0, row0 + view_rows, sp, on_screen, &on_screen_count);
+        stage_sprites(dm, lanes, n, L, 0, SW, row0, row0 + view_rows, sp, &on_screen_count);
         __syncthreads();
-        if (tid < SW && on_screen_count > 0) sprite_column(dm, lanes, sc, local, n, L, sp, on_screen, on_screen_count, tid, row0, row0 + view_rows, frame);
+        if (tid < SW && on_screen_count > 0) sprite_column(dm, lanes, sc, local, n, L, sp, on_screen_count, tid, row0, row0 + view_rows, frame);
     }
     __syncthreads();
     // --- the player's weapon and its muzzle flash (engine.py:15051-15110)
@@ -5485,8 +5624,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     const bool billboards_split = beside && has_billboards && !decals;
     const bool may_blend = lanes->sprite_style != nullptr;   // without styles no lane blends: the launches for such lanes are left out
     auto paint_billboards = [&](hipStream_t on, int lane_pick) {
-        const size_t shared = (size_t)lanes->sprite_slots * (sizeof(SpriteRec) + sizeof(unsigned short));
-        hipLaunchKernelGGL(sprite_columns_kernel, dim3((SW + SPRITE_COLUMNS - 1) / SPRITE_COLUMNS, count), dim3(SPRITE_COLUMNS * SPRITE_ROW_PARTS), shared, on, r->dm, *lanes, base, count, sc, frame_base, frame_stride, lane_pick);
+        hipLaunchKernelGGL(sprite_pixels_kernel, dim3(SW / SPRITE_COLUMNS, count, count >= SPRITE_TALL_LANES ? 1 : SPRITE_ROW_PARTS), dim3(SPRITE_THREADS), 0, on, r->dm, *lanes, base, count, sc, frame_base, frame_stride, lane_pick);
     };
     if (!fused && !(billboards_split && !may_blend)) hipLaunchKernelGGL(flat_shade_kernel, flat_grid(4, 4096), dim3(64), 0, stream, r->dm, sc, frame_base, frame_stride, billboards_split ? LANES_BLENDING : LANES_ALL);
     if (beside) {
@@ -5511,7 +5649,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         finish.final_hwc = out->final_frames_layout == GD_LAYOUT_HWC;
         finish.source_rows = source_rows;
         const bool sprites = lanes->sprite_slots > 0 && lanes->sprite_x;
-        size_t shared = sprites ? (size_t)lanes->sprite_slots * (sizeof(SpriteRec) + sizeof(unsigned short)) : 0;
+        size_t shared = sprites ? (size_t)lanes->sprite_slots * sizeof(SpriteRec) : 0;
         if (shared <= (size_t)LDS_SECTORS * sizeof(float4) + 32 * 256) shared = 0;   // the records reuse the shading tables' LDS
         hipLaunchKernelGGL(band_finish_kernel, dim3(BAND_COUNT, count), dim3(BAND_THREADS), shared, stream, r->dm, r->overlays, *lanes, base, count, sc, finish);
         mark();
@@ -5774,7 +5912,7 @@ static int check_render_args(gd_renderer *r, const gd_lanes_desc *lanes, const g
                                   !lanes->angle_bam || !lanes->pitch_bam || !lanes->ray_cos || !lanes->ray_sin))
         return fail(GD_E_ARG, "missing lane tensor");
     if (out->stack_mode != GD_STACK_STEP && out->stack_mode != GD_STACK_RESET) return fail(GD_E_ARG, "unknown stack_mode");
-    if (lanes->sprite_slots < 0 || lanes->sprite_slots > 512) return fail(GD_E_ARG, "sprite_slots must be in [0, 512]");
+    if (lanes->sprite_slots < 0 || lanes->sprite_slots > SPRITE_SLOTS_MAX) return fail(GD_E_ARG, "sprite_slots must be in [0, 512]");
     if (lanes->decal_slots < 0) return fail(GD_E_ARG, "negative decal_slots");
     if (lanes->decal_slots > 0 && (lanes->decal_state != nullptr) != (lanes->decal_geom != nullptr))
         return fail(GD_E_ARG, "decal_state and decal_geom go together");
