@@ -84,13 +84,25 @@ static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and it
 #define CF_LEDGE 4
 #define CF_ALONG_HI 8   // along > 0.5: the ray is nearer the linedef's end vertex
 #define CF_FF 16        // camera on the front side of the linedef (float32 test)
+// facts of the linedef itself: a pass asks for them of every linedef it considers, and a load from the lane's records would be
+// another trip to memory (0.9 GB of records for 4096 lanes) in the chain it waits for
+#define CF_ENDS_HERE 32 // its clipped span ends at this column
+#define CF_NARROW 64    // its clipped span is at most two columns wide
+#define CF_SHORT 128    // at most 32 map units long
+#define CF_SUBPIXEL 256 // two-sided, and its clipped span at most one column wide
 
 // wall record flags
 #define WF_HC 1        // owns at least one column after every span test
-#define WF_FF 2        // front facing (float32 test of engine.py:11376-11381)
-#define WF_SUBPIXEL 4  // two-sided and at most one column wide (engine.py:11589-11591)
+#define WF_SPLIT 2     // projects through BSP fragments (engine.py:11472-11545, 12310-12380)
 #define WF_ANYGEO 8    // some column ray hits the segment
-#define WF_SPLIT 16    // projects through BSP fragments (engine.py:11472-11545, 12310-12380)
+// the facts a candidate shows at every column, in its flags' places (eval_segment copies them)
+#define WF_FF CF_FF             // front facing (float32 test of engine.py:11376-11381)
+#define WF_NARROW CF_NARROW
+#define WF_SHORT CF_SHORT
+#define WF_SUBPIXEL CF_SUBPIXEL // two-sided and at most one column wide (engine.py:11589-11591)
+#define WF_SHOWN (WF_FF | WF_NARROW | WF_SHORT | WF_SUBPIXEL)
+#define WF_END_SHIFT 16   // bits 16 and up: the column at which the clipped span ends, WF_END_NONE if that is not a column
+#define WF_END_NONE 1023
 
 struct LaneCtx {
     float x, y, view_z, pitch_offset, fsin, fcos;
@@ -190,6 +202,10 @@ struct Eval {      // distances/along/geometric/projected/left-edge of one lined
     int flags;
 };
 
+#define WALL_ONE_SIDED 1
+#define WALL_SPLIT 2
+#define WALL_SHORT 4     // at most 32 map units long
+#define WALL_BLOCKING_SHIFT 4
 struct DeviceMap {  // device copy of gd_map_desc (device pointers) + fixed tables
     gd_map_desc d;
     const i64 *fine_sine;     // [8192]
@@ -215,7 +231,7 @@ struct DeviceMap {  // device copy of gd_map_desc (device pointers) + fixed tabl
     const WallSide *wall_side;           // [W,2]
     const int *masked_slot;              // [W] number of the linedef among those with a mid-texture on a two-sided side, else -1
     int masked_count;                    // how many there are
-    const int *wall_blocking_slot;       // [W] position of the linedef in blocking_walls, -1 when it does not block
+    const int *wall_facts;               // [W] WALL_*, and from bit WALL_BLOCKING_SHIFT on the linedef's position in blocking_walls plus one, 0 when it does not block
     const unsigned int *sector_level;    // [S] index of the floor in floor_levels | index of the ceiling in ceil_levels << 16;
                                          // null when some sector's height is missing from the level lists
 };
@@ -695,7 +711,7 @@ __device__ __forceinline__ Eval eval_segment(const float4 wl, int rec_flags, int
     Eval out;
     out.dist = valid ? d : GD_INF;
     out.flags = (g ? CF_GEO : 0) | (p ? CF_PROJ : 0) | ((x == rec_pl) ? CF_LEDGE : 0) | ((a > 0.5f) ? CF_ALONG_HI : 0) |
-                ((rec_flags & WF_FF) ? CF_FF : 0);
+                (((rec_flags >> WF_END_SHIFT) == x) ? CF_ENDS_HERE : 0) | (rec_flags & WF_SHOWN);
     return out;
 }
 
@@ -806,7 +822,9 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
                 RecSpan span;
                 span.pl = 0; span.pr = 0;
                 // an unseen linedef has an empty span (sr == sl), so a two-sided one counts as at most one column wide
-                span.flags = (ff ? WF_FF : 0) | (m->wall_sectors[2 * w + 1] < 0 ? 0 : WF_SUBPIXEL) | (m->wall_split_slot[w] >= 0 ? WF_SPLIT : 0);
+                const int facts = dm.wall_facts[w];
+                span.flags = (ff ? WF_FF : 0) | ((facts & WALL_ONE_SIDED) ? 0 : WF_SUBPIXEL) | ((facts & WALL_SPLIT) ? WF_SPLIT : 0) |
+                             WF_NARROW | ((facts & WALL_SHORT) ? WF_SHORT : 0) | (WF_END_NONE << WF_END_SHIFT);
                 sc.span[(size_t)local * m->wall_count + w] = span;
             }
         }
@@ -849,7 +867,8 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
         }
     }
     if (!live) { scan_lo = 1; scan_hi = 0; }
-    const int blocking_slot = dm.wall_blocking_slot[w];
+    const int facts = dm.wall_facts[w];
+    const int blocking_slot = (facts >> WALL_BLOCKING_SHIFT) - 1;
     u64 *block_hits = sc.block_hit + (size_t)local * SW;
     int first = 0, last = SW - 1; bool any = false;
     float numer_d = offx * segy - offy * segx;
@@ -954,7 +973,8 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
     bool os = s1 < 0;
     r.pl = (short)screen_left; r.pr = (short)screen_right;
     r.flags = (hc ? WF_HC : 0) | (ff ? WF_FF : 0) | (((sr - sl <= 1) && !os) ? WF_SUBPIXEL : 0) | (any ? WF_ANYGEO : 0) |
-              (m->wall_split_slot[w] >= 0 ? WF_SPLIT : 0);
+              ((facts & WALL_SPLIT) ? WF_SPLIT : 0) | (sr - sl <= 2 ? WF_NARROW : 0) | ((facts & WALL_SHORT) ? WF_SHORT : 0) |
+              ((sr >= 0 && sr < SW ? (int)sr : WF_END_NONE) << WF_END_SHIFT);
     if (live) {
         sc.rec[(size_t)local * m->wall_count + w] = r;
         RecSpan span;
@@ -974,7 +994,7 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
     const int packed_sectors = (s0 & 0xFFFF) | (s1 << 16);
     const int packed_vertices = (int)(((unsigned)m->wall_vertex[2 * w] & 0xFFFFu) | ((unsigned)m->wall_vertex[2 * w + 1] << 16));
     const bool masked_side = !os && m->side_tex[(w * 2 + (ff ? 0 : 1)) * 3] >= 0;
-    const int packed_span = (r.flags & 0xFF) | (os ? 0x100 : 0) | (masked_side ? 0x200 : 0);
+    const int packed_span = r.flags | (os ? 0x200 : 0) | (masked_side ? 0x400 : 0);   // bits 9 and 10 of the flags are free
     const int rec_pl = r.pl, rec_pr = r.pr;
     // Most linedefs cover a few columns only, so several of them share a turn: eight with eight lanes each, then
     // four with sixteen, then two with thirty-two; a wider one has the wavefront to itself.
@@ -1005,9 +1025,9 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
             const int x = b_lo + group_lane;
             if (owner < 0 || x >= b_hi) continue;
             float rx, ry; ray_direction(c, x, &rx, &ry);
-            const Eval e = eval_segment(b_wl, b_span & 0xFF, b_pl, b_pr, (b_span & 0x100) != 0, c, x, rx, ry);
+            const Eval e = eval_segment(b_wl, b_span, b_pl, b_pr, (b_span & 0x200) != 0, c, x, rx, ry);
             if (!finitef(e.dist)) continue;
-            if ((b_span & 0x200) && (e.flags & CF_PROJ)) note_masked(b_wall, x, e);
+            if ((b_span & 0x400) && (e.flags & CF_PROJ)) note_masked(b_wall, x, e);
             const int slot = atomicAdd(&counts[x], 1);
             if (slot < CAND_MAX) {
                 Cand entry;
@@ -1036,9 +1056,9 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
         entry.v0 = (unsigned short)(b_vertices & 0xFFFF); entry.v1 = (unsigned short)((unsigned)b_vertices >> 16);
         for (int x = b_lo + slot_in_wave; x < b_hi; x += 64) {
             float rx, ry; ray_direction(c, x, &rx, &ry);
-            Eval e = eval_segment(b_wl, b_span & 0xFF, b_pl, b_pr, (b_span & 0x100) != 0, c, x, rx, ry);
+            Eval e = eval_segment(b_wl, b_span, b_pl, b_pr, (b_span & 0x200) != 0, c, x, rx, ry);
             if (finitef(e.dist)) {
-                if ((b_span & 0x200) && (e.flags & CF_PROJ)) note_masked(entry.wall, x, e);
+                if ((b_span & 0x400) && (e.flags & CF_PROJ)) note_masked(entry.wall, x, e);
                 int slot = atomicAdd(&counts[x], 1);
                 if (slot < CAND_MAX) {
                     entry.flags = (unsigned short)e.flags;
@@ -2128,7 +2148,7 @@ __device__ __forceinline__ i64 wall_shade(float light, i64 visibility) {
 __device__ __forceinline__ void endpoint_owner(const ColumnCtx &cc, int w, const Eval &cw, int *owner_index, float *owner_distance) {
     const gd_map_desc *m = cc.m;
     const int K = m->neighbor_slots;
-    const bool subpixel = cc.spans[cc.rec_base + (unsigned)w].flags & WF_SUBPIXEL;
+    const bool subpixel = cw.flags & CF_SUBPIXEL;
     float tol_w = tolerance_of(cw.dist);
     // the owner only matters for a linedef that does not own this column itself (engine.py:11716)
     if (cw.flags & CF_PROJ) { *owner_index = w; *owner_distance = cw.dist; return; }
@@ -2402,7 +2422,7 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
         pend_ep_has_forward_bridge = cc.eval(fb_idx).dist > distance + 1e-3f;
     bool completes_pending_endpoint_bridge = (c.flags & ST_EB) && (wi == c.pend_eb_index);
     bool sel_is_proj = cwi.flags & CF_PROJ;
-    bool sel_excl_right = cc.rec(wi).sr == x;
+    bool sel_excl_right = cwi.flags & CF_ENDS_HERE;
     // d. projected solid owner (engine.py:11872-11954)
     float ps_path_distance = distance; int ps_path_index = wi;
     bool ps_path_geo = cwi.flags & CF_GEO;
@@ -2452,10 +2472,7 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
     int no_path_other = no_from_front ? mv.sec(no_path_index, 1) : mv.sec(no_path_index, 0);
     // f. near projected owner (engine.py:12002-12179)
     bool so_is_proj = cwi.flags & CF_PROJ;
-    const WallRec &so_rec = cc.rec(wi);
-    bool so_excl_right = so_rec.sr == x;
-    i64 so_span = so_rec.sr - so_rec.sl;
-    bool so_short = m->wall_len[wi] <= 32.0f;
+    const bool so_excl_right = cwi.flags & CF_ENDS_HERE, so_narrow = cwi.flags & CF_NARROW, so_short = cwi.flags & CF_SHORT;
     float npd = GD_INF; int npi = 0x7fffffff; int npi_flags = 0;
     const int so_s0 = mv.sec(wi, 0), so_s1 = mv.sec(wi, 1);
     if (!so_is_proj) {
@@ -2464,10 +2481,10 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
             if (!(incident_c(q) && (q.s1 >= 0) && (q.flags & CF_PROJ) && (q.dist > prev_eps))) return;
             bool le = q.flags & CF_LEDGE;
             bool same_pair = (q.s0 == so_s0 && q.s1 == so_s1) || (q.s0 == so_s1 && q.s1 == so_s0);
-            bool close = (same_pair || (le && so_excl_right && ((so_span <= 2) || (shares_sel_c(q) && so_short)))) &&
+            bool close = (same_pair || (le && so_excl_right && (so_narrow || (shares_sel_c(q) && so_short)))) &&
                          (fabsf(q.dist - distance) <= tolerance_of(q.dist));
             bool topo = false;
-            if (!close && le && so_excl_right && so_span <= 2) { int dummy; topo = mv.sector_bridge((q.flags & CF_ALONG_HI) ? 1 : 0, w, no_path_index, &dummy); }
+            if (!close && le && so_excl_right && so_narrow) { int dummy; topo = mv.sector_bridge((q.flags & CF_ALONG_HI) ? 1 : 0, w, no_path_index, &dummy); }
             if ((close || topo) && (q.dist < npd || (q.dist == npd && w < npi))) { npd = q.dist; npi = w; npi_flags = q.flags; }
         };
         for (u64 rest = incident_beyond; rest;) {
@@ -2507,7 +2524,7 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
     bool completes_poab = (c.flags & ST_EP) && final_proj && !final_geo && mv.opposing(pe_wall, wi);
     // g. validity (engine.py:12197-12239)
     bool valid = finitef(distance);
-    bool excl_only = !so_is_proj && so_excl_right && !replace_np && (so_span <= 2) && !boundary_has_po;
+    bool excl_only = !so_is_proj && so_excl_right && !replace_np && so_narrow && !boundary_has_po;
     bool raster_valid = valid && !excl_only && !continues_po_boundary &&
                         !((pend_ep_has_forward_bridge || completes_pending_endpoint_bridge) && !sel_is_proj && sel_excl_right && !replace_np);
     bool geometric_intersection = replace_np ? no_path_geo : (replace_eo ? eo_path_geo : final_geo);
@@ -3539,6 +3556,7 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     cc.set_list(sc, local, x);
     cc.x = x;
     ray_direction(lane_ctx, x, &cc.rx, &cc.ry);
+    bool boundary_has_po = false;   // does some entry's span begin at this column
     if (STAGED) {
         // every lane copies its own column's entries and reads only those: no barrier
         char *mine = reinterpret_cast<char *>(staged_entries) + lane_id * 16;
@@ -3550,6 +3568,7 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
             for (int j = 0; j < CAND_BATCH; ++j) {
                 union { uint4 raw; Cand c; } u;
                 u.c = batch[j];
+                boundary_has_po |= (batch[j].flags & CF_LEDGE) != 0;   // slots past the end repeat the last entry
                 if (k0 + j < depth) *reinterpret_cast<uint4 *>(mine + (k0 + j) * (PART_COLS * 16)) = u.raw;
             }
         }
@@ -3563,8 +3582,14 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     st.previous_distance = 0.0f;
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
-    bool boundary_has_po = false;
-    for (int k = 0; k < cc.count; ++k) if (cc.cand(k).flags & CF_LEDGE) { boundary_has_po = true; break; }
+    if (!STAGED) {
+        for (int k0 = 0; k0 < cc.count && !boundary_has_po; k0 += CAND_BATCH) {
+            Cand batch[CAND_BATCH];
+            cc.cand_batch(k0, batch);
+#pragma unroll
+            for (int j = 0; j < CAND_BATCH; ++j) boundary_has_po |= (batch[j].flags & CF_LEDGE) != 0;   // slots past the end repeat the last entry
+        }
+    }
     PassRec *records = sc.pass_rec + sc.pass_at(0, local, x);
     float *path_distances = sc.pass_path_distance + sc.pass_at(0, local, x);
     const size_t pass_stride = (size_t)sc.lane_stride * SW;
@@ -5789,13 +5814,15 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
                 around[l] = make_float4(std::fmin(around[l].x, box.x), std::fmin(around[l].y, box.y), std::fmax(around[l].z, box.z), std::fmax(around[l].w, box.w));
             }
         if (rc == GD_OK) rc = upload(r, around.data(), around.size(), &r->dm.level_box);
-        std::vector<int> blocking_slot(W, -1);
+        std::vector<int> facts(W, 0);
+        for (size_t w = 0; w < W; ++w)
+            facts[w] = (h->wall_sectors[2 * w + 1] < 0 ? WALL_ONE_SIDED : 0) | (h->wall_split_slot[w] >= 0 ? WALL_SPLIT : 0) | (h->wall_len[w] <= 32.0f ? WALL_SHORT : 0);
         for (int b = 0; b < h->blocking_count; ++b) {
             const int w = h->blocking_walls[b];
             if (w < 0 || (size_t)w >= W) { if (rc == GD_OK) rc = fail(GD_E_ARG, "blocking_walls holds a linedef index out of range"); continue; }
-            if (blocking_slot[w] < 0) blocking_slot[w] = b;   // the first slot wins ties, like the scan it replaces
+            if ((facts[w] >> WALL_BLOCKING_SHIFT) == 0) facts[w] |= (b + 1) << WALL_BLOCKING_SHIFT;   // the first slot wins ties, like the scan it replaces
         }
-        if (rc == GD_OK) rc = upload(r, blocking_slot.data(), blocking_slot.size(), &r->dm.wall_blocking_slot);
+        if (rc == GD_OK) rc = upload(r, facts.data(), facts.size(), &r->dm.wall_facts);
         std::vector<WallSide> sides(W * 2);
         std::vector<int> masked_slot(W, -1);
         r->dm.masked_count = 0;
