@@ -1936,8 +1936,12 @@ __global__ void __launch_bounds__(SW) flat_span_finish_kernel(Scratch sc) {
 // walls: engine.py:11462-13745
 // ---------------------------------------------------------------------------------------------
 #define CAND_BATCH 8
-#define SELECT_STAGED_STRIPS 512   // wall_select_kernel's launch for the longest strips: how many strips,
-#define SELECT_STAGED_PARTS 4      // and over how many wavefronts each is shared out
+// wall_select_kernel's launch for the longest strips
+#define SELECT_STAGED_STRIPS 512   // how many strips,
+#define SELECT_PARTS 8             // and over how many wavefronts each is shared out;
+#define SELECT_FINE_STRIPS 128     // in a batch of fewer than SELECT_FINE_LANES lanes the very longest are shared out over more
+#define SELECT_FINE_PARTS 32
+#define SELECT_FINE_LANES 1536
 #define WALL_ROWS 8          // rows painted / clipped per step of the wall traversal
 struct ColumnCtx {
     const Tables *tb;
@@ -1952,8 +1956,8 @@ struct ColumnCtx {
     int count;
     int x;
     float rx, ry;
-    // wall_select_kernel's staged launch: this column's list copied to LDS (entry k at staged + k * 256 bytes: a row of
-    // the wavefront's 16 columns), unused everywhere else.  (One or the other for a whole kernel: a choice per load would become one flat
+    // wall_select_kernel's staged launch: this column's list copied to LDS (entry k at staged + k * 128 bytes: a row of
+    // the wavefront's 8 columns), unused everywhere else.  (One or the other for a whole kernel: a choice per load would become one flat
     // load of a selected address.)
     typedef __attribute__((address_space(3))) const char LdsByte;
     LdsByte *staged;
@@ -1978,7 +1982,7 @@ struct ColumnCtx {
         typedef unsigned int Words4 __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) const Words4 LdsEntry;
         union { uint4 raw; Words4 words; Cand c; } u;
-        if (use_staged) u.words = *(LdsEntry *)(staged + (unsigned)k * (64 / SELECT_STAGED_PARTS * 16u));   // all of the list is there
+        if (use_staged) u.words = *(LdsEntry *)(staged + (unsigned)k * (64 / SELECT_PARTS * 16u));   // all of the list is there
         else u.raw = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(list) + (list_column + (unsigned)k * (SW * 16u)));   // one 16-byte load
         return u.c;
     }
@@ -3518,22 +3522,31 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(int strips, Scratch s
 // chip to themselves, all of them together 1.22 ms, all but the 4096 longest 0.53 ms.  Such a strip's wavefront is held
 // up by its candidate scans (the longest lists, read from device memory beside 20,000 other wavefronts) and by running,
 // pass after pass, every rule that any of its 64 columns takes.  So the SELECT_STAGED_STRIPS longest strips (they lead
-// the order) go to a launch of their own (STAGED): a strip is shared out over SELECT_STAGED_PARTS wavefronts of 16 columns
-// each, which first copy their columns' lists to LDS (16 KB a wavefront) and scan them there.  It runs beside the
-// launch for all other strips: 1.22 -> 0.99 ms.  (Measured: 256 to 1024 strips, 1, 2, 4 or 8 parts; lists left in device
-// memory: no gain.)
+// the order) go to a launch of their own (STAGED): a strip is shared out over SELECT_PARTS wavefronts of 8 columns
+// each, which first copy their columns' lists to LDS (8 KB a wavefront) and scan them there.  It runs beside the
+// launch for all other strips.  The fewer columns a wavefront has, the fewer rules it runs in a pass, and the more wavefronts
+// take slots from the other launch.  4096 lanes, this launch / the other, wavefronts a strip: 4: 0.88 / 0.97 ms, 8: 0.75 / 0.92,
+// 16: 0.81 / 1.00; 2048 lanes on a 1400-linedef map 4: 0.24 / 0.26, 8: 0.20 / 0.27, 16: 0.25 / 0.28.  A smaller batch leaves room and
+// lasts as long as its very longest strips: 512 lanes 4: 0.74 / 0.38, 8: 0.65 / 0.39, 16: 0.51 / 0.40, and 32 for 128 of the
+// strips, 8 for the others 0.45 / 0.41 (32 for 256: 0.49; 64 for 128: 0.54); 256 lanes 0.161 / 0.086, 0.128 / 0.090, 0.116 / 0.099,
+// 0.121 / 0.106; 1024 lanes 4: 0.38 / 0.28, 0.30 / 0.30 the last way.  Lists left in device memory: no gain.
 static_assert(SEG_COLS == 64 && SELECT_STRIPS_PER_GROUP == 1, "wall_select_kernel's staged launch: parts of one whole strip per work-group");
 template <bool SPLIT, bool STAGED>
-__global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kernel(DeviceMap dm, int lane_count, Scratch sc, int staged_slots) {
+__global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kernel(DeviceMap dm, int lane_count, Scratch sc, int staged_slots, int fine_slots) {
     const gd_map_desc *m = &dm.d;
     __shared__ LaneCtx lane_ctxs[SELECT_STRIPS_PER_GROUP][64 / SEG_COLS];
-    constexpr int PARTS = STAGED ? SELECT_STAGED_PARTS : 1, PART_COLS = 64 / PARTS;
-    __shared__ uint4 staged_entries[STAGED ? CAND_MAX * PART_COLS : 1];   // [CAND_MAX][PART_COLS] in the staged launch
+    constexpr int ROW = 64 / SELECT_PARTS;                              // columns of a wavefront of the staged launch, at most
+    __shared__ uint4 staged_entries[STAGED ? CAND_MAX * ROW : 1];       // [CAND_MAX][ROW] in the staged launch
+    // the staged launch: fine_slots strips of SELECT_FINE_PARTS wavefronts each, then the others of SELECT_PARTS
+    const int block = blockIdx.x, fine_blocks = fine_slots * SELECT_FINE_PARTS;
+    const bool fine = STAGED && block < fine_blocks;
+    const int parts = !STAGED ? 1 : (fine ? SELECT_FINE_PARTS : SELECT_PARTS), part_cols = 64 / parts;
+    const int from_block = STAGED && !fine ? block - fine_blocks : block, from_slot = STAGED && !fine ? fine_slots : 0;
     const int wave_in_group = threadIdx.x >> 6;
     const int lane_id = threadIdx.x & 63;
     const int segment_in_wave = lane_id / SEG_COLS;
-    const int segment_slot = (blockIdx.x / PARTS * SELECT_STRIPS_PER_GROUP + wave_in_group) * (64 / SEG_COLS) + segment_in_wave;
-    const int part = blockIdx.x % PARTS;
+    const int segment_slot = from_slot + (from_block / parts * SELECT_STRIPS_PER_GROUP + wave_in_group) * (64 / SEG_COLS) + segment_in_wave;
+    const int part = from_block % parts;
     const bool live = segment_slot < (STAGED ? staged_slots : lane_count * SEGS_PER_LANE);
     const int segment = live ? sc.strip_order[segment_slot] : 0;
     const int local = segment / SEGS_PER_LANE;
@@ -3546,8 +3559,8 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     const int strip_x = (segment - local * SEGS_PER_LANE) * SEG_COLS;
     const bool long_lists = __ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + lane_id] >> SPILL_SHIFT) != 0) != 0;
     if (STAGED ? long_lists : (segment_slot < staged_slots && !long_lists)) return;   // the same in the whole wavefront
-    if (lane_id >= PART_COLS) return;
-    const int x = strip_x + part * PART_COLS + lane_id;
+    if (lane_id >= part_cols) return;
+    const int x = strip_x + part * part_cols + lane_id;
     ColumnCtx cc;
     cc.tb = nullptr; cc.m = m; cc.mv.m = m; cc.c = &lane_ctx;
     cc.recs = sc.rec; cc.spans = sc.span;
@@ -3569,7 +3582,7 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
                 union { uint4 raw; Cand c; } u;
                 u.c = batch[j];
                 boundary_has_po |= (batch[j].flags & CF_LEDGE) != 0;   // slots past the end repeat the last entry
-                if (k0 + j < depth) *reinterpret_cast<uint4 *>(mine + (k0 + j) * (PART_COLS * 16)) = u.raw;
+                if (k0 + j < depth) *reinterpret_cast<uint4 *>(mine + (k0 + j) * (ROW * 16)) = u.raw;
             }
         }
         cc.staged = (ColumnCtx::LdsByte *)mine;
@@ -5588,12 +5601,13 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
             HIP_TRY(hipEventRecord(r->fork_event, stream));
             HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
             auto staged_kernel = split ? wall_select_kernel<true, true> : wall_select_kernel<false, true>;
-            hipLaunchKernelGGL(staged_kernel, dim3(staged_strips * SELECT_STAGED_PARTS), select_block, 0, stream, r->dm, count, sc, staged_strips);
-            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, r->side_stream, r->dm, count, sc, staged_strips);
+            const int fine_strips = count >= SELECT_FINE_LANES ? 0 : (strips < SELECT_FINE_STRIPS ? strips : SELECT_FINE_STRIPS);
+            hipLaunchKernelGGL(staged_kernel, dim3(fine_strips * SELECT_FINE_PARTS + (staged_strips - fine_strips) * SELECT_PARTS), select_block, 0, stream, r->dm, count, sc, staged_strips, fine_strips);
+            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, r->side_stream, r->dm, count, sc, staged_strips, 0);
             HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
             HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
         } else {
-            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0);
+            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0, 0);
         }
         mark();
         hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(count), dim3(SW), 0, stream, r->dm, count, sc);
