@@ -3656,6 +3656,11 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
 // sixteen of these wavefronts at 128 registers).  After the staging barrier the wavefronts never meet again.
 #define WALL_STRIPS_PER_GROUP 2
 #define RASTER_WAVES 4
+// A strip's wavefront draws, pass after pass, the rows that any of its columns draws; a small batch, which leaves wavefront slots
+// free and lasts as long as its longest strips, shares a strip out over several.  1 / 2 / 4 / 8 wavefronts a strip: 16 lanes
+// 0.123 / 0.103 / 0.105 / 0.094 ms, 48 lanes 0.201 / 0.162 / 0.148 / 0.147, 256 lanes 0.206 / 0.182 / 0.163 / 0.191, 512 lanes
+// 0.489 / 0.464 / 0.447 / 0.464, 1024 lanes 0.345 / 0.289 / 0.407 / 0.683.
+__host__ __device__ constexpr int raster_parts(int lanes) { return lanes <= 640 ? 4 : (lanes < 1536 ? 2 : 1); }
 // DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
 // BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
@@ -3672,7 +3677,9 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     const int wave_in_group = threadIdx.x >> 6;
     const int lane_id = threadIdx.x & 63;
     const int segment_in_wave = lane_id / SEG_COLS;
-    const int segment_slot = (blockIdx.x * WALL_STRIPS_PER_GROUP + wave_in_group) * (64 / SEG_COLS) + segment_in_wave;
+    const int wavefront = blockIdx.x * WALL_STRIPS_PER_GROUP + wave_in_group;
+    const int parts = raster_parts(lane_count);
+    const int segment_slot = wavefront / parts, part = wavefront % parts, part_cols = SEG_COLS / parts;
     const bool live = segment_slot < lane_count * SEGS_PER_LANE;
     const int segment = live ? sc.strip_order[segment_slot] : 0;
     const int local = segment / SEGS_PER_LANE;
@@ -3684,7 +3691,10 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     __syncthreads();
     if (!live) return;   // whole segments: the groups of four columns that exchange values below live or leave together
     const LaneCtx &lane_ctx = lane_ctxs[wave_in_group][segment_in_wave];
-    const int x = (segment - local * SEGS_PER_LANE) * SEG_COLS + (lane_id & (SEG_COLS - 1));
+    // a wavefront's columns are its first part_cols lanes; the others stand in for columns without a pass (the exchanges and
+    // the row walks of the wavefront need them executing) and leave before a column's end is written
+    const bool own_column = lane_id < part_cols;
+    const int x = (segment - local * SEGS_PER_LANE) * SEG_COLS + part * part_cols + (lane_id & (part_cols - 1));
     bool window_dirty = false;
     GapRange gaps; gaps.reset();
     ColumnCtx cc;
@@ -3711,7 +3721,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
     SilhouetteBounds sb; sb.bot_row = VH; sb.top_row = 0; sb.bot_depth = -GD_INF; sb.top_depth = -GD_INF;
-    const int passes = sc.pass_count[(size_t)local * SW + x];
+    const int passes = own_column ? sc.pass_count[(size_t)local * SW + x] : 0;
     const size_t first_record = sc.pass_at(0, local, x), pass_stride = (size_t)sc.lane_stride * SW;
     const unsigned int *geo_slots = sc.geo_slot + cc.rec_base;
     // A pass's record names its linedef, the linedef's slot where it lies in geo: the next pass's slot and the record after it
@@ -3771,6 +3781,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
             pass_advance<GENERAL, ADVANCE_CLIPS>(cc, st, pc, pb, sb, !window_dirty, gaps, &sc, first_record + (size_t)pass * pass_stride);
         }
     }
+    if (!own_column) return;
     // what is left of a window no one-sided drawseg closed shows the flat pass's picture
     if (!window_dirty) zero_rows(pb, gaps, x, st.ceiling_clip <= 0.0f ? 0 : (int)st.ceiling_clip, st.floor_clip >= (float)VH ? VH : (int)st.floor_clip);
     if (dm.masked_count > 0) masked_midtexture<DEPTH, GENERAL>(dm, cc, sc, local, st, pb, colormap_lds);
@@ -5611,7 +5622,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         }
         mark();
         hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(count), dim3(SW), 0, stream, r->dm, count, sc);
-        const dim3 grid((wavefronts + WALL_STRIPS_PER_GROUP - 1) / WALL_STRIPS_PER_GROUP), block(64 * WALL_STRIPS_PER_GROUP);
+        const dim3 grid((wavefronts * raster_parts(count) + WALL_STRIPS_PER_GROUP - 1) / WALL_STRIPS_PER_GROUP), block(64 * WALL_STRIPS_PER_GROUP);
         const bool general = split || m.sector_count > LDS_SECTORS || m.texture_count > LDS_TEXTURES;
         auto kernel = decals ? (general ? wall_raster_kernel<true, true> : wall_raster_kernel<true, false>)
                              : (general ? wall_raster_kernel<false, true> : wall_raster_kernel<false, false>);

@@ -1,0 +1,37 @@
+"""Batches on either side of the sizes at which the traversal shares a strip out over more or fewer wavefronts: every lane's
+frame is the one the CPU oracle draws for its camera."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from random_cases import closed_door_parts  # noqa: E402
+
+CAMERAS = 5
+
+
+@pytest.mark.parametrize("lanes", [1, 5, 25, 26, 103, 640, 641, 1535, 1536])
+def test_batches_around_the_sizes_of_the_traversals_rules_match_the_oracle(oracle, lanes):
+    from gradoom_amd import hostmath, mapbuild
+    from gradoom_amd.renderer import HipRenderer, LaneState
+    from gradoom_amd.selfcheck import make_lane_arrays
+
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    smap, poses, sprites, styles = closed_door_parts(6002, CAMERAS, mixed=True)
+    arrays = make_lane_arrays(smap, poses, sprites)
+    arrays["sprite_style"] = styles
+    tables = mapbuild.build_map_tables(smap)
+    expected = torch.as_tensor(oracle.render(tables, arrays, cosine)["indexed"]).to("cuda:0")
+    which = np.arange(lanes) % CAMERAS
+    renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+    indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+    state = LaneState.from_numpy({name: np.ascontiguousarray(value[which]) for name, value in arrays.items()}, "cuda:0")
+    renderer.render(state, indexed=indexed)
+    torch.cuda.synchronize()
+    assert renderer.status() == 0
+    assert torch.equal(indexed, expected[torch.as_tensor(which, device="cuda:0")])
+    renderer.close()
