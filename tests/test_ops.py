@@ -124,3 +124,23 @@ def test_both_operators_trace_through_torch_compile():
     renderer.close()
     with pytest.raises(RuntimeError, match="renderer is closed"):
         ops.render_lanes_(token, lanes, indexed=direct_indexed)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [208, 240])
+@pytest.mark.parametrize("offset", [0, 4, 5])
+def test_pooling_is_exact_for_any_address_of_the_frames(oracle, rows, offset):
+    # frames on 16 bytes, on words and on neither take different loads; the last columns read a word past their row
+    from gradoom_amd import ops
+
+    rng = np.random.default_rng(rows + offset)
+    indexed = rng.integers(0, 256, (3, rows, 320), dtype=np.uint8)
+    indexed[2] = 255
+    palette = rng.integers(0, 256, (256, 3), dtype=np.uint8)
+    palette[255] = 255   # the largest sums there are
+    expected, _ = oracle.observe(indexed, palette)
+    held = torch.zeros(indexed.size + 16, dtype=torch.uint8, device="cuda:0")
+    frames = held[offset:offset + indexed.size].view(indexed.shape)
+    frames.copy_(torch.as_tensor(indexed))
+    pooled = ops.policy_area_grayscale(frames, torch.as_tensor(palette).to("cuda:0"))
+    np.testing.assert_array_equal(pooled.cpu().numpy(), expected)
