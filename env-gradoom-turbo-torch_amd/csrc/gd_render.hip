@@ -4293,9 +4293,9 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(Device
                 if (listed <= SPRITE_CHUNK) s = sp[by_rank[tid]];
                 else (void)sprite_record(dm, lanes, n, L, by_rank[first + tid], x_first, x_first + SPRITE_COLUMNS, row_first, row_first + rows, s);
             }
-            if (tid < SPRITE_COLUMNS) cover[tid] = 0;
-            __syncthreads();                       // (also: every pixel of the chunk before is painted)
+            __syncthreads();                       // every pixel of the chunk before is painted: its records and bit sets are free
             if (tid < length) sp[tid] = s;
+            if (tid < SPRITE_COLUMNS) cover[tid] = 0;
             if (tid == 0) next_tile = 0;
             __syncthreads();
         }

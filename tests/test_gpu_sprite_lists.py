@@ -47,3 +47,40 @@ def test_billboard_lists_of_any_length_match_the_oracle(oracle, slots):
         assert renderer.status() == 0
         assert torch.equal(indexed.cpu(), expected.repeat(copies, 1, 1)), lanes
         renderer.close()
+
+
+@pytest.mark.parametrize("copies", [1, 128])   # quarters of a strip's rows, all rows at once
+def test_eight_chunks_of_billboards_in_one_strip_match_the_oracle(oracle, copies):
+    """All 512 slots a few degrees apart: one strip's list is painted in eight chunks, whose wavefronts end far apart since most
+    billboards reach the last rows only."""
+
+    from gradoom_amd import hostmath, mapbuild, synthmap
+    from gradoom_amd.renderer import HipRenderer, LaneState
+    from gradoom_amd.selfcheck import make_lane_arrays
+
+    slots = 512
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    smap, poses, _sprites, _styles = closed_door_parts(301, LANES, variants=False)
+    smap = synthmap.with_blend_tables(smap, 302)
+    sprites = synthmap.generate_sprites(smap, LANES, slots, 304)
+    rng = np.random.default_rng(305)
+    degrees = rng.uniform(2, 8, (LANES, slots)) + poses.angle_bam[:, None].astype(np.float64) / 4294967296.0 * 360.0
+    reach = rng.uniform(20, 400, (LANES, slots))
+    sprites.x[...] = poses.x[:, None] + (reach * np.cos(np.deg2rad(degrees))).astype(np.float32)
+    sprites.y[...] = poses.y[:, None] + (reach * np.sin(np.deg2rad(degrees))).astype(np.float32)
+    sprites.z[...] = poses.view_z[:, None] - 41.0 - (reach * rng.uniform(0, 0.4, (LANES, slots))).astype(np.float32)
+    arrays = make_lane_arrays(smap, poses, sprites)
+    arrays["sprite_style"] = rng.choice(np.array([-1, -1, -2, 0, 1], dtype=np.int8), size=(LANES, slots))
+    arrays["sprite_style"][::2] = -1
+    tables = mapbuild.build_map_tables(smap)
+    expected = torch.as_tensor(oracle.render(tables, arrays, cosine)["indexed"])
+    lanes = LANES * copies
+    tiled = {name: np.tile(value, (copies,) + (1,) * (value.ndim - 1)) for name, value in arrays.items()}
+    renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+    indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+    print(f"{lanes} lanes", flush=True)
+    renderer.render(LaneState.from_numpy(tiled, "cuda:0"), indexed=indexed)
+    torch.cuda.synchronize()
+    assert renderer.status() == 0
+    assert torch.equal(indexed.cpu(), expected.repeat(copies, 1, 1))
+    renderer.close()
