@@ -5279,6 +5279,7 @@ __global__ void __launch_bounds__(64) pack_weapon_kernel(gd_weapon_desc d) {
 // Every kernel of a frame runs on the caller's stream.  (Cutting a batch into chunks or halves pipelined over
 // more streams measured no faster: the kernels already fill the machine.)
 struct gd_renderer {
+    int device;                              // where everything below lies
     DeviceMap dm;
     Scratch sc;
     int chunk_lanes;
@@ -5777,9 +5778,10 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
     std::memset(&r->sc, 0, sizeof(r->sc));
     std::memset(&r->overlays, 0, sizeof(r->overlays));
     r->dm.d = *h;
+    r->device = 0;
     gd_map_desc &d = r->dm.d;
     const size_t W = h->wall_count, S = h->sector_count, V = h->vertex_count, K = h->neighbor_slots;
-    int rc = GD_OK;
+    int rc = hipGetDevice(&r->device) == hipSuccess ? GD_OK : fail(GD_E_HIP, "hipGetDevice");
 #define UP(field, count) if (rc == GD_OK) rc = upload(r, h->field, (size_t)(count), &d.field)
     UP(walls, W * 4); UP(walls_fixed, W * 4); UP(wall_sectors, W * 2); UP(wall_vertex, W * 2);
     UP(side_tex, W * 6); UP(side_off, W * 4); UP(wall_len, W);
@@ -5924,7 +5926,7 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
         }
     }
     if (rc == GD_OK) {
-        // in host memory: asking for it then is a wait for the device, not a copy behind the wait as well
+        // in host memory: whoever has waited for a frame reads them as they are (gd_renderer_status_seen)
         void *words = nullptr;
         if (hipHostMalloc(&words, 64) != hipSuccess) rc = fail(GD_E_HIP, "hipHostMalloc status");
         else { sc.status = static_cast<unsigned char *>(words); sc.status[0] = 0; sc.status[1] = 0; }
@@ -6046,13 +6048,24 @@ int gd_render_timed(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_o
     return GD_OK;
 }
 
-/* Sticky status bits of the renderer (synchronises the device): bit0 = a column had more than
-   CAND_MAX candidate linedefs and its list was truncated. Replaces nothing in the reference. */
-int gd_renderer_status(gd_renderer *r, int32_t *status) {
+/* Sticky status bits of the renderer: bit0 = a column had more than CAND_MAX candidate linedefs and its list was truncated.
+   Replaces nothing in the reference. */
+int gd_renderer_status_seen(gd_renderer *r, int32_t *status) {
     if (!r || !status) return fail(GD_E_ARG, "null argument");
-    HIP_TRY(hipDeviceSynchronize());
     *status = (r->sc.status[STATUS_CAND_OVERFLOW] ? 1 : 0) | (r->sc.status[STATUS_PASS_OVERFLOW] ? 2 : 0);
     return GD_OK;
+}
+
+/* The same once the renderer's device, which need not be the current one, has done all it was given. */
+int gd_renderer_status(gd_renderer *r, int32_t *status) {
+    if (!r || !status) return fail(GD_E_ARG, "null argument");
+    int current = 0;
+    HIP_TRY(hipGetDevice(&current));
+    if (current != r->device) HIP_TRY(hipSetDevice(r->device));
+    const hipError_t waited = hipDeviceSynchronize();
+    if (current != r->device) HIP_TRY(hipSetDevice(current));
+    HIP_TRY(waited);
+    return gd_renderer_status_seen(r, status);
 }
 
 /* Fill the renderer's working memory with one byte value.

@@ -379,7 +379,7 @@ class GraDoomVecEnv:
         else:
             done = transition.terminated | transition.truncated
             done_count = int(torch.count_nonzero(done))  # env.py:919: one host sync for the reference renderer
-        self.check_renderer_status()      # the device is idle here anyway
+        self.check_renderer_status()      # the stream has been waited for here anyway
         if not done_count:
             return DeviceAutoResetTransition(
                 transition.observations, transition.rewards, transition.terminated, transition.truncated,
@@ -405,9 +405,13 @@ class GraDoomVecEnv:
         batch (every column of up to eight lanes).
 
         Such a frame may differ from the reference's, which has no such bound, so it must not pass for a good one.
-        Synchronises the device: called where the environment already waits for it.
+        Waits for the current stream (called where the environment has waited for it already): what other streams run goes on.
         """
-        status = getattr(self._renderer, "status", None)
+        status = getattr(self._renderer, "status_seen", None)
+        if status is not None and self._native:
+            self._wait()
+        elif status is None:
+            status = getattr(self._renderer, "status", None)
         flags = status() if status is not None else 0
         if flags & 1:
             raise RuntimeError(
@@ -566,6 +570,8 @@ class GraDoomVecEnv:
         if not self.closed:
             self.closed = True
             try:
+                if self._native:
+                    torch.cuda.synchronize(self.device)   # frames may have been drawn on any stream
                 self.check_renderer_status()
             finally:
                 self._close_renderer()

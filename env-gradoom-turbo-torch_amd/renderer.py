@@ -141,8 +141,17 @@ class HipRenderer:
             pass
 
     def status(self) -> int:
+        """The sticky status bits, after a wait for everything on the renderer's device."""
+
         value = C.c_int32()
         _lib.check(self._lib.gd_renderer_status(self._handle, C.byref(value)))
+        return int(value.value)
+
+    def status_seen(self) -> int:
+        """The sticky status bits as the frames that have ended left them: no wait (the caller has waited for its frames)."""
+
+        value = C.c_int32()
+        _lib.check(self._lib.gd_renderer_status_seen(self._handle, C.byref(value)))
         return int(value.value)
 
     def set_assembly(self, assembly: str) -> None:

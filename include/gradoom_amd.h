@@ -288,7 +288,7 @@ int gd_render(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_out *ou
 int gd_render_static(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_out *out, void *stream);
 
 /*
- * Sticky status bits (synchronises the device).  bit0: some screen column had
+ * Sticky status bits (synchronises the renderer's device, every stream of it).  bit0: some screen column had
  * more candidate linedefs than the library keeps and was truncated - the frame
  * of that lane is not trustworthy.  A column keeps 64 in its own slots; one
  * that sees more moves to a spill pool (up to 256 per column; every column of
@@ -297,6 +297,12 @@ int gd_render_static(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_
  * Replaces nothing in the reference.
  */
 int gd_renderer_status(gd_renderer *r, int32_t *status);
+
+/*
+ * The same bits as the frames that have ended left them; waits for nothing.  For a caller that has waited for its own frames and
+ * would not wait for what other streams of the device run.  Replaces nothing in the reference.
+ */
+int gd_renderer_status_seen(gd_renderer *r, int32_t *status);
 
 /*
  * How a frame is put together once the walls are traversed.  GD_ASSEMBLY_SEPARATE: kernel by kernel through a

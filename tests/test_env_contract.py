@@ -290,3 +290,29 @@ def test_deferred_step_runs_when_waited_for(env):
         env.step_wait()
     env.step_async(torch.zeros(4, dtype=torch.int64))
     env.step_wait()
+
+
+def test_the_environment_asks_for_the_status_without_a_wait_for_the_device():
+    """It has waited for its own stream; a wait for the device would hold a step up for what other streams run."""
+    from gradoom_amd.env import GraDoomVecEnv
+
+    class SeenRenderer(RecordingRenderer):
+        def status(self):
+            raise AssertionError("a wait for the whole device")
+
+        def status_seen(self):
+            return self.status_value
+
+    renderer = SeenRenderer()
+    env = GraDoomVecEnv(load_fixture("tiny_stages")[2], 4, device="cpu", render_mode="rgb_array", renderer=renderer, episode_timeout=2)
+    env.reset_device(torch.ones(4, dtype=torch.bool), torch.arange(4))
+    actions = torch.zeros(4, dtype=torch.int64)
+    for _ in range(3):   # with and without lanes that end
+        env.step_and_reset_device(actions, torch.arange(4))
+    env.render()
+    env.get_images()
+    renderer.status_value = 2
+    with pytest.raises(RuntimeError, match="list of drawsegs"):
+        env.step_and_reset_device(actions, torch.arange(4))
+    with pytest.raises(RuntimeError, match="list of drawsegs"):
+        env.close()

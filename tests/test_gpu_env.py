@@ -108,3 +108,36 @@ def test_more_than_256_linedefs_in_one_column_raise_in_the_environment(monkeypat
     with pytest.raises(RuntimeError, match="truncated"):
         env.close()
     assert env.closed
+
+
+def test_a_step_does_not_wait_for_other_streams():
+    from gradoom_amd.env import GraDoomVecEnv
+
+    _meta, _data, smap, _tables = load_fixture("tiny_stages")
+    lanes = 3
+    env = GraDoomVecEnv(smap, lanes, device="cuda:0", episode_timeout=2)
+    env.reset_device(torch.ones(lanes, dtype=torch.bool, device="cuda:0"), torch.arange(lanes, device="cuda:0"))
+    actions, seeds = torch.zeros(lanes, dtype=torch.int64, device="cuda:0"), torch.arange(lanes, device="cuda:0")
+    for _ in range(4):
+        env.step_and_reset_device(actions, seeds)
+    # a kernel of some 50 ms on another stream; streams share a few hardware queues, so one of several must do
+    started, ended = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    cycles = 100_000
+    torch.cuda._sleep(cycles)
+    started.record()
+    torch.cuda._sleep(cycles)
+    ended.record()
+    torch.cuda.synchronize()
+    cycles = int(cycles * 50.0 / max(started.elapsed_time(ended), 0.01))
+    still_running = 0
+    for stream in [torch.cuda.Stream() for _ in range(6)]:
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(cycles)
+            ended.record()
+        env.step_and_reset_device(actions, seeds)
+        still_running += not ended.query()
+        torch.cuda.synchronize()
+    print(f"{still_running} of 6 steps ended before the other stream's kernel", flush=True)
+    assert still_running > 0
+    assert env._renderer.status_seen() == env._renderer.status() == 0
+    env.close()
