@@ -320,13 +320,21 @@ class GraDoomVecEnv:
         self.pending_reset.masked_fill_(device_mask, False)   # engine.py:2409
         self._update_signals()
 
+    def _lane_rows(self, rows: torch.Tensor) -> LaneState:
+        """The lane state of some lanes.  A dynamics object owes ``lane_state()`` and no more; the pool's own also takes the lanes."""
+
+        lane_state = self._dynamics.lane_state
+        if getattr(lane_state, "__func__", None) is PosePoolDynamics.lane_state:
+            return lane_state(rows)
+        return lane_state().select(rows)
+
     def _reset_rows(self, device_mask: torch.Tensor, seeds: torch.Tensor, count: int):
         """``_reset`` of the ``count`` lanes that ``_done_rows`` lists: only they are rendered, four copies each into their stacks."""
 
         device_seeds = self._require_device_tensor(seeds, "seeds", shape=(self.num_envs,), dtypes=INDEX_DTYPES).to(torch.int64).contiguous()
         self._dynamics.reset(device_mask, device_seeds)
         rows = self._done_rows[:count]
-        state = self._dynamics.lane_state(rows) if isinstance(self._dynamics, PosePoolDynamics) else self._dynamics.lane_state().select(rows)
+        state = self._lane_rows(rows)
         obs = torch.empty((count, 84, 84), dtype=torch.uint8, device=self.device)
         self._renderer.render(state, obs=obs)
         with torch.cuda.device(self.device):

@@ -316,3 +316,44 @@ def test_the_environment_asks_for_the_status_without_a_wait_for_the_device():
         env.step_and_reset_device(actions, torch.arange(4))
     with pytest.raises(RuntimeError, match="list of drawsegs"):
         env.close()
+
+
+def _overridden(smap, how):
+    """A pose pool whose ``lane_state`` takes no lanes: a method of a subclass, an attribute of the object, another class altogether."""
+    from gradoom_amd.env import PosePoolDynamics
+
+    class Lifted(PosePoolDynamics):
+        def lane_state(self):
+            state = super().lane_state()
+            state.view_z = state.view_z + 1.0
+            return state
+
+    class Wrapper:
+        def __init__(self, pool):
+            self.reset, self.step, self._pool = pool.reset, pool.step, pool
+
+        episode_time = property(lambda self: self._pool.episode_time)
+
+        def lane_state(self):
+            return self._pool.lane_state()
+
+    pool = (Lifted if how == "subclass" else PosePoolDynamics)(smap, 4, "cpu", sprites=3, episode_timeout=2)
+    if how == "attribute":
+        whole = pool.lane_state
+        pool.lane_state = lambda: whole()
+    return Wrapper(pool) if how == "wrapper" else pool
+
+
+@pytest.mark.parametrize("how", ["plain", "subclass", "attribute", "wrapper"])
+def test_the_lanes_that_reset_come_from_any_dynamics_lane_state(how):
+    from gradoom_amd.env import GraDoomVecEnv
+
+    smap = load_fixture("tiny_stages")[2]
+    dynamics = _overridden(smap, how)
+    env = GraDoomVecEnv(smap, 4, device="cpu", dynamics=dynamics, renderer=RecordingRenderer())
+    env.reset_device(torch.ones(4, dtype=torch.bool), torch.tensor([5, 3, 9, 1]))
+    rows = torch.tensor([1, 3])
+    whole, some = dynamics.lane_state(), env._lane_rows(rows)
+    for name, value in vars(whole).items():
+        assert (value is None) == (getattr(some, name) is None), name
+        assert value is None or torch.equal(getattr(some, name), value[rows]), name

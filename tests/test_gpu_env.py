@@ -141,3 +141,28 @@ def test_a_step_does_not_wait_for_other_streams():
     assert still_running > 0
     assert env._renderer.status_seen() == env._renderer.status() == 0
     env.close()
+
+
+def test_a_pose_pool_whose_lane_state_takes_no_lanes_resets_the_lanes_that_end():
+    from gradoom_amd.env import GraDoomVecEnv, PosePoolDynamics
+
+    class Lifted(PosePoolDynamics):
+        def lane_state(self):
+            state = super().lane_state()
+            state.view_z = state.view_z + 7.0
+            return state
+
+    _meta, _data, smap, _tables = load_fixture("tiny_stages")
+    lanes = 5
+    env = GraDoomVecEnv(smap, lanes, device="cuda:0", dynamics=Lifted(smap, lanes, "cuda:0", pool=7, episode_timeout=3))
+    env.reset_device(torch.ones(lanes, dtype=torch.bool, device="cuda:0"), torch.arange(lanes, device="cuda:0"))
+    actions, seeds = torch.zeros(lanes, dtype=torch.int64, device="cuda:0"), torch.arange(lanes, 0, -1, device="cuda:0")
+    env._dynamics.episode_time[3:] = 2       # two lanes end in the next step
+    transition = env.step_and_reset_device(actions, seeds)
+    assert transition.truncated.tolist() == [False, False, False, True, True]
+    obs = torch.zeros((lanes, 84, 84), dtype=torch.uint8, device="cuda:0")
+    env._renderer.render(env._dynamics.lane_state(), obs=obs)
+    for lane in (3, 4):
+        assert all(torch.equal(env.frames[lane, k], obs[lane]) for k in range(4))
+    assert torch.equal(env.frames[:3], transition.final_observations[:3])
+    env.close()
