@@ -320,6 +320,16 @@ class GraDoomVecEnv:
         self.pending_reset.masked_fill_(device_mask, False)   # engine.py:2409
         self._update_signals()
 
+    def _resets_alone(self) -> bool:
+        """May the lanes that end be rendered alone, around ``reset_device`` and the renderer's own stack update?
+
+        Only where both are this package's: an environment that overrides ``reset_device`` has it called, and another renderer
+        is asked for the frames of all lanes with a reset mask, as its interface has it.
+        """
+
+        own = lambda method, function: getattr(method, "__func__", None) is function  # noqa: E731
+        return own(self.reset_device, GraDoomVecEnv.reset_device) and own(getattr(self._renderer, "render", None), HipRenderer.render)
+
     def _lane_rows(self, rows: torch.Tensor) -> LaneState:
         """The lane state of some lanes.  A dynamics object owes ``lane_state()`` and no more; the pool's own also takes the lanes."""
 
@@ -393,7 +403,7 @@ class GraDoomVecEnv:
                 transition.observations, transition.rewards, transition.terminated, transition.truncated,
                 transition.signals, transition.info_histories, final_observations, final_signals, final_info_histories,
             )
-        if listed and done_count <= 65535:
+        if listed and done_count <= 65535 and self._resets_alone():
             observations, signals = self._reset_rows(self.pending_reset.clone(), reset_seeds, done_count)
         else:
             done = transition.terminated | transition.truncated

@@ -166,3 +166,39 @@ def test_a_pose_pool_whose_lane_state_takes_no_lanes_resets_the_lanes_that_end()
         assert all(torch.equal(env.frames[lane, k], obs[lane]) for k in range(4))
     assert torch.equal(env.frames[:3], transition.final_observations[:3])
     env.close()
+
+
+@pytest.mark.parametrize("how", ["environment", "renderer"])
+def test_a_reset_device_or_a_renderer_of_the_users_own_is_the_one_that_resets(how):
+    from gradoom_amd.env import GraDoomVecEnv
+    from gradoom_amd.renderer import HipRenderer
+
+    class Counting(GraDoomVecEnv):
+        resets = 0
+
+        def reset_device(self, mask, seeds):
+            self.resets += 1
+            return super().reset_device(mask, seeds)
+
+    class StackRenderer(HipRenderer):   # knows the calls that an environment made until now, and nothing of single observations
+        resets = 0
+
+        def render(self, lanes, *, frames, final_frames=None, reset_mask=None, obs=None, stack_only_masked=False, final_layout="chw"):
+            assert int(lanes.x.shape[0]) == self.max_lanes and obs is None
+            self.resets += reset_mask is not None
+            super().render(lanes, frames=frames, final_frames=final_frames, reset_mask=reset_mask, stack_only_masked=stack_only_masked, final_layout=final_layout)
+
+    _meta, _data, smap, _tables = load_fixture("tiny_stages")
+    lanes = 3
+    make = dict(device="cuda:0", episode_timeout=2)
+    plain = GraDoomVecEnv(smap, lanes, **make)
+    env = Counting(smap, lanes, **make) if how == "environment" else GraDoomVecEnv(smap, lanes, renderer=StackRenderer(smap, lanes, "cuda:0"), **make)
+    actions, seeds = torch.zeros(lanes, dtype=torch.int64, device="cuda:0"), torch.arange(lanes, device="cuda:0")
+    for each in (plain, env):
+        each.reset_device(torch.ones(lanes, dtype=torch.bool, device="cuda:0"), seeds)
+    for _ in range(3):               # every lane ends in the second
+        ours, theirs = env.step_and_reset_device(actions, seeds), plain.step_and_reset_device(actions, seeds)
+        assert torch.equal(ours.observations, theirs.observations) and torch.equal(ours.final_observations, theirs.final_observations)
+    assert (env if how == "environment" else env._renderer).resets == 2
+    for each in (plain, env):
+        each.close()
