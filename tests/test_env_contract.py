@@ -357,3 +357,57 @@ def test_the_lanes_that_reset_come_from_any_dynamics_lane_state(how):
     for name, value in vars(whole).items():
         assert (value is None) == (getattr(some, name) is None), name
         assert value is None or torch.equal(getattr(some, name), value[rows]), name
+
+
+def test_the_frames_handed_out_are_arrays_of_their_own(env):
+    env.reset_device(torch.ones(4, dtype=torch.bool), torch.arange(4))
+    frames = env.get_images() + [env.render_lane(2), env.render()]
+    assert isinstance(frames, list) and len(frames) == 6
+    for frame in frames:
+        assert frame.flags.owndata and frame.flags.writeable and frame.shape == (240, 320, 3) and frame.dtype == np.uint8 and frame.flags.c_contiguous
+
+
+def test_pooled_frames_keep_no_memory_but_their_own_and_give_it_back():
+    from gradoom_amd.env import _FramePool
+
+    class User:
+        pass
+
+    pool = _FramePool(2)
+    first, second = User(), User()
+    leave, _ = pool.join(first), pool.join(second)
+    picture = lambda value: np.full(_FramePool.SHAPE, value, dtype=np.uint8)  # noqa: E731
+    frames = [pool.copy_of(picture(k)) for k in range(4)]
+    for frame in frames:
+        assert frame.flags.writeable and frame.flags.c_contiguous and type(frame) is np.ndarray and frame.shape == _FramePool.SHAPE
+    assert [int(frame.min()) for frame in frames] == [int(frame.max()) for frame in frames] == [0, 1, 2, 3]
+    assert not any(np.shares_memory(a, b) for i, a in enumerate(frames) for b in frames[:i])
+    # a view keeps its frame's memory, also a view of a view and a tensor, and none but that
+    row, tensor, frame = frames[0][3][::2], torch.from_numpy(frames[1]), None
+    frames.clear()
+    assert len(pool._free) == 2
+    later = [pool.copy_of(picture(9)) for _ in range(3)]
+    assert not pool._free and int(row.max()) == 0 and int(tensor.min()) == int(tensor.max()) == 1
+    row = tensor = None
+    assert len(pool._free) == 2          # two more came back
+    later.clear()
+    assert len(pool._free) == 2          # and no more than two are kept
+    kept = pool.copy_of(picture(5))
+    leave()
+    leave()                              # leaving twice is leaving once
+    assert len(pool._free) == 1
+    del second                           # the last user, gone without a word
+    assert not pool._free
+    assert int(kept.min()) == int(kept.max()) == 5
+    del kept
+    assert not pool._free                # nobody would take it
+
+
+def test_an_environment_that_is_closed_leaves_the_frame_pool(env):
+    from gradoom_amd import env as module
+
+    users = module._FRAMES._users
+    env.close()
+    assert module._FRAMES._users == users - 1
+    env.close()
+    assert module._FRAMES._users == users - 1

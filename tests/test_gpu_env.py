@@ -202,3 +202,31 @@ def test_a_reset_device_or_a_renderer_of_the_users_own_is_the_one_that_resets(ho
     assert (env if how == "environment" else env._renderer).resets == 2
     for each in (plain, env):
         each.close()
+
+
+@pytest.mark.parametrize("room", [1, 2, 64])   # frames that the pinned staging memory holds
+def test_rgb_frames_are_arrays_of_their_own(monkeypatch, room):
+    from gradoom_amd.env import GraDoomVecEnv
+
+    monkeypatch.setattr(GraDoomVecEnv, "RGB_STAGING_BYTES", room * 240 * 320 * 3)
+    _meta, _data, smap, _tables = load_fixture("tiny_stages")
+    env = GraDoomVecEnv(smap, 5, device="cuda:0", render_mode="rgb_array")
+    env.reset_device(torch.ones(5, dtype=torch.bool, device="cuda:0"), torch.arange(5, device="cuda:0"))
+    rgb = torch.zeros((5, 240, 320, 3), dtype=torch.uint8, device="cuda:0")
+    env._renderer.render(env._dynamics.lane_state(), rgb=rgb)
+    expected = rgb.cpu().numpy()
+    frames = env.get_images()
+    assert len(frames) == 5 and all(np.array_equal(frame, expected[lane]) for lane, frame in enumerate(frames))
+    assert np.array_equal(env.render_lane(3), expected[3])
+    every = frames + env.get_images() + [env.render_lane(3)]
+    for at, frame in enumerate(every):   # an array each, none of which keeps another's memory
+        frame.fill(at)
+    assert all(int(frame.min()) == int(frame.max()) == at and frame.nbytes == 240 * 320 * 3 for at, frame in enumerate(every))
+    assert not any(np.shares_memory(frame, other) for at, frame in enumerate(every) for other in every[:at])
+    held = every[1][5]
+    frame = other = None
+    every.clear()
+    frames.clear()
+    assert all(np.array_equal(frame, expected[lane]) for lane, frame in enumerate(env.get_images()))
+    assert (held == 1).all()
+    env.close()
