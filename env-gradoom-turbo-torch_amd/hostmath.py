@@ -14,7 +14,8 @@ the lane tensors live on:
 * retained view angle ``bam.float() * (2π / 2³²)``      (``engine.py:10651``)
 
 Tensors on a ROCm device take one kernel of the library for the ray tables and one for the sprite depths, which
-give the Torch expressions' bits (``gd_ray_tables``, ``gd_sprite_depth``); everything else takes the expressions.
+give the Torch expressions' bits (``gd_ray_tables``, ``gd_sprite_depth``); everything else takes the expressions, and so
+does a call that Torch records, transforms or traces (a gradient, ``vmap``, forward mode, ``torch.compile``, fake tensors).
 """
 
 from __future__ import annotations
@@ -22,6 +23,8 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 SCREEN_WIDTH = 320
 BAM_TO_RADIANS = 2.0 * math.pi / float(1 << 32)
@@ -36,11 +39,25 @@ def cosine_correction(device) -> torch.Tensor:
     return torch.cos(native_ray_offsets(device))
 
 
+def _plain_call(*tensors: torch.Tensor) -> bool:
+    """Does this call want the values of these tensors and nothing else: is nothing recorded, transformed or traced?"""
+
+    return (
+        not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+        and all(type(t) is torch.Tensor and not t.is_neg() for t in tensors)
+        and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+        and forward_ad._current_level < 0                                  # dual numbers
+        and torch._C._functorch.peek_interpreter_stack() is None           # vmap, grad, jvp
+        and torch._C._len_torch_dispatch_stack() == 0                      # fake tensors, make_fx
+        and all(type(mode) is DeviceContext for mode in torch.overrides._get_current_function_mode_stack())   # torch.set_default_device is no matter
+    )
+
+
 def _on_device(*tensors: torch.Tensor) -> bool:
-    """Are these contiguous float32 tensors of one ROCm device, as the library's kernels read them?"""
+    """Are these contiguous float32 tensors of one ROCm device, as the library's kernels read them, and is only their result wanted?"""
 
     device = tensors[0].device
-    return device.type == "cuda" and all(t.dtype is torch.float32 and t.device == device and t.is_contiguous() for t in tensors)
+    return device.type == "cuda" and all(t.dtype is torch.float32 and t.device == device and t.is_contiguous() for t in tensors) and _plain_call(*tensors)
 
 
 def ray_tables(angle: torch.Tensor, offsets: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
