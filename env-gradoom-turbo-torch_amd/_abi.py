@@ -24,7 +24,7 @@ GD_E_ARG = -1
 GD_E_HIP = -2
 GD_E_UNSUPPORTED = -3
 
-ABI_VERSION = 4  # GD_ABI_VERSION
+ABI_VERSION = 5  # GD_ABI_VERSION
 
 _P = C.c_void_p
 
@@ -402,7 +402,7 @@ class PoseDesc(_Sized):
     """``gd_pose_desc``: a pool of poses, which of them each lane shows, and the lane tensors ``gd_pose_lanes`` writes."""
 
     _fields_ = (
-        [("struct_size", C.c_uint32), ("lane_count", C.c_int32), ("sprite_slots", C.c_int32), ("pool_size", C.c_int32), ("phase", _P), ("rows", _P)]
+        [("struct_size", C.c_uint32), ("lane_count", C.c_int32), ("sprite_slots", C.c_int32), ("pool_size", C.c_int32), ("phase_count", C.c_int32), ("phase", _P), ("rows", _P)]
         + [("pool_" + name, _P) for name in POSE_POOL_FIELDS]
         + [(name, _P) for name in POSE_LANE_FIELDS + POSE_SPRITE_FIELDS]
     )

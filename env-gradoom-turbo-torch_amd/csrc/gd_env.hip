@@ -22,10 +22,9 @@ __device__ __forceinline__ i64 floor_mod(i64 v, i64 n) { const i64 r = v % n; re
 // One work-group per lane: its pose by the first threads, its billboards by all of them.
 __global__ void __launch_bounds__(POSE_THREADS) pose_lanes_kernel(gd_pose_desc d) {
     const int lane = blockIdx.x;
-    const i64 row = d.rows ? d.rows[lane] : lane;
-    i64 pose = d.phase[row];
-    pose = pose < 0 ? pose + d.pool_size : pose;                                        // a negative index counts from the end
-    pose = pose < 0 ? 0 : (pose >= d.pool_size ? d.pool_size - 1 : pose);
+    // a negative index counts from the end; one beyond either end is the one there
+    auto inside = [](i64 at, i64 count) { at = at < 0 ? at + count : at; return at < 0 ? 0 : (at >= count ? count - 1 : at); };
+    const i64 pose = inside(d.phase[d.rows ? inside(d.rows[lane], d.phase_count) : lane], d.pool_size);
     if (threadIdx.x == 0) {
         const float BAM_TO_RADIANS = (float)(2.0 * 3.14159265358979323846 / 4294967296.0);   // engine.py:10651
         const float x = d.pool_x[pose], y = d.pool_y[pose];
@@ -133,7 +132,8 @@ extern "C" {
 int gd_pose_lanes(const gd_pose_desc *d, void *stream) {
     if (!d) return gd_fail(GD_E_ARG, "null argument");
     GD_SIZE_CHECK(d, gd_pose_desc);
-    if (d->lane_count < 0 || d->sprite_slots < 0 || d->pool_size <= 0) return gd_fail(GD_E_ARG, "gd_pose_desc holds a count out of range");
+    if (d->lane_count < 0 || d->sprite_slots < 0 || d->pool_size <= 0 || d->phase_count <= 0 || (!d->rows && d->lane_count > d->phase_count))
+        return gd_fail(GD_E_ARG, "gd_pose_desc holds a count out of range");
     if (d->lane_count == 0) return GD_OK;
     const void *const needed[] = {d->phase, d->pool_x, d->pool_y, d->pool_view_z, d->pool_angle_bam, d->pool_pitch_bam, d->pool_flash_light,
                                   d->x, d->y, d->angle, d->view_z, d->x_fixed, d->y_fixed, d->angle_bam, d->pitch_bam, d->flash_light};

@@ -196,10 +196,11 @@ class PosePoolDynamics:
         return rewards, terminated, truncated
 
     def lane_state(self, rows: torch.Tensor | None = None) -> LaneState:
-        """The lane state of every lane, or of the lanes that ``rows`` (int64, on the device) names."""
+        """The lane state of every lane, or of the lanes that ``rows`` (indices of one dimension, on the device) names."""
 
         pool = self._pool
-        if self._on_device() and all(value.is_contiguous() for value in pool.values()):
+        taken = rows is None or (isinstance(rows, torch.Tensor) and rows.dim() == 1 and _kernel_ready(rows, torch.int64, rows.shape[0], self.phase.device))
+        if taken and self._on_device() and all(value.is_contiguous() for value in pool.values()):
             return self._lane_state_kernel(rows)
         index = self.phase if rows is None else self.phase[rows]
         x, y = pool["x"][index], pool["y"][index]
@@ -217,7 +218,7 @@ class PosePoolDynamics:
         count = self.num_envs if rows is None else int(rows.shape[0])
         device = self.device
         desc = _abi.PoseDesc()
-        desc.lane_count, desc.pool_size, desc.phase = count, self._pool_size, self.phase.data_ptr()
+        desc.lane_count, desc.pool_size, desc.phase, desc.phase_count = count, self._pool_size, self.phase.data_ptr(), self.num_envs
         if rows is not None:
             desc.rows = rows.data_ptr()
         pool = self._pool

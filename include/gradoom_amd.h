@@ -45,7 +45,7 @@ extern "C" {
  * Layout version of the structs below.  Every descriptor also starts with its own sizeof, which each entry
  * point checks: a caller built against another header gets GD_E_ARG instead of a wild read.
  */
-#define GD_ABI_VERSION 4
+#define GD_ABI_VERSION 5
 
 #define GD_OK 0
 #define GD_E_ARG (-1)       /* bad argument: null pointer, negative count, size over a limit */
@@ -523,8 +523,10 @@ int gd_sprite_depth(const float *x, const float *y, const float *angle, const fl
 typedef struct gd_pose_desc {
     uint32_t struct_size;    /* sizeof(gd_pose_desc) of the header the caller was built with */
     int32_t lane_count, sprite_slots, pool_size;
+    int32_t phase_count;                 /* entries of phase */
     const int64_t *phase;
-    const int64_t *rows;                 /* [lane_count], or null */
+    const int64_t *rows;                 /* [lane_count] entries of phase to show (negative: from the end; beyond either end: the one there),
+                                            or null: the first lane_count */
     const float *pool_x;                 /* [pool_size] */
     const float *pool_y;
     const float *pool_view_z;

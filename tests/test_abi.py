@@ -141,3 +141,32 @@ def test_create_refuses_indices_outside_their_tables(small_tables, field, index,
     lib, desc, keep, cosine, handle = _create(tables)
     with pytest.raises(ValueError, match=message):
         _lib.check(lib.gd_renderer_create(ctypes.byref(desc), cosine.ctypes.data, 4, ctypes.byref(handle)))
+
+
+def test_the_pose_descriptor_lies_where_the_header_has_it(tmp_path):
+    import subprocess
+
+    from gradoom_amd import _abi
+
+    fields = [name for name, _ in _abi.PoseDesc._fields_]
+    source = tmp_path / "offsets.c"
+    source.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "gradoom_amd.h"\nint main(void) { printf("%zu", sizeof(gd_pose_desc));\n'
+                      + "".join(f'printf(" %zu", offsetof(gd_pose_desc, {name}));\n' for name in fields) + "return 0; }\n")
+    binary = tmp_path / "offsets"
+    subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), str(source), "-o", str(binary)], check=True)
+    numbers = [int(v) for v in subprocess.run([str(binary)], check=True, capture_output=True, text=True).stdout.split()]
+    assert numbers == [ctypes.sizeof(_abi.PoseDesc)] + [getattr(_abi.PoseDesc, name).offset for name in fields]
+
+
+@pytest.mark.parametrize("phase_count, rows, lanes", [(0, False, 1), (-1, True, 1), (3, False, 4)])
+def test_pose_lanes_beyond_the_phases_are_refused_on_the_host(phase_count, rows, lanes):
+    from gradoom_amd import _abi, _build, _lib
+
+    if not os.path.exists(_build.LIBRARY):
+        pytest.skip("libgradoom_amd.so not built (run __graft_entry__.build())")
+    desc = _abi.PoseDesc()
+    desc.lane_count, desc.pool_size, desc.phase_count = lanes, 7, phase_count
+    if rows:
+        desc.rows = 256
+    with pytest.raises(ValueError, match="count out of range"):
+        _lib.check(_lib.library().gd_pose_lanes(ctypes.byref(desc), None))

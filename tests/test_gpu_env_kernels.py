@@ -76,3 +76,25 @@ def test_rgb_expansion_in_device_and_pinned_memory(lanes, rows):
         assert np.array_equal(rgb.cpu().numpy(), np.asarray(tables["playpal"])[indexed.cpu().numpy()])
         assert bool((guarded[offset + lanes * rows * 960 :] == 7).all())
     renderer.close()
+
+
+@pytest.mark.parametrize("form", ["int64", "int32", "strided", "two_dimensions", "list", "negative", "none"])
+def test_the_lanes_asked_of_a_pose_pool_may_come_in_any_form(form):
+    """A kernel reads int64 rows of one contiguous piece; whatever else is handed in goes the way of the Torch expressions."""
+    from gradoom_amd.env import PosePoolDynamics
+
+    _meta, _data, smap, _tables = load_fixture("tiny_stages")
+    pools = [PosePoolDynamics(smap, 9, device, pool=7, sprites=3, seed=5) for device in ("cuda:0", "cpu")]
+    rows = torch.tensor([8, 1, 1, 0, 5, 3])
+    rows = {"int64": rows, "int32": rows.to(torch.int32), "strided": torch.stack([rows, rows.flip(0)], 1)[:, 1], "two_dimensions": rows.view(2, 3),
+            "list": rows.tolist(), "negative": rows - 9, "none": rows[:0]}[form]
+    for pool in pools:
+        pool.reset(torch.ones(9, dtype=torch.bool, device=pool.device), torch.arange(9, device=pool.device))
+    on_device = rows if isinstance(rows, list) else rows.to("cuda:0")
+    if form == "strided":
+        on_device = torch.stack([on_device, on_device], 1)[:, 0]
+        assert not on_device.is_contiguous()
+    print(form, flush=True)
+    ours, theirs = pools[0].lane_state(on_device), pools[1].lane_state(rows)
+    for name, value in vars(theirs).items():
+        assert value is None or torch.equal(getattr(ours, name).cpu(), value), name
