@@ -286,7 +286,8 @@ struct Scratch {    // per-chunk working memory, sized at create
     float *pass_path_distance;  // [pass_slots,L,320] distance of the portal path of a pass that carries PB_PS_KEEPS (written for those only)
     unsigned char *pass_count;  // [L,320] passes recorded for the column: up to its last pass that draws or moves a clip
     unsigned int *meta;    // [L,208,320] filled | floor | plane_sector+1 | clip_wall+1
-    unsigned char *masked_texel; // [L,208,320] palette indices of masked mid-textures, where no frame takes them (band_finish_kernel)
+    unsigned char *masked_texel; // [L,208,320] palette indices of masked mid-textures, where no frame takes them (band_finish_kernel); null
+                                 // unless the assembly in LDS was chosen
     unsigned char *frame;  // [L,240,320] when the caller wants no indexed output
     u64 *block_hit;        // [L,320] nearest blocking linedef of the column ray: float bits of the distance << 32 |
                            // slot in blocking_walls, all ones when no ray hits (engine.py:10534-10557)
@@ -5300,6 +5301,18 @@ struct gd_renderer {
 
 namespace {
 
+// A renderer's device as the current one, for a call that does not launch on a caller's stream.
+struct OnDevice {
+    int before = -1;
+    hipError_t error;
+    explicit OnDevice(int device) {
+        error = hipGetDevice(&before);
+        if (error == hipSuccess && before != device) error = hipSetDevice(device);
+        else before = -1;
+    }
+    ~OnDevice() { if (before >= 0) (void)hipSetDevice(before); }
+};
+
 // Working memory of callers that may not allocate (gd_render_static): one array per device, held until the
 // process ends.  In host code the array's name only stands for the symbol; its address on the current
 // device comes from hipGetSymbolAddress, once per device.
@@ -5369,9 +5382,8 @@ size_t spill_pool_blocks(int lanes) {
 // Lay the per-chunk buffers of `sc` out in one block of device memory for `L` lanes of map `h` (every buffer
 // 256-byte aligned) and return the bytes the layout takes; with a null `base` nothing is assigned and the call
 // only measures.  `status` is not part of the block: the renderer keeps it.  `depth`: also the scene depth plane
-// of frames that draw decals.
-size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_desc &h, int masked_count, bool depth, size_t spill_blocks) {
-    // `depth`: frames that draw decals also need a scene depth plane
+// of frames that draw decals; `fused`: also the texels of masked mid-textures that are put together in LDS.
+size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_desc &h, int masked_count, bool depth, bool fused, size_t spill_blocks) {
     size_t used = 0;
     auto take = [&](auto **field, size_t count) {
         typedef typename std::remove_reference<decltype(**field)>::type T;
@@ -5413,7 +5425,7 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.pass_rows, L * (size_t)sc.pass_slots * SW);
     take(&sc.pass_count, L * SW);
     take(&sc.meta, L * PX);
-    take(&sc.masked_texel, L * PX);
+    if (fused && masked_count > 0) take(&sc.masked_texel, L * PX);
     take(&sc.level_reach, L * levels);
     take(&sc.level_far, L * levels);
     take(&sc.level_masks, L * LEVEL_BUCKETS * (size_t)(levels <= 32 * LEVEL_MASK_WORDS_MAX ? (levels + 31) / 32 : 1));
@@ -5587,6 +5599,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     if (!decals) sc.scene_depth = nullptr;
     if (decals && (!sc.scene_depth || !sc.frame)) return fail(GD_E_ARG, "decal working memory missing");
     const bool fused = !decals && (r->assembly == GD_ASSEMBLY_FUSED || (r->assembly == GD_ASSEMBLY_AUTO && !out->indexed && !sc.frame));
+    if (fused && r->dm.masked_count > 0 && !sc.masked_texel) return fail(GD_E_ARG, "masked mid-texture working memory missing");
     unsigned char *frame_base = nullptr;
     if (!fused) {
         frame_base = out->indexed ? out->indexed + (size_t)base * frame_stride : sc.frame;
@@ -5918,10 +5931,10 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
     Scratch &sc = r->sc;
     if (rc == GD_OK && chunk > 0) {
         unsigned char *block = nullptr;
-        const size_t bytes = carve_scratch(sc, nullptr, (size_t)chunk, *h, r->dm.masked_count, false, spill_pool_blocks(chunk));
+        const size_t bytes = carve_scratch(sc, nullptr, (size_t)chunk, *h, r->dm.masked_count, false, false, spill_pool_blocks(chunk));
         rc = scratch_alloc(r, bytes, &block);
         if (rc == GD_OK) {
-            carve_scratch(sc, block, (size_t)chunk, *h, r->dm.masked_count, false, spill_pool_blocks(chunk));
+            carve_scratch(sc, block, (size_t)chunk, *h, r->dm.masked_count, false, false, spill_pool_blocks(chunk));
             r->scratch_block = block; r->scratch_bytes = bytes;
         }
     }
@@ -6003,17 +6016,19 @@ int gd_render_static(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_
     const gd_map_desc &m = r->dm.d;
     const bool decals = lanes->decal_slots > 0 && lanes->decal_state && lanes->decal_geom && r->overlays.d.decal_variant_count > 0;
     Scratch sc = r->sc;   // keeps the renderer's status word
-    const size_t one = carve_scratch(sc, nullptr, 1, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS), two = carve_scratch(sc, nullptr, 2, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS);
+    const bool fused = r->assembly == GD_ASSEMBLY_FUSED;
+    auto carve = [&](unsigned char *at, size_t L) { return carve_scratch(sc, at, L, m, r->dm.masked_count, decals, fused, STATIC_SPILL_BLOCKS); };
+    const size_t one = carve(nullptr, 1), two = carve(nullptr, 2);
     if (one > STATIC_SCRATCH_BYTES)
         return fail(GD_E_ARG, "map too large for gd_render_static: one lane needs " + std::to_string(one) + " bytes of working memory, the static block holds " +
                                   std::to_string(STATIC_SCRATCH_BYTES));
     // the layout grows by a fixed amount per lane, up to the padding between its buffers
     size_t fit = 1 + (STATIC_SCRATCH_BYTES - one) / (two - one);
-    while (fit > 1 && carve_scratch(sc, nullptr, fit, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS) > STATIC_SCRATCH_BYTES) --fit;
+    while (fit > 1 && carve(nullptr, fit) > STATIC_SCRATCH_BYTES) --fit;
     const int chunk = fit > 4096 ? 4096 : (int)fit;
     if (lanes->lane_count > GD_STATIC_MAX_LANES)
         return fail(GD_E_ARG, "gd_render_static renders at most " + std::to_string(GD_STATIC_MAX_LANES) + " lanes per call");
-    carve_scratch(sc, block, (size_t)chunk, m, r->dm.masked_count, decals, STATIC_SPILL_BLOCKS);
+    carve(block, (size_t)chunk);
     hipStream_t caller = static_cast<hipStream_t>(stream);
     // the block keeps whatever the last call left: the kernels expect nothing of it
     for (int base = 0; base < lanes->lane_count; base += chunk) {
@@ -6059,12 +6074,9 @@ int gd_renderer_status_seen(gd_renderer *r, int32_t *status) {
 /* The same once the renderer's device, which need not be the current one, has done all it was given. */
 int gd_renderer_status(gd_renderer *r, int32_t *status) {
     if (!r || !status) return fail(GD_E_ARG, "null argument");
-    int current = 0;
-    HIP_TRY(hipGetDevice(&current));
-    if (current != r->device) HIP_TRY(hipSetDevice(r->device));
-    const hipError_t waited = hipDeviceSynchronize();
-    if (current != r->device) HIP_TRY(hipSetDevice(current));
-    HIP_TRY(waited);
+    OnDevice on(r->device);
+    HIP_TRY(on.error);
+    HIP_TRY(hipDeviceSynchronize());
     return gd_renderer_status_seen(r, status);
 }
 
@@ -6076,6 +6088,8 @@ int gd_renderer_scribble(gd_renderer *r, int32_t value, void *stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     const unsigned int byte = (unsigned int)value & 0xFFu, word = byte * 0x01010101u;
     hipLaunchKernelGGL(fill_words_kernel, dim3(4096), dim3(256), 0, st, reinterpret_cast<unsigned int *>(r->scratch_block), r->scratch_bytes / 4, word);
+    if (r->sc.masked_texel)
+        hipLaunchKernelGGL(fill_words_kernel, dim3(4096), dim3(256), 0, st, reinterpret_cast<unsigned int *>(r->sc.masked_texel), (size_t)r->chunk_lanes * VH * SW / 4, word);
     HIP_TRY(hipGetLastError());
     return GD_OK;
 }
@@ -6083,6 +6097,12 @@ int gd_renderer_scribble(gd_renderer *r, int32_t value, void *stream) {
 int gd_renderer_set_assembly(gd_renderer *r, int32_t assembly) {
     if (!r) return fail(GD_E_ARG, "null argument");
     if (assembly != GD_ASSEMBLY_AUTO && assembly != GD_ASSEMBLY_FUSED && assembly != GD_ASSEMBLY_SEPARATE) return fail(GD_E_ARG, "unknown assembly");
+    if (assembly == GD_ASSEMBLY_FUSED && r->chunk_lanes > 0 && r->dm.masked_count > 0 && !r->sc.masked_texel) {
+        // the one plane that only this assembly uses: 65 KB a lane
+        OnDevice on(r->device);
+        HIP_TRY(on.error);
+        if (int rc = scratch_alloc(r, (size_t)r->chunk_lanes * VH * SW, &r->sc.masked_texel)) return rc;
+    }
     r->assembly = assembly;
     return GD_OK;
 }

@@ -316,6 +316,7 @@ int gd_renderer_status_seen(gd_renderer *r, int32_t *status);
 #define GD_ASSEMBLY_AUTO 0
 #define GD_ASSEMBLY_FUSED 1
 #define GD_ASSEMBLY_SEPARATE 2
+/* The first call with GD_ASSEMBLY_FUSED allocates 65 KB of working memory a lane where the map has masked mid-textures. */
 int gd_renderer_set_assembly(gd_renderer *r, int32_t assembly);
 
 /*
