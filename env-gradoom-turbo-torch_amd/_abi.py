@@ -18,7 +18,7 @@ LAYOUT_CHW = 0
 LAYOUT_HWC = 1
 
 GD_OK = 0
-STATIC_SCRATCH_MIB = 64  # gd_render_static: the fixed per-GPU working memory
+STATIC_SCRATCH_MIB = 96  # gd_render_static: the fixed per-GPU working memory
 STATIC_MAX_LANES = 65536
 GD_E_ARG = -1
 GD_E_HIP = -2

@@ -5314,7 +5314,8 @@ struct OnDevice {
 };
 
 // Working memory of callers that may not allocate (gd_render_static): one array per device, held until the
-// process ends.  In host code the array's name only stands for the symbol; its address on the current
+// process ends; about twenty lanes of a 4000-linedef map.  (A batch lasts as long as its longest strips, so a chunk more costs the
+// time of a small batch: 16 such lanes 0.55 ms in one chunk, 0.97 ms in the two that 64 MiB make of them.)  In host code the array's name only stands for the symbol; its address on the current
 // device comes from hipGetSymbolAddress, once per device.
 #define STATIC_SCRATCH_BYTES ((size_t)GD_STATIC_SCRATCH_MIB << 20)
 #define STATIC_SCRATCH_DEVICES 64

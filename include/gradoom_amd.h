@@ -283,7 +283,7 @@ int gd_render(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_out *ou
  * for more than GD_STATIC_MAX_LANES lanes.  Calls no hipMalloc / hipFree.  Every call on a GPU uses that
  * GPU's one array: calls that overlap on one GPU (two streams, two threads) race.
  */
-#define GD_STATIC_SCRATCH_MIB 64
+#define GD_STATIC_SCRATCH_MIB 96
 #define GD_STATIC_MAX_LANES 65536
 int gd_render_static(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_out *out, void *stream);
 

@@ -170,3 +170,11 @@ def test_pose_lanes_beyond_the_phases_are_refused_on_the_host(phase_count, rows,
         desc.rows = 256
     with pytest.raises(ValueError, match="count out of range"):
         _lib.check(_lib.library().gd_pose_lanes(ctypes.byref(desc), None))
+
+
+def test_the_static_array_is_as_long_as_the_binding_says():
+    from gradoom_amd import _abi
+
+    text = open(os.path.join(ROOT, "include", "gradoom_amd.h")).read()
+    assert int(re.search(r"#define GD_STATIC_SCRATCH_MIB (\d+)", text).group(1)) == _abi.STATIC_SCRATCH_MIB
+    assert int(re.search(r"#define GD_STATIC_MAX_LANES (\d+)", text).group(1)) == _abi.STATIC_MAX_LANES
