@@ -1940,9 +1940,15 @@ __global__ void __launch_bounds__(SW) flat_span_finish_kernel(Scratch sc) {
 // wall_select_kernel's launch for the longest strips
 #define SELECT_STAGED_STRIPS 512   // how many strips,
 #define SELECT_PARTS 8             // and over how many wavefronts each is shared out;
-#define SELECT_FINE_STRIPS 128     // in a batch of fewer than SELECT_FINE_LANES lanes the very longest are shared out over more
+#define SELECT_FINE_STRIPS 128     // in a small batch the very longest are shared out over more
 #define SELECT_FINE_PARTS 32
-#define SELECT_FINE_LANES 1536
+// A small batch lasts as long as its longest strips, a larger one as long as all of its strips together take on the wavefront
+// slots there are; sharing the longest strips out further shortens the first and adds to the second.  Up to where that pays
+// follows the map's linedefs, which make the longest lists: 160 lanes at 320 linedefs, 400 at 800 (450 at 701 in bricks), 500 at 1400, 650 at 2000,
+// 1000 at 3000, 1250 at 4000.  Stage times in us without / with fine parts: 320 linedefs, 128 lanes 88 / 81, 384 lanes 94 / 118, 1024 lanes
+// 140 / 155; 800, 256 lanes 147 / 128, 512 lanes 149 / 158; 2000, 256 lanes 263 / 196, 512 lanes 269 / 244, 768 lanes 283 / 283, 1024 lanes 309 / 317;
+// 4000, 256 lanes 534 / 372, 768 lanes 585 / 498, 1024 lanes 612 / 551, 1280 lanes 628 / 617, 1536 lanes 657 / 665.
+bool select_finely(int lanes, int linedefs) { return lanes < 192 + (linedefs < 4096 ? linedefs : 4096) / 4; }   // no map of more was timed
 #define WALL_ROWS 8          // rows painted / clipped per step of the wall traversal
 struct ColumnCtx {
     const Tables *tb;
@@ -3657,11 +3663,20 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
 // sixteen of these wavefronts at 128 registers).  After the staging barrier the wavefronts never meet again.
 #define WALL_STRIPS_PER_GROUP 2
 #define RASTER_WAVES 4
-// A strip's wavefront draws, pass after pass, the rows that any of its columns draws; a small batch, which leaves wavefront slots
-// free and lasts as long as its longest strips, shares a strip out over several.  1 / 2 / 4 / 8 wavefronts a strip: 16 lanes
-// 0.123 / 0.103 / 0.105 / 0.094 ms, 48 lanes 0.201 / 0.162 / 0.148 / 0.147, 256 lanes 0.206 / 0.182 / 0.163 / 0.191, 512 lanes
-// 0.489 / 0.464 / 0.447 / 0.464, 1024 lanes 0.345 / 0.289 / 0.407 / 0.683.
-__host__ __device__ constexpr int raster_parts(int lanes) { return lanes <= 640 ? 4 : (lanes < 1536 ? 2 : 1); }
+// A strip's wavefront draws, pass after pass, the rows that any of its columns draws.  A small batch, which lasts as long as its
+// longest strips, shares a strip out over four wavefronts, a larger one over two.  Where the lines lie best depends on how much
+// longer a map's longest strips are than its others, which the host does not know: four are as good as two at 430 (320 linedefs) to 700
+// lanes (701 linedefs in bricks), two as good as one at 1150 to some 1700; both lines lie between, where no map loses much to
+// the other choice.  Stage times in us (wall_geometry_kernel among them) for 1 / 2 / 4 / 8 wavefronts a strip:
+//   lanes             320 linedefs        2000                4000                701, bricks
+//     128       190 / 165 / 156 / 157   240 / 210 / 205   402 / 380 / 359   412 / 370 / 338 / 339
+//     512       217 / 198 / 211 / 318   300 / 266 / 286   493 / 441 / 413   453 / 380 / 353 / 412
+//     640       243 / 213 / 250         320 / 290 / 328   518 / 470 / 449   475 / 396 / 367
+//    1024       275 / 264 / 366         375 / 358 / 477   616 / 529 / 666   524 / 439 / 495
+//    1280       302 / 314               400 / 426         653 / 618         544 / 451
+//    1536       320 / 362               456 / 495         695 / 704         561 / 511
+//    2048       383 / 464               535 / 633         755 / 881
+__host__ __device__ constexpr int raster_parts(int lanes) { return lanes <= 560 ? 4 : (lanes <= 1344 ? 2 : 1); }
 // DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
 // BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
@@ -5632,7 +5647,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
             HIP_TRY(hipEventRecord(r->fork_event, stream));
             HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
             auto staged_kernel = split ? wall_select_kernel<true, true> : wall_select_kernel<false, true>;
-            const int fine_strips = count >= SELECT_FINE_LANES ? 0 : (strips < SELECT_FINE_STRIPS ? strips : SELECT_FINE_STRIPS);
+            const int fine_strips = !select_finely(count, m.wall_count) ? 0 : (strips < SELECT_FINE_STRIPS ? strips : SELECT_FINE_STRIPS);
             hipLaunchKernelGGL(staged_kernel, dim3(fine_strips * SELECT_FINE_PARTS + (staged_strips - fine_strips) * SELECT_PARTS), select_block, 0, stream, r->dm, count, sc, staged_strips, fine_strips);
             hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, r->side_stream, r->dm, count, sc, staged_strips, 0);
             HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
