@@ -42,22 +42,31 @@ def cosine_correction(device) -> torch.Tensor:
 def _plain_call(*tensors: torch.Tensor) -> bool:
     """Does this call want the values of these tensors and nothing else: is nothing recorded, transformed or traced?"""
 
-    return (
-        not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-        and all(type(t) is torch.Tensor and not t.is_neg() for t in tensors)
-        and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-        and forward_ad._current_level < 0                                  # dual numbers
-        and torch._C._functorch.peek_interpreter_stack() is None           # vmap, grad, jvp
-        and torch._C._len_torch_dispatch_stack() == 0                      # fake tensors, make_fx
-        and all(type(mode) is DeviceContext for mode in torch.overrides._get_current_function_mode_stack())   # torch.set_default_device is no matter
-    )
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0:   # vmap, grad, jvp; dual numbers
+        return False
+    if torch._C._len_torch_dispatch_stack() > 0:                                                     # fake tensors, make_fx
+        return False
+    if torch._C._len_torch_function_stack() > 0 and any(type(mode) is not DeviceContext for mode in torch.overrides._get_current_function_mode_stack()):
+        return False                                                                                 # (torch.set_default_device is no matter)
+    recorded = torch.is_grad_enabled()
+    for tensor in tensors:
+        if type(tensor) is not torch.Tensor or tensor.is_neg() or (recorded and tensor.requires_grad):
+            return False
+    return True
 
 
 def _on_device(*tensors: torch.Tensor) -> bool:
     """Are these contiguous float32 tensors of one ROCm device, as the library's kernels read them, and is only their result wanted?"""
 
     device = tensors[0].device
-    return device.type == "cuda" and all(t.dtype is torch.float32 and t.device == device and t.is_contiguous() for t in tensors) and _plain_call(*tensors)
+    if device.type != "cuda" or not _plain_call(*tensors):
+        return False
+    for tensor in tensors:
+        if tensor.dtype is not torch.float32 or tensor.device != device or not tensor.is_contiguous():
+            return False
+    return True
 
 
 def ray_tables(angle: torch.Tensor, offsets: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
