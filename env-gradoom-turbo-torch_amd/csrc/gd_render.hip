@@ -2576,7 +2576,7 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
 // The runs of rows are stored through buffer descriptors (put): a column that has nothing to store in a row the wavefront walks stores
 // beyond the descriptor's end, which the hardware drops.  With a branch around the store instead, the compiler no longer knows how
 // many stores are under way, so that the next use of a loaded texel waits for all of them to reach memory: every row
-// waited for the row before (wall_raster_kernel, 4096 lanes on the 4000-linedef map: 69 % of its wavefront cycles).
+// waited for the row before (wall_raster_kernel, 4096 lanes on the 4000-linedef map: 1.33 ms with the branches, 1.03 without).
 #define BUFFER_WORDS 0x00027000   // descriptor word 3: 32-bit elements
 #define BUFFER_NOWHERE 0x80000000u   // an offset beyond every plane: 4096 lanes are 1.1 GB
 struct PixelBuffers {
@@ -2813,7 +2813,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
             // once, not for its stores and then for its loads.
             // The wavefront walks the rows together (as above): neighbouring columns then read neighbouring texels and store
             // neighbouring words.  Each column starting at its own first row, every load and store touched 64 cache lines
-            // (338 million cache accesses for 4096 lanes on the 4000-linedef map, 0.55 ms of every compute unit's time).
+            // (372 million cache accesses for 4096 lanes on the 4000-linedef map when a sprite clip plane was kept as well, 288 million now).
             // First run: a one-sided drawseg's rows, or the upper tier; second run: the lower tier.
             const bool runs = fresh && !tiers_overlap;
 #pragma unroll 1
@@ -3682,7 +3682,7 @@ __host__ __device__ constexpr int raster_parts(int lanes) { return lanes <= 560 
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
 // 4096 lanes on the 4000-linedef map: 1.78 -> 1.00 ms (with wall_geometry_kernel 1.33): the linedefs' lines 1.53, no sprite clip plane
 // and the rows walked together 1.33, no branch around a load or a store 1.03.  It is left at four wavefronts a SIMD (128 registers, four
-// of them spilled; at 96 registers the spills in the row loops make it 1.6 ms), 55 % of their cycles waiting.
+// of them spilled; at 96 registers the spills in the row loops make it 1.6 ms), 60 % of their cycles waiting.
 template <bool DEPTH, bool GENERAL>
 __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(RASTER_WAVES, RASTER_WAVES))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
@@ -4685,7 +4685,7 @@ __device__ __forceinline__ void store_stack_word(unsigned char *stack_lane, unsi
 // the weighted sum factors into a pass along the rows and one down the columns, all in integers.  The first pass
 // looks every frame pixel's colour up once per observation column it touches (five taps per frame row and
 // observation column), the second adds four row sums per observation pixel: 10,752 palette taps per block where a
-// pixel-by-pixel pooling takes 11,760.  Bound by the vector instructions these take (85 % of the issue slots), so a tap is
+// pixel-by-pixel pooling takes 11,760.  Bound by the vector instructions these take (95 % of the issue slots), so a tap is
 // short: a thread's five bytes come in two words, and a 24-bit product carries red and green together, a dot product blue.
 // Frames on 16 bytes are staged by 16-byte loads.  4096 frames: 0.202 ms with a byte load and three dot products a tap, 0.153 ms now.
 #define OBS_BLOCK_ROWS 7

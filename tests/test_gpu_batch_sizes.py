@@ -1,5 +1,5 @@
-"""Batches on either side of the sizes at which the traversal shares a strip out over more or fewer wavefronts: every lane's
-frame is the one the CPU oracle draws for its camera."""
+"""Batches of many sizes, and on either side of those at which the traversal shares a strip out over more or fewer wavefronts: every
+lane's frame is the one the CPU oracle draws for its camera."""
 
 from __future__ import annotations
 
