@@ -39,6 +39,7 @@ SYMBOLS = (
     "gd_env_reset",
     "gd_env_check",
     "gd_fill_stacks",
+    "gd_copy_pieces",
 )
 
 _LIBRARY = None
@@ -108,6 +109,7 @@ def library() -> C.CDLL:
         ("gd_env_reset", [C.c_void_p] * 3 + [C.c_int32] + [C.c_void_p] * 5),
         ("gd_env_check", [C.c_void_p] * 3 + [C.c_int32, C.c_int32] + [C.c_void_p] * 2),
         ("gd_fill_stacks", [C.c_void_p] * 2 + [C.c_int32] + [C.c_void_p] * 2),
+        ("gd_copy_pieces", [C.c_void_p] * 2 + [C.c_int32, C.c_int64]),
     ):
         function = getattr(lib, name)
         function.restype, function.argtypes = C.c_int, arguments

@@ -6,7 +6,10 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
+#include <exception>
 #include <string>
+#include <thread>
 
 #include "../../include/gradoom_amd.h"
 #include "gd_internal.h"
@@ -203,6 +206,25 @@ int gd_fill_stacks(const uint8_t *obs, const int64_t *rows, int32_t count, uint8
     hipLaunchKernelGGL(fill_stacks_kernel, dim3((unsigned)((words + 255) / 256), (unsigned)count), dim3(256), 0, static_cast<hipStream_t>(stream),
                        reinterpret_cast<const unsigned int *>(obs), rows, reinterpret_cast<unsigned int *>(frames));
     GD_HIP_TRY(hipGetLastError());
+    return GD_OK;
+}
+
+// Most of such a copy is waiting for memory the device has just written, or for fresh pages: the caller's thread and up to three more take
+// every fourth piece.  48 frames of 230,400 bytes: 0.29 ms by one thread, 0.18 by four, 0.23 by eight.
+int gd_copy_pieces(const void *source, void *const *targets, int32_t count, int64_t bytes) {
+    if (count < 0 || bytes < 0) return gd_fail(GD_E_ARG, "count out of range");
+    if (count == 0 || bytes == 0) return GD_OK;
+    if (!source || !targets) return gd_fail(GD_E_ARG, "null argument");
+    for (int32_t k = 0; k < count; ++k) if (!targets[k]) return gd_fail(GD_E_ARG, "null target");
+    constexpr int THREADS = 4;
+    auto copy = [=](int first) { for (int64_t k = first; k < count; k += THREADS) std::memcpy(targets[k], static_cast<const char *>(source) + k * bytes, (size_t)bytes); };
+    std::thread helpers[THREADS - 1];
+    for (int t = 1; t < THREADS; ++t) {
+        if (count <= t || bytes * count < (1 << 20)) { copy(t); continue; }      // too little to be worth a thread
+        try { helpers[t - 1] = std::thread(copy, t); } catch (const std::exception &) { copy(t); }   // no thread to be had
+    }
+    copy(0);
+    for (std::thread &helper : helpers) if (helper.joinable()) helper.join();
     return GD_OK;
 }
 

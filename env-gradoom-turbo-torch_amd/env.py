@@ -92,10 +92,18 @@ class _FramePool:
 
     SHAPE = (240, 320, 3)
 
+    class _Memory:
+        __slots__ = ("array", "address", "interface")
+
+        def __init__(self):
+            self.array = np.empty(_FramePool.SHAPE, dtype=np.uint8)
+            self.address, self.interface = self.array.ctypes.data, self.array.__array_interface__
+
     class _Lent:   # the base of a frame handed out: lives as long as the frame and its views
+        __slots__ = ("_pool", "_memory", "__array_interface__")
+
         def __init__(self, pool, memory):
-            self._pool, self._memory = pool, memory
-            self.__array_interface__ = memory.__array_interface__
+            self._pool, self._memory, self.__array_interface__ = pool, memory, memory.interface
 
         def __del__(self):
             if self._pool._users > 0:
@@ -104,7 +112,7 @@ class _FramePool:
     def __init__(self, limit: int):
         self._free = collections.deque(maxlen=limit)   # its operations are whole ones to other threads
         self._users = 0
-        self._lock = threading.Lock()
+        self._lock = threading.RLock()   # a user may be found gone while the thread holds it
 
     def join(self, user):
         """A call that ends ``user``'s part in the pool; made by itself when ``user`` is gone."""
@@ -119,13 +127,19 @@ class _FramePool:
             if self._users == 0:
                 self._free.clear()
 
-    def copy_of(self, frame: np.ndarray) -> np.ndarray:
+    def _memory(self) -> _Memory:
         try:
-            memory = self._free.pop()
+            return self._free.pop()
         except IndexError:
-            memory = np.empty(self.SHAPE, dtype=np.uint8)
-        np.copyto(memory, frame)
-        return np.asarray(self._Lent(self, memory))
+            return self._Memory()
+
+    def copies_of(self, frames: np.ndarray) -> list[np.ndarray]:
+        """Every frame of a contiguous ``uint8 [N, 240, 320, 3]``, each in memory of its own."""
+
+        memories = [self._memory() for _ in range(len(frames))]
+        targets = (C.c_void_p * len(memories))(*[memory.address for memory in memories])
+        _lib.check(_lib.library().gd_copy_pieces(frames.ctypes.data, targets, len(memories), 240 * 320 * 3))
+        return [np.asarray(self._Lent(self, memory)) for memory in memories]
 
 
 RGB_STAGING_BYTES = 64 << 20   # of frames on their way to the host: pinned, an environment; let go of, all of them together
@@ -597,8 +611,8 @@ class GraDoomVecEnv:
             self._renderer.render(state, rgb=rgb)
             return [frame.copy() for frame in rgb.detach().to("cpu").numpy()]
         # The expansion writes the frames into pinned host memory, over PCIe, as it makes them: no second copy of them on the device
-        # and no staging by the runtime.  Each frame then goes to memory of its own: 48 frames 0.3 ms into memory that was touched
-        # before (hence the pool), 1.6 ms into fresh pages.
+        # and no staging by the runtime.  Each frame then goes to memory of its own, which was touched before where it can be (hence the
+        # pool: fresh pages cost several times the copy).
         frame_bytes = 240 * 320 * 3
         room = max(1, min(count, self.RGB_STAGING_BYTES // frame_bytes))
         if self._rgb_staging is None or self._rgb_staging.shape[0] < room:
@@ -609,7 +623,7 @@ class GraDoomVecEnv:
             staging = self._rgb_staging[:part]
             render_to_host(state if part == count else state.select(slice(base, base + part)), staging)
             self._wait()
-            frames += [_FRAMES.copy_of(frame) for frame in staging.numpy()]
+            frames += _FRAMES.copies_of(staging.numpy())
         return frames
 
     def render_lane(self, lane: int):  # env.py:1037-1053

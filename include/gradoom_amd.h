@@ -309,7 +309,7 @@ int gd_renderer_status_seen(gd_renderer *r, int32_t *status);
  * 320x240 frame in device memory, gd_frame_out.indexed or, when the caller takes none, a frame of the working memory's
  * own.  GD_ASSEMBLY_FUSED: band by band in LDS, where shading, billboards, overlays, PLAYPAL expansion, pooling and the
  * stack update all happen; the frame only goes to device memory if the caller asks for it (observations only: no
- * 320x240 frame is ever written: a fifth less device-memory traffic in the assembly, nine tenths of the speed).
+ * 320x240 frame is ever written: a fifth less device-memory traffic in the assembly, five sixths of the speed).
  * GD_ASSEMBLY_AUTO (the default): separate, the faster of the two on MI355X.  Frames that draw wall decals are always
  * assembled separately.  Both give the same bytes.  Replaces nothing in the reference.
  */
@@ -576,6 +576,9 @@ int gd_env_check(const uint8_t *initialized, const uint8_t *pending, const int64
                  void *stream);
 /* frames [., 4, 84, 84]: the stacks of the lanes that rows names become four copies of obs [count, 84, 84] (engine.py:2443-2450). */
 int gd_fill_stacks(const uint8_t *obs, const int64_t *rows, int32_t count, uint8_t *frames, void *stream);
+/* HOST memory: the `count` pieces of `bytes` bytes that follow each other from `source` on, each to an address of its own; done when the
+   call returns.  A batch of RGB frames becomes arrays of their own this way (env.py:1058-1064 copies frame by frame). */
+int gd_copy_pieces(const void *source, void *const *targets, int32_t count, int64_t bytes);
 
 /*
  * Time `launches` back-to-back gd_render launches with HIP events on `stream`

@@ -178,3 +178,23 @@ def test_the_static_array_is_as_long_as_the_binding_says():
     text = open(os.path.join(ROOT, "include", "gradoom_amd.h")).read()
     assert int(re.search(r"#define GD_STATIC_SCRATCH_MIB (\d+)", text).group(1)) == _abi.STATIC_SCRATCH_MIB
     assert int(re.search(r"#define GD_STATIC_MAX_LANES (\d+)", text).group(1)) == _abi.STATIC_MAX_LANES
+
+
+@pytest.mark.parametrize("count, size", [(0, 7), (1, 1), (2, 5), (3, 230400), (5, 230400), (9, 131072), (48, 230400)])
+def test_pieces_of_host_memory_each_land_at_their_own_address(count, size):
+    import numpy as np
+
+    from gradoom_amd import _build, _lib
+
+    if not os.path.exists(_build.LIBRARY):
+        pytest.skip("libgradoom_amd.so not built (run __graft_entry__.build())")
+    source = np.random.default_rng(count).integers(0, 256, (count, size), dtype=np.uint8)
+    targets = [np.full(size + 16, 7, dtype=np.uint8) for _ in range(count)]
+    addresses = (ctypes.c_void_p * count)(*[target.ctypes.data + 8 for target in targets])
+    _lib.check(_lib.library().gd_copy_pieces(source.ctypes.data, addresses, count, size))
+    for piece, target in zip(source, targets):
+        assert np.array_equal(target[8 : 8 + size], piece) and (target[:8] == 7).all() and (target[8 + size :] == 7).all()
+    for bad in ((source.ctypes.data, addresses, -1, size), (None, addresses, 1, size), (source.ctypes.data, None, 1, size),
+                (source.ctypes.data, (ctypes.c_void_p * 1)(None), 1, size)):
+        with pytest.raises(ValueError):
+            _lib.check(_lib.library().gd_copy_pieces(*bad))
