@@ -69,16 +69,22 @@ def _on_device(*tensors: torch.Tensor) -> bool:
     return True
 
 
+def ray_tables_kernel(angle: torch.Tensor, offsets: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """``ray_tables`` of tensors that are known to be what the kernel reads (``[N]`` and ``[320]``), by the kernel."""
+
+    from . import _lib  # noqa: PLC0415
+
+    tables = torch.empty((2, angle.shape[0], SCREEN_WIDTH), dtype=torch.float32, device=angle.device)
+    ray_cos, ray_sin = tables[0], tables[1]
+    with torch.cuda.device(angle.device):
+        _lib.check(_lib.library().gd_ray_tables(angle.data_ptr(), offsets.data_ptr(), angle.shape[0], ray_cos.data_ptr(), ray_sin.data_ptr(),
+                                                torch.cuda.current_stream(angle.device).cuda_stream))
+    return ray_cos, ray_sin
+
+
 def ray_tables(angle: torch.Tensor, offsets: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     if _on_device(angle, offsets) and angle.dim() == 1 and offsets.shape == (SCREEN_WIDTH,):
-        from . import _lib  # noqa: PLC0415
-
-        tables = torch.empty((2, angle.shape[0], SCREEN_WIDTH), dtype=torch.float32, device=angle.device)
-        ray_cos, ray_sin = tables[0], tables[1]
-        with torch.cuda.device(angle.device):
-            _lib.check(_lib.library().gd_ray_tables(angle.data_ptr(), offsets.data_ptr(), angle.shape[0], ray_cos.data_ptr(), ray_sin.data_ptr(),
-                                                    torch.cuda.current_stream(angle.device).cuda_stream))
-        return ray_cos, ray_sin
+        return ray_tables_kernel(angle, offsets)
     ray_angles = angle[:, None] + offsets[None, :]
     return torch.cos(ray_angles).contiguous(), torch.sin(ray_angles).contiguous()
 
@@ -87,15 +93,21 @@ def angle_from_bam(angle_bam: torch.Tensor) -> torch.Tensor:
     return angle_bam.to(torch.float32) * BAM_TO_RADIANS
 
 
+def sprite_depth_kernel(x, y, angle, sprite_x, sprite_y) -> torch.Tensor:
+    """``sprite_depth`` of tensors that are known to be what the kernel reads (``[N]`` three times, ``[N, A]`` twice), by the kernel."""
+
+    from . import _lib  # noqa: PLC0415
+
+    depth = torch.empty_like(sprite_x)
+    with torch.cuda.device(x.device):
+        _lib.check(_lib.library().gd_sprite_depth(x.data_ptr(), y.data_ptr(), angle.data_ptr(), sprite_x.data_ptr(), sprite_y.data_ptr(), sprite_x.shape[0],
+                                                  sprite_x.shape[1], depth.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream))
+    return depth
+
+
 def sprite_depth(x, y, angle, sprite_x, sprite_y) -> torch.Tensor:
     if _on_device(x, y, angle, sprite_x, sprite_y) and x.shape == y.shape == angle.shape == sprite_x.shape[:1] and sprite_x.shape == sprite_y.shape and sprite_x.dim() == 2:
-        from . import _lib  # noqa: PLC0415
-
-        depth = torch.empty_like(sprite_x)
-        with torch.cuda.device(x.device):
-            _lib.check(_lib.library().gd_sprite_depth(x.data_ptr(), y.data_ptr(), angle.data_ptr(), sprite_x.data_ptr(), sprite_y.data_ptr(), sprite_x.shape[0],
-                                                      sprite_x.shape[1], depth.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream))
-        return depth
+        return sprite_depth_kernel(x, y, angle, sprite_x, sprite_y)
     dx = sprite_x - x[:, None]
     dy = sprite_y - y[:, None]
     distance = torch.sqrt(dx * dx + dy * dy).clamp_min(1)

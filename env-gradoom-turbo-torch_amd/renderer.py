@@ -157,7 +157,7 @@ class HipRenderer:
     def set_assembly(self, assembly: str) -> None:
         """``"separate"`` (kernel by kernel through a frame in device memory, the caller's or the working memory's own),
         ``"fused"`` (every frame is put together band by band in LDS and never reaches device memory unless asked for: a
-        fifth less traffic in the assembly, nine tenths of the speed) or ``"auto"`` (the default: separate).  Both give the same bytes."""
+        fifth less traffic in the assembly, five sixths of the speed) or ``"auto"`` (the default: separate).  Both give the same bytes."""
 
         codes = {"auto": 0, "fused": 1, "separate": 2}
         if assembly not in codes:
@@ -204,7 +204,7 @@ class HipRenderer:
         for name in ("x_fixed", "y_fixed", "angle_bam", "pitch_bam", "flash_light"):
             setattr(desc, name, _require(getattr(lanes, name), name, torch.int64, (count,), device).data_ptr())
         if lanes.ray_cos is None or lanes.ray_sin is None:
-            ray_cos, ray_sin = hostmath.ray_tables(lanes.angle, self.ray_offsets)
+            ray_cos, ray_sin = hostmath.ray_tables_kernel(lanes.angle, _require(self.ray_offsets, "ray_offsets", torch.float32, (320,), device))
         else:
             ray_cos, ray_sin = lanes.ray_cos, lanes.ray_sin
         keep += [ray_cos, ray_sin]
@@ -232,7 +232,7 @@ class HipRenderer:
                 desc.sprite_style = _require(lanes.sprite_style, "sprite_style", torch.int8, (count, slots), device).data_ptr()
             depth = lanes.sprite_depth
             if depth is None:
-                depth = hostmath.sprite_depth(lanes.x, lanes.y, lanes.angle, lanes.sprite_x, lanes.sprite_y)
+                depth = hostmath.sprite_depth_kernel(lanes.x, lanes.y, lanes.angle, lanes.sprite_x, lanes.sprite_y)
             keep.append(depth)
             desc.sprite_depth = _require(depth, "sprite_depth", torch.float32, (count, slots), device).data_ptr()
         if lanes.weapon_state is not None:
