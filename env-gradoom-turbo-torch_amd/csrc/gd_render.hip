@@ -3533,10 +3533,10 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(int strips, Scratch s
 // each, which first copy their columns' lists to LDS (8 KB a wavefront) and scan them there.  It runs beside the
 // launch for all other strips.  The fewer columns a wavefront has, the fewer rules it runs in a pass, and the more wavefronts
 // take slots from the other launch.  4096 lanes, this launch / the other, wavefronts a strip: 4: 0.88 / 0.97 ms, 8: 0.75 / 0.92,
-// 16: 0.81 / 1.00; 2048 lanes on a 1400-linedef map 4: 0.24 / 0.26, 8: 0.20 / 0.27, 16: 0.25 / 0.28.  A smaller batch leaves room and
-// lasts as long as its very longest strips: 512 lanes 4: 0.74 / 0.38, 8: 0.65 / 0.39, 16: 0.51 / 0.40, and 32 for 128 of the
-// strips, 8 for the others 0.45 / 0.41 (32 for 256: 0.49; 64 for 128: 0.54); 256 lanes 0.161 / 0.086, 0.128 / 0.090, 0.116 / 0.099,
-// 0.121 / 0.106; 1024 lanes 4: 0.38 / 0.28, 0.30 / 0.30 the last way.  Lists left in device memory: no gain.
+// 16: 0.81 / 1.00; 2048 lanes on a 1400-linedef map 4: 0.24 / 0.26, 8: 0.20 / 0.27, 16: 0.25 / 0.28.  A smaller batch
+// lasts as long as its very longest strips: 512 lanes on the 4000-linedef map 4: 0.74 / 0.38, 8: 0.65 / 0.39, 16: 0.51 / 0.40, and 32 for
+// 128 of the strips, 8 for the others 0.45 / 0.41 (32 for 256: 0.49; 64 for 128: 0.54); 256 lanes on an 800-linedef map 0.161 / 0.086, 0.128 /
+// 0.090, 0.116 / 0.099, 0.121 / 0.106 (up to which batch that pays: select_finely).  Lists left in device memory: no gain.
 static_assert(SEG_COLS == 64 && SELECT_STRIPS_PER_GROUP == 1, "wall_select_kernel's staged launch: parts of one whole strip per work-group");
 template <bool SPLIT, bool STAGED>
 __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kernel(DeviceMap dm, int lane_count, Scratch sc, int staged_slots, int fine_slots) {
@@ -4250,8 +4250,11 @@ __device__ __forceinline__ void sprite_column(const DeviceMap &dm, const gd_lane
 #define SPRITE_SLOTS_MAX 512
 #define SPRITE_COLUMNS 64     // a work-group for the whole lane: 0.95 ms instead of 0.70 (4 wavefronts), 0.86 (8)
 #define SPRITE_ROW_PARTS 4    // of a small batch's work-groups
-// Lanes from which a work-group takes all rows of its columns: fewer listings, but the last work-groups last longer.  Whole columns /
-// quarters: 256 lanes 0.099 / 0.071 ms, 512 lanes 0.176 / 0.232, 1024 lanes 0.131 / 0.141, 4096 lanes 0.70 / 0.84.
+// Lanes from which a work-group takes all rows of its columns: fewer listings, but the last work-groups last longer.  Quarters and whole
+// columns cost the same at 230 (4000 linedefs, 128 billboards) to 1100 lanes (320 linedefs, 32 billboards); the line lies between.  us, quarters /
+// whole columns, two sets of poses each: 320 linedefs, 32 billboards, 256 lanes 66 / 97, 512 lanes 101 / 122, 1024 lanes 170 / 174; with 128
+// 105 / 139, 174 / 179, 336 / 296; 2000 linedefs with 128 128 / 117, 170 / 144, 256 / 212; 4000 with 32 81 / 90, 125 / 125, 185 / 172; with 128 186 /
+// 172, 218 / 192, 299 / 250; 4096 lanes of it 840 / 700.
 #define SPRITE_TALL_LANES 512
 static_assert(SPRITE_COLUMNS == 64 && SW % SPRITE_COLUMNS == 0 && VH % (SPRITE_ROW_PARTS * SPRITE_TILE_H) == 0 && VH <= SPRITE_THREADS, "sprite_pixels_kernel: whole tiles");
 static_assert(SPRITE_CHUNK == 64 && SPRITE_CHUNK <= SPRITE_THREADS, "sprite_pixels_kernel: a bit an entry");
@@ -5610,7 +5613,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     // observation from it), the caller's `indexed` or the working memory's own: the faster way on this chip (its kernels
     // run at full occupancy), and the only one for frames that draw wall decals, which need a per-pixel scene depth.  Or
     // band by band in LDS (band_finish_kernel), the frame never reaching device memory: a fifth less traffic in the
-    // assembly for a caller that only wants observations, at nine tenths of the speed; chosen with gd_renderer_set_assembly.
+    // assembly for a caller that only wants observations, at five sixths of the speed; chosen with gd_renderer_set_assembly.
     const bool decals = lanes->decal_slots > 0 && lanes->decal_state && lanes->decal_geom && r->overlays.d.decal_variant_count > 0;
     if (!decals) sc.scene_depth = nullptr;
     if (decals && (!sc.scene_depth || !sc.frame)) return fail(GD_E_ARG, "decal working memory missing");

@@ -22,7 +22,7 @@ FIXTURE_DIR = os.path.join(ROOT, "tests", "golden", "fixtures")
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
 def fixture_names():

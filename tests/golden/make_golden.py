@@ -8,7 +8,7 @@ imported through ``refdrive``), and the inputs + outputs are stored as
 ``tests/golden/fixtures/<name>.npz``:
 
 * lane inputs exactly as ``gd_lanes_desc`` wants them (including the Torch
-  float32 ray tables and sprite depths, so nothing on the GPU box needs the
+  float32 ray tables and sprite depths, so nothing that runs on a GPU needs the
   reference or a particular Torch CPU build);
 * ``indexed``  uint8 [N,240,320]  ``_render_native_indexed_frame(include_hud=True)`` (engine.py:15338)
 * ``obs``      uint8 [N,84,84]    ``render_reference_frame()`` CPU float path (engine.py:15436)

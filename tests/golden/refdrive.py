@@ -5,7 +5,7 @@ The reference package cannot be imported as ``gradoom`` here because its
 ``gradoom.engine`` + ``gradoom.scenario`` which only need torch/numpy.  This
 module registers an empty parent package whose ``__path__`` points at the
 reference sources and imports just those two modules.  It is used only by
-``make_golden.py`` to write fixtures; nothing on the GPU box imports it.
+``make_golden.py`` to write fixtures; nothing that runs on a GPU imports it.
 """
 
 from __future__ import annotations
