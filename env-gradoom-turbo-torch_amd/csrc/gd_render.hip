@@ -18,7 +18,7 @@
 //                                             visplane repair of the rows where a gap pixel stayed unresolved
 //   flat_shade      1 wave / gap column       the gap pixels' flats
 //   decal           320 threads / lane        bullet chips on the wall tiers they hit (frames that carry decals
-//                                             also keep a per-pixel scene depth: wall_raster<true>, plane_shade<true>)
+//                                             also keep the depth of wall pixels: wall_raster<true>)
 //   sprite_pixels   thread per view pixel     billboards, nearest visible one first, or blended far -> near
 //   weapon_overlay, hud                       player weapon, muzzle flash and status bar patches
 //   observe         1 thread / obs pixel      PLAYPAL + exact area pool + gray + 4-frame stack
@@ -255,8 +255,8 @@ struct Scratch {    // per-chunk working memory, sized at create
                            // projection that owns the column, CAND_KEY_NONE if none (engine.py:13436-13460)
     uint2 *pass_rows;      // [pass_slots,L,320] the eight projected rows of a pass whose record carries REC_OWN_ROWS (written for those only)
     WallRec *frag_rec;     // [L,split_count,fragment_slots] FWallCoords of the BSP fragments of split linedefs
-    float *scene_depth;    // [L,208,320] depth of the surface each pixel shows (engine.py:11553, 12700, 13411, 13740),
-                           // kept only for frames that draw wall decals, else null
+    float *scene_depth;    // [L,208,320] depth of the wall tier or masked texture a pixel shows (engine.py:11553, 12700, 13740),
+                           // kept only for frames that draw wall decals, else null; scene_depth_at() has the others
     Cand *cand;            // [L,CAND_MAX,320], then the spill pool [spill_slots / 320, SPILL_DEPTH, 320]
     int *cand_count;       // [L,320] entries listed (beyond CAND_MAX: the column wanted more than its own slots hold), or for
                            // a column with a pool slot: entries in the pool | (slot + 1) << SPILL_SHIFT
@@ -3823,9 +3823,9 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
 #define SHADE_TILES 13   // tiles (256 runs) per block: 65 tiles per view = 5 blocks per lane (each block stages the tables once)
 #define SHADE_GROUP 1    // tiles per step
 static_assert(SW % SHADE_RUN == 0 && SHADE_RUN == 4, "plane_shade_kernel: a run is one 16-byte load of per-pixel words and one 4-byte store");
-// DEPTH: also keep the depth of every pixel no wall tier covers (frames that draw decals).  STAGED: the lane's plane table
-// is short enough for LDS (the kernel then reads it with LDS instructions; a pointer that may be either costs more).
-template <bool DEPTH, bool STAGED>
+// STAGED: the lane's plane table is short enough for LDS (the kernel then reads it with LDS instructions; a pointer that may be
+// either costs more).
+template <bool STAGED>
 // Eight wavefronts per SIMD.  The kernel runs beside the flat pass (launch_chunk) and the billboards follow it on the same
 // stream: the sooner it is done, the sooner they are (with the billboards still after the flat pass, five wavefronts per
 // SIMD and two tiles per step were better: the flat pass's kernels found more room beside it).
@@ -3939,11 +3939,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
                     const bool is_floor = (word & META_FLOOR) != 0;
                     if (shades[g] & (1u << k)) { colour = colormap_lds[colormap_row[g][k] * 256 + texel[g][k]]; writes = true; }
                     else if (!(word & META_MASKED)) { colour = flat_pixel(tb, colormap_lds, c, ps, is_floor, x0 + k, y); writes = true; }
-                    if (DEPTH && !(word & META_MASKED)) {   // exact plane depth (engine.py:13406-13416)
-                        const float flat_center_px = (103.0f + c.pitch_offset) + 0.5f;
-                        const float plane_height = is_floor ? (c.view_z - tb.floor_h(ps)) : (tb.ceil_h(ps) - c.view_z);
-                        sc.scene_depth[(size_t)local * VH * SW + first_pixel[g] + k] = plane_height * 192.0f / fmaxf(fabsf((float)y - flat_center_px), 0.5f);
-                    }
                 }
                 colours |= colour << (8 * k);
                 if (writes) written |= 1u << k;
@@ -3959,8 +3954,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
     }
 }
 
-// The listed gap pixels, painted with the flat the flat pass settled on (engine.py:11145-11163); frames that
-// draw decals also keep the depth that pass leaves there (engine.py:11140-11166).
+// The listed gap pixels, painted with the flat the flat pass settled on (engine.py:11145-11163).
 __device__ void flat_shade_pixel(const DeviceMap &dm, const Scratch &sc, const LaneCtx &c, int local, int pixel, unsigned char *frame) {
     const gd_map_desc *m = &dm.d;
     Tables tb; tb.m = m; tb.sector = nullptr; tb.tex_bits = nullptr; tb.tex_odd = nullptr; tb.sector_cached = 0; tb.tex_cached = 0;
@@ -3969,17 +3963,6 @@ __device__ void flat_shade_pixel(const DeviceMap &dm, const Scratch &sc, const L
     const int s = sc.flat_sector[i];
     const float delta = (float)y - flat_center(c);
     frame[pixel] = flat_pixel(tb, m->colormap, c, s, delta > 0, x, y);
-    if (sc.scene_depth) {
-        const unsigned char flags = sc.flat_flags[i];
-        const float plane_height = delta > 0 ? (c.view_z - tb.floor_h(s)) : (tb.ceil_h(s) - c.view_z);
-        const float perpendicular = plane_height * 192.0f / fmaxf(fabsf(delta), 0.5f);
-        const float cosine = dm.cosine_correction[x];
-        float depth;
-        if (flags & (2 | 8)) depth = perpendicular;             // repaired: its visplane's depth
-        else if (flags & 1) depth = GD_INF;                    // no sector found along the ray
-        else depth = (perpendicular / cosine) * cosine;        // ray distance of the hit, corrected back
-        sc.scene_depth[i] = depth;
-    }
 }
 
 // lane_pick: LANES_ALL, or one half of launch_chunk's split: LANES_PLAIN for the lanes whose billboards were painted first and
@@ -4423,7 +4406,29 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(Device
 // wall decals: engine.py:13747-13991, drawn after the walls and before the sprites
 // ---------------------------------------------------------------------------------------------
 // One thread per screen column; a lane's decals are painted oldest first, each only where the scene
-// depth is the decal's own ray distance (which ties it to the wall tier it sits on).
+// depth is the decal's own ray distance (which ties it to the wall tier it sits on).  What the walls drew has its depth in
+// Scratch::scene_depth; that of the other pixels follows from their words, and only the few a decal reaches are asked for it (a plane
+// of it, stored by the shading for every plane pixel, made that kernel 0.75 ms instead of 0.57 for 2048 lanes, beside the flat pass).
+__device__ __forceinline__ float scene_depth_at(const DeviceMap &dm, const Scratch &sc, const LaneCtx &c, size_t i, int x, int y) {
+    const gd_map_desc *m = &dm.d;
+    const unsigned int word = sc.meta[i];
+    if (word & (META_FILLED | META_MASKED)) return sc.scene_depth[i];
+    const int plane = (int)((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1;
+    if (plane >= 0) {   // exact plane depth (engine.py:13406-13416)
+        const float plane_height = (word & META_FLOOR) ? (c.view_z - m->sector_heights[2 * plane]) : (m->sector_heights[2 * plane + 1] - c.view_z);
+        return plane_height * 192.0f / fmaxf(fabsf((float)y - ((103.0f + c.pitch_offset) + 0.5f)), 0.5f);
+    }
+    // the depth the flat pass leaves (engine.py:11140-11166)
+    const int s = sc.flat_sector[i], flags = sc.flat_flags[i];
+    const float delta = (float)y - flat_center(c);
+    const float plane_height = delta > 0 ? (c.view_z - m->sector_heights[2 * s]) : (m->sector_heights[2 * s + 1] - c.view_z);
+    const float perpendicular = plane_height * 192.0f / fmaxf(fabsf(delta), 0.5f);
+    if (flags & (2 | 8)) return perpendicular;             // repaired: its visplane's depth
+    if (flags & 1) return GD_INF;                          // no sector found along the ray
+    const float cosine = dm.cosine_correction[x];
+    return (perpendicular / cosine) * cosine;              // ray distance of the hit, corrected back
+}
+
 __global__ void __launch_bounds__(SW) decal_kernel(DeviceMap dm, Overlays ov, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
                                                    unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
@@ -4437,7 +4442,6 @@ __global__ void __launch_bounds__(SW) decal_kernel(DeviceMap dm, Overlays ov, gd
     const int width = o.decal_max_w;
     const float center = 104.0f + L.pitch_offset;
     unsigned char *frame = frame_base + (size_t)local * frame_stride;
-    const float *scene_depth = sc.scene_depth + (size_t)local * VH * SW;
     float rx, ry; ray_direction(L, x, &rx, &ry);
     for (int k = 0; k < D; ++k) {
         const int *state = lanes.decal_state + ((size_t)n * D + k) * 3;
@@ -4505,7 +4509,7 @@ __global__ void __launch_bounds__(SW) decal_kernel(DeviceMap dm, Overlays ov, gd
             if (!(tv >= 0 && tv < height)) continue;
             if (flip_y) tv = height - 1 - tv;
             const size_t i = (size_t)y * SW + x;
-            if (!(fabsf(scene_depth[i] - distance) <= 1e-3f)) continue;
+            if (!(fabsf(scene_depth_at(dm, sc, L, (size_t)local * VH * SW + i, x, y) - distance) <= 1e-3f)) continue;
             const unsigned char source = o.decal_atlas[((size_t)variant * o.decal_max_h + tv) * o.decal_max_w + tu];
             if (source == 0) continue;
             const unsigned char opacity = o.decal_opacity_lut[shade * 256 + source];
@@ -5707,9 +5711,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         if (fused) return;
         const dim3 grid(((VH * SW / SHADE_RUN + 255) / 256 + SHADE_TILES - 1) / SHADE_TILES, count);
         const bool staged = m.floor_level_count + m.ceil_level_count <= 2 * PLANE_LEVELS;
-        auto kernel = decals ? (staged ? plane_shade_kernel<true, true> : plane_shade_kernel<true, false>)
-                             : (staged ? plane_shade_kernel<false, true> : plane_shade_kernel<false, false>);
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, shade_stream, r->dm, count, sc, frame_base, frame_stride);
+        hipLaunchKernelGGL(staged ? plane_shade_kernel<true> : plane_shade_kernel<false>, grid, dim3(256), 0, shade_stream, r->dm, count, sc, frame_base, frame_stride);
     };
     if (!beside) shade_planes();
     mark();

@@ -26,7 +26,7 @@ def test_weapon_patches_at_and_past_every_edge_of_the_view_match_the_oracle(orac
     smap, tables, arrays = closed_door_case(301, lanes)
     rng = np.random.default_rng(7)
     words = np.zeros((lanes, 5), dtype=np.int64)
-    words[:, 0], words[:, 1] = rng.integers(-1, patches + 1, lanes), rng.integers(-1, patches + 1, lanes)   # none, and one past the last
+    words[:, 0], words[:, 1] = rng.integers(0, patches, lanes), rng.integers(-1, patches, lanes)
     words[:, 2] = np.repeat(across, len(down)) * 65536 + rng.integers(0, 65536, lanes)
     words[:, 3] = np.tile(down, len(across)) * 65536 + rng.integers(0, 65536, lanes)
     words[:, 4] = 1
@@ -37,6 +37,53 @@ def test_weapon_patches_at_and_past_every_edge_of_the_view_match_the_oracle(orac
     renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
     renderer.set_overlays(overlays)
     renderer.set_assembly(assembly)
+    indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+    renderer.render(LaneState.from_numpy(arrays, "cuda:0"), indexed=indexed)
+    torch.cuda.synchronize()
+    assert renderer.status() == 0
+    assert np.array_equal(indexed.cpu().numpy(), expected)
+    renderer.close()
+
+
+@pytest.mark.parametrize("where", ["inside", "outside"])
+def test_chips_over_pixels_of_every_kind_match_the_oracle(oracle, where):
+    """Chips cut off by tiers, planes and masked textures before them, and (cameras in the void) chips whose rows reach pixels that show
+    the flat pass's picture, resolved, repaired and not."""
+    import sys
+    import types
+
+    from conftest import ROOT
+    from gradoom_amd import hostmath, mapbuild, overlay_inputs, synthmap
+    from gradoom_amd.renderer import HipRenderer, LaneState
+    from gradoom_amd.selfcheck import make_lane_arrays
+    from random_cases import closed_door_parts, outside_parts
+
+    sys.path.insert(0, f"{ROOT}/tests/golden")
+    import refdrive
+
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    overlays = synthmap.generate_overlays(32)
+    lanes, slots = 16, 64
+    smap, poses, sprites = closed_door_parts(305, lanes, mixed=True)[:3] if where == "inside" else outside_parts(lanes)
+    tables = mapbuild.build_map_tables(smap)
+    arrays = make_lane_arrays(smap, poses, sprites)
+    engine = types.SimpleNamespace(num_envs=lanes, hitscan_decal_slots=slots, **{name: arrays[name] for name in ("x", "y", "angle", "view_z")})
+    for name, dtype, value in (("wall", torch.int64, 0), ("along", torch.float32, 0), ("z", torch.float32, 0), ("style", torch.int64, 0), ("serial", torch.int64, -1)):
+        setattr(engine, "hitscan_decal_" + name, torch.full((lanes, slots), value, dtype=dtype))
+    refdrive.set_decals(engine, smap, 306)
+    state, geometry = overlay_inputs.decal_inputs(
+        engine.hitscan_decal_serial, engine.hitscan_decal_wall, engine.hitscan_decal_along, engine.hitscan_decal_z, engine.hitscan_decal_style,
+        torch.as_tensor(np.asarray(tables["walls"], dtype=np.float32)), overlay_inputs.fine_sine_fixed(),
+    )
+    plain = oracle.render(tables, arrays, cosine)["indexed"]
+    arrays["decal_state"], arrays["decal_geom"] = state.numpy(), geometry.numpy()
+    oracle.set_overlays(overlays)
+    expected = oracle.render(tables, arrays, cosine)["indexed"]
+    oracle.set_overlays(None)
+    assert (expected != plain).any()                  # some chips show
+    renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+    renderer.set_overlays(overlays)
+    renderer.scribble(0xFF)
     indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
     renderer.render(LaneState.from_numpy(arrays, "cuda:0"), indexed=indexed)
     torch.cuda.synchronize()
