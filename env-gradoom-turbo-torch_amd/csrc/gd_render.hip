@@ -11,7 +11,7 @@
 //   wall_select     1 wave / strip            portal traversal: which drawseg every column pass selects, one record each
 //   wall_geometry   1 block / lane            the linedefs those passes draw, as lines over the columns: every division of the drawing
 //   wall_raster     1 wave / strip            the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
-//   plane_shade     1 thread / 12 pixels      flat texel + light for every pixel a plane of the wall pass shows,
+//   plane_shade     1 wave / 64 columns x 16 rows  flat texel + light for every pixel a plane of the wall pass shows,
 //                                             the wall tiers' palette indices
 //   flat_gap        4 waves / gap column      per-pixel plane rays (fine point raster) for the gap pixels, vertical repair
 //   flat_rows, flat_span_select, flat_tail, flat_span_finish
@@ -1653,7 +1653,7 @@ struct Tables {
 };
 
 // Cooperative fill of the LDS tables by the whole block (call before a __syncthreads()).
-struct TexLds { unsigned char bits[LDS_TEXTURES]; unsigned int odd[LDS_TEXTURES / 32]; };   // 252 bytes: plane_shade_kernel's LDS budget is exact
+struct TexLds { unsigned char bits[LDS_TEXTURES]; unsigned int odd[LDS_TEXTURES / 32]; };
 __device__ __forceinline__ void stage_tables(const gd_map_desc *m, float4 *sector_lds, TexLds *tex_lds, Tables &tb) {
     int sectors = m->sector_count < LDS_SECTORS ? m->sector_count : LDS_SECTORS;
     int textures = m->texture_count < LDS_TEXTURES ? m->texture_count : LDS_TEXTURES;
@@ -1759,42 +1759,58 @@ __device__ __forceinline__ size_t flat_sample_tabled(const Tables &tb, const Lan
     return (size_t)(((unsigned)texture * (unsigned)m->tex_max_h + v) * (unsigned)m->tex_max_w + u);   // the atlas is below 4 GiB (checked at create)
 }
 
-// flat_sample_tabled for a run of neighbouring pixels of one row that show the same plane: what depends on the row and the
-// plane is worked out once (plane_span), each pixel then costs two 64-bit additions and two products (plane_span_texel).
-// The same integers: base + px * step is (base + px0 * step) + k * step in 64-bit arithmetic.
+// flat_sample_tabled for neighbouring pixels of one row that show the same plane.  Of distance * (base + x * step) only bits 16..47 are
+// looked at, and distance * base + x * (distance * step) is the same number modulo 2^48: both products are worked out once
+// for the run, and a pixel costs two 24-bit multiply-adds an axis.
 struct PlaneSpan {
-    i64 distance, xfrac_base, yfrac_base, xstep, ystep;
-    unsigned pviewx, pviewy, texture_row0, atlas_width;
-    int width_shift, height_shift, colormap_row;
+    uint4 start;         // the fraction at the strip's first column, its lower and upper 24 bits: horizontal, then vertical
+    uint4 step;          // what a column adds, likewise; the four upper bytes: 24 - log2 width, colormap row, 24 - log2 height, nothing
+    unsigned texture;    // the texture's first texel in the atlas (which is below 4 GiB: checked at create)
+    // the texel `column` (0..63) columns into the strip
+    __device__ __forceinline__ unsigned texel(unsigned column, unsigned atlas_width) const {
+        const unsigned x = __umul24(step.y, column) + start.y + ((__umul24(step.x, column) + start.x) >> 24);
+        const unsigned y = __umul24(step.w, column) + start.w + ((__umul24(step.z, column) + start.z) >> 24);
+        return texture + __umul24((y & 0xFFFFFFu) >> (step.z >> 24), atlas_width) + ((x & 0xFFFFFFu) >> (step.x >> 24));
+    }
+    __device__ __forceinline__ unsigned colormap_row() const { return step.y >> 24; }
 };
-__device__ __forceinline__ PlaneSpan plane_span(const Tables &tb, const LaneCtx &c, const LaneTables &lt, i64 yslope, int level_index, int sector,
-                                                bool is_floor, int px0, int py) {
-    const gd_map_desc *m = tb.m;
-    PlaneSpan s;
-    const int texture = is_floor ? tb.floor_tex(sector) : tb.ceil_tex(sector);
-    const int width_bits = tb.width_bits(texture), height_bits = tb.height_bits(texture);
-    const i64 *plane = lt.level_plane + 2 * (is_floor ? level_index : lt.floors + level_index);
-    const i64 plane_height_fixed = plane[0], glob = plane[1];
-    s.xstep = lt.step_scale[width_bits]; s.ystep = lt.step_scale[16 + height_bits];
-    s.xfrac_base = lt.step_scale[32 + width_bits] + mul64_u32(s.xstep, (unsigned)px0);
-    s.yfrac_base = lt.step_scale[48 + height_bits] + mul64_u32(s.ystep, (unsigned)px0);
-    s.pviewx = (unsigned)lt.step_scale[64 + width_bits]; s.pviewy = (unsigned)lt.step_scale[80 + height_bits];
-    s.distance = mul64_u32(plane_height_fixed, (unsigned)yslope) >> 16;
-    s.width_shift = 31 - width_bits; s.height_shift = 31 - height_bits;
-    const float light = tb.light(sector) + (float)(c.flash_light * 16);
-    i64 row = c.center_fixed - (i64)py * FIXED_UNIT;
+__device__ __forceinline__ PlaneSpan plane_span(const DeviceMap &dm, const Scratch &sc, const LaneCtx &c, int local, int sector, bool is_floor, int x_first, int y) {
+    const gd_map_desc *m = &dm.d;
+    const int texture = is_floor ? m->sector_floor_tex[sector] : m->sector_ceil_tex[sector];
+    const float light = m->sector_lights[sector] + (float)(c.flash_light * 16);
+    const i64 yslope = sc.row_slope[(size_t)local * VH + y];
+    i64 plane_height_fixed, glob;
+    if (dm.sector_level) {       // the lane's table of plane levels
+        const int floors = m->floor_level_count, levels = floors + m->ceil_level_count;
+        const unsigned int pair = dm.sector_level[sector];
+        const longlong2 plane = reinterpret_cast<const longlong2 *>(sc.level_plane)[(size_t)local * levels + (is_floor ? (int)(pair & 0xFFFFu) : floors + (int)(pair >> 16))];
+        plane_height_fixed = plane.x; glob = plane.y;
+    } else {
+        plane_height_fixed = round_to_i64((is_floor ? c.view_z - m->sector_heights[2 * sector] : m->sector_heights[2 * sector + 1] - c.view_z) * 65536.0f);
+        glob = min64(tdiv(FLOOR_VISIBILITY_FIXED << 16, max64(plane_height_fixed, 1)), (1LL << 31) - 1);
+    }
+    const int width_bits = ilog2(m->tex_w[texture]), height_bits = ilog2(m->tex_h[texture]);
+    const i64 *scale = sc.step_scale + (size_t)local * STEP_TABLE;
+    const i64 xstep = scale[width_bits], ystep = scale[16 + height_bits];
+    // the same integers as flat_texture_coordinates: base + (x - 159) * step is (base - 159 * step) + x * step; the row slope and the
+    // visibility factor are below 2^31 and not negative (lane_tables_kernel clamps both)
+    const u64 distance = (u64)(mul64_u32(plane_height_fixed, (unsigned)yslope) >> 16);
+    const u64 xadd = distance * (u64)xstep, yadd = distance * (u64)ystep;
+    // the camera's offset in the texture is added to bits 16..47
+    const u64 x = distance * (u64)(scale[32 + width_bits] + mul64_u32(xstep, (unsigned)x_first)) + ((u64)scale[64 + width_bits] << 16);
+    const u64 v = distance * (u64)(scale[48 + height_bits] + mul64_u32(ystep, (unsigned)x_first)) + ((u64)scale[80 + height_bits] << 16);
+    i64 row = c.center_fixed - (i64)y * FIXED_UNIT;
     if (row < 0) row = -row;
     const i64 visibility = min64(mul64_u32(row, (unsigned)glob) >> 16, 24 * FIXED_UNIT);
     const i64 plane_shade = 64 * FIXED_UNIT - ((i64)light + 12) * (FIXED_UNIT / 4);
-    s.colormap_row = (int)clampi((plane_shade - visibility) >> 16, 0, 31);
-    s.texture_row0 = (unsigned)texture * (unsigned)m->tex_max_h; s.atlas_width = (unsigned)m->tex_max_w;
+    const unsigned colormap_row = (unsigned)clampi((plane_shade - visibility) >> 16, 0, 31);
+    auto low = [](u64 value) { return (unsigned)value & 0xFFFFFFu; };
+    auto high = [](u64 value) { return (unsigned)(value >> 24) & 0xFFFFFFu; };
+    PlaneSpan s;
+    s.start = make_uint4(low(x), high(x), low(v), high(v));
+    s.step = make_uint4(low(xadd) | ((24u - (unsigned)width_bits) << 24), high(xadd) | (colormap_row << 24), low(yadd) | ((24u - (unsigned)height_bits) << 24), high(yadd));
+    s.texture = (unsigned)texture * (unsigned)m->tex_max_h * (unsigned)m->tex_max_w;
     return s;
-}
-__device__ __forceinline__ unsigned plane_span_texel(const PlaneSpan &s, int k) {   // pixel px0 + k
-    const unsigned xfrac = mul64_bits_16_47(s.distance, s.xfrac_base + mul64_u32(s.xstep, (unsigned)k)) + s.pviewx;
-    const unsigned yfrac = mul64_bits_16_47(s.distance, s.yfrac_base + mul64_u32(s.ystep, (unsigned)k)) + s.pviewy;
-    const unsigned u = (xfrac >> s.width_shift) >> 1, v = (yfrac >> s.height_shift) >> 1;   // two shifts: a size of one shifts by 32
-    return (s.texture_row0 + v) * s.atlas_width + u;   // the atlas is below 4 GiB (checked at create)
 }
 
 // Visplane repair (engine.py:11026-11135) of the noted row ranges.  Every pixel of those rows is selected first (the repairs
@@ -3814,142 +3830,113 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
 }
 
 // ---------------------------------------------------------------------------------------------
-// plane shading, one thread per view pixel.  A pixel no wall tier owns shows a flat: the
-// visplane the wall traversal marked for it (engine.py:13372-13405) or, where no drawseg marked
-// one, the sector the per-pixel plane rays selected (engine.py:11145-11163).  Doing both here
-// shades every pixel once, in a kernel light enough to run at full occupancy.
+// plane shading.  A pixel no wall tier owns shows a flat: the visplane the wall traversal marked for it (engine.py:13372-13405)
+// or, where no drawseg marked one, the sector the per-pixel plane rays selected (engine.py:11145-11163).  Doing the first for every
+// pixel here and the second in flat_shade_kernel shades every pixel once.
 // ---------------------------------------------------------------------------------------------
-#define SHADE_RUN 4      // neighbouring pixels of a row per thread
-#define SHADE_TILES 13   // tiles (256 runs) per block: 65 tiles per view = 5 blocks per lane (each block stages the tables once)
-#define SHADE_GROUP 1    // tiles per step
-static_assert(SW % SHADE_RUN == 0 && SHADE_RUN == 4, "plane_shade_kernel: a run is one 16-byte load of per-pixel words and one 4-byte store");
-// STAGED: the lane's plane table is short enough for LDS (the kernel then reads it with LDS instructions; a pointer that may be
-// either costs more).
-template <bool STAGED>
-// Eight wavefronts per SIMD.  The kernel runs beside the flat pass (launch_chunk) and the billboards follow it on the same
-// stream: the sooner it is done, the sooner they are (with the billboards still after the flat pass, five wavefronts per
-// SIMD and two tiles per step were better: the flat pass's kernels found more room beside it).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) plane_shade_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
+// A wavefront takes a tile of 64 columns and SHADE_ROWS rows, a column a lane.  Everything but the texel is the same along a run of
+// pixels of a row that show one plane: each run's leftmost pixel is listed, a lane works out each listed run (PlaneSpan, one pass for
+// up to 64 of them: a tile has some forty), and its pixels read it back from LDS.  Bound by the per-pixel words in, gathers from the
+// textures and LDS; a work-group is four tiles (all of a lane's by two work-groups: 0.41 ms, five tiles 0.44, stores of four columns' words 0.54).
+// 4096 lanes on the 4000-linedef map: 0.69 ms with a run of four pixels a thread (three times the vector instructions, each plane of the
+// four worked out again), 0.38 now; 1024 lanes 0.202 -> 0.106, 16 lanes 0.043 -> 0.013.
+#define SHADE_ROWS 16
+#define SHADE_BATCH 4        // rows whose texels are asked for together
+#define RUN_NONE 0x7FFu      // the number of a pixel's run, or that it has none (a tile has at most 1024)
+#define RUN_BEGINS 0x8000u
+#define SHADE_THREADS 256
+#define SHADE_TILES ((SW / 64) * (VH / SHADE_ROWS))      // a lane's; a wavefront takes one
+static_assert(SW % 64 == 0 && VH % SHADE_ROWS == 0 && SHADE_ROWS <= 16, "plane_shade_kernel: whole tiles, of at most 1024 runs");
+static_assert((GD_SCREEN_HEIGHT - VH) * SW / 4 <= SHADE_TILES * 64, "plane_shade_kernel: a tile clears a word of the status bar a lane");
+__global__ void __launch_bounds__(SHADE_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) plane_shade_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
-    __shared__ float4 sector_lds[LDS_SECTORS];
-    __shared__ unsigned int sector_level_lds[LDS_SECTORS];
-    __shared__ TexLds tex_lds;
-    __shared__ unsigned char colormap_lds[32 * 256];
-    __shared__ i64 level_plane_lds[2 * PLANE_LEVELS * 2];
-    __shared__ i64 step_scale_lds[STEP_TABLE];
+    constexpr int WAVES = SHADE_THREADS / 64;
+    __shared__ __align__(16) unsigned char colormap_lds[32 * 256];
+    __shared__ uint4 start_lds[WAVES][64], step_lds[WAVES][64];
+    __shared__ unsigned int texture_lds[WAVES][64];     // a listed run, until its lane puts the run's texture there
     const int local = blockIdx.y;
     if (local >= lane_count) return;     // uniform over the block
-    Tables tb;
-    stage_tables(m, sector_lds, &tex_lds, tb);
-    for (int k = threadIdx.x; k < 32 * 256 / 4; k += blockDim.x) reinterpret_cast<unsigned int *>(colormap_lds)[k] = reinterpret_cast<const unsigned int *>(m->colormap)[k];
-    const int floors = m->floor_level_count, levels = floors + m->ceil_level_count;
-    const bool tabled = dm.sector_level != nullptr;
-    const bool levels_staged = STAGED;
-    if (tabled) {
-        for (int s = threadIdx.x; s < tb.sector_cached; s += blockDim.x) sector_level_lds[s] = dm.sector_level[s];
-        if (levels_staged) for (int k = threadIdx.x; k < 2 * levels; k += blockDim.x) level_plane_lds[k] = sc.level_plane[(size_t)local * levels * 2 + k];
-        if (threadIdx.x < STEP_TABLE) step_scale_lds[threadIdx.x] = sc.step_scale[(size_t)local * STEP_TABLE + threadIdx.x];
-    }
-    __syncthreads();
-    LaneTables lt; lt.step_scale = step_scale_lds; lt.floors = floors;
-    if (STAGED) lt.level_plane = level_plane_lds;
-    else lt.level_plane = sc.level_plane + (size_t)local * levels * 2;
     const LaneCtx &c = sc.ctx[local];
+    const int lane_id = threadIdx.x & 63, wave = threadIdx.x >> 6;
     unsigned char *frame = frame_base + (size_t)local * frame_stride;
-    const bool frame_aligned = (reinterpret_cast<size_t>(frame) & 3) == 0;
-    const uint4 *meta_groups = reinterpret_cast<const uint4 *>(sc.meta + (size_t)local * VH * SW);
-    // A thread takes SHADE_RUN neighbouring pixels of a row (a row is a whole number of runs): their per-pixel words arrive
-    // in one load, pixels that show the same plane share everything but two products, and the run's bytes leave in
-    // one store.  SHADE_GROUP runs, a tile apart, per step, each stage's loads issued together.
-    for (int tile0 = 0; tile0 < SHADE_TILES; tile0 += SHADE_GROUP) {
-        unsigned int meta[SHADE_GROUP][SHADE_RUN];
-        int first_pixel[SHADE_GROUP];
+    // the lane's words and view pixels as buffers: a pixel that is not this kernel's is stored beyond the end, which the hardware drops
+    // (with a branch around every store the rows' addresses and masks alone would fill the registers)
+    const __amdgpu_buffer_rsrc_t words = __builtin_amdgcn_make_buffer_rsrc(sc.meta + (size_t)local * VH * SW, 0, VH * SW * 4, BUFFER_WORDS);
+    const __amdgpu_buffer_rsrc_t pixels = __builtin_amdgcn_make_buffer_rsrc(frame, 0, VH * SW, BUFFER_WORDS);
+    const unsigned atlas_width = (unsigned)m->tex_max_w;
+    // what names a pixel's plane in its word: the sector and which of its two planes
+    const unsigned int PLANE_KEY = (META_SECTOR_MASK << META_SECTOR_SHIFT) | META_FLOOR;
+    const int tile = blockIdx.x * WAVES + wave, x_first = tile % (SW / 64) * 64, y_first = tile / (SW / 64) * SHADE_ROWS;
+    const unsigned at = (unsigned)(y_first * SW + x_first + lane_id);
+    auto put = [&](bool own, int r, unsigned colour) { __builtin_amdgcn_raw_buffer_store_b8((unsigned char)colour, pixels, own ? at : BUFFER_NOWHERE, r * SW, 0); };
+    unsigned int meta[SHADE_ROWS];
 #pragma unroll
-        for (int g = 0; g < SHADE_GROUP; ++g) {
-            const int run = (blockIdx.x * SHADE_TILES + tile0 + g) * 256 + threadIdx.x;
-            const bool valid = tile0 + g < SHADE_TILES && run < VH * SW / SHADE_RUN;
-            first_pixel[g] = valid ? run * SHADE_RUN : -1;
-            const uint4 words = meta_groups[valid ? run : 0];
-            meta[g][0] = words.x; meta[g][1] = words.y; meta[g][2] = words.z; meta[g][3] = words.w;
-            if (valid && run < (GD_SCREEN_HEIGHT - VH) * SW / SHADE_RUN) {   // the empty status bar, rows 208..239
-                unsigned char *bar = frame + (size_t)VH * SW + (size_t)run * SHADE_RUN;
-                if (frame_aligned) *reinterpret_cast<unsigned int *>(bar) = 0u;
-                else for (int k = 0; k < SHADE_RUN; ++k) bar[k] = 0;
-            }
+    for (int r = 0; r < SHADE_ROWS; ++r) meta[r] = __builtin_amdgcn_raw_buffer_load_b32(words, at * 4u, r * (SW * 4), 0);
+    for (int k = threadIdx.x; k < 32 * 256 / 16; k += SHADE_THREADS) reinterpret_cast<uint4 *>(colormap_lds)[k] = reinterpret_cast<const uint4 *>(m->colormap)[k];
+    __syncthreads();
+    if (tile < (GD_SCREEN_HEIGHT - VH) * SW / 4 / 64) {   // the empty status bar, rows 208..239
+        unsigned char *bar = frame + (size_t)VH * SW + (size_t)(tile * 64 + lane_id) * 4;
+        if ((reinterpret_cast<size_t>(frame) & 3) == 0) *reinterpret_cast<unsigned int *>(bar) = 0u;
+        else for (int k = 0; k < 4; ++k) bar[k] = 0;
+    }
+    if (tile >= SHADE_TILES) return;     // the last work-group's spare wavefronts; their words lay beyond the buffer
+    // Each pixel's word becomes: what names its plane, the number of its run, whether it begins the run; or a tier's colour.
+    int total = 0;
+#pragma unroll
+    for (int r = 0; r < SHADE_ROWS; ++r) {
+        // no run where no plane shows (a wall tier, a masked texture, or neither tier nor plane: the flat pass's picture, which
+        // flat_shade_kernel paints once that pass has run)
+        const unsigned int word = meta[r];
+        const bool plane = !(word & (META_FILLED | META_MASKED)) && (word & (META_SECTOR_MASK << META_SECTOR_SHIFT));
+        const unsigned int key = plane ? word & PLANE_KEY : 0u;
+        const unsigned int left = (unsigned)__builtin_amdgcn_update_dpp(0, (int)key, 0x138 /* wave_shr:1 */, 0xF, 0xF, false);
+        const u64 begins = __ballot(key != 0u && key != left), before = begins >> 1;
+        const int run = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(before >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)before, 0u)) + (total + (int)(begins & 1) - 1);
+        const bool tier = (word & (META_FILLED | META_MASKED)) == META_FILLED;
+        meta[r] = plane ? key | (unsigned)run | (key != left ? RUN_BEGINS : 0u) : (tier ? (word & (META_FILLED | (META_SECTOR_MASK << META_SECTOR_SHIFT))) : 0u) | RUN_NONE;
+        if (key != 0u && key != left && run < 64) texture_lds[wave][run] = key | (unsigned)r;
+        total += __popcll(begins);
+    }
+    for (unsigned first = 0;;) {     // one round, but for the most varied tiles
+        wave_lds_fence();
+        if (first + lane_id < (unsigned)total) {
+            const unsigned int listed = texture_lds[wave][lane_id];
+            const PlaneSpan span = plane_span(dm, sc, c, local, (int)((listed >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1, (listed & META_FLOOR) != 0, x_first, y_first + (int)(listed & 0xFFFFu));
+            start_lds[wave][lane_id] = span.start; step_lds[wave][lane_id] = span.step; texture_lds[wave][lane_id] = span.texture;
         }
-        int colormap_row[SHADE_GROUP][SHADE_RUN]; unsigned char texel[SHADE_GROUP][SHADE_RUN];
-        unsigned int shades[SHADE_GROUP];   // bit k: pixel k of the run shows a visplane's flat
+        wave_lds_fence();
 #pragma unroll
-        for (int g = 0; g < SHADE_GROUP; ++g) {
-            shades[g] = 0;
-            const int pixel0 = first_pixel[g] < 0 ? 0 : first_pixel[g];
-            const int y = pixel0 / SW, x0 = pixel0 - y * SW;
-            // what names a pixel's plane in its word: the sector and which of its two planes
-            const unsigned int PLANE_KEY = (META_SECTOR_MASK << META_SECTOR_SHIFT) | META_FLOOR;
-            int leader = -1;
+        for (int r0 = 0; r0 < SHADE_ROWS; r0 += SHADE_BATCH) {
+            unsigned shade_at[SHADE_BATCH]; unsigned char texel[SHADE_BATCH];
+            bool any = false;
 #pragma unroll
-            for (int k = 0; k < SHADE_RUN; ++k) {
-                const int ps = (int)((meta[g][k] >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1;
-                texel[g][k] = 0; colormap_row[g][k] = 0;
-                if (tabled && first_pixel[g] >= 0 && ps >= 0 && !(meta[g][k] & (META_FILLED | META_MASKED))) {
-                    shades[g] |= 1u << k;
-                    if (leader < 0) leader = k;
+            for (int j = 0; j < SHADE_BATCH; ++j) { any |= (meta[r0 + j] & RUN_NONE) - first < 64u; shade_at[j] = 0u; texel[j] = 0; }
+            if (__any(any)) {
+#pragma unroll
+                for (int j = 0; j < SHADE_BATCH; ++j) {
+                    unsigned run = (meta[r0 + j] & RUN_NONE) - first;
+                    run = run < 64u ? run : 0u;        // a pixel without one asks for a texel of the first run's: in the atlas too
+                    PlaneSpan span;
+                    span.start = start_lds[wave][run]; span.step = step_lds[wave][run]; span.texture = texture_lds[wave][run];
+                    texel[j] = m->tex_atlas[span.texel((unsigned)lane_id, atlas_width)];
+                    shade_at[j] = span.colormap_row() * 256;
                 }
             }
-            if (leader < 0) continue;
-            const i64 yslope = sc.row_slope[(size_t)local * VH + y];
-            unsigned int leader_word = meta[g][0];
 #pragma unroll
-            for (int k = 1; k < SHADE_RUN; ++k) if (leader == k) leader_word = meta[g][k];
-            auto span_of = [&](unsigned int word) {
-                const int sector = (int)((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1;
-                const bool is_floor = (word & META_FLOOR) != 0;
-                const unsigned int pair = sector < tb.sector_cached ? sector_level_lds[sector] : dm.sector_level[sector];
-                return plane_span(tb, c, lt, yslope, is_floor ? (pair & 0xFFFF) : (pair >> 16), sector, is_floor, x0, y);
-            };
-            const PlaneSpan shared = span_of(leader_word);
-#pragma unroll
-            for (int k = 0; k < SHADE_RUN; ++k) {
-                if (!(shades[g] & (1u << k))) continue;
-                if (((meta[g][k] ^ leader_word) & PLANE_KEY) == 0) {
-                    colormap_row[g][k] = shared.colormap_row;
-                    texel[g][k] = m->tex_atlas[plane_span_texel(shared, k)];
-                } else {   // another plane starts inside the run
-                    const PlaneSpan own = span_of(meta[g][k]);
-                    colormap_row[g][k] = own.colormap_row;
-                    texel[g][k] = m->tex_atlas[plane_span_texel(own, k)];
-                }
+            for (int j = 0; j < SHADE_BATCH; ++j) {
+                const bool tier = (meta[r0 + j] & META_FILLED) && first == 0;
+                put(tier || (meta[r0 + j] & RUN_NONE) - first < 64u, r0 + j, tier ? meta[r0 + j] >> META_SECTOR_SHIFT : colormap_lds[shade_at[j] + texel[j]]);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
+        first += 64;
+        if (first >= (unsigned)total) break;
+        wave_lds_fence();
 #pragma unroll
-        for (int g = 0; g < SHADE_GROUP; ++g) {
-            if (first_pixel[g] < 0) continue;
-            const int y = first_pixel[g] / SW, x0 = first_pixel[g] - y * SW;
-            unsigned int colours = 0, written = 0;   // bit k of `written`: this kernel decides pixel k
-#pragma unroll
-            for (int k = 0; k < SHADE_RUN; ++k) {
-                const unsigned int word = meta[g][k];
-                const int ps = (int)((word >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1;
-                unsigned int colour = 0; bool writes = false;
-                if (word & META_FILLED) {   // a wall tier's pixel, unless a masked texture went over it
-                    colour = (word >> META_SECTOR_SHIFT) & 0xFFu; writes = !(word & META_MASKED);
-                } else if (ps >= 0) {
-                    // (neither tier nor plane: the flat pass's picture shows there, unless a masked texture covers it;
-                    // flat_shade_kernel paints the pixel once that pass has run)
-                    const bool is_floor = (word & META_FLOOR) != 0;
-                    if (shades[g] & (1u << k)) { colour = colormap_lds[colormap_row[g][k] * 256 + texel[g][k]]; writes = true; }
-                    else if (!(word & META_MASKED)) { colour = flat_pixel(tb, colormap_lds, c, ps, is_floor, x0 + k, y); writes = true; }
-                }
-                colours |= colour << (8 * k);
-                if (writes) written |= 1u << k;
-            }
-            unsigned char *out = frame + first_pixel[g];
-            if (written == (1u << SHADE_RUN) - 1 && frame_aligned) {
-                *reinterpret_cast<unsigned int *>(out) = colours;
-            } else {   // some pixel of the run is the flat pass's or a masked texture's: byte by byte
-#pragma unroll
-                for (int k = 0; k < SHADE_RUN; ++k) if (written & (1u << k)) out[k] = (unsigned char)(colours >> (8 * k));
-            }
+        for (int r = 0; r < SHADE_ROWS; ++r) {
+            asm volatile("" : "+v"(meta[r]));      // worked on afresh in every round: kept over the rounds, its derivatives would fill the registers
+            const unsigned run = (meta[r] & RUN_NONE) - first;
+            if ((meta[r] & RUN_BEGINS) && run < 64u) texture_lds[wave][run] = (meta[r] & PLANE_KEY) | (unsigned)r;
         }
     }
 }
@@ -5709,9 +5696,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     // timed (and so serial): shading, then the flat pass, each between its own marks
     auto shade_planes = [&]() {
         if (fused) return;
-        const dim3 grid(((VH * SW / SHADE_RUN + 255) / 256 + SHADE_TILES - 1) / SHADE_TILES, count);
-        const bool staged = m.floor_level_count + m.ceil_level_count <= 2 * PLANE_LEVELS;
-        hipLaunchKernelGGL(staged ? plane_shade_kernel<true> : plane_shade_kernel<false>, grid, dim3(256), 0, shade_stream, r->dm, count, sc, frame_base, frame_stride);
+        hipLaunchKernelGGL(plane_shade_kernel, dim3((SHADE_TILES + SHADE_THREADS / 64 - 1) / (SHADE_THREADS / 64), count), dim3(SHADE_THREADS), 0, shade_stream, r->dm, count, sc, frame_base, frame_stride);
     };
     if (!beside) shade_planes();
     mark();
