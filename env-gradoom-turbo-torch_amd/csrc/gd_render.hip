@@ -4,7 +4,7 @@
 //
 //   lane_setup      1 thread / lane           view basis, pitch centre, camera sector
 //   lane_tables     1 thread / (lane, row)    per-lane distance bounds of every height level, plane rows, row slopes
-//   wall_setup      1 wave-slot / (lane,wall) FWallCoords span+depths, span ownership bounds, the linedef's
+//   wall_setup      1 block / lane or 256 linedefs  FWallCoords span+depths, span ownership bounds, the linedef's
 //                                             entry in the candidate list of every column it can own, and the
 //                                             nearest blocking hit of every column (64-bit atomicMin)
 //   strip_key/order 1 thread / 64-col strip   longest strip first (counting sort on the blocking distance)
@@ -380,6 +380,13 @@ __device__ __forceinline__ i64 tdiv(i64 a, i64 b) {
     const u64 sign = (u64)((a ^ b) >> 63);
     return (i64)((uq ^ sign) - sign);
 }
+// Lanes of one wavefront leave words in LDS for one another: the order is the program's, the compiler has to keep it.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Value of `v` in lane `lane` of the wavefront; `lane` must be the same in every active lane.
 __device__ __forceinline__ int bcast(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ float bcast(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
@@ -694,7 +701,9 @@ __global__ void lane_setup_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_ba
 
 __device__ __forceinline__ void ray_direction(const LaneCtx &c, int x, float *rx, float *ry) {
     // engine.py:10660-10670
-    float col = ((float)x - 160.0f) / 160.0f;
+    // (x - 160) / 160, correctly rounded: the reciprocal's product and one step (every column's quotient is the division's)
+    const float across = (float)x - 160.0f, inverse = 1.0f / 160.0f, near = across * inverse;
+    const float col = __builtin_fmaf(__builtin_fmaf(-160.0f, near, across), inverse, near);
     *rx = c.fcos + c.fsin * col;
     *ry = c.fsin - c.fcos * col;
 }
@@ -786,28 +795,78 @@ __device__ __forceinline__ void request_spill_slot(const Scratch &sc, int column
     else sc.status[STATUS_CAND_OVERFLOW] = 1;
 }
 
-// One thread owns one linedef for the per-linedef arithmetic.  The two per-column loops have
-// wildly different trip counts per linedef (none for most, up to 320 for a few), so they are
-// run by the whole wavefront together: the linedefs with a non-empty column range take turns,
-// their parameters are broadcast from the owning lane, and the 64 lanes each take one column.
+// One thread owns one linedef for the per-linedef arithmetic; its columns are looked at by the whole wavefront together, since
+// linedefs reach from none of them to all 320.  A linedef has a window of columns its rays or its owned span can lie in, so one
+// look at each of them says where its rays hit it, which gives the span it owns, which says where it is a candidate.  Windows of up
+// to 8, 16 and 32 columns share a turn, as many linedefs as fit, a wider one has the wavefront to itself.  What a turn asks of its
+// linedefs lies in LDS, and so do the lists of linedefs by width.
 //
 // Three quarters of a map's linedefs lie wholly behind the camera or wholly to one side of its view: no
 // column ray can hit such a linedef and FWallCoords rejects it, so nothing of it is ever looked at beyond
-// the ray-test facts of RecSpan (no owned span).  A block first sorts its SETUP_WALLS linedefs into those and the
-// rest, and only the rest, packed into as few wavefronts as they fill, get the arithmetic below.
-#define SETUP_WALLS 256
-__global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, int lane_count, Scratch sc) {
+// the ray-test facts of RecSpan (no owned span).  A block first sorts its linedefs into those and the
+// rest, and only the rest are shared out over its wavefronts.
+// Bound by its vector instructions, then by the latency of a turn's steps.  4096 lanes on the 4000-linedef map: 0.61 ms with two looks a
+// column (one for the hits, one for the candidates), parameters by lane exchange and counts by atomics in device memory, 0.53 with one
+// look and LDS parameters, 0.45 with counts in LDS; 16 lanes on the 320-linedef map 0.040 -> 0.019.
+#define SETUP_THREADS 256
+#define SETUP_WHOLE_THREADS 512
+// A work-group takes a whole lane where there are lanes enough for the chip, and where a lane's linedefs would be two work-groups at
+// most anyway.  Stages up to the strips' order in us, dealt out / whole lanes: 120 linedefs, 16 lanes 48 / 37, 512 lanes 57 / 51; 320, 16 lanes 51 / 45,
+// 512 lanes 67 / 58; 701, 16 lanes 49 / 55, 640 lanes 75 / 76; 1400, 256 lanes 64 / 73, 768 lanes 99 / 97, 1024 lanes 115 / 114; 2000, 256 lanes
+// 68 / 104, 768 lanes 106 / 114, 1024 lanes 126 / 123; 4000, 256 lanes 79 / 116, 768 lanes 152 / 159, 1024 lanes 188 / 179, 4096 lanes 708 / 509.
+bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || linedefs <= 2 * SETUP_THREADS; }
+#define SETUP_WALLS_MAX 4096      // linedefs sorted at a time
+struct SetupWall {                // a linedef as the columns' look at it asks for it
+    float segx, segy, offx, offy;
+    float numer;                  // of the ray distance
+    int window;                   // first column | one past the last << 16
+    int facts;                    // WF_* but for WF_HC and WF_ANYGEO, and SETUP_*
+    int ends;                     // screen column of the left endpoint | of the right one << 9 | their visibility << 18, 19
+    int sectors, vertices, wall;
+    int blocking;                 // its position in blocking_walls, -1
+};
+#define SETUP_ONE_SIDED 0x200     // free bits of the WF_* word
+#define SETUP_MASKED 0x400        // a mid-texture on the side facing the camera
+#define SETUP_SPANS 0x800         // FWallCoords' span is not empty
+// The span a linedef owns (engine.py:11347-11427), within [0, 320]: first column | one past the last << 16, bit 31 when it owns any.
+__device__ __forceinline__ int setup_owned(int facts, int ends, bool any, int first, int last) {
+    const int left = ends & 511, right = (ends >> 9) & 511;
+    const bool left_visible = (ends >> 18) & 1, right_visible = (ends >> 19) & 1;
+    const bool both = left_visible && right_visible;
+    const int from = both || (any && left_visible) ? left : first, to = both || (any && right_visible) ? right : last + 1;
+    const bool owns = (both ? to > from : any) && (facts & SETUP_SPANS);
+    return from | (to << 16) | (owns ? (int)0x80000000u : 0);
+}
+// WHOLE: one work-group goes over all linedefs of a lane, SETUP_WALLS_MAX at a time, and keeps what its columns count in LDS; else the
+// linedefs of a lane are dealt out, SETUP_THREADS a work-group, and they count in device memory.
+template <bool WHOLE>
+__global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) wall_setup_kernel(DeviceMap dm, int lane_count, Scratch sc) {
     const gd_map_desc *m = &dm.d;
-    __shared__ int alive_list[SETUP_WALLS];
+    constexpr int THREADS = WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS, WAVES = THREADS / 64, ROUND = WHOLE ? SETUP_WALLS_MAX : SETUP_THREADS;
+    __shared__ unsigned short alive_list[ROUND];
     __shared__ int alive_count;
-    const int slot_in_wave = threadIdx.x & 63;
+    __shared__ __align__(16) SetupWall walls_lds[WAVES][64];
+    __shared__ int hits_lds[WAVES][64];                  // per linedef: first column a ray hits it at | one past the last << 16
+    __shared__ unsigned char by_width[WAVES][3][64];     // the linedefs with windows of up to 8, 16, 32 columns
+    __shared__ float wide_lds[WAVES][SW];                // a wide window's looks: the ray distance, negative where the ray is nearer the end, 0 for none
+    __shared__ u64 wide_hits[WAVES][SW / 64];            // and the rays that hit, a word a turn
+    __shared__ u64 block_lds[WHOLE ? SW : 1], masked_lds[WHOLE ? SW : 1];
+    __shared__ int count_lds[WHOLE ? SW : 1];
+    const int slot = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int local = blockIdx.y;
     if (local >= lane_count) return;          // uniform over the block
     const LaneCtx &c = sc.ctx[local];
+    u64 *block_hits = WHOLE ? block_lds : sc.block_hit + (size_t)local * SW, *masked_hits = WHOLE ? masked_lds : sc.masked_hit + (size_t)local * SW;
+    int *counts = WHOLE ? count_lds : sc.cand_count + (size_t)local * SW;
+    Cand *list = sc.cand + (size_t)local * CAND_MAX * SW;
+    if (WHOLE) for (int x = threadIdx.x; x < SW; x += THREADS) { block_lds[x] = ~0ULL; masked_lds[x] = CAND_KEY_NONE; count_lds[x] = 0; }
+    for (int round0 = WHOLE ? 0 : blockIdx.x * ROUND; round0 < (WHOLE ? m->wall_count : (int)(blockIdx.x + 1) * ROUND); round0 += ROUND) {
+    __syncthreads();                                     // nobody reads the list of the round before any more
     if (threadIdx.x == 0) alive_count = 0;
     __syncthreads();
-    {
-        const int w = blockIdx.x * SETUP_WALLS + threadIdx.x;
+    for (int k = threadIdx.x; k < ROUND; k += THREADS) {
+        const int w = round0 + k;
+        bool kept = false;
         if (w < m->wall_count) {
             const float4 wl = *reinterpret_cast<const float4 *>(m->walls + 4 * w);
             const float ax = wl.x - c.x, ay = wl.y - c.y, bx = wl.z - c.x, by = wl.w - c.y;
@@ -818,10 +877,8 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
             // unit to spare, far more than float32 and 16.16 coordinates can disagree): no ray reaches it, FWallCoords finds
             // no span.  Linedef 0 and the first blocking linedef stand in where a scan finds nothing, and are always kept.
             const bool unseen = (f0 < -1.0f && f1 < -1.0f) || (r0 > f0 + 1.0f && r1 > f1 + 1.0f) || (r0 < -f0 - 1.0f && r1 < -f1 - 1.0f);
-            const bool kept = !unseen || w == 0 || (m->blocking_count > 0 && w == m->blocking_walls[0]);
-            if (kept) {
-                alive_list[atomicAdd(&alive_count, 1)] = w;
-            } else {
+            kept = !unseen || w == 0 || (m->blocking_count > 0 && w == m->blocking_walls[0]);
+            if (!kept) {
                 const float vfx = c.x - wl.x, vfy = c.y - wl.y;
                 const bool ff = ((wl.z - wl.x) * vfy - (wl.w - wl.y) * vfx) < 0;
                 RecSpan span;
@@ -833,245 +890,194 @@ __global__ void __launch_bounds__(SETUP_WALLS) wall_setup_kernel(DeviceMap dm, i
                 sc.span[(size_t)local * m->wall_count + w] = span;
             }
         }
+        const u64 keeps = __ballot(kept);
+        int base = 0;
+        if (slot == 0 && keeps) base = atomicAdd(&alive_count, __popcll(keeps));
+        base = __builtin_amdgcn_readfirstlane(base);
+        if (kept) alive_list[base + __popcll(keeps & ((1ULL << slot) - 1))] = (unsigned short)w;
     }
     __syncthreads();
     const int alive = alive_count;
-    if ((int)(threadIdx.x & ~63u) >= alive) return;   // whole wavefronts beyond the kept linedefs leave
-    const bool live = (int)threadIdx.x < alive;  // dead lanes of the last wavefront still help with the column loops
-    const int w = live ? alive_list[threadIdx.x] : 0;
-    const int *wf = m->walls_fixed + 4 * w;
-    WallRec r;
-    i64 endpoint_quotient[2];
-    wall_coords(c, wf, r, endpoint_quotient);
-    const i64 tx0 = r.tx0, tx1v = r.tx1, ty0 = r.ty0, ty1v = r.ty1;
-    const i64 sl = r.sl, sr = r.sr;
-    const i64 center = 160 * FIXED_UNIT;
-
-    // Ray x segment: first / last column whose ray hits the segment (engine.py:11323-11348).
-    // A ray of column parameter col = (x-160)/160 is forward + col*right; an endpoint with view
-    // coordinates (f, r) lies on it when r = col*f.  The float test below can only pass where the
-    // two endpoints are not both clearly (> half a map unit) on one side of the ray, so for a
-    // segment wholly in front of the camera only the columns between its endpoint columns
-    // (padded) are examined; segments reaching behind the camera get the full scan.
-    const float4 wl = *reinterpret_cast<const float4 *>(m->walls + 4 * w);
-    float segx = wl.z - wl.x, segy = wl.w - wl.y;
-    float offx = wl.x - c.x, offy = wl.y - c.y;
-    int scan_lo = 0, scan_hi = SW - 1;
-    {
-        float e1x = offx + segx, e1y = offy + segy;
-        float f0 = offx * c.fcos + offy * c.fsin, r0 = offx * c.fsin - offy * c.fcos;
-        float f1 = e1x * c.fcos + e1y * c.fsin, r1 = e1x * c.fsin - e1y * c.fcos;
-        if (f0 > 1.0f && f1 > 1.0f) {
-            float c0 = r0 / f0, c1 = r1 / f1, p0 = 0.5f / f0, p1 = 0.5f / f1;
-            float lo = fminf(c0 - p0, c1 - p1), hi = fmaxf(c0 + p0, c1 + p1);
-            float xlo = floorf(160.0f + 160.0f * lo) - 1.0f, xhi = ceilf(160.0f + 160.0f * hi) + 1.0f;
-            scan_lo = xlo < 0.0f ? 0 : (xlo > 320.0f ? 320 : (int)xlo);
-            scan_hi = xhi > 319.0f ? 319 : (xhi < -1.0f ? -1 : (int)xhi);
-        } else if (f0 < -1.0f && f1 < -1.0f) {
-            scan_lo = 1; scan_hi = 0;   // wholly behind the camera: no ray reaches it
+    // the kept linedefs go to the wavefronts in equal shares, of at most 64
+    const int shares = WHOLE ? (alive + 64 * WAVES - 1) / (64 * WAVES) * WAVES : WAVES;
+    const int each = max((alive + shares - 1) / max(shares, 1), 8);
+    for (int first_alive = wave * each; first_alive < alive; first_alive += WAVES * each) {
+        const bool live = slot < each && first_alive + slot < alive;   // the other lanes help with the columns
+        const int w = live ? alive_list[first_alive + slot] : 0;
+        WallRec r;
+        i64 endpoint_quotient[2];
+        wall_coords(c, m->walls_fixed + 4 * w, r, endpoint_quotient);
+        // Ray x segment: the columns whose ray hits the segment (engine.py:11323-11348).
+        // A ray of column parameter col = (x-160)/160 is forward + col*right; an endpoint with view
+        // coordinates (f, r) lies on it when r = col*f.  The float test below can only pass where the
+        // two endpoints are not both clearly (> half a map unit) on one side of the ray, so for a
+        // segment wholly in front of the camera only the columns between its endpoint columns
+        // (padded) are examined; segments reaching behind the camera get the full scan.
+        const float4 wl = *reinterpret_cast<const float4 *>(m->walls + 4 * w);
+        const float segx = wl.z - wl.x, segy = wl.w - wl.y;
+        const float offx = wl.x - c.x, offy = wl.y - c.y;
+        int lo = 0, hi = SW;
+        {
+            const float e1x = offx + segx, e1y = offy + segy;
+            const float f0 = offx * c.fcos + offy * c.fsin, r0 = offx * c.fsin - offy * c.fcos;
+            const float f1 = e1x * c.fcos + e1y * c.fsin, r1 = e1x * c.fsin - e1y * c.fcos;
+            if (f0 > 1.0f && f1 > 1.0f) {
+                const float c0 = r0 / f0, c1 = r1 / f1, p0 = 0.5f / f0, p1 = 0.5f / f1;
+                const float left = fminf(c0 - p0, c1 - p1), right = fmaxf(c0 + p0, c1 + p1);
+                const float xlo = floorf(160.0f + 160.0f * left) - 1.0f, xhi = ceilf(160.0f + 160.0f * right) + 1.0f;
+                lo = xlo < 0.0f ? 0 : (xlo > 320.0f ? 320 : (int)xlo);
+                hi = (xhi > 319.0f ? 319 : (xhi < -1.0f ? -1 : (int)xhi)) + 1;
+            } else if (f0 < -1.0f && f1 < -1.0f) {
+                lo = SW; hi = 0;   // wholly behind the camera: no ray reaches it
+            }
         }
-    }
-    if (!live) { scan_lo = 1; scan_hi = 0; }
-    const int facts = dm.wall_facts[w];
-    const int blocking_slot = (facts >> WALL_BLOCKING_SHIFT) - 1;
-    u64 *block_hits = sc.block_hit + (size_t)local * SW;
-    int first = 0, last = SW - 1; bool any = false;
-    float numer_d = offx * segy - offy * segx;
-    // Most scan ranges are a few columns wide, so several linedefs share a turn (eight lanes each for eight of
-    // them, sixteen for four, thirty-two for two); a wider range has the wavefront to itself.
-    const int scan_width = scan_hi - scan_lo + 1;
-    auto shared_scans = [&](bool member, int lanes_each) {
-        const int group = slot_in_wave / lanes_each, group_lane = slot_in_wave - group * lanes_each;
-        const int groups = 64 / lanes_each;
-        const u64 group_mask = (lanes_each == 64 ? ~0ULL : ((1ULL << lanes_each) - 1)) << (group * lanes_each);
-        for (u64 pending = __ballot(member); pending;) {
-            int owners[8];
-            int owner = -1;
+        const bool ff = (segx * (c.y - wl.y) - segy * (c.x - wl.x)) < 0;
+        int ends = 0;
+        bool visible[2];
+        {   // the endpoints' screen columns: tx * center / ty, as wall_coords divided it
+            const i64 tx[2] = {r.tx0, r.tx1}, ty[2] = {r.ty0, r.ty1};
+            int column[2];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                owners[k] = -1;
-                if (k >= groups) continue;               // the same in every lane
-                owners[k] = pending ? __ffsll((long long)pending) - 1 : -1;
-                pending &= pending - 1;
-                if (group == k) owner = owners[k];
+            for (int e = 0; e < 2; ++e) {
+                const i64 col = ((160 * FIXED_UNIT + endpoint_quotient[e]) >> 16) + (tx[e] >= 0);
+                visible[e] = (ty[e] > 0) && (tx[e] >= -ty[e]) && (tx[e] <= ty[e]) && (col >= 0) && (col <= SW);
+                column[e] = visible[e] ? (int)col : 0;
             }
-            const int source = owner < 0 ? 0 : owner;
-            const float b_segx = __shfl(segx, source), b_segy = __shfl(segy, source);
-            const float b_offx = __shfl(offx, source), b_offy = __shfl(offy, source), b_numer = __shfl(numer_d, source);
-            const int b_lo = __shfl(scan_lo, source), b_hi = __shfl(scan_hi, source);
-            const int b_block = __shfl(blocking_slot, source);
-            const int x = b_lo + group_lane;
-            float rx, ry; ray_direction(c, x, &rx, &ry);
-            float den = rx * b_segy - ry * b_segx;
-            bool ok = fabsf(den) >= 1e-6f;
-            float safe = ok ? den : 1.0f;
-            float d = b_numer / safe;
-            float a = (b_offx * ry - b_offy * rx) / safe;
-            bool g = owner >= 0 && x <= b_hi && ok && (d > 0) && (a >= 0) && (a <= 1);
-            if (g && b_block >= 0) atomicMin(&block_hits[x], ((u64)__float_as_uint(d) << 32) | (u64)(unsigned)b_block);
-            const u64 hits = __ballot(g) & group_mask;
-            // every lane of a group holds its linedef's first / last hit column; the linedef's own lane fetches them
-            const int group_first = hits ? b_lo + (__ffsll((long long)hits) - 1 - group * lanes_each) : SW;
-            const int group_last = hits ? b_lo + (63 - __clzll((long long)hits) - group * lanes_each) : -1;
+            // the owned span begins at the start of a linedef that faces the camera, at the end of one that does not
+            ends = ff ? (column[0] | (column[1] << 9) | (visible[0] ? 1 << 18 : 0) | (visible[1] ? 1 << 19 : 0))
+                      : (column[1] | (column[0] << 9) | (visible[1] ? 1 << 18 : 0) | (visible[0] ? 1 << 19 : 0));
+        }
+        // the window: where rays can hit, and the ends of what the linedef can own
+        const bool scans = lo < hi;
+        int window0 = scans ? lo : SW, window1 = scans ? hi : 0;
+        if (ends & (1 << 18)) window0 = min(window0, ends & 511);
+        if (ends & (1 << 19)) window1 = max(window1, (ends >> 9) & 511);
+        const int s0 = m->wall_sectors[2 * w], s1 = m->wall_sectors[2 * w + 1];
+        const bool os = s1 < 0;
+        const int known = dm.wall_facts[w];
+        const i64 span = r.sr - r.sl;
+        const int facts = (ff ? WF_FF : 0) | ((span <= 1 && !os) ? WF_SUBPIXEL : 0) | ((known & WALL_SPLIT) ? WF_SPLIT : 0) | (span <= 2 ? WF_NARROW : 0) |
+                          ((known & WALL_SHORT) ? WF_SHORT : 0) | ((r.sr >= 0 && r.sr < SW ? (int)r.sr : WF_END_NONE) << WF_END_SHIFT) |
+                          (os ? SETUP_ONE_SIDED : 0) | (!os && m->side_tex[(w * 2 + (ff ? 0 : 1)) * 3] >= 0 ? SETUP_MASKED : 0) | (span > 0 ? SETUP_SPANS : 0);
+        {
+            SetupWall mine;
+            mine.segx = segx; mine.segy = segy; mine.offx = offx; mine.offy = offy;
+            mine.numer = offx * segy - offy * segx;
+            mine.window = window0 | (window1 << 16);
+            mine.facts = facts; mine.ends = ends;
+            mine.sectors = (s0 & 0xFFFF) | (s1 << 16);
+            mine.vertices = (int)(((unsigned)m->wall_vertex[2 * w] & 0xFFFFu) | ((unsigned)m->wall_vertex[2 * w + 1] << 16));
+            mine.wall = w; mine.blocking = (known >> WALL_BLOCKING_SHIFT) - 1;
+            walls_lds[wave][slot] = mine;
+            hits_lds[wave][slot] = SW;                    // none: first 320, one past the last 0
+        }
+        const int width = live ? max(window1 - window0, 0) : 0;
+        int members[3];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                if (k >= groups || owners[k] < 0) continue;   // the same in every lane
-                const int k_first = bcast(group_first, k * lanes_each), k_last = bcast(group_last, k * lanes_each);
-                if (slot_in_wave == owners[k] && k_last >= 0) { first = k_first; last = k_last; any = true; }
-            }
+        for (int k = 0; k < 3; ++k) {
+            const bool member = width > (k ? 4 << k : 0) && width <= (8 << k);
+            const u64 all = __ballot(member);
+            if (member) by_width[wave][k][__popcll(all & ((1ULL << slot) - 1))] = (unsigned char)slot;
+            members[k] = __popcll(all);
         }
-    };
-    const bool scans = scan_lo <= scan_hi;
-    shared_scans(scans && scan_width <= 8, 8);
-    shared_scans(scans && scan_width > 8 && scan_width <= 16, 16);
-    shared_scans(scans && scan_width > 16 && scan_width <= 32, 32);
-    for (u64 pending = __ballot(scans && scan_width > 32); pending; pending &= pending - 1) {
-        const int owner = __ffsll((long long)pending) - 1;
-        const float b_segx = bcast(segx, owner), b_segy = bcast(segy, owner);
-        const float b_offx = bcast(offx, owner), b_offy = bcast(offy, owner), b_numer = bcast(numer_d, owner);
-        const int b_lo = bcast(scan_lo, owner), b_hi = bcast(scan_hi, owner);
-        const int b_block = bcast(blocking_slot, owner);
-        int hit_first = SW, hit_last = -1;
-        for (int x0 = b_lo; x0 <= b_hi; x0 += 64) {
-            const int x = x0 + slot_in_wave;
+        wave_lds_fence();
+        // The linedef at column x, its rays and owned span known: a candidate there if its distance is finite (engine.py:11446-11451).
+        // List order is irrelevant: scans break ties on the linedef index.
+        auto enter = [&](const SetupWall &q, int x, bool ok, bool g, bool along_high, float d, int owned) {
+            const int from = owned & 0xFFFF, to = (owned >> 16) & 0x7FFF;
+            const bool p = ok && d > 0 && owned < 0 && x >= from && x < to;
+            const bool valid = (q.facts & SETUP_ONE_SIDED) ? p && (q.facts & WF_FF) : (g || p);
+            if (!valid || !finitef(d)) return;
+            const int flags = (g ? CF_GEO : 0) | (p ? CF_PROJ : 0) | ((x == from) ? CF_LEDGE : 0) | (along_high ? CF_ALONG_HI : 0) |
+                              (((q.facts >> WF_END_SHIFT) == x) ? CF_ENDS_HERE : 0) | (q.facts & WF_SHOWN);
+            Cand entry;
+            entry.flags = (unsigned short)flags; entry.wall = (unsigned short)q.wall;
+            entry.s0 = (short)(q.sectors & 0xFFFF); entry.s1 = (short)(q.sectors >> 16);
+            entry.v0 = (unsigned short)(q.vertices & 0xFFFF); entry.v1 = (unsigned short)((unsigned)q.vertices >> 16);
+            entry.dist = d;
+            if ((q.facts & SETUP_MASKED) && p) atomicMin(&masked_hits[x], cand_key(entry));
+            const int at = atomicAdd(&counts[x], 1);
+            if (at < CAND_MAX) list[(size_t)at * SW + x] = entry;
+            // else: the count says so, and the column is listed afresh in the spill pool (strip_key_kernel, cand_spill_kernel)
+        };
+        auto look = [&](const SetupWall &q, int x, bool &ok, bool &along_high, float &d) -> bool {   // eval_segment's ray test
             float rx, ry; ray_direction(c, x, &rx, &ry);
-            float den = rx * b_segy - ry * b_segx;
-            bool ok = fabsf(den) >= 1e-6f;
-            float safe = ok ? den : 1.0f;
-            float d = b_numer / safe;
-            float a = (b_offx * ry - b_offy * rx) / safe;
-            bool g = x <= b_hi && ok && (d > 0) && (a >= 0) && (a <= 1);
-            // the sprite pass wants the nearest blocking linedef each column ray hits, lowest slot on ties
-            if (g && b_block >= 0) atomicMin(&block_hits[x], ((u64)__float_as_uint(d) << 32) | (u64)(unsigned)b_block);
-            const u64 hits = __ballot(g);
-            if (hits) {
-                if (hit_last < 0) hit_first = x0 + __ffsll((long long)hits) - 1;
-                hit_last = x0 + 63 - __clzll((long long)hits);
-            }
-        }
-        if (slot_in_wave == owner && hit_last >= 0) { first = hit_first; last = hit_last; any = true; }
-    }
-    float vfx = c.x - wl.x, vfy = c.y - wl.y;
-    bool ff = (segx * vfy - segy * vfx) < 0;
-    i64 screen_left = first, screen_right = (i64)last + 1;
-    bool hc = any;
-    i64 ep_col[2]; bool ep_vis[2];
-    i64 txe[2] = {tx0, tx1v}, tye[2] = {ty0, ty1v};
-    for (int e = 0; e < 2; ++e) {
-        i64 projected_fixed = center + endpoint_quotient[e];   // tx * center / ty, as wall_coords divided it
-        ep_col[e] = (projected_fixed >> 16) + (txe[e] >= 0);
-        ep_vis[e] = (tye[e] > 0) && (txe[e] >= -tye[e]) && (txe[e] <= tye[e]) && (ep_col[e] >= 0) && (ep_col[e] <= SW);
-    }
-    for (int e = 0; e < 2; ++e) {
-        bool visible = ep_vis[e] && hc;
-        bool owns_left = ff ? (e == 0) : (e == 1);
-        if (visible && owns_left) screen_left = ep_col[e];
-        if (visible && !owns_left) screen_right = ep_col[e];
-    }
-    if (ep_vis[0] && ep_vis[1]) {
-        screen_left = ff ? ep_col[0] : ep_col[1];
-        screen_right = ff ? ep_col[1] : ep_col[0];
-        hc = screen_right > screen_left;
-    }
-    hc = hc && (sr > sl);
-    const int s0 = m->wall_sectors[2 * w], s1 = m->wall_sectors[2 * w + 1];
-    bool os = s1 < 0;
-    r.pl = (short)screen_left; r.pr = (short)screen_right;
-    r.flags = (hc ? WF_HC : 0) | (ff ? WF_FF : 0) | (((sr - sl <= 1) && !os) ? WF_SUBPIXEL : 0) | (any ? WF_ANYGEO : 0) |
-              ((facts & WALL_SPLIT) ? WF_SPLIT : 0) | (sr - sl <= 2 ? WF_NARROW : 0) | ((facts & WALL_SHORT) ? WF_SHORT : 0) |
-              ((sr >= 0 && sr < SW ? (int)sr : WF_END_NONE) << WF_END_SHIFT);
-    if (live) {
-        sc.rec[(size_t)local * m->wall_count + w] = r;
-        RecSpan span;
-        span.pl = r.pl; span.pr = r.pr; span.flags = r.flags;
-        sc.span[(size_t)local * m->wall_count + w] = span;
-    }
-    // Enter the linedef in the candidate list of every column where its distance can be
-    // finite: its owned span (projected) and, for two-sided lines, the columns its rays hit
-    // (engine.py:11446-11451).  List order is irrelevant: scans break ties on the linedef index.
-    int a_lo = SW, a_hi = 0;
-    if (hc && (!os || ff)) { a_lo = r.pl; a_hi = r.pr; }
-    if (!os && any) { a_lo = a_lo < first ? a_lo : first; a_hi = a_hi > last + 1 ? a_hi : last + 1; }
-    a_lo = a_lo < 0 ? 0 : a_lo; a_hi = a_hi > SW ? SW : a_hi;
-    if (!live) { a_lo = SW; a_hi = 0; }
-    Cand *list = sc.cand + (size_t)local * CAND_MAX * SW;
-    int *counts = sc.cand_count + (size_t)local * SW;
-    const int packed_sectors = (s0 & 0xFFFF) | (s1 << 16);
-    const int packed_vertices = (int)(((unsigned)m->wall_vertex[2 * w] & 0xFFFFu) | ((unsigned)m->wall_vertex[2 * w + 1] << 16));
-    const bool masked_side = !os && m->side_tex[(w * 2 + (ff ? 0 : 1)) * 3] >= 0;
-    const int packed_span = r.flags | (os ? 0x200 : 0) | (masked_side ? 0x400 : 0);   // bits 9 and 10 of the flags are free
-    const int rec_pl = r.pl, rec_pr = r.pr;
-    // Most linedefs cover a few columns only, so several of them share a turn: eight with eight lanes each, then
-    // four with sixteen, then two with thirty-two; a wider one has the wavefront to itself.
-    auto note_masked = [&](int wall, int x, const Eval &e) {
-        atomicMin(&sc.masked_hit[(size_t)local * SW + x], ((u64)__float_as_uint(e.dist) << 32) | ((u64)wall << 16) | (u64)e.flags);
-    };
-    const bool listed = a_lo < a_hi;
-    const bool narrow = listed && (a_hi - a_lo <= 32);
-    auto shared_turns = [&](bool member, int lanes_each) {
-        const int group = slot_in_wave / lanes_each, group_lane = slot_in_wave - group * lanes_each;
-        const int groups = 64 / lanes_each;
-        for (u64 pending = __ballot(member); pending;) {
-            int owner = -1;
+            const float den = rx * q.segy - ry * q.segx;
+            ok = fabsf(den) >= 1e-6f;
+            const float safe = ok ? den : 1.0f;
+            d = q.numer / safe;
+            const float along = (q.offx * ry - q.offy * rx) / safe;
+            along_high = along > 0.5f;
+            return ok && (d > 0) && (along >= 0) && (along <= 1);
+        };
 #pragma unroll
-            for (int g = 0; g < 8; ++g) {
-                if (g >= groups) break;                  // the same in every lane
-                const int next = pending ? __ffsll((long long)pending) - 1 : -1;
-                pending &= pending - 1;
-                if (group == g) owner = next;
+        for (int k = 0; k < 3; ++k) {
+            const int lanes_each = 8 << k, groups = 64 / lanes_each;
+            const int group = slot / lanes_each, group_lane = slot - group * lanes_each;
+            for (int turn = 0; turn < members[k]; turn += groups) {
+                const bool taken = turn + group < members[k];
+                const int owner = by_width[wave][k][taken ? turn + group : turn];
+                const SetupWall q = walls_lds[wave][owner];
+                const int x = (q.window & 0xFFFF) + group_lane;
+                const bool inside = taken && x < (q.window >> 16);
+                bool ok, along_high; float d;
+                const bool g = look(q, x, ok, along_high, d) && inside;
+                // the nearest blocking linedef each column ray hits, lowest slot on ties, hides billboards
+                if (g && q.blocking >= 0) atomicMin(&block_hits[x], ((u64)__float_as_uint(d) << 32) | (u64)(unsigned)q.blocking);
+                const unsigned int hits = (unsigned int)(__ballot(g) >> (group * lanes_each)) & (lanes_each == 32 ? ~0u : (1u << lanes_each) - 1u);
+                const bool any = hits != 0;
+                const int first = any ? x - group_lane + __ffs((int)hits) - 1 : 0, last = any ? x - group_lane + 31 - __clz((int)hits) : SW - 1;
+                if (group_lane == 0 && taken && any) hits_lds[wave][owner] = first | ((last + 1) << 16);
+                if (inside) enter(q, x, ok, g, along_high, d, setup_owned(q.facts, q.ends, any, first, last));
             }
-            const int source = owner < 0 ? 0 : owner;
-            float4 b_wl;
-            b_wl.x = __shfl(wl.x, source); b_wl.y = __shfl(wl.y, source); b_wl.z = __shfl(wl.z, source); b_wl.w = __shfl(wl.w, source);
-            const int b_span = __shfl(packed_span, source), b_pl = __shfl(rec_pl, source), b_pr = __shfl(rec_pr, source);
-            const int b_sectors = __shfl(packed_sectors, source), b_vertices = __shfl(packed_vertices, source);
-            const int b_lo = __shfl(a_lo, source), b_hi = __shfl(a_hi, source);
-            const int b_wall = __shfl(w, source);
-            const int x = b_lo + group_lane;
-            if (owner < 0 || x >= b_hi) continue;
-            float rx, ry; ray_direction(c, x, &rx, &ry);
-            const Eval e = eval_segment(b_wl, b_span, b_pl, b_pr, (b_span & 0x200) != 0, c, x, rx, ry);
-            if (!finitef(e.dist)) continue;
-            if ((b_span & 0x400) && (e.flags & CF_PROJ)) note_masked(b_wall, x, e);
-            const int slot = atomicAdd(&counts[x], 1);
-            if (slot < CAND_MAX) {
-                Cand entry;
-                entry.wall = (unsigned short)b_wall;
-                entry.s0 = (short)(b_sectors & 0xFFFF); entry.s1 = (short)(b_sectors >> 16);
-                entry.v0 = (unsigned short)(b_vertices & 0xFFFF); entry.v1 = (unsigned short)((unsigned)b_vertices >> 16);
-                entry.flags = (unsigned short)e.flags;
-                entry.dist = e.dist;
-                list[(size_t)slot * SW + x] = entry;
-            }   // else: the count says so, and the column is listed afresh in the spill pool (strip_key_kernel, cand_spill_kernel)
         }
-    };
-    shared_turns(listed && (a_hi - a_lo <= 8), 8);
-    shared_turns(listed && (a_hi - a_lo > 8) && (a_hi - a_lo <= 16), 16);
-    shared_turns(listed && (a_hi - a_lo > 16) && (a_hi - a_lo <= 32), 32);
-    for (u64 pending = __ballot(listed && !narrow); pending; pending &= pending - 1) {
-        const int owner = __ffsll((long long)pending) - 1;
-        float4 b_wl;
-        b_wl.x = bcast(wl.x, owner); b_wl.y = bcast(wl.y, owner); b_wl.z = bcast(wl.z, owner); b_wl.w = bcast(wl.w, owner);
-        const int b_span = bcast(packed_span, owner), b_pl = bcast(rec_pl, owner), b_pr = bcast(rec_pr, owner);
-        const int b_sectors = bcast(packed_sectors, owner), b_vertices = bcast(packed_vertices, owner);
-        const int b_lo = bcast(a_lo, owner), b_hi = bcast(a_hi, owner);
-        Cand entry;
-        entry.wall = (unsigned short)bcast(w, owner);
-        entry.s0 = (short)(b_sectors & 0xFFFF); entry.s1 = (short)(b_sectors >> 16);
-        entry.v0 = (unsigned short)(b_vertices & 0xFFFF); entry.v1 = (unsigned short)((unsigned)b_vertices >> 16);
-        for (int x = b_lo + slot_in_wave; x < b_hi; x += 64) {
-            float rx, ry; ray_direction(c, x, &rx, &ry);
-            Eval e = eval_segment(b_wl, b_span, b_pl, b_pr, (b_span & 0x200) != 0, c, x, rx, ry);
-            if (finitef(e.dist)) {
-                if ((b_span & 0x400) && (e.flags & CF_PROJ)) note_masked(entry.wall, x, e);
-                int slot = atomicAdd(&counts[x], 1);
-                if (slot < CAND_MAX) {
-                    entry.flags = (unsigned short)e.flags;
-                    entry.dist = e.dist;
-                    list[(size_t)slot * SW + x] = entry;
+        for (u64 pending = __ballot(width > 32); pending; pending &= pending - 1) {
+            const int owner = __ffsll((long long)pending) - 1;
+            const SetupWall q = walls_lds[wave][owner];
+            const int from = q.window & 0xFFFF, to = q.window >> 16;
+            int first = 0, last = SW - 1; bool any = false;
+            for (int x = from + slot; x - slot < to; x += 64) {
+                bool ok, along_high; float d;
+                const bool g = look(q, x, ok, along_high, d) && x < to;
+                if (g && q.blocking >= 0) atomicMin(&block_hits[x], ((u64)__float_as_uint(d) << 32) | (u64)(unsigned)q.blocking);
+                const u64 hits = __ballot(g);
+                if (slot == 0) wide_hits[wave][(x - from) / 64] = hits;
+                if (hits) {
+                    if (!any) first = x - slot + __ffsll((long long)hits) - 1;
+                    last = x - slot + 63 - __clzll((long long)hits);
+                    any = true;
                 }
+                if (x < to) wide_lds[wave][x] = !(ok && d > 0) ? 0.0f : (along_high ? -d : d);
             }
+            if (slot == 0 && any) hits_lds[wave][owner] = first | ((last + 1) << 16);
+            const int owned = setup_owned(q.facts, q.ends, any, first, last);
+            wave_lds_fence();
+            for (int x = from + slot; x < to; x += 64) {
+                const float d = wide_lds[wave][x];
+                enter(q, x, true, (wide_hits[wave][(x - from) / 64] >> slot) & 1, d < 0.0f, fabsf(d), owned);
+            }
+            wave_lds_fence();
         }
+        wave_lds_fence();
+        if (live) {
+            const int hits = hits_lds[wave][slot];
+            const bool any = (hits >> 16) != 0;
+            const int owned = setup_owned(facts, ends, any, any ? hits & 0xFFFF : 0, any ? (hits >> 16) - 1 : SW - 1);
+            RecSpan shown;
+            shown.pl = (short)(owned & 0xFFFF); shown.pr = (short)((owned >> 16) & 0x7FFF);
+            shown.flags = (facts & ~(SETUP_ONE_SIDED | SETUP_MASKED | SETUP_SPANS)) | (owned < 0 ? WF_HC : 0) | (any ? WF_ANYGEO : 0);
+            r.pl = shown.pl; r.pr = shown.pr; r.flags = shown.flags;
+            sc.rec[(size_t)local * m->wall_count + w] = r;
+            sc.span[(size_t)local * m->wall_count + w] = shown;
+        }
+        wave_lds_fence();                                // the next share takes the LDS over
+    }
+    }
+    if (!WHOLE) return;
+    __syncthreads();
+    for (int x = threadIdx.x; x < SW; x += THREADS) {
+        const size_t at = (size_t)local * SW + x;
+        sc.block_hit[at] = block_lds[x]; sc.masked_hit[at] = masked_lds[x]; sc.cand_count[at] = count_lds[x];
     }
 }
 
@@ -1220,13 +1226,6 @@ __device__ __forceinline__ int cell_sector(const DeviceMap &dm, bool is_floor, i
         if ((item.x & GRID_ALWAYS_INSIDE) || inside_edge_copies(dm.cell_edge, item.z, item.w, px, py)) found = s;
     }
     return found;
-}
-
-// Lanes of one wavefront leave words in LDS for one another: the order is the program's, the compiler has to keep it.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // One pixel's flat ray, tested by PROBE_LANES lanes of a wavefront (a wavefront takes four pixels, of any lanes): the sector of the
@@ -5644,7 +5643,8 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     mark();
     hipLaunchKernelGGL(lane_setup_kernel, dim3((count + 63) / 64), dim3(64), 0, stream, r->dm, *lanes, base, count, sc);
     hipLaunchKernelGGL(lane_tables_kernel, dim3(count), dim3(256), 0, stream, r->dm, *lanes, base, count, sc);
-    hipLaunchKernelGGL(wall_setup_kernel, dim3((m.wall_count + SETUP_WALLS - 1) / SETUP_WALLS, count), dim3(SETUP_WALLS), 0, stream, r->dm, count, sc);
+    if (setup_whole_lanes(count, m.wall_count)) hipLaunchKernelGGL(wall_setup_kernel<true>, dim3(1, count), dim3(SETUP_WHOLE_THREADS), 0, stream, r->dm, count, sc);
+    else hipLaunchKernelGGL(wall_setup_kernel<false>, dim3((m.wall_count + SETUP_THREADS - 1) / SETUP_THREADS, count), dim3(SETUP_THREADS), 0, stream, r->dm, count, sc);
     if (m.split_count > 0)
         hipLaunchKernelGGL(fragment_setup_kernel, dim3((m.split_count * m.fragment_slots + 63) / 64, count), dim3(64), 0, stream, r->dm, count, sc);
     hipLaunchKernelGGL(strip_key_kernel, dim3((count * (SW / 64) + 3) / 4), dim3(256), 0, stream, count, sc);
