@@ -291,6 +291,7 @@ struct Scratch {    // per-chunk working memory, sized at create
     unsigned char *frame;  // [L,240,320] when the caller wants no indexed output
     u64 *block_hit;        // [L,320] nearest blocking linedef of the column ray: float bits of the distance << 32 |
                            // slot in blocking_walls, all ones when no ray hits (engine.py:10534-10557)
+    int *sprite_listed;    // [L] the lane's billboards that reach the view at all (sprite_list_kernel)
     int *lane_blends;      // [L] does some live billboard of the lane blend with the pixel below it (sprite_style other than -1)?
                            // lane_tables_kernel says; launch_chunk's two billboard launches split the lanes by it
     unsigned char *strip_key;  // [L*SEGS_PER_LANE] expected traversal length of each (lane, segment of SEG_COLS columns)
@@ -4202,25 +4203,73 @@ __device__ __forceinline__ void sprite_column(const DeviceMap &dm, const gd_lane
     }
 }
 
-// A thread a view pixel.  A work-group takes SPRITE_COLUMNS columns of a lane and 1 / gridDim.z of its rows: it lists the
-// billboards that reach them, orders the list near to far, and notes as bit sets over that order which entries show in each
+// The billboards of a lane that reach the view, for all the work-groups that paint its columns: their records in no order, and their
+// places and reach near to far, equal depths by slot.  They lie where the lane's candidate lists were, which nothing reads once every
+// strip is selected.
+#define SPRITE_SLOTS_MAX 512
+struct __align__(8) SpriteHead {
+    short x0, x1;            // columns and rows of the view it can reach
+    unsigned char y0, y1;
+    unsigned short record;
+};
+static_assert(SPRITE_SLOTS_MAX * (sizeof(SpriteRec) + sizeof(SpriteHead)) <= CAND_MAX * SW * sizeof(Cand), "sprite lists: room in a lane's candidate lists");
+__device__ __forceinline__ SpriteRec *sprite_records(const Scratch &sc, int local) { return reinterpret_cast<SpriteRec *>(sc.cand + (size_t)local * CAND_MAX * SW); }
+__device__ __forceinline__ SpriteHead *sprite_heads(const Scratch &sc, int local) { return reinterpret_cast<SpriteHead *>(sprite_records(sc, local) + SPRITE_SLOTS_MAX); }
+
+// One work-group per lane.  It runs beside the drawing of the walls: the work-groups that paint 64 columns each used to work out the records
+// of all slots, five times a lane, and to order their own lists, which was what they were bound by.  0.05 ms for 4096 lanes with 128 slots,
+// hidden behind wall_geometry_kernel and wall_raster_kernel.
+#define LIST_THREADS 128
+__global__ void __launch_bounds__(LIST_THREADS) sprite_list_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
+    __shared__ float depth_of[SPRITE_SLOTS_MAX];
+    __shared__ unsigned short slot_of[SPRITE_SLOTS_MAX];
+    __shared__ SpriteHead head_of[SPRITE_SLOTS_MAX];
+    __shared__ int listed_count;
+    const int local = blockIdx.x;
+    if (local >= lane_count) return;
+    if (threadIdx.x == 0) listed_count = 0;
+    __syncthreads();
+    const LaneCtx &L = sc.ctx[local];
+    SpriteRec *records = sprite_records(sc, local);
+    for (int a = threadIdx.x; a < lanes.sprite_slots; a += LIST_THREADS) {
+        SpriteRec s;
+        if (!sprite_record(dm, lanes, lane_base + local, L, a, 0, SW, 0, VH, s)) continue;
+        const int at = atomicAdd(&listed_count, 1);
+        records[at] = s;
+        depth_of[at] = s.depth; slot_of[at] = (unsigned short)a;
+        SpriteHead h;
+        h.x0 = (short)clampi(s.left, 0, SW); h.x1 = (short)clampi(s.right, 0, SW);
+        h.y0 = (unsigned char)((unsigned)s.flags >> 16); h.y1 = (unsigned char)((unsigned)s.flags >> 24);
+        h.record = (unsigned short)at;
+        head_of[at] = h;
+    }
+    __syncthreads();
+    const int listed = listed_count;
+    if (threadIdx.x == 0) sc.sprite_listed[local] = listed;
+    SpriteHead *heads = sprite_heads(sc, local);
+    for (int i = threadIdx.x; i < listed; i += LIST_THREADS) {   // an entry's place is the number of entries before it
+        const float depth = depth_of[i]; const int slot = slot_of[i];
+        int before = 0;
+        for (int j = 0; j < listed; ++j) before += depth_of[j] < depth || (depth_of[j] == depth && slot_of[j] < slot);
+        heads[before] = head_of[i];
+    }
+}
+
+// A thread a view pixel.  A work-group takes SPRITE_COLUMNS columns of a lane and 1 / gridDim.z of its rows: it picks the billboards that
+// reach them from the lane's list, near to far, and notes as bit sets over that order which entries show in each
 // column and which have a source row in each row; a pixel then walks the entries in both sets and stops at the first that is
 // visible and opaque there (in a lane with billboards that blend it then goes back over those it passed).  What clips
 // billboards at the pixel is read once, not once per billboard: on the 4000-linedef map most of what a column ray passes is behind
 // walls, and a column's thread used to read word, linedef and patch for every row of every one of them (and the flat ray's
 // decision, which does not depend on the billboard, each time as well), waiting for one before the next.
 // A list longer than SPRITE_CHUNK, one word of bits, is painted in chunks of that many, the farthest first: the LDS a group
-// needs (13 KB) does not follow the slots a lane has.
-// Bound by the listing (six 64-bit divisions a billboard in front of the camera, in every work-group), then by the waits of
-// pixels that show something.  4096 lanes with 128 billboards, beside the flat pass: 2.71 ms a column and quarter of its rows a
-// thread, 1.38 a pixel a thread with tiles dealt out beforehand, 0.70 with tiles taken when a wavefront is free; 2048 lanes with an
-// engine's 512 slots 0.62 -> 0.35, 512 lanes 0.33 -> 0.18, 256 lanes with 32 billboards 0.086 -> 0.071.
+// needs does not follow the slots a lane has.
+// Bound by the waits of pixels that show something.
 #define SPRITE_THREADS 256
 #define SPRITE_TILE_W 16      // columns of a wavefront's tile: 8 to 64 within 3 %
 #define SPRITE_TILE_H (64 / SPRITE_TILE_W)
 #define SPRITE_TILES 4        // tiles of a wavefront whose words are asked for together
 #define SPRITE_CHUNK 64
-#define SPRITE_SLOTS_MAX 512
 #define SPRITE_COLUMNS 64     // a work-group for the whole lane: 0.95 ms instead of 0.70 (4 wavefronts), 0.86 (8)
 #define SPRITE_ROW_PARTS 4    // of a small batch's work-groups
 // Lanes from which a work-group takes all rows of its columns: fewer listings, but the last work-groups last longer.  Quarters and whole
@@ -4235,9 +4284,8 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(Device
                                                                           unsigned char *frame_base, size_t frame_stride, int lane_pick) {
     __shared__ SpriteRec sp[SPRITE_CHUNK];         // the chunk's records, near to far
     __shared__ u64 cover[SPRITE_COLUMNS], in_row[VH];
-    __shared__ float depth_of[SPRITE_SLOTS_MAX];   // the whole list, in no order
-    __shared__ unsigned short slot_of[SPRITE_SLOTS_MAX], by_rank[SPRITE_SLOTS_MAX];
-    __shared__ int listed_count, next_tile;
+    __shared__ unsigned short picked[SPRITE_SLOTS_MAX];   // the records of the billboards that reach the group's columns and rows, near to far
+    __shared__ int wave_picks[SPRITE_SLOTS_MAX / 64], next_tile;
     const int local = blockIdx.y;
     if (local >= lane_count) return;
     // lane_pick: LANES_ALL, or one half of launch_chunk's split: LANES_PLAIN (lanes whose billboards all simply cover what is
@@ -4249,44 +4297,54 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(Device
     const int n = lane_base + local, tid = threadIdx.x;
     const int rows = VH / gridDim.z;
     const int x_first = blockIdx.x * SPRITE_COLUMNS, row_first = blockIdx.z * rows;
-    if (tid == 0) listed_count = 0;
-    __syncthreads();
     const LaneCtx &L = sc.ctx[local];
-    for (int a = tid; a < lanes.sprite_slots; a += SPRITE_THREADS) {
-        SpriteRec s;
-        if (!sprite_record(dm, lanes, n, L, a, x_first, x_first + SPRITE_COLUMNS, row_first, row_first + rows, s)) continue;
-        const int at = atomicAdd(&listed_count, 1);
-        depth_of[at] = s.depth; slot_of[at] = (unsigned short)a;
-        if (at < SPRITE_CHUNK) sp[at] = s;
-    }
-    __syncthreads();
-    const int listed = listed_count;
-    if (listed == 0) return;                       // the same in the whole block
-    // near to far, equal depths by slot: an entry's place is the number of entries before it
-    for (int i = tid; i < listed; i += SPRITE_THREADS) {
-        const float depth = depth_of[i]; const int slot = slot_of[i];
-        int before = 0;
-        for (int j = 0; j < listed; ++j) before += depth_of[j] < depth || (depth_of[j] == depth && slot_of[j] < slot);
-        by_rank[before] = (unsigned short)(listed <= SPRITE_CHUNK ? i : slot);
-    }
-    __syncthreads();
-    unsigned int *meta = sc.meta + (size_t)local * VH * SW;
-    unsigned char *frame = frame_base + (size_t)local * frame_stride;
     const int lane_id = tid & 63, wave = tid >> 6;
     constexpr int WAVES = SPRITE_THREADS / 64;
+    const int on_view = sc.sprite_listed[local];
+    if (on_view == 0) return;                      // the same in the whole block
+    const SpriteHead *heads = sprite_heads(sc, local);
+    u64 picks[SPRITE_SLOTS_MAX / SPRITE_THREADS]; unsigned short record[SPRITE_SLOTS_MAX / SPRITE_THREADS];
+#pragma unroll
+    for (int k = 0; k < SPRITE_SLOTS_MAX / SPRITE_THREADS; ++k) {   // 64 entries a wavefront and turn
+        const int i = k * SPRITE_THREADS + tid;
+        picks[k] = 0; record[k] = 0;
+        if (k * SPRITE_THREADS >= on_view) continue;                // the same in the whole block
+        bool pick = false;
+        if (i < on_view) {
+            const SpriteHead head = heads[i];
+            pick = head.x1 > x_first && head.x0 < x_first + SPRITE_COLUMNS && head.y1 > row_first && head.y0 < row_first + rows;
+            record[k] = head.record;
+        }
+        picks[k] = __ballot(pick);
+        if (lane_id == 0) wave_picks[k * WAVES + wave] = __popcll(picks[k]);
+    }
+    __syncthreads();
+    int listed = 0;
+#pragma unroll
+    for (int k = 0; k < SPRITE_SLOTS_MAX / SPRITE_THREADS; ++k) {
+        if (k * SPRITE_THREADS >= on_view) continue;
+        int before = listed;
+#pragma unroll
+        for (int q = 0; q < WAVES; ++q) { before += q < wave ? wave_picks[k * WAVES + q] : 0; listed += wave_picks[k * WAVES + q]; }
+        if ((picks[k] >> lane_id) & 1) picked[before + __popcll(picks[k] & ((1ULL << lane_id) - 1))] = record[k];
+    }
+    if (listed == 0) return;                       // the same in the whole block
+    __syncthreads();
+    const unsigned int *records = reinterpret_cast<const unsigned int *>(sprite_records(sc, local));
+    unsigned int *meta = sc.meta + (size_t)local * VH * SW;
+    unsigned char *frame = frame_base + (size_t)local * frame_stride;
     constexpr int TILES_ACROSS = SPRITE_COLUMNS / SPRITE_TILE_W;
     const int tiles = TILES_ACROSS * (rows / SPRITE_TILE_H);
     const int tile_x = lane_id % SPRITE_TILE_W, tile_y = lane_id / SPRITE_TILE_W;
     for (int first = (listed - 1) / SPRITE_CHUNK * SPRITE_CHUNK; first >= 0; first -= SPRITE_CHUNK) {
         const int length = listed - first < SPRITE_CHUNK ? listed - first : SPRITE_CHUNK;
         {   // the chunk's records into their places
-            SpriteRec s;
-            if (tid < length) {
-                if (listed <= SPRITE_CHUNK) s = sp[by_rank[tid]];
-                else (void)sprite_record(dm, lanes, n, L, by_rank[first + tid], x_first, x_first + SPRITE_COLUMNS, row_first, row_first + rows, s);
+            constexpr int WORDS = sizeof(SpriteRec) / 4;
+            if (first + SPRITE_CHUNK < listed) __syncthreads();   // every pixel of the chunk before is painted: its records and bit sets are free
+            for (int k = tid; k < length * WORDS; k += SPRITE_THREADS) {
+                const int entry = k / WORDS;
+                reinterpret_cast<unsigned int *>(sp)[k] = records[picked[first + entry] * WORDS + (k - entry * WORDS)];
             }
-            __syncthreads();                       // every pixel of the chunk before is painted: its records and bit sets are free
-            if (tid < length) sp[tid] = s;
             if (tid < SPRITE_COLUMNS) cover[tid] = 0;
             if (tid == 0) next_tile = 0;
             __syncthreads();
@@ -5468,6 +5526,7 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.row_slope, L * (size_t)VH);
     take(&sc.step_scale, L * STEP_TABLE);
     take(&sc.block_hit, L * SW);
+    take(&sc.sprite_listed, L);
     take(&sc.lane_blends, L);
     take(&sc.strip_key, L * SEGS_PER_LANE);
     take(&sc.strip_order, L * SEGS_PER_LANE);
@@ -5640,6 +5699,8 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         frame_base = out->indexed ? out->indexed + (size_t)base * frame_stride : sc.frame;
         if (!frame_base) return fail(GD_E_ARG, "assembling the frame kernel by kernel needs an indexed output");
     }
+    const bool has_billboards = lanes->sprite_slots > 0 && lanes->sprite_x;
+    auto list_billboards = [&](hipStream_t on) { hipLaunchKernelGGL(sprite_list_kernel, dim3(count), dim3(LIST_THREADS), 0, on, r->dm, *lanes, base, count, sc); };
     mark();
     hipLaunchKernelGGL(lane_setup_kernel, dim3((count + 63) / 64), dim3(64), 0, stream, r->dm, *lanes, base, count, sc);
     hipLaunchKernelGGL(lane_tables_kernel, dim3(count), dim3(256), 0, stream, r->dm, *lanes, base, count, sc);
@@ -5674,6 +5735,14 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
             HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
         } else {
             hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0, 0);
+        }
+        // the billboards' lists beside the walls' drawing, on the side stream (when stages are being timed, with the billboards)
+        if (has_billboards && !fused && !timed) {
+            if (r->side_ready) {
+                HIP_TRY(hipEventRecord(r->fork_event, stream));
+                HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
+            }
+            list_billboards(r->side_ready ? r->side_stream : stream);
         }
         mark();
         hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(count), dim3(SW), 0, stream, r->dm, count, sc);
@@ -5721,7 +5790,6 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     // flat chain, which waits for memory most of its time, then has the billboards beside it as well as the shading.  Lanes
     // with a billboard that blends with the pixel below (sprite_style) keep the order flat pass, then billboards; so do
     // frames with decals, which go between the two.
-    const bool has_billboards = lanes->sprite_slots > 0 && lanes->sprite_x;
     const bool billboards_split = beside && has_billboards && !decals;
     const bool may_blend = lanes->sprite_style != nullptr;   // without styles no lane blends: the launches for such lanes are left out
     auto paint_billboards = [&](hipStream_t on, int lane_pick) {
@@ -5760,6 +5828,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     }
     if (decals)
         hipLaunchKernelGGL(decal_kernel, dim3(count), dim3(SW), 0, stream, r->dm, r->overlays, *lanes, base, count, sc, frame_base, frame_stride);
+    if (has_billboards && timed) list_billboards(stream);
     if (has_billboards && !(billboards_split && !may_blend)) paint_billboards(stream, billboards_split ? LANES_BLENDING : LANES_ALL);
     if (lanes->weapon_state && r->overlays.d.weapon_patch_count > 0)
         hipLaunchKernelGGL(weapon_overlay_kernel, dim3(WEAPON_PARTS, count), dim3(WEAPON_THREADS), 0, stream, r->overlays, lanes->weapon_state, base, count,
