@@ -229,6 +229,7 @@ struct DeviceMap {  // device copy of gd_map_desc (device pointers) + fixed tabl
                                          // index << 8 (or -1 when not recorded), first edge, one past the last
     const float4 *cell_edge;             // [item edges] x1, y1, x2, y2
     const WallSide *wall_side;           // [W,2]
+    const unsigned int *sprite_texels;   // [patches, spr_max_h, spr_max_w] texel | its post's first row << 8 | opaque << 16: one load instead of three
     const int *masked_slot;              // [W] number of the linedef among those with a mid-texture on a two-sided side, else -1
     int masked_count;                    // how many there are
     const int *wall_facts;               // [W] WALL_*, and from bit WALL_BLOCKING_SHIFT on the linedef's position in blocking_walls plus one, 0 when it does not block
@@ -1156,29 +1157,6 @@ __device__ bool flat_level_hit(const DeviceMap &dm, bool is_floor, float level, 
     return false;
 }
 //
-// Does the flat ray of one pixel resolve at all, i.e. does the probe point of some plane level lie in a
-// sector of that level (engine.py:10981-11024)?  `plane` is the sector whose plane the wall pass shows at the
-// pixel: its own level nearly always answers yes at once.
-__device__ bool flat_ray_resolves(const DeviceMap &dm, const LaneCtx &c, float rc, float rs, float cc, int y, int plane) {
-    const gd_map_desc *m = &dm.d;
-    const float delta = (float)y - flat_center(c);
-    const bool is_floor = delta > 0;
-    const float denom = fmaxf(fabsf(delta), 0.5f);
-    const float *levels = is_floor ? m->floor_levels : m->ceil_levels;
-    const int level_count = is_floor ? m->floor_level_count : m->ceil_level_count;
-    const float own = m->sector_heights[2 * plane + (is_floor ? 0 : 1)];
-    for (int k = -1; k < level_count; ++k) {
-        const float level = k < 0 ? own : levels[k];
-        if (k >= 0 && level == own) continue;
-        const float height = is_floor ? (c.view_z - level) : (level - c.view_z);
-        if (!(height > 0)) continue;
-        const float cd = (height * 192.0f / denom) / cc;
-        if (!(finitef(cd) && cd > 0)) continue;
-        if (flat_level_hit(dm, is_floor, level, c.x + rc * cd, c.y + rs * cd)) return true;
-    }
-    return false;
-}
-//
 // The plane levels of one half of the screen (floors or ceilings) as one lane sees them.
 struct LevelSide {
     const float *level, *reach, *far;   // plane height, and the bounds of the distance to the sectors of that level
@@ -1227,6 +1205,51 @@ __device__ __forceinline__ int cell_sector(const DeviceMap &dm, bool is_floor, i
         if ((item.x & GRID_ALWAYS_INSIDE) || inside_edge_copies(dm.cell_edge, item.z, item.w, px, py)) found = s;
     }
     return found;
+}
+
+// Does the flat ray of one pixel resolve at all, i.e. does the probe point of some plane level lie in a
+// sector of that level (engine.py:10981-11024)?  `plane` is the sector whose plane the wall pass shows at the
+// pixel: its own level nearly always answers yes at once.  Where it does not, the levels that the pixel's bucket names are asked, and
+// of those only the ones whose probe point meets the box around their sectors are looked up (with all 400 levels of a half looked up,
+// one after the other, sprite_pixels_kernel took 0.51 ms for 4096 lanes, now 0.39).
+__device__ bool flat_ray_resolves(const DeviceMap &dm, const Scratch &sc, int local, const LaneCtx &c, float rc, float rs, float cc, int y, int plane) {
+    const gd_map_desc *m = &dm.d;
+    const float delta = (float)y - flat_center(c);
+    const bool is_floor = delta > 0;
+    const float denom = fmaxf(fabsf(delta), 0.5f);
+    const LevelSide side = level_side(dm, sc, local, is_floor);
+    const float own = m->sector_heights[2 * plane + (is_floor ? 0 : 1)];
+    const unsigned int *row = side.masks + level_bucket((192.0f / denom) / cc) * side.mask_words;
+    const int end = side.first + side.count;
+    int base = (side.first & ~31) - 32;
+    unsigned int bits = 0u;
+    for (bool first = true;; first = false) {       // one copy of the test: the own level, then the named ones
+        float level = own;
+        float4 box = make_float4(-GD_INF, -GD_INF, GD_INF, GD_INF);
+        if (!first) {
+            while (bits == 0u) {
+                base += 32;
+                if (base >= end) return false;
+                bits = side.mask_words > 0 ? row[base >> 5] : ~0u;
+                if (base < side.first) bits &= ~0u << (side.first - base);
+                if (base + 32 > end) bits &= (1u << (end - base)) - 1u;
+            }
+            // the pixels of a wavefront name much the same levels: those that name the first one's next take it together
+            const int at = __builtin_amdgcn_readfirstlane(base + __ffs((int)bits) - 1);
+            const unsigned int bit = (at & ~31) == base ? 1u << (at & 31) : 0u;
+            if (!(bits & bit)) continue;
+            bits &= ~bit;
+            level = at < m->floor_level_count ? m->floor_levels[at] : m->ceil_levels[at - m->floor_level_count];
+            box = dm.level_box[at];
+            if (level == own) continue;
+        }
+        const float height = is_floor ? (c.view_z - level) : (level - c.view_z);
+        const float cd = (height * 192.0f / denom) / cc;
+        const float px = c.x + rc * cd, py = c.y + rs * cd;
+        if (!(height > 0 && finitef(cd) && cd > 0)) continue;
+        if (!first && !(px >= box.x && px <= box.z && py >= box.y && py <= box.w)) continue;
+        if (flat_level_hit(dm, is_floor, level, px, py)) return true;
+    }
 }
 
 // One pixel's flat ray, tested by PROBE_LANES lanes of a wavefront (a wavefront takes four pixels, of any lanes): the sector of the
@@ -4187,7 +4210,7 @@ __device__ __forceinline__ void sprite_column(const DeviceMap &dm, const gd_lane
                     live[j] = s.depth < GD_INF;   // no clip linedef: the clip depth is infinite
                     // only a billboard standing behind the plane needs to know whether the flat ray resolves
                     if (live[j] && clip.plane >= 0 && !(s.depth < clip.plane_depth))
-                        live[j] = flat_ray_resolves(dm, L, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x],
+                        live[j] = flat_ray_resolves(dm, sc, local, L, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x],
                                                     dm.cosine_correction[x], yb + j, clip.plane);
                 }
             }
@@ -4264,7 +4287,8 @@ __global__ void __launch_bounds__(LIST_THREADS) sprite_list_kernel(DeviceMap dm,
 // decision, which does not depend on the billboard, each time as well), waiting for one before the next.
 // A list longer than SPRITE_CHUNK, one word of bits, is painted in chunks of that many, the farthest first: the LDS a group
 // needs does not follow the slots a lane has.
-// Bound by the waits of pixels that show something.
+// Bound by the waits of pixels that show something: their clip, their texels (one word: three bytes each cost 3 % more), and the flat ray.
+// Five wavefronts a SIMD (seven registers spilled) are better than four by 4 %, six worse by 25 %.
 #define SPRITE_THREADS 256
 #define SPRITE_TILE_W 16      // columns of a wavefront's tile: 8 to 64 within 3 %
 #define SPRITE_TILE_H (64 / SPRITE_TILE_W)
@@ -4280,7 +4304,7 @@ __global__ void __launch_bounds__(LIST_THREADS) sprite_list_kernel(DeviceMap dm,
 #define SPRITE_TALL_LANES 512
 static_assert(SPRITE_COLUMNS == 64 && SW % SPRITE_COLUMNS == 0 && VH % (SPRITE_ROW_PARTS * SPRITE_TILE_H) == 0 && VH <= SPRITE_THREADS, "sprite_pixels_kernel: whole tiles");
 static_assert(SPRITE_CHUNK == 64 && SPRITE_CHUNK <= SPRITE_THREADS, "sprite_pixels_kernel: a bit an entry");
-__global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
+__global__ void __launch_bounds__(SPRITE_THREADS, 5) sprite_pixels_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
                                                                           unsigned char *frame_base, size_t frame_stride, int lane_pick) {
     __shared__ SpriteRec sp[SPRITE_CHUNK];         // the chunk's records, near to far
     __shared__ u64 cover[SPRITE_COLUMNS], in_row[VH];
@@ -4404,10 +4428,9 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(Device
                 // its colour at the pixel after the colormap, -1 where the patch has none
                 auto colour = [&](const SpriteRec &s) -> int {
                     const i64 su = mul64((i64)x - s.left, s.hstep) >> 16, sv = (s.fraction_base + mul64((i64)y, s.iscale)) >> 16;
-                    const size_t at = s.texel_base + (size_t)sv * m->spr_max_w + su;
-                    const unsigned char opaque = m->spr_opaque[at], post_top = m->spr_post_top[at], texel = m->spr_atlas[at];
-                    if (!opaque || (i64)y < ((s.top_fixed + mul64(s.yscale, post_top)) >> 16)) return -1;
-                    return m->colormap[(s.flags & 31) * 256 + texel];
+                    const unsigned int texel = dm.sprite_texels[s.texel_base + (size_t)sv * m->spr_max_w + su];
+                    if (!(texel >> 16) || (i64)y < ((s.top_fixed + mul64(s.yscale, (texel >> 8) & 255u)) >> 16)) return -1;
+                    return m->colormap[(s.flags & 31) * 256 + (texel & 255u)];
                 };
                 u64 bits = entries[j], blended = 0;
                 bool undecided;
@@ -4426,7 +4449,7 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 4) sprite_pixels_kernel(Device
                     }
                     // a pixel that has to know whether its flat ray resolves leaves the walk for it, once: those that do ask together
                     if (undecided)
-                        resolves = flat_ray_resolves(dm, L, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x],
+                        resolves = flat_ray_resolves(dm, sc, local, L, lanes.ray_cos[(size_t)n * SW + x], lanes.ray_sin[(size_t)n * SW + x],
                                                      dm.cosine_correction[x], y, clip.plane) ? 1 : 0;
                 } while (undecided);
                 if (blended) {                         // from the opaque entry back to the eye
@@ -5925,6 +5948,11 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
     UP(playpal, 768); UP(colormap, 34 * 256);
     const size_t sprels = (size_t)h->sprite_count * h->spr_max_h * h->spr_max_w;
     UP(spr_atlas, sprels); UP(spr_opaque, sprels); UP(spr_post_top, sprels);
+    {
+        std::vector<unsigned int> words(sprels);
+        for (size_t k = 0; k < sprels; ++k) words[k] = (unsigned)h->spr_atlas[k] | ((unsigned)h->spr_post_top[k] << 8) | (h->spr_opaque[k] ? 1u << 16 : 0u);
+        if (rc == GD_OK) rc = upload(r, words.data(), words.size(), &r->dm.sprite_texels);
+    }
     UP(spr_w, h->sprite_count); UP(spr_h, h->sprite_count); UP(spr_left, h->sprite_count); UP(spr_top, h->sprite_count);
     UP(additive_luts, 2 * 256 * 256); UP(translucent_lut, 256 * 256);
 #undef UP
