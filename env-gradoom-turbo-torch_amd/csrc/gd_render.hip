@@ -9,7 +9,7 @@
 //                                             nearest blocking hit of every column (64-bit atomicMin)
 //   strip_key/order 1 thread / 64-col strip   longest strip first (counting sort on the blocking distance)
 //   wall_select     1 wave / strip            portal traversal: which drawseg every column pass selects, one record each
-//   wall_geometry   1 block / lane            the linedefs those passes draw, as lines over the columns: every division of the drawing
+//   wall_geometry   13 to 21 waves / lane            the linedefs those passes draw, as lines over the columns: every division of the drawing
 //   wall_raster     1 wave / strip            the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
 //   plane_shade     1 wave / 64 columns x 16 rows  flat texel + light for every pixel a plane of the wall pass shows,
 //                                             the wall tiers' palette indices
@@ -245,8 +245,7 @@ struct Scratch {    // per-chunk working memory, sized at create
     LaneCtx *ctx;          // [L]
     WallRec *rec;          // [L,W] written for the linedefs wall_setup_kernel does not cull; never read for the others
     RecSpan *span;         // [L,W] every linedef
-    WallGeo *geo;          // [L*W] the linedefs some column pass draws, those of a lane in a run of their own (wall_geometry_kernel)
-    int *geo_count;        // [1] how many there are (cleared by lane_setup_kernel)
+    WallGeo *geo;          // [L,W] the linedefs some column pass draws, a lane's from the start of its run on (wall_geometry_kernel)
     unsigned int *geo_slot;// [L,W] where in geo (written for those linedefs only)
     unsigned int *named;   // [L,(W+31)/32] a bit per linedef some column pass draws (cleared by lane_tables_kernel, set by wall_select_kernel)
     unsigned int *own_rows;// [L] bit k: strip k holds a pass with REC_OWN_ROWS (the same)
@@ -698,7 +697,7 @@ __global__ void lane_setup_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_ba
     sc.ctx[local] = c;
     int *span = sc.flat_span + (size_t)local * 4;
     span[0] = VH; span[1] = -1; span[2] = VH; span[3] = -1;
-    if (local == 0) { *sc.geo_count = 0; *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
+    if (local == 0) { *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
 }
 
 __device__ __forceinline__ void ray_direction(const LaneCtx &c, int x, float *rx, float *ry) {
@@ -3437,90 +3436,100 @@ __device__ __forceinline__ void wall_lines(const DeviceMap &dm, const LaneCtx &c
 
 // The linedefs that the recorded passes of a lane draw, each worked out once (WallGeo) for all the columns and passes that draw it.
 // The drawing half used to do this per column and pass: some 25 64-bit divisions, two thirds of its instructions, for what is
-// the same in every column of a linedef.  One work-group per lane: it turns the bits wall_select_kernel left into a list, takes as many
-// slots of geo, and gives four threads to a linedef (one a height; the wallscan light's four ends likewise).  4096 lanes on the
-// 4000-linedef map draw 1.3 million linedefs: 0.33 ms here, 0.3 ms off wall_raster_kernel.
-#define GEO_LIST 1024                            // linedefs listed at a time
+// the same in every column of a linedef.  `parts` (a power of two) work-groups of one wavefront a lane, none of which waits for another: each goes
+// over the bits wall_select_kernel left, takes every parts-th group of sixteen of the linedefs they name, and gives four threads to a
+// linedef (one a height; the wallscan light's four ends likewise).  Five more take a strip of columns each: masked mid-textures and the passes
+// with rows of their own.  4096 lanes on the 4000-linedef map draw 1.3 million linedefs: 0.34 ms by one work-group a lane, whose 320 threads
+// waited at barriers for the slowest, 0.29 by wavefronts that do strips after linedefs, 0.24 side by side in work-groups of four, 0.226 now;
+// 512 lanes 0.084 -> 0.045, 16 lanes of the 320-linedef map 0.012 -> 0.008.  It waits for records and heights, then for its stores.
+// Wavefronts a lane for linedefs, 4 / 8 / 16, in us: 16 lanes 13.6 / 10.7 / 8.3, 512 lanes 63 / 48 / 46, 1024 lanes 48 / 41 / 42, 4096 lanes 263 / 242 / 247.
+#define GEO_LIST 64                              // linedefs a wavefront lists at a time
+int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
 template <bool SPLIT>
-__global__ void __launch_bounds__(SW) wall_geometry_kernel(DeviceMap dm, int lane_count, Scratch sc) {
+__global__ void __launch_bounds__(64) wall_geometry_kernel(DeviceMap dm, int lane_count, Scratch sc, int parts) {
     const gd_map_desc *m = &dm.d;
-    __shared__ unsigned short list[GEO_LIST];
-    __shared__ int listed, list_end, first_slot, masked_listed;
-    __shared__ unsigned short masked_list[SW];
-    const int local = blockIdx.x;
-    if (local >= lane_count) return;              // uniform over the block
-    const int x = threadIdx.x, k = threadIdx.x & 3;
+    __shared__ unsigned short list[GEO_LIST], masked_list[64];
+    const int slot = threadIdx.x, k = slot & 3, quad = slot >> 2, shift = __ffs(parts) - 1;
+    const int part = blockIdx.x, local = blockIdx.y;
+    if (local >= lane_count) return;
     const LaneCtx &c = sc.ctx[local];
     const WallRec *recs = sc.rec + (size_t)local * m->wall_count;
     unsigned int *slots = sc.geo_slot + (size_t)local * m->wall_count;
-    unsigned int *named = sc.named + (size_t)local * named_words(m);
-    if (threadIdx.x == 0) { listed = 0; list_end = GEO_LIST; masked_listed = 0; }
-    __syncthreads();
-    if (dm.masked_count > 0) {
-        // masked mid-textures: the linedef of every column's nearest one (its light and its texture mapping are WallGeo's)
-        const u64 hit = sc.masked_hit[(size_t)local * SW + x];
-        const int w = cand_key_wall(hit);
-        if (hit != CAND_KEY_NONE) atomicOr(&named[w >> 5], 1u << (w & 31));
-        // runs of columns share theirs: the first of a run (within its 16 columns) lists it
-        if (hit != CAND_KEY_NONE && __builtin_amdgcn_update_dpp(-1, w, 0x111 /* row_shr:1 */, 0xF, 0xF, false) != w) masked_list[atomicAdd(&masked_listed, 1)] = (unsigned short)w;
-        __syncthreads();                          // the bits are in place too: the barrier orders the block's memory
-        MaskedGeo *masked = sc.masked_geo + (size_t)local * dm.masked_count;
-        for (int task = threadIdx.x; task < 4 * masked_listed; task += SW) {
-            const int w = masked_list[task >> 2];
-            masked_lines(dm, c, recs[w], w, k, masked[dm.masked_slot[w]]);
-        }
-    }
+    const unsigned int *named = sc.named + (size_t)local * named_words(m);
+    const unsigned int first_slot = (unsigned)local * (unsigned)m->wall_count;   // the lane's run of geo
     const int words = named_words(m);
-    for (int word0 = 0; word0 < words; word0 += SW) {
-        // the bits of SW words at a time: a thread a word, as many of them as the list holds
-        unsigned int bits = word0 + x < words ? __hip_atomic_load(&named[word0 + x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-        for (;;) {
-            if (bits) {
-                const int mine = __popc(bits);
-                int at = atomicAdd(&listed, mine);
-                if (at + mine <= GEO_LIST) {
-                    for (; bits; bits &= bits - 1u) list[at++] = (unsigned short)((word0 + x) * 32 + __ffs((int)bits) - 1);
-                } else {
-                    atomicMin(&list_end, at);     // full: the first to find it so ends the list, everybody after it finds it so too
-                }
+    if (part < parts) for (int pass = 0;; ++pass) {   // one, but for lanes that draw more than GEO_LIST * parts linedefs
+        int total = 0;
+        for (int word0 = 0; word0 < words; word0 += 64) {
+            unsigned int bits = word0 + slot < words ? named[word0 + slot] : 0u;
+            const int mine = __popc(bits);
+            int upto = mine;
+#pragma unroll
+            for (int step = 1; step < 64; step <<= 1) { const int left = __shfl_up(upto, step); upto += slot >= step ? left : 0; }
+            for (int rank = total + upto - mine; bits; bits &= bits - 1u, ++rank) {
+                const int group = rank >> 4, at = (group >> shift) * 16 + (rank & 15) - pass * GEO_LIST;
+                if ((group & (parts - 1)) == part && (unsigned)at < GEO_LIST) list[at] = (unsigned short)((word0 + slot) * 32 + __ffs((int)bits) - 1);
             }
-            const int waiting = __syncthreads_or(bits != 0u);
-            const int count = min(listed, list_end);
-            if (threadIdx.x == 0 && count > 0) first_slot = atomicAdd(sc.geo_count, count);
-            __syncthreads();
-            for (int task = threadIdx.x; task < 4 * count; task += SW) {   // the four threads of a linedef are one DPP quad
-                const int w = list[task >> 2], slot = first_slot + (task >> 2);
-                wall_lines(dm, c, recs[w], w, k, sc.geo[slot]);
-                if (k == 0) slots[w] = (unsigned int)slot;
-            }
-            __syncthreads();
-            if (threadIdx.x == 0) { listed = 0; list_end = GEO_LIST; }
-            __syncthreads();
-            if (!waiting) break;                  // the same in the whole block
+            total += bcast(upto, 63);
         }
+        wave_lds_fence();
+        for (int j = 0; j < GEO_LIST / 16; ++j) {
+            const int rank0 = ((pass * (GEO_LIST / 16) + j) * parts + part) * 16;
+            if (rank0 >= total) break;            // the same in the whole wavefront
+            if (rank0 + quad < total) {           // the four threads of a linedef are one DPP quad
+                const int w = list[j * 16 + quad];
+                const unsigned int at = first_slot + (unsigned)(rank0 + quad);
+                wall_lines(dm, c, recs[w], w, k, sc.geo[at]);
+                if (k == 0) slots[w] = at;
+            }
+        }
+        if (((pass + 1) * (GEO_LIST / 16) * parts + part) * 16 >= total) return;
+        wave_lds_fence();
     }
-    // the few passes whose rows are their own, column by column
-    if (!((sc.own_rows[local] >> (x >> 6)) & 1u)) return;
-    const WallRec *frags = sc.frag_rec + (size_t)local * m->split_count * m->fragment_slots;
-    const int passes = sc.pass_count[(size_t)local * SW + x];
-    for (int pass = 0; pass < passes; ++pass) {
-        const size_t at = sc.pass_at(pass, local, x);
-        const PassRec rec = sc.pass_rec[at];
-        if (!(rec.bits & (PB_RASTER | PB_PS_KEEPS)) || !(rec.marks & REC_OWN_ROWS)) continue;
-        const int other = m->wall_sectors[2 * rec.wall + ((rec.marks & REC_SIDE1) ? 0 : 1)];
-        unsigned int rows[2] = {0u, 0u};
-#pragma unroll 1
-        for (int h = 0; h < 8; ++h) {
-            if (h < 4 ? (h >= 2 && (rec.bits & PB_ONE_SIDED)) : !(rec.bits & PB_PS_KEEPS)) continue;
-            const int w = h < 4 ? rec.wall : rec.ps_path;
-            const int behind = h < 4 ? other : (int)rec.ps_other;
-            const int sector = (h & 2) ? (behind < 0 ? 0 : behind) : (int)rec.render_current;
-            const float z = m->sector_heights[2 * sector + ((h & 3) == 0 || (h & 3) == 3 ? 1 : 0)];
-            const FragmentChoice fragment = choose_fragment<SPLIT>(m, frags, recs[w], w, x);
-            const unsigned int row = (unsigned int)project(c, recs[w], fragment, z, x);
-            rows[h >> 2] |= row << (8 * (h & 3));
+    {   // the other wavefronts: a strip of columns each
+        const int strip = part - parts, x = strip * 64 + slot;
+        if (dm.masked_count > 0) {
+            // masked mid-textures: the linedef of every column's nearest one (its light and its texture mapping are WallGeo's)
+            const u64 hit = sc.masked_hit[(size_t)local * SW + x];
+            const int w = cand_key_wall(hit);
+            // runs of columns share theirs: the first of a run (within its 16 columns) lists it
+            const bool lists_it = hit != CAND_KEY_NONE && __builtin_amdgcn_update_dpp(-1, w, 0x111 /* row_shr:1 */, 0xF, 0xF, false) != w;
+            const u64 listing = __ballot(lists_it);
+            wave_lds_fence();
+            if (lists_it) masked_list[__popcll(listing & ((1ULL << slot) - 1))] = (unsigned short)w;
+            wave_lds_fence();
+            MaskedGeo *masked = sc.masked_geo + (size_t)local * dm.masked_count;
+            for (int entry = quad; entry < __popcll(listing); entry += 16) {
+                const int mw = masked_list[entry];
+                masked_lines(dm, c, recs[mw], mw, k, masked[dm.masked_slot[mw]]);
+            }
         }
-        sc.pass_rows[at] = make_uint2(rows[0], rows[1]);
+        // the few passes whose rows are their own, column by column
+        if (!((sc.own_rows[local] >> strip) & 1u)) return;
+        const WallRec *frags = sc.frag_rec + (size_t)local * m->split_count * m->fragment_slots;
+        const int passes = sc.pass_count[(size_t)local * SW + x];
+        PassRec next = {};
+        if (passes > 0) next = sc.pass_rec[sc.pass_at(0, local, x)];
+        for (int pass = 0; pass < passes; ++pass) {
+            const size_t at = sc.pass_at(pass, local, x);
+            const PassRec rec = next;
+            if (pass + 1 < passes) next = sc.pass_rec[sc.pass_at(pass + 1, local, x)];
+            if (!(rec.bits & (PB_RASTER | PB_PS_KEEPS)) || !(rec.marks & REC_OWN_ROWS)) continue;
+            const int other = m->wall_sectors[2 * rec.wall + ((rec.marks & REC_SIDE1) ? 0 : 1)];
+            unsigned int rows[2] = {0u, 0u};
+#pragma unroll 1
+            for (int h = 0; h < 8; ++h) {
+                if (h < 4 ? (h >= 2 && (rec.bits & PB_ONE_SIDED)) : !(rec.bits & PB_PS_KEEPS)) continue;
+                const int w = h < 4 ? rec.wall : rec.ps_path;
+                const int behind = h < 4 ? other : (int)rec.ps_other;
+                const int sector = (h & 2) ? (behind < 0 ? 0 : behind) : (int)rec.render_current;
+                const float z = m->sector_heights[2 * sector + ((h & 3) == 0 || (h & 3) == 3 ? 1 : 0)];
+                const FragmentChoice fragment = choose_fragment<SPLIT>(m, frags, recs[w], w, x);
+                const unsigned int row = (unsigned int)project(c, recs[w], fragment, z, x);
+                rows[h >> 2] |= row << (8 * (h & 3));
+            }
+            sc.pass_rows[at] = make_uint2(rows[0], rows[1]);
+        }
     }
 }
 
@@ -3659,6 +3668,12 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     // the linedefs the recorded passes draw get a bit each; columns that draw what the column before them draws leave it to that one
     unsigned int *named = sc.named + (size_t)local * named_words(m);
     int last_named = -1;
+    if (dm.masked_count > 0) {   // so do those whose masked mid-texture is a column's nearest
+        const u64 hit = sc.masked_hit[(size_t)local * SW + x];
+        const int w = cand_key_wall(hit);
+        const int left = __builtin_amdgcn_update_dpp(-1, w, 0x111 /* row_shr:1 */, 0xF, 0xF, false);
+        if (hit != CAND_KEY_NONE && left != w) atomicOr(&named[w >> 5], 1u << (w & 31));
+    }
     PixelBuffers no_pixels; SilhouetteBounds no_bounds; GapRange no_gaps;   // the state part of pass_advance touches none of them
     PassColumn pc;
     bool done = false;
@@ -5512,7 +5527,6 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.rec, L * W);
     take(&sc.span, L * W);
     take(&sc.geo, L * W);
-    take(&sc.geo_count, 1);
     take(&sc.geo_slot, L * W);
     take(&sc.named, L * ((W + 31) / 32));
     take(&sc.own_rows, L);
@@ -5768,7 +5782,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
             list_billboards(r->side_ready ? r->side_stream : stream);
         }
         mark();
-        hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(count), dim3(SW), 0, stream, r->dm, count, sc);
+        hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(geometry_parts(count) + SW / 64, count), dim3(64), 0, stream, r->dm, count, sc, geometry_parts(count));
         const dim3 grid((wavefronts * raster_parts(count) + WALL_STRIPS_PER_GROUP - 1) / WALL_STRIPS_PER_GROUP), block(64 * WALL_STRIPS_PER_GROUP);
         const bool general = split || m.sector_count > LDS_SECTORS || m.texture_count > LDS_TEXTURES;
         auto kernel = decals ? (general ? wall_raster_kernel<true, true> : wall_raster_kernel<true, false>)

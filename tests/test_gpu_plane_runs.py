@@ -1,5 +1,6 @@
-"""Plane shading where a tile of the view (64 columns, 16 rows) holds more runs of pixels than a wavefront works out at once, against
-the CPU oracle."""
+"""Plane shading where a tile of the view (64 columns, 16 rows) holds more runs of pixels than a wavefront works out at once, and (the
+smaller cells) lanes that draw two thousand linedefs, more than the wavefronts of wall_geometry_kernel list at once, against the CPU
+oracle."""
 
 from __future__ import annotations
 
