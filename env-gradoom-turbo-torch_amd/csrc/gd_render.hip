@@ -13,7 +13,7 @@
 //   wall_raster     1 wave / strip            the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
 //   plane_shade     1 wave / 64 columns x 16 rows  flat texel + light for every pixel a plane of the wall pass shows,
 //                                             the wall tiers' palette indices
-//   flat_gap        4 waves / gap column      per-pixel plane rays (fine point raster) for the gap pixels, vertical repair
+//   flat_gap        8 or 16 waves / gap column     per-pixel plane rays (fine point raster) for the gap pixels, vertical repair
 //   flat_rows, flat_span_select, flat_tail, flat_span_finish
 //                                             visplane repair of the rows where a gap pixel stayed unresolved
 //   flat_shade      1 wave / gap column       the gap pixels' flats
@@ -1568,10 +1568,14 @@ __device__ __forceinline__ void note_row(const Scratch &sc, int local, int half,
     if (atomicMin(&span[0], y) == VH) sc.flat_spans[atomicAdd(sc.flat_span_count, 1)] = (local << 1) | half;
 }
 
-// GAP_WAVES wavefronts a column, which probe 16 of its rows at a time: first the gap pixels', then the others' from the topmost
+// GAP_WAVES wavefronts a column, which probe four rows each at a time: first the gap pixels', then the others' from the topmost
 // unresolved gap pixel down, until the lowest one is past and a resolved pixel below it is found (or the half ends).
-#define GAP_WAVES 4
 #define ROW_UNPROBED -2
+// The fewer the lanes, the fewer such columns and the longer the kernel lasts as its slowest one.  us with 4 / 8 / 16 wavefronts a column: 512
+// lanes 95 / 71 / 62, 1024 lanes (2000 linedefs) 100 / 64 / 52, 4096 lanes 118 / 115 / 141; the whole selection at 2048 lanes of 800, 2000 and
+// 4000 linedefs 164 / 153 / 161, 179 / 144 / 152, 253 / 221 / 230, at 1024 lanes 136 / 111 / 111, 146 / 112 / 97, 193 / 160 / 146.
+int gap_waves(int lanes) { return lanes <= 1536 ? 16 : 8; }
+template <int GAP_WAVES>
 __global__ void __launch_bounds__(64 * GAP_WAVES) flat_gap_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
     __shared__ ProbeLds probe_lds[GAP_WAVES];
     __shared__ short row_sector[VH];                  // the sector of each row's pixel, -1 unresolved, ROW_UNPROBED
@@ -5815,7 +5819,8 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     auto flat_grid = [count](int per_lane, int most) { return dim3((unsigned)(count >= most / per_lane ? most : (count * per_lane < 32 ? 32 : count * per_lane))); };
     const int plane_levels = m.floor_level_count + m.ceil_level_count;
     const bool level_masks = plane_levels > LEVEL_MASK_MIN_LEVELS && plane_levels <= 32 * LEVEL_MASK_WORDS_MAX;   // level_mask_words() > 0
-    hipLaunchKernelGGL(flat_gap_kernel, flat_grid(4, 2048), dim3(64 * GAP_WAVES), 0, stream, r->dm, *lanes, base, sc);
+    if (gap_waves(count) == 16) hipLaunchKernelGGL(flat_gap_kernel<16>, flat_grid(4, 1024), dim3(64 * 16), 0, stream, r->dm, *lanes, base, sc);
+    else hipLaunchKernelGGL(flat_gap_kernel<8>, flat_grid(4, 2048), dim3(64 * 8), 0, stream, r->dm, *lanes, base, sc);
     hipLaunchKernelGGL(flat_rows_kernel, dim3(count), dim3(64), 0, stream, count, sc);
     hipLaunchKernelGGL(level_masks ? flat_span_select_kernel<true> : flat_span_select_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, sc);
     mark();
