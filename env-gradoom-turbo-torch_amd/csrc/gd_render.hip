@@ -5714,6 +5714,13 @@ int validate_map(const gd_map_desc *h) {
 
 const int STAGE_COUNT = 9;
 
+// A frame that goes to the side stream and back pays some 20 us for it.  Batches whose strips are all selected by one launch do without
+// where there is little to put there: no billboards, or a few lanes.  A frame in us with / without, 1 lane with billboards on 120 to 4000
+// linedefs 139 / 119, 261 / 236, 210 / 185, 243 / 235, 433 / 414, 8 lanes 256 / 285, 284 / 259, 293 / 312, 396 / 394, 450 / 428, 48 lanes
+// 323 / 356, 405 / 436, 439 / 468, 586 / 611, 878 / 891; without billboards on 320, 800 and 4000 linedefs, 16 lanes 256 / 241, 364 / 351,
+// 533 / 520, 64 lanes 437 / 429, 434 / 426, 884 / 878.
+bool side_stream_pays(int lanes, bool billboards) { return lanes * SEGS_PER_LANE > SELECT_STAGED_STRIPS || (billboards && lanes >= 4); }
+
 int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_desc *lanes, const gd_frame_out *out, int base, int count, hipStream_t stream, bool timed) {
     const gd_map_desc &m = r->dm.d;
     Scratch sc = chunk_scratch;
@@ -5742,6 +5749,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     }
     const bool has_billboards = lanes->sprite_slots > 0 && lanes->sprite_x;
     auto list_billboards = [&](hipStream_t on) { hipLaunchKernelGGL(sprite_list_kernel, dim3(count), dim3(LIST_THREADS), 0, on, r->dm, *lanes, base, count, sc); };
+    const bool aside = r->side_ready && side_stream_pays(count, has_billboards);
     mark();
     hipLaunchKernelGGL(lane_setup_kernel, dim3((count + 63) / 64), dim3(64), 0, stream, r->dm, *lanes, base, count, sc);
     hipLaunchKernelGGL(lane_tables_kernel, dim3(count), dim3(256), 0, stream, r->dm, *lanes, base, count, sc);
@@ -5766,24 +5774,29 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         const int staged_strips = r->side_ready ? (strips < SELECT_STAGED_STRIPS ? strips : SELECT_STAGED_STRIPS) : 0;
         auto select_kernel = split ? wall_select_kernel<true, false> : wall_select_kernel<false, false>;
         if (staged_strips > 0) {
-            HIP_TRY(hipEventRecord(r->fork_event, stream));
-            HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
+            const bool alone = staged_strips == strips;   // the other launch is left with strips of spilled columns: it follows
+            if (!alone) {
+                HIP_TRY(hipEventRecord(r->fork_event, stream));
+                HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
+            }
             auto staged_kernel = split ? wall_select_kernel<true, true> : wall_select_kernel<false, true>;
             const int fine_strips = !select_finely(count, m.wall_count) ? 0 : (strips < SELECT_FINE_STRIPS ? strips : SELECT_FINE_STRIPS);
             hipLaunchKernelGGL(staged_kernel, dim3(fine_strips * SELECT_FINE_PARTS + (staged_strips - fine_strips) * SELECT_PARTS), select_block, 0, stream, r->dm, count, sc, staged_strips, fine_strips);
-            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, r->side_stream, r->dm, count, sc, staged_strips, 0);
-            HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
-            HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
+            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, alone ? stream : r->side_stream, r->dm, count, sc, staged_strips, 0);
+            if (!alone) {
+                HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
+                HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
+            }
         } else {
             hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0, 0);
         }
         // the billboards' lists beside the walls' drawing, on the side stream (when stages are being timed, with the billboards)
         if (has_billboards && !fused && !timed) {
-            if (r->side_ready) {
+            if (aside) {
                 HIP_TRY(hipEventRecord(r->fork_event, stream));
                 HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
             }
-            list_billboards(r->side_ready ? r->side_stream : stream);
+            list_billboards(aside ? r->side_stream : stream);
         }
         mark();
         hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(geometry_parts(count) + SW / 64, count), dim3(64), 0, stream, r->dm, count, sc, geometry_parts(count));
@@ -5800,7 +5813,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     // caller's stream, where its first kernel starts the moment the traversal ends, and the shading goes to the renderer's
     // side stream, a few microseconds behind (the other way round the shading takes every compute unit before the first
     // block of the flat pass is placed).  (Not when stages are being timed.)
-    const bool beside = !fused && !timed && r->side_ready;
+    const bool beside = !fused && !timed && aside;
     hipStream_t shade_stream = stream;
     if (beside) {
         HIP_TRY(hipEventRecord(r->fork_event, stream));
