@@ -2,12 +2,12 @@
 //
 // One frame for N lanes runs as a short chain of kernels on the caller's stream:
 //
-//   lane_setup      1 thread / lane           view basis, pitch centre, camera sector
-//   lane_tables     1 thread / (lane, row)    per-lane distance bounds of every height level, plane rows, row slopes
+//   lane_tables     1 block / lane            view basis, pitch centre, camera sector; distance bounds of every height
+//                                             level, plane rows, row slopes
 //   wall_setup      1 block / lane or 256 linedefs  FWallCoords span+depths, span ownership bounds, the linedef's
 //                                             entry in the candidate list of every column it can own, and the
 //                                             nearest blocking hit of every column (64-bit atomicMin)
-//   strip_key/order 1 thread / 64-col strip   longest strip first (counting sort on the blocking distance)
+//   strip_key/order 1 thread / 64-col strip   longest strip first (counting sort on the longest list); columns that see more than 64 linedefs
 //   wall_select     1 wave / strip            portal traversal: which drawseg every column pass selects, one record each
 //   wall_geometry   13 to 21 waves / lane            the linedefs those passes draw, as lines over the columns: every division of the drawing
 //   wall_raster     1 wave / strip            the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
@@ -56,7 +56,7 @@ typedef unsigned long long u64;
 #define VH 208
 #define CAND_MAX 64          // candidate linedefs a screen column keeps in its own slots
 // A column whose ray can reach more than CAND_MAX linedefs (a long corridor seen end on) gets a slot in the chunk's spill
-// pool, where cand_spill_kernel lists all of them, up to SPILL_DEPTH.  The pool continues the candidate blocks with
+// pool, where strip_order_kernel lists all of them, up to SPILL_DEPTH.  The pool continues the candidate blocks with
 // the same layout (entry k of a column lies k * 320 entries on), SPILL_DEPTH x 320 entries per pool block, so a
 // spilled column differs from the others only in where its list starts and how long it may be.
 #define SPILL_DEPTH 256
@@ -261,7 +261,7 @@ struct Scratch {    // per-chunk working memory, sized at create
     int *cand_count;       // [L,320] entries listed (beyond CAND_MAX: the column wanted more than its own slots hold), or for
                            // a column with a pool slot: entries in the pool | (slot + 1) << SPILL_SHIFT
     int *spill_columns;    // [spill_slots] the columns (lane * 320 + column) that were given pool slots, in slot order
-    int *spill_count;      // [1] columns that asked for a slot (cleared by lane_setup_kernel, counted by strip_key_kernel)
+    int *spill_count;      // [1] columns that asked for a slot (cleared by lane_tables_kernel, counted by note_length)
     unsigned spill_base;   // where the pool starts in `cand`, in entries
     int spill_slots;       // pool slots of this chunk (a multiple of 320)
     unsigned short *flat_sector;// [L,208,320]
@@ -269,16 +269,16 @@ struct Scratch {    // per-chunk working memory, sized at create
     int2 *gap_columns;     // [L*320] the screen columns that hold view pixels no wall tier, plane or masked texture covers (they
                            // show the flat pass's picture), of every lane, as one work list: lane << 9 | column, and the rows
                            // they lie in, first | one past the last << 8.  Listed by wall_raster_kernel.
-    int *gap_column_count; // [1] its length (cleared by lane_setup_kernel)
+    int *gap_column_count; // [1] its length (cleared by lane_tables_kernel)
     int *flat_tail;        // [L,2,320] per screen half and column: the sector of the first resolved pixel below the
                            // half's noted rows, -1 if the column was not looking for one or found none
     int *flat_span;        // [L,4] first / last row of the ceiling half, then of the floor half, that holds a shown
                            // pixel the flat pass could not resolve and whose repair reads its row (208, -1 = none):
                            // the rows the row repairs work on
     int *flat_spans;       // [L*2] the (lane << 1 | half) with such rows, as one work list
-    int *flat_span_count;  // [1] its length (cleared by lane_setup_kernel)
+    int *flat_span_count;  // [1] its length (cleared by lane_tables_kernel)
     int *flat_rows;        // [L*208] the noted rows of every lane as one work list, entry = lane << 8 | row
-    int *flat_row_count;   // [1] its length (cleared by lane_setup_kernel, filled by flat_rows_kernel)
+    int *flat_row_count;   // [1] its length (cleared by lane_tables_kernel, filled by flat_rows_kernel)
     int pass_slots;        // passes a column can record in this chunk
     // where pass `pass` of a column lies in the three planes below: the passes that most columns make lie close together
     __device__ __forceinline__ size_t pass_at(int pass, int local, int x) const { return ((size_t)pass * (size_t)lane_stride + (size_t)local) * SW + (size_t)x; }
@@ -388,6 +388,16 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Smallest / largest value of the wavefront, by lane moves (all lanes executing; the result is uniform).
+template <int CONTROL, int ROWS> __device__ __forceinline__ int wave_move(int other, int v) { return __builtin_amdgcn_update_dpp(other, v, CONTROL, ROWS, 0xF, false); }
+__device__ __forceinline__ int wave_min(int v) {
+    const int none = 0x7fffffff;
+    v = min(v, wave_move<0x111, 0xF>(none, v)); v = min(v, wave_move<0x112, 0xF>(none, v));   // row_shr:1, 2, 4, 8: the last lane of
+    v = min(v, wave_move<0x114, 0xF>(none, v)); v = min(v, wave_move<0x118, 0xF>(none, v));   // every sixteen holds their smallest
+    v = min(v, wave_move<0x142, 0xA>(none, v)); v = min(v, wave_move<0x143, 0xC>(none, v));   // row_bcast:15, 31: lane 63 that of all
+    return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
 // Value of `v` in lane `lane` of the wavefront; `lane` must be the same in every active lane.
 __device__ __forceinline__ int bcast(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ float bcast(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
@@ -576,7 +586,43 @@ __device__ __forceinline__ int level_bucket(float g) {
     return b <= 0.0f ? 0 : (b >= (float)(LEVEL_BUCKETS - 1) ? LEVEL_BUCKETS - 1 : (int)b);
 }
 
-// Per-lane tables for the flat kernels, one block per lane (after lane_setup):
+// The lane's view (engine.py:10648-10658, 2122-2133, 9622-9631, 12384-12391, 9619), but for last_ceiling_row.
+__device__ __forceinline__ LaneCtx lane_view(const DeviceMap &dm, const gd_lanes_desc &lanes, int n) {
+    const float BAM_TO_RADIANS = (float)(2.0 * 3.14159265358979323846 / 4294967296.0);
+    LaneCtx c;
+    c.x = lanes.x[n]; c.y = lanes.y[n]; c.view_z = lanes.view_z[n];
+    float angle = lanes.angle[n];
+    i64 pitch_bam = lanes.pitch_bam[n];
+    c.flash_light = lanes.flash_light ? lanes.flash_light[n] : 0;
+    i64 retained_bam = lanes.angle_bam[n];
+    float visible_angle = (float)retained_bam * BAM_TO_RADIANS;
+    i64 angle_bam = retained_bam;
+    if (angle != visible_angle) {
+        float two_pi = (float)(2.0 * 3.14159265358979323846);
+        float r = fmodf(angle, two_pi);
+        if (r != 0.0f && (r < 0.0f)) r += two_pi;   // torch.remainder with a positive divisor
+        angle_bam = round_to_i64(r / BAM_TO_RADIANS) & UINT32_MASK;
+    }
+    i64 xf = lanes.x_fixed[n], yf = lanes.y_fixed[n];
+    float visible_x = (float)xf / 65536.0f, visible_y = (float)yf / 65536.0f;
+    c.view_x_fixed = (c.x != visible_x) ? round_to_i64(c.x * 65536.0f) : xf;
+    c.view_y_fixed = (c.y != visible_y) ? round_to_i64(c.y * 65536.0f) : yf;
+    int fine = (int)((angle_bam >> 19) & (FINE_ANGLES - 1));
+    c.vsin = dm.fine_sine[fine];
+    c.vcos = dm.fine_sine[(fine + FINE_ANGLES / 4) & (FINE_ANGLES - 1)];
+    c.fsin = (float)c.vsin / 65536.0f;
+    c.fcos = (float)c.vcos / 65536.0f;
+    i64 tangent_index = clampi((ANGLE_90 - pitch_bam) >> 19, 0, FINE_ANGLES / 2 - 1);
+    i64 tangent = dm.fine_tangent[tangent_index];
+    c.center_fixed = (i64)(VH / 2) * FIXED_UNIT + ((FOCAL_Y_FIXED * tangent) >> 16);
+    c.upper_clip = tdiv(shl64(-c.center_fixed, 16), FOCAL_Y_FIXED);
+    c.lower_clip = tdiv(shl64((i64)VH * FIXED_UNIT - c.center_fixed, 16), FOCAL_Y_FIXED);
+    c.pitch_offset = (float)((tangent * 12582912LL) >> 16) / 65536.0f;
+    c.sector = sector_at(&dm.d, c.x, c.y);
+    return c;
+}
+
+// A lane's view, by one thread of its block, while the others clear the lane's lists; then the tables for the flat kernels:
 //  * per plane level, how far the camera is, at least, from every sector at that level: a flat
 //    probe nearer than that cannot land in such a sector (engine.py:10981-11024 tests the point
 //    against every sector; here the far ones are ruled out by their bounding boxes);
@@ -585,11 +631,18 @@ __device__ __forceinline__ int level_bucket(float g) {
 //  * per log2 texture size, the per-column texture steps (engine.py:10895-10902).
 // The last three only depend on (lane, level), (lane, row) and (lane, size), so dividing once
 // here spares plane shading four 64-bit divisions per pixel.
-__global__ void lane_tables_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
+__global__ void __launch_bounds__(256) lane_tables_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
     const int local = blockIdx.x;
     const int floors = dm.d.floor_level_count, levels = floors + dm.d.ceil_level_count;
     if (local >= lane_count) return;
-    const LaneCtx &c = sc.ctx[local];
+    __shared__ LaneCtx c;
+    __shared__ unsigned int masks_lds[LEVEL_BUCKETS * LEVEL_MASK_WORDS_MAX];
+    if (threadIdx.x == 0) c = lane_view(dm, lanes, lane_base + local);
+    else if (threadIdx.x == 64) {
+        int *span = sc.flat_span + (size_t)local * 4;
+        span[0] = VH; span[1] = -1; span[2] = VH; span[3] = -1;
+        if (local == 0) { *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
+    }
     // the lane's per-column lists start empty
     for (int x = threadIdx.x; x < SW; x += blockDim.x) { sc.cand_count[(size_t)local * SW + x] = 0; sc.block_hit[(size_t)local * SW + x] = ~0ULL; sc.masked_hit[(size_t)local * SW + x] = CAND_KEY_NONE; }
     for (int k = threadIdx.x; k < named_words(&dm.d); k += blockDim.x) sc.named[(size_t)local * named_words(&dm.d) + k] = 0u;
@@ -605,10 +658,15 @@ __global__ void lane_tables_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_b
         if (threadIdx.x == 0) sc.lane_blends[local] = any;
     }
     const float cx = lanes.x[lane_base + local], cy = lanes.y[lane_base + local];
-    __shared__ unsigned int masks_lds[LEVEL_BUCKETS * LEVEL_MASK_WORDS_MAX];
     const int mask_words = level_mask_words(&dm.d);
     for (int k = threadIdx.x; k < LEVEL_BUCKETS * mask_words; k += blockDim.x) masks_lds[k] = 0u;
     __syncthreads();
+    {
+        // rows 0 .. last_ceiling_row look at ceilings
+        static_assert(VH <= 256, "lane_tables_kernel: a thread a row");
+        const int ceiling_rows = __syncthreads_count((int)threadIdx.x < VH && !(((float)(int)threadIdx.x - (103.5f + c.pitch_offset)) > 0));   // flat_center()
+        if (threadIdx.x == 0) { c.last_ceiling_row = ceiling_rows - 1; sc.ctx[local] = c; }
+    }
     for (int l = threadIdx.x; l < levels; l += blockDim.x) {
         float reach = GD_INF, far = 0.0f;
         for (int k = dm.level_box_ofs[l]; k < dm.level_box_ofs[l + 1]; ++k) {
@@ -652,52 +710,6 @@ __global__ void lane_tables_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_b
         entry[32 + k] = (shl64(k < 16 ? c.vcos : -c.vsin, 32 - (k & 15)) >> 16) - mul64(SW / 2 - 1, step);
         entry[64 + k] = shl64(k < 16 ? c.view_x_fixed : -c.view_y_fixed, 32 - (k & 15)) >> 16;
     }
-}
-
-// ---------------------------------------------------------------------------------------------
-// lane_setup: engine.py:10648-10658, 2122-2133, 9622-9631, 12384-12391, 9619
-// ---------------------------------------------------------------------------------------------
-__global__ void lane_setup_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
-    int local = blockIdx.x * blockDim.x + threadIdx.x;
-    if (local >= lane_count) return;
-    int n = lane_base + local;
-    const float BAM_TO_RADIANS = (float)(2.0 * 3.14159265358979323846 / 4294967296.0);
-    LaneCtx c;
-    c.x = lanes.x[n]; c.y = lanes.y[n]; c.view_z = lanes.view_z[n];
-    float angle = lanes.angle[n];
-    i64 pitch_bam = lanes.pitch_bam[n];
-    c.flash_light = lanes.flash_light ? lanes.flash_light[n] : 0;
-    i64 retained_bam = lanes.angle_bam[n];
-    float visible_angle = (float)retained_bam * BAM_TO_RADIANS;
-    i64 angle_bam = retained_bam;
-    if (angle != visible_angle) {
-        float two_pi = (float)(2.0 * 3.14159265358979323846);
-        float r = fmodf(angle, two_pi);
-        if (r != 0.0f && (r < 0.0f)) r += two_pi;   // torch.remainder with a positive divisor
-        angle_bam = round_to_i64(r / BAM_TO_RADIANS) & UINT32_MASK;
-    }
-    i64 xf = lanes.x_fixed[n], yf = lanes.y_fixed[n];
-    float visible_x = (float)xf / 65536.0f, visible_y = (float)yf / 65536.0f;
-    c.view_x_fixed = (c.x != visible_x) ? round_to_i64(c.x * 65536.0f) : xf;
-    c.view_y_fixed = (c.y != visible_y) ? round_to_i64(c.y * 65536.0f) : yf;
-    int fine = (int)((angle_bam >> 19) & (FINE_ANGLES - 1));
-    c.vsin = dm.fine_sine[fine];
-    c.vcos = dm.fine_sine[(fine + FINE_ANGLES / 4) & (FINE_ANGLES - 1)];
-    c.fsin = (float)c.vsin / 65536.0f;
-    c.fcos = (float)c.vcos / 65536.0f;
-    i64 tangent_index = clampi((ANGLE_90 - pitch_bam) >> 19, 0, FINE_ANGLES / 2 - 1);
-    i64 tangent = dm.fine_tangent[tangent_index];
-    c.center_fixed = (i64)(VH / 2) * FIXED_UNIT + ((FOCAL_Y_FIXED * tangent) >> 16);
-    c.upper_clip = tdiv(shl64(-c.center_fixed, 16), FOCAL_Y_FIXED);
-    c.lower_clip = tdiv(shl64((i64)VH * FIXED_UNIT - c.center_fixed, 16), FOCAL_Y_FIXED);
-    c.pitch_offset = (float)((tangent * 12582912LL) >> 16) / 65536.0f;
-    c.sector = sector_at(&dm.d, c.x, c.y);
-    c.last_ceiling_row = -1;
-    for (int y = 0; y < VH; ++y) if (!(((float)y - (103.5f + c.pitch_offset)) > 0)) c.last_ceiling_row = y;   // flat_center()
-    sc.ctx[local] = c;
-    int *span = sc.flat_span + (size_t)local * 4;
-    span[0] = VH; span[1] = -1; span[2] = VH; span[3] = -1;
-    if (local == 0) { *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
 }
 
 __device__ __forceinline__ void ray_direction(const LaneCtx &c, int x, float *rx, float *ry) {
@@ -794,6 +806,15 @@ __device__ __forceinline__ void request_spill_slot(const Scratch &sc, int column
     const int slot = atomicAdd(sc.spill_count, 1);
     if (slot < sc.spill_slots) sc.spill_columns[slot] = column;
     else sc.status[STATUS_CAND_OVERFLOW] = 1;
+}
+
+// The expected traversal length of a strip, from its columns' counts, a lane a column (see strip_order_kernel); columns that see too
+// many linedefs ask for a slot of the spill pool.
+__device__ __forceinline__ void note_length(const Scratch &sc, int local, int x, int length) {
+    static_assert(SEG_COLS == 64, "note_length: a strip a wavefront");
+    if (length > CAND_MAX) { request_spill_slot(sc, local * SW + x); length = CAND_MAX; }
+    length = wave_max(length);
+    if ((x & (SEG_COLS - 1)) == 0) sc.strip_key[local * SEGS_PER_LANE + x / SEG_COLS] = (unsigned char)length;   // at most CAND_MAX
 }
 
 // One thread owns one linedef for the per-linedef arithmetic; its columns are looked at by the whole wavefront together, since
@@ -999,7 +1020,7 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
             if ((q.facts & SETUP_MASKED) && p) atomicMin(&masked_hits[x], cand_key(entry));
             const int at = atomicAdd(&counts[x], 1);
             if (at < CAND_MAX) list[(size_t)at * SW + x] = entry;
-            // else: the count says so, and the column is listed afresh in the spill pool (strip_key_kernel, cand_spill_kernel)
+            // else: the count says so, and the column is listed afresh in the spill pool (note_length, strip_order_kernel)
         };
         auto look = [&](const SetupWall &q, int x, bool &ok, bool &along_high, float &d) -> bool {   // eval_segment's ray test
             float rx, ry; ray_direction(c, x, &rx, &ry);
@@ -1076,23 +1097,25 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
     }
     if (!WHOLE) return;
     __syncthreads();
-    for (int x = threadIdx.x; x < SW; x += THREADS) {
+    static_assert(!WHOLE || THREADS >= SW, "wall_setup_kernel: a thread a column");
+    if (threadIdx.x < SW) {                              // whole wavefronts
+        const int x = threadIdx.x;
         const size_t at = (size_t)local * SW + x;
         sc.block_hit[at] = block_lds[x]; sc.masked_hit[at] = masked_lds[x]; sc.cand_count[at] = count_lds[x];
+        note_length(sc, local, x, count_lds[x]);
     }
 }
 
 // The candidate list of every column that was given a spill slot, written afresh into the pool: one wavefront per
 // column tests the column's ray against every linedef of the map (eval_wall: the same test, on the same per-linedef
 // facts, that entered the linedef in wall_setup_kernel) and keeps those with a finite distance, in linedef order.
-// A fixed, small grid: the kernel is launched every frame and nearly always finds no column to do.
-#define SPILL_BLOCKS 1024
-__global__ void __launch_bounds__(64) cand_spill_kernel(DeviceMap dm, Scratch sc) {
+// Nearly every frame finds no column to do: the work-groups beside the one that orders the strips look.
+__device__ __forceinline__ void list_spilled_columns(const DeviceMap &dm, const Scratch &sc, int wavefront, int wavefronts) {
     const gd_map_desc *m = &dm.d;
     const int wanted = *sc.spill_count;
     const int total = wanted < sc.spill_slots ? wanted : sc.spill_slots;
-    const int walls = m->wall_count;
-    for (int slot = blockIdx.x; slot < total; slot += gridDim.x) {
+    const int walls = m->wall_count, lane_id = threadIdx.x & 63;
+    for (int slot = wavefront; slot < total; slot += wavefronts) {
         const int column = sc.spill_columns[slot];
         const int local = column / SW, x = column - local * SW;
         const LaneCtx &c = sc.ctx[local];
@@ -1101,7 +1124,7 @@ __global__ void __launch_bounds__(64) cand_spill_kernel(DeviceMap dm, Scratch sc
         Cand *list = sc.cand + sc.spill_base + ((size_t)(slot / SW) * SPILL_DEPTH * SW + (size_t)(slot % SW));
         int listed = 0;
         for (int w0 = 0; w0 < walls; w0 += 64) {
-            const int w = w0 + (int)threadIdx.x;
+            const int w = w0 + lane_id;
             bool keep = false;
             Cand entry;
             if (w < walls) {
@@ -1115,14 +1138,14 @@ __global__ void __launch_bounds__(64) cand_spill_kernel(DeviceMap dm, Scratch sc
                 entry.dist = e.dist;
             }
             const u64 keeps = __ballot(keep);
-            const int position = listed + __popcll(keeps & ((1ULL << threadIdx.x) - 1ULL));
+            const int position = listed + __popcll(keeps & ((1ULL << lane_id) - 1ULL));
             if (keep) {
                 if (position < SPILL_DEPTH) list[(size_t)position * SW] = entry;
                 else sc.status[STATUS_CAND_OVERFLOW] = 1;
             }
             listed += __popcll(keeps);
         }
-        if (threadIdx.x == 0) sc.cand_count[column] = (listed < SPILL_DEPTH ? listed : SPILL_DEPTH) | ((slot + 1) << SPILL_SHIFT);
+        if (lane_id == 0) sc.cand_count[column] = (listed < SPILL_DEPTH ? listed : SPILL_DEPTH) | ((slot + 1) << SPILL_SHIFT);
     }
 }
 
@@ -2745,17 +2768,6 @@ __device__ __forceinline__ float quad_min(float v) {
     return fminf(v, __int_as_float(quad_move<0x4E>(__float_as_int(v))));
 }
 
-// Smallest / largest value of the wavefront, by lane moves (all lanes executing; the result is uniform).
-template <int CONTROL, int ROWS> __device__ __forceinline__ int wave_move(int other, int v) { return __builtin_amdgcn_update_dpp(other, v, CONTROL, ROWS, 0xF, false); }
-__device__ __forceinline__ int wave_min(int v) {
-    const int none = 0x7fffffff;
-    v = min(v, wave_move<0x111, 0xF>(none, v)); v = min(v, wave_move<0x112, 0xF>(none, v));   // row_shr:1, 2, 4, 8: the last lane of
-    v = min(v, wave_move<0x114, 0xF>(none, v)); v = min(v, wave_move<0x118, 0xF>(none, v));   // every sixteen holds their smallest
-    v = min(v, wave_move<0x142, 0xA>(none, v)); v = min(v, wave_move<0x143, 0xC>(none, v));   // row_bcast:15, 31: lane 63 that of all
-    return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
-
 // engine.py:12637-12884
 // `window_dirty` says whether some pixel inside the open window [ceiling_clip, floor_clip) may
 // already be filled, plane-owned or carry a sprite-clip depth.  A two-sided drawseg only writes
@@ -3543,24 +3555,25 @@ __global__ void __launch_bounds__(64) wall_geometry_kernel(DeviceMap dm, int lan
 // 64 / SEG_COLS segments of about the same length (whatever lanes they belong to), and the longest go first.  The length
 // is taken to be the longest candidate list of the segment, which wall_setup_kernel has counted anyway: walking the lists
 // to count the portals proper orders the segments a little better (the traversal gains 0.04 ms on the 4000-linedef map)
-// but the walk costs 0.11 ms.  strip_key_kernel takes the maxima, strip_order_kernel sorts them (one block, counting sort).
+// but the walk costs 0.11 ms.  wall_setup_kernel or strip_key_kernel takes the maxima, strip_order_kernel sorts them (one block, counting sort).
 // Narrow segments waste fewer column passes (on the 4000-linedef map 69 % of the passes a wavefront runs are useful with
 // whole 64-column strips, 80 % with two sorted 32-column segments, 89 % with four of 16), but unrelated segments share no
 // linedefs, branches or row ranges, and a pass costs what the union of its columns' paths costs: measured, the traversal
 // takes 3.86 ms with 64 or 32 columns a segment, 4.06 ms with 16 and 4.23 ms with 8.  Hence whole strips.
-__global__ void __launch_bounds__(256) strip_key_kernel(int lane_count, Scratch sc) {
+__global__ void __launch_bounds__(256) strip_key_kernel(int lane_count, Scratch sc) {   // of lanes whose linedefs were dealt out (wall_setup_kernel)
     const int strip = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int local = strip / (SW / 64);
     if (local >= lane_count) return;
     const int x = (strip - local * (SW / 64)) * 64 + (threadIdx.x & 63);
-    int length = sc.cand_count[(size_t)local * SW + x];
-    if (length > CAND_MAX) { request_spill_slot(sc, local * SW + x); length = CAND_MAX; }   // cand_spill_kernel runs next
-#pragma unroll
-    for (int step = 1; step < SEG_COLS; step <<= 1) length = max(length, __shfl_xor(length, step));
-    if ((x & (SEG_COLS - 1)) == 0) sc.strip_key[local * SEGS_PER_LANE + x / SEG_COLS] = (unsigned char)length;   // at most CAND_MAX
+    note_length(sc, local, x, sc.cand_count[(size_t)local * SW + x]);
 }
 
-__global__ void __launch_bounds__(1024) strip_order_kernel(int strips, Scratch sc) {
+#define SPILL_BLOCKS 64
+__global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int strips, Scratch sc) {
+    if (blockIdx.x > 0) {        // the others list the spilled columns afresh
+        list_spilled_columns(dm, sc, (blockIdx.x - 1) * 16 + (threadIdx.x >> 6), (gridDim.x - 1) * 16);
+        return;
+    }
     __shared__ int histogram[CAND_MAX + 1], position[CAND_MAX + 1];
     for (int k = threadIdx.x; k <= CAND_MAX; k += blockDim.x) histogram[k] = 0;
     __syncthreads();
@@ -5751,16 +5764,15 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     auto list_billboards = [&](hipStream_t on) { hipLaunchKernelGGL(sprite_list_kernel, dim3(count), dim3(LIST_THREADS), 0, on, r->dm, *lanes, base, count, sc); };
     const bool aside = r->side_ready && side_stream_pays(count, has_billboards);
     mark();
-    hipLaunchKernelGGL(lane_setup_kernel, dim3((count + 63) / 64), dim3(64), 0, stream, r->dm, *lanes, base, count, sc);
     hipLaunchKernelGGL(lane_tables_kernel, dim3(count), dim3(256), 0, stream, r->dm, *lanes, base, count, sc);
-    if (setup_whole_lanes(count, m.wall_count)) hipLaunchKernelGGL(wall_setup_kernel<true>, dim3(1, count), dim3(SETUP_WHOLE_THREADS), 0, stream, r->dm, count, sc);
+    const bool whole_lanes = setup_whole_lanes(count, m.wall_count);
+    if (whole_lanes) hipLaunchKernelGGL(wall_setup_kernel<true>, dim3(1, count), dim3(SETUP_WHOLE_THREADS), 0, stream, r->dm, count, sc);
     else hipLaunchKernelGGL(wall_setup_kernel<false>, dim3((m.wall_count + SETUP_THREADS - 1) / SETUP_THREADS, count), dim3(SETUP_THREADS), 0, stream, r->dm, count, sc);
     if (m.split_count > 0)
         hipLaunchKernelGGL(fragment_setup_kernel, dim3((m.split_count * m.fragment_slots + 63) / 64, count), dim3(64), 0, stream, r->dm, count, sc);
-    hipLaunchKernelGGL(strip_key_kernel, dim3((count * (SW / 64) + 3) / 4), dim3(256), 0, stream, count, sc);
-    if (sc.spill_slots > 0)
-        hipLaunchKernelGGL(cand_spill_kernel, dim3(sc.spill_slots < SPILL_BLOCKS ? sc.spill_slots : SPILL_BLOCKS), dim3(64), 0, stream, r->dm, sc);
-    hipLaunchKernelGGL(strip_order_kernel, dim3(1), dim3(1024), 0, stream, count * SEGS_PER_LANE, sc);
+    if (!whole_lanes) hipLaunchKernelGGL(strip_key_kernel, dim3((count * (SW / 64) + 3) / 4), dim3(256), 0, stream, count, sc);
+    const int spill_blocks = (sc.spill_slots + 15) / 16;
+    hipLaunchKernelGGL(strip_order_kernel, dim3(1 + (spill_blocks < SPILL_BLOCKS ? spill_blocks : SPILL_BLOCKS)), dim3(1024), 0, stream, r->dm, count * SEGS_PER_LANE, sc);
     mark();
     {
         const int wavefronts = (count * SEGS_PER_LANE + 64 / SEG_COLS - 1) / (64 / SEG_COLS);
