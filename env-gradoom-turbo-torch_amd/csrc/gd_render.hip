@@ -381,6 +381,8 @@ __device__ __forceinline__ i64 tdiv(i64 a, i64 b) {
     const u64 sign = (u64)((a ^ b) >> 63);
     return (i64)((uq ^ sign) - sign);
 }
+// Lanes of one wavefront leave words in memory for one another: the hardware keeps a wavefront's loads and stores of one place in order, the compiler has to.
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 // Lanes of one wavefront leave words in LDS for one another: the order is the program's, the compiler has to keep it.
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -2298,28 +2300,13 @@ __device__ __forceinline__ bool same_state(const ColumnState &a, const ColumnSta
 struct PassColumn {
     int wall, side, render_current, other_sector;
     float distance;
-    i64 visibility;
-    float view_floor, view_ceiling, other_floor, other_ceiling;
-    float clipped_top, clipped_bottom, clipped_upper_bottom, clipped_lower_top;
-    int side_tex[3];
     int ps_path_index, ps_other, no_path_other, sel_vertex, fb_idx;
     float ps_path_distance, no_path_distance;
     int bits, marks;       // PB_*, REC_*
-    // what the drawing half adds (pass_geometry, pass_clip)
-    int render_other;       // the sector behind the drawn side, -1 for none
-    float one_top, one_bottom, lower_top, upper_bottom;              // the four heights' projected rows, not yet clipped
-    i64 u_base, swall;      // texture column before wrapping, texture step (engine.py:12762-12807)
-    float offset_y;         // the side's vertical texture offset
-    float fake_contrast;    // +16 on vertical linedefs, -16 on horizontal ones (engine.py:12853-12861)
 };
 #define PB_VALID 0x1
 #define PB_RASTER 0x2
 #define PB_ONE_SIDED 0x4
-#define PB_TIER0 0x8
-#define PB_TIER1 0x10
-#define PB_TIER2 0x20
-#define PB_MARK_CEILING 0x40
-#define PB_MARK_FLOOR 0x80
 #define PB_PS_KEEPS 0x100
 #define PB_NO_KEEPS 0x200
 #define PB_GEOMETRIC 0x400
@@ -2354,8 +2341,13 @@ __device__ __forceinline__ WallRows wall_rows(const WallGeo &geo, bool back, int
     const HeightBend b0 = geo.bend[first], b1 = geo.bend[first + next], b2 = geo.bend[first + 2 * next], b3 = geo.bend[first + 3 * next];
     const int span0 = geo.span0, span1 = geo.span1;
     WallRows r;
-    r.ceiling = bent_row(height_row(l0, x), b0, x); r.floor = bent_row(height_row(l1, x), b1, x);
-    r.other_floor = bent_row(height_row(l2, x), b2, x); r.other_ceiling = bent_row(height_row(l3, x), b3, x);
+    r.ceiling = height_row(l0, x); r.floor = height_row(l1, x);
+    r.other_floor = height_row(l2, x); r.other_ceiling = height_row(l3, x);
+    // nearly always every height of the linedef is one line over the whole screen
+    if (__any((int)((b0.bottom | b1.bottom | b2.bottom | b3.bottom) >> 31))) {
+        r.ceiling = bent_row(r.ceiling, b0, x); r.floor = bent_row(r.floor, b1, x);
+        r.other_floor = bent_row(r.other_floor, b2, x); r.other_ceiling = bent_row(r.other_ceiling, b3, x);
+    }
     if ((x < span0 || x >= span1) && ((b0.bottom | b1.bottom | b2.bottom | b3.bottom) >> 31)) {
         if (bends(b0)) r.ceiling = height_row(geo.outside[first], x);
         if (bends(b1)) r.floor = height_row(geo.outside[first + next], x);
@@ -2376,41 +2368,130 @@ __device__ __forceinline__ void texture_column(const Ends &ends, bool past_left,
     *u_base = (h + ws.offset_x) >> 16;
 }
 
-// engine.py:12240-12620, 12969-13010: what one column draws of the drawseg a pass selected, as far as it depends on the selection alone
-// and not on the column's clips: the side and sectors drawn from, the wallscan light, the four heights' projected rows, and
-// those of a portal path behind a projected solid.  All of it is read off the lines wall_geometry_kernel left for the linedef
-// (a pass marked REC_OWN_ROWS has its rows in Scratch::pass_rows); `at` is the record's place in the chunk's planes.
 struct WallEnds { int tx0, tx1, ty0, ty1; };
-struct PassTexture { WallEnds ends; bool past_left; WallSide side; };   // what the texture columns of the pass's tiers come from
+// Exchanges inside the aligned groups of four lanes (DPP quads): the value of the group's first lane, and the
+// conjunction, the largest and the smallest of the four.  All four lanes must be executing.
+template <int PATTERN> __device__ __forceinline__ int quad_move(int v) { return __builtin_amdgcn_mov_dpp(v, PATTERN, 0xF, 0xF, true); }
+__device__ __forceinline__ int quad_first(int v) { return quad_move<0x00>(v); }                 // lanes 0,0,0,0
+__device__ __forceinline__ int quad_and(int v) { v &= quad_move<0xB1>(v); return v & quad_move<0x4E>(v); }   // lanes 1,0,3,2 then 2,3,0,1
+__device__ __forceinline__ float quad_max(float v) {
+    v = fmaxf(v, __int_as_float(quad_move<0xB1>(__float_as_int(v))));
+    return fmaxf(v, __int_as_float(quad_move<0x4E>(__float_as_int(v))));
+}
+__device__ __forceinline__ float quad_min(float v) {
+    v = fminf(v, __int_as_float(quad_move<0xB1>(__float_as_int(v))));
+    return fminf(v, __int_as_float(quad_move<0x4E>(__float_as_int(v))));
+}
+
+// What one column draws of the drawseg a pass selected, as far as it depends on the selection alone and not on the column's clips
+// (engine.py:12240-12807, 12969-13010).  A column's lanes prepare as many passes at once, one each, and pass them around (wall_raster_kernel).
+// Of the up to two tiers of a drawseg, `a` is a one-sided drawseg's only one, or the lower one; `b` is the upper one.
+struct PassDraw {
+    unsigned int flags;       // DRAW_*; DRAW_SHADES: the column's own colormap row, then its group's; DRAW_BITS: floor(log2 height) of the tiers' textures
+    unsigned int wall_sector; // the linedef | the sector drawn from << 16 | DRAW_MASKED
+    unsigned int rows;        // the four heights' projected rows, not yet clipped: top, bottom, lower tier's top, upper tier's bottom
+    unsigned int column_a, frac_a, step_a, column_b, frac_b, step_b;   // a tier's texture column in the atlas, its texture row (in the upper bits) at screen row 0, the step from row to row
+    float distance;
+};
+#define DRAW_RASTER 0x1
+#define DRAW_ONE_SIDED 0x2
+#define DRAW_PS_KEEPS 0x4
+#define DRAW_MARK_CEILING 0x8
+#define DRAW_MARK_FLOOR 0x10
+#define DRAW_LOWER 0x20       // the sector behind has the higher floor, or the lower ceiling
+#define DRAW_UPPER 0x40
+#define DRAW_TEXTURE_A 0x80
+#define DRAW_TEXTURE_B 0x100
+#define DRAW_CLIPS_BOTTOM 0x200   // the drawseg leaves a silhouette for the sprites behind it
+#define DRAW_CLIPS_TOP 0x400
+#define DRAW_GROUP 0x800      // the column's group of four draws this side of this linedef
+#define DRAW_SHADES 12        // five bits each from here on
+#define DRAW_BITS 22
+#define DRAW_MASKED 0x20000000u   // a two-sided drawseg with a masked mid-texture (a sector's number has 13 bits: META_SECTOR_MASK)
+static_assert(META_SECTOR_MASK < 1u << 13, "PassDraw packs a flag above the sector");
+
+// A tier's texture row at screen row y is bits 32-height_bits .. 31 of
+//   fraction(y) = (texture_mid << (16 - height_bits)) + ((step * (y * 65536 + 65536 - center)) >> 16).
+// step * y * 65536 has no low 16 bits, so it shifts out of the floor unchanged, and only the low 32 bits of
+// the sum are looked at: they advance by the low 32 bits of step per row, whatever the 64-bit terms wrap to.
+__device__ __forceinline__ void tier_texture(const ColumnCtx &cc, int id, float origin, float offset_y, i64 u_base, i64 swall, unsigned &column, unsigned &frac, unsigned &step, unsigned &bits) {
+    const Tables &tb = *cc.tb;
+    bits = (unsigned)tb.height_bits(id);
+    const i64 step64 = mul64(swall, shl64(1, 14 - (int)bits));
+    const i64 base = shl64(round_to_i64((origin - cc.c->view_z) * 65536.0f + offset_y * 65536.0f), 16 - (int)bits);
+    step = (unsigned)step64;
+    frac = (unsigned)base + mul64_bits_16_47(step64, FIXED_UNIT - cc.c->center_fixed);
+    column = (unsigned)id * (unsigned)(cc.m->tex_max_h * cc.m->tex_max_w) + (unsigned)tb.wrap_column(id, u_base);   // the atlas is below 4 GiB
+}
+
+// All of it is read off the lines wall_geometry_kernel left for the linedef (a pass marked REC_OWN_ROWS has its rows in
+// Scratch::pass_rows); `at` is the record's place in the chunk's planes.  `draws`: the pass draws something; a column without a pass, or one whose pass
+// draws nothing, paints no row and draws no tier.  The whole wavefront comes here.
 template <bool GENERAL>
-__device__ __forceinline__ void pass_geometry(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, const WallGeo &geo, size_t at, int marks, PassColumn &r, PassTexture &texture) {
-    const int x = cc.x, wi = r.wall, side = (marks & REC_SIDE1) ? 1 : 0;
-    texture.side = dm.wall_side[2 * wi + side];
-    texture.ends.tx0 = geo.tx0; texture.ends.tx1 = geo.tx1; texture.ends.ty0 = geo.ty0; texture.ends.ty1 = geo.ty1;
-    texture.past_left = geo.past_left != 0;
-    const ColumnLine visibility = geo.visibility[side];
-    const WallRows rows = wall_rows(geo, side != 0, x);
-    r.side = side; r.render_other = texture.side.other;
-    r.side_tex[0] = texture.side.tex[0]; r.side_tex[1] = texture.side.tex[1]; r.side_tex[2] = texture.side.tex[2];
-    r.visibility = visibility.at(x);
-    if (GENERAL) {   // wallscan light interpolates over the fragment where a linedef has several
-        const WallRec &wr = cc.rec(wi);
-        const FragmentChoice fragment = choose_fragment<true>(cc.m, cc.frags, wr, wi, x);
-        if (fragment.lights) r.visibility = wall_visibility(*fragment.rec, side, x);
+__device__ __forceinline__ PassDraw pass_draw(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, bool draws, const PassRec &rec, unsigned int geo_at, size_t at) {
+    PassDraw d = {};
+    const int x = cc.x;
+    const int side = draws && (rec.marks & REC_SIDE1) ? 1 : 0, wi = draws ? (int)rec.wall : 0;
+    const Tables &tb = *cc.tb;
+    float light = 0.0f;
+    i64 visibility = 0;
+    if (draws) {
+        const WallGeo &geo = sc.geo[geo_at];
+        const WallSide ws = dm.wall_side[2 * wi + side];
+        WallEnds ends;
+        ends.tx0 = geo.tx0; ends.tx1 = geo.tx1; ends.ty0 = geo.ty0; ends.ty1 = geo.ty1;
+        const bool past_left = geo.past_left != 0;
+        const ColumnLine visibility_line = geo.visibility[side];
+        const WallRows rows = wall_rows(geo, side != 0, x);
+        visibility = visibility_line.at(x);
+        if (GENERAL) {   // wallscan light interpolates over the fragment where a linedef has several
+            const WallRec &wr = cc.rec(wi);
+            const FragmentChoice fragment = choose_fragment<true>(cc.m, cc.frags, wr, wi, x);
+            if (fragment.lights) visibility = wall_visibility(*fragment.rec, side, x);
+        }
+        // the sector behind only matters across a two-sided linedef (every use of its heights is behind !one_sided)
+        d.rows = (unsigned)rows.ceiling | ((unsigned)rows.floor << 8) | ((unsigned)rows.other_floor << 16) | ((unsigned)rows.other_ceiling << 24);
+        if (rec.marks & REC_OWN_ROWS) d.rows = sc.pass_rows[at].x;
+        d.distance = rec.distance;
+        const int current = rec.render_current, other = ws.other < 0 ? 0 : ws.other;
+        const bool raster = rec.bits & PB_RASTER, one_sided = rec.bits & PB_ONE_SIDED, masked = !one_sided && ws.tex[0] >= 0;
+        const float view_floor = tb.floor_h(current), view_ceiling = tb.ceil_h(current), other_floor = tb.floor_h(other), other_ceiling = tb.ceil_h(other);
+        const float view_z = cc.c->view_z;
+        light = (tb.light(current) + (float)(cc.c->flash_light * 16)) + ws.contrast;
+        // k. plane marks (engine.py:12621-12636)
+        const bool light_differs = tb.light(current) != tb.light(other);
+        const bool mark_ceiling = one_sided || (view_ceiling != other_ceiling) || (tb.ceil_tex(current) != tb.ceil_tex(other)) || light_differs;
+        const bool mark_floor = one_sided || (view_floor != other_floor) || (tb.floor_tex(current) != tb.floor_tex(other)) || light_differs;
+        const bool lower = !one_sided && view_floor < other_floor, upper = !one_sided && view_ceiling > other_ceiling;
+        const int tex_a = ws.tex[one_sided ? 0 : 1], tex_b = one_sided ? -1 : ws.tex[2];
+        d.wall_sector = (unsigned)wi | ((unsigned)current << 16) | (masked ? DRAW_MASKED : 0u);
+        d.flags = (raster ? DRAW_RASTER : 0) | (one_sided ? DRAW_ONE_SIDED : 0) | ((rec.bits & PB_PS_KEEPS) ? DRAW_PS_KEEPS : 0) | (mark_ceiling ? DRAW_MARK_CEILING : 0) |
+                  (mark_floor ? DRAW_MARK_FLOOR : 0) | (lower ? DRAW_LOWER : 0) | (upper ? DRAW_UPPER : 0) | (tex_a >= 0 ? DRAW_TEXTURE_A : 0) | (tex_b >= 0 ? DRAW_TEXTURE_B : 0) |
+                  // sprite silhouettes (engine.py:12943-12964)
+                  (!one_sided && (view_floor > other_floor || view_z < other_floor || masked) ? DRAW_CLIPS_BOTTOM : 0) |
+                  (!one_sided && (view_ceiling < other_ceiling || view_z > other_ceiling || masked) ? DRAW_CLIPS_TOP : 0);
+        const bool paints_a = raster && tex_a >= 0 && (one_sided || lower), paints_b = raster && tex_b >= 0 && upper;
+        if (paints_a || paints_b) {
+            i64 u_base, swall;
+            texture_column(ends, past_left, ws, side, x, &u_base, &swall);
+            unsigned bits_a = 0, bits_b = 0;
+            if (paints_a) tier_texture(cc, tex_a, one_sided ? view_ceiling : other_floor, ws.offset_y, u_base, swall, d.column_a, d.frac_a, d.step_a, bits_a);
+            if (paints_b) tier_texture(cc, tex_b, other_ceiling, ws.offset_y, u_base, swall, d.column_b, d.frac_b, d.step_b, bits_b);
+            d.flags |= (bits_a | (bits_b << 5)) << DRAW_BITS;
+        }
     }
-    r.one_top = rows.ceiling; r.one_bottom = rows.floor;
-    // the sector behind only matters across a two-sided linedef (every use of its heights is behind !one_sided)
-    r.lower_top = rows.other_floor; r.upper_bottom = rows.other_ceiling;
-    if (marks & REC_OWN_ROWS) {
-        const unsigned int own = sc.pass_rows[at].x;
-        r.one_top = (float)(own & 255u); r.one_bottom = (float)((own >> 8) & 255u);
-        r.lower_top = (float)((own >> 16) & 255u); r.upper_bottom = (float)(own >> 24);
-    }
+    // 4-column wallscan groups (engine.py:12688-12761): the four lanes of a group are one DPP quad, so every exchange is a vector move with
+    // a lane pattern (no trip through the LDS crossbar).  Every lane of the wavefront is active here.
+    const int wall_first = quad_first(wi), side_first = quad_first(side);
+    const bool agrees = quad_and(wi == wall_first && side == side_first ? 1 : 0) != 0;
+    const i64 group_visibility = ((i64)quad_first((int)(visibility >> 32)) << 32) | (i64)(unsigned)quad_first((int)(visibility & 0xFFFFFFFFLL));
+    d.flags |= (agrees ? DRAW_GROUP : 0) | ((unsigned)wall_shade(light, visibility) << DRAW_SHADES) | ((unsigned)wall_shade(light, group_visibility) << (DRAW_SHADES + 5));
+    return d;
 }
 
 // The rows of the portal path behind a projected solid (PB_PS_KEEPS, one pass in a thousand).
-__device__ __forceinline__ WallRows path_rows(const ColumnCtx &cc, const Scratch &sc, size_t at, int marks, const PassColumn &r) {
-    if (!(marks & REC_OWN_ROWS)) return wall_rows(sc.geo[sc.geo_slot[cc.rec_base + (unsigned)r.ps_path_index]], !(r.bits & PB_PS_FROM_FRONT), cc.x);
+__device__ __forceinline__ WallRows path_rows(const ColumnCtx &cc, const Scratch &sc, size_t at, const PassRec &rec) {
+    if (!(rec.marks & REC_OWN_ROWS)) return wall_rows(sc.geo[sc.geo_slot[cc.rec_base + (unsigned)rec.ps_path]], !(rec.bits & PB_PS_FROM_FRONT), cc.x);
     const unsigned int own = sc.pass_rows[at].y;
     WallRows rows;
     rows.ceiling = (float)(own & 255u); rows.floor = (float)((own >> 8) & 255u);
@@ -2418,27 +2499,15 @@ __device__ __forceinline__ WallRows path_rows(const ColumnCtx &cc, const Scratch
     return rows;
 }
 
-// engine.py:12607-12636: the projected rows of pass_geometry against the column's clips, the plane marks and the tiers.
-// r.side and r.render_other come from pass_geometry.
-__device__ __forceinline__ void pass_clip(const ColumnCtx &cc, float ceiling_clip, float floor_clip, PassColumn &r) {
-    const Tables &tb = *cc.tb;
-    const int render_current = r.render_current;
-    const int safe_other = r.render_other < 0 ? 0 : r.render_other;
-    const bool raster_valid = r.bits & PB_RASTER, one_sided = r.bits & PB_ONE_SIDED;
-    r.view_floor = tb.floor_h(render_current); r.view_ceiling = tb.ceil_h(render_current);
-    r.other_floor = tb.floor_h(safe_other); r.other_ceiling = tb.ceil_h(safe_other);
-    r.clipped_top = fmaxf(r.one_top, ceiling_clip);
-    r.clipped_bottom = fminf(r.one_bottom, floor_clip);
-    r.clipped_upper_bottom = fmaxf(fminf(r.upper_bottom, floor_clip), r.clipped_top);
-    r.clipped_lower_top = fminf(fmaxf(r.lower_top, ceiling_clip), r.clipped_bottom);
-    // k. plane marks (engine.py:12621-12636)
-    bool light_differs = tb.light(render_current) != tb.light(safe_other);
-    bool mark_ceiling = one_sided || (r.view_ceiling != r.other_ceiling) || (tb.ceil_tex(render_current) != tb.ceil_tex(safe_other)) || light_differs;
-    bool mark_floor = one_sided || (r.view_floor != r.other_floor) || (tb.floor_tex(render_current) != tb.floor_tex(safe_other)) || light_differs;
-    bool tier0 = one_sided && raster_valid && (r.side_tex[0] >= 0) && (r.clipped_top < r.clipped_bottom);
-    bool tier1 = !one_sided && raster_valid && (r.view_floor < r.other_floor) && (r.side_tex[1] >= 0) && (r.clipped_lower_top < r.clipped_bottom);
-    bool tier2 = !one_sided && raster_valid && (r.view_ceiling > r.other_ceiling) && (r.side_tex[2] >= 0) && (r.clipped_top < r.clipped_upper_bottom);
-    r.bits |= (tier0 ? PB_TIER0 : 0) | (tier1 ? PB_TIER1 : 0) | (tier2 ? PB_TIER2 : 0) | (mark_ceiling ? PB_MARK_CEILING : 0) | (mark_floor ? PB_MARK_FLOOR : 0);
+// engine.py:12607-12620: the projected rows of a pass against the column's clips
+struct PassRows { float top, bottom, upper_bottom, lower_top; };
+__device__ __forceinline__ PassRows clip_pass(const PassDraw &d, float ceiling_clip, float floor_clip) {
+    PassRows r;
+    r.top = fmaxf((float)(d.rows & 255u), ceiling_clip);
+    r.bottom = fminf((float)((d.rows >> 8) & 255u), floor_clip);
+    r.upper_bottom = fmaxf(fminf((float)(d.rows >> 24), floor_clip), r.top);
+    r.lower_top = fminf(fmaxf((float)((d.rows >> 16) & 255u), ceiling_clip), r.bottom);
+    return r;
 }
 
 // engine.py:11769-12239: selection of the pass's drawseg for one column
@@ -2648,7 +2717,7 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
 // waited for the row before (wall_raster_kernel, 4096 lanes on the 4000-linedef map: 1.33 ms with the branches, 1.03 without).
 #define BUFFER_WORDS 0x00027000   // descriptor word 3: 32-bit elements
 #define BUFFER_NOWHERE 0x80000000u   // an offset beyond every plane: 4096 lanes are 1.1 GB
-struct PixelBuffers {
+template <int LANES> struct PixelBuffers {
     unsigned char *frame;   // [L][240][320] or null
     unsigned int *meta;     // [L][208][320]
     unsigned char *masked_texel;   // [L][208][320], used where there is no frame
@@ -2656,10 +2725,15 @@ struct PixelBuffers {
     __amdgpu_buffer_rsrc_t words, depths;   // meta and scene_depth once more, as buffers: see put()
     unsigned word_column;   // byte offset of (lane, row 0, column) in the four-byte planes
     unsigned frame_column;  // and in the frame
+    // A column may have several lanes of its wavefront (wall_raster_kernel): all of them hold the same state, and of the rows of a run
+    // the lane `row_lane` of them takes every row_lanes-th, from the run's `row_lane`-th on.
+    static constexpr int row_lanes = LANES;
+    int row_lane;
+    unsigned put_column;    // word_column, `row_lane` rows further on
     __device__ __forceinline__ unsigned int &m(int y) const { return *reinterpret_cast<unsigned int *>(reinterpret_cast<char *>(meta) + (word_column + (unsigned)y * (SW * 4u))); }
-    // `y` is the same in the whole wavefront
-    __device__ __forceinline__ void put(bool active, int y, unsigned int word) const { __builtin_amdgcn_raw_buffer_store_b32(word, words, active ? word_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
-    __device__ __forceinline__ void put_depth(bool active, int y, float depth) const { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(depth), depths, active ? word_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
+    // into row y + row_lane; `y` is the same in the whole wavefront
+    __device__ __forceinline__ void put(bool active, int y, unsigned int word) const { __builtin_amdgcn_raw_buffer_store_b32(word, words, active ? put_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
+    __device__ __forceinline__ void put_depth(bool active, int y, float depth) const { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(depth), depths, active ? put_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
     __device__ __forceinline__ unsigned char &t(int y) const { return masked_texel[(word_column >> 2) + (unsigned)y * (unsigned)SW]; }
     __device__ __forceinline__ float &s(int y) const { return *reinterpret_cast<float *>(reinterpret_cast<char *>(scene_depth) + (word_column + (unsigned)y * (SW * 4u))); }
     __device__ __forceinline__ unsigned char &f(int y) const { return frame[frame_column + (unsigned)y * (unsigned)SW]; }
@@ -2683,26 +2757,31 @@ __device__ __forceinline__ float clip_distance(const ColumnCtx &cc, int w) {
 
 // Rows [first, last) of one column take `distance` / `wall` as their sprite clip where it is nearer
 // than what they hold.  WALL_ROWS rows at a time, loads first, so the rows' memory latencies overlap.
-__device__ __forceinline__ void clip_rows(const ColumnCtx &cc, PixelBuffers &pb, int first, int last, float distance, int wall) {
+template <typename Pixels>
+__device__ __forceinline__ void clip_rows(const ColumnCtx &cc, Pixels &pb, int first, int last, float distance, int wall) {
     unsigned int held_wall = 0;           // linedef + 1 of the row before and its distance: rows of one clip are neighbours
     float held = GD_INF;                  // no clip recorded yet: infinite
-    for (int y0 = first; y0 < last; y0 += WALL_ROWS) {
+    const int step = pb.row_lanes;
+    wave_fence();                         // the column's other lanes may have written these rows
+    for (int y0 = first + pb.row_lane; y0 < last; y0 += WALL_ROWS * step) {
         unsigned int meta[WALL_ROWS];
 #pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) meta[j] = pb.m(y0 + j < last ? y0 + j : last - 1);
+        for (int j = 0; j < WALL_ROWS; ++j) meta[j] = pb.m(min(y0 + j * step, last - 1));
 #pragma unroll
         for (int j = 0; j < WALL_ROWS; ++j) {
-            if (y0 + j >= last) break;
+            const int y = y0 + j * step;
+            if (y >= last) break;
             const unsigned int row_wall = meta[j] & META_WALL_MASK;
             if (row_wall != held_wall) { held_wall = row_wall; held = row_wall ? clip_distance(cc, (int)row_wall - 1) : GD_INF; }
-            if (distance < held) pb.m(y0 + j) = (meta[j] & ~META_WALL_MASK) | (unsigned)(wall + 1);
+            if (distance < held) pb.m(y) = (meta[j] & ~META_WALL_MASK) | (unsigned)(wall + 1);
         }
     }
 }
 
 // `done_from` / `done_to`: rows [done_from, done_to) already carry this silhouette (pass_paint wrote it with
 // the rows the pass took out of a window nothing had touched); an empty range otherwise.
-__device__ __forceinline__ void apply_silhouette(const ColumnCtx &cc, PixelBuffers &pb, SilhouetteBounds &sb, bool bottom, bool top, float floor_clip, float ceiling_clip, float distance, int wall,
+template <typename Pixels>
+__device__ __forceinline__ void apply_silhouette(const ColumnCtx &cc, Pixels &pb, SilhouetteBounds &sb, bool bottom, bool top, float floor_clip, float ceiling_clip, float distance, int wall,
                                                  int done_from, int done_to) {
     if (bottom) {
         int first = floor_clip <= 0.0f ? 0 : (floor_clip >= (float)VH ? VH : (int)floor_clip);   // clips hold integers
@@ -2722,9 +2801,8 @@ __device__ __forceinline__ void apply_silhouette(const ColumnCtx &cc, PixelBuffe
 
 // May pass_paint write a two-sided pass's sprite silhouettes along with the rows the pass takes out of an untouched
 // window?  Only while its lower and upper tier do not overlap on screen.
-__device__ __forceinline__ bool silhouette_folds(const PassColumn &r) {
-    const bool lower_on = r.view_floor < r.other_floor, upper_on = r.view_ceiling > r.other_ceiling;
-    return !(lower_on && upper_on && r.clipped_lower_top < r.clipped_upper_bottom);
+__device__ __forceinline__ bool silhouette_folds(const PassDraw &d, const PassRows &r) {
+    return (d.flags & (DRAW_LOWER | DRAW_UPPER)) != (DRAW_LOWER | DRAW_UPPER) || !(r.lower_top < r.upper_bottom);
 }
 
 // The meta plane is never cleared between frames.  Instead the traversal keeps every row of its column that lies
@@ -2747,25 +2825,12 @@ struct GapRange {
     __device__ __forceinline__ void set_filled(int lo, int hi) { rows = (rows & 0x0000ffffu) | ((unsigned)lo << 16) | ((unsigned)hi << 24); }
 };
 static_assert(VH < 256, "GapRange packs row numbers into bytes");
-__device__ __forceinline__ void zero_rows(PixelBuffers &pb, GapRange &gaps, int x, int first, int last) {
+template <typename Pixels>
+__device__ __forceinline__ void zero_rows(Pixels &pb, GapRange &gaps, int x, int first, int last) {
     first = first < 0 ? 0 : first; last = last > VH ? VH : last;
     if (first >= last) return;
-    for (int y = first; y < last; ++y) pb.m(y) = 0u;
+    for (int y = first + pb.row_lane; y < last; y += pb.row_lanes) pb.m(y) = 0u;
     gaps.set_zeroed(min(first, gaps.lo()), max(last, gaps.hi()));
-}
-
-// Exchanges inside the aligned groups of four lanes (DPP quads): the value of the group's first lane, and the
-// conjunction, the largest and the smallest of the four.  All four lanes must be executing.
-template <int PATTERN> __device__ __forceinline__ int quad_move(int v) { return __builtin_amdgcn_mov_dpp(v, PATTERN, 0xF, 0xF, true); }
-__device__ __forceinline__ int quad_first(int v) { return quad_move<0x00>(v); }                 // lanes 0,0,0,0
-__device__ __forceinline__ int quad_and(int v) { v &= quad_move<0xB1>(v); return v & quad_move<0x4E>(v); }   // lanes 1,0,3,2 then 2,3,0,1
-__device__ __forceinline__ float quad_max(float v) {
-    v = fmaxf(v, __int_as_float(quad_move<0xB1>(__float_as_int(v))));
-    return fmaxf(v, __int_as_float(quad_move<0x4E>(__float_as_int(v))));
-}
-__device__ __forceinline__ float quad_min(float v) {
-    v = fminf(v, __int_as_float(quad_move<0xB1>(__float_as_int(v))));
-    return fminf(v, __int_as_float(quad_move<0x4E>(__float_as_int(v))));
 }
 
 // engine.py:12637-12884
@@ -2774,51 +2839,46 @@ __device__ __forceinline__ float quad_min(float v) {
 // rows that its own clip update then removes from the window, so the window stays untouched
 // until a one-sided drawseg (which leaves the clips alone) has painted; until then painting
 // needs no reads and visits only the rows it writes.
-template <bool DEPTH>
-__device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnState &c, const PassColumn &r, PixelBuffers &pb,
-                           const bool group_valid[3], const float group_bottom[3], i64 first_group_visibility,
-                           const unsigned char *colormap, bool &window_dirty, GapRange &gaps) {
+template <bool DEPTH, typename Pixels>
+__device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnState &c, const PassDraw &d, const PassRows &r, Pixels &pb,
+                           const bool group_valid[3], const float group_bottom[3], const unsigned char *colormap, bool &window_dirty, GapRange &gaps) {
     // The whole wavefront comes here together, columns with nothing to draw as well: they take part in the walks over the rows.
-    const bool active = (r.bits & PB_RASTER) != 0;
+    const bool active = (d.flags & DRAW_RASTER) != 0;
     const gd_map_desc *m = cc.m;
-    const LaneCtx &L = *cc.c;
-    const int x = cc.x, wi = r.wall, side = r.side;
-    const bool one_sided = r.bits & PB_ONE_SIDED;
-    const float ceiling_plane_bottom = fminf(r.clipped_top, c.floor_clip);
-    const float floor_plane_top = fmaxf(r.clipped_bottom, c.ceiling_clip);
-    const i64 u_base = r.u_base, swall = r.swall;
-    const Tables &tb = *cc.tb;
-    float light = (tb.light(r.render_current) + (float)(L.flash_light * 16)) + r.fake_contrast;
-    const i64 shade_own = wall_shade(light, r.visibility);
-    const i64 shade_group = wall_shade(light, first_group_visibility);
+    const int x = cc.x, wi = (int)(d.wall_sector & 0xFFFFu);
+    const unsigned sector = (d.wall_sector >> 16) & META_SECTOR_MASK;
+    const bool one_sided = d.flags & DRAW_ONE_SIDED, texture_a = d.flags & DRAW_TEXTURE_A, texture_b = d.flags & DRAW_TEXTURE_B;
+    const float ceiling_plane_bottom = fminf(r.top, c.floor_clip);
+    const float floor_plane_top = fmaxf(r.bottom, c.ceiling_clip);
+    const unsigned char *own_shades = colormap + ((d.flags >> DRAW_SHADES) & 31u) * 256, *group_shades = colormap + ((d.flags >> (DRAW_SHADES + 5)) & 31u) * 256;
     // every span of this pass lies inside the open window [ceiling_clip, floor_clip)
     int y0 = c.ceiling_clip <= 0.0f ? 0 : (int)c.ceiling_clip;
     int y1 = c.floor_clip >= (float)VH ? VH : (int)c.floor_clip;
-    const bool lower_on = !one_sided && (r.view_floor < r.other_floor);
-    const bool upper_on = !one_sided && (r.view_ceiling > r.other_ceiling);
+    const bool lower_on = d.flags & DRAW_LOWER, upper_on = d.flags & DRAW_UPPER;
+    // a one-row texture (no bits) must shift everything out of its row: two shifts
+    const unsigned shift_a = 31u - ((d.flags >> DRAW_BITS) & 31u), shift_b = 31u - (d.flags >> (DRAW_BITS + 5));
+    const unsigned atlas_w = (unsigned)m->tex_max_w;
     const bool fresh = active && !window_dirty;
     if (__any(fresh)) {
         // clips and projections hold integers in [0, 208]
-        const unsigned claim = (unsigned)(r.render_current + 1) << META_SECTOR_SHIFT;
+        const unsigned claim = (sector + 1u) << META_SECTOR_SHIFT;
         // The sprite silhouettes of a two-sided drawseg (engine.py:12943-12964) give every row that this pass
         // takes out of the window the pass's own (distance, linedef) as sprite clip.  Those rows are untouched
         // so far, so what this pass writes there carries the clip along and pass_advance need not revisit them:
         // tier rows hold it anyway, plane rows get it with their claim, rows left bare get it alone.
         // (Not where the lower and the upper tier overlap, a closed door say: a row of both that the lower tier
         // leaves undrawn for want of a texture would be missed.  silhouette_folds() is asked here and there.)
-        const bool masked_texture = r.side_tex[0] >= 0;
-        const bool folds = !one_sided && silhouette_folds(r);
-        const bool sil_bottom = folds && ((r.view_floor > r.other_floor) || (L.view_z < r.other_floor) || masked_texture);
-        const bool sil_top = folds && ((r.view_ceiling < r.other_ceiling) || (L.view_z > r.other_ceiling) || masked_texture);
+        const bool folds = !one_sided && silhouette_folds(d, r);
+        const bool sil_bottom = folds && (d.flags & DRAW_CLIPS_BOTTOM), sil_top = folds && (d.flags & DRAW_CLIPS_TOP);
         const unsigned clip_word = (unsigned)(wi + 1);
         int ceiling_rows_end = 0; bool ceiling_claims = false;
         auto walk = [&](int first, int last, unsigned int word) {
             const unsigned rows = (unsigned)max(last - first, 0);
-            for (int y = wave_min(first), wave_last = wave_max(last); y < wave_last; ++y) pb.put((unsigned)(y - first) < rows, y, word);
+            for (int y = wave_min(first), wave_last = wave_max(last); y < wave_last; y += pb.row_lanes) pb.put((unsigned)(y + pb.row_lane - first) < rows, y, word);
         };
         {
-            const bool claims = r.bits & PB_MARK_CEILING;
-            const bool bare = !claims && sil_top && upper_on && (r.side_tex[2] >= 0);   // the upper tier lowers the clip past these rows
+            const bool claims = d.flags & DRAW_MARK_CEILING;
+            const bool bare = !claims && sil_top && upper_on && texture_b;   // the upper tier lowers the clip past these rows
             // The wavefront walks the rows together, each column writing where its own range has the row: neighbouring
             // columns then store to neighbouring words, where loops that start at each column's own first row would
             // scatter every store over as many rows as the edges' slopes spread them.
@@ -2829,8 +2889,8 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
             ceiling_rows_end = last; ceiling_claims = claims;
         }
         {
-            const bool claims = r.bits & PB_MARK_FLOOR;
-            const bool bare = !claims && sil_bottom && lower_on && (r.side_tex[1] >= 0);   // the lower tier raises the clip past these rows
+            const bool claims = d.flags & DRAW_MARK_FLOOR;
+            const bool bare = !claims && sil_bottom && lower_on && texture_a;   // the lower tier raises the clip past these rows
             const bool writes = fresh && (claims || bare);
             const int first = writes ? max((int)floor_plane_top, 0) : VH, last = writes ? y1 : 0;
             const unsigned word = (claims ? (claim | META_FLOOR) : 0u) | (sil_bottom ? clip_word : 0u);
@@ -2841,28 +2901,19 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
             if (__any(first < ceiling_rows_end)) {
                 const int both_end = min(last, ceiling_rows_end);
                 const unsigned both = (claims ? (claim | META_FLOOR) : (ceiling_claims ? claim : 0u)) | ((sil_top || sil_bottom) ? clip_word : 0u);
-                for (int y = first; y < both_end; ++y) {
-                    pb.m(y) = both;
-                }
+                for (int y = first + pb.row_lane; y < both_end; y += pb.row_lanes) pb.m(y) = both;
             }
         }
         // Rows that leave the window without being written: those the upper tier covers but that belong to a lower
         // tier without a texture (the lower tier has the say there), and a one-sided drawseg's own rows when it has none.
-        if (fresh && lower_on && upper_on && r.side_tex[1] < 0 && r.side_tex[2] >= 0)
-            zero_rows(pb, gaps, x, max((int)r.clipped_top, (int)r.clipped_lower_top), min((int)r.clipped_upper_bottom, (int)r.clipped_bottom));
-        if (fresh && one_sided && r.side_tex[0] < 0) zero_rows(pb, gaps, x, max((int)r.clipped_top, y0), min((int)r.clipped_bottom, y1));
+        if (fresh && lower_on && upper_on && !texture_a && texture_b)
+            zero_rows(pb, gaps, x, max((int)r.top, (int)r.lower_top), min((int)r.upper_bottom, (int)r.bottom));
+        if (fresh && one_sided && !texture_a) zero_rows(pb, gaps, x, max((int)r.top, y0), min((int)r.bottom, y1));
         int t0 = VH, t1 = 0;
-        if (one_sided) { t0 = (int)r.clipped_top; t1 = (int)r.clipped_bottom; }
-        if (lower_on) { t0 = min(t0, (int)r.clipped_lower_top); t1 = max(t1, (int)r.clipped_bottom); }
-        if (upper_on) { t0 = min(t0, (int)r.clipped_top); t1 = max(t1, (int)r.clipped_upper_bottom); }
-        // The texture row of screen row y is bits 32-height_bits .. 31 of
-        //   fraction(y) = (texture_mid << (16 - height_bits)) + ((step * (y * 65536 + 65536 - center)) >> 16).
-        // step * y * 65536 has no low 16 bits, so it shifts out of the floor unchanged, and only the low 32 bits of
-        // the sum are looked at: they advance by the low 32 bits of step per row, whatever the 64-bit terms wrap to.
-        const float toff_y = r.offset_y * 65536.0f;
-        const unsigned atlas_w = (unsigned)m->tex_max_w;
-        const int side_tex0 = r.side_tex[0], side_tex1 = r.side_tex[1], side_tex2 = r.side_tex[2];
-        const bool tiers_overlap = lower_on && upper_on && r.clipped_lower_top < r.clipped_upper_bottom;
+        if (one_sided) { t0 = (int)r.top; t1 = (int)r.bottom; }
+        if (lower_on) { t0 = min(t0, (int)r.lower_top); t1 = max(t1, (int)r.bottom); }
+        if (upper_on) { t0 = min(t0, (int)r.top); t1 = max(t1, (int)r.upper_bottom); }
+        const bool tiers_overlap = lower_on && upper_on && r.lower_top < r.upper_bottom;
         {
             // The usual case: the rows of a tier are one run, [top, bottom) of a one-sided drawseg, or the upper tier
             // above the lower one.  Each run is painted by a loop that knows its texture, so a row costs an add, a
@@ -2877,44 +2928,41 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
 #pragma unroll 1
             for (int run = 0; run < 2; ++run) {   // one copy of the loop: the kernel is larger than the instruction cache as it is
                 const bool second = run != 0;
-                const int texture = second ? side_tex1 : (one_sided ? side_tex0 : side_tex2);
-                int first = (int)(second ? r.clipped_lower_top : r.clipped_top), last = (int)(second || one_sided ? r.clipped_bottom : r.clipped_upper_bottom);
-                const bool paints = runs && (second ? lower_on : one_sided || upper_on) && texture >= 0 && first < last;
+                const bool tier_a = second || one_sided;
+                int first = (int)(second ? r.lower_top : r.top), last = (int)(tier_a ? r.bottom : r.upper_bottom);
+                const bool paints = runs && (second ? lower_on : one_sided || upper_on) && (tier_a ? texture_a : texture_b) && first < last;
                 if (!__any(paints)) continue;
                 first = paints ? first : VH; last = paints ? last : 0;
-                const float origin = second ? r.other_floor : (one_sided ? r.view_ceiling : r.other_ceiling);
                 const bool has_tail = second ? group_valid[1] : (one_sided ? group_valid[0] : group_valid[2]);
                 const float tail_from = second ? group_bottom[1] : (one_sided ? group_bottom[0] : group_bottom[2]);
-                const int id = paints ? texture : 0;
-                const int bits = tb.height_bits(id);
-                const i64 step64 = mul64(swall, shl64(1, 14 - bits));
-                const i64 base = shl64(round_to_i64((origin - L.view_z) * 65536.0f + toff_y), 16 - bits);
-                const unsigned shift = (unsigned)(31 - bits);   // a one-row texture (bits == 0) must shift everything out: two shifts
-                const unsigned step = (unsigned)step64;
+                const unsigned shift = tier_a ? shift_a : shift_b, step = tier_a ? d.step_a : d.step_b;
                 const int wave_first = wave_min(first), wave_last = wave_max(last);
-                unsigned frac = (unsigned)base + mul64_bits_16_47(step64, FIXED_UNIT - L.center_fixed) + step * (unsigned)wave_first;
-                // every texel asked for is the texture's own, whatever the row: the loads need no branch either
-                const unsigned column = (unsigned)id * (unsigned)(m->tex_max_h * m->tex_max_w) + (unsigned)(paints ? tb.wrap_column(id, u_base) : 0);   // the atlas is below 4 GiB
+                const int stride = pb.row_lanes;
+                unsigned frac = (tier_a ? d.frac_a : d.frac_b) + step * (unsigned)(wave_first + pb.row_lane);
+                const unsigned advance = step * (unsigned)stride;
+                // every texel asked for is the texture's own, whatever the row: the loads need no branch either.  (Of a tier that is not
+                // there: the first texel of the atlas.)
+                const unsigned column = tier_a ? d.column_a : d.column_b;
                 // rows from tail_row on take the group's shade: (float)y >= tail_from, which no row meets if that is not a number
                 const int tail_row = !has_tail || !(tail_from < (float)VH) ? VH : (tail_from <= 0.0f ? 0 : (int)ceilf(tail_from));
                 const unsigned meta_word = META_FILLED | (unsigned)(wi + 1), rows = (unsigned)max(last - first, 0);
-                const unsigned char *own_shades = colormap + shade_own * 256, *group_shades = colormap + shade_group * 256;
                 auto load_rows = [&](unsigned char (&texel)[WALL_ROWS]) {
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) { texel[j] = m->tex_atlas[column + __umul24((frac >> shift) >> 1, atlas_w)]; frac += step; }
+                    for (int j = 0; j < WALL_ROWS; ++j) { texel[j] = m->tex_atlas[column + __umul24((frac >> shift) >> 1, atlas_w)]; frac += advance; }
                 };
                 unsigned char texel[WALL_ROWS];
                 load_rows(texel);
-                for (int yb = wave_first; yb < wave_last; yb += WALL_ROWS) {
+                for (int yb = wave_first; yb < wave_last; yb += WALL_ROWS * stride) {
+                    const int y = yb + pb.row_lane;
                     unsigned char next_texel[WALL_ROWS]; unsigned colour[WALL_ROWS];
                     load_rows(next_texel);
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) colour[j] = (yb + j >= tail_row ? group_shades : own_shades)[texel[j]];
+                    for (int j = 0; j < WALL_ROWS; ++j) colour[j] = (y + j * stride >= tail_row ? group_shades : own_shades)[texel[j]];
 #pragma unroll
                     for (int j = 0; j < WALL_ROWS; ++j) {
-                        const bool own = (unsigned)(yb + j - first) < rows;
-                        if (DEPTH) pb.put_depth(own, yb + j, r.distance);
-                        pb.put(own, yb + j, meta_word | (colour[j] << META_SECTOR_SHIFT));
+                        const bool own = (unsigned)(y + j * stride - first) < rows;
+                        if (DEPTH) pb.put_depth(own, yb + j * stride, d.distance);
+                        pb.put(own, yb + j * stride, meta_word | (colour[j] << META_SECTOR_SHIFT));
                     }
 #pragma unroll
                     for (int j = 0; j < WALL_ROWS; ++j) texel[j] = next_texel[j];
@@ -2923,20 +2971,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
         }
         if (fresh && tiers_overlap) {
             // The lower and the upper tier share rows (a closed door, say): the lower tier has the say there, row by row.
-                int tier_tex[3]; unsigned tier_frac[3], tier_step[3], tier_shift[3]; size_t tier_texel[3];
-            const float tier_origin[3] = {r.view_ceiling, r.other_floor, r.other_ceiling};
-#pragma unroll
-            for (int t = 0; t < 3; ++t) {
-                tier_tex[t] = r.side_tex[t];
-                const int id = tier_tex[t] < 0 ? 0 : tier_tex[t];
-                const int bits = tb.height_bits(id);
-                const i64 step = mul64(swall, shl64(1, 14 - bits));
-                const i64 base = shl64(round_to_i64((tier_origin[t] - L.view_z) * 65536.0f + toff_y), 16 - bits);
-                tier_shift[t] = (unsigned)(31 - bits);   // a one-row texture (bits == 0) must shift everything out: two shifts
-                tier_step[t] = (unsigned)step;
-                tier_frac[t] = (unsigned)(base + (mul64(step, FIXED_UNIT - L.center_fixed) >> 16)) + (unsigned)step * (unsigned)t0;
-                tier_texel[t] = (size_t)id * m->tex_max_h * m->tex_max_w + (size_t)tb.wrap_column(id, u_base);
-            }
+            unsigned frac_a = d.frac_a + d.step_a * (unsigned)t0, frac_b = d.frac_b + d.step_b * (unsigned)t0;
             // WALL_ROWS rows at a time, one batch ahead: the texels of the next batch are asked for before the rows of
             // this one are stored, so that a step waits for memory once, not for its stores and then for its loads
             auto load_rows = [&](int yb, unsigned char (&texel)[WALL_ROWS], unsigned &draw, unsigned &tail) {
@@ -2945,22 +2980,18 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 for (int j = 0; j < WALL_ROWS; ++j) {
                     const int y = yb + j;
                     const float py = (float)y;
-                    const bool one_span = one_sided && (py >= r.clipped_top) && (py < r.clipped_bottom);
-                    const bool lower_span = lower_on && (py >= r.clipped_lower_top) && (py < r.clipped_bottom);
-                    const bool upper_span = upper_on && (py >= r.clipped_top) && (py < r.clipped_upper_bottom);
-                    const int t = one_span ? 0 : (lower_span ? 1 : 2);
-                    const bool draws = y < t1 && (one_span || lower_span || upper_span) && tier_tex[t] >= 0;
+                    const bool lower_span = (py >= r.lower_top) && (py < r.bottom);
+                    const bool upper_span = (py >= r.top) && (py < r.upper_bottom);
+                    const bool draws = y < t1 && (lower_span ? texture_a : upper_span && texture_b);
                     if (draws) draw |= 1u << j;
                     // rows that both tiers cover take the group's shade if either tier's common bottom has been passed
-                    if ((one_span && group_valid[0] && py >= group_bottom[0]) || (lower_span && group_valid[1] && py >= group_bottom[1]) ||
-                        (upper_span && group_valid[2] && py >= group_bottom[2])) tail |= 1u << j;
+                    if ((lower_span && group_valid[1] && py >= group_bottom[1]) || (upper_span && group_valid[2] && py >= group_bottom[2])) tail |= 1u << j;
                     texel[j] = 0;
                     if (draws) {
-                        const unsigned tv = (tier_frac[t] >> tier_shift[t]) >> 1;
-                        texel[j] = m->tex_atlas[tier_texel[t] + __umul24(tv, atlas_w)];
+                        const unsigned tv = ((lower_span ? frac_a >> shift_a : frac_b >> shift_b) >> 1);
+                        texel[j] = m->tex_atlas[(lower_span ? d.column_a : d.column_b) + __umul24(tv, atlas_w)];
                     }
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) tier_frac[k] += tier_step[k];
+                    frac_a += d.step_a; frac_b += d.step_b;
                 }
             };
             unsigned char texel[WALL_ROWS]; unsigned draw = 0, tail = 0;
@@ -2973,8 +3004,8 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
 #pragma unroll
                 for (int j = 0; j < WALL_ROWS; ++j) {
                     if (!(draw & (1u << j))) continue;
-                    const unsigned colour = colormap[((tail & (1u << j)) ? shade_group : shade_own) * 256 + texel[j]];
-                    if (DEPTH) pb.s(yb + j) = r.distance;
+                    const unsigned colour = ((tail & (1u << j)) ? group_shades : own_shades)[texel[j]];
+                    if (DEPTH) pb.s(yb + j) = d.distance;
                     pb.m(yb + j) = META_FILLED | (colour << META_SECTOR_SHIFT) | (unsigned)(wi + 1);
                 }
 #pragma unroll
@@ -2984,7 +3015,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
         }
         if (fresh && one_sided) {
             window_dirty = true;
-            if (r.side_tex[0] >= 0 && t0 < t1) gaps.set_filled(max(t0, 0), min(t1, VH));   // every row of [t0, t1) was drawn just now
+            if (texture_a && t0 < t1) gaps.set_filled(max(t0, 0), min(t1, VH));   // every row of [t0, t1) was drawn just now
         }
     }
     if (!active || fresh) return;
@@ -2994,51 +3025,42 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
     // this column had to zero.  Only those rows are visited (usually none).  Few columns come here (one pass in 300 on the
     // 4000-linedef map) but every eighth wavefront pass has one, so the loop is kept plain and light on registers.
     int lo = VH, hi = 0;
-    if (one_sided) { lo = (int)r.clipped_top; hi = (int)r.clipped_bottom; }
-    if (lower_on) { lo = min(lo, (int)r.clipped_lower_top); hi = max(hi, (int)r.clipped_bottom); }
-    if (upper_on) { lo = min(lo, (int)r.clipped_top); hi = max(hi, (int)r.clipped_upper_bottom); }
+    if (one_sided) { lo = (int)r.top; hi = (int)r.bottom; }
+    if (lower_on) { lo = min(lo, (int)r.lower_top); hi = max(hi, (int)r.bottom); }
+    if (upper_on) { lo = min(lo, (int)r.top); hi = max(hi, (int)r.upper_bottom); }
     if (gaps.lo() < gaps.hi()) { lo = min(lo, gaps.lo()); hi = max(hi, gaps.hi()); }
     lo = max(lo, y0); hi = min(hi, y1);
     const int filled_lo = gaps.filled_lo(), filled_hi = gaps.filled_hi();
-    // copies taken by value: a choice between members of `r` made per row would be a choice between addresses and
-    // would keep the whole record in private memory
-    const int side_tex0 = r.side_tex[0], side_tex1 = r.side_tex[1], side_tex2 = r.side_tex[2];
-    const float origin0 = r.view_ceiling, origin1 = r.other_floor, origin2 = r.other_ceiling;
     const bool tail0 = group_valid[0], tail1 = group_valid[1], tail2 = group_valid[2];
     const float tail_row0 = group_bottom[0], tail_row1 = group_bottom[1], tail_row2 = group_bottom[2];
-    for (int y = lo; y < hi; ++y) {
-        if (y >= filled_lo && y < filled_hi) { y = filled_hi - 1; continue; }   // tier pixels already: nothing to add
+    wave_fence();                         // the column's other lanes may have written these rows
+    for (int y = lo + pb.row_lane; y < hi; y += pb.row_lanes) {
+        if (y >= filled_lo && y < filled_hi) { y += (filled_hi - 1 - y) & -pb.row_lanes; continue; }   // tier pixels already: nothing to add
         const float py = (float)y;
         unsigned int meta = pb.m(y);
-        bool ceiling_span = (r.bits & PB_MARK_CEILING) && (py >= c.ceiling_clip) && (py < ceiling_plane_bottom);
-        bool floor_span = (r.bits & PB_MARK_FLOOR) && (py >= floor_plane_top) && (py < c.floor_clip);
+        bool ceiling_span = (d.flags & DRAW_MARK_CEILING) && (py >= c.ceiling_clip) && (py < ceiling_plane_bottom);
+        bool floor_span = (d.flags & DRAW_MARK_FLOOR) && (py >= floor_plane_top) && (py < c.floor_clip);
         bool meta_dirty = false;
         if (!(meta & META_FILLED) && ((meta >> META_SECTOR_SHIFT) & META_SECTOR_MASK) == 0 && (ceiling_span || floor_span)) {
-            meta |= ((unsigned)(r.render_current + 1) << META_SECTOR_SHIFT) | (floor_span ? META_FLOOR : 0);
+            meta |= ((sector + 1u) << META_SECTOR_SHIFT) | (floor_span ? META_FLOOR : 0);
             meta_dirty = true;
         }
-        bool one_span = one_sided && (py >= r.clipped_top) && (py < r.clipped_bottom);
-        bool lower_span = lower_on && (py >= r.clipped_lower_top) && (py < r.clipped_bottom);
-        bool upper_span = upper_on && (py >= r.clipped_top) && (py < r.clipped_upper_bottom);
+        bool one_span = one_sided && (py >= r.top) && (py < r.bottom);
+        bool lower_span = lower_on && (py >= r.lower_top) && (py < r.bottom);
+        bool upper_span = upper_on && (py >= r.top) && (py < r.upper_bottom);
         if (one_span || lower_span || upper_span) {
-            int texture_id = one_span ? side_tex0 : (lower_span ? side_tex1 : side_tex2);
-            if (texture_id >= 0 && !(meta & META_FILLED)) {
+            const bool tier_a = one_span || lower_span;
+            if ((tier_a ? texture_a : texture_b) && !(meta & META_FILLED)) {
                 bool bottom_tail = (one_span && tail0 && py >= tail_row0) ||
                                    (lower_span && tail1 && py >= tail_row1) ||
                                    (upper_span && tail2 && py >= tail_row2);
-                i64 tu = tb.wrap_column(texture_id, u_base);
-                float origin_z = one_span ? origin0 : (lower_span ? origin1 : origin2);
-                int height_bits = tb.height_bits(texture_id);
-                i64 vertical_step = mul64(swall, shl64(1, 14 - height_bits));
-                i64 screen_delta = (i64)y * FIXED_UNIT - L.center_fixed + FIXED_UNIT;
-                i64 texture_mid = round_to_i64((origin_z - L.view_z) * 65536.0f + r.offset_y * 65536.0f);
-                i64 fraction = shl64(texture_mid, 16 - height_bits) + (mul64(vertical_step, screen_delta) >> 16);
-                i64 tv = (fraction & UINT32_MASK) >> (32 - height_bits);
-                unsigned char texel = m->tex_atlas[((size_t)texture_id * m->tex_max_h + tv) * m->tex_max_w + tu];
-                const unsigned colour = colormap[(bottom_tail ? shade_group : shade_own) * 256 + texel];
-                if (DEPTH) pb.s(y) = r.distance;
+                const unsigned fraction = (tier_a ? d.frac_a : d.frac_b) + (tier_a ? d.step_a : d.step_b) * (unsigned)y;
+                const unsigned tv = (fraction >> (tier_a ? shift_a : shift_b)) >> 1;
+                unsigned char texel = m->tex_atlas[(tier_a ? d.column_a : d.column_b) + __umul24(tv, atlas_w)];
+                const unsigned colour = (bottom_tail ? group_shades : own_shades)[texel];
+                if (DEPTH) pb.s(y) = d.distance;
                 const float held = (meta & META_WALL_MASK) ? clip_distance(cc, (int)(meta & META_WALL_MASK) - 1) : GD_INF;   // no clip recorded yet
-                if (r.distance < held) { meta = (meta & ~META_WALL_MASK) | (unsigned)(wi + 1); }
+                if (d.distance < held) { meta = (meta & ~META_WALL_MASK) | (unsigned)(wi + 1); }
                 meta = (meta & ~(META_SECTOR_MASK << META_SECTOR_SHIFT)) | (colour << META_SECTOR_SHIFT) | META_FILLED;
                 meta_dirty = true;
             }
@@ -3047,46 +3069,31 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
     }
 }
 
-// engine.py:12885-13371.  PART: ADVANCE_ALL, or only the column's clips, masked-drawseg snapshot and sprite silhouettes
-// (ADVANCE_CLIPS: what needs the projected rows and touches pixels), or only the traversal state (ADVANCE_STATE: next
-// sector, previous distance, pending boundaries; it reads neither rows nor clips).
-#define ADVANCE_ALL 0
-#define ADVANCE_STATE 1
-#define ADVANCE_CLIPS 2
-template <bool SPLIT, int PART>
-__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c, const PassColumn &r, PixelBuffers &pb, SilhouetteBounds &sb, bool window_untouched, GapRange &gaps,
-                             const Scratch *sc = nullptr, size_t at = 0) {   // the pass's place in the chunk's planes, for the clips
+// engine.py:12885-13069: what a pass does to its column's clips, its masked drawseg snapshot and its sprite silhouettes
+template <typename Pixels>
+__device__ __forceinline__ void advance_clips(const ColumnCtx &cc, ColumnState &c, const PassDraw &d, const PassRows &r, Pixels &pb, SilhouetteBounds &sb, bool window_untouched, GapRange &gaps,
+                              const Scratch &sc, size_t at) {   // the pass's place in the chunk's planes
     const gd_map_desc *m = cc.m;
-    const MapView &mv = cc.mv;
     const LaneCtx &L = *cc.c;
     const ColumnState before = c;
-    const int x = cc.x;
-    const int cs = c.current_sector;
-    const int cur = cs < 0 ? 0 : cs;
-    const int wi = r.wall;
-    const float distance = r.distance;
-    const bool valid = r.bits & PB_VALID, raster_valid = r.bits & PB_RASTER, one_sided = r.bits & PB_ONE_SIDED;
-    auto incident = [&](int w) { return mv.sec(w, 0) == cur || mv.sec(w, 1) == cur; };
-  if (PART != ADVANCE_STATE) {
-    // o. clip updates (engine.py:12888-12913)
-    bool draws_upper = (r.view_ceiling > r.other_ceiling) && (r.side_tex[2] >= 0);
-    if (raster_valid && !one_sided && (draws_upper || (r.bits & PB_MARK_CEILING))) c.ceiling_clip = draws_upper ? r.clipped_upper_bottom : r.clipped_top;
-    bool draws_lower = (r.view_floor < r.other_floor) && (r.side_tex[1] >= 0);
-    if (raster_valid && !one_sided && (draws_lower || (r.bits & PB_MARK_FLOOR))) c.floor_clip = draws_lower ? r.clipped_lower_top : r.clipped_bottom;
-    // p. masked drawseg snapshot (engine.py:12914-12939)
-    if (raster_valid && !one_sided && (r.side_tex[0] >= 0) && (distance < c.masked_distance)) {
-        c.masked_ceiling_clip = c.ceiling_clip; c.masked_floor_clip = c.floor_clip; c.masked_distance = distance; c.masked_wall = wi;
-    }
-    // q. sprite silhouettes (engine.py:12943-12964)
-    if (raster_valid && !one_sided) {
-        bool masked_texture = r.side_tex[0] >= 0;
-        bool bottom_sil = (r.view_floor > r.other_floor) || (L.view_z < r.other_floor) || masked_texture;
-        bool top_sil = (r.view_ceiling < r.other_ceiling) || (L.view_z > r.other_ceiling) || masked_texture;
+    const int x = cc.x, wi = (int)(d.wall_sector & 0xFFFFu);
+    const float distance = d.distance;
+    auto row_of = [](float clip) { return clip <= 0.0f ? 0 : (clip >= (float)VH ? VH : (int)clip); };
+    if ((d.flags & (DRAW_RASTER | DRAW_ONE_SIDED)) == DRAW_RASTER) {
+        // o. clip updates (engine.py:12888-12913)
+        const bool draws_upper = (d.flags & (DRAW_UPPER | DRAW_TEXTURE_B)) == (DRAW_UPPER | DRAW_TEXTURE_B), draws_lower = (d.flags & (DRAW_LOWER | DRAW_TEXTURE_A)) == (DRAW_LOWER | DRAW_TEXTURE_A);
+        if (draws_upper || (d.flags & DRAW_MARK_CEILING)) c.ceiling_clip = draws_upper ? r.upper_bottom : r.top;
+        if (draws_lower || (d.flags & DRAW_MARK_FLOOR)) c.floor_clip = draws_lower ? r.lower_top : r.bottom;
+        // p. masked drawseg snapshot (engine.py:12914-12939)
+        if ((d.wall_sector & DRAW_MASKED) && distance < c.masked_distance) {
+            c.masked_ceiling_clip = c.ceiling_clip; c.masked_floor_clip = c.floor_clip; c.masked_distance = distance; c.masked_wall = wi;
+        }
+        // q. sprite silhouettes (engine.py:12943-12964)
+        const bool bottom_sil = d.flags & DRAW_CLIPS_BOTTOM, top_sil = d.flags & DRAW_CLIPS_TOP;
         // pass_paint, finding the window untouched, has written the silhouette into the rows that this pass took out
         // of it: [new floor clip, old floor clip) at the bottom, [old ceiling clip, new ceiling clip) at the top
-        auto row_of = [](float clip) { return clip <= 0.0f ? 0 : (clip >= (float)VH ? VH : (int)clip); };
         const int old_floor = row_of(before.floor_clip), old_ceiling = row_of(before.ceiling_clip);
-        if (window_untouched && silhouette_folds(r)) {
+        if (window_untouched && silhouette_folds(d, r)) {
             // one call per side: the rows already done differ.  pass_paint stays inside the old window, and a sector whose
             // ceiling lies below its floor can carry a clip past the window's other end: then the rows beyond that end
             // are not done, and the range is cut there (apply_silhouette then takes no short cut and visits them all).
@@ -3097,43 +3104,58 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c
         }
     }
     // r. clips of the geometric portal behind a projected solid (engine.py:12969-13069)
-    if (r.bits & PB_PS_KEEPS) {
-        int path = r.ps_path_index;
-        int path_safe_other = r.ps_other < 0 ? 0 : r.ps_other;
+    if (d.flags & DRAW_PS_KEEPS) {
+        const PassRec rec = sc.pass_rec[at];
+        const int path = rec.ps_path, current = rec.render_current;
+        const int path_safe_other = rec.ps_other < 0 ? 0 : rec.ps_other;
         const Tables &tb = *cc.tb;
+        const float view_floor = tb.floor_h(current), view_ceiling = tb.ceil_h(current);
         float pof = tb.floor_h(path_safe_other), poc = tb.ceil_h(path_safe_other);
-        int pside = (r.bits & PB_PS_FROM_FRONT) ? 0 : 1;
+        int pside = (rec.bits & PB_PS_FROM_FRONT) ? 0 : 1;
         const int *ptex = m->side_tex + (path * 2 + pside) * 3;
-        const WallRows rows = path_rows(cc, *sc, at, r.marks, r);
-        const float path_distance = sc->pass_path_distance[at];
+        const WallRows rows = path_rows(cc, sc, at, rec);
+        const float path_distance = sc.pass_path_distance[at];
         float pct = fmaxf(rows.ceiling, c.ceiling_clip);
         float pcb = fminf(rows.floor, c.floor_clip);
         float pcub = fmaxf(fminf(rows.other_ceiling, c.floor_clip), pct);
         float pclt = fminf(fmaxf(rows.other_floor, c.ceiling_clip), pcb);
-        bool light_differs = tb.light(r.render_current) != tb.light(path_safe_other);
-        bool p_draws_upper = (r.view_ceiling > poc) && (ptex[2] >= 0);
-        bool p_marks_ceiling = (r.view_ceiling != poc) || (tb.ceil_tex(r.render_current) != tb.ceil_tex(path_safe_other)) || light_differs;
-        bool p_draws_lower = (r.view_floor < pof) && (ptex[1] >= 0);
-        bool p_marks_floor = (r.view_floor != pof) || (tb.floor_tex(r.render_current) != tb.floor_tex(path_safe_other)) || light_differs;
+        bool light_differs = tb.light(current) != tb.light(path_safe_other);
+        bool p_draws_upper = (view_ceiling > poc) && (ptex[2] >= 0);
+        bool p_marks_ceiling = (view_ceiling != poc) || (tb.ceil_tex(current) != tb.ceil_tex(path_safe_other)) || light_differs;
+        bool p_draws_lower = (view_floor < pof) && (ptex[1] >= 0);
+        bool p_marks_floor = (view_floor != pof) || (tb.floor_tex(current) != tb.floor_tex(path_safe_other)) || light_differs;
         float new_ceiling = c.ceiling_clip, new_floor = c.floor_clip;
         if (p_draws_upper || p_marks_ceiling) new_ceiling = p_draws_upper ? pcub : pct;
         if (p_draws_lower || p_marks_floor) new_floor = p_draws_lower ? pclt : pcb;
         if (window_untouched) {
             // These clips move without anything being painted or claimed: the rows they take out of an untouched
             // window would leave it unwritten.  They show the flat pass's picture.
-            auto row_of = [](float clip) { return clip <= 0.0f ? 0 : (clip >= (float)VH ? VH : (int)clip); };
             const int window_top = row_of(c.ceiling_clip), window_bottom = row_of(c.floor_clip);
             zero_rows(pb, gaps, x, window_top, min(row_of(new_ceiling), window_bottom));
             zero_rows(pb, gaps, x, max(row_of(new_floor), window_top), window_bottom);
         }
         c.ceiling_clip = new_ceiling; c.floor_clip = new_floor;
         bool pmasked = ptex[0] >= 0;
-        bool pbottom = (r.view_floor > pof) || (L.view_z < pof) || pmasked;
-        bool ptop = (r.view_ceiling < poc) || (L.view_z > poc) || pmasked;
+        bool pbottom = (view_floor > pof) || (L.view_z < pof) || pmasked;
+        bool ptop = (view_ceiling < poc) || (L.view_z > poc) || pmasked;
         apply_silhouette(cc, pb, sb, pbottom, ptop, c.floor_clip, c.ceiling_clip, path_distance, path, 0, 0);
     }
-  }
-    if (PART == ADVANCE_CLIPS) return false;
+}
+
+// engine.py:13070-13371: where a pass takes its column's traversal: next sector, previous distance, pending boundaries
+template <bool SPLIT>
+__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c, const PassColumn &r) {
+    const gd_map_desc *m = cc.m;
+    const MapView &mv = cc.mv;
+    const LaneCtx &L = *cc.c;
+    const ColumnState before = c;
+    const int x = cc.x;
+    const int cs = c.current_sector;
+    const int cur = cs < 0 ? 0 : cs;
+    const int wi = r.wall;
+    const float distance = r.distance;
+    const bool valid = r.bits & PB_VALID, one_sided = r.bits & PB_ONE_SIDED;
+    auto incident = [&](int w) { return mv.sec(w, 0) == cur || mv.sec(w, 1) == cur; };
     // s. next sector (engine.py:13070-13241)
     const float prior = before.previous_distance;
     const float prior_eps = prior + 1e-3f;
@@ -3238,8 +3260,8 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c
 }
 
 // engine.py:13424-13744 for one column
-template <bool DEPTH, bool GENERAL>
-__device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, int local, const ColumnState &c, PixelBuffers &pb, const unsigned char *colormap) {
+template <bool DEPTH, bool GENERAL, typename Pixels>
+__device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, int local, const ColumnState &c, Pixels &pb, const unsigned char *colormap) {
     const gd_map_desc *m = cc.m;
     const LaneCtx &L = *cc.c;
     const int x = cc.x;
@@ -3312,11 +3334,13 @@ __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const Col
     const unsigned row_base = (unsigned)(shl64(texture_mid, 16 - height_bits) + (mul64(vertical_step, FIXED_UNIT - center_fixed) >> 16));
     const size_t texel_base = (size_t)texture_id * m->tex_max_h * m->tex_max_w + (size_t)mu;
     const unsigned atlas_w = (unsigned)m->tex_max_w;
-    for (int yb = y0; yb < y1; yb += WALL_ROWS) {
+    const int stride = pb.row_lanes;
+    wave_fence();                         // the column's other lanes may have written these rows
+    for (int yb = y0 + pb.row_lane; yb < y1; yb += WALL_ROWS * stride) {
         unsigned char texel[WALL_ROWS]; unsigned int word[WALL_ROWS];
 #pragma unroll
         for (int j = 0; j < WALL_ROWS; ++j) {
-            const int y = yb + j < y1 ? yb + j : y1 - 1;
+            const int y = min(yb + j * stride, y1 - 1);
             const unsigned fraction = row_base + row_step * (unsigned)y;
             const unsigned mv_ = (fraction >> (31 - height_bits)) >> 1;
             texel[j] = m->tex_atlas[texel_base + __umul24(mv_, atlas_w)];
@@ -3324,7 +3348,7 @@ __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const Col
         }
 #pragma unroll
         for (int j = 0; j < WALL_ROWS; ++j) {
-            const int y = yb + j;
+            const int y = yb + j * stride;
             if (y >= y1) continue;
             // the texel goes to the frame where there is one; otherwise it waits for the kernel that assembles the frame
             const unsigned char colour = colormap[shade * 256 + texel[j]];
@@ -3589,8 +3613,8 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int str
 
 // The traversal in two kernels.  Which drawseg a column pass selects, and where the column goes next, depends on the map,
 // the camera and the column's ray alone, never on projected rows or clips: wall_select_kernel runs that half
-// (pass_select without the projection, pass_advance's state part) and records one PassRec per pass; wall_raster_kernel
-// runs the other half over the records (pass_geometry, pass_clip, pass_paint, pass_advance's clip part, the masked mid-texture).
+// (pass_select without the projection, pass_advance) and records one PassRec per pass; wall_raster_kernel
+// runs the other half over the records (pass_draw, clip_pass, pass_paint, advance_clips, the masked mid-texture).
 // Each half is lighter in registers and in code than the two together, so more of its wavefronts share a SIMD and
 // its pass loop fits the instruction cache.  Same segment order and one wavefront per segment in both.
 #define SELECT_STRIPS_PER_GROUP 1
@@ -3691,7 +3715,6 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
         const int left = __builtin_amdgcn_update_dpp(-1, w, 0x111 /* row_shr:1 */, 0xF, 0xF, false);
         if (hit != CAND_KEY_NONE && left != w) atomicOr(&named[w >> 5], 1u << (w & 31));
     }
-    PixelBuffers no_pixels; SilhouetteBounds no_bounds; GapRange no_gaps;   // the state part of pass_advance touches none of them
     PassColumn pc;
     bool done = false;
     int recorded = 0;
@@ -3723,7 +3746,7 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
                     sc.status[STATUS_PASS_OVERFLOW] = 1;
                 }
             }
-            const bool changed = pass_advance<SPLIT, ADVANCE_STATE>(cc, st, pc, no_pixels, no_bounds, false, no_gaps);
+            const bool changed = pass_advance<SPLIT>(cc, st, pc);
             // A pass that found nothing and changed nothing repeats identically for ever.
             if (!(pc.bits & PB_VALID) && !changed) done = true;
         }
@@ -3738,27 +3761,49 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
 // sixteen of these wavefronts at 128 registers).  After the staging barrier the wavefronts never meet again.
 #define WALL_STRIPS_PER_GROUP 2
 #define RASTER_WAVES 4
+// The pass that the lane `k` of each column's PARTS lanes prepared, for all of them.
+template <int PARTS>
+__device__ __forceinline__ PassDraw hand_round(const PassDraw &prepared, int k, int lane_id) {
+    if (PARTS == 1) return prepared;
+    constexpr int COLUMNS = SEG_COLS / PARTS;
+    const int from = (k * COLUMNS + (lane_id & (COLUMNS - 1))) * 4;
+    auto take = [&](unsigned int v) { return (unsigned int)__builtin_amdgcn_ds_bpermute(from, (int)v); };
+    PassDraw d;
+    d.flags = take(prepared.flags); d.wall_sector = take(prepared.wall_sector); d.rows = take(prepared.rows);
+    d.column_a = take(prepared.column_a); d.frac_a = take(prepared.frac_a); d.step_a = take(prepared.step_a);
+    d.column_b = take(prepared.column_b); d.frac_b = take(prepared.frac_b); d.step_b = take(prepared.step_b);
+    d.distance = __uint_as_float(take(__float_as_uint(prepared.distance)));
+    return d;
+}
 // A strip's wavefront draws, pass after pass, the rows that any of its columns draws.  A small batch, which lasts as long as its
-// longest strips, shares a strip out over four wavefronts, a larger one over two.  Where the lines lie best depends on how much
-// longer a map's longest strips are than its others, which the host does not know: four are as good as two at 430 (320 linedefs) to 700
-// lanes (701 linedefs in bricks), two as good as one at 1150 to some 1700; both lines lie between, where no map loses much to
-// the other choice.  Stage times in us (wall_geometry_kernel among them) for 1 / 2 / 4 / 8 wavefronts a strip:
-//   lanes             320 linedefs        2000                4000                701, bricks
-//     128       190 / 165 / 156 / 157   240 / 210 / 205   402 / 380 / 359   412 / 370 / 338 / 339
-//     512       217 / 198 / 211 / 318   300 / 266 / 286   493 / 441 / 413   453 / 380 / 353 / 412
-//     640       243 / 213 / 250         320 / 290 / 328   518 / 470 / 449   475 / 396 / 367
-//    1024       275 / 264 / 366         375 / 358 / 477   616 / 529 / 666   524 / 439 / 495
-//    1280       302 / 314               400 / 426         653 / 618         544 / 451
-//    1536       320 / 362               456 / 495         695 / 704         561 / 511
-//    2048       383 / 464               535 / 633         755 / 881
-__host__ __device__ constexpr int raster_parts(int lanes) { return lanes <= 560 ? 4 : (lanes <= 1344 ? 2 : 1); }
+// longest strips, shares a strip out over eight wavefronts, a larger one over four, over two.  The wavefront's columns then have eight,
+// four or two lanes each: these prepare as many passes at once and share every run of rows out, so that both the chain of waits and the
+// vector instructions of a column shrink with them (when the spare lanes stood idle, eight wavefronts never paid).  What a strip more
+// wavefronts costs is room on the SIMDs.  Stage times in us (wall_geometry_kernel among them) for 1 / 2 / 4 / 8 wavefronts a
+// strip, in brackets with idle lanes and the lines of then (four up to 560 lanes, two up to 1344):
+//   lanes           320 linedefs                     2000                             4000                             701, bricks
+//      16         / 90 / 72 / 65 (106)            / 136 / 110 / 97 (155)           / 184 / 149 / 139 (196)          / 263 / 218 / 188 (285)
+//     256        / 142 / 119 / 113 (155)         / 198 / 161 / 145 (212)          / 328 / 259 / 229 (327)          / 291 / 238 / 208 (310)
+//     384        / 148 / 121 / 136 (174)         / 206 / 175 / 170 (229)          / 349 / 276 / 274 (345)          / 298 / 247 / 219 (322)
+//     512        / 156 / 126 / 175 (202)         / 219 / 189 / 222 (250)          / 425 / 401 / 367 (480)          / 313 / 256 / 249 (318)
+//     640        / 165 / 156 / 222 (202)         / 233 / 204 / 279 (277)          / 432 / 416 / 394 (498)          / 346 / 273 / 309 (408)
+//     768     235 / 173 / 187 / 270 (214)     328 / 239 / 236 / 333 (282)      527 / 445 / 422 / 457 (513)      430 / 345 / 283 / 371 (415)
+//    1024     253 / 204 / 233 / 351 (249)     385 / 270 / 303 / 437 (330)      555 / 466 / 445 / 598 (539)      449 / 354 / 334 / 487 (431)
+//    1536     294 / 287 / 342 (298)           438 / 383 / 440 (448)            597 / 528 / 630 (619)            479 / 392 / 490 (501)
+//    2048     365 / 357 / 450 (364)           492 / 478 / 583 (487)            701 / 674 / 835 (695)            524 / 509 / 643 (536)
+//    2560     439 / 425 (440)                 596 / 589 (583)                  831 / 845 (820)                  639 / 625 (649)
+//    3072     519 / 542 (514)                 700 / 722 (683)                  930 / 969 (918)                  751 / 744 (753)
+__host__ __device__ constexpr int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 2400 ? 2 : 1)); }
 // DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
 // BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
-// 4096 lanes on the 4000-linedef map: 1.78 -> 1.00 ms (with wall_geometry_kernel 1.33): the linedefs' lines 1.53, no sprite clip plane
-// and the rows walked together 1.33, no branch around a load or a store 1.03.  It is left at four wavefronts a SIMD (128 registers, four
-// of them spilled; at 96 registers the spills in the row loops make it 1.6 ms), 60 % of their cycles waiting.
-template <bool DEPTH, bool GENERAL>
+// 4096 lanes on the 4000-linedef map: 1.78 -> 1.00 ms: the linedefs' lines 1.53, no sprite clip plane
+// and the rows walked together 1.33, no branch around a load or a store 1.03.  It is left at four wavefronts a SIMD (128 registers;
+// at 96 the spills in the row loops make it 1.6 ms), 60 % of their cycles waiting.  By itself, with a column's lanes sharing its passes and
+// rows: 16 lanes on the 2000-linedef map 97 -> 53 us, 512 on the 4000-linedef map 443 -> 350, 1024 on the 320-linedef map 286 -> 226 (rows alone
+// 71, 426, 252).  The passes are handed round from register to register: through LDS there are no spills, but the 1024 lanes take 268.  Working
+// out the textures of visible tiers only makes the 1024 lanes 241, and 4096 1.11 ms.
+template <bool DEPTH, bool GENERAL, int PARTS>
 __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(RASTER_WAVES, RASTER_WAVES))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
     __shared__ LaneCtx lane_ctxs[WALL_STRIPS_PER_GROUP][64 / SEG_COLS];
@@ -3769,8 +3814,8 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     const int lane_id = threadIdx.x & 63;
     const int segment_in_wave = lane_id / SEG_COLS;
     const int wavefront = blockIdx.x * WALL_STRIPS_PER_GROUP + wave_in_group;
-    const int parts = raster_parts(lane_count);
-    const int segment_slot = wavefront / parts, part = wavefront % parts, part_cols = SEG_COLS / parts;
+    constexpr int part_cols = SEG_COLS / PARTS;
+    const int segment_slot = wavefront / PARTS, part = wavefront % PARTS;
     const bool live = segment_slot < lane_count * SEGS_PER_LANE;
     const int segment = live ? sc.strip_order[segment_slot] : 0;
     const int local = segment / SEGS_PER_LANE;
@@ -3782,8 +3827,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     __syncthreads();
     if (!live) return;   // whole segments: the groups of four columns that exchange values below live or leave together
     const LaneCtx &lane_ctx = lane_ctxs[wave_in_group][segment_in_wave];
-    // a wavefront's columns are its first part_cols lanes; the others stand in for columns without a pass (the exchanges and
-    // the row walks of the wavefront need them executing) and leave before a column's end is written
+    // a wavefront's part_cols columns have `parts` lanes each, which do everything alike and share the rows out
     const bool own_column = lane_id < part_cols;
     const int x = (segment - local * SEGS_PER_LANE) * SEG_COLS + part * part_cols + (lane_id & (part_cols - 1));
     bool window_dirty = false;
@@ -3795,7 +3839,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     cc.frags = sc.frag_rec + (size_t)local * m->split_count * m->fragment_slots;
     cc.x = x;
     ray_direction(lane_ctx, x, &cc.rx, &cc.ry);
-    PixelBuffers pb;
+    PixelBuffers<PARTS> pb;
     pb.frame = frame_base;
     pb.meta = sc.meta; pb.masked_texel = sc.masked_texel;
     pb.scene_depth = DEPTH ? sc.scene_depth : nullptr;
@@ -3803,6 +3847,8 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     pb.words = __builtin_amdgcn_make_buffer_rsrc(sc.meta, 0, lane_count * (VH * SW * 4), BUFFER_WORDS);
     pb.depths = __builtin_amdgcn_make_buffer_rsrc(pb.scene_depth, 0, DEPTH ? lane_count * (VH * SW * 4) : 0, BUFFER_WORDS);
     pb.frame_column = (unsigned)local * (unsigned)frame_stride + (unsigned)x;
+    pb.row_lane = PARTS == 1 ? 0 : lane_id / part_cols;
+    pb.put_column = pb.word_column + (unsigned)pb.row_lane * (SW * 4u);
     // the meta plane arrives with whatever the last frame left: see GapRange for how every row gets written
     ColumnState st;   // only the clips and the masked-drawseg snapshot live here; the traversal state stayed in wall_select_kernel
     st.current_sector = -1;
@@ -3812,76 +3858,71 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
     SilhouetteBounds sb; sb.bot_row = VH; sb.top_row = 0; sb.bot_depth = -GD_INF; sb.top_depth = -GD_INF;
-    const int passes = own_column ? sc.pass_count[(size_t)local * SW + x] : 0;
+    const int passes = sc.pass_count[(size_t)local * SW + x];
     const size_t first_record = sc.pass_at(0, local, x), pass_stride = (size_t)sc.lane_stride * SW;
     const unsigned int *geo_slots = sc.geo_slot + cc.rec_base;
+    // Each of a column's lanes prepares every PARTS-th pass, so that what a pass has to ask memory for is on its way for PARTS of them
+    // at once; then the passes are drawn one after the other, each handed round from the lane that prepared it.
     // A pass's record names its linedef, the linedef's slot where it lies in geo: the next pass's slot and the record after it
     // are asked for a pass ahead.  (Columns past their last pass keep asking for their first one.)
     PassRec record = {}, next_record = {};
     unsigned int slot = 0u, slot_wall = 0u;      // a pass that draws nothing names no linedef: the slot of the last one asked for will do
+    const size_t group_stride = PARTS * pass_stride;
+    size_t prepared_at = first_record + (size_t)pb.row_lane * pass_stride;
     if (passes > 0) {
-        record = sc.pass_rec[first_record]; next_record = sc.pass_rec[first_record + (passes > 1 ? pass_stride : (size_t)0)];
+        record = sc.pass_rec[pb.row_lane < passes ? prepared_at : first_record]; next_record = sc.pass_rec[pb.row_lane + PARTS < passes ? prepared_at + group_stride : first_record];
         slot_wall = record.bits ? record.wall : 0u;
         slot = geo_slots[slot_wall];
     }
-    for (int pass = 0; __ballot(pass < passes) != 0; ++pass) {
-        const bool mine = pass < passes;
-        bool draws = false;
-        PassColumn pc = {};   // a finished column, or one whose pass draws nothing, paints no row and draws no tier: its group of four has no common tail
-        if (mine) {
-            const PassRec rec = record;
-            const unsigned int geo_at = slot;
-            const size_t at = first_record + (size_t)pass * pass_stride;
+    for (int group = 0; __ballot(group < passes) != 0; group += PARTS) {
+        const int pass = group + pb.row_lane;
+        const PassRec rec = record;
+        const unsigned int geo_at = slot;
+        if (group < passes) {
             record = next_record;
             slot_wall = record.bits ? record.wall : slot_wall;
             slot = geo_slots[slot_wall];
-            next_record = sc.pass_rec[pass + 2 < passes ? at + 2 * pass_stride : first_record];
-            draws = (rec.bits & (PB_RASTER | PB_PS_KEEPS)) != 0;
-            pc.bits = draws ? (int)rec.bits : 0;
-            if (draws) {
-                pc.wall = rec.wall; pc.render_current = rec.render_current; pc.distance = rec.distance;
-                pc.ps_path_index = rec.ps_path; pc.ps_other = rec.ps_other; pc.marks = rec.marks;
-                PassTexture texture;
-                pass_geometry<GENERAL>(dm, cc, sc, sc.geo[geo_at], at, rec.marks, pc, texture);
-                pass_clip(cc, st.ceiling_clip, st.floor_clip, pc);
-                if (pc.bits & (PB_TIER0 | PB_TIER1 | PB_TIER2)) {
-                    texture_column(texture.ends, texture.past_left, texture.side, pc.side, x, &pc.u_base, &pc.swall);
-                    pc.offset_y = texture.side.offset_y; pc.fake_contrast = texture.side.contrast;
-                }
-            }
+            next_record = sc.pass_rec[pass + 2 * PARTS < passes ? prepared_at + 2 * group_stride : first_record];
         }
-        // 4-column wallscan groups (engine.py:12688-12761): the aligned group of four columns agrees on its drawseg, on
-        // which tiers all four draw and on the rows all four share.  The four lanes of a group are one DPP quad, so every
-        // exchange is a vector move with a lane pattern (no trip through the LDS crossbar), and the minima, maxima and
-        // conjunctions take two steps each.  Every lane of the wavefront is active here.
-        const int w0 = quad_first(pc.wall), s0 = quad_first(pc.side);
-        const int GROUP_AGREES = 0x1;   // takes PB_VALID's place in the word that is and-ed over the group
-        const int agreed = quad_and((pc.bits & (PB_TIER0 | PB_TIER1 | PB_TIER2)) | ((pc.wall == w0 && pc.side == s0) ? GROUP_AGREES : 0));
-        const bool same_group = (agreed & GROUP_AGREES) != 0;
-        // a value that is not a number never becomes a common top or bottom (std::max(-inf, nan) is -inf)
-        const float shared_top = fmaxf(-GD_INF, quad_max(pc.clipped_top)), shared_lower_top = fmaxf(-GD_INF, quad_max(pc.clipped_lower_top));
-        const float shared_bottom = fminf(GD_INF, quad_min(pc.clipped_bottom)), shared_upper_bottom = fminf(GD_INF, quad_min(pc.clipped_upper_bottom));
-        const float common_bottom[3] = {shared_bottom, shared_bottom, shared_upper_bottom};
-        const i64 first_group_visibility = ((i64)quad_first((int)(pc.visibility >> 32)) << 32) | (i64)(unsigned)quad_first((int)(pc.visibility & 0xFFFFFFFFLL));
-        bool group_valid[3];
-        group_valid[0] = same_group && (agreed & PB_TIER0) && (shared_top < shared_bottom);
-        group_valid[1] = same_group && (agreed & PB_TIER1) && (shared_lower_top < shared_bottom);
-        group_valid[2] = same_group && (agreed & PB_TIER2) && (shared_top < shared_upper_bottom);
-        pass_paint<DEPTH>(cc, st, pc, pb, group_valid, common_bottom, first_group_visibility, colormap_lds, window_dirty, gaps);
-        if (draws) {
-            pass_advance<GENERAL, ADVANCE_CLIPS>(cc, st, pc, pb, sb, !window_dirty, gaps, &sc, first_record + (size_t)pass * pass_stride);
+        const PassDraw prepared = pass_draw<GENERAL>(dm, cc, sc, pass < passes && (rec.bits & (PB_RASTER | PB_PS_KEEPS)) != 0, rec, geo_at, prepared_at);
+        prepared_at += group_stride;
+#pragma unroll 1
+        for (int k = 0; k < PARTS; ++k) {
+            if (PARTS > 1 && __ballot(group + k < passes) == 0) break;
+            const PassDraw d = hand_round<PARTS>(prepared, k, lane_id);
+            const PassRows rows = clip_pass(d, st.ceiling_clip, st.floor_clip);
+            // The aligned group of four columns agrees on which tiers all four draw and on the rows all four share: minima, maxima and
+            // conjunctions over the quad take two steps each.  Every lane of the wavefront is active here.
+            const bool raster = d.flags & DRAW_RASTER, one_sided = d.flags & DRAW_ONE_SIDED, texture_a = d.flags & DRAW_TEXTURE_A;
+            const bool tier0 = raster && one_sided && texture_a && rows.top < rows.bottom;
+            const bool tier1 = raster && (d.flags & DRAW_LOWER) && texture_a && rows.lower_top < rows.bottom;
+            const bool tier2 = raster && (d.flags & DRAW_UPPER) && (d.flags & DRAW_TEXTURE_B) && rows.top < rows.upper_bottom;
+            const int agreed = quad_and((tier0 ? 1 : 0) | (tier1 ? 2 : 0) | (tier2 ? 4 : 0));
+            const bool same_group = d.flags & DRAW_GROUP;
+            const float shared_top = quad_max(rows.top), shared_lower_top = quad_max(rows.lower_top);
+            const float shared_bottom = quad_min(rows.bottom), shared_upper_bottom = quad_min(rows.upper_bottom);
+            const float common_bottom[3] = {shared_bottom, shared_bottom, shared_upper_bottom};
+            bool group_valid[3];
+            group_valid[0] = same_group && (agreed & 1) && (shared_top < shared_bottom);
+            group_valid[1] = same_group && (agreed & 2) && (shared_lower_top < shared_bottom);
+            group_valid[2] = same_group && (agreed & 4) && (shared_top < shared_upper_bottom);
+            pass_paint<DEPTH>(cc, st, d, rows, pb, group_valid, common_bottom, colormap_lds, window_dirty, gaps);
+            if (d.flags & (DRAW_RASTER | DRAW_PS_KEEPS)) advance_clips(cc, st, d, rows, pb, sb, !window_dirty, gaps, sc, first_record + (size_t)(group + k) * pass_stride);
         }
     }
-    if (!own_column) return;
     // what is left of a window no one-sided drawseg closed shows the flat pass's picture
     if (!window_dirty) zero_rows(pb, gaps, x, st.ceiling_clip <= 0.0f ? 0 : (int)st.ceiling_clip, st.floor_clip >= (float)VH ? VH : (int)st.floor_clip);
     if (dm.masked_count > 0) masked_midtexture<DEPTH, GENERAL>(dm, cc, sc, local, st, pb, colormap_lds);
     // The columns with view pixels that no wall tier, plane or masked texture covers join the flat pass's work list, those of a
     // wavefront in one piece (flat_gap_kernel selects the pixels, flat_shade_kernel paints them).
     bool holds_gap = false;
-    for (int y = gaps.lo(), gap_end = gaps.hi(); y < gap_end && !holds_gap; ++y) holds_gap = gap_pixel(pb.m(y));
-    const u64 holders = __ballot(holds_gap);
+    wave_fence();
+    for (int y = gaps.lo() + pb.row_lane, gap_end = gaps.hi(); y < gap_end && !holds_gap; y += PARTS) holds_gap = gap_pixel(pb.m(y));
+    u64 holders = __ballot(holds_gap);
     if (holders == 0) return;
+    for (int other = 32; other >= part_cols; other >>= 1) holders |= holders >> other;   // a column's lanes
+    holders &= ~0ULL >> (64 - part_cols);
+    holds_gap = own_column && (holders >> lane_id & 1);
     int list_base = 0;
     if (lane_id == 0) list_base = atomicAdd(sc.gap_column_count, __popcll(holders));
     list_base = __builtin_amdgcn_readfirstlane(list_base);
@@ -5814,8 +5855,13 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(geometry_parts(count) + SW / 64, count), dim3(64), 0, stream, r->dm, count, sc, geometry_parts(count));
         const dim3 grid((wavefronts * raster_parts(count) + WALL_STRIPS_PER_GROUP - 1) / WALL_STRIPS_PER_GROUP), block(64 * WALL_STRIPS_PER_GROUP);
         const bool general = split || m.sector_count > LDS_SECTORS || m.texture_count > LDS_TEXTURES;
-        auto kernel = decals ? (general ? wall_raster_kernel<true, true> : wall_raster_kernel<true, false>)
-                             : (general ? wall_raster_kernel<false, true> : wall_raster_kernel<false, false>);
+        auto pick = [&](auto parts) {
+            constexpr int P = decltype(parts)::value;
+            return decals ? (general ? wall_raster_kernel<true, true, P> : wall_raster_kernel<true, false, P>)
+                          : (general ? wall_raster_kernel<false, true, P> : wall_raster_kernel<false, false, P>);
+        };
+        const int parts = raster_parts(count);
+        auto kernel = parts == 8 ? pick(std::integral_constant<int, 8>()) : parts == 4 ? pick(std::integral_constant<int, 4>()) : parts == 2 ? pick(std::integral_constant<int, 2>()) : pick(std::integral_constant<int, 1>());
         hipLaunchKernelGGL(kernel, grid, block, 0, stream, r->dm, count, sc, frame_base, frame_stride);
     }
     mark();
