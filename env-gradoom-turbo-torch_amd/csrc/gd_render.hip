@@ -2008,18 +2008,30 @@ __global__ void __launch_bounds__(SW) flat_span_finish_kernel(Scratch sc) {
 // walls: engine.py:11462-13745
 // ---------------------------------------------------------------------------------------------
 #define CAND_BATCH 8
-// wall_select_kernel's launch for the longest strips
-#define SELECT_STAGED_STRIPS 512   // how many strips,
-#define SELECT_PARTS 8             // and over how many wavefronts each is shared out;
-#define SELECT_FINE_STRIPS 128     // in a small batch the very longest are shared out over more
-#define SELECT_FINE_PARTS 32
-// A small batch lasts as long as its longest strips, a larger one as long as all of its strips together take on the wavefront
-// slots there are; sharing the longest strips out further shortens the first and adds to the second.  Up to where that pays
-// follows the map's linedefs, which make the longest lists: 160 lanes at 320 linedefs, 400 at 800 (450 at 701 in bricks), 500 at 1400, 650 at 2000,
-// 1000 at 3000, 1250 at 4000.  Stage times in us without / with fine parts: 320 linedefs, 128 lanes 88 / 81, 384 lanes 94 / 118, 1024 lanes
-// 140 / 155; 800, 256 lanes 147 / 128, 512 lanes 149 / 158; 2000, 256 lanes 263 / 196, 512 lanes 269 / 244, 768 lanes 283 / 283, 1024 lanes 309 / 317;
-// 4000, 256 lanes 534 / 372, 768 lanes 585 / 498, 1024 lanes 612 / 551, 1280 lanes 628 / 617, 1536 lanes 657 / 665.
-bool select_finely(int lanes, int linedefs) { return lanes < 192 + (linedefs < 4096 ? linedefs : 4096) / 4; }   // no map of more was timed
+// wall_select_kernel's launch for the longest strips: how many of them, and how many lanes a column has there.  More strips and more lanes
+// shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a
+// large one's does.  Where the lists are short (they follow the map's linedefs) there is little to shorten: none where the lanes are as many
+// as six times the linedefs beyond 160.  Stage times in us of no such launch / 768 strips (1024 from 1400 linedefs on) of 8 / of 16 lanes
+// (of 32), in brackets what it took with the lists in LDS and 8 columns of one lane a wavefront:
+//   lanes       120              320                        800                         2000                          4000
+//      16    46 / 55 / 76     97 / 53 / 64 (61; [60])    168 / 74 / 62 (52)         339 / 120 / 89 (68; [151])     361 / 119 / 90 (69; [156])
+//     128    55 / 60 / 77     133 / 69 / 81 ([83])       181 / 83 / 71              436 / 153 / 113 (104; [203])   1003 / 236 / 172 (145; [430])
+//     256    59 / 73          137 / 84 / 96 ([102])      212 / 106 / 99             447 / 164 / 132 ([214])        999 / 247 / 197 ([420])
+//     512    63 / 81          140 / 107 / 119 ([111])    220 / 126 / 128            453 / 172 / 178 ([267])        1003 / 275 / 257 ([463])
+//    1024    69               149 / 146 ([138])          241 / 174 / 174            520 / 265 / 264 ([336])        1060 / 408 / 413 ([563])
+//    2048    80               166 / 180 ([171])          277 / 234 / 235            549 / 371 / 370 ([411])        1120 / 652 / 647 ([727])
+//    4096    130              230 / 288 ([279])          328 / 363                  667 / 604 / 576 ([600])        1249 / 945 / 887 ([966])
+// (the last two rows with 768 and with 512 strips.)
+int select_strips(int lanes, int linedefs) {
+    if (lanes >= 6 * (linedefs - 160)) return 0;
+    return lanes < 1792 ? (linedefs < 1024 ? 768 : 1024) : (lanes < 3584 ? 768 : 512);
+}
+int select_lanes(int lanes, int linedefs) {
+    const int w = linedefs < 4096 ? linedefs : 4096;      // no map of more was timed
+    if (w < 512) return 8;
+    if (lanes <= 64 + w / 24) return 32;
+    return lanes <= 128 + w / 8 || (lanes >= 1536 && w >= 1024) ? 16 : 8;
+}
 #define WALL_ROWS 8          // rows painted / clipped per step of the wall traversal
 struct ColumnCtx {
     const Tables *tb;
@@ -2034,12 +2046,6 @@ struct ColumnCtx {
     int count;
     int x;
     float rx, ry;
-    // wall_select_kernel's staged launch: this column's list copied to LDS (entry k at staged + k * 128 bytes: a row of
-    // the wavefront's 8 columns), unused everywhere else.  (One or the other for a whole kernel: a choice per load would become one flat
-    // load of a selected address.)
-    typedef __attribute__((address_space(3))) const char LdsByte;
-    LdsByte *staged;
-    bool use_staged = false;
     __device__ __forceinline__ const WallRec &rec(int w) const { return recs[rec_base + (unsigned)w]; }
     // Where the list of column `x` of the chunk's lane `local` starts and how many entries it has: the column's own
     // slots, or its slot in the spill pool.
@@ -2057,11 +2063,8 @@ struct ColumnCtx {
         }
     }
     __device__ __forceinline__ Cand cand(int k) const {
-        typedef unsigned int Words4 __attribute__((ext_vector_type(4)));
-        typedef __attribute__((address_space(3))) const Words4 LdsEntry;
-        union { uint4 raw; Words4 words; Cand c; } u;
-        if (use_staged) u.words = *(LdsEntry *)(staged + (unsigned)k * (64 / SELECT_PARTS * 16u));   // all of the list is there
-        else u.raw = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(list) + (list_column + (unsigned)k * (SW * 16u)));   // one 16-byte load
+        union { uint4 raw; Cand c; } u;
+        u.raw = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(list) + (list_column + (unsigned)k * (SW * 16u)));   // one 16-byte load
         return u.c;
     }
     // Entries k0 .. k0+CAND_BATCH-1 of this column's list, loaded together so that their memory
@@ -2082,6 +2085,77 @@ struct ColumnCtx {
         for (int j = 0; j < CAND_BATCH; ++j) out[j] = cand(at[j] < 0 ? 0 : at[j]);
     }
     __device__ Eval eval(int w) const { return eval_wall(m, *c, spans + rec_base, x, w, rx, ry); }
+};
+
+// A column's list as wall_select_kernel's LANES lanes of the column hold it between them: entry k in registers of lane k % LANES.  Each
+// looks at its own in a scan, and what the scan is after, the smallest of some keys, is exchanged.  One lane alone reads the list where it is.
+template <int LANES> struct ListShare {
+    static constexpr int ENTRIES = CAND_MAX / LANES;
+    Cand own[ENTRIES];
+    // an entry that is not there lies nearer than any distance a scan asks for: none takes it
+    __device__ __forceinline__ void load(const ColumnCtx &cc, int lane) {
+#pragma unroll
+        for (int j = 0; j < ENTRIES; ++j) own[j] = cc.cand(max(min(j * LANES + lane, cc.count - 1), 0));
+#pragma unroll
+        for (int j = 0; j < ENTRIES; ++j)
+            if (j * LANES + lane >= cc.count) { own[j].dist = -GD_INF; own[j].flags = 0; }
+    }
+    // the smallest of the column's lanes; all of them are executing
+    template <int CONTROL> static __device__ __forceinline__ u64 moved(u64 v) {
+        return ((u64)(unsigned)__builtin_amdgcn_mov_dpp((int)(v >> 32), CONTROL, 0xF, 0xF, true) << 32) | (u64)(unsigned)__builtin_amdgcn_mov_dpp((int)(v & 0xFFFFFFFFu), CONTROL, 0xF, 0xF, true);
+    }
+    static __device__ __forceinline__ u64 smallest(u64 v) {
+        u64 o;
+        if (LANES >= 2) { o = moved<0xB1>(v); v = o < v ? o : v; }      // lanes 1,0,3,2
+        if (LANES >= 4) { o = moved<0x4E>(v); v = o < v ? o : v; }      // lanes 2,3,0,1
+        if (LANES >= 8) { o = moved<0x141>(v); v = o < v ? o : v; }     // the eight lanes mirrored
+        if (LANES >= 16) { o = moved<0x140>(v); v = o < v ? o : v; }    // the sixteen lanes mirrored
+        if (LANES >= 32) { o = ((u64)(unsigned)__builtin_amdgcn_ds_swizzle((int)(v >> 32), 0x401F) << 32) | (u64)(unsigned)__builtin_amdgcn_ds_swizzle((int)(v & 0xFFFFFFFFu), 0x401F); v = o < v ? o : v; }
+        return v;
+    }
+    static __device__ __forceinline__ unsigned smallest(unsigned v) {
+        if (LANES >= 2) v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true));
+        if (LANES >= 4) v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true));
+        if (LANES >= 8) v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true));
+        if (LANES >= 16) v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true));
+        if (LANES >= 32) v = min(v, (unsigned)__builtin_amdgcn_ds_swizzle((int)v, 0x401F));
+        return v;
+    }
+    // every entry of the column that this lane looks at
+    template <typename Look> __device__ __forceinline__ void each(const ColumnCtx &cc, Look look) const {
+#pragma unroll
+        for (int j = 0; j < ENTRIES; ++j) look(own[j]);
+    }
+};
+// The nearest of the candidates a scan takes, the lowest linedef on ties, and its flags.
+template <int LANES> struct NearestOf {
+    u64 key = CAND_KEY_NONE;
+    __device__ __forceinline__ void take(const Cand &q) { const u64 k = cand_key(q); key = k < key ? k : key; }
+    __device__ __forceinline__ void share() { key = ListShare<LANES>::smallest(key); }     // what the column's lanes took
+    __device__ __forceinline__ float distance() const { return cand_key_distance(key); }
+    __device__ __forceinline__ int wall() const { return cand_key_wall(key); }
+    __device__ __forceinline__ int flags() const { return cand_key_flags(key); }
+};
+template <> struct NearestOf<1> {
+    float d = GD_INF; int w = 0x7fffffff, f = 0;
+    __device__ __forceinline__ void take(const Cand &q) { if (q.dist < d || (q.dist == d && (int)q.wall < w)) { d = q.dist; w = q.wall; f = q.flags; } }
+    __device__ __forceinline__ void share() {}
+    __device__ __forceinline__ float distance() const { return d; }
+    __device__ __forceinline__ int wall() const { return w; }
+    __device__ __forceinline__ int flags() const { return f; }
+};
+template <> struct ListShare<1> {
+    static __device__ __forceinline__ u64 smallest(u64 v) { return v; }
+    static __device__ __forceinline__ unsigned smallest(unsigned v) { return v; }
+    template <typename Look> __device__ __forceinline__ void each(const ColumnCtx &cc, Look look) const {
+        for (int k0 = 0; k0 < cc.count; k0 += CAND_BATCH) {
+            Cand batch[CAND_BATCH];
+            cc.cand_batch(k0, batch);
+#pragma unroll
+            for (int j = 0; j < CAND_BATCH; ++j)
+                if (k0 + j < cc.count) look(batch[j]);
+        }
+    }
 };
 
 // The projection fragment of a linedef at one column (engine.py:11511-11529, 12324-12376): the first
@@ -2511,8 +2585,8 @@ __device__ __forceinline__ PassRows clip_pass(const PassDraw &d, float ceiling_c
 }
 
 // engine.py:11769-12239: selection of the pass's drawseg for one column
-template <bool SPLIT>
-__device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnState &c, bool boundary_has_po, PassColumn &r) {
+template <bool SPLIT, int LANES>
+__device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ListShare<LANES> &list, const ColumnState &c, bool boundary_has_po, PassColumn &r) {
     const gd_map_desc *m = cc.m;
     const MapView &mv = cc.mv;
     const int x = cc.x;
@@ -2535,7 +2609,15 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
         // b. equal-depth solid (engine.py:11784-11807): the nearest one-sided candidate replaces
         // the selection when it lies within 1e-3 of the nearest candidate, found in the same scan.
         u64 nearest = CAND_KEY_NONE, nearest_solid = CAND_KEY_NONE;
-        for (int k0 = 0; k0 < cc.count; k0 += CAND_BATCH) {
+        if constexpr (LANES > 1) {
+            list.each(cc, [&](const Cand &q) {
+                const u64 key = incident_c(q) && q.dist > prev ? cand_key(q) : CAND_KEY_NONE;
+                nearest = key < nearest ? key : nearest;
+                const u64 solid_key = q.s1 < 0 ? key : CAND_KEY_NONE;
+                nearest_solid = solid_key < nearest_solid ? solid_key : nearest_solid;
+            });
+            nearest = list.smallest(nearest); nearest_solid = list.smallest(nearest_solid);
+        } else for (int k0 = 0; k0 < cc.count; k0 += CAND_BATCH) {
             Cand batch[CAND_BATCH];
             cc.cand_batch(k0, batch);
             unsigned batch_bits = 0u;
@@ -2576,22 +2658,45 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
     float ps_path_distance = distance; int ps_path_index = wi;
     bool ps_path_geo = cwi.flags & CF_GEO;
     float psd = GD_INF; int psi = 0x7fffffff; int psi_flags = 0;
-    if (!sel_is_proj) {
-        auto solid_owner = [&](const Cand &q) {
-            bool owner = incident_c(q) && (q.s1 < 0) && (q.flags & CF_PROJ) && (q.flags & CF_LEDGE) && shares_sel_c(q) && (q.dist > prev_eps);
-            if (owner && (q.dist < psd || (q.dist == psd && (int)q.wall < psi))) { psd = q.dist; psi = q.wall; psi_flags = q.flags; }
-        };
-        for (u64 rest = incident_beyond; rest;) {
-            Cand batch[CAND_BATCH]; int at[CAND_BATCH];
-            cc.cand_batch_of(rest, batch, at);
+    // A later scan of the pass: over the positions `incident_beyond` names, or over all of a lane's own.  `look` says whether `ask`, of
+    // which there is one copy, has to be asked about the candidate as well.
+    auto look_beyond = [&](auto look, auto ask) {
+        if constexpr (LANES > 1) {
+            unsigned asked = 0;
 #pragma unroll
-            for (int j = 0; j < CAND_BATCH; ++j) {
-                if (at[j] < 0) continue;
-                solid_owner(batch[j]);
+            for (int j = 0; j < list.ENTRIES; ++j) asked |= look(list.own[j]) ? 1u << j : 0u;
+            for (; asked; asked &= asked - 1) {
+                Cand q = list.own[0];
+#pragma unroll
+                for (int j = 1; j < list.ENTRIES; ++j)
+                    if ((asked & ((2u << j) - 1u)) == 1u << j) q = list.own[j];
+                ask(q);
             }
+        } else {
+            u64 asked = 0;
+            for (u64 rest = incident_beyond; rest;) {
+                Cand batch[CAND_BATCH]; int at[CAND_BATCH];
+                cc.cand_batch_of(rest, batch, at);
+#pragma unroll
+                for (int j = 0; j < CAND_BATCH; ++j)
+                    if (at[j] >= 0 && look(batch[j])) asked |= 1ULL << at[j];
+            }
+            for (; asked; asked &= asked - 1) ask(cc.cand(__ffsll((long long)asked) - 1));
+            for (int k = 64; k < cc.count; ++k)   // a spilled column's further entries
+                if ((incident_beyond >> (k & 63)) & 1ULL) {
+                    const Cand q = cc.cand(k);
+                    if (look(q)) ask(q);
+                }
         }
-        for (int k = 64; k < cc.count; ++k)   // a spilled column's further entries
-            if ((incident_beyond >> (k & 63)) & 1ULL) solid_owner(cc.cand(k));
+    };
+    if (!sel_is_proj) {
+        NearestOf<LANES> solid;
+        look_beyond([&](const Cand &q) {
+            if (incident_c(q) && (q.s1 < 0) && (q.flags & CF_PROJ) && (q.flags & CF_LEDGE) && shares_sel_c(q) && (q.dist > prev_eps)) solid.take(q);
+            return false;
+        }, [](const Cand &) {});
+        solid.share();
+        psd = solid.distance(); psi = solid.wall(); psi_flags = solid.flags();
         if (sel_excl_right) {
             const int *ofs = sel_start ? m->solid_bridge_start_ofs : m->solid_bridge_end_ofs;
             const int *idx = sel_start ? m->solid_bridge_start_idx : m->solid_bridge_end_idx;
@@ -2625,28 +2730,21 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ColumnSta
     float npd = GD_INF; int npi = 0x7fffffff; int npi_flags = 0;
     const int so_s0 = mv.sec(wi, 0), so_s1 = mv.sec(wi, 1);
     if (!so_is_proj) {
-        auto near_owner = [&](const Cand &q) {
-            int w = q.wall;
-            if (!(incident_c(q) && (q.s1 >= 0) && (q.flags & CF_PROJ) && (q.dist > prev_eps))) return;
+        NearestOf<LANES> near;
+        look_beyond([&](const Cand &q) {
+            if (!(incident_c(q) && (q.s1 >= 0) && (q.flags & CF_PROJ) && (q.dist > prev_eps))) return false;
             bool le = q.flags & CF_LEDGE;
             bool same_pair = (q.s0 == so_s0 && q.s1 == so_s1) || (q.s0 == so_s1 && q.s1 == so_s0);
             bool close = (same_pair || (le && so_excl_right && (so_narrow || (shares_sel_c(q) && so_short)))) &&
                          (fabsf(q.dist - distance) <= tolerance_of(q.dist));
-            bool topo = false;
-            if (!close && le && so_excl_right && so_narrow) { int dummy; topo = mv.sector_bridge((q.flags & CF_ALONG_HI) ? 1 : 0, w, no_path_index, &dummy); }
-            if ((close || topo) && (q.dist < npd || (q.dist == npd && w < npi))) { npd = q.dist; npi = w; npi_flags = q.flags; }
-        };
-        for (u64 rest = incident_beyond; rest;) {
-            Cand batch[CAND_BATCH]; int at[CAND_BATCH];
-            cc.cand_batch_of(rest, batch, at);
-#pragma unroll
-            for (int j = 0; j < CAND_BATCH; ++j) {
-                if (at[j] < 0) continue;
-                near_owner(batch[j]);
-            }
-        }
-        for (int k = 64; k < cc.count; ++k)   // a spilled column's further entries
-            if ((incident_beyond >> (k & 63)) & 1ULL) near_owner(cc.cand(k));
+            if (close) near.take(q);
+            return !close && le && so_excl_right && so_narrow;
+        }, [&](const Cand &q) {
+            int dummy;
+            if (mv.sector_bridge((q.flags & CF_ALONG_HI) ? 1 : 0, q.wall, no_path_index, &dummy)) near.take(q);
+        });
+        near.share();
+        npd = near.distance(); npi = near.wall(); npi_flags = near.flags();
     }
     int pe_wall = c.pend_ep_wall;
     int pe_s0 = mv.sec(pe_wall, 0), pe_s1 = mv.sec(pe_wall, 1);
@@ -3143,8 +3241,8 @@ __device__ __forceinline__ void advance_clips(const ColumnCtx &cc, ColumnState &
 }
 
 // engine.py:13070-13371: where a pass takes its column's traversal: next sector, previous distance, pending boundaries
-template <bool SPLIT>
-__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c, const PassColumn &r) {
+template <bool SPLIT, int LANES>
+__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, const ListShare<LANES> &list, ColumnState &c, const PassColumn &r) {
     const gd_map_desc *m = cc.m;
     const MapView &mv = cc.mv;
     const LaneCtx &L = *cc.c;
@@ -3168,35 +3266,31 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ColumnState &c
     int ppb_idx = 0, gp_other = -1; float gpd = GD_INF;
     if (endpoint_only_portal) {
         const float dist_eps = distance + 1e-3f;
-        float cnd = GD_INF, ond = GD_INF; int cni = 0x7fffffff, oni = 0x7fffffff;
-        float csd = GD_INF, osd = GD_INF;
-        int gpi = 0x7fffffff; bool gp_along_hi = false;
+        NearestOf<LANES> current_next, other_next, geometric;
+        const unsigned none = __float_as_uint(GD_INF);
+        unsigned current_solid = none, other_solid = none;      // distances: positive, so their bits order as they do
         const int v0 = mv.vert(wi, 0), v1 = mv.vert(wi, 1);
-        for (int k0 = 0; k0 < cc.count; k0 += CAND_BATCH) {
-            Cand batch[CAND_BATCH];
-            cc.cand_batch(k0, batch);
-#pragma unroll
-            for (int j = 0; j < CAND_BATCH; ++j) {
-                if (k0 + j >= cc.count) continue;
-                const Cand q = batch[j];
-                int w = q.wall; float d = q.dist;
-                bool os = q.s1 < 0;
-                bool inc = (q.s0 == cur || q.s1 == cur), oinc = (q.s0 == other_sector || q.s1 == other_sector);
-                bool future = ((q.flags & CF_GEO) || os) && (d > dist_eps);
-                if (future) {
-                    if (inc) take_min(d, w, cnd, cni);
-                    if (oinc) take_min(d, w, ond, oni);
-                }
-                bool shares_endpoint = (int)q.v0 == v0 || (int)q.v0 == v1 || (int)q.v1 == v0 || (int)q.v1 == v1;
-                bool shared_solid = os && (shares_endpoint || (q.flags & CF_LEDGE)) && (d > prior_eps) && (d <= dist_eps);
-                if (shared_solid) {
-                    if (inc && d < csd) csd = d;
-                    if (oinc && d < osd) osd = d;
-                }
-                bool sgp = (q.flags & CF_GEO) && inc && shares_endpoint && !os && (d > prior_eps) && (fabsf(d - distance) <= (1.0f / 16.0f));
-                if (sgp && (d < gpd || (d == gpd && w < gpi))) { gpd = d; gpi = w; gp_along_hi = (q.flags & CF_ALONG_HI) != 0; }
-            }
-        }
+        list.each(cc, [&](const Cand &q) {
+            const float d = q.dist;
+            bool os = q.s1 < 0;
+            bool inc = (q.s0 == cur || q.s1 == cur), oinc = (q.s0 == other_sector || q.s1 == other_sector);
+            bool future = ((q.flags & CF_GEO) || os) && (d > dist_eps);
+            if (future && inc) current_next.take(q);
+            if (future && oinc) other_next.take(q);
+            bool shares_endpoint = (int)q.v0 == v0 || (int)q.v0 == v1 || (int)q.v1 == v0 || (int)q.v1 == v1;
+            bool shared_solid = os && (shares_endpoint || (q.flags & CF_LEDGE)) && (d > prior_eps) && (d <= dist_eps);
+            if (shared_solid && inc) current_solid = min(current_solid, __float_as_uint(d));
+            if (shared_solid && oinc) other_solid = min(other_solid, __float_as_uint(d));
+            bool sgp = (q.flags & CF_GEO) && inc && shares_endpoint && !os && (d > prior_eps) && (fabsf(d - distance) <= (1.0f / 16.0f));
+            if (sgp) geometric.take(q);
+        });
+        current_next.share(); other_next.share(); geometric.share();
+        current_solid = list.smallest(current_solid); other_solid = list.smallest(other_solid);
+        const float cnd = current_next.distance(), ond = other_next.distance(), csd = __uint_as_float(current_solid), osd = __uint_as_float(other_solid);
+        int cni = current_next.wall(), oni = other_next.wall();
+        const int gpi = geometric.wall();
+        const bool gp_along_hi = (geometric.flags() & CF_ALONG_HI) != 0;
+        gpd = geometric.distance();
         if (!finitef(cnd)) cni = 0;
         if (!finitef(ond)) oni = 0;
         bool enters_tied_strip = finitef(cnd) && (cni == oni) && mv.opposing(wi, cni);
@@ -3621,46 +3715,39 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int str
 // The kernel lasts as long as its longest strips: on the 4000-linedef map the 256 longest of 20,480 take 0.94 ms with the
 // chip to themselves, all of them together 1.22 ms, all but the 4096 longest 0.53 ms.  Such a strip's wavefront is held
 // up by its candidate scans (the longest lists, read from device memory beside 20,000 other wavefronts) and by running,
-// pass after pass, every rule that any of its 64 columns takes.  So the SELECT_STAGED_STRIPS longest strips (they lead
-// the order) go to a launch of their own (STAGED): a strip is shared out over SELECT_PARTS wavefronts of 8 columns
-// each, which first copy their columns' lists to LDS (8 KB a wavefront) and scan them there.  It runs beside the
-// launch for all other strips.  The fewer columns a wavefront has, the fewer rules it runs in a pass, and the more wavefronts
-// take slots from the other launch.  4096 lanes, this launch / the other, wavefronts a strip: 4: 0.88 / 0.97 ms, 8: 0.75 / 0.92,
-// 16: 0.81 / 1.00; 2048 lanes on a 1400-linedef map 4: 0.24 / 0.26, 8: 0.20 / 0.27, 16: 0.25 / 0.28.  A smaller batch
-// lasts as long as its very longest strips: 512 lanes on the 4000-linedef map 4: 0.74 / 0.38, 8: 0.65 / 0.39, 16: 0.51 / 0.40, and 32 for
-// 128 of the strips, 8 for the others 0.45 / 0.41 (32 for 256: 0.49; 64 for 128: 0.54); 256 lanes on an 800-linedef map 0.161 / 0.086, 0.128 /
-// 0.090, 0.116 / 0.099, 0.121 / 0.106 (up to which batch that pays: select_finely).  Lists left in device memory: no gain.
-static_assert(SEG_COLS == 64 && SELECT_STRIPS_PER_GROUP == 1, "wall_select_kernel's staged launch: parts of one whole strip per work-group");
-template <bool SPLIT, bool STAGED>
-__global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kernel(DeviceMap dm, int lane_count, Scratch sc, int staged_slots, int fine_slots) {
+// pass after pass, every rule that any of its 64 columns takes.  So the longest strips (they lead the order; select_strips) go to a launch of
+// their own, beside the launch for all other strips, in which a column has LANES lanes: a strip is LANES wavefronts, the lanes of a
+// column hold its list between them in registers, each scans its own entries, and what a scan is after is the smallest of the lanes' keys, three to
+// five lane moves away.  All else they do alike, and the first of them writes the records.  Next to eight wavefronts of 8 columns with one lane
+// each, their lists copied to LDS: 16 lanes on the 2000-linedef map 151 -> 68 us, 512 on the 4000-linedef map 463 -> 257, 4096 of them 0.97 -> 0.89 ms.  What the
+// rules ask beyond the list (a sector bridge) they ask behind the scan, once for each entry concerned: a copy of that code for every entry made the
+// kernels larger than the instruction cache.
+static_assert(SEG_COLS == 64 && SELECT_STRIPS_PER_GROUP == 1, "wall_select_kernel's launch for the longest strips: parts of one whole strip per work-group");
+template <bool SPLIT, int LANES>
+__global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kernel(DeviceMap dm, int lane_count, Scratch sc, int longest) {
     const gd_map_desc *m = &dm.d;
+    constexpr bool SHARED = LANES > 1;     // the launch for the longest strips
+    constexpr int parts = LANES, part_cols = 64 / LANES;
     __shared__ LaneCtx lane_ctxs[SELECT_STRIPS_PER_GROUP][64 / SEG_COLS];
-    constexpr int ROW = 64 / SELECT_PARTS;                              // columns of a wavefront of the staged launch, at most
-    __shared__ uint4 staged_entries[STAGED ? CAND_MAX * ROW : 1];       // [CAND_MAX][ROW] in the staged launch
-    // the staged launch: fine_slots strips of SELECT_FINE_PARTS wavefronts each, then the others of SELECT_PARTS
-    const int block = blockIdx.x, fine_blocks = fine_slots * SELECT_FINE_PARTS;
-    const bool fine = STAGED && block < fine_blocks;
-    const int parts = !STAGED ? 1 : (fine ? SELECT_FINE_PARTS : SELECT_PARTS), part_cols = 64 / parts;
-    const int from_block = STAGED && !fine ? block - fine_blocks : block, from_slot = STAGED && !fine ? fine_slots : 0;
+    const int block = blockIdx.x;
     const int wave_in_group = threadIdx.x >> 6;
     const int lane_id = threadIdx.x & 63;
     const int segment_in_wave = lane_id / SEG_COLS;
-    const int segment_slot = from_slot + (from_block / parts * SELECT_STRIPS_PER_GROUP + wave_in_group) * (64 / SEG_COLS) + segment_in_wave;
-    const int part = from_block % parts;
-    const bool live = segment_slot < (STAGED ? staged_slots : lane_count * SEGS_PER_LANE);
+    const int segment_slot = (block / parts * SELECT_STRIPS_PER_GROUP + wave_in_group) * (64 / SEG_COLS) + segment_in_wave;
+    const int part = block % parts, lane_of_column = lane_id & (LANES - 1);
+    const bool live = segment_slot < (SHARED ? longest : lane_count * SEGS_PER_LANE);
     const int segment = live ? sc.strip_order[segment_slot] : 0;
     const int local = segment / SEGS_PER_LANE;
     if ((lane_id & (SEG_COLS - 1)) == 0 && live) lane_ctxs[wave_in_group][segment_in_wave] = sc.ctx[local];
     __syncthreads();
     if (!live) return;
     const LaneCtx &lane_ctx = lane_ctxs[wave_in_group][segment_in_wave];
-    // A strip with a column in the spill pool (more entries than the LDS copy holds) is left to the other launch, which
-    // covers the staged launch's slots as well and otherwise leaves them alone.  Both ask all 64 columns of the strip.
+    // A strip with a column in the spill pool (more entries than its lanes hold) is left to the other launch, which
+    // covers the longest strips' slots as well and otherwise leaves them alone.  Both ask all 64 columns of the strip.
     const int strip_x = (segment - local * SEGS_PER_LANE) * SEG_COLS;
     const bool long_lists = __ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + lane_id] >> SPILL_SHIFT) != 0) != 0;
-    if (STAGED ? long_lists : (segment_slot < staged_slots && !long_lists)) return;   // the same in the whole wavefront
-    if (lane_id >= part_cols) return;
-    const int x = strip_x + part * part_cols + lane_id;
+    if (SHARED ? long_lists : (segment_slot < longest && !long_lists)) return;   // the same in the whole wavefront
+    const int x = strip_x + part * part_cols + lane_id / LANES;
     ColumnCtx cc;
     cc.tb = nullptr; cc.m = m; cc.mv.m = m; cc.c = &lane_ctx;
     cc.recs = sc.rec; cc.spans = sc.span;
@@ -3670,23 +3757,12 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     cc.x = x;
     ray_direction(lane_ctx, x, &cc.rx, &cc.ry);
     bool boundary_has_po = false;   // does some entry's span begin at this column
-    if (STAGED) {
-        // every lane copies its own column's entries and reads only those: no barrier
-        char *mine = reinterpret_cast<char *>(staged_entries) + lane_id * 16;
-        const int depth = cc.count;
-        for (int k0 = 0; k0 < depth; k0 += CAND_BATCH) {
-            Cand batch[CAND_BATCH];
-            cc.cand_batch(k0, batch);
-#pragma unroll
-            for (int j = 0; j < CAND_BATCH; ++j) {
-                union { uint4 raw; Cand c; } u;
-                u.c = batch[j];
-                boundary_has_po |= (batch[j].flags & CF_LEDGE) != 0;   // slots past the end repeat the last entry
-                if (k0 + j < depth) *reinterpret_cast<uint4 *>(mine + (k0 + j) * (ROW * 16)) = u.raw;
-            }
-        }
-        cc.staged = (ColumnCtx::LdsByte *)mine;
-        cc.use_staged = true;
+    ListShare<LANES> list;
+    if constexpr (SHARED) {
+        list.load(cc, lane_of_column);
+        unsigned first = 1u;
+        list.each(cc, [&](const Cand &q) { first = (q.flags & CF_LEDGE) ? 0u : first; });
+        boundary_has_po = list.smallest(first) == 0u;
     }
     ColumnState st;
     st.current_sector = lane_ctx.sector;
@@ -3695,7 +3771,7 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     st.previous_distance = 0.0f;
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
-    if (!STAGED) {
+    if (!SHARED) {
         for (int k0 = 0; k0 < cc.count && !boundary_has_po; k0 += CAND_BATCH) {
             Cand batch[CAND_BATCH];
             cc.cand_batch(k0, batch);
@@ -3709,11 +3785,12 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     // the linedefs the recorded passes draw get a bit each; columns that draw what the column before them draws leave it to that one
     unsigned int *named = sc.named + (size_t)local * named_words(m);
     int last_named = -1;
+    auto neighbour = [](int v) { return LANES < 16 ? __builtin_amdgcn_update_dpp(-1, v, 0x110 + (LANES & 15) /* row_shr */, 0xF, 0xF, false) : -1; };
     if (dm.masked_count > 0) {   // so do those whose masked mid-texture is a column's nearest
         const u64 hit = sc.masked_hit[(size_t)local * SW + x];
         const int w = cand_key_wall(hit);
-        const int left = __builtin_amdgcn_update_dpp(-1, w, 0x111 /* row_shr:1 */, 0xF, 0xF, false);
-        if (hit != CAND_KEY_NONE && left != w) atomicOr(&named[w >> 5], 1u << (w & 31));
+        const int left = neighbour(w);
+        if (lane_of_column == 0 && hit != CAND_KEY_NONE && left != w) atomicOr(&named[w >> 5], 1u << (w & 31));
     }
     PassColumn pc;
     bool done = false;
@@ -3721,9 +3798,15 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
     const int sectors = m->sector_count;
     for (int pass = 0; pass < sectors; ++pass) {
         if (!done) {
-            pass_select<SPLIT>(cc, st, boundary_has_po, pc);
+            pass_select<SPLIT>(cc, list, st, boundary_has_po, pc);
             if (pc.bits & (PB_RASTER | PB_PS_KEEPS)) {
-                if (pass < sc.pass_slots) {
+                const bool repeats = last_named == pc.wall;
+                last_named = pc.wall;
+                // a neighbour that does not take part in this pass shows the linedef it named last
+                const bool names = !repeats && neighbour(last_named) != last_named;
+                if (lane_of_column != 0) {
+                    recorded = pass + 1;
+                } else if (pass < sc.pass_slots) {
                     PassRec rec;
                     rec.wall = (unsigned short)pc.wall; rec.render_current = (unsigned short)pc.render_current;
                     rec.bits = (unsigned short)pc.bits; rec.ps_path = (unsigned short)pc.ps_path_index;
@@ -3731,11 +3814,7 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
                     // passes between two recorded ones keep whatever the slot held: the drawing half skips them by their bits
                     for (int skipped = recorded; skipped < pass; ++skipped) records[(size_t)skipped * pass_stride].bits = 0;
                     records[(size_t)pass * pass_stride] = rec;
-                    const bool repeats = last_named == pc.wall;
-                    last_named = pc.wall;
-                    // a neighbour that does not take part in this pass shows the linedef it named last
-                    if (!repeats && __builtin_amdgcn_update_dpp(-1, last_named, 0x111 /* row_shr:1 */, 0xF, 0xF, false) != last_named)
-                        atomicOr(&named[pc.wall >> 5], 1u << (pc.wall & 31));
+                    if (names) atomicOr(&named[pc.wall >> 5], 1u << (pc.wall & 31));
                     if (pc.bits & PB_PS_KEEPS) {
                         path_distances[(size_t)pass * pass_stride] = pc.ps_path_distance;
                         atomicOr(&named[pc.ps_path_index >> 5], 1u << (pc.ps_path_index & 31));
@@ -3746,13 +3825,13 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
                     sc.status[STATUS_PASS_OVERFLOW] = 1;
                 }
             }
-            const bool changed = pass_advance<SPLIT>(cc, st, pc);
+            const bool changed = pass_advance<SPLIT>(cc, list, st, pc);
             // A pass that found nothing and changed nothing repeats identically for ever.
             if (!(pc.bits & PB_VALID) && !changed) done = true;
         }
         if (__ballot(!done) == 0) break;
     }
-    sc.pass_count[(size_t)local * SW + x] = (unsigned char)recorded;
+    if (lane_of_column == 0) sc.pass_count[(size_t)local * SW + x] = (unsigned char)recorded;
 }
 
 // One wavefront per 64 / SEG_COLS segments.  Segments share nothing but read-only tables; a work-group of the drawing
@@ -5768,12 +5847,12 @@ int validate_map(const gd_map_desc *h) {
 
 const int STAGE_COUNT = 9;
 
-// A frame that goes to the side stream and back pays some 20 us for it.  Batches whose strips are all selected by one launch do without
+// A frame that goes to the side stream and back pays some 20 us for it.  Batches of up to 102 lanes do without
 // where there is little to put there: no billboards, or a few lanes.  A frame in us with / without, 1 lane with billboards on 120 to 4000
 // linedefs 139 / 119, 261 / 236, 210 / 185, 243 / 235, 433 / 414, 8 lanes 256 / 285, 284 / 259, 293 / 312, 396 / 394, 450 / 428, 48 lanes
 // 323 / 356, 405 / 436, 439 / 468, 586 / 611, 878 / 891; without billboards on 320, 800 and 4000 linedefs, 16 lanes 256 / 241, 364 / 351,
 // 533 / 520, 64 lanes 437 / 429, 434 / 426, 884 / 878.
-bool side_stream_pays(int lanes, bool billboards) { return lanes * SEGS_PER_LANE > SELECT_STAGED_STRIPS || (billboards && lanes >= 4); }
+bool side_stream_pays(int lanes, bool billboards) { return lanes > 102 || (billboards && lanes >= 4); }
 
 int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_desc *lanes, const gd_frame_out *out, int base, int count, hipStream_t stream, bool timed) {
     const gd_map_desc &m = r->dm.d;
@@ -5819,29 +5898,31 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         const int wavefronts = (count * SEGS_PER_LANE + 64 / SEG_COLS - 1) / (64 / SEG_COLS);
         const bool split = m.split_count > 0;
         const dim3 select_block(64 * SELECT_STRIPS_PER_GROUP);
-        // The longest strips here with their lists in LDS, the others on the side stream, both at once.  This way round: the
-        // side stream starts a few microseconds behind, time enough for the staged launch's work-groups to be placed;
+        // The longest strips here, the others on the side stream, both at once.  This way round: the
+        // side stream starts a few microseconds behind, time enough for the longest strips' work-groups to be placed;
         // started together, the other launch's 20,000 take every wavefront slot first and the strips that decide how long
         // the pair lasts begin last.
         const int strips = count * SEGS_PER_LANE;
-        const int staged_strips = r->side_ready ? (strips < SELECT_STAGED_STRIPS ? strips : SELECT_STAGED_STRIPS) : 0;
-        auto select_kernel = split ? wall_select_kernel<true, false> : wall_select_kernel<false, false>;
-        if (staged_strips > 0) {
-            const bool alone = staged_strips == strips;   // the other launch is left with strips of spilled columns: it follows
+        const int longest_wanted = select_strips(count, m.wall_count);
+        const int longest = r->side_ready ? (strips < longest_wanted ? strips : longest_wanted) : 0;
+        auto select_kernel = split ? wall_select_kernel<true, 1> : wall_select_kernel<false, 1>;
+        if (longest > 0) {
+            const bool alone = longest == strips;   // the other launch is left with strips of spilled columns: it follows
             if (!alone) {
                 HIP_TRY(hipEventRecord(r->fork_event, stream));
                 HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
             }
-            auto staged_kernel = split ? wall_select_kernel<true, true> : wall_select_kernel<false, true>;
-            const int fine_strips = !select_finely(count, m.wall_count) ? 0 : (strips < SELECT_FINE_STRIPS ? strips : SELECT_FINE_STRIPS);
-            hipLaunchKernelGGL(staged_kernel, dim3(fine_strips * SELECT_FINE_PARTS + (staged_strips - fine_strips) * SELECT_PARTS), select_block, 0, stream, r->dm, count, sc, staged_strips, fine_strips);
-            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, alone ? stream : r->side_stream, r->dm, count, sc, staged_strips, 0);
+            const int column_lanes = select_lanes(count, m.wall_count);
+            auto pick = [&](auto lanes) { constexpr int L = decltype(lanes)::value; return split ? wall_select_kernel<true, L> : wall_select_kernel<false, L>; };
+            auto longest_kernel = column_lanes == 32 ? pick(std::integral_constant<int, 32>()) : (column_lanes == 16 ? pick(std::integral_constant<int, 16>()) : pick(std::integral_constant<int, 8>()));
+            hipLaunchKernelGGL(longest_kernel, dim3(longest * column_lanes), select_block, 0, stream, r->dm, count, sc, longest);
+            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, alone ? stream : r->side_stream, r->dm, count, sc, longest);
             if (!alone) {
                 HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
                 HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
             }
         } else {
-            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0, 0);
+            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0);
         }
         // the billboards' lists beside the walls' drawing, on the side stream (when stages are being timed, with the billboards)
         if (has_billboards && !fused && !timed) {

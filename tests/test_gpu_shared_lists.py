@@ -1,0 +1,50 @@
+"""The selection's columns that share their candidate lists out over 8, 16 or 32 lanes: on either side of the lines at which their number
+changes, and with all of a batch's strips, some of them or none among the longest, every lane's frame is the one the CPU oracle draws."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CAMERAS = 4
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("linedefs", [320, 700, 1100])
+def test_batches_at_the_lines_of_the_lists_shares_match_the_oracle(oracle, linedefs, split):
+    from gradoom_amd import hostmath, mapbuild, synthmap
+    from gradoom_amd.renderer import HipRenderer, LaneState
+    from gradoom_amd.selfcheck import make_lane_arrays
+
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    cells = {320: 7, 700: 10, 1100: 12}[linedefs]
+    smap = synthmap.generate_map(linedefs, grid=(cells, cells), sectors=cells * cells * 4 // 5, linedefs=linedefs, layout="brick", midtex=0.1)
+    smap = synthmap.with_variant(smap, linedefs + 1, heights="doors", textures="npot", lights=True)
+    if split:
+        smap = synthmap.split_linedefs(smap, linedefs + 2)
+    poses = synthmap.generate_poses(smap, CAMERAS, linedefs + 3, pitch=True, flash=True, margin=0.005)
+    arrays = make_lane_arrays(smap, poses, synthmap.generate_sprites(smap, CAMERAS, 16, linedefs + 4))
+    tables = mapbuild.build_map_tables(smap)
+    expected = torch.as_tensor(oracle.render(tables, arrays, cosine)["indexed"]).to("cuda:0")
+    count = len(tables["walls"])
+    assert count >= linedefs
+    strips = 768 if count < 1024 else 1024                                           # select_strips and select_lanes in gd_render.hip
+    lines = {strips // 5 + 1, 64 + count // 24 + 1, 128 + count // 8 + 1}            # the first batch beyond each
+    none_longest = 6 * (count - 160)
+    if none_longest <= 1600:
+        lines.add(none_longest)
+    if count >= 1024:
+        lines.add(1536)
+    for lanes in sorted({1} | lines | {line - 1 for line in lines}):
+        print(f"{count} linedefs: {lanes} lanes", flush=True)
+        which = np.arange(lanes) % CAMERAS
+        renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+        indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+        renderer.render(LaneState.from_numpy({name: np.ascontiguousarray(value[which]) for name, value in arrays.items()}, "cuda:0"), indexed=indexed)
+        torch.cuda.synchronize()
+        assert renderer.status() == 0
+        assert torch.equal(indexed, expected[torch.as_tensor(which, device="cuda:0")])
+        renderer.close()
