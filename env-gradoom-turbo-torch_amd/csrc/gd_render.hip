@@ -3956,12 +3956,17 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     for (int group = 0; __ballot(group < passes) != 0; group += PARTS) {
         const int pass = group + pb.row_lane;
         const PassRec rec = record;
-        const unsigned int geo_at = slot;
+        unsigned int geo_at = slot;
         if (group < passes) {
-            record = next_record;
-            slot_wall = record.bits ? record.wall : slot_wall;
-            slot = geo_slots[slot_wall];
-            next_record = sc.pass_rec[pass + 2 * PARTS < passes ? prepared_at + 2 * group_stride : first_record];
+            if constexpr (PARTS == 1) {
+                record = next_record;
+                slot_wall = record.bits ? record.wall : slot_wall;
+                slot = geo_slots[slot_wall];
+                next_record = sc.pass_rec[pass + 2 * PARTS < passes ? prepared_at + 2 * group_stride : first_record];
+            } else {
+                geo_at = geo_slots[rec.bits ? rec.wall : 0];
+                record = sc.pass_rec[pass + PARTS < passes ? prepared_at + group_stride : first_record];
+            }
         }
         const PassDraw prepared = pass_draw<GENERAL>(dm, cc, sc, pass < passes && (rec.bits & (PB_RASTER | PB_PS_KEEPS)) != 0, rec, geo_at, prepared_at);
         prepared_at += group_stride;
