@@ -30,6 +30,8 @@ SYMBOLS = (
     "gd_expand_rgb24",
     "gd_pack_actors",
     "gd_pack_weapon",
+    "gd_pack_decals",
+    "gd_screen_blend",
     "gd_ray_tables",
     "gd_sprite_depth",
     "gd_pose_lanes",
@@ -97,6 +99,10 @@ def library() -> C.CDLL:
     lib.gd_pack_actors.argtypes = [C.POINTER(_abi.ActorDesc), C.c_void_p]
     lib.gd_pack_weapon.restype = C.c_int
     lib.gd_pack_weapon.argtypes = [C.POINTER(_abi.WeaponDesc), C.c_void_p]
+    lib.gd_pack_decals.restype = C.c_int
+    lib.gd_pack_decals.argtypes = [C.c_void_p] * 6 + [C.c_int32, C.c_void_p, C.c_int32, C.c_int32] + [C.c_void_p] * 3
+    lib.gd_screen_blend.restype = C.c_int
+    lib.gd_screen_blend.argtypes = [C.c_void_p] * 3 + [C.c_int32] + [C.c_void_p] * 2
     lib.gd_ray_tables.restype = C.c_int
     lib.gd_ray_tables.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.gd_sprite_depth.restype = C.c_int

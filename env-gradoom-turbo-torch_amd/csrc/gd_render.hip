@@ -5544,6 +5544,54 @@ __global__ void __launch_bounds__(64) pack_weapon_kernel(gd_weapon_desc d) {
     if (d.flash_light) d.flash_light[lane] = d.weapon_flash_lights[entry];
 }
 
+// gd_pack_decals: one wavefront per lane.  A slot's place is the number of slots before it in the order (a stable one), counted against
+// 64 slots' keys in LDS at a time.  Each float operation is rounded on its own, as in the Torch expressions.  2048 lanes of 64 slots: some thirty
+// Torch kernels, a sort among them, 0.20 ms; one kernel, 0.011 ms.
+#define DECAL_FREE 2147483647LL      // the place in the order of a slot without an impact
+__global__ void __launch_bounds__(64) pack_decals_kernel(const int64_t *serial, const int64_t *wall, const float *along, const float *impact_z, const int64_t *style,
+                                                         const float *walls, int wall_count, const int64_t *fine_sine, int slots, int32_t *decal_state, float *decal_geom) {
+    __shared__ i64 keys[64];
+    const size_t lane = (size_t)blockIdx.x * (size_t)slots;
+    const float TWO_PI = (float)(2.0 * 3.14159265358979323846), FINE_PER_RADIAN = (float)(FINE_ANGLES / (2.0 * 3.14159265358979323846));
+    for (int base = 0; base < slots; base += 64) {
+        const int s = base + (int)threadIdx.x;
+        const bool held = s < slots;
+        const i64 own = held ? serial[lane + s] : -1, key = own >= 0 ? own : DECAL_FREE;
+        int place = 0;
+        for (int other = 0; other < slots; other += 64) {
+            const int j = other + (int)threadIdx.x;
+            const i64 theirs = j < slots ? serial[lane + j] : -1;
+            __syncthreads();
+            keys[threadIdx.x] = theirs >= 0 ? theirs : DECAL_FREE;
+            __syncthreads();
+            const int count = min(64, slots - other);
+            for (int k = 0; k < count; ++k) place += keys[k] < key || (keys[k] == key && other + k < s);
+        }
+        if (!held) continue;
+        const i64 linedef = clampi(wall[lane + s], 0, wall_count - 1), kind = style[lane + s];
+        const float4 ends = reinterpret_cast<const float4 *>(walls)[linedef];
+        float dx = ends.z - ends.x, dy = ends.w - ends.y;
+        if (kind < 0 || kind >= 20) { dx = -dx; dy = -dy; }      // the seg runs backwards on sidedef 1
+        float turn = fmodf(atan2f(dy, dx), TWO_PI);
+        if (turn != 0.0f && turn < 0.0f) turn += TWO_PI;         // torch.remainder with a positive divisor
+        const i64 fine = (i64)floorf(turn * FINE_PER_RADIAN) & (FINE_ANGLES - 1);
+        int32_t *state = decal_state + (lane + place) * 3;
+        state[0] = (int32_t)linedef; state[1] = (int32_t)kind; state[2] = own >= 0 ? 1 : 0;
+        float *geom = decal_geom + (lane + place) * 4;
+        geom[0] = along[lane + s]; geom[1] = impact_z[lane + s];
+        geom[2] = (float)fine_sine[(fine + FINE_ANGLES / 4) & (FINE_ANGLES - 1)] / 65536.0f; geom[3] = (float)fine_sine[fine] / 65536.0f;
+    }
+}
+
+// gd_screen_blend: one thread per lane.  Torch divides by a constant on the device by multiplying with its reciprocal.
+__global__ void __launch_bounds__(256) screen_blend_kernel(const int64_t *bonus_count, const int64_t *damage_count, const float *damage_to_alpha, int lane_count, float *blend) {
+    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
+    if (lane >= lane_count) return;
+    const float per = 1.0f / 255.0f, bonus = (float)bonus_count[lane] * 8.0f;
+    blend[2 * (size_t)lane] = (bonus < 128.0f ? bonus : 128.0f) * per;
+    blend[2 * (size_t)lane + 1] = damage_to_alpha[clampi(damage_count[lane], 0, 113)] * per;
+}
+
 #define HIP_TRY GD_HIP_TRY
 #define SIZE_CHECK GD_SIZE_CHECK
 
@@ -6575,6 +6623,29 @@ int gd_pack_weapon(const gd_weapon_desc *w, void *stream) {
     if (w->flash_light && !w->weapon_flash_lights) return fail(GD_E_ARG, "flash_light needs weapon_flash_lights");
     if (w->lane_count == 0) return GD_OK;
     hipLaunchKernelGGL(pack_weapon_kernel, dim3((unsigned)((w->lane_count + 63) / 64)), dim3(64), 0, static_cast<hipStream_t>(stream), *w);
+    HIP_TRY(hipGetLastError());
+    return GD_OK;
+}
+
+int gd_pack_decals(const int64_t *serial, const int64_t *wall, const float *along, const float *impact_z, const int64_t *style, const float *walls,
+                   int32_t wall_count, const int64_t *fine_sine, int32_t lane_count, int32_t slots, int32_t *decal_state, float *decal_geom, void *stream) {
+    if (lane_count < 0 || slots < 0 || slots > (1 << 20)) return fail(GD_E_ARG, "count out of range");
+    if (lane_count == 0 || slots == 0) return GD_OK;      // nothing to pack: the tensors may have no address
+    if (!serial || !wall || !along || !impact_z || !style || !walls || !fine_sine || !decal_state || !decal_geom) return fail(GD_E_ARG, "null argument");
+    if (wall_count <= 0) return fail(GD_E_ARG, "decals need linedefs");
+    if (reinterpret_cast<uintptr_t>(walls) & 15) return fail(GD_E_ARG, "walls must lie on 16 bytes");
+    hipLaunchKernelGGL(pack_decals_kernel, dim3((unsigned)lane_count), dim3(64), 0, static_cast<hipStream_t>(stream), serial, wall, along, impact_z, style, walls, wall_count,
+                       fine_sine, slots, decal_state, decal_geom);
+    HIP_TRY(hipGetLastError());
+    return GD_OK;
+}
+
+int gd_screen_blend(const int64_t *bonus_count, const int64_t *damage_count, const float *damage_to_alpha, int32_t lane_count, float *screen_blend, void *stream) {
+    if (lane_count < 0) return fail(GD_E_ARG, "negative count");
+    if (lane_count == 0) return GD_OK;
+    if (!bonus_count || !damage_count || !damage_to_alpha || !screen_blend) return fail(GD_E_ARG, "null argument");
+    hipLaunchKernelGGL(screen_blend_kernel, dim3((unsigned)((lane_count + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), bonus_count, damage_count, damage_to_alpha,
+                       lane_count, screen_blend);
     HIP_TRY(hipGetLastError());
     return GD_OK;
 }

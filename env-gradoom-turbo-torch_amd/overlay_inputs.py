@@ -13,6 +13,8 @@ import math
 import numpy as np
 import torch
 
+from . import hostmath
+
 FIXED_UNIT = 65536
 FINE_ANGLES = 8192
 WEAPON_LOWER_TICS = 16          # engine.py:111
@@ -199,6 +201,16 @@ def hud_state(
     return torch.stack(columns, dim=1).to(torch.int32).contiguous()
 
 
+def _read_in_place(whole: tuple[torch.Tensor, ...], real: tuple[torch.Tensor, ...]) -> bool:
+    """Are these contiguous int64 and float32 tensors of one ROCm device, as the library's kernels read them, and is only their result wanted?"""
+
+    tensors = whole + real
+    device = tensors[0].device
+    if device.type != "cuda" or not all(t.device == device and t.is_contiguous() for t in tensors):
+        return False
+    return all(t.dtype is torch.int64 for t in whole) and all(t.dtype is torch.float32 for t in real) and hostmath._plain_call(*tensors)
+
+
 def screen_blend(bonus_count: torch.Tensor, damage_count: torch.Tensor, damage_to_alpha: torch.Tensor) -> torch.Tensor:
     """f32 [N,2]: the pickup and damage alphas of ``_native_indexed_to_rgb`` (engine.py:15385-15394).
 
@@ -206,6 +218,17 @@ def screen_blend(bonus_count: torch.Tensor, damage_count: torch.Tensor, damage_t
     tensor get PLAYPAL mixed with gold and then red before the RGB24 frame and the observation.
     """
 
+    if _read_in_place((bonus_count, damage_count), (damage_to_alpha,)) and bonus_count.shape == damage_count.shape and bonus_count.dim() == 1 and damage_to_alpha.numel() >= 114:
+        import ctypes as C
+
+        from . import _lib
+
+        blend = torch.empty((bonus_count.shape[0], 2), dtype=torch.float32, device=bonus_count.device)
+        with torch.cuda.device(blend.device):
+            stream = torch.cuda.current_stream(blend.device).cuda_stream
+            _lib.check(_lib.library().gd_screen_blend(
+                bonus_count.data_ptr(), damage_count.data_ptr(), damage_to_alpha.data_ptr(), bonus_count.shape[0], blend.data_ptr(), C.c_void_p(stream)))
+        return blend
     bonus = torch.minimum(bonus_count.to(torch.float32) * 8.0, torch.full_like(bonus_count, 128.0, dtype=torch.float32))
     flash = damage_to_alpha.to(torch.float32)[damage_count.clamp(0, 113).to(torch.int64)]
     return torch.stack((bonus / 255.0, flash / 255.0), dim=1).contiguous()
@@ -224,6 +247,23 @@ def decal_inputs(serial, wall, along, impact_z, style, portal_walls, fine_sine_f
 
     if serial.shape[1] == 0:
         return None
+    table = torch.as_tensor(fine_sine_fixed)
+    if (_read_in_place((serial, wall, style, table), (along, impact_z, portal_walls)) and serial.dim() == 2 and portal_walls.dim() == 2 and portal_walls.shape[1] == 4
+            and portal_walls.shape[0] > 0 and portal_walls.data_ptr() % 16 == 0 and table.shape == (FINE_ANGLES,) and serial.shape[1] <= 1 << 20
+            and serial.shape == wall.shape == along.shape == impact_z.shape == style.shape):
+        import ctypes as C
+
+        from . import _lib
+
+        lanes, slots = serial.shape
+        state = torch.empty((lanes, slots, 3), dtype=torch.int32, device=serial.device)
+        geom = torch.empty((lanes, slots, 4), dtype=torch.float32, device=serial.device)
+        with torch.cuda.device(serial.device):
+            stream = torch.cuda.current_stream(serial.device).cuda_stream
+            _lib.check(_lib.library().gd_pack_decals(
+                serial.data_ptr(), wall.data_ptr(), along.data_ptr(), impact_z.data_ptr(), style.data_ptr(), portal_walls.data_ptr(), portal_walls.shape[0],
+                table.data_ptr(), lanes, slots, state.data_ptr(), geom.data_ptr(), C.c_void_p(stream)))
+        return state, geom
     serial = serial.to(torch.int64)
     active = serial >= 0
     order = torch.argsort(torch.where(active, serial, torch.full_like(serial, torch.iinfo(torch.int32).max)), dim=1, stable=True)
@@ -238,7 +278,7 @@ def decal_inputs(serial, wall, along, impact_z, style, portal_walls, fine_sine_f
     oriented = torch.where((side == 0)[..., None], vector, -vector)
     angle = torch.atan2(oriented[..., 1], oriented[..., 0])
     fine = torch.floor(torch.remainder(angle, 2.0 * math.pi) * (8192 / (2.0 * math.pi))).to(torch.int64) & 8191
-    table = torch.as_tensor(fine_sine_fixed, dtype=torch.int64).to(serial.device)
+    table = table.to(torch.int64).to(serial.device)
     sine = table[fine].to(torch.float32) / 65536
     cosine = table[(fine + 2048) & 8191].to(torch.float32) / 65536
     state = torch.stack((wall_index, style_index, alive.to(torch.int64)), dim=-1).to(torch.int32).contiguous()

@@ -502,6 +502,18 @@ typedef struct gd_weapon_desc {
 int gd_pack_weapon(const gd_weapon_desc *weapon, void *stream);
 
 /*
+ * gd_pack_decals: gd_lanes_desc.decal_state [N,D,3] and decal_geom [N,D,4] from an engine's decal slots [N,D] (engine.py:13756-13829): the live
+ * ones (serial >= 0) first and oldest first, then the free ones.  walls [wall_count,4] are the map's linedefs, fine_sine the 8192-entry
+ * table in 16.16.
+ * gd_screen_blend: gd_lanes_desc.screen_blend [N,2] from the pickup and damage counters and the 114 alphas of the latter
+ * (engine.py:15385-15394).
+ * All pointers are device pointers to contiguous arrays.  Both return GD_E_ARG for a null pointer or a count out of range.
+ */
+int gd_pack_decals(const int64_t *serial, const int64_t *wall, const float *along, const float *impact_z, const int64_t *style, const float *walls,
+                   int32_t wall_count, const int64_t *fine_sine, int32_t lane_count, int32_t slots, int32_t *decal_state, float *decal_geom, void *stream);
+int gd_screen_blend(const int64_t *bonus_count, const int64_t *damage_count, const float *damage_to_alpha, int32_t lane_count, float *screen_blend, void *stream);
+
+/*
  * The float32 inputs of gd_lanes_desc that the reference evaluates with Torch, in one kernel each; bit for bit what the Torch
  * expressions give on this device (each operation is rounded on its own, cos / sin / atan2 / fmod are the device library's).
  *   gd_ray_tables:    ray_cos / ray_sin [N,320] = cos / sin(angle[n] + ray_offsets[x])                 (engine.py:10966-10974)

@@ -1,0 +1,67 @@
+"""The kernels that pack decal slots and screen flashes against the Torch expressions on the same device (which tensors that are not laid
+out as the kernels read them still take): equal bit for bit."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def spread(tensor: torch.Tensor) -> torch.Tensor:
+    """The same values, every second place of a wider tensor."""
+
+    return torch.stack((tensor, tensor), dim=-1)[..., 0]
+
+
+@pytest.mark.parametrize("slots", [1, 63, 64, 65, 130])
+def test_decal_slots_are_packed_as_the_torch_expressions_pack_them(slots):
+    from gradoom_amd import overlay_inputs
+
+    rng = torch.Generator(device="cuda:0").manual_seed(slots)
+    lanes, linedefs = 37, 4096
+    whole = lambda low, high: torch.randint(low, high, (lanes, slots), generator=rng, device="cuda:0")  # noqa: E731
+    real = lambda *shape: torch.randn(shape, generator=rng, device="cuda:0")  # noqa: E731
+    serial = whole(-20, 40)                                    # free slots, and impacts of one number
+    serial[0] = -1
+    serial[1] = whole(0, 200)[0] + (1 << 31) - 100         # numbers on both sides of a free slot's place in the order
+    wall, style = whole(-2, linedefs + 2), whole(-25, 60)
+    walls = torch.round(real(linedefs, 4) * 300)
+    walls[:64, 2:] = walls[:64, :2]                            # no direction at all
+    walls[64:128, 2] = walls[64:128, 0]                        # along the axes
+    walls[128:192, 3] = walls[128:192, 1]
+    walls[192:1024] = real(832, 4)
+    along, impact = real(lanes, slots), real(lanes, slots)
+    table = torch.as_tensor(overlay_inputs.fine_sine_fixed(), device="cuda:0")
+    state, geometry = overlay_inputs.decal_inputs(serial, wall, along, impact, style, walls, table)
+    expected_state, expected_geometry = overlay_inputs.decal_inputs(spread(serial), wall, along, impact, style, walls, table)
+    assert state.dtype == torch.int32 and torch.equal(state, expected_state)
+    assert geometry.dtype == torch.float32 and torch.equal(geometry.view(torch.int32), expected_geometry.view(torch.int32))
+
+
+def test_every_direction_takes_the_torch_expressions_place_in_the_fine_table():
+    from gradoom_amd import overlay_inputs
+
+    count = 1 << 18
+    turn = torch.arange(count, dtype=torch.float64, device="cuda:0") * (2.0 * torch.pi / count)
+    walls = torch.zeros((count, 4), dtype=torch.float32, device="cuda:0")
+    walls[:, 2], walls[:, 3] = torch.cos(turn).to(torch.float32) * 1000, torch.sin(turn).to(torch.float32) * 1000
+    wall = torch.arange(count, device="cuda:0").reshape(-1, 64)
+    ones = torch.ones_like(wall, dtype=torch.float32)
+    table = torch.as_tensor(overlay_inputs.fine_sine_fixed(), device="cuda:0")
+    for style in (torch.zeros_like(wall), torch.full_like(wall, 20)):
+        packed = overlay_inputs.decal_inputs(wall, wall, ones, ones, style, walls, table)
+        expected = overlay_inputs.decal_inputs(spread(wall), wall, ones, ones, style, walls, table)
+        assert torch.equal(packed[0], expected[0]) and torch.equal(packed[1], expected[1])
+
+
+@pytest.mark.parametrize("lanes", [1, 256, 257])
+def test_screen_flashes_are_packed_as_the_torch_expressions_pack_them(lanes):
+    from gradoom_amd import overlay_inputs
+
+    rng = torch.Generator(device="cuda:0").manual_seed(lanes)
+    bonus = torch.randint(-3, 300, (lanes,), generator=rng, device="cuda:0")
+    damage = torch.randint(-3, 200, (lanes,), generator=rng, device="cuda:0")
+    alphas = torch.rand((114,), generator=rng, device="cuda:0") * 200
+    assert torch.equal(overlay_inputs.screen_blend(bonus, damage, alphas), overlay_inputs.screen_blend(spread(bonus), damage, alphas))
