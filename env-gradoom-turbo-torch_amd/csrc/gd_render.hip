@@ -3711,7 +3711,6 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int str
 // runs the other half over the records (pass_draw, clip_pass, pass_paint, advance_clips, the masked mid-texture).
 // Each half is lighter in registers and in code than the two together, so more of its wavefronts share a SIMD and
 // its pass loop fits the instruction cache.  Same segment order and one wavefront per segment in both.
-#define SELECT_STRIPS_PER_GROUP 1
 // The kernel lasts as long as its longest strips: on the 4000-linedef map the 256 longest of 20,480 take 0.94 ms with the
 // chip to themselves, all of them together 1.22 ms, all but the 4096 longest 0.53 ms.  Such a strip's wavefront is held
 // up by its candidate scans (the longest lists, read from device memory beside 20,000 other wavefronts) and by running,
@@ -3722,31 +3721,14 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int str
 // each, their lists copied to LDS: 16 lanes on the 2000-linedef map 151 -> 68 us, 512 on the 4000-linedef map 463 -> 257, 4096 of them 0.97 -> 0.89 ms.  What the
 // rules ask beyond the list (a sector bridge) they ask behind the scan, once for each entry concerned: a copy of that code for every entry made the
 // kernels larger than the instruction cache.
-static_assert(SEG_COLS == 64 && SELECT_STRIPS_PER_GROUP == 1, "wall_select_kernel's launch for the longest strips: parts of one whole strip per work-group");
+static_assert(SEG_COLS == 64, "wall_select_kernel: a work-group is one wavefront, with columns of one strip");
+// The columns of one wavefront: 64 / LANES of a strip's, from the `part`-th such share on.
 template <bool SPLIT, int LANES>
-__global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kernel(DeviceMap dm, int lane_count, Scratch sc, int longest) {
+__device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratch &sc, const LaneCtx &lane_ctx, int local, int strip_x, int part) {
     const gd_map_desc *m = &dm.d;
-    constexpr bool SHARED = LANES > 1;     // the launch for the longest strips
-    constexpr int parts = LANES, part_cols = 64 / LANES;
-    __shared__ LaneCtx lane_ctxs[SELECT_STRIPS_PER_GROUP][64 / SEG_COLS];
-    const int block = blockIdx.x;
-    const int wave_in_group = threadIdx.x >> 6;
-    const int lane_id = threadIdx.x & 63;
-    const int segment_in_wave = lane_id / SEG_COLS;
-    const int segment_slot = (block / parts * SELECT_STRIPS_PER_GROUP + wave_in_group) * (64 / SEG_COLS) + segment_in_wave;
-    const int part = block % parts, lane_of_column = lane_id & (LANES - 1);
-    const bool live = segment_slot < (SHARED ? longest : lane_count * SEGS_PER_LANE);
-    const int segment = live ? sc.strip_order[segment_slot] : 0;
-    const int local = segment / SEGS_PER_LANE;
-    if ((lane_id & (SEG_COLS - 1)) == 0 && live) lane_ctxs[wave_in_group][segment_in_wave] = sc.ctx[local];
-    __syncthreads();
-    if (!live) return;
-    const LaneCtx &lane_ctx = lane_ctxs[wave_in_group][segment_in_wave];
-    // A strip with a column in the spill pool (more entries than its lanes hold) is left to the other launch, which
-    // covers the longest strips' slots as well and otherwise leaves them alone.  Both ask all 64 columns of the strip.
-    const int strip_x = (segment - local * SEGS_PER_LANE) * SEG_COLS;
-    const bool long_lists = __ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + lane_id] >> SPILL_SHIFT) != 0) != 0;
-    if (SHARED ? long_lists : (segment_slot < longest && !long_lists)) return;   // the same in the whole wavefront
+    constexpr bool SHARED = LANES > 1;
+    constexpr int part_cols = 64 / LANES;
+    const int lane_id = threadIdx.x & 63, lane_of_column = lane_id & (LANES - 1);
     const int x = strip_x + part * part_cols + lane_id / LANES;
     ColumnCtx cc;
     cc.tb = nullptr; cc.m = m; cc.mv.m = m; cc.c = &lane_ctx;
@@ -3832,6 +3814,25 @@ __global__ void __launch_bounds__(64 * SELECT_STRIPS_PER_GROUP) wall_select_kern
         if (__ballot(!done) == 0) break;
     }
     if (lane_of_column == 0) sc.pass_count[(size_t)local * SW + x] = (unsigned char)recorded;
+}
+
+// The strips from `first_slot` on in the order, as many as the grid has wavefronts for.  A strip of the longest that its lanes cannot hold is
+// drawn here too, not in a launch behind this one, which small batches paid 7 us for.  (16 lanes: 130 registers left to itself, 128 as told.)
+template <bool SPLIT, int LANES>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES == 8 ? 3 : 4))) wall_select_kernel(DeviceMap dm, Scratch sc, int first_slot) {
+    __shared__ LaneCtx lane_ctx;
+    const int segment = sc.strip_order[first_slot + (int)blockIdx.x / LANES], part = (int)blockIdx.x % LANES;
+    const int local = segment / SEGS_PER_LANE, strip_x = (segment - local * SEGS_PER_LANE) * SEG_COLS;
+    if (threadIdx.x == 0) lane_ctx = sc.ctx[local];
+    __syncthreads();
+    if constexpr (LANES > 1) {
+        // A strip with a column in the spill pool (more entries than its lanes hold) is the first of its wavefronts', a lane a column.
+        if (__ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + threadIdx.x] >> SPILL_SHIFT) != 0) != 0) {
+            if (part == 0) select_columns<SPLIT, 1>(dm, sc, lane_ctx, local, strip_x, 0);
+            return;
+        }
+    }
+    select_columns<SPLIT, LANES>(dm, sc, lane_ctx, local, strip_x, part);
 }
 
 // One wavefront per 64 / SEG_COLS segments.  Segments share nothing but read-only tables; a work-group of the drawing
@@ -5950,7 +5951,6 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     {
         const int wavefronts = (count * SEGS_PER_LANE + 64 / SEG_COLS - 1) / (64 / SEG_COLS);
         const bool split = m.split_count > 0;
-        const dim3 select_block(64 * SELECT_STRIPS_PER_GROUP);
         // The longest strips here, the others on the side stream, both at once.  This way round: the
         // side stream starts a few microseconds behind, time enough for the longest strips' work-groups to be placed;
         // started together, the other launch's 20,000 take every wavefront slot first and the strips that decide how long
@@ -5960,7 +5960,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         const int longest = r->side_ready ? (strips < longest_wanted ? strips : longest_wanted) : 0;
         auto select_kernel = split ? wall_select_kernel<true, 1> : wall_select_kernel<false, 1>;
         if (longest > 0) {
-            const bool alone = longest == strips;   // the other launch is left with strips of spilled columns: it follows
+            const bool alone = longest == strips;
             if (!alone) {
                 HIP_TRY(hipEventRecord(r->fork_event, stream));
                 HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
@@ -5968,14 +5968,14 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
             const int column_lanes = select_lanes(count, m.wall_count);
             auto pick = [&](auto lanes) { constexpr int L = decltype(lanes)::value; return split ? wall_select_kernel<true, L> : wall_select_kernel<false, L>; };
             auto longest_kernel = column_lanes == 32 ? pick(std::integral_constant<int, 32>()) : (column_lanes == 16 ? pick(std::integral_constant<int, 16>()) : pick(std::integral_constant<int, 8>()));
-            hipLaunchKernelGGL(longest_kernel, dim3(longest * column_lanes), select_block, 0, stream, r->dm, count, sc, longest);
-            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, alone ? stream : r->side_stream, r->dm, count, sc, longest);
+            hipLaunchKernelGGL(longest_kernel, dim3(longest * column_lanes), dim3(64), 0, stream, r->dm, sc, 0);
+            if (!alone) hipLaunchKernelGGL(select_kernel, dim3(strips - longest), dim3(64), 0, r->side_stream, r->dm, sc, longest);
             if (!alone) {
                 HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
                 HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
             }
         } else {
-            hipLaunchKernelGGL(select_kernel, dim3(strips), select_block, 0, stream, r->dm, count, sc, 0);
+            hipLaunchKernelGGL(select_kernel, dim3(strips), dim3(64), 0, stream, r->dm, sc, 0);
         }
         // the billboards' lists beside the walls' drawing, on the side stream (when stages are being timed, with the billboards)
         if (has_billboards && !fused && !timed) {
