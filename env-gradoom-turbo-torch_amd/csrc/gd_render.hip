@@ -9,8 +9,9 @@
 //                                             nearest blocking hit of every column (64-bit atomicMin)
 //   strip_key/order 1 thread / 64-col strip   longest strip first (counting sort on the longest list); columns that see more than 64 linedefs
 //   wall_select     1 wave / strip            portal traversal: which drawseg every column pass selects, one record each
+//                   (the longest: 8 to 32)
 //   wall_geometry   13 to 21 waves / lane            the linedefs those passes draw, as lines over the columns: every division of the drawing
-//   wall_raster     1 wave / strip            the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
+//   wall_raster     1 to 8 waves / strip      the recorded passes drawn: projection, clips, tiers, planes, masked mid-textures
 //   plane_shade     1 wave / 64 columns x 16 rows  flat texel + light for every pixel a plane of the wall pass shows,
 //                                             the wall tiers' palette indices
 //   flat_gap        8 or 16 waves / gap column     per-pixel plane rays (fine point raster) for the gap pixels, vertical repair

@@ -39,7 +39,8 @@ def test_batches_around_the_sizes_of_the_traversals_rules_match_the_oracle(oracl
 
 @pytest.mark.parametrize("rule", ["selection", "four_parts", "two_parts"])
 def test_batches_on_both_sides_of_a_sharing_rules_line_match_the_oracle(oracle, rule):
-    """The first of them depends on the map's linedefs: see select_finely and raster_parts in gd_render.hip."""
+    """Lines that sharing rules have had, the first of them following the map's linedefs.  (Where they lie now: test_gpu_shared_columns.py and
+    test_gpu_shared_lists.py.)"""
 
     from gradoom_amd import hostmath, mapbuild
     from gradoom_amd.renderer import HipRenderer, LaneState
