@@ -218,7 +218,8 @@ def screen_blend(bonus_count: torch.Tensor, damage_count: torch.Tensor, damage_t
     tensor get PLAYPAL mixed with gold and then red before the RGB24 frame and the observation.
     """
 
-    if _read_in_place((bonus_count, damage_count), (damage_to_alpha,)) and bonus_count.shape == damage_count.shape and bonus_count.dim() == 1 and damage_to_alpha.numel() >= 114:
+    if (_read_in_place((bonus_count, damage_count), (damage_to_alpha,)) and bonus_count.shape == damage_count.shape and bonus_count.dim() == 1
+            and damage_to_alpha.dim() == 1 and damage_to_alpha.shape[0] >= 114):
         import ctypes as C
 
         from . import _lib

@@ -65,3 +65,26 @@ def test_screen_flashes_are_packed_as_the_torch_expressions_pack_them(lanes):
     damage = torch.randint(-3, 200, (lanes,), generator=rng, device="cuda:0")
     alphas = torch.rand((114,), generator=rng, device="cuda:0") * 200
     assert torch.equal(overlay_inputs.screen_blend(bonus, damage, alphas), overlay_inputs.screen_blend(spread(bonus), damage, alphas))
+
+
+@pytest.mark.parametrize("shape", [(114, 1), (1, 114), (2, 114)])
+def test_a_table_of_alphas_with_two_dimensions_is_refused_as_the_torch_expressions_refuse_it(shape):
+    from gradoom_amd import overlay_inputs
+
+    bonus = torch.arange(5, device="cuda:0")
+    damage = torch.arange(5, device="cuda:0").clamp(max=shape[0] - 1)      # every index the expressions take lies in the table
+    alphas = torch.ones(shape, device="cuda:0")
+    for counters in ((bonus, damage), (bonus.cpu(), damage.cpu())):
+        with pytest.raises(RuntimeError, match="stack expects each tensor to be equal size"):
+            overlay_inputs.screen_blend(*counters, alphas.to(counters[0].device))
+
+
+def test_screen_flashes_of_other_shapes_are_packed_as_on_the_host():
+    from gradoom_amd import overlay_inputs
+
+    bonus, damage, alphas = torch.arange(6) * 5, torch.arange(6) * 40 - 20, torch.arange(200, dtype=torch.float32)
+    for counters in ((bonus, damage, alphas), (bonus[:, None], damage, alphas[:, None]), (bonus[:, None], damage[:, None], alphas), (bonus[:0], damage[:0], alphas)):
+        packed = overlay_inputs.screen_blend(*(t.to("cuda:0") for t in counters))
+        expected = overlay_inputs.screen_blend(*counters)
+        # the device multiplies with the divisor's reciprocal: two roundings of 2^-24 where the host's division has one
+        assert packed.shape == expected.shape and torch.allclose(packed.cpu(), expected, rtol=2.0**-22, atol=0)
