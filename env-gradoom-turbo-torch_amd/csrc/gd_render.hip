@@ -44,6 +44,7 @@
 
 #include "../../include/gradoom_amd.h"
 #include "gd_internal.h"
+#include "gd_rules.h"
 
 thread_local std::string g_error;
 int gd_fail(int code, const std::string &message) { g_error = message; return code; }
@@ -833,13 +834,7 @@ __device__ __forceinline__ void note_length(const Scratch &sc, int local, int x,
 // Bound by its vector instructions, then by the latency of a turn's steps.  4096 lanes on the 4000-linedef map: 0.61 ms with two looks a
 // column (one for the hits, one for the candidates), parameters by lane exchange and counts by atomics in device memory, 0.53 with one
 // look and LDS parameters, 0.45 with counts in LDS; 16 lanes on the 320-linedef map 0.040 -> 0.019.
-#define SETUP_THREADS 256
 #define SETUP_WHOLE_THREADS 512
-// A work-group takes a whole lane where there are lanes enough for the chip, and where a lane's linedefs would be two work-groups at
-// most anyway.  Stages up to the strips' order in us, dealt out / whole lanes: 120 linedefs, 16 lanes 48 / 37, 512 lanes 57 / 51; 320, 16 lanes 51 / 45,
-// 512 lanes 67 / 58; 701, 16 lanes 49 / 55, 640 lanes 75 / 76; 1400, 256 lanes 64 / 73, 768 lanes 99 / 97, 1024 lanes 115 / 114; 2000, 256 lanes
-// 68 / 104, 768 lanes 106 / 114, 1024 lanes 126 / 123; 4000, 256 lanes 79 / 116, 768 lanes 152 / 159, 1024 lanes 188 / 179, 4096 lanes 708 / 509.
-bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || linedefs <= 2 * SETUP_THREADS; }
 #define SETUP_WALLS_MAX 4096      // linedefs sorted at a time
 struct SetupWall {                // a linedef as the columns' look at it asks for it
     float segx, segy, offx, offy;
@@ -1597,10 +1592,6 @@ __device__ __forceinline__ void note_row(const Scratch &sc, int local, int half,
 // GAP_WAVES wavefronts a column, which probe four rows each at a time: first the gap pixels', then the others' from the topmost
 // unresolved gap pixel down, until the lowest one is past and a resolved pixel below it is found (or the half ends).
 #define ROW_UNPROBED -2
-// The fewer the lanes, the fewer such columns and the longer the kernel lasts as its slowest one.  us with 4 / 8 / 16 wavefronts a column: 512
-// lanes 95 / 71 / 62, 1024 lanes (2000 linedefs) 100 / 64 / 52, 4096 lanes 118 / 115 / 141; the whole selection at 2048 lanes of 800, 2000 and
-// 4000 linedefs 164 / 153 / 161, 179 / 144 / 152, 253 / 221 / 230, at 1024 lanes 136 / 111 / 111, 146 / 112 / 97, 193 / 160 / 146.
-int gap_waves(int lanes) { return lanes <= 1536 ? 16 : 8; }
 template <int GAP_WAVES>
 __global__ void __launch_bounds__(64 * GAP_WAVES) flat_gap_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
     __shared__ ProbeLds probe_lds[GAP_WAVES];
@@ -2009,30 +2000,6 @@ __global__ void __launch_bounds__(SW) flat_span_finish_kernel(Scratch sc) {
 // walls: engine.py:11462-13745
 // ---------------------------------------------------------------------------------------------
 #define CAND_BATCH 8
-// wall_select_kernel's launch for the longest strips: how many of them, and how many lanes a column has there.  More strips and more lanes
-// shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a
-// large one's does.  Where the lists are short (they follow the map's linedefs) there is little to shorten: none where the lanes are as many
-// as six times the linedefs beyond 160.  Stage times in us of no such launch / 768 strips (1024 from 1400 linedefs on) of 8 / of 16 lanes
-// (of 32), in brackets what it took with the lists in LDS and 8 columns of one lane a wavefront:
-//   lanes       120              320                        800                         2000                          4000
-//      16    46 / 55 / 76     97 / 53 / 64 (61; [60])    168 / 74 / 62 (52)         339 / 120 / 89 (68; [151])     361 / 119 / 90 (69; [156])
-//     128    55 / 60 / 77     133 / 69 / 81 ([83])       181 / 83 / 71              436 / 153 / 113 (104; [203])   1003 / 236 / 172 (145; [430])
-//     256    59 / 73          137 / 84 / 96 ([102])      212 / 106 / 99             447 / 164 / 132 ([214])        999 / 247 / 197 ([420])
-//     512    63 / 81          140 / 107 / 119 ([111])    220 / 126 / 128            453 / 172 / 178 ([267])        1003 / 275 / 257 ([463])
-//    1024    69               149 / 146 ([138])          241 / 174 / 174            520 / 265 / 264 ([336])        1060 / 408 / 413 ([563])
-//    2048    80               166 / 180 ([171])          277 / 234 / 235            549 / 371 / 370 ([411])        1120 / 652 / 647 ([727])
-//    4096    130              230 / 288 ([279])          328 / 363                  667 / 604 / 576 ([600])        1249 / 945 / 887 ([966])
-// (the last two rows with 768 and with 512 strips.)
-int select_strips(int lanes, int linedefs) {
-    if (lanes >= 6 * (linedefs - 160)) return 0;
-    return lanes < 1792 ? (linedefs < 1024 ? 768 : 1024) : (lanes < 3584 ? 768 : 512);
-}
-int select_lanes(int lanes, int linedefs) {
-    const int w = linedefs < 4096 ? linedefs : 4096;      // no map of more was timed
-    if (w < 512) return 8;
-    if (lanes <= 64 + w / 24) return 32;
-    return lanes <= 128 + w / 8 || (lanes >= 1536 && w >= 1024) ? 16 : 8;
-}
 #define WALL_ROWS 8          // rows painted / clipped per step of the wall traversal
 struct ColumnCtx {
     const Tables *tb;
@@ -3577,9 +3544,7 @@ __device__ __forceinline__ void wall_lines(const DeviceMap &dm, const LaneCtx &c
 // with rows of their own.  4096 lanes on the 4000-linedef map draw 1.3 million linedefs: 0.34 ms by one work-group a lane, whose 320 threads
 // waited at barriers for the slowest, 0.29 by wavefronts that do strips after linedefs, 0.24 side by side in work-groups of four, 0.226 now;
 // 512 lanes 0.084 -> 0.045, 16 lanes of the 320-linedef map 0.012 -> 0.008.  It waits for records and heights, then for its stores.
-// Wavefronts a lane for linedefs, 4 / 8 / 16, in us: 16 lanes 13.6 / 10.7 / 8.3, 512 lanes 63 / 48 / 46, 1024 lanes 48 / 41 / 42, 4096 lanes 263 / 242 / 247.
 #define GEO_LIST 64                              // linedefs a wavefront lists at a time
-int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
 template <bool SPLIT>
 __global__ void __launch_bounds__(64) wall_geometry_kernel(DeviceMap dm, int lane_count, Scratch sc, int parts) {
     const gd_map_desc *m = &dm.d;
@@ -3856,25 +3821,6 @@ __device__ __forceinline__ PassDraw hand_round(const PassDraw &prepared, int k, 
     d.distance = __uint_as_float(take(__float_as_uint(prepared.distance)));
     return d;
 }
-// A strip's wavefront draws, pass after pass, the rows that any of its columns draws.  A small batch, which lasts as long as its
-// longest strips, shares a strip out over eight wavefronts, a larger one over four, over two.  The wavefront's columns then have eight,
-// four or two lanes each: these prepare as many passes at once and share every run of rows out, so that both the chain of waits and the
-// vector instructions of a column shrink with them (when the spare lanes stood idle, eight wavefronts never paid).  What a strip more
-// wavefronts costs is room on the SIMDs.  Stage times in us (wall_geometry_kernel among them) for 1 / 2 / 4 / 8 wavefronts a
-// strip, in brackets with idle lanes and the lines of then (four up to 560 lanes, two up to 1344):
-//   lanes           320 linedefs                     2000                             4000                             701, bricks
-//      16         / 90 / 72 / 65 (106)            / 136 / 110 / 97 (155)           / 184 / 149 / 139 (196)          / 263 / 218 / 188 (285)
-//     256        / 142 / 119 / 113 (155)         / 198 / 161 / 145 (212)          / 328 / 259 / 229 (327)          / 291 / 238 / 208 (310)
-//     384        / 148 / 121 / 136 (174)         / 206 / 175 / 170 (229)          / 349 / 276 / 274 (345)          / 298 / 247 / 219 (322)
-//     512        / 156 / 126 / 175 (202)         / 219 / 189 / 222 (250)          / 425 / 401 / 367 (480)          / 313 / 256 / 249 (318)
-//     640        / 165 / 156 / 222 (202)         / 233 / 204 / 279 (277)          / 432 / 416 / 394 (498)          / 346 / 273 / 309 (408)
-//     768     235 / 173 / 187 / 270 (214)     328 / 239 / 236 / 333 (282)      527 / 445 / 422 / 457 (513)      430 / 345 / 283 / 371 (415)
-//    1024     253 / 204 / 233 / 351 (249)     385 / 270 / 303 / 437 (330)      555 / 466 / 445 / 598 (539)      449 / 354 / 334 / 487 (431)
-//    1536     294 / 287 / 342 (298)           438 / 383 / 440 (448)            597 / 528 / 630 (619)            479 / 392 / 490 (501)
-//    2048     365 / 357 / 450 (364)           492 / 478 / 583 (487)            701 / 674 / 835 (695)            524 / 509 / 643 (536)
-//    2560     439 / 425 (440)                 596 / 589 (583)                  831 / 845 (820)                  639 / 625 (649)
-//    3072     519 / 542 (514)                 700 / 722 (683)                  930 / 969 (918)                  751 / 744 (753)
-__host__ __device__ constexpr int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 2400 ? 2 : 1)); }
 // DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
 // BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
@@ -4454,13 +4400,6 @@ __global__ void __launch_bounds__(LIST_THREADS) sprite_list_kernel(DeviceMap dm,
 #define SPRITE_TILES 4        // tiles of a wavefront whose words are asked for together
 #define SPRITE_CHUNK 64
 #define SPRITE_COLUMNS 64     // a work-group for the whole lane: 0.95 ms instead of 0.70 (4 wavefronts), 0.86 (8)
-#define SPRITE_ROW_PARTS 4    // of a small batch's work-groups
-// Lanes from which a work-group takes all rows of its columns: fewer listings, but the last work-groups last longer.  Quarters and whole
-// columns cost the same at 230 (4000 linedefs, 128 billboards) to 1100 lanes (320 linedefs, 32 billboards); the line lies between.  us, quarters /
-// whole columns, two sets of poses each: 320 linedefs, 32 billboards, 256 lanes 66 / 97, 512 lanes 101 / 122, 1024 lanes 170 / 174; with 128
-// 105 / 139, 174 / 179, 336 / 296; 2000 linedefs with 128 128 / 117, 170 / 144, 256 / 212; 4000 with 32 81 / 90, 125 / 125, 185 / 172; with 128 186 /
-// 172, 218 / 192, 299 / 250; 4096 lanes of it 840 / 700.
-#define SPRITE_TALL_LANES 512
 static_assert(SPRITE_COLUMNS == 64 && SW % SPRITE_COLUMNS == 0 && VH % (SPRITE_ROW_PARTS * SPRITE_TILE_H) == 0 && VH <= SPRITE_THREADS, "sprite_pixels_kernel: whole tiles");
 static_assert(SPRITE_CHUNK == 64 && SPRITE_CHUNK <= SPRITE_THREADS, "sprite_pixels_kernel: a bit an entry");
 __global__ void __launch_bounds__(SPRITE_THREADS, 5) sprite_pixels_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
@@ -5902,13 +5841,6 @@ int validate_map(const gd_map_desc *h) {
 
 const int STAGE_COUNT = 9;
 
-// A frame that goes to the side stream and back pays some 20 us for it.  Batches of up to 102 lanes do without
-// where there is little to put there: no billboards, or a few lanes.  A frame in us with / without, 1 lane with billboards on 120 to 4000
-// linedefs 139 / 119, 261 / 236, 210 / 185, 243 / 235, 433 / 414, 8 lanes 256 / 285, 284 / 259, 293 / 312, 396 / 394, 450 / 428, 48 lanes
-// 323 / 356, 405 / 436, 439 / 468, 586 / 611, 878 / 891; without billboards on 320, 800 and 4000 linedefs, 16 lanes 256 / 241, 364 / 351,
-// 533 / 520, 64 lanes 437 / 429, 434 / 426, 884 / 878.
-bool side_stream_pays(int lanes, bool billboards) { return lanes > 102 || (billboards && lanes >= 4); }
-
 int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_desc *lanes, const gd_frame_out *out, int base, int count, hipStream_t stream, bool timed) {
     const gd_map_desc &m = r->dm.d;
     Scratch sc = chunk_scratch;
@@ -6041,7 +5973,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     const bool billboards_split = beside && has_billboards && !decals;
     const bool may_blend = lanes->sprite_style != nullptr;   // without styles no lane blends: the launches for such lanes are left out
     auto paint_billboards = [&](hipStream_t on, int lane_pick) {
-        hipLaunchKernelGGL(sprite_pixels_kernel, dim3(SW / SPRITE_COLUMNS, count, count >= SPRITE_TALL_LANES ? 1 : SPRITE_ROW_PARTS), dim3(SPRITE_THREADS), 0, on, r->dm, *lanes, base, count, sc, frame_base, frame_stride, lane_pick);
+        hipLaunchKernelGGL(sprite_pixels_kernel, dim3(SW / SPRITE_COLUMNS, count, sprite_row_parts(count)), dim3(SPRITE_THREADS), 0, on, r->dm, *lanes, base, count, sc, frame_base, frame_stride, lane_pick);
     };
     if (!fused && !(billboards_split && !may_blend)) hipLaunchKernelGGL(flat_shade_kernel, flat_grid(4, 4096), dim3(64), 0, stream, r->dm, sc, frame_base, frame_stride, billboards_split ? LANES_BLENDING : LANES_ALL);
     if (beside) {

@@ -1,0 +1,84 @@
+// How a frame's launches are cut, by the lanes of a chunk and the linedefs of its map.  Host code without any of the library's types, so
+// that tests can ask each rule where it changes its answer and render on both sides.
+#ifndef GD_RULES_H
+#define GD_RULES_H
+
+#define SETUP_THREADS 256     // linedefs of a work-group that shares a lane's
+// wall_setup_kernel: a work-group takes a whole lane where there are lanes enough for the chip, and where a lane's linedefs would be two
+// work-groups at most anyway.  Stages up to the strips' order in us, dealt out / whole lanes: 120 linedefs, 16 lanes 48 / 37, 512 lanes
+// 57 / 51; 320, 16 lanes 51 / 45, 512 lanes 67 / 58; 701, 16 lanes 49 / 55, 640 lanes 75 / 76; 1400, 256 lanes 64 / 73, 768 lanes 99 / 97, 1024 lanes
+// 115 / 114; 2000, 256 lanes 68 / 104, 768 lanes 106 / 114, 1024 lanes 126 / 123; 4000, 256 lanes 79 / 116, 768 lanes 152 / 159, 1024 lanes
+// 188 / 179, 4096 lanes 708 / 509.
+inline bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || linedefs <= 2 * SETUP_THREADS; }
+
+// wall_select_kernel's launch for the longest strips: how many of them, and how many lanes a column has there.  More strips and more lanes
+// shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a
+// large one's does.  Where the lists are short (they follow the map's linedefs) there is little to shorten: none where the lanes are as many
+// as six times the linedefs beyond 160.  Stage times in us of no such launch / 768 strips (1024 from 1400 linedefs on) of 8 / of 16 lanes
+// (of 32), in brackets what it took with the lists in LDS and 8 columns of one lane a wavefront:
+//   lanes       120              320                        800                         2000                          4000
+//      16    46 / 55 / 76     97 / 53 / 64 (61; [60])    168 / 74 / 62 (52)         339 / 120 / 89 (68; [151])     361 / 119 / 90 (69; [156])
+//     128    55 / 60 / 77     133 / 69 / 81 ([83])       181 / 83 / 71              436 / 153 / 113 (104; [203])   1003 / 236 / 172 (145; [430])
+//     256    59 / 73          137 / 84 / 96 ([102])      212 / 106 / 99             447 / 164 / 132 ([214])        999 / 247 / 197 ([420])
+//     512    63 / 81          140 / 107 / 119 ([111])    220 / 126 / 128            453 / 172 / 178 ([267])        1003 / 275 / 257 ([463])
+//    1024    69               149 / 146 ([138])          241 / 174 / 174            520 / 265 / 264 ([336])        1060 / 408 / 413 ([563])
+//    2048    80               166 / 180 ([171])          277 / 234 / 235            549 / 371 / 370 ([411])        1120 / 652 / 647 ([727])
+//    4096    130              230 / 288 ([279])          328 / 363                  667 / 604 / 576 ([600])        1249 / 945 / 887 ([966])
+// (the last two rows with 768 and with 512 strips.)
+inline int select_strips(int lanes, int linedefs) {
+    if (lanes >= 6 * (linedefs - 160)) return 0;
+    return lanes < 1792 ? (linedefs < 1024 ? 768 : 1024) : (lanes < 3584 ? 768 : 512);
+}
+inline int select_lanes(int lanes, int linedefs) {
+    const int w = linedefs < 4096 ? linedefs : 4096;      // no map of more was timed
+    if (w < 512) return 8;
+    if (lanes <= 64 + w / 24) return 32;
+    return lanes <= 128 + w / 8 || (lanes >= 1536 && w >= 1024) ? 16 : 8;
+}
+
+// wall_geometry_kernel: wavefronts a lane for its linedefs (a power of two).  us with 4 / 8 / 16 of them: 16 lanes 13.6 / 10.7 / 8.3, 512 lanes
+// 63 / 48 / 46, 1024 lanes 48 / 41 / 42, 4096 lanes 263 / 242 / 247.
+inline int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
+
+// wall_raster_kernel: wavefronts a strip.  One draws, pass after pass, the rows that any of its columns draws.  A small batch, which lasts as
+// long as its longest strips, shares a strip out over eight wavefronts, a larger one over four, over two.  The wavefront's columns then have
+// eight, four or two lanes each: these prepare as many passes at once and share every run of rows out, so that both the chain of waits and
+// the vector instructions of a column shrink with them (when the spare lanes stood idle, eight wavefronts never paid).  What a strip more
+// wavefronts costs is room on the SIMDs.  Stage times in us (wall_geometry_kernel among them) for 1 / 2 / 4 / 8 wavefronts a
+// strip, in brackets with idle lanes and the lines of then (four up to 560 lanes, two up to 1344):
+//   lanes           320 linedefs                     2000                             4000                             701, bricks
+//      16         / 90 / 72 / 65 (106)            / 136 / 110 / 97 (155)           / 184 / 149 / 139 (196)          / 263 / 218 / 188 (285)
+//     256        / 142 / 119 / 113 (155)         / 198 / 161 / 145 (212)          / 328 / 259 / 229 (327)          / 291 / 238 / 208 (310)
+//     384        / 148 / 121 / 136 (174)         / 206 / 175 / 170 (229)          / 349 / 276 / 274 (345)          / 298 / 247 / 219 (322)
+//     512        / 156 / 126 / 175 (202)         / 219 / 189 / 222 (250)          / 425 / 401 / 367 (480)          / 313 / 256 / 249 (318)
+//     640        / 165 / 156 / 222 (202)         / 233 / 204 / 279 (277)          / 432 / 416 / 394 (498)          / 346 / 273 / 309 (408)
+//     768     235 / 173 / 187 / 270 (214)     328 / 239 / 236 / 333 (282)      527 / 445 / 422 / 457 (513)      430 / 345 / 283 / 371 (415)
+//    1024     253 / 204 / 233 / 351 (249)     385 / 270 / 303 / 437 (330)      555 / 466 / 445 / 598 (539)      449 / 354 / 334 / 487 (431)
+//    1536     294 / 287 / 342 (298)           438 / 383 / 440 (448)            597 / 528 / 630 (619)            479 / 392 / 490 (501)
+//    2048     365 / 357 / 450 (364)           492 / 478 / 583 (487)            701 / 674 / 835 (695)            524 / 509 / 643 (536)
+//    2560     439 / 425 (440)                 596 / 589 (583)                  831 / 845 (820)                  639 / 625 (649)
+//    3072     519 / 542 (514)                 700 / 722 (683)                  930 / 969 (918)                  751 / 744 (753)
+inline int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 2400 ? 2 : 1)); }
+
+// flat_gap_kernel: wavefronts a column.  The fewer the lanes, the fewer such columns and the longer the kernel lasts as its slowest one.  us
+// with 4 / 8 / 16 wavefronts a column: 512 lanes 95 / 71 / 62, 1024 lanes (2000 linedefs) 100 / 64 / 52, 4096 lanes 118 / 115 / 141; the whole
+// selection at 2048 lanes of 800, 2000 and 4000 linedefs 164 / 153 / 161, 179 / 144 / 152, 253 / 221 / 230, at 1024 lanes 136 / 111 / 111,
+// 146 / 112 / 97, 193 / 160 / 146.
+inline int gap_waves(int lanes) { return lanes <= 1536 ? 16 : 8; }
+
+// sprite_pixels_kernel: work-groups that share the rows of a block of columns.  From 512 lanes on one takes them all: fewer listings, but the
+// last work-groups last longer.  Quarters and whole columns cost the same at 230 (4000 linedefs, 128 billboards) to 1100 lanes (320 linedefs,
+// 32 billboards); the line lies between.  us, quarters / whole columns, two sets of poses each: 320 linedefs, 32 billboards, 256 lanes 66 / 97,
+// 512 lanes 101 / 122, 1024 lanes 170 / 174; with 128 105 / 139, 174 / 179, 336 / 296; 2000 linedefs with 128 128 / 117, 170 / 144, 256 / 212; 4000
+// with 32 81 / 90, 125 / 125, 185 / 172; with 128 186 / 172, 218 / 192, 299 / 250; 4096 lanes of it 840 / 700.
+#define SPRITE_ROW_PARTS 4
+inline int sprite_row_parts(int lanes) { return lanes >= 512 ? 1 : SPRITE_ROW_PARTS; }
+
+// A frame that goes to the side stream and back pays some 20 us for it.  Batches of up to 102 lanes do without
+// where there is little to put there: no billboards, or a few lanes.  A frame in us with / without, 1 lane with billboards on 120 to 4000
+// linedefs 139 / 119, 261 / 236, 210 / 185, 243 / 235, 433 / 414, 8 lanes 256 / 285, 284 / 259, 293 / 312, 396 / 394, 450 / 428, 48 lanes
+// 323 / 356, 405 / 436, 439 / 468, 586 / 611, 878 / 891; without billboards on 320, 800 and 4000 linedefs, 16 lanes 256 / 241, 364 / 351,
+// 533 / 520, 64 lanes 437 / 429, 434 / 426, 884 / 878.
+inline bool side_stream_pays(int lanes, bool billboards) { return lanes > 102 || (billboards && lanes >= 4); }
+
+#endif

@@ -18,6 +18,7 @@ CAMERAS, SLOTS = 16, 64
 @pytest.mark.parametrize("chips", [False, True])
 @pytest.mark.parametrize("inverted", [False, True])
 def test_batches_at_the_lines_of_the_columns_shares_match_the_oracle(oracle, inverted, chips):
+    import launch_rules
     from conftest import ROOT
     from gradoom_amd import hostmath, mapbuild, overlay_inputs, synthmap
     from gradoom_amd.renderer import HipRenderer, LaneState
@@ -46,7 +47,9 @@ def test_batches_at_the_lines_of_the_columns_shares_match_the_oracle(oracle, inv
     oracle.set_overlays(overlays)
     expected = torch.as_tensor(oracle.render(tables, arrays, cosine)["indexed"]).to("cuda:0")
     oracle.set_overlays(None)
-    for lanes in (1, 336, 337, 704, 705, 2400, 2401):          # raster_parts in gd_render.hip
+    lines = launch_rules.lines("raster_parts")
+    assert len(lines) == 3
+    for lanes in sorted({1} | set(lines) | {line - 1 for line in lines}):
         print(f"{lanes} lanes", flush=True)
         which = np.arange(lanes) % CAMERAS
         renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)

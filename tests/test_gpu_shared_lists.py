@@ -15,6 +15,7 @@ CAMERAS = 4
 @pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("linedefs", [320, 700, 1100])
 def test_batches_at_the_lines_of_the_lists_shares_match_the_oracle(oracle, linedefs, split):
+    import launch_rules
     from gradoom_amd import hostmath, mapbuild, synthmap
     from gradoom_amd.renderer import HipRenderer, LaneState
     from gradoom_amd.selfcheck import make_lane_arrays
@@ -31,13 +32,8 @@ def test_batches_at_the_lines_of_the_lists_shares_match_the_oracle(oracle, lined
     expected = torch.as_tensor(oracle.render(tables, arrays, cosine)["indexed"]).to("cuda:0")
     count = len(tables["walls"])
     assert count >= linedefs
-    strips = 768 if count < 1024 else 1024                                           # select_strips and select_lanes in gd_render.hip
-    lines = {strips // 5 + 1, 64 + count // 24 + 1, 128 + count // 8 + 1}            # the first batch beyond each
-    none_longest = 6 * (count - 160)
-    if none_longest <= 1600:
-        lines.add(none_longest)
-    if count >= 1024:
-        lines.add(1536)
+    lines = {launch_rules.ask("select_strips", 1, count) // 5 + 1}                   # the first batch beyond each: some strips are not among the longest
+    lines.update(launch_rules.lines("select_strips", count), launch_rules.lines("select_lanes", count))
     for lanes in sorted({1} | lines | {line - 1 for line in lines}):
         print(f"{count} linedefs: {lanes} lanes", flush=True)
         which = np.arange(lanes) % CAMERAS
