@@ -13,8 +13,9 @@ inline bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || 
 
 // wall_select_kernel's launch for the longest strips: how many of them, and how many lanes a column has there.  More strips and more lanes
 // shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a
-// large one's does.  Where the lists are short (they follow the map's linedefs) there is little to shorten: none where the lanes are as many
-// as six times the linedefs beyond 160.  Stage times in us of no such launch / 768 strips (1024 from 1400 linedefs on) of 8 / of 16 lanes
+// large one's does.  Where the lists are short (they follow the map's linedefs) there is little to shorten: fewer strips in large batches, and none
+// where the lanes are as many as twelve times the linedefs beyond a hundred, in the largest batches of up to 900 linedefs, or on the
+// smallest maps.  Stage times in us of no such launch / 768 strips (1024 from 1024 linedefs on) of 8 / of 16 lanes
 // (of 32), in brackets what it took with the lists in LDS and 8 columns of one lane a wavefront:
 //   lanes       120              320                        800                         2000                          4000
 //      16    46 / 55 / 76     97 / 53 / 64 (61; [60])    168 / 74 / 62 (52)         339 / 120 / 89 (68; [151])     361 / 119 / 90 (69; [156])
@@ -24,10 +25,26 @@ inline bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || 
 //    1024    69               149 / 146 ([138])          241 / 174 / 174            520 / 265 / 264 ([336])        1060 / 408 / 413 ([563])
 //    2048    80               166 / 180 ([171])          277 / 234 / 235            549 / 371 / 370 ([411])        1120 / 652 / 647 ([727])
 //    4096    130              230 / 288 ([279])          328 / 363                  667 / 604 / 576 ([600])        1249 / 945 / 887 ([966])
-// (the last two rows with 768 and with 512 strips.)
+// (the last two rows with 768 and with 512 strips.)  None / 256 / 512 / 768 strips of 8 lanes on maps below 1024 linedefs, in brackets as above:
+//   lanes         200 linedefs            240                   320                330, bricks               500                701, bricks               1000
+//     256    93/ 72/ 64/ 67 ( 67)   91/ 72/ 66/ 66 ( 72)  136/ 97/ 82/ 83 (104)  154/109/ 89/ 92 (105)  159/107/ 85/ 87 (116)  294/160/127/129 (166)
+//     512    97/ 84/ 80/ 85 ( 79)   95/ 92/ 83/ 80 ( 81)  138/121/109/105 (111)  176/131/120/112 (127)  198/131/123/115 (127)  303/188/176/151 (190)
+//     768   101/ 97/ 91/ 96 ( 90)   98/ 99/ 90/ 92 ( 89)  145/134/127/127 (128)  182/142/144/135 (145)  200/160/144/146 (148)  321/240/204/195 (210)  351/219/194/183 (215)
+//    1024   105/102/ 98/106 ( 97)  102/106/101/103 (100)  147/138/142/141 (138)  190/150/151/152 (150)  204/165/160/158 (160)  325/265/227/215 (231)  360/249/231/205 (235)
+//    1280   107/107/110/111 (108)  104/109/112/110 (110)  151/147/151/151 (146)  200/160/162/159 (162)  211/177/174/171 (173)  340/273/243/234 (250)  369/267/240/218 (248)
+//    1536   109/116/113/120 (113)  108/118/115/115 (115)  157/155/159/163 (157)  203/169/172/169 (171)  216/181/187/188 (186)  350/297/269/255 (280)  381/281/252/244 (263)
+//    2048   116/122/128/139 (124)  114/128/124/131 (125)  165/166/177/191 (170)  214/190/188/198 (184)  239/198/209/223 (206)  363/310/298/303 (312)  386/298/282/290 (296)
+//    2560   120/137/145/157 (137)  120/142/138/148 (132)  179/192/204/218 (194)  224/199/209/222 (200)  249/224/238/252 (228)  379/330/335/353 (344)  402/334/321/340 (326)
+//    3072   127/153/162/173 (153)  137/148/154/164 (146)  188/219/232/246 (220)  231/225/238/251 (225)  260/255/268/285 (259)  395/369/385/402 (372)  424/356/366/382 (358)
+//    4096   150/189/197/209 (189)  148/184/190/200 (182)  227/276/289/306 (279)  252/289/301/314 (288)  284/326/342/359 (332)  425/466/483/500 (472)  475/449/465/482 (458)
+// Over these and thirteen more maps of 60 to 800 linedefs, 16 to 4096 lanes, the rule's choice takes 1.2 % more in the mean than the best of the
+// four, 16 % at most.  Against the brackets' it is 7 % faster in the geometric mean; it is more than 5 % slower on maps of up to 240 linedefs
+// (by 4 to 12 us, mostly at 48 to 384 lanes) and at two places on 280.
 inline int select_strips(int lanes, int linedefs) {
-    if (lanes >= 6 * (linedefs - 160)) return 0;
-    return lanes < 1792 ? (linedefs < 1024 ? 768 : 1024) : (lanes < 3584 ? 768 : 512);
+    if (linedefs <= 128 || lanes >= 12 * (linedefs - 100) || (lanes >= 3584 && linedefs < 900)) return 0;
+    if (linedefs < 512) return lanes < 832 ? 768 : (lanes < 1152 ? 512 : 256);
+    if (linedefs < 1024) return lanes < 2304 ? 768 : (lanes < 2816 ? 512 : 256);
+    return lanes < 1792 ? 1024 : (lanes < 3584 ? 768 : 512);
 }
 inline int select_lanes(int lanes, int linedefs) {
     const int w = linedefs < 4096 ? linedefs : 4096;      // no map of more was timed
