@@ -91,11 +91,23 @@ inline int gap_waves(int lanes) { return lanes <= 1536 ? 16 : 8; }
 #define SPRITE_ROW_PARTS 4
 inline int sprite_row_parts(int lanes) { return lanes >= 512 ? 1 : SPRITE_ROW_PARTS; }
 
-// A frame that goes to the side stream and back pays some 20 us for it.  Batches of up to 102 lanes do without
-// where there is little to put there: no billboards, or a few lanes.  A frame in us with / without, 1 lane with billboards on 120 to 4000
-// linedefs 139 / 119, 261 / 236, 210 / 185, 243 / 235, 433 / 414, 8 lanes 256 / 285, 284 / 259, 293 / 312, 396 / 394, 450 / 428, 48 lanes
-// 323 / 356, 405 / 436, 439 / 468, 586 / 611, 878 / 891; without billboards on 320, 800 and 4000 linedefs, 16 lanes 256 / 241, 364 / 351,
-// 533 / 520, 64 lanes 437 / 429, 434 / 426, 884 / 878.
-inline bool side_stream_pays(int lanes, bool billboards) { return lanes > 102 || (billboards && lanes >= 4); }
+// A frame that goes to the side stream and back pays some 20 us for it.  Without billboards only the shading goes there: batches of up to 112
+// lanes do without.  With them it is their painting too, and which side gains is up to the cameras: where the flat pass has little to
+// do, staying saves the 20 us up to some 10 lanes, elsewhere going saves as much from 2 lanes on; 4 lies between.
+// A frame in us with the side stream / without it:
+//   billboards, lanes   120 linedefs     320           701, bricks      800            2000           4000
+//         0     96       283 / 280     376 / 374      415 / 413      358 / 354      431 / 429      550 / 547
+//         0    112       292 / 292     376 / 376      416 / 415      352 / 351      435 / 433      565 / 563
+//         0    128       296 / 297     390 / 390      440 / 441      354 / 355      446 / 446      602 / 602
+//         0    160       309 / 312     401 / 415      433 / 449      435 / 449      463 / 466      645 / 646
+//        24      1       165 /  94     186 / 166      290 / 268      159 / 138      184 / 167      280 / 256
+//        24      2       176 / 189     202 / 181      354 / 337      198 / 219      207 / 202      289 / 268
+//        24      4       216 / 239     202 / 183      364 / 343      214 / 235      232 / 229      289 / 268
+//        24      8       215 / 239     205 / 187      366 / 377      220 / 242      237 / 234      289 / 269
+//        24     16       251 / 281     225 / 223      368 / 391      283 / 306      256 / 256      373 / 384
+//        24     32       259 / 293     266 / 297      382 / 413      330 / 357      372 / 397      496 / 508
+//        96      4       215 / 258     214 / 198      365 / 351      216 / 230      237 / 239      294 / 274
+//        96     16       251 / 293     232 / 234      376 / 408      283 / 315      274 / 277      374 / 403
+inline bool side_stream_pays(int lanes, bool billboards) { return lanes > 112 || (billboards && lanes >= 4); }
 
 #endif
