@@ -75,6 +75,9 @@ inline int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
 //    2048     365 / 357 / 450 (364)           492 / 478 / 583 (487)            701 / 674 / 835 (695)            524 / 509 / 643 (536)
 //    2560     439 / 425 (440)                 596 / 589 (583)                  831 / 845 (820)                  639 / 625 (649)
 //    3072     519 / 542 (514)                 700 / 722 (683)                  930 / 969 (918)                  751 / 744 (753)
+// With one lane a column nothing is shared, and the stage takes up to 1.7 % longer than before columns could share: on one card at 4096 lanes 679 -> 684,
+// 886 -> 901, 1229 -> 1238 and 971 -> 974 us.  (A prepared pass's flags and rows kept in registers of their own there, not packed into words,
+// issue 1.5 % fewer instructions and take as long: 686, 905, 1239, 975.)
 inline int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 2400 ? 2 : 1)); }
 
 // flat_gap_kernel: wavefronts a column.  The fewer the lanes, the fewer such columns and the longer the kernel lasts as its slowest one.  us
