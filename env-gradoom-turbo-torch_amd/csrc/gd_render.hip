@@ -43,6 +43,7 @@
 #include <vector>
 
 #include "../../include/gradoom_amd.h"
+#include "gd_divide.h"
 #include "gd_internal.h"
 #include "gd_rules.h"
 
@@ -346,43 +347,7 @@ __device__ __forceinline__ unsigned mul64_bits_16_47(i64 a, i64 b) {
     const unsigned cross = __umul24(al & 0xFFFFu, bh & 0xFFFFu) + __umul24(ah & 0xFFFFu, bl & 0xFFFFu);
     return (unsigned)(low >> 16) + (cross << 16);
 }
-// C truncating division (engine.py:3115-3118).  gfx950 has no 64-bit integer divider; when both
-// magnitudes are below 2^52 the quotient comes from float64 arithmetic.  Larger operands take the compiler's long division.
-// The rare large-operand case is a compact shift-subtract loop rather than the compiler's
-// unrolled long division, which would be replicated at every call site and push the kernels
-// far past the instruction cache.
-__device__ __forceinline__ u64 udiv_long(u64 n, u64 d) {
-    u64 q = 0, r = 0;
-#pragma unroll 1
-    for (int i = 63; i >= 0; --i) {
-        r = (r << 1) | ((n >> i) & 1);
-        if (r >= d) { r -= d; q |= 1ULL << i; }
-    }
-    return q;
-}
-__device__ __forceinline__ i64 tdiv(i64 a, i64 b) {
-    u64 ua = a < 0 ? (u64)0 - (u64)a : (u64)a;
-    u64 ub = b < 0 ? (u64)0 - (u64)b : (u64)b;
-    if (((ua | ub) >> 52) != 0 || ub == 0) {
-        const u64 uq = ub == 0 ? 0 : udiv_long(ua, ub);
-        return ((a < 0) != (b < 0)) ? -(i64)uq : (i64)uq;
-    }
-    // A magnitude under the exponent of 2^52 is that power plus the magnitude, and the other way round.  The reciprocal (good to some 22
-    // bits at least) takes one Newton step, the quotient one step of its own: it is then within an eighth of its last place
-    // but one of the true quotient, so within 0.7 of it after rounding to a whole number, which is the quotient or one above.
-    // The remainder, below 2^53, is exact in a fused multiply-add, and its sign tells which.  (With an IEEE division and the
-    // library's conversions the chain of 4096 lanes on the 4000-linedef map takes 4.79 ms stage by stage, so 4.76.)
-    const double UNIT = 4503599627370496.0;    // 2^52
-    const double ad = __longlong_as_double((i64)(ua | 0x4330000000000000ULL)) - UNIT, bd = __longlong_as_double((i64)(ub | 0x4330000000000000ULL)) - UNIT;
-    double r = __builtin_amdgcn_rcp(bd);
-    r = __builtin_fma(__builtin_fma(-bd, r, 1.0), r, r);
-    double q = ad * r;
-    q = __builtin_fma(__builtin_fma(-q, bd, ad), r, q);
-    const double whole = q + UNIT;
-    const u64 uq = ((u64)__double_as_longlong(whole) & 0xFFFFFFFFFFFFFULL) - (__builtin_fma(-(whole - UNIT), bd, ad) < 0.0 ? 1u : 0u);
-    const u64 sign = (u64)((a ^ b) >> 63);
-    return (i64)((uq ^ sign) - sign);
-}
+__device__ __forceinline__ i64 tdiv(i64 a, i64 b) { return truncated_quotient(a, b, [](double d) { return __builtin_amdgcn_rcp(d); }); }
 // Lanes of one wavefront leave words in memory for one another: the hardware keeps a wavefront's loads and stores of one place in order, the compiler has to.
 __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 // Lanes of one wavefront leave words in LDS for one another: the order is the program's, the compiler has to keep it.
