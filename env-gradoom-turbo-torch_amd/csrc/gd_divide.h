@@ -27,11 +27,11 @@ __device__ __forceinline__ long long truncated_quotient(long long a, long long b
         return ((a < 0) != (b < 0)) ? -(long long)uq : (long long)uq;
     }
     // A magnitude under the exponent of 2^52 is that power plus the magnitude, and the other way round.  The reciprocal (off by 2^-24.3
-    // of its value at most over 2.1e9 divisors; 2^-22 would do) takes one Newton step, the quotient one step of its own: it is then the true quotient but for one rounding.  That is
-    // none where the divisor is one; elsewhere the quotient is below 2^51 and the rounding below an eighth.  Rounded to a whole number it
-    // is within 0.7 of the true one, so the quotient or one above.  The remainder, below 2^53, is exact in a fused multiply-add, and its sign
-    // tells which.  (With an IEEE division and the library's conversions the chain of 4096 lanes on the 4000-linedef map takes 4.79 ms
-    // stage by stage, so 4.76.)
+    // of its value at most over 2.1e9 divisors; 2^-22 would do) takes one Newton step, the quotient one step of its own: it is then the
+    // true quotient but for one rounding.  That is none where the divisor is one; elsewhere the quotient is below 2^51 and the rounding
+    // below an eighth.  Rounded to a whole number it is within 0.7 of the true one, so the quotient or one above.  The remainder, below
+    // 2^53, is exact in a fused multiply-add, and its sign tells which.  (With an IEEE division and the library's conversions the chain of
+    // 4096 lanes on the 4000-linedef map takes 4.79 ms stage by stage, so 4.76.)
     const double UNIT = 4503599627370496.0;    // 2^52
     const double ad = __builtin_bit_cast(double, ua | 0x4330000000000000ULL) - UNIT, bd = __builtin_bit_cast(double, ub | 0x4330000000000000ULL) - UNIT;
     double r = reciprocal(bd);
