@@ -59,12 +59,12 @@ typedef unsigned long long u64;
 #define VH 208
 #define CAND_MAX 64          // candidate linedefs a screen column keeps in its own slots
 // A column whose ray can reach more than CAND_MAX linedefs (a long corridor seen end on) gets a slot in the chunk's spill
-// pool, where strip_order_kernel lists all of them, up to SPILL_DEPTH.  The pool continues the candidate blocks with
-// the same layout (entry k of a column lies k * 320 entries on), SPILL_DEPTH x 320 entries per pool block, so a
+// pool, where strip_order_kernel lists all of them, up to SPILL_OBS_AHEAD.  The pool continues the candidate blocks with
+// the same layout (entry k of a column lies k * 320 entries on), SPILL_OBS_AHEAD x 320 entries per pool block, so a
 // spilled column differs from the others only in where its list starts and how long it may be.
-#define SPILL_DEPTH 256
+#define SPILL_OBS_AHEAD 256
 #define SPILL_SHIFT 12       // cand_count of a spilled column: entries | (pool slot + 1) << SPILL_SHIFT
-static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and its pool slot share a word");
+static_assert(SPILL_OBS_AHEAD < (1 << SPILL_SHIFT), "a spilled column's count and its pool slot share a word");
 #define SEG_COLS 64           // columns of a traversal segment; a wavefront takes 64 / SEG_COLS segments, of any lanes
 #define SEGS_PER_LANE (SW / SEG_COLS)
 #define GD_INF __builtin_inff()
@@ -79,7 +79,7 @@ static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and it
 #define FOCAL_Y_FIXED (160LL * Y_ASPECT_FIXED)
 #define FLOOR_VISIBILITY_FIXED ((160LL * 65536LL * (8LL * 65536LL)) / FOCAL_Y_FIXED)
 #define WALL_VISIBILITY_FIXED (((FOCAL_Y_FIXED * (320LL * 600LL) / (320LL * 240LL * 3LL)) * (8LL * 65536LL)) >> 16)
-#define SPRITE_MIN_DEPTH_FIXED 8192LL
+#define SPRITE_MIN_OBS_AHEAD_FIXED 8192LL
 
 // candidate flags
 #define CF_GEO 1
@@ -260,7 +260,7 @@ struct Scratch {    // per-chunk working memory, sized at create
     WallRec *frag_rec;     // [L,split_count,fragment_slots] FWallCoords of the BSP fragments of split linedefs
     float *scene_depth;    // [L,208,320] depth of the wall tier or masked texture a pixel shows (engine.py:11553, 12700, 13740),
                            // kept only for frames that draw wall decals, else null; scene_depth_at() has the others
-    Cand *cand;            // [L,CAND_MAX,320], then the spill pool [spill_slots / 320, SPILL_DEPTH, 320]
+    Cand *cand;            // [L,CAND_MAX,320], then the spill pool [spill_slots / 320, SPILL_OBS_AHEAD, 320]
     int *cand_count;       // [L,320] entries listed (beyond CAND_MAX: the column wanted more than its own slots hold), or for
                            // a column with a pool slot: entries in the pool | (slot + 1) << SPILL_SHIFT
     int *spill_columns;    // [spill_slots] the columns (lane * 320 + column) that were given pool slots, in slot order
@@ -1084,7 +1084,7 @@ __device__ __forceinline__ void list_spilled_columns(const DeviceMap &dm, const 
         const LaneCtx &c = sc.ctx[local];
         float rx, ry; ray_direction(c, x, &rx, &ry);
         const RecSpan *spans = sc.span + (size_t)local * walls;
-        Cand *list = sc.cand + sc.spill_base + ((size_t)(slot / SW) * SPILL_DEPTH * SW + (size_t)(slot % SW));
+        Cand *list = sc.cand + sc.spill_base + ((size_t)(slot / SW) * SPILL_OBS_AHEAD * SW + (size_t)(slot % SW));
         int listed = 0;
         for (int w0 = 0; w0 < walls; w0 += 64) {
             const int w = w0 + lane_id;
@@ -1103,12 +1103,12 @@ __device__ __forceinline__ void list_spilled_columns(const DeviceMap &dm, const 
             const u64 keeps = __ballot(keep);
             const int position = listed + __popcll(keeps & ((1ULL << lane_id) - 1ULL));
             if (keep) {
-                if (position < SPILL_DEPTH) list[(size_t)position * SW] = entry;
+                if (position < SPILL_OBS_AHEAD) list[(size_t)position * SW] = entry;
                 else sc.status[STATUS_CAND_OVERFLOW] = 1;
             }
             listed += __popcll(keeps);
         }
-        if (lane_id == 0) sc.cand_count[column] = (listed < SPILL_DEPTH ? listed : SPILL_DEPTH) | ((slot + 1) << SPILL_SHIFT);
+        if (lane_id == 0) sc.cand_count[column] = (listed < SPILL_OBS_AHEAD ? listed : SPILL_OBS_AHEAD) | ((slot + 1) << SPILL_SHIFT);
     }
 }
 
@@ -1988,7 +1988,7 @@ struct ColumnCtx {
         const unsigned spill = (unsigned)listed >> SPILL_SHIFT;
         if (spill) {
             const unsigned slot = spill - 1;
-            list_column = (sc.spill_base + (slot / SW) * (unsigned)(SPILL_DEPTH * SW) + slot % SW) * 16u;
+            list_column = (sc.spill_base + (slot / SW) * (unsigned)(SPILL_OBS_AHEAD * SW) + slot % SW) * 16u;
             count = listed & ((1 << SPILL_SHIFT) - 1);
         } else {
             list_column = ((unsigned)local * (CAND_MAX * SW) + (unsigned)column) * 16u;
@@ -2870,7 +2870,7 @@ __device__ __forceinline__ void zero_rows(Pixels &pb, GapRange &gaps, int x, int
 // rows that its own clip update then removes from the window, so the window stays untouched
 // until a one-sided drawseg (which leaves the clips alone) has painted; until then painting
 // needs no reads and visits only the rows it writes.
-template <bool DEPTH, typename Pixels>
+template <bool OBS_AHEAD, typename Pixels>
 __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnState &c, const PassDraw &d, const PassRows &r, Pixels &pb,
                            const bool group_valid[3], const float group_bottom[3], const unsigned char *colormap, bool &window_dirty, GapRange &gaps) {
     // The whole wavefront comes here together, columns with nothing to draw as well: they take part in the walks over the rows.
@@ -2992,7 +2992,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
 #pragma unroll
                     for (int j = 0; j < WALL_ROWS; ++j) {
                         const bool own = (unsigned)(y + j * stride - first) < rows;
-                        if (DEPTH) pb.put_depth(own, yb + j * stride, d.distance);
+                        if (OBS_AHEAD) pb.put_depth(own, yb + j * stride, d.distance);
                         pb.put(own, yb + j * stride, meta_word | (colour[j] << META_SECTOR_SHIFT));
                     }
 #pragma unroll
@@ -3036,7 +3036,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 for (int j = 0; j < WALL_ROWS; ++j) {
                     if (!(draw & (1u << j))) continue;
                     const unsigned colour = ((tail & (1u << j)) ? group_shades : own_shades)[texel[j]];
-                    if (DEPTH) pb.s(yb + j) = d.distance;
+                    if (OBS_AHEAD) pb.s(yb + j) = d.distance;
                     pb.m(yb + j) = META_FILLED | (colour << META_SECTOR_SHIFT) | (unsigned)(wi + 1);
                 }
 #pragma unroll
@@ -3089,7 +3089,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 const unsigned tv = (fraction >> (tier_a ? shift_a : shift_b)) >> 1;
                 unsigned char texel = m->tex_atlas[(tier_a ? d.column_a : d.column_b) + __umul24(tv, atlas_w)];
                 const unsigned colour = (bottom_tail ? group_shades : own_shades)[texel];
-                if (DEPTH) pb.s(y) = d.distance;
+                if (OBS_AHEAD) pb.s(y) = d.distance;
                 const float held = (meta & META_WALL_MASK) ? clip_distance(cc, (int)(meta & META_WALL_MASK) - 1) : GD_INF;   // no clip recorded yet
                 if (d.distance < held) { meta = (meta & ~META_WALL_MASK) | (unsigned)(wi + 1); }
                 meta = (meta & ~(META_SECTOR_MASK << META_SECTOR_SHIFT)) | (colour << META_SECTOR_SHIFT) | META_FILLED;
@@ -3287,7 +3287,7 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, const ListShar
 }
 
 // engine.py:13424-13744 for one column
-template <bool DEPTH, bool GENERAL, typename Pixels>
+template <bool OBS_AHEAD, bool GENERAL, typename Pixels>
 __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, int local, const ColumnState &c, Pixels &pb, const unsigned char *colormap) {
     const gd_map_desc *m = cc.m;
     const LaneCtx &L = *cc.c;
@@ -3382,7 +3382,7 @@ __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const Col
             if (pb.frame) pb.f(y) = colour;
             else pb.t(y) = colour;
             pb.m(y) = word[j] | META_MASKED;
-            if (DEPTH) pb.s(y) = md;
+            if (OBS_AHEAD) pb.s(y) = md;
         }
     }
 }
@@ -3786,7 +3786,7 @@ __device__ __forceinline__ PassDraw hand_round(const PassDraw &prepared, int k, 
     d.distance = __uint_as_float(take(__float_as_uint(prepared.distance)));
     return d;
 }
-// DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
+// OBS_AHEAD: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
 // BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
 // 4096 lanes on the 4000-linedef map: 1.78 -> 1.00 ms: the linedefs' lines 1.53, no sprite clip plane
@@ -3795,7 +3795,7 @@ __device__ __forceinline__ PassDraw hand_round(const PassDraw &prepared, int k, 
 // rows: 16 lanes on the 2000-linedef map 97 -> 53 us, 512 on the 4000-linedef map 443 -> 350, 1024 on the 320-linedef map 286 -> 226 (rows alone
 // 71, 426, 252).  The passes are handed round from register to register: through LDS there are no spills, but the 1024 lanes take 268.  Working
 // out the textures of visible tiers only makes the 1024 lanes 241, and 4096 1.11 ms.
-template <bool DEPTH, bool GENERAL, int PARTS>
+template <bool OBS_AHEAD, bool GENERAL, int PARTS>
 __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(RASTER_WAVES, RASTER_WAVES))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
     __shared__ LaneCtx lane_ctxs[WALL_STRIPS_PER_GROUP][64 / SEG_COLS];
@@ -3834,10 +3834,10 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     PixelBuffers<PARTS> pb;
     pb.frame = frame_base;
     pb.meta = sc.meta; pb.masked_texel = sc.masked_texel;
-    pb.scene_depth = DEPTH ? sc.scene_depth : nullptr;
+    pb.scene_depth = OBS_AHEAD ? sc.scene_depth : nullptr;
     pb.word_column = ((unsigned)local * (VH * SW) + (unsigned)x) * 4u;
     pb.words = __builtin_amdgcn_make_buffer_rsrc(sc.meta, 0, lane_count * (VH * SW * 4), BUFFER_WORDS);
-    pb.depths = __builtin_amdgcn_make_buffer_rsrc(pb.scene_depth, 0, DEPTH ? lane_count * (VH * SW * 4) : 0, BUFFER_WORDS);
+    pb.depths = __builtin_amdgcn_make_buffer_rsrc(pb.scene_depth, 0, OBS_AHEAD ? lane_count * (VH * SW * 4) : 0, BUFFER_WORDS);
     pb.frame_column = (unsigned)local * (unsigned)frame_stride + (unsigned)x;
     pb.row_lane = PARTS == 1 ? 0 : lane_id / part_cols;
     pb.put_column = pb.word_column + (unsigned)pb.row_lane * (SW * 4u);
@@ -3903,13 +3903,13 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
             group_valid[0] = same_group && (agreed & 1) && (shared_top < shared_bottom);
             group_valid[1] = same_group && (agreed & 2) && (shared_lower_top < shared_bottom);
             group_valid[2] = same_group && (agreed & 4) && (shared_top < shared_upper_bottom);
-            pass_paint<DEPTH>(cc, st, d, rows, pb, group_valid, common_bottom, colormap_lds, window_dirty, gaps);
+            pass_paint<OBS_AHEAD>(cc, st, d, rows, pb, group_valid, common_bottom, colormap_lds, window_dirty, gaps);
             if (d.flags & (DRAW_RASTER | DRAW_PS_KEEPS)) advance_clips(cc, st, d, rows, pb, sb, !window_dirty, gaps, sc, first_record + (size_t)(group + k) * pass_stride);
         }
     }
     // what is left of a window no one-sided drawseg closed shows the flat pass's picture
     if (!window_dirty) zero_rows(pb, gaps, x, st.ceiling_clip <= 0.0f ? 0 : (int)st.ceiling_clip, st.floor_clip >= (float)VH ? VH : (int)st.floor_clip);
-    if (dm.masked_count > 0) masked_midtexture<DEPTH, GENERAL>(dm, cc, sc, local, st, pb, colormap_lds);
+    if (dm.masked_count > 0) masked_midtexture<OBS_AHEAD, GENERAL>(dm, cc, sc, local, st, pb, colormap_lds);
     // The columns with view pixels that no wall tier, plane or masked texture covers join the flat pass's work list, those of a
     // wavefront in one piece (flat_gap_kernel selects the pixels, flat_shade_kernel paints them).
     bool holds_gap = false;
@@ -4098,7 +4098,7 @@ __device__ __forceinline__ bool sprite_record(const DeviceMap &dm, const gd_lane
     const i64 rx = ax - L.view_x_fixed, ry = ay - L.view_y_fixed;
     s.depth_fixed = (rx * L.vcos + ry * L.vsin) >> 20;
     const i64 side_fixed = (rx * L.vsin - ry * L.vcos) >> 16;
-    const i64 xscale = tdiv(FOCAL_X_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
+    const i64 xscale = tdiv(FOCAL_X_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_OBS_AHEAD_FIXED));
     const i64 left_fixed = side_fixed - (i64)m->spr_left[id] * FIXED_UNIT;
     s.width = m->spr_w[id];
     s.left = SW / 2 + (mul64(left_fixed, xscale) >> 32);
@@ -4107,7 +4107,7 @@ __device__ __forceinline__ bool sprite_record(const DeviceMap &dm, const gd_lane
     if (!(s.right > x_first && s.left < x_end && s.right > s.left)) return false;
     s.height = m->spr_h[id];
     s.hstep = tdiv((i64)s.width << 16, max64(s.right - s.left, 1));
-    s.yscale = tdiv(FOCAL_Y_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
+    s.yscale = tdiv(FOCAL_Y_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_OBS_AHEAD_FIXED));
     const i64 texmid = (i64)m->spr_top[id] * FIXED_UNIT - round_to_i64((L.view_z - z) * 65536.0f);
     s.top_fixed = L.center_fixed - (mul64(texmid, s.yscale) >> 16);
     s.iscale = tdiv(UINT32_MASK, max64(s.yscale, 1));
@@ -4843,131 +4843,211 @@ __device__ __forceinline__ void store_stack_word(unsigned char *stack_lane, unsi
     }
 }
 
-// One block per lane and OBS_BLOCK_ROWS = 7 observation rows, which pool exactly OBS_SOURCE_ROWS = 20 frame rows
-// (84 observation rows x 240 / 84 frame rows each).  An observation pixel covers 240/84 frame rows and 320/84 frame
-// columns; its weights (y_overlap * x_overlap) // 48 are exactly (y_overlap / 12) * (x_overlap / 4), since row
-// overlaps are multiples of 12 and column overlaps multiples of 4 (84 = 12 * 7 = 4 * 21, 240 = 12 * 20, 320 = 4 * 80):
-// the weighted sum factors into a pass along the rows and one down the columns, all in integers.  The first pass
-// looks every frame pixel's colour up once per observation column it touches (five taps per frame row and
-// observation column), the second adds four row sums per observation pixel: 10,752 palette taps per block where a
-// pixel-by-pixel pooling takes 11,760.  Bound by the vector instructions these take (95 % of the issue slots), so a tap is
-// short: a thread's five bytes come in two words, and a 24-bit product carries red and green together, a dot product blue.
-// Frames on 16 bytes are staged by 16-byte loads.  4096 frames: 0.202 ms with a byte load and three dot products a tap, 0.153 ms now.
-#define OBS_BLOCK_ROWS 7
+// The pooling of a frame as two products of small whole numbers, which the matrix cores take (v_mfma_i32_16x16x64_i8).  An observation pixel
+// covers 240/84 frame rows and 320/84 frame columns; its weights (y_overlap * x_overlap) // 48 are exactly (y_overlap / 12) * (x_overlap / 4),
+// since row overlaps are multiples of 12 and column overlaps multiples of 4 (84 = 12 * 7 = 4 * 21, 240 = 12 * 20, 320 = 4 * 80): the
+// weighted sum is (down weights) x (colours) x (along weights), both weights banded and below 22.
+//   along: a wavefront takes 14 observation columns, whose frame columns lie in a window of 64 that starts on 16 bytes: one product for 16
+//     frame rows and a channel.  A lane loads sixteen neighbouring pixels of a row, which is the product's layout.
+//   down: 14 observation rows pool exactly 40 frame rows, which lie in three of the tiles of 16 rows of a block of 80.  The sums of the first
+//     product stay in the lane that they come out in: the order of a product's inner index is free, and the down weights are laid out
+//     in the order that the first product leaves (row 16 t + 4 g + r in byte 4 t + r of the lanes of group g).
+// Colours are taken less 128, so that they and the sums' two bytes (256 * high + low, low from -128 to 127) are signed bytes.
+// What is left for the vector units is to fetch a pixel's colour and to put the channels in words of their own, some five instructions
+// a pixel where sums by multiply-add took 21.  The fetches are from 32 copies of the palette, a bank of LDS each: no two lanes of a half
+// wavefront ever meet in a bank.  4096 frames of 240 rows: 0.153 ms by multiply-add, 0.105 ms now (the copy of as many bytes takes 0.066).  Tried:
+// colour words as the product's bytes as they are (a quarter of the products, 84 a block instead of 27: 0.145); copies 256 bytes apart, so
+// that one byte move makes an address (64 KB a work-group leave one a compute unit: 0.136); all of a block's pixels asked for at once (0.118).
+#define OBS_TILE 14             // observation columns of a wavefront, observation rows of a product down the columns
+#define OBS_WAVES (GD_OBS_SIZE / OBS_TILE)
+#define OBS_THREADS (64 * OBS_WAVES)
+#define OBS_BLOCK_ROWS (2 * OBS_TILE)
 #define OBS_SOURCE_ROWS (OBS_BLOCK_ROWS * GD_SCREEN_HEIGHT / GD_OBS_SIZE)
-static_assert(GD_OBS_SIZE % OBS_BLOCK_ROWS == 0 && OBS_SOURCE_ROWS * GD_OBS_SIZE == OBS_BLOCK_ROWS * GD_SCREEN_HEIGHT, "observe_kernel: seven rows pool twenty");
-static_assert((OBS_BLOCK_ROWS * GD_OBS_SIZE) % 4 == 0 && 3 * GD_OBS_SIZE <= 256, "observe_kernel: whole words, three rows of threads");
-__global__ void __launch_bounds__(256) observe_kernel(const unsigned char *indexed, size_t lane_stride, int source_rows, const unsigned char *playpal,
+#define OBS_BLOCKS (GD_OBS_SIZE / OBS_BLOCK_ROWS)      // a frame's blocks of rows
+#define OBS_ROW_TILES (OBS_SOURCE_ROWS / 16)
+#define OBS_COPIES 32
+#define OBS_AHEAD 2             // tiles whose pixels are asked for ahead
+static_assert(OBS_WAVES * OBS_TILE == GD_OBS_SIZE && OBS_BLOCKS * OBS_BLOCK_ROWS == GD_OBS_SIZE, "observe_kernel: whole tiles");
+static_assert(OBS_SOURCE_ROWS * GD_OBS_SIZE == OBS_BLOCK_ROWS * GD_SCREEN_HEIGHT && OBS_ROW_TILES * 16 == OBS_SOURCE_ROWS && VH % 16 == 0, "observe_kernel: whole rows");
+typedef int int4v __attribute__((ext_vector_type(4)));
+
+struct PoolWeights { unsigned char along[OBS_WAVES][64][16], down[2][64][16]; };   // as the products take them: [tile][lane][byte]
+constexpr int obs_window(int tile) {   // the first frame column of a tile's window
+    const int first = tile * OBS_TILE * 320 / GD_OBS_SIZE / 16 * 16;
+    return first > SW - 64 ? SW - 64 : first;
+}
+constexpr int overlap(int a0, int a1, int b0, int b1) {
+    const int low = a0 > b0 ? a0 : b0, high = a1 < b1 ? a1 : b1;
+    return high > low ? high - low : 0;
+}
+constexpr PoolWeights pool_weights() {
+    PoolWeights w{};
+    for (int lane = 0; lane < 64; ++lane) {
+        const int column = lane & 15, group = lane >> 4;
+        for (int k = 0; k < 16 && column < OBS_TILE; ++k) {
+            for (int tile = 0; tile < OBS_WAVES; ++tile) {
+                const int ox = tile * OBS_TILE + column, x = obs_window(tile) + 16 * group + k;
+                w.along[tile][lane][k] = (unsigned char)(overlap(ox * 320, ox * 320 + 320, x * 84, x * 84 + 84) / 4);
+            }
+            for (int half = 0; half < 2 && k < 12; ++half) {
+                const int oy = half * OBS_TILE + column, y = 16 * (2 * half + (k >> 2)) + 4 * group + (k & 3);
+                w.down[half][lane][k] = (unsigned char)(overlap(oy * 240, oy * 240 + 240, y * 84, y * 84 + 84) / 12);
+            }
+        }
+    }
+    return w;
+}
+constexpr bool pool_weights_whole() {   // every observation pixel has all its weight: 80 along a row, 20 down a column
+    const PoolWeights w = pool_weights();
+    for (int column = 0; column < OBS_TILE; ++column) {
+        for (int tile = 0; tile < OBS_WAVES; ++tile) {
+            int sum = 0;
+            for (int k = 0; k < 64; ++k) sum += w.along[tile][column + 16 * (k >> 4)][k & 15];
+            if (sum != 80) return false;
+        }
+        for (int half = 0; half < 2; ++half) {
+            int sum = 0;
+            for (int k = 0; k < 64; ++k) sum += w.down[half][column + 16 * (k >> 4)][k & 15];
+            if (sum != 20) return false;
+        }
+    }
+    return true;
+}
+static_assert(pool_weights_whole(), "observe_kernel: a tile's window holds its columns, a block's tiles its rows");
+__device__ const __align__(16) PoolWeights POOL_WEIGHTS = pool_weights();
+
+// A work-group takes a run of the frames' blocks of rows, a wavefront OBS_TILE observation columns of each.  The next block's pixels are asked
+// for as soon as a tile's own are used up.
+// ALIGNED: the frames start on 16 bytes.
+template <bool ALIGNED>
+__global__ void __launch_bounds__(OBS_THREADS, 6) observe_kernel(const unsigned char *indexed, size_t lane_stride, int source_rows, const unsigned char *playpal,
                                int lane_count, unsigned char *obs, unsigned char *frames, const unsigned char *reset_mask, int stack_mode,
                                unsigned char *final_frames, bool final_hwc, const float *blend) {
-    __shared__ unsigned int pal[256];   // PLAYPAL after the lane's screen blend, one word per colour (red | green << 16 | blue << 24)
-    __shared__ __align__(16) unsigned int tile[OBS_SOURCE_ROWS * (SW / 4) + 4];   // the last column reads a word past its row, with weight 0
-    __shared__ unsigned int along_rg[OBS_SOURCE_ROWS * GD_OBS_SIZE];      // per frame row and observation column: red | green << 16 summed along the row
-    __shared__ unsigned short along_b[OBS_SOURCE_ROWS * GD_OBS_SIZE];     // and blue (each at most 80 * 255)
-    __shared__ unsigned int gray_words[OBS_BLOCK_ROWS * GD_OBS_SIZE / 4];
-    int n = blockIdx.y;
-    if (n >= lane_count) return;                   // the same in the whole block
-    const unsigned char *src = indexed + (size_t)n * lane_stride;
-    const int first_row = blockIdx.x * OBS_BLOCK_ROWS;
-    const int tile_first = blockIdx.x * OBS_SOURCE_ROWS;
-    // Everything the block reads from memory is asked for up front (palette entry, tile words, the stack words
-    // that the roll keeps), so that the block waits for memory once.
+    __shared__ unsigned int pal[256];   // PLAYPAL after the lane's screen blend, one word per colour (red | green << 8 | blue << 16, each less 128)
+    __shared__ __align__(16) unsigned int copies[256 * OBS_COPIES];
+    __shared__ unsigned int gray_words[2][OBS_BLOCK_ROWS * GD_OBS_SIZE / 4];
+    const int tasks = lane_count * OBS_BLOCKS;
+    const int first_task = (int)((long long)tasks * blockIdx.x / gridDim.x), end_task = (int)((long long)tasks * (blockIdx.x + 1) / gridDim.x);
+    const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63, group = lane_id >> 4, column = lane_id & 15;
     const size_t F = (size_t)GD_OBS_SIZE * GD_OBS_SIZE / 4;     // words per observation
-    const size_t word = (size_t)first_row * GD_OBS_SIZE / 4 + threadIdx.x;
-    const bool rolls = threadIdx.x < OBS_BLOCK_ROWS * GD_OBS_SIZE / 4;
     const bool stack_aligned = ((reinterpret_cast<size_t>(frames) | reinterpret_cast<size_t>(final_frames)) & 3) == 0;
-    unsigned char *stack_bytes = frames ? frames + ((size_t)n * GD_FRAME_STACK * F + word) * 4 : nullptr;
     auto load_word = [](const unsigned char *p, bool aligned) -> unsigned int {
         if (aligned) return *reinterpret_cast<const unsigned int *>(p);
         return (unsigned)p[0] | ((unsigned)p[1] << 8) | ((unsigned)p[2] << 16) | ((unsigned)p[3] << 24);
     };
-    const bool resets = reset_mask && reset_mask[n];
-    unsigned int kept[GD_FRAME_STACK];
-    for (int k = 0; k < GD_FRAME_STACK; ++k) kept[k] = (rolls && frames && !resets) ? load_word(stack_bytes + k * F * 4, stack_aligned) : 0u;
-    {
-        const int k = threadIdx.x;   // 256 threads, 256 colours
-        unsigned int r = playpal[3 * k], g = playpal[3 * k + 1], b = playpal[3 * k + 2];
-        if (blend) {
-            const float bonus = blend[2 * n], flash = blend[2 * n + 1];
-            r = blended_channel((unsigned char)r, 0, bonus, flash); g = blended_channel((unsigned char)g, 1, bonus, flash); b = blended_channel((unsigned char)b, 2, bonus, flash);
-        }
-        pal[k] = r | (g << 16) | (b << 24);
-    }
-    {
-        // the block's frame rows are one piece; rows past the source are neither loaded nor read
-        const unsigned char *piece = src + (size_t)tile_first * SW;
-        const int rows = min(source_rows - tile_first, OBS_SOURCE_ROWS);
-        if ((reinterpret_cast<size_t>(src) & 15) == 0) {
-            for (int k = threadIdx.x; k < rows * (SW / 16); k += blockDim.x) reinterpret_cast<uint4 *>(tile)[k] = reinterpret_cast<const uint4 *>(piece)[k];
-        } else {
-            const bool aligned = (reinterpret_cast<size_t>(src) & 3) == 0;
-            for (int k = threadIdx.x; k < rows * (SW / 4); k += blockDim.x) tile[k] = load_word(piece + 4 * (size_t)k, aligned);
-        }
-    }
-    __syncthreads();
-    // three rows of 84 threads: thread (slot, ox) takes observation column ox of every third row
-    const int slot = min((int)threadIdx.x / GD_OBS_SIZE, 2), ox = min((int)threadIdx.x - slot * GD_OBS_SIZE, GD_OBS_SIZE - 1);
-    const bool works = threadIdx.x < 3 * GD_OBS_SIZE;
-    {
-        // along the rows: up to five frame columns overlap an observation column, by multiples of 4 out of 84
-        const int x_start = ox * 320, x_end = x_start + 320, first_x = x_start / 84;
-        unsigned int weight[5], weight_b[5];
+    const unsigned int at = (unsigned)(obs_window(wave) + 16 * group + column * SW);      // lane strides are multiples of 16, like the window's start
+    auto load_tile = [&](int task, int t) -> uint4 {      // a lane's sixteen pixels of a tile; past the source, or the run, those of some row before
+        task = min(task, end_task - 1);
+        const int n = task / OBS_BLOCKS, row = min((task - n * OBS_BLOCKS) * OBS_SOURCE_ROWS + 16 * t, source_rows - 16);
+        const unsigned char *first = indexed + (size_t)n * lane_stride + (size_t)row * SW;
+        if (ALIGNED) return *reinterpret_cast<const uint4 *>(first + at);
+        const bool aligned = (reinterpret_cast<size_t>(indexed) & 3) == 0;
+        return make_uint4(load_word(first + at, aligned), load_word(first + at + 4, aligned), load_word(first + at + 8, aligned), load_word(first + at + 12, aligned));
+    };
+    uint4 pixels[OBS_ROW_TILES];
 #pragma unroll
-        for (int sx = 0; sx < 5; ++sx) {
-            const int source_x = first_x + sx;
-            const int over = min(x_end, (source_x + 1) * 84) - max(x_start, source_x * 84);
-            weight[sx] = (source_x >= SW || over <= 0) ? 0u : (unsigned)over >> 2;
-            weight_b[sx] = weight[sx] << 24;   // a four-byte dot product with a colour word is blue times the weight
-        }
-        const int first_word = first_x / 4, shift = 8 * (first_x & 3);   // five columns from any byte of a word lie in two words
-        for (int sy = slot; sy < OBS_SOURCE_ROWS && works; sy += 3) {
-            unsigned int rg = 0, bs = 0;
-            if (tile_first + sy < source_rows) {
-                const unsigned int *at = tile + sy * (SW / 4) + first_word;
-                const unsigned int low = at[0], high = at[1];
-                const unsigned int four = __builtin_amdgcn_alignbit(high, low, shift), fifth = (high >> shift) & 255u;
-                const unsigned int colour[5] = {pal[four & 255u], pal[(four >> 8) & 255u], pal[(four >> 16) & 255u], pal[four >> 24], pal[fifth]};
-#pragma unroll
-                for (int sx = 0; sx < 5; ++sx) {
-                    rg += __umul24(colour[sx], weight[sx]);   // the low 24 bits: red and green in one product, at most 80 * 255 each
-                    bs = __builtin_amdgcn_udot4(colour[sx], weight_b[sx], bs, false);
+    for (int t = 0; t < OBS_AHEAD; ++t) pixels[t] = load_tile(first_task, t);
+    const int4v along = *reinterpret_cast<const int4v *>(POOL_WEIGHTS.along[wave][lane_id]);
+    const int4v down[2] = {*reinterpret_cast<const int4v *>(POOL_WEIGHTS.down[0][lane_id]), *reinterpret_cast<const int4v *>(POOL_WEIGHTS.down[1][lane_id])};
+    const unsigned int bank = lane_id & (OBS_COPIES - 1);
+    auto colour_of = [&](unsigned int word, int k) { return copies[((word >> (8 * k)) & 255u) * OBS_COPIES + bank]; };
+    for (int task = first_task; task < end_task; ++task) {
+        const int n = task / OBS_BLOCKS, block = task - n * OBS_BLOCKS;
+        if (task == first_task || (blend && block == 0)) {      // nobody reads the last lane's copies any more: its last block has been put together
+            if (threadIdx.x < 256) {
+                const int k = threadIdx.x;
+                unsigned int r = playpal[3 * k], g = playpal[3 * k + 1], b = playpal[3 * k + 2];
+                if (blend) {
+                    const float bonus = blend[2 * n], flash = blend[2 * n + 1];
+                    r = blended_channel((unsigned char)r, 0, bonus, flash); g = blended_channel((unsigned char)g, 1, bonus, flash); b = blended_channel((unsigned char)b, 2, bonus, flash);
                 }
+                pal[k] = (r | (g << 8) | (b << 16)) ^ 0x808080u;
             }
-            along_rg[sy * GD_OBS_SIZE + ox] = rg;
-            along_b[sy * GD_OBS_SIZE + ox] = (unsigned short)bs;
+            __syncthreads();
+            for (int k = threadIdx.x; k < 256 * OBS_COPIES / 4; k += OBS_THREADS) {
+                const unsigned int colour = pal[k / (OBS_COPIES / 4)];
+                reinterpret_cast<uint4 *>(copies)[k] = make_uint4(colour, colour, colour, colour);
+            }
+            __syncthreads();
         }
-    }
-    __syncthreads();
-    // down the columns: up to four frame rows overlap an observation row, by multiples of 12 out of 84
-    for (int row_in_block = slot; row_in_block < OBS_BLOCK_ROWS && works; row_in_block += 3) {
-        const int y_start = row_in_block * 240, y_end = y_start + 240, first_y = y_start / 84;   // relative to the block's first frame row
-        unsigned int rs = 0, gs = 0, bs = 0;
+        const bool resets = reset_mask && reset_mask[n];
+        int low[OBS_ROW_TILES][3], high[OBS_ROW_TILES][3];      // the sums along the rows, a byte each of four rows a word
+        const int4v start = {20 * 80 * 128 + 800, 20 * 80 * 128 + 800, 20 * 80 * 128 + 800, 20 * 80 * 128 + 800};      // the colours' 128, and half of 1600
+        auto down_columns = [&](int half) __attribute__((always_inline)) {
+            int4v total[3];
 #pragma unroll
-        for (int sy = 0; sy < 4; ++sy) {
-            const int source_y = first_y + sy;
-            const int over = min(y_end, (source_y + 1) * 84) - max(y_start, source_y * 84);
-            const unsigned int weight = (source_y >= OBS_SOURCE_ROWS || over <= 0) ? 0u : (unsigned)over / 12u;
-            const int at = min(source_y, OBS_SOURCE_ROWS - 1) * GD_OBS_SIZE + ox;
-            const unsigned int rg = along_rg[at];
-            rs += __umul24(rg & 0xFFFFu, weight); gs += __umul24(rg >> 16, weight); bs += __umul24(along_b[at], weight);
+            for (int c = 0; c < 3; ++c) {
+                const int4v upper = __builtin_amdgcn_mfma_i32_16x16x64_i8(down[half], int4v{high[2 * half][c], high[2 * half + 1][c], high[2 * half + 2][c], 0}, int4v{0, 0, 0, 0}, 0, 0, 0);
+                total[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(down[half], int4v{low[2 * half][c], low[2 * half + 1][c], low[2 * half + 2][c], 0}, start, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) total[c][r] = (upper[r] << 8) + total[c][r];
+            }
+            unsigned char *out = reinterpret_cast<unsigned char *>(gray_words[task & 1]) + (half * OBS_TILE + 4 * group) * GD_OBS_SIZE + wave * OBS_TILE + column;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                // v / 1600 for v <= 1600 * 255 + 800: 2684355 is 2^32 / 1600 and 0.44 more, which takes v / 1600 up by less than 1 / 1600
+                const unsigned int red = __umulhi((unsigned)total[0][r], 2684355u), green = __umulhi((unsigned)total[1][r], 2684355u), blue = __umulhi((unsigned)total[2][r], 2684355u);
+                const unsigned int gray = __umul24(red, 77u << 8) + __umul24(green, 150u << 8) + __umul24(blue, 29u << 8) + (128u << 8);
+                if (4 * group + r < OBS_TILE && column < OBS_TILE) out[r * GD_OBS_SIZE] = (unsigned char)(gray >> 16);
+            }
+        };
+#pragma unroll
+        for (int t = 0; t < OBS_ROW_TILES; ++t) {
+            pixels[(t + OBS_AHEAD) % OBS_ROW_TILES] = load_tile(task + (t + OBS_AHEAD) / OBS_ROW_TILES, (t + OBS_AHEAD) % OBS_ROW_TILES);
+            const unsigned int word[4] = {pixels[t].x, pixels[t].y, pixels[t].z, pixels[t].w};
+            int4v channel[3];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const unsigned int c0 = colour_of(word[j], 0), c1 = colour_of(word[j], 1), c2 = colour_of(word[j], 2), c3 = colour_of(word[j], 3);
+                const unsigned int front = __builtin_amdgcn_perm(c1, c0, 0x05010400u), back = __builtin_amdgcn_perm(c3, c2, 0x05010400u);   // two reds, two greens
+                channel[0][j] = (int)__builtin_amdgcn_perm(back, front, 0x05040100u);
+                channel[1][j] = (int)__builtin_amdgcn_perm(back, front, 0x07060302u);
+                channel[2][j] = (int)__builtin_amdgcn_perm(__builtin_amdgcn_perm(c3, c2, 0x06020602u), __builtin_amdgcn_perm(c1, c0, 0x06020602u), 0x05040100u);
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int4v sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(channel[c], along, int4v{128, 128, 128, 128}, 0, 0, 0);   // 128 more: the byte above rounds
+                const unsigned int front = __builtin_amdgcn_perm((unsigned)sums[1], (unsigned)sums[0], 0x05010400u), back = __builtin_amdgcn_perm((unsigned)sums[3], (unsigned)sums[2], 0x05010400u);
+                low[t][c] = (int)(__builtin_amdgcn_perm(back, front, 0x05040100u) ^ 0x80808080u);
+                high[t][c] = (int)__builtin_amdgcn_perm(back, front, 0x07060302u);
+                if (16 * t >= VH % OBS_SOURCE_ROWS && block * OBS_SOURCE_ROWS + 16 * t >= source_rows) { low[t][c] = 0; high[t][c] = (int)0xD8D8D8D8u; }   // black: 80 * -128 = 256 * -40
+            }
+            if (t == 2) down_columns(0);
+            if (t == 4) down_columns(1);
         }
-        // (v + 800) / 1600 for v <= 1600 * 255: 64 divides by a shift, and y / 25 is y * 5243 >> 17 while 3 y < 2^17 (25 * 5243 = 2^17 + 3)
-        const unsigned int r = __umul24((rs + 800u) >> 6, 5243u) >> 17, g = __umul24((gs + 800u) >> 6, 5243u) >> 17, b = __umul24((bs + 800u) >> 6, 5243u) >> 17;
-        reinterpret_cast<unsigned char *>(gray_words)[row_in_block * GD_OBS_SIZE + ox] = (unsigned char)((r * 77u + g * 150u + b * 29u + 128u) >> 8);
+        // the stack words that the roll keeps
+        constexpr int WORDS = OBS_BLOCK_ROWS * GD_OBS_SIZE / 4, ROUNDS = (WORDS + OBS_THREADS - 1) / OBS_THREADS;
+        const size_t first_word = (size_t)block * WORDS;
+        unsigned int kept[ROUNDS][GD_FRAME_STACK];
+#pragma unroll
+        for (int j = 0; j < ROUNDS; ++j) {
+            const int k = threadIdx.x + j * OBS_THREADS;
+#pragma unroll
+            for (int f = 0; f < GD_FRAME_STACK; ++f)
+                kept[j][f] = k < WORDS && frames && !resets ? load_word(frames + ((size_t)n * GD_FRAME_STACK * F + f * F + first_word + k) * 4, stack_aligned) : 0u;
+        }
+        __syncthreads();
+        // the block's pixels are contiguous in the observation; they go out, and the stack is rolled, a word (four pixels) per thread
+#pragma unroll
+        for (int j = 0; j < ROUNDS; ++j) {
+            const int k = threadIdx.x + j * OBS_THREADS;
+            if (k >= WORDS) break;
+            const unsigned int grays = gray_words[task & 1][k];
+            const size_t word = first_word + k;
+            if (obs) {
+                unsigned char *out = obs + ((size_t)n * F + word) * 4;
+                if ((reinterpret_cast<size_t>(obs) & 3) == 0) *reinterpret_cast<unsigned int *>(out) = grays;
+                else for (int b = 0; b < 4; ++b) out[b] = (unsigned char)(grays >> (8 * b));
+            }
+            // a stack is [4][84][84] bytes, so word access only needs the tensors themselves word aligned
+            if (frames) store_stack_word(frames + (size_t)n * GD_FRAME_STACK * F * 4, final_frames ? final_frames + (size_t)n * GD_FRAME_STACK * F * 4 : nullptr,
+                                         final_hwc, stack_aligned, word, kept[j], grays, resets, stack_mode);
+        }
     }
-    __syncthreads();
-    // The block's pixels are contiguous in the observation; they go out, and the stack is rolled, a word (four
-    // pixels) per thread.
-    if (!rolls) return;
-    const unsigned int grays = gray_words[threadIdx.x];
-    if (obs) {
-        unsigned char *out = obs + ((size_t)n * F + word) * 4;
-        if ((reinterpret_cast<size_t>(obs) & 3) == 0) *reinterpret_cast<unsigned int *>(out) = grays;
-        else for (int k = 0; k < 4; ++k) out[k] = (unsigned char)(grays >> (8 * k));
-    }
-    // a stack is [4][84][84] bytes, so word access only needs the tensors themselves word aligned
-    if (frames) store_stack_word(frames + (size_t)n * GD_FRAME_STACK * F * 4, final_frames ? final_frames + (size_t)n * GD_FRAME_STACK * F * 4 : nullptr,
-                                 final_hwc, stack_aligned, word, kept, grays, resets, stack_mode);
+}
+
+decltype(&observe_kernel<true>) observe_kernel_for(const unsigned char *indexed) {
+    return (reinterpret_cast<size_t>(indexed) & 15) == 0 ? observe_kernel<true> : observe_kernel<false>;
 }
 
 // engine.py:15381-15384: PLAYPAL expansion.  A thread takes sixteen pixels: one 16-byte load, sixteen palette words from LDS; the 48 bytes
@@ -5630,7 +5710,7 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.masked_geo, L * (size_t)masked_count);
     take(&sc.masked_hit, L * SW);
     take(&sc.frag_rec, L * (size_t)(h.split_count > 0 ? h.split_count * h.fragment_slots : 1));
-    take(&sc.cand, L * CAND_MAX * SW + spill_blocks * SPILL_DEPTH * SW);   // byte offsets into it are 32 bits wide: L <= 4096, spill_blocks <= 512
+    take(&sc.cand, L * CAND_MAX * SW + spill_blocks * SPILL_OBS_AHEAD * SW);   // byte offsets into it are 32 bits wide: L <= 4096, spill_blocks <= 512
     sc.spill_base = (unsigned)(L * CAND_MAX * SW); sc.spill_slots = (int)(spill_blocks * SW);
     take(&sc.cand_count, L * SW);
     take(&sc.spill_columns, spill_blocks * SW);
@@ -5982,7 +6062,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         hipLaunchKernelGGL(hud_kernel, dim3(count), dim3(256), 0, stream, r->overlays, lanes->hud_state, base, count, frame_base, frame_stride);
     mark();
     if (out->obs || out->frames) {
-        hipLaunchKernelGGL(observe_kernel, dim3(GD_OBS_SIZE / OBS_BLOCK_ROWS, count), dim3(256), 0, stream,
+        hipLaunchKernelGGL(observe_kernel_for(frame_base), dim3(observe_groups(count * OBS_BLOCKS)), dim3(OBS_THREADS), 0, stream,
                            frame_base, frame_stride, source_rows, m.playpal, count, out->obs ? out->obs + (size_t)base * F : nullptr,
                            out->frames ? out->frames + (size_t)base * GD_FRAME_STACK * F : nullptr,
                            out->reset_mask ? out->reset_mask + base : nullptr, out->stack_mode,
@@ -6436,7 +6516,7 @@ int gd_observe(const uint8_t *indexed, int32_t source_rows, const uint8_t *playp
     for (int base = 0; base < lane_count; base += 32768) {
         int count = lane_count - base < 32768 ? lane_count - base : 32768;
         const size_t F = (size_t)GD_OBS_SIZE * GD_OBS_SIZE;
-        hipLaunchKernelGGL(observe_kernel, dim3(GD_OBS_SIZE / OBS_BLOCK_ROWS, count), dim3(256), 0, static_cast<hipStream_t>(stream),
+        hipLaunchKernelGGL(observe_kernel_for(indexed), dim3(observe_groups(count * OBS_BLOCKS)), dim3(OBS_THREADS), 0, static_cast<hipStream_t>(stream),
                            indexed + (size_t)base * source_rows * SW, (size_t)source_rows * SW, source_rows, playpal, count,
                            obs ? obs + (size_t)base * F : nullptr, frames ? frames + (size_t)base * GD_FRAME_STACK * F : nullptr,
                            reset_mask ? reset_mask + base : nullptr, stack_mode, nullptr, false, nullptr);
