@@ -376,6 +376,16 @@ class ActorDesc(_Sized):
     )
 
 
+class FacingDesc(_Sized):
+    """``gd_facing_desc``: what ``gd_pack_actors_facing`` works the sprite rotations out of."""
+
+    _fields_ = (
+        [("struct_size", C.c_uint32), ("doll_stride", C.c_int32), ("item_stride", C.c_int32)]
+        + [(name, _P) for name in ("x", "y", "enemy_angle", "doll_degrees", "projectile_velocity_x", "projectile_velocity_y",
+                                   "enemy_projectile_velocity_x", "enemy_projectile_velocity_y")]
+    )
+
+
 WEAPON_INPUTS = (
     "active_weapon", "weapon_state_cooldown", "weapon_fire_count", "weapon_ready_tics", "weapon_lower_cooldown",
     "weapon_raise_cooldown", "pending_weapon", "episode_time", "player_bob_fixed", "player_dead",

@@ -29,7 +29,9 @@ SYMBOLS = (
     "gd_observe",
     "gd_expand_rgb24",
     "gd_pack_actors",
+    "gd_pack_actors_facing",
     "gd_pack_weapon",
+    "gd_pack_weapon_narrow",
     "gd_pack_decals",
     "gd_screen_blend",
     "gd_ray_tables",
@@ -108,6 +110,8 @@ def library() -> C.CDLL:
     lib.gd_sprite_depth.restype = C.c_int
     lib.gd_sprite_depth.argtypes = [C.c_void_p] * 5 + [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p]
     for name, arguments in (
+        ("gd_pack_actors_facing", [C.POINTER(_abi.ActorDesc), C.POINTER(_abi.FacingDesc), C.c_void_p]),
+        ("gd_pack_weapon_narrow", [C.POINTER(_abi.WeaponDesc), C.c_uint32, C.c_void_p]),
         ("gd_pose_lanes", [C.POINTER(_abi.PoseDesc), C.c_void_p]),
         ("gd_pose_step", [C.c_void_p] * 3 + [C.c_int32, C.c_int64, C.c_int64] + [C.c_void_p] * 4),
         ("gd_pose_reset", [C.c_void_p] * 4 + [C.c_int32, C.c_int64, C.c_void_p]),

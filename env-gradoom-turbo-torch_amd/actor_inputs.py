@@ -8,8 +8,9 @@ teleport fog, bullet puffs, map items, drops), each trimmed to the slots some la
 slot draws nothing and ties between equally distant sprites are broken by list order, which trimming
 does not change, so the picture is the same while the shapes are fixed and nothing waits for the host.
 
-Only Torch ops on the engine's own tensors are used (the float32 ``atan2`` that picks a sprite rotation
-among them), so the result is the reference's own on whatever device the engine lives.
+``pack_actors`` uses only Torch ops on the engine's own tensors (the float32 ``atan2`` that picks a sprite rotation
+among them), so the result is the reference's own on whatever device the engine lives; ``pack_actors_fused`` gives the
+same list on a ROCm device by one kernel.
 """
 
 from __future__ import annotations
@@ -19,6 +20,8 @@ import math
 
 import numpy as np
 import torch
+
+from . import hostmath
 
 OPAQUE, TRANSLUCENT = -1, -2
 
@@ -244,14 +247,36 @@ def compact_actors(packed: dict[str, torch.Tensor], limit: int) -> dict[str, tor
 
 
 _TORCH_OF = {np.float32: torch.float32, np.uint8: torch.uint8, np.int64: torch.int64, np.int32: torch.int32, np.int8: torch.int8}
+_ROTATIONS = frozenset(("enemy_rotation", "doll_rotation", "projectile_rotation", "enemy_projectile_rotation"))
+_COLUMNS = frozenset(("doll_x", "doll_y", "item_x", "item_y"))       # of the map's player_starts and item_spawns
+
+
+def _faced_in_place(engine, lanes: int) -> bool:
+    """Are the tensors that sprite rotations come from laid out as the kernel reads them, and is only its result wanted?"""
+
+    x, enemy, shot, fireball = engine.x, engine.enemy_x, engine.projectile_x, engine.enemy_projectile_x
+    alike = (
+        (x, engine.y), (enemy, engine.enemy_y, engine.enemy_angle),
+        (shot, engine.projectile_y, engine.projectile_velocity_x, engine.projectile_velocity_y),
+        (fireball, engine.enemy_projectile_y, engine.enemy_projectile_velocity_x, engine.enemy_projectile_velocity_y),
+    )
+    if not hostmath._on_device(*(t for kind in alike for t in kind)) or any(t.shape != kind[0].shape for kind in alike for t in kind):
+        return False
+    if x.dim() != 1 or any(kind[0].dim() != 2 or kind[0].shape[0] != lanes for kind in alike[1:]):
+        return False
+    tables = (engine.map.player_starts, engine.map.item_spawns)
+    return hostmath._plain_call(*tables) and all(
+        t.dtype is torch.float32 and t.device == x.device and t.dim() == 2 and t.shape[1] >= 2 and t.stride(0) < 1 << 31 for t in tables
+    ) and tables[0].shape[0] >= 2 and tables[0].shape[1] >= 3      # at least one doll
 
 
 def pack_actors_fused(engine, limit: int = 512) -> dict[str, torch.Tensor]:
-    """``pack_actors`` as one HIP kernel (``gd_pack_actors``): same list, same order, same dtypes.
+    """``pack_actors`` as one HIP kernel (``gd_pack_actors_facing``): same list, same order, same dtypes.
 
-    The four sprite rotations still come from the reference's float32 Torch ops (``atan2``); everything
-    else - frame selection, patch lookup, flags, the concatenation - happens in one launch that reads the
-    engine's tensors where they are.  Needs the engine on a ROCm device and the library built.
+    Frame selection, sprite rotations, patch lookup, flags and the concatenation happen in one launch that reads the engine's tensors
+    where they are.  Where the tensors that rotations come from are not laid out as the kernel reads them (or a call is recorded,
+    transformed or traced), the rotations are Torch's expressions and the kernel (``gd_pack_actors``) reads those.  Needs the engine on a ROCm device and the
+    library built.
     """
 
     from . import _abi, _lib
@@ -262,17 +287,20 @@ def pack_actors_fused(engine, limit: int = 512) -> dict[str, torch.Tensor]:
         raise RuntimeError("pack_actors_fused needs the engine's tensors on the GPU")
     lanes = int(engine.x.shape[0])
     dolls = m.player_starts[:-1]
-    rotations = dict(
-        enemy_rotation=_rotation(_seen_from(engine, engine.enemy_x, engine.enemy_y), engine.enemy_angle),
-        projectile_rotation=_rotation(_seen_from(engine, engine.projectile_x, engine.projectile_y),
-                                      torch.atan2(engine.projectile_velocity_y, engine.projectile_velocity_x)),
-        enemy_projectile_rotation=_rotation(_seen_from(engine, engine.enemy_projectile_x, engine.enemy_projectile_y),
-                                            torch.atan2(engine.enemy_projectile_velocity_y, engine.enemy_projectile_velocity_x)),
-    )
-    if len(dolls):
-        doll_x = dolls[None, :, 0].expand(lanes, -1)
-        doll_y = dolls[None, :, 1].expand(lanes, -1)
-        rotations["doll_rotation"] = _rotation(_seen_from(engine, doll_x, doll_y), torch.deg2rad(dolls[None, :, 2]).expand(lanes, -1))
+    faced = _faced_in_place(engine, lanes)
+    rotations = {}
+    if not faced:
+        rotations = dict(
+            enemy_rotation=_rotation(_seen_from(engine, engine.enemy_x, engine.enemy_y), engine.enemy_angle),
+            projectile_rotation=_rotation(_seen_from(engine, engine.projectile_x, engine.projectile_y),
+                                          torch.atan2(engine.projectile_velocity_y, engine.projectile_velocity_x)),
+            enemy_projectile_rotation=_rotation(_seen_from(engine, engine.enemy_projectile_x, engine.enemy_projectile_y),
+                                                torch.atan2(engine.enemy_projectile_velocity_y, engine.enemy_projectile_velocity_x)),
+        )
+        if len(dolls):
+            doll_x = dolls[None, :, 0].expand(lanes, -1)
+            doll_y = dolls[None, :, 1].expand(lanes, -1)
+            rotations["doll_rotation"] = _rotation(_seen_from(engine, doll_x, doll_y), torch.deg2rad(dolls[None, :, 2]).expand(lanes, -1))
     derived = dict(
         doll_x=dolls[:, 0], doll_y=dolls[:, 1], doll_z=engine._player_start_z[:-1],
         item_x=m.item_spawns[:, 0], item_y=m.item_spawns[:, 1], item_z=engine._item_z,
@@ -297,6 +325,8 @@ def pack_actors_fused(engine, limit: int = 512) -> dict[str, torch.Tensor]:
         raise ValueError("raw_static_sprite_ids needs at least 15 entries")
     keep = []
     for name, dtype in _abi.ACTOR_ARRAYS:
+        if faced and name in _ROTATIONS:
+            continue
         if name in rotations:
             value = rotations[name].to(torch.uint8)
         elif name in derived:
@@ -312,7 +342,8 @@ def pack_actors_fused(engine, limit: int = 512) -> dict[str, torch.Tensor]:
             raise TypeError(f"{name} must be {wanted}, got {value.dtype}")
         if value.device != device:
             raise TypeError(f"{name} must live on {device}")
-        value = value.contiguous()
+        if not (faced and name in _COLUMNS):
+            value = value.contiguous()
         keep.append(value)
         setattr(desc, name, value.data_ptr() if value.numel() else None)
     width = (2 * desc.enemy_slots + desc.doll_count + 2 * desc.player_projectile_slots + 2 * desc.enemy_projectile_slots
@@ -322,6 +353,17 @@ def pack_actors_fused(engine, limit: int = 512) -> dict[str, torch.Tensor]:
         packed[name] = torch.empty((lanes, width), dtype=_TORCH_OF[dtype], device=device)
         setattr(desc, name, packed[name].data_ptr())
     stream = torch.cuda.current_stream(device).cuda_stream
-    _lib.check(_lib.library().gd_pack_actors(C.byref(desc), C.c_void_p(stream)))
+    if faced:
+        facing = _abi.FacingDesc()
+        facing.doll_stride, facing.item_stride = m.player_starts.stride(0), m.item_spawns.stride(0)
+        for name, value in (
+            ("x", engine.x), ("y", engine.y), ("enemy_angle", engine.enemy_angle), ("doll_degrees", dolls[:, 2]),
+            ("projectile_velocity_x", engine.projectile_velocity_x), ("projectile_velocity_y", engine.projectile_velocity_y),
+            ("enemy_projectile_velocity_x", engine.enemy_projectile_velocity_x), ("enemy_projectile_velocity_y", engine.enemy_projectile_velocity_y),
+        ):
+            setattr(facing, name, value.data_ptr() if value.numel() else None)
+        _lib.check(_lib.library().gd_pack_actors_facing(C.byref(desc), C.byref(facing), C.c_void_p(stream)))
+    else:
+        _lib.check(_lib.library().gd_pack_actors(C.byref(desc), C.c_void_p(stream)))
     del keep
     return compact_actors(packed, limit) if limit else packed

@@ -5373,7 +5373,20 @@ __device__ __forceinline__ i64 explosion_patch(const gd_actor_desc &a, i64 kind,
     return a.raw_projectile_explosion_sprite_ids[kind * F + frame];
 }
 
-__global__ void __launch_bounds__(64) pack_actors_kernel(gd_actor_desc a, int width) {
+// Doom's clockwise 1..8 sprite rotation as 0..7 (engine.py:13994-14009) of an actor at (x, y) that faces `heading`, one rounded operation at a
+// time as Torch evaluates the expression on a device, where a tensor over a number is multiplied by the number's reciprocal.
+__device__ __forceinline__ int facing_of(const gd_facing_desc &f, int n, float x, float y, float heading) {
+    const float TWO_PI = (float)(2.0 * 3.14159265358979323846), EIGHTH_PI = (float)(3.14159265358979323846 / 8), PER_QUARTER_PI = 1.0f / (float)(3.14159265358979323846 / 4);
+    float turn = fmodf((atan2f(f.y[n] - y, f.x[n] - x) - heading) + EIGHTH_PI, TWO_PI);
+    if (turn != 0.0f && turn < 0.0f) turn += TWO_PI;         // torch.remainder with a positive divisor
+    return (int)((i64)floorf(turn * PER_QUARTER_PI) & 7);
+}
+
+// FACING: rotations are worked out here (gd_pack_actors_facing), not read.  As Torch operators they were some forty kernels, and the copies of
+// the map's columns and the weapon's words a dozen more: with them an engine's frame of 2048 lanes took 2484 us, of one lane (which the host's
+// launches take longest for) 619 us; without 2229 and 303 us.  This kernel takes 29 us at 2048 lanes of 495 slots, 26 where it reads rotations.
+template <bool FACING>
+__global__ void __launch_bounds__(64) pack_actors_kernel(gd_actor_desc a, gd_facing_desc f, int width) {
     const int slot = blockIdx.x * blockDim.x + threadIdx.x;
     const int n = blockIdx.y;
     if (slot >= width || n >= a.lane_count) return;
@@ -5384,7 +5397,7 @@ __global__ void __launch_bounds__(64) pack_actors_kernel(gd_actor_desc a, int wi
         const size_t i = (size_t)n * Se + k;
         x = a.enemy_x[i]; y = a.enemy_y[i]; z = a.enemy_z[i]; alive = a.enemy_alive[i] != 0;
         const i64 kind = clamp_type(a.enemy_type[i], 5);
-        const int facing = a.enemy_rotation[i];
+        const int facing = FACING ? facing_of(f, n, x, y, f.enemy_angle[i]) : a.enemy_rotation[i];
         const int tics = a.enemy_animation_tics[i];
         int walking = (tics / a.enemy_walk_frame_tics[kind]) % 4;
         int idling = (tics / a.enemy_idle_frame_tics[kind]) % 2;
@@ -5404,8 +5417,10 @@ __global__ void __launch_bounds__(64) pack_actors_kernel(gd_actor_desc a, int wi
         if (a.enemy_pain_tics[i] > 0) patch = a.enemy_pain_sprite_ids[kind * 8 + facing];
         bright = (kind == 1 && phase == 2 && recovering) || (kind == 3 && (phase == 2 || phase == 3));
     } else if ((k -= Se) < Sd) {                    // the other players' start dolls (engine.py:14345-14379)
-        x = a.doll_x[k]; y = a.doll_y[k]; z = a.doll_z[k]; alive = a.player_dead[n] == 0;
-        patch = a.enemy_walk_sprite_ids[(2 * 4 + 0) * 8 + a.doll_rotation[(size_t)n * Sd + k]];
+        const size_t row = FACING ? (size_t)k * f.doll_stride : k;
+        x = a.doll_x[row]; y = a.doll_y[row]; z = a.doll_z[k]; alive = a.player_dead[n] == 0;
+        const int facing = FACING ? facing_of(f, n, x, y, f.doll_degrees[row] * (float)(3.14159265358979323846 / 180)) : a.doll_rotation[(size_t)n * Sd + k];
+        patch = a.enemy_walk_sprite_ids[(2 * 4 + 0) * 8 + facing];
     } else if ((k -= Sd) < Se) {                    // corpses (engine.py:14079-14106)
         const size_t i = (size_t)n * Se + k;
         x = a.enemy_x[i]; y = a.enemy_y[i]; z = a.enemy_z[i]; alive = a.enemy_death_tics[i] > 0;
@@ -5423,13 +5438,15 @@ __global__ void __launch_bounds__(64) pack_actors_kernel(gd_actor_desc a, int wi
         x = a.projectile_x[i]; y = a.projectile_y[i]; z = a.projectile_z[i]; alive = a.projectile_alive[i] != 0;
         const i64 shot = clamp_type(a.projectile_type[i], 1);
         const int frame = shot == 1 ? (a.projectile_age[i] / 6) % 2 : 0;
-        patch = a.raw_projectile_flight_sprite_ids[(shot * 2 + frame) * 8 + a.projectile_rotation[i]];
+        const int facing = FACING ? facing_of(f, n, x, y, atan2f(f.projectile_velocity_y[i], f.projectile_velocity_x[i])) : a.projectile_rotation[i];
+        patch = a.raw_projectile_flight_sprite_ids[(shot * 2 + frame) * 8 + facing];
         bright = alive; style = shot == 1 ? 0 : -1;
     } else if ((k -= Sp) < Sq) {                    // monster fireballs in flight (engine.py:14462-14510)
         const size_t i = (size_t)n * Sq + k;
         x = a.enemy_projectile_x[i]; y = a.enemy_projectile_y[i]; z = a.enemy_projectile_z[i]; alive = a.enemy_projectile_alive[i] != 0;
         const int frame = (a.enemy_projectile_age[i] / 4) % 2;
-        patch = a.raw_projectile_flight_sprite_ids[(2 * 2 + frame) * 8 + a.enemy_projectile_rotation[i]];
+        const int facing = FACING ? facing_of(f, n, x, y, atan2f(f.enemy_projectile_velocity_y[i], f.enemy_projectile_velocity_x[i])) : a.enemy_projectile_rotation[i];
+        patch = a.raw_projectile_flight_sprite_ids[(2 * 2 + frame) * 8 + facing];
         bright = alive; style = 1;
     } else if ((k -= Sq) < Sp) {                    // the player's explosions (engine.py:14512-14541)
         const size_t i = (size_t)n * Sp + k;
@@ -5462,7 +5479,8 @@ __global__ void __launch_bounds__(64) pack_actors_kernel(gd_actor_desc a, int wi
         bright = frame == 0; style = -2;
     } else if ((k -= a.puff_slots) < a.item_count) {   // map items (engine.py:14258-14317, 14632-14655)
         const size_t i = (size_t)n * a.item_count + k;
-        x = a.item_x[k]; y = a.item_y[k]; z = a.item_z[k]; alive = a.item_available[i] != 0;
+        const size_t row = FACING ? (size_t)k * f.item_stride : k;
+        x = a.item_x[row]; y = a.item_y[row]; z = a.item_z[k]; alive = a.item_available[i] != 0;
         const i64 kind = a.item_types[k];
         const i64 elapsed = (i64)a.episode_time[n] + (6 - (i64)a.item_animation_initial_tics[i]);
         const i64 sixth = elapsed >= 0 ? elapsed / 6 : -((-elapsed + 5) / 6);
@@ -5500,25 +5518,27 @@ int fail(int code, const std::string &message) { return gd_fail(code, message); 
 // alternates every four tics instead) and by the tics left of the weapon's state; a weapon being lowered or raised sits
 // six map pixels lower per tic, as does one raised at the start of an episode; a ready weapon sways with the player's bob
 // along a circle of the fine sine table that advances 128 steps a tic.
-__global__ void __launch_bounds__(64) pack_weapon_kernel(gd_weapon_desc d) {
+__global__ void __launch_bounds__(64) pack_weapon_kernel(gd_weapon_desc d, unsigned narrow) {
     const int lane = blockIdx.x * blockDim.x + threadIdx.x;
     if (lane >= d.lane_count) return;
+    // word k of the descriptor's nine, which is 32 bits wide where bit k of `narrow` is set
+    const auto word = [&](const int64_t *words, int k) -> i64 { return (narrow >> k) & 1u ? reinterpret_cast<const int32_t *>(words)[lane] : words[lane]; };
     const i64 slots = d.cooldown_slots;
-    const i64 weapon = clampi(d.active_weapon[lane], 0, 7);
-    const i64 state_tics = d.weapon_state_cooldown[lane];
+    const i64 weapon = clampi(word(d.active_weapon, 0), 0, 7);
+    const i64 state_tics = word(d.weapon_state_cooldown, 1);
     const i64 tic = clampi(state_tics, 0, slots - 1);
-    i64 parity = d.weapon_fire_count[lane] % 2;
+    i64 parity = word(d.weapon_fire_count, 2) % 2;
     if (parity < 0) parity += 2;                    // torch.remainder: the sign of the divisor
-    if (weapon == 1 && tic == 0) parity = (max64(d.weapon_ready_tics[lane] - 1, 0) / 4) % 2;
+    if (weapon == 1 && tic == 0) parity = (max64(word(d.weapon_ready_tics, 3) - 1, 0) / 4) % 2;
     const i64 entry = (weapon * 2 + parity) * slots + tic;
-    const i64 switching = d.pending_weapon[lane] >= 0;
-    const i64 raising = d.weapon_raise_cooldown[lane];
-    i64 lowered = switching ? clampi(16 - d.weapon_lower_cooldown[lane], 0, 16) : raising;      // engine.py:111 (16 tics to lower)
-    const i64 time = d.episode_time[lane];
+    const i64 switching = word(d.pending_weapon, 6) >= 0;
+    const i64 raising = word(d.weapon_raise_cooldown, 5);
+    i64 lowered = switching ? clampi(16 - word(d.weapon_lower_cooldown, 4), 0, 16) : raising;      // engine.py:111 (16 tics to lower)
+    const i64 time = word(d.episode_time, 7);
     lowered = max64(lowered, clampi(14 - (time - 1), 0, 14));                                   // engine.py:114 (14 tics to raise at spawn)
     const bool steady = state_tics <= 0 && raising <= 0 && !switching;
     const i64 swing = mul64(time, 128) & (FINE_ANGLES - 1);
-    const i64 bob = d.player_bob_fixed[lane];
+    const i64 bob = word(d.player_bob_fixed, 8);
     const i64 sway_x = steady ? mul64(bob, d.fine_sine[(swing + FINE_ANGLES / 4) & (FINE_ANGLES - 1)]) >> 16 : 0;
     const i64 sway_y = steady ? mul64(bob, d.fine_sine[swing & (FINE_ANGLES / 2 - 1)]) >> 16 : 0;
     int64_t *out = d.weapon_state + (size_t)lane * 5;
@@ -6540,30 +6560,62 @@ int gd_expand_rgb24(const uint8_t *indexed, int32_t rows, const uint8_t *playpal
     return GD_OK;
 }
 
-int gd_pack_actors(const gd_actor_desc *a, void *stream) {
-    if (!a) return fail(GD_E_ARG, "null argument");
-    SIZE_CHECK(a, gd_actor_desc);
+namespace {
+int pack_actors(const gd_actor_desc *a, const gd_facing_desc *facing, void *stream) {
     const int32_t counts[] = {a->lane_count, a->enemy_slots, a->doll_count, a->player_projectile_slots, a->enemy_projectile_slots,
                               a->fog_slots, a->puff_slots, a->item_count, a->drop_slots};
     for (int32_t v : counts) if (v < 0) return fail(GD_E_ARG, "negative count");
     if (a->attack_frames < 3 || a->death_frames < 1 || a->xdeath_frames < 1 || a->explosion_frames < 1)
         return fail(GD_E_ARG, "animation tables need at least 3 attack frames and 1 frame of every other kind");
     // every pointer of the descriptor sits between the scalars and the end of the struct
-    const void *const *first = reinterpret_cast<const void *const *>(&a->enemy_x);
-    const void *const *last = reinterpret_cast<const void *const *>(&a->sprite_style);
-    for (const void *const *p = first; p <= last; ++p) {
-        const bool doll = p >= reinterpret_cast<const void *const *>(&a->doll_x) && p <= reinterpret_cast<const void *const *>(&a->doll_rotation);
-        const bool item = p >= reinterpret_cast<const void *const *>(&a->item_x) && p <= reinterpret_cast<const void *const *>(&a->item_animation_initial_tics);
-        if (!*p && !(doll && a->doll_count == 0) && !(item && a->item_count == 0)) return fail(GD_E_ARG, "null tensor in gd_actor_desc");
+    const auto at = [](const void *field) { return static_cast<const void *const *>(field); };
+    for (const void *const *p = at(&a->enemy_x); p <= at(&a->sprite_style); ++p) {
+        const bool doll = p >= at(&a->doll_x) && p <= at(&a->doll_rotation);
+        const bool item = p >= at(&a->item_x) && p <= at(&a->item_animation_initial_tics);
+        const bool rotation = p == at(&a->enemy_rotation) || p == at(&a->doll_rotation) || p == at(&a->projectile_rotation) || p == at(&a->enemy_projectile_rotation);
+        if (!*p && !(doll && a->doll_count == 0) && !(item && a->item_count == 0) && !(rotation && facing)) return fail(GD_E_ARG, "null tensor in gd_actor_desc");
+    }
+    if (facing) {
+        if (facing->doll_stride < 0 || facing->item_stride < 0) return fail(GD_E_ARG, "negative stride");
+        const bool missing = !facing->x || !facing->y || !facing->enemy_angle || (!facing->doll_degrees && a->doll_count) || !facing->projectile_velocity_x ||
+                             !facing->projectile_velocity_y || !facing->enemy_projectile_velocity_x || !facing->enemy_projectile_velocity_y;
+        if (missing) return fail(GD_E_ARG, "null tensor in gd_facing_desc");
     }
     const long long width = 2LL * a->enemy_slots + a->doll_count + 2LL * a->player_projectile_slots + 2LL * a->enemy_projectile_slots +
                             a->fog_slots + a->puff_slots + a->item_count + a->drop_slots;
     if (a->lane_count == 0 || width == 0) return GD_OK;
     if (width > 65535 * 64LL || a->lane_count > 65535) return fail(GD_E_ARG, "too many slots or lanes for one launch");
-    hipLaunchKernelGGL(pack_actors_kernel, dim3((unsigned)((width + 63) / 64), (unsigned)a->lane_count), dim3(64), 0,
-                       static_cast<hipStream_t>(stream), *a, (int)width);
+    hipLaunchKernelGGL(facing ? pack_actors_kernel<true> : pack_actors_kernel<false>, dim3((unsigned)((width + 63) / 64), (unsigned)a->lane_count), dim3(64), 0,
+                       static_cast<hipStream_t>(stream), *a, facing ? *facing : gd_facing_desc{}, (int)width);
     HIP_TRY(hipGetLastError());
     return GD_OK;
+}
+
+int pack_weapon(const gd_weapon_desc *w, unsigned narrow, void *stream) {
+    if (w->lane_count < 0 || w->cooldown_slots <= 0) return fail(GD_E_ARG, "gd_weapon_desc holds a count out of range");
+    const void *const needed[] = {w->active_weapon, w->weapon_state_cooldown, w->weapon_fire_count, w->weapon_ready_tics, w->weapon_lower_cooldown,
+                                  w->weapon_raise_cooldown, w->pending_weapon, w->episode_time, w->player_bob_fixed, w->player_dead,
+                                  w->weapon_frame_ids, w->weapon_flash_ids, w->fine_sine, w->weapon_state};
+    for (const void *p : needed) if (!p) return fail(GD_E_ARG, "null tensor in gd_weapon_desc");
+    if (w->flash_light && !w->weapon_flash_lights) return fail(GD_E_ARG, "flash_light needs weapon_flash_lights");
+    if (w->lane_count == 0) return GD_OK;
+    hipLaunchKernelGGL(pack_weapon_kernel, dim3((unsigned)((w->lane_count + 63) / 64)), dim3(64), 0, static_cast<hipStream_t>(stream), *w, narrow);
+    HIP_TRY(hipGetLastError());
+    return GD_OK;
+}
+}  // namespace
+
+int gd_pack_actors(const gd_actor_desc *a, void *stream) {
+    if (!a) return fail(GD_E_ARG, "null argument");
+    SIZE_CHECK(a, gd_actor_desc);
+    return pack_actors(a, nullptr, stream);
+}
+
+int gd_pack_actors_facing(const gd_actor_desc *a, const gd_facing_desc *facing, void *stream) {
+    if (!a || !facing) return fail(GD_E_ARG, "null argument");
+    SIZE_CHECK(a, gd_actor_desc);
+    SIZE_CHECK(facing, gd_facing_desc);
+    return pack_actors(a, facing, stream);
 }
 
 int gd_ray_tables(const float *angle, const float *ray_offsets, int32_t lane_count, float *ray_cos, float *ray_sin, void *stream) {
@@ -6593,16 +6645,14 @@ int gd_sprite_depth(const float *x, const float *y, const float *angle, const fl
 int gd_pack_weapon(const gd_weapon_desc *w, void *stream) {
     if (!w) return fail(GD_E_ARG, "null argument");
     SIZE_CHECK(w, gd_weapon_desc);
-    if (w->lane_count < 0 || w->cooldown_slots <= 0) return fail(GD_E_ARG, "gd_weapon_desc holds a count out of range");
-    const void *const needed[] = {w->active_weapon, w->weapon_state_cooldown, w->weapon_fire_count, w->weapon_ready_tics, w->weapon_lower_cooldown,
-                                  w->weapon_raise_cooldown, w->pending_weapon, w->episode_time, w->player_bob_fixed, w->player_dead,
-                                  w->weapon_frame_ids, w->weapon_flash_ids, w->fine_sine, w->weapon_state};
-    for (const void *p : needed) if (!p) return fail(GD_E_ARG, "null tensor in gd_weapon_desc");
-    if (w->flash_light && !w->weapon_flash_lights) return fail(GD_E_ARG, "flash_light needs weapon_flash_lights");
-    if (w->lane_count == 0) return GD_OK;
-    hipLaunchKernelGGL(pack_weapon_kernel, dim3((unsigned)((w->lane_count + 63) / 64)), dim3(64), 0, static_cast<hipStream_t>(stream), *w);
-    HIP_TRY(hipGetLastError());
-    return GD_OK;
+    return pack_weapon(w, 0u, stream);
+}
+
+int gd_pack_weapon_narrow(const gd_weapon_desc *w, uint32_t narrow, void *stream) {
+    if (!w) return fail(GD_E_ARG, "null argument");
+    SIZE_CHECK(w, gd_weapon_desc);
+    if (narrow >> 9) return fail(GD_E_ARG, "gd_weapon_desc has nine words a lane");
+    return pack_weapon(w, narrow, stream);
 }
 
 int gd_pack_decals(const int64_t *serial, const int64_t *wall, const float *along, const float *impact_z, const int64_t *style, const float *walls,

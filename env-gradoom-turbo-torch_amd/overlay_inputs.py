@@ -55,7 +55,7 @@ def weapon_state(*, weapon_frame_ids: torch.Tensor, weapon_flash_ids: torch.Tens
     ``fine_sine`` the table of :func:`fine_sine_fixed`.  With ``want_flash_light`` the muzzle flash's extra light level
     comes back as well (``int64 [N]``).
 
-    Tensors on a ROCm device are read where they are by one kernel (``gd_pack_weapon``): no host synchronisation.
+    Tensors on a ROCm device are read where they are by one kernel (``gd_pack_weapon_narrow``): no host synchronisation.
     Host tensors (tests, fixture scripts) take the NumPy restatement below.
     """
 
@@ -90,8 +90,11 @@ def _weapon_state_device(engine, frame_ids, flash_ids, flash_lights, fine_sine, 
         keep.append(tensor)
         return tensor.data_ptr()
 
-    for name in _WEAPON_INPUTS:
-        setattr(desc, name, pointer(engine[name], torch.int64))
+    narrow = 0
+    for k, name in enumerate(_WEAPON_INPUTS):
+        tics = engine[name].dtype is torch.int32       # read as they are: a conversion would be a kernel each
+        setattr(desc, name, pointer(engine[name], torch.int32 if tics else torch.int64))
+        narrow |= int(tics) << k
     desc.player_dead = pointer(engine["player_dead"], torch.uint8)
     desc.weapon_frame_ids = pointer(frame_ids, torch.int64)
     desc.weapon_flash_ids = pointer(flash_ids, torch.int64)
@@ -107,7 +110,7 @@ def _weapon_state_device(engine, frame_ids, flash_ids, flash_lights, fine_sine, 
         desc.flash_light = light.data_ptr()
     with torch.cuda.device(device):
         stream = torch.cuda.current_stream(device).cuda_stream
-        _lib.check(_lib.library().gd_pack_weapon(C.byref(desc), C.c_void_p(stream)))
+        _lib.check(_lib.library().gd_pack_weapon_narrow(C.byref(desc), narrow, C.c_void_p(stream)))
     del keep
     return (words, light) if want_flash_light else words
 

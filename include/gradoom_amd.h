@@ -466,6 +466,27 @@ typedef struct gd_actor_desc {
 int gd_pack_actors(const gd_actor_desc *actors, void *stream);
 
 /*
+ * gd_pack_actors with the rotations worked out in the kernel, to the bits of the Torch expressions on this device (each operation is rounded
+ * on its own, atan2 and fmod are the device library's): the *_rotation arrays of gd_actor_desc are not read and may be null.  doll_x, doll_y
+ * and doll_degrees step by doll_stride floats from one doll to the next, item_x and item_y by item_stride: columns of the map's
+ * player_starts and item_spawns.
+ */
+typedef struct gd_facing_desc {
+    uint32_t struct_size;    /* sizeof(gd_facing_desc) of the header the caller was built with */
+    int32_t doll_stride, item_stride;
+    const float *x;  /* [N] the cameras */
+    const float *y;
+    const float *enemy_angle;  /* [N,Se] */
+    const float *doll_degrees;  /* [Sd] player_starts[:-1,2] */
+    const float *projectile_velocity_x;  /* [N,Sp] */
+    const float *projectile_velocity_y;
+    const float *enemy_projectile_velocity_x;  /* [N,Sq] */
+    const float *enemy_projectile_velocity_y;
+} gd_facing_desc;
+
+int gd_pack_actors_facing(const gd_actor_desc *actors, const gd_facing_desc *facing, void *stream);
+
+/*
  * The five weapon_state words of every lane (gd_lanes_desc.weapon_state) and the muzzle flash's extra light
  * (gd_lanes_desc.flash_light), from the gameplay tensors, in one kernel with no host synchronisation.
  * Replaces the per-lane part of the reference's weapon layer: frame / flash selection
@@ -500,6 +521,9 @@ typedef struct gd_weapon_desc {
 } gd_weapon_desc;
 
 int gd_pack_weapon(const gd_weapon_desc *weapon, void *stream);
+/* gd_pack_weapon with the words as wide as the engine keeps them: where bit k of `narrow` is set, the k-th of the nine words a lane (in the
+ * descriptor's order, active_weapon to player_bob_fixed) points to int32_t. */
+int gd_pack_weapon_narrow(const gd_weapon_desc *weapon, uint32_t narrow, void *stream);
 
 /*
  * gd_pack_decals: gd_lanes_desc.decal_state [N,D,3] and decal_geom [N,D,4] from an engine's decal slots [N,D] (engine.py:13756-13829): the live

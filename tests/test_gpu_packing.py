@@ -88,3 +88,68 @@ def test_screen_flashes_of_other_shapes_are_packed_as_on_the_host():
         expected = overlay_inputs.screen_blend(*counters)
         # the device multiplies with the divisor's reciprocal: two roundings of 2^-24 where the host's division has one
         assert packed.shape == expected.shape and torch.allclose(packed.cpu(), expected, rtol=2.0**-22, atol=0)
+
+
+@pytest.mark.parametrize("lanes", [1, 33, 257])
+@pytest.mark.parametrize("form", ["plain", "wide tables", "two starts"])
+def test_actors_face_the_camera_as_the_torch_expressions_have_them(lanes, form):
+    """The kernel's own rotations against Torch's, which tensors that are not laid out as it reads them still take: every octant, actors on
+    the camera, along the axes, and values that are no numbers."""
+    from conftest import load_fixture
+    from test_actor_inputs import stored_engine
+
+    from gradoom_amd import actor_inputs
+
+    engine = stored_engine(load_fixture("actors")[1])
+    rng = torch.Generator(device="cuda:0").manual_seed(lanes)
+    per_map = ("_enemy_walk_frame_tics", "_enemy_idle_frame_tics", "_enemy_attack_recovery", "_player_start_z", "_item_z")
+    for field in actor_inputs.ENGINE_FIELDS:
+        value = getattr(engine, field)
+        if field not in per_map:
+            value = value[torch.arange(lanes) % value.shape[0]]
+        setattr(engine, field, value.to("cuda:0"))
+    m = engine.map
+    for field in actor_inputs.MAP_FIELDS:
+        setattr(m, field, getattr(m, field).to("cuda:0"))
+    for kind, first, second in (("enemy", "x", "y"), ("projectile", "velocity_x", "velocity_y"), ("enemy_projectile", "x", "y"), ("enemy_projectile", "velocity_x", "velocity_y")):
+        for name, other in ((first, second), (second, first)):
+            values = getattr(engine, f"{kind}_{name}")
+            values.copy_(torch.randn(values.shape, generator=rng, device="cuda:0") * 300)
+            values[:, 0], getattr(engine, f"{kind}_{other}")[:, 0] = 0.0, -0.0
+            values[:, 1] = float("inf")
+            values[:, 2] = float("nan")
+    engine.enemy_x[:, 3], engine.enemy_y[:, 3] = engine.x, engine.y
+    engine.enemy_x[:, 4] = engine.x
+    angles = torch.arange(engine.enemy_angle.shape[1], device="cuda:0") * (torch.pi / 8)
+    engine.enemy_angle.copy_(torch.where(torch.rand(engine.enemy_angle.shape, generator=rng, device="cuda:0") < 0.5, angles, -7.0 * angles))
+    if form == "wide tables":
+        m.player_starts, m.item_spawns = (torch.cat((t, t), dim=1)[:, : t.shape[1]] for t in (m.player_starts, m.item_spawns))
+    if form == "two starts":
+        m.player_starts, engine._player_start_z = m.player_starts[:2], engine._player_start_z[:2]
+    assert actor_inputs._faced_in_place(engine, lanes)
+    packed = actor_inputs.pack_actors_fused(engine, limit=0)
+    engine.enemy_angle = spread(engine.enemy_angle)
+    assert not actor_inputs._faced_in_place(engine, lanes)
+    expected = actor_inputs.pack_actors_fused(engine, limit=0)
+    for key in expected:
+        same = packed[key] == expected[key]
+        if key in ("sprite_x", "sprite_y"):
+            same |= packed[key].isnan() & expected[key].isnan()
+        assert packed[key].dtype == expected[key].dtype and bool(same.all()), key
+
+
+@pytest.mark.parametrize("narrow", range(10))
+def test_weapon_words_are_read_as_wide_as_they_are_kept(narrow):
+    from gradoom_amd import overlay_inputs
+
+    rng = torch.Generator(device="cuda:0").manual_seed(5)
+    lanes = 65
+    words = {name: torch.randint(-3, 40, (lanes,), generator=rng, device="cuda:0") for name in overlay_inputs._WEAPON_INPUTS}
+    tables = {name: torch.randint(0, 50, (8, 2, 11), generator=rng, device="cuda:0") for name in ("weapon_frame_ids", "weapon_flash_ids", "weapon_flash_lights")}
+    tables.update(fine_sine=torch.as_tensor(overlay_inputs.fine_sine_fixed(), device="cuda:0"), player_dead=torch.arange(lanes, device="cuda:0") % 3 == 0)
+    expected = overlay_inputs.weapon_state(**words, **tables, want_flash_light=True)
+    for k, name in enumerate(words):
+        if narrow == 9 or k == narrow:
+            words[name] = words[name].to(torch.int32)
+    packed = overlay_inputs.weapon_state(**words, **tables, want_flash_light=True)
+    assert torch.equal(packed[0], expected[0]) and torch.equal(packed[1], expected[1])
