@@ -403,6 +403,19 @@ class WeaponDesc(_Sized):
     )
 
 
+HUD_REALS = ("hud_ready_ammo", "health", "armor", "weapons", "hud_ammo_counts")
+HUD_COUNTERS = ("mugshot_face_index", "mugshot_grin_tics", "mugshot_pain_tics", "mugshot_pain_direction", "attack_held_tics")
+
+
+class HudDesc(_Sized):
+    """``gd_hud_desc``: the gameplay tensors ``gd_pack_hud`` reads and the words it writes."""
+
+    _fields_ = (
+        [("struct_size", C.c_uint32)] + [(name, C.c_int32) for name in ("lane_count", "weapon_columns", "ammo_columns", "narrow")]
+        + [(name, _P) for name in ("ammo_slot", *HUD_REALS, *HUD_COUNTERS, "mugshot_ouch", "hud_state")]
+    )
+
+
 POSE_LANE_FIELDS = ("x", "y", "angle", "view_z", "x_fixed", "y_fixed", "angle_bam", "pitch_bam", "flash_light")
 POSE_SPRITE_FIELDS = ("sprite_x", "sprite_y", "sprite_z", "sprite_id", "sprite_alive", "sprite_fullbright")
 POSE_POOL_FIELDS = ("x", "y", "view_z", "angle_bam", "pitch_bam", "flash_light") + POSE_SPRITE_FIELDS

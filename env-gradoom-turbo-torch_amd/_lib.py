@@ -32,6 +32,7 @@ SYMBOLS = (
     "gd_pack_actors_facing",
     "gd_pack_weapon",
     "gd_pack_weapon_narrow",
+    "gd_pack_hud",
     "gd_pack_decals",
     "gd_screen_blend",
     "gd_ray_tables",
@@ -112,6 +113,7 @@ def library() -> C.CDLL:
     for name, arguments in (
         ("gd_pack_actors_facing", [C.POINTER(_abi.ActorDesc), C.POINTER(_abi.FacingDesc), C.c_void_p]),
         ("gd_pack_weapon_narrow", [C.POINTER(_abi.WeaponDesc), C.c_uint32, C.c_void_p]),
+        ("gd_pack_hud", [C.POINTER(_abi.HudDesc), C.c_void_p]),
         ("gd_pose_lanes", [C.POINTER(_abi.PoseDesc), C.c_void_p]),
         ("gd_pose_step", [C.c_void_p] * 3 + [C.c_int32, C.c_int64, C.c_int64] + [C.c_void_p] * 4),
         ("gd_pose_reset", [C.c_void_p] * 4 + [C.c_int32, C.c_int64, C.c_void_p]),

@@ -5589,6 +5589,28 @@ __global__ void __launch_bounds__(64) pack_decals_kernel(const int64_t *serial, 
     }
 }
 
+// gd_pack_hud: one thread per lane (engine.py:15209-15262).  As Torch operators these are some forty kernels, which the host takes 0.33 ms to
+// launch: as much as all else of a small batch's frame.
+__global__ void __launch_bounds__(64) pack_hud_kernel(gd_hud_desc d) {
+    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
+    if (lane >= d.lane_count) return;
+    const auto word = [&](const int64_t *words, int k) -> i64 { return (d.narrow >> k) & 1 ? reinterpret_cast<const int32_t *>(words)[lane] : words[lane]; };
+    const auto shown = [](float v) -> i64 { return (i64)(v < 0.0f ? 0.0f : (v > 999.0f ? 999.0f : v)); };      // clamp keeps what is not a number
+    const i64 health = shown(d.health[lane]), armor = shown(d.armor[lane]);
+    const i64 hurt = 100 - health, twentieth = hurt >= 0 ? hurt / 20 : -((19 - hurt) / 20), pain = clampi(twentieth, 0, 4);
+    i64 face = 13 + pain * 3 + word(d.mugshot_face_index, 0);
+    if (word(d.attack_held_tics, 4) >= 70) face = 49 + pain;                       // engine.py:175 (70 tics of fire to a rampage)
+    if (word(d.mugshot_pain_tics, 2) > 0) face = d.mugshot_ouch[lane] ? 59 + pain : 44 + 5 * word(d.mugshot_pain_direction, 3) + pain;
+    if (word(d.mugshot_grin_tics, 1) > 0) face = 64 + pain;
+    if (health <= 0) face = 69;
+    int owned = 0;
+    for (int weapon = 0; weapon < 5; ++weapon) owned |= (d.weapons[(size_t)lane * d.weapon_columns + weapon + 1] != 0.0f ? 1 : 0) << weapon;
+    int32_t *out = d.hud_state + (size_t)lane * 9;
+    out[0] = (int32_t)(i64)(d.ammo_slot[lane] < 0 ? 0.0f : d.hud_ready_ammo[lane]);
+    out[1] = (int32_t)health; out[2] = (int32_t)armor; out[3] = (int32_t)face; out[4] = owned;
+    for (int k = 0; k < 4; ++k) out[5 + k] = (int32_t)(i64)d.hud_ammo_counts[(size_t)lane * d.ammo_columns + k];
+}
+
 // gd_screen_blend: one thread per lane.  Torch divides by a constant on the device by multiplying with its reciprocal.
 __global__ void __launch_bounds__(256) screen_blend_kernel(const int64_t *bonus_count, const int64_t *damage_count, const float *damage_to_alpha, int lane_count, float *blend) {
     const int lane = blockIdx.x * blockDim.x + threadIdx.x;
@@ -6653,6 +6675,18 @@ int gd_pack_weapon_narrow(const gd_weapon_desc *w, uint32_t narrow, void *stream
     SIZE_CHECK(w, gd_weapon_desc);
     if (narrow >> 9) return fail(GD_E_ARG, "gd_weapon_desc has nine words a lane");
     return pack_weapon(w, narrow, stream);
+}
+
+int gd_pack_hud(const gd_hud_desc *h, void *stream) {
+    if (!h) return fail(GD_E_ARG, "null argument");
+    SIZE_CHECK(h, gd_hud_desc);
+    if (h->lane_count < 0 || h->weapon_columns < 6 || h->ammo_columns < 4 || h->narrow >> 5) return fail(GD_E_ARG, "gd_hud_desc holds a count out of range");
+    if (h->lane_count == 0) return GD_OK;
+    const auto at = [](const void *field) { return static_cast<const void *const *>(field); };
+    for (const void *const *p = at(&h->ammo_slot); p <= at(&h->hud_state); ++p) if (!*p) return fail(GD_E_ARG, "null tensor in gd_hud_desc");
+    hipLaunchKernelGGL(pack_hud_kernel, dim3((unsigned)((h->lane_count + 63) / 64)), dim3(64), 0, static_cast<hipStream_t>(stream), *h);
+    HIP_TRY(hipGetLastError());
+    return GD_OK;
 }
 
 int gd_pack_decals(const int64_t *serial, const int64_t *wall, const float *along, const float *impact_z, const int64_t *style, const float *walls,

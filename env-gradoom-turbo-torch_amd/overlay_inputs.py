@@ -188,6 +188,13 @@ def hud_state(
     """
 
     ammo_slot = weapon_ammo_slot[active_weapon.to(torch.int64)]
+    words = _hud_words_device(
+        ammo_slot, dict(hud_ready_ammo=hud_ready_ammo, health=health, armor=armor, weapons=weapons, hud_ammo_counts=hud_ammo_counts),
+        dict(mugshot_face_index=mugshot_face_index, mugshot_grin_tics=mugshot_grin_tics, mugshot_pain_tics=mugshot_pain_tics,
+             mugshot_pain_direction=mugshot_pain_direction, attack_held_tics=attack_held_tics), mugshot_ouch,
+    )
+    if words is not None:
+        return words
     ammo = torch.where(ammo_slot < 0, torch.zeros_like(hud_ready_ammo), hud_ready_ammo).to(torch.int64)
     health_int = health.clamp(0, 999).to(torch.int64)
     armor_int = armor.clamp(0, 999).to(torch.int64)
@@ -202,6 +209,37 @@ def hud_state(
     counts = hud_ammo_counts.to(torch.int64)
     columns = (ammo, health_int, armor_int, face, owned, counts[:, 0], counts[:, 1], counts[:, 2], counts[:, 3])
     return torch.stack(columns, dim=1).to(torch.int32).contiguous()
+
+
+def _hud_words_device(ammo_slot: torch.Tensor, reals: dict, counters: dict, ouch: torch.Tensor) -> torch.Tensor | None:
+    """The words of :func:`hud_state` by one kernel (``gd_pack_hud``), or ``None`` where the tensors are not as it reads them."""
+
+    lanes = ammo_slot.shape[0] if ammo_slot.dim() == 1 else -1
+    weapons, counts = reals["weapons"], reals["hud_ammo_counts"]
+    if not _read_in_place((ammo_slot,), tuple(reals.values())) or not hostmath._plain_call(*counters.values(), ouch):
+        return None
+    per_lane = (reals["hud_ready_ammo"], reals["health"], reals["armor"], ouch, *counters.values())
+    if any(t.shape != ammo_slot.shape or t.device != ammo_slot.device or not t.is_contiguous() for t in per_lane) or ouch.dtype is not torch.bool:
+        return None
+    if any(t.dtype not in (torch.int32, torch.int64) for t in counters.values()):
+        return None
+    if any(t.dim() != 2 or t.shape[0] != lanes or not least <= t.shape[1] < 1 << 31 for t, least in ((weapons, 6), (counts, 4))):
+        return None
+    import ctypes as C
+
+    from . import _abi, _lib
+
+    words = torch.empty((lanes, 9), dtype=torch.int32, device=ammo_slot.device)
+    desc = _abi.HudDesc()
+    desc.lane_count, desc.weapon_columns, desc.ammo_columns = lanes, weapons.shape[1], counts.shape[1]
+    desc.ammo_slot, desc.mugshot_ouch, desc.hud_state = ammo_slot.data_ptr(), ouch.data_ptr(), words.data_ptr()
+    for name, tensor in (*reals.items(), *counters.items()):
+        setattr(desc, name, tensor.data_ptr())
+    desc.narrow = sum((counters[name].dtype is torch.int32) << k for k, name in enumerate(_abi.HUD_COUNTERS))
+    with torch.cuda.device(words.device):
+        stream = torch.cuda.current_stream(words.device).cuda_stream
+        _lib.check(_lib.library().gd_pack_hud(C.byref(desc), C.c_void_p(stream)))
+    return words
 
 
 def _read_in_place(whole: tuple[torch.Tensor, ...], real: tuple[torch.Tensor, ...]) -> bool:

@@ -526,6 +526,33 @@ int gd_pack_weapon(const gd_weapon_desc *weapon, void *stream);
 int gd_pack_weapon_narrow(const gd_weapon_desc *weapon, uint32_t narrow, void *stream);
 
 /*
+ * The nine hud_state words of every lane (gd_lanes_desc.hud_state) from the gameplay tensors: what _native_render_hud reads with
+ * int(tensor.item()) per lane (engine.py:15240-15262) and the face of _native_mugshot_patch_index (engine.py:15209-15230).  Fields are the
+ * engine's attributes of the same names, device arrays of lane_count entries; ammo_slot is weapon_ammo_slot[active_weapon].  Where bit k of
+ * `narrow` is set, the k-th of the five counters (mugshot_face_index, mugshot_grin_tics, mugshot_pain_tics, mugshot_pain_direction,
+ * attack_held_tics) points to int32_t.  Returns GD_E_ARG for a null pointer or a count out of range.
+ */
+typedef struct gd_hud_desc {
+    uint32_t struct_size;    /* sizeof(gd_hud_desc) of the header the caller was built with */
+    int32_t lane_count, weapon_columns, ammo_columns, narrow;
+    const int64_t *ammo_slot;
+    const float *hud_ready_ammo;
+    const float *health;
+    const float *armor;
+    const float *weapons;  /* [N,weapon_columns], at least six */
+    const float *hud_ammo_counts;  /* [N,ammo_columns], at least four */
+    const int64_t *mugshot_face_index;
+    const int64_t *mugshot_grin_tics;
+    const int64_t *mugshot_pain_tics;
+    const int64_t *mugshot_pain_direction;
+    const int64_t *attack_held_tics;
+    const uint8_t *mugshot_ouch;  /* bool */
+    int32_t *hud_state;  /* [N,9] */
+} gd_hud_desc;
+
+int gd_pack_hud(const gd_hud_desc *hud, void *stream);
+
+/*
  * gd_pack_decals: gd_lanes_desc.decal_state [N,D,3] and decal_geom [N,D,4] from an engine's decal slots [N,D] (engine.py:13756-13829): the live
  * ones (serial >= 0) first and oldest first, then the free ones.  walls [wall_count,4] are the map's linedefs, fine_sine the 8192-entry
  * table in 16.16.

@@ -153,3 +153,28 @@ def test_weapon_words_are_read_as_wide_as_they_are_kept(narrow):
             words[name] = words[name].to(torch.int32)
     packed = overlay_inputs.weapon_state(**words, **tables, want_flash_light=True)
     assert torch.equal(packed[0], expected[0]) and torch.equal(packed[1], expected[1])
+
+
+@pytest.mark.parametrize("lanes", [1, 64, 65, 1000])
+@pytest.mark.parametrize("narrow", [0, 0b01010, 0b11111])
+def test_status_bar_words_are_packed_as_the_torch_expressions_pack_them(lanes, narrow):
+    from gradoom_amd import _abi, overlay_inputs
+
+    rng = torch.Generator(device="cuda:0").manual_seed(lanes)
+    whole = lambda low, high: torch.randint(low, high, (lanes,), generator=rng, device="cuda:0")  # noqa: E731
+    real = lambda *shape: torch.rand((lanes, *shape), generator=rng, device="cuda:0")  # noqa: E731
+    counters = {name: whole(-2, 3) for name in _abi.HUD_COUNTERS}
+    counters["attack_held_tics"] = whole(66, 74)
+    counters["mugshot_pain_direction"] = whole(0, 3)
+    for k, name in enumerate(_abi.HUD_COUNTERS):
+        if (narrow >> k) & 1:
+            counters[name] = counters[name].to(torch.int32)
+    reals = dict(hud_ready_ammo=real() * 500 - 50, health=real() * 260 - 40, armor=real() * 1200 - 100, weapons=(real(7) < 0.5).to(torch.float32), hud_ammo_counts=real(5) * 900 - 100)
+    for name in ("hud_ready_ammo", "health", "armor"):
+        reals[name][: lanes // 8] = torch.tensor([float("nan"), float("inf"), -float("inf"), 3e9, -3e9, 1e19, 999.5, -0.5], device="cuda:0")[torch.arange(lanes // 8) % 8]
+    fields = dict(active_weapon=whole(0, 8), weapon_ammo_slot=torch.tensor([-1, -1, 0, 1, 0, 3, 2, 1], device="cuda:0"), mugshot_ouch=real() < 0.5, **reals, **counters)
+    words = overlay_inputs.hud_state(**fields)
+    fields["health"] = spread(fields["health"])
+    assert lanes == 1 or overlay_inputs._hud_words_device(whole(0, 3), dict(reals, health=fields["health"]), counters, fields["mugshot_ouch"]) is None
+    expected = overlay_inputs.hud_state(**fields)
+    assert words.dtype == torch.int32 and words.is_contiguous() and torch.equal(words, expected)
