@@ -90,3 +90,41 @@ def test_chips_over_pixels_of_every_kind_match_the_oracle(oracle, where):
     assert renderer.status() == 0
     assert np.array_equal(indexed.cpu().numpy(), expected)
     renderer.close()
+
+
+@pytest.mark.parametrize("assembly", ["separate", "fused"])
+@pytest.mark.parametrize("patches", [None, 40, 1])
+def test_status_bars_of_every_kind_of_number_match_the_oracle(oracle, assembly, patches):
+    """Numbers of one to three digits and beyond, with and without a sign, faces that are no patches, offsets that move glyphs past the bar's edges,
+    and lists whose last patches do not exist."""
+    from gradoom_amd import hostmath, synthmap
+    from gradoom_amd.renderer import HipRenderer, LaneState
+
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    overlays = dict(synthmap.generate_overlays(33))
+    rng = np.random.default_rng(11)
+    for name, reach in (("hud_left", 12), ("hud_top", 20)):
+        overlays[name] = (overlays[name] + rng.integers(-reach, reach + 1, overlays[name].shape)).astype(overlays[name].dtype)
+    count = patches or len(overlays["hud_w"])
+    whole = dict(overlays, hud_w=overlays["hud_w"].copy())
+    whole["hud_w"][count:] = 0                       # what the oracle is given for the patches that the renderer's list ends before
+    overlays.update({name: overlays[name][:count] for name in overlays if name.startswith("hud_")})
+    numbers = np.array([0, 1, 9, 10, 99, 100, 999, 1000, -1, -9, -10, -99, -100, 2**31 - 1, -(2**31), 50, 300], dtype=np.int64)
+    lanes = 48
+    smap, tables, arrays = closed_door_case(301, lanes)
+    words = numbers[rng.integers(0, len(numbers), (lanes, 9))]
+    words[:, 3] = rng.integers(-2, count + 3, lanes)
+    words[:, 4] = rng.integers(0, 64, lanes)
+    arrays["hud_state"] = words.astype(np.int32)
+    oracle.set_overlays(whole)
+    expected = oracle.render(tables, arrays, cosine)["indexed"]
+    oracle.set_overlays(None)
+    assert len({bar.tobytes() for bar in expected[:, 208:]}) > (0 if patches == 1 else 20)
+    renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+    renderer.set_overlays(overlays)
+    renderer.set_assembly(assembly)
+    indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+    renderer.render(LaneState.from_numpy(arrays, "cuda:0"), indexed=indexed)
+    torch.cuda.synchronize()
+    assert np.array_equal(indexed.cpu().numpy(), expected)
+    renderer.close()
