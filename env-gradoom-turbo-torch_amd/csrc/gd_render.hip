@@ -1554,67 +1554,63 @@ __device__ __forceinline__ void note_row(const Scratch &sc, int local, int half,
     if (atomicMin(&span[0], y) == VH) sc.flat_spans[atomicAdd(sc.flat_span_count, 1)] = (local << 1) | half;
 }
 
-// GAP_WAVES wavefronts a column, which probe four rows each at a time: first the gap pixels', then the others' from the topmost
-// unresolved gap pixel down, until the lowest one is past and a resolved pixel below it is found (or the half ends).
-#define ROW_UNPROBED -2
+// GAP_WAVES wavefronts a column's half of the screen, which probe four rows each at a time, from the topmost gap pixel down, until the lowest one is
+// past and, if any is unresolved, a resolved pixel below the last of those is found (or the half ends).  The kernel lasts as long as
+// its slowest halves, rounds of probes one after the other.  Rows between gap pixels, and below them as far as the last round
+// reaches, are probed along with them, needed or not: 93 % of the halves hold an unresolved pixel, and the round lasts as long either way.
+// (Gap pixels first, then the rows between and below, the halves of a column one after the other: 42 us where this takes 24 at 256 lanes of 800
+// linedefs, 83 and 65 at 512 lanes of 4000.)
 template <int GAP_WAVES>
 __global__ void __launch_bounds__(64 * GAP_WAVES) flat_gap_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
     __shared__ ProbeLds probe_lds[GAP_WAVES];
-    __shared__ short row_sector[VH];                  // the sector of each row's pixel, -1 unresolved, ROW_UNPROBED
-    __shared__ int unresolved_first, unresolved_last;
+    __shared__ short row_sector[VH];                  // the sector of each row's pixel, -1 unresolved
+    __shared__ int unresolved_first, unresolved_last, resolved_last;
     const int total = *sc.gap_column_count;
     const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63, group = wave * PROBE_GROUPS + lane_id / PROBE_LANES;
     const bool speaks = (lane_id & (PROBE_LANES - 1)) == 0;
     constexpr int ROWS = GAP_WAVES * PROBE_GROUPS;
-    for (int entry = blockIdx.x; entry < total; entry += gridDim.x) {
-        const int2 packed = sc.gap_columns[entry];
-        const int x = packed.x & 511, local = packed.x >> 9;
+    for (int task = blockIdx.x; task < 2 * total; task += gridDim.x) {
+        const int2 packed = sc.gap_columns[task >> 1];
+        const int half = task & 1, x = packed.x & 511, local = packed.x >> 9;
         const LaneCtx &c = sc.ctx[local];
         const int n = lane_base + local, last_ceiling_row = c.last_ceiling_row;
+        const int half_end = half ? VH - 1 : last_ceiling_row;
+        const int lo = max(packed.y & 255, half ? last_ceiling_row + 1 : 0), hi = min((packed.y >> 8) - 1, half_end);
+        if (lo > hi) continue;                        // the same in the whole block, like everything that steers it here
         const unsigned int *meta = sc.meta + (size_t)local * VH * SW + x;
         unsigned short *sector = sc.flat_sector + (size_t)local * VH * SW + x;
         unsigned char *flags = sc.flat_flags + (size_t)local * VH * SW + x;
-        for (int half = 0; half < 2; ++half) {
-            const int half_end = half ? VH - 1 : last_ceiling_row;
-            const int lo = max(packed.y & 255, half ? last_ceiling_row + 1 : 0), hi = min((packed.y >> 8) - 1, half_end);
-            if (lo > hi) continue;                    // the same in the whole block, like everything that steers it here
-            __syncthreads();                          // nobody reads the previous column's rows any more
-            if (threadIdx.x == 0) { unresolved_first = VH; unresolved_last = -1; }
-            __syncthreads();
-            for (int y0 = lo; y0 <= hi; y0 += ROWS) {
-                const int y = y0 + group;
-                const bool shown = y <= hi && gap_pixel(meta[(size_t)y * SW]);
-                const int s = flat_probe_group(dm, sc, lanes, local, n, x, y <= hi ? y : lo, shown, &probe_lds[wave]);
-                if (y > hi || !speaks) continue;
-                row_sector[y] = shown ? (short)s : (short)ROW_UNPROBED;
-                if (!shown) continue;
-                sector[(size_t)y * SW] = (unsigned short)(s < 0 ? c.sector : s);
-                flags[(size_t)y * SW] = s < 0 ? 1 : 0;
-                if (s < 0) { atomicMin(&unresolved_first, y); atomicMax(&unresolved_last, y); }
-            }
-            __syncthreads();
-            const int first = unresolved_first, last = unresolved_last;
-            if (last < 0) continue;
-            int rows_end = hi + 1;                    // rows below it are known or were found not to matter
-            for (int y0 = first + 1; y0 <= half_end; y0 += ROWS) {
-                const int y = y0 + group;
-                const bool live = y <= half_end && (y > hi || row_sector[y] == ROW_UNPROBED);
-                const int s = flat_probe_group(dm, sc, lanes, local, n, x, y <= half_end ? y : lo, live, &probe_lds[wave]);
-                if (live && speaks) row_sector[y] = (short)s;
-                rows_end = max(rows_end, min(y0 + ROWS, half_end + 1));
-                if (__syncthreads_or(y <= half_end && y > last && (live ? s : (int)row_sector[y]) >= 0)) break;
-            }
-            __syncthreads();
-            for (int y = first + (int)threadIdx.x; y <= last; y += blockDim.x) {
-                if (row_sector[y] != -1 || !gap_pixel(meta[(size_t)y * SW])) continue;
-                int below = -1;
-                for (int j = y + 1; j < rows_end && below < 0; ++j) below = row_sector[j];
-                if (below >= 0 && below != c.sector) {
-                    sector[(size_t)y * SW] = (unsigned short)below;
-                    flags[(size_t)y * SW] = (unsigned char)(1 | 2 | 4 | 8);
-                } else {
-                    note_row(sc, local, half, y);
+        __syncthreads();                              // nobody reads the previous half's rows any more
+        if (threadIdx.x == 0) { unresolved_first = VH; unresolved_last = -1; resolved_last = -1; }
+        int rows_end = lo;
+        for (bool more = true; more && rows_end <= half_end;) {
+            __syncthreads();                          // the bounds are set, and everyone has seen the last round's
+            const int y = rows_end + group;
+            const bool live = y <= half_end, shown = y <= hi && gap_pixel(meta[(size_t)y * SW]);
+            const int s = flat_probe_group(dm, sc, lanes, local, n, x, live ? y : lo, live, &probe_lds[wave]);
+            if (live && speaks) {
+                row_sector[y] = (short)s;
+                if (s >= 0) atomicMax(&resolved_last, y);
+                if (shown) {
+                    sector[(size_t)y * SW] = (unsigned short)(s < 0 ? c.sector : s);
+                    flags[(size_t)y * SW] = s < 0 ? 1 : 0;
+                    if (s < 0) { atomicMin(&unresolved_first, y); atomicMax(&unresolved_last, y); }
                 }
+            }
+            rows_end += ROWS;
+            __syncthreads();
+            more = rows_end <= hi || (unresolved_last >= 0 && resolved_last < unresolved_last);
+        }
+        rows_end = min(rows_end, half_end + 1);
+        for (int y = unresolved_first + (int)threadIdx.x; y <= unresolved_last; y += blockDim.x) {
+            if (row_sector[y] != -1 || !gap_pixel(meta[(size_t)y * SW])) continue;
+            int below = -1;
+            for (int j = y + 1; j < rows_end && below < 0; ++j) below = row_sector[j];
+            if (below >= 0 && below != c.sector) {
+                sector[(size_t)y * SW] = (unsigned short)below;
+                flags[(size_t)y * SW] = (unsigned char)(1 | 2 | 4 | 8);
+            } else {
+                note_row(sc, local, half, y);
             }
         }
     }
@@ -6055,8 +6051,9 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     auto flat_grid = [count](int per_lane, int most) { return dim3((unsigned)(count >= most / per_lane ? most : (count * per_lane < 32 ? 32 : count * per_lane))); };
     const int plane_levels = m.floor_level_count + m.ceil_level_count;
     const bool level_masks = plane_levels > LEVEL_MASK_MIN_LEVELS && plane_levels <= 32 * LEVEL_MASK_WORDS_MAX;   // level_mask_words() > 0
-    if (gap_waves(count) == 16) hipLaunchKernelGGL(flat_gap_kernel<16>, flat_grid(4, 1024), dim3(64 * 16), 0, stream, r->dm, *lanes, base, sc);
-    else hipLaunchKernelGGL(flat_gap_kernel<8>, flat_grid(4, 2048), dim3(64 * 8), 0, stream, r->dm, *lanes, base, sc);
+    const int waves = gap_waves(count);
+    hipLaunchKernelGGL(waves == 16 ? flat_gap_kernel<16> : (waves == 8 ? flat_gap_kernel<8> : flat_gap_kernel<4>), flat_grid(8, 16384 / waves), dim3(64 * waves), 0, stream,
+                       r->dm, *lanes, base, sc);
     hipLaunchKernelGGL(flat_rows_kernel, dim3(count), dim3(64), 0, stream, count, sc);
     hipLaunchKernelGGL(level_masks ? flat_span_select_kernel<true> : flat_span_select_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, sc);
     mark();

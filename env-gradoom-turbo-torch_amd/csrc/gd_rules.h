@@ -80,11 +80,17 @@ inline int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
 // issue 1.5 % fewer instructions and take as long: 686, 905, 1239, 975.)
 inline int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 2400 ? 2 : 1)); }
 
-// flat_gap_kernel: wavefronts a column.  The fewer the lanes, the fewer such columns and the longer the kernel lasts as its slowest one.  us
-// with 4 / 8 / 16 wavefronts a column: 512 lanes 95 / 71 / 62, 1024 lanes (2000 linedefs) 100 / 64 / 52, 4096 lanes 118 / 115 / 141; the whole
-// selection at 2048 lanes of 800, 2000 and 4000 linedefs 164 / 153 / 161, 179 / 144 / 152, 253 / 221 / 230, at 1024 lanes 136 / 111 / 111,
-// 146 / 112 / 97, 193 / 160 / 146.
-inline int gap_waves(int lanes) { return lanes <= 1536 ? 16 : 8; }
+// flat_gap_kernel: wavefronts a half of a column.  The fewer the lanes, the fewer such halves and the longer the kernel lasts as its slowest one; the
+// more, the longer a large work-group waits for room beside the shading.  A frame in us with 2 / 4 / 8 / 16 wavefronts (32 billboards, two
+// sets of poses; in brackets with a column's halves one after the other, 16 wavefronts up to 1536 lanes, 8 beyond):
+//   lanes        320 linedefs                    2000                            4000                          1400, 13 plane levels
+//    256   484 / 464 / 451 / 445 (464)   570 / 542 / 524 / 514 (542)     801 / 757 / 739 / 723 (746)      500 / 479 / 476 / 486 (495)
+//    512   570 / 562 / 554 / 555 (560)   713 / 692 / 670 / 682 (682)    1142 /1103 /1089 /1076 (1098)     690 / 670 / 689 / 716 (728)
+//    768   707 / 700 / 700 / 701 (705)   861 / 844 / 834 / 857 (842)    1370 /1340 /1316 /1351 (1322)     904 / 888 / 942 / 959 (968)
+//   1024   802 / 798 / 798 / 803 (815)  1025 /1004 /1010 /1026 (1031)   1532 /1520 /1491 /1531 (1512)    1049 /1061 /1125 /1144 (1172)
+//   2048  1260 /1260 /1266 /1285 (1278) 1624 /1632 /1639 /1696 (1659)   2347 /2338 /2346 /2404 (2371)    1721 /1737 /1833 /1888 (1870)
+//   4096  2188 /2199 /2201 /2241 (2248) 2864 /2881 /2939 /2955 (2965)   3851 /3856 /3922 /3985 (3870)    3001 /2995 /3166 /3264 (3205)
+inline int gap_waves(int lanes) { return lanes <= 384 ? 16 : (lanes <= 896 ? 8 : 4); }
 
 // sprite_pixels_kernel: work-groups that share the rows of a block of columns.  From 512 lanes on one takes them all: fewer listings, but the
 // last work-groups last longer.  Quarters and whole columns cost the same at 230 (4000 linedefs, 128 billboards) to 1100 lanes (320 linedefs,
