@@ -59,12 +59,12 @@ typedef unsigned long long u64;
 #define VH 208
 #define CAND_MAX 64          // candidate linedefs a screen column keeps in its own slots
 // A column whose ray can reach more than CAND_MAX linedefs (a long corridor seen end on) gets a slot in the chunk's spill
-// pool, where strip_order_kernel lists all of them, up to SPILL_OBS_AHEAD.  The pool continues the candidate blocks with
-// the same layout (entry k of a column lies k * 320 entries on), SPILL_OBS_AHEAD x 320 entries per pool block, so a
+// pool, where strip_order_kernel lists all of them, up to SPILL_DEPTH.  The pool continues the candidate blocks with
+// the same layout (entry k of a column lies k * 320 entries on), SPILL_DEPTH x 320 entries per pool block, so a
 // spilled column differs from the others only in where its list starts and how long it may be.
-#define SPILL_OBS_AHEAD 256
+#define SPILL_DEPTH 256
 #define SPILL_SHIFT 12       // cand_count of a spilled column: entries | (pool slot + 1) << SPILL_SHIFT
-static_assert(SPILL_OBS_AHEAD < (1 << SPILL_SHIFT), "a spilled column's count and its pool slot share a word");
+static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and its pool slot share a word");
 #define SEG_COLS 64           // columns of a traversal segment; a wavefront takes 64 / SEG_COLS segments, of any lanes
 #define SEGS_PER_LANE (SW / SEG_COLS)
 #define GD_INF __builtin_inff()
@@ -79,7 +79,7 @@ static_assert(SPILL_OBS_AHEAD < (1 << SPILL_SHIFT), "a spilled column's count an
 #define FOCAL_Y_FIXED (160LL * Y_ASPECT_FIXED)
 #define FLOOR_VISIBILITY_FIXED ((160LL * 65536LL * (8LL * 65536LL)) / FOCAL_Y_FIXED)
 #define WALL_VISIBILITY_FIXED (((FOCAL_Y_FIXED * (320LL * 600LL) / (320LL * 240LL * 3LL)) * (8LL * 65536LL)) >> 16)
-#define SPRITE_MIN_OBS_AHEAD_FIXED 8192LL
+#define SPRITE_MIN_DEPTH_FIXED 8192LL
 
 // candidate flags
 #define CF_GEO 1
@@ -260,7 +260,7 @@ struct Scratch {    // per-chunk working memory, sized at create
     WallRec *frag_rec;     // [L,split_count,fragment_slots] FWallCoords of the BSP fragments of split linedefs
     float *scene_depth;    // [L,208,320] depth of the wall tier or masked texture a pixel shows (engine.py:11553, 12700, 13740),
                            // kept only for frames that draw wall decals, else null; scene_depth_at() has the others
-    Cand *cand;            // [L,CAND_MAX,320], then the spill pool [spill_slots / 320, SPILL_OBS_AHEAD, 320]
+    Cand *cand;            // [L,CAND_MAX,320], then the spill pool [spill_slots / 320, SPILL_DEPTH, 320]
     int *cand_count;       // [L,320] entries listed (beyond CAND_MAX: the column wanted more than its own slots hold), or for
                            // a column with a pool slot: entries in the pool | (slot + 1) << SPILL_SHIFT
     int *spill_columns;    // [spill_slots] the columns (lane * 320 + column) that were given pool slots, in slot order
@@ -1084,7 +1084,7 @@ __device__ __forceinline__ void list_spilled_columns(const DeviceMap &dm, const 
         const LaneCtx &c = sc.ctx[local];
         float rx, ry; ray_direction(c, x, &rx, &ry);
         const RecSpan *spans = sc.span + (size_t)local * walls;
-        Cand *list = sc.cand + sc.spill_base + ((size_t)(slot / SW) * SPILL_OBS_AHEAD * SW + (size_t)(slot % SW));
+        Cand *list = sc.cand + sc.spill_base + ((size_t)(slot / SW) * SPILL_DEPTH * SW + (size_t)(slot % SW));
         int listed = 0;
         for (int w0 = 0; w0 < walls; w0 += 64) {
             const int w = w0 + lane_id;
@@ -1103,12 +1103,12 @@ __device__ __forceinline__ void list_spilled_columns(const DeviceMap &dm, const 
             const u64 keeps = __ballot(keep);
             const int position = listed + __popcll(keeps & ((1ULL << lane_id) - 1ULL));
             if (keep) {
-                if (position < SPILL_OBS_AHEAD) list[(size_t)position * SW] = entry;
+                if (position < SPILL_DEPTH) list[(size_t)position * SW] = entry;
                 else sc.status[STATUS_CAND_OVERFLOW] = 1;
             }
             listed += __popcll(keeps);
         }
-        if (lane_id == 0) sc.cand_count[column] = (listed < SPILL_OBS_AHEAD ? listed : SPILL_OBS_AHEAD) | ((slot + 1) << SPILL_SHIFT);
+        if (lane_id == 0) sc.cand_count[column] = (listed < SPILL_DEPTH ? listed : SPILL_DEPTH) | ((slot + 1) << SPILL_SHIFT);
     }
 }
 
@@ -1984,7 +1984,7 @@ struct ColumnCtx {
         const unsigned spill = (unsigned)listed >> SPILL_SHIFT;
         if (spill) {
             const unsigned slot = spill - 1;
-            list_column = (sc.spill_base + (slot / SW) * (unsigned)(SPILL_OBS_AHEAD * SW) + slot % SW) * 16u;
+            list_column = (sc.spill_base + (slot / SW) * (unsigned)(SPILL_DEPTH * SW) + slot % SW) * 16u;
             count = listed & ((1 << SPILL_SHIFT) - 1);
         } else {
             list_column = ((unsigned)local * (CAND_MAX * SW) + (unsigned)column) * 16u;
@@ -2866,7 +2866,7 @@ __device__ __forceinline__ void zero_rows(Pixels &pb, GapRange &gaps, int x, int
 // rows that its own clip update then removes from the window, so the window stays untouched
 // until a one-sided drawseg (which leaves the clips alone) has painted; until then painting
 // needs no reads and visits only the rows it writes.
-template <bool OBS_AHEAD, typename Pixels>
+template <bool DEPTH, typename Pixels>
 __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnState &c, const PassDraw &d, const PassRows &r, Pixels &pb,
                            const bool group_valid[3], const float group_bottom[3], const unsigned char *colormap, bool &window_dirty, GapRange &gaps) {
     // The whole wavefront comes here together, columns with nothing to draw as well: they take part in the walks over the rows.
@@ -2988,7 +2988,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
 #pragma unroll
                     for (int j = 0; j < WALL_ROWS; ++j) {
                         const bool own = (unsigned)(y + j * stride - first) < rows;
-                        if (OBS_AHEAD) pb.put_depth(own, yb + j * stride, d.distance);
+                        if (DEPTH) pb.put_depth(own, yb + j * stride, d.distance);
                         pb.put(own, yb + j * stride, meta_word | (colour[j] << META_SECTOR_SHIFT));
                     }
 #pragma unroll
@@ -3032,7 +3032,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 for (int j = 0; j < WALL_ROWS; ++j) {
                     if (!(draw & (1u << j))) continue;
                     const unsigned colour = ((tail & (1u << j)) ? group_shades : own_shades)[texel[j]];
-                    if (OBS_AHEAD) pb.s(yb + j) = d.distance;
+                    if (DEPTH) pb.s(yb + j) = d.distance;
                     pb.m(yb + j) = META_FILLED | (colour << META_SECTOR_SHIFT) | (unsigned)(wi + 1);
                 }
 #pragma unroll
@@ -3085,7 +3085,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 const unsigned tv = (fraction >> (tier_a ? shift_a : shift_b)) >> 1;
                 unsigned char texel = m->tex_atlas[(tier_a ? d.column_a : d.column_b) + __umul24(tv, atlas_w)];
                 const unsigned colour = (bottom_tail ? group_shades : own_shades)[texel];
-                if (OBS_AHEAD) pb.s(y) = d.distance;
+                if (DEPTH) pb.s(y) = d.distance;
                 const float held = (meta & META_WALL_MASK) ? clip_distance(cc, (int)(meta & META_WALL_MASK) - 1) : GD_INF;   // no clip recorded yet
                 if (d.distance < held) { meta = (meta & ~META_WALL_MASK) | (unsigned)(wi + 1); }
                 meta = (meta & ~(META_SECTOR_MASK << META_SECTOR_SHIFT)) | (colour << META_SECTOR_SHIFT) | META_FILLED;
@@ -3283,7 +3283,7 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, const ListShar
 }
 
 // engine.py:13424-13744 for one column
-template <bool OBS_AHEAD, bool GENERAL, typename Pixels>
+template <bool DEPTH, bool GENERAL, typename Pixels>
 __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, int local, const ColumnState &c, Pixels &pb, const unsigned char *colormap) {
     const gd_map_desc *m = cc.m;
     const LaneCtx &L = *cc.c;
@@ -3378,7 +3378,7 @@ __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const Col
             if (pb.frame) pb.f(y) = colour;
             else pb.t(y) = colour;
             pb.m(y) = word[j] | META_MASKED;
-            if (OBS_AHEAD) pb.s(y) = md;
+            if (DEPTH) pb.s(y) = md;
         }
     }
 }
@@ -3782,7 +3782,7 @@ __device__ __forceinline__ PassDraw hand_round(const PassDraw &prepared, int k, 
     d.distance = __uint_as_float(take(__float_as_uint(prepared.distance)));
     return d;
 }
-// OBS_AHEAD: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
+// DEPTH: also keep the depth of every wall pixel (frames that draw decals).  GENERAL: the map has linedefs with
 // BSP projection fragments, or more sectors or textures than the LDS tables hold (a table that may be in either place is read
 // behind a branch, and behind a branch with a load in it a wavefront waits for every store it has under way).
 // 4096 lanes on the 4000-linedef map: 1.78 -> 1.00 ms: the linedefs' lines 1.53, no sprite clip plane
@@ -3791,7 +3791,7 @@ __device__ __forceinline__ PassDraw hand_round(const PassDraw &prepared, int k, 
 // rows: 16 lanes on the 2000-linedef map 97 -> 53 us, 512 on the 4000-linedef map 443 -> 350, 1024 on the 320-linedef map 286 -> 226 (rows alone
 // 71, 426, 252).  The passes are handed round from register to register: through LDS there are no spills, but the 1024 lanes take 268.  Working
 // out the textures of visible tiers only makes the 1024 lanes 241, and 4096 1.11 ms.
-template <bool OBS_AHEAD, bool GENERAL, int PARTS>
+template <bool DEPTH, bool GENERAL, int PARTS>
 __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(RASTER_WAVES, RASTER_WAVES))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
     __shared__ LaneCtx lane_ctxs[WALL_STRIPS_PER_GROUP][64 / SEG_COLS];
@@ -3830,10 +3830,10 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     PixelBuffers<PARTS> pb;
     pb.frame = frame_base;
     pb.meta = sc.meta; pb.masked_texel = sc.masked_texel;
-    pb.scene_depth = OBS_AHEAD ? sc.scene_depth : nullptr;
+    pb.scene_depth = DEPTH ? sc.scene_depth : nullptr;
     pb.word_column = ((unsigned)local * (VH * SW) + (unsigned)x) * 4u;
     pb.words = __builtin_amdgcn_make_buffer_rsrc(sc.meta, 0, lane_count * (VH * SW * 4), BUFFER_WORDS);
-    pb.depths = __builtin_amdgcn_make_buffer_rsrc(pb.scene_depth, 0, OBS_AHEAD ? lane_count * (VH * SW * 4) : 0, BUFFER_WORDS);
+    pb.depths = __builtin_amdgcn_make_buffer_rsrc(pb.scene_depth, 0, DEPTH ? lane_count * (VH * SW * 4) : 0, BUFFER_WORDS);
     pb.frame_column = (unsigned)local * (unsigned)frame_stride + (unsigned)x;
     pb.row_lane = PARTS == 1 ? 0 : lane_id / part_cols;
     pb.put_column = pb.word_column + (unsigned)pb.row_lane * (SW * 4u);
@@ -3899,13 +3899,13 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
             group_valid[0] = same_group && (agreed & 1) && (shared_top < shared_bottom);
             group_valid[1] = same_group && (agreed & 2) && (shared_lower_top < shared_bottom);
             group_valid[2] = same_group && (agreed & 4) && (shared_top < shared_upper_bottom);
-            pass_paint<OBS_AHEAD>(cc, st, d, rows, pb, group_valid, common_bottom, colormap_lds, window_dirty, gaps);
+            pass_paint<DEPTH>(cc, st, d, rows, pb, group_valid, common_bottom, colormap_lds, window_dirty, gaps);
             if (d.flags & (DRAW_RASTER | DRAW_PS_KEEPS)) advance_clips(cc, st, d, rows, pb, sb, !window_dirty, gaps, sc, first_record + (size_t)(group + k) * pass_stride);
         }
     }
     // what is left of a window no one-sided drawseg closed shows the flat pass's picture
     if (!window_dirty) zero_rows(pb, gaps, x, st.ceiling_clip <= 0.0f ? 0 : (int)st.ceiling_clip, st.floor_clip >= (float)VH ? VH : (int)st.floor_clip);
-    if (dm.masked_count > 0) masked_midtexture<OBS_AHEAD, GENERAL>(dm, cc, sc, local, st, pb, colormap_lds);
+    if (dm.masked_count > 0) masked_midtexture<DEPTH, GENERAL>(dm, cc, sc, local, st, pb, colormap_lds);
     // The columns with view pixels that no wall tier, plane or masked texture covers join the flat pass's work list, those of a
     // wavefront in one piece (flat_gap_kernel selects the pixels, flat_shade_kernel paints them).
     bool holds_gap = false;
@@ -4094,7 +4094,7 @@ __device__ __forceinline__ bool sprite_record(const DeviceMap &dm, const gd_lane
     const i64 rx = ax - L.view_x_fixed, ry = ay - L.view_y_fixed;
     s.depth_fixed = (rx * L.vcos + ry * L.vsin) >> 20;
     const i64 side_fixed = (rx * L.vsin - ry * L.vcos) >> 16;
-    const i64 xscale = tdiv(FOCAL_X_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_OBS_AHEAD_FIXED));
+    const i64 xscale = tdiv(FOCAL_X_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
     const i64 left_fixed = side_fixed - (i64)m->spr_left[id] * FIXED_UNIT;
     s.width = m->spr_w[id];
     s.left = SW / 2 + (mul64(left_fixed, xscale) >> 32);
@@ -4103,7 +4103,7 @@ __device__ __forceinline__ bool sprite_record(const DeviceMap &dm, const gd_lane
     if (!(s.right > x_first && s.left < x_end && s.right > s.left)) return false;
     s.height = m->spr_h[id];
     s.hstep = tdiv((i64)s.width << 16, max64(s.right - s.left, 1));
-    s.yscale = tdiv(FOCAL_Y_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_OBS_AHEAD_FIXED));
+    s.yscale = tdiv(FOCAL_Y_FIXED << 12, max64(s.depth_fixed, SPRITE_MIN_DEPTH_FIXED));
     const i64 texmid = (i64)m->spr_top[id] * FIXED_UNIT - round_to_i64((L.view_z - z) * 65536.0f);
     s.top_fixed = L.center_fixed - (mul64(texmid, s.yscale) >> 16);
     s.iscale = tdiv(UINT32_MASK, max64(s.yscale, 1));
@@ -5759,7 +5759,7 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.masked_geo, L * (size_t)masked_count);
     take(&sc.masked_hit, L * SW);
     take(&sc.frag_rec, L * (size_t)(h.split_count > 0 ? h.split_count * h.fragment_slots : 1));
-    take(&sc.cand, L * CAND_MAX * SW + spill_blocks * SPILL_OBS_AHEAD * SW);   // byte offsets into it are 32 bits wide: L <= 4096, spill_blocks <= 512
+    take(&sc.cand, L * CAND_MAX * SW + spill_blocks * SPILL_DEPTH * SW);   // byte offsets into it are 32 bits wide: L <= 4096, spill_blocks <= 512
     sc.spill_base = (unsigned)(L * CAND_MAX * SW); sc.spill_slots = (int)(spill_blocks * SW);
     take(&sc.cand_count, L * SW);
     take(&sc.spill_columns, spill_blocks * SW);
