@@ -1879,79 +1879,130 @@ __global__ void __launch_bounds__(64 * TAIL_ROWS) flat_tail_kernel(DeviceMap dm,
     }
 }
 
-// The repairs of one half of a lane's screen, one thread per column, one block per entry of the work list.
-__global__ void __launch_bounds__(SW) flat_span_finish_kernel(Scratch sc) {
-    __shared__ u64 anchors[VH][SW / 64];              // per noted row and 64 columns: the pixels that are anchors
-    const int x = threadIdx.x, wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63;
+// The repairs of one half of a lane's screen, a work-group per entry of the work list.  The kernel lasts as long as its tallest ranges, whose rows
+// depend on each other from the lowest up; so a band of rows is read at once, four columns of FINISH_ROWS rows a thread, and what the
+// rows below found travels through LDS in one step.  The rows wait in LDS and not in registers so that only the loads are unrolled: a
+// work-group runs through its code once, and what it waits for most is the code.  (A thread a column, eight rows at a time with stores between the
+// loads: 62 us for 94 rows of one of 16 lanes, 79 us for 4096 lanes; rows in registers, all loops unrolled, 20 and 40 us; now 14 and 25.)
+#define FINISH_QUADS (SW / 4)
+#define FINISH_CHUNKS 12          // threads that share four columns
+#define FINISH_ROWS 9             // rows a thread takes: a band of 108 rows, the half of a level view
+#define FINISH_THREADS (FINISH_QUADS * FINISH_CHUNKS)
+#define FINISH_BAND (FINISH_CHUNKS * FINISH_ROWS)
+#define FINISH_NONE 0xFFFFu       // no resolved pixel (sectors are below 8191)
+__global__ void __launch_bounds__(FINISH_THREADS) flat_span_finish_kernel(Scratch sc) {
+    __shared__ uint2 row_sectors[FINISH_ROWS][FINISH_THREADS];
+    __shared__ unsigned int row_flags[FINISH_ROWS][FINISH_THREADS];
+    __shared__ uint2 topmost[FINISH_CHUNKS][FINISH_QUADS];   // the sectors of four columns' topmost resolved pixels in a thread's rows
+    __shared__ unsigned int anchors[FINISH_BAND][SW / 32];   // per row of the band, a bit a column: the pixels that are anchors
+    __shared__ unsigned int open[FINISH_BAND][SW / 32];      // likewise: shown, unresolved and no anchors
+    const int chunk = threadIdx.x / FINISH_QUADS, quad = threadIdx.x - chunk * FINISH_QUADS, x0 = quad * 4;
     const int total = *sc.flat_span_count;
+    auto sector_of = [](const uint2 &four, int k) { return ((k < 2 ? four.x : four.y) >> (16 * (k & 1))) & 0xFFFFu; };
     for (int entry = blockIdx.x; entry < total; entry += gridDim.x) {
         const int packed = sc.flat_spans[entry], local = packed >> 1, half = packed & 1;
         const int lo = sc.flat_span[(size_t)local * 4 + 2 * half], hi = sc.flat_span[(size_t)local * 4 + 2 * half + 1];
-        const int camera_sector = sc.ctx[local].sector;
+        const unsigned camera_sector = (unsigned)sc.ctx[local].sector;
         unsigned short *sector = sc.flat_sector + (size_t)local * VH * SW;
         unsigned char *flags = sc.flat_flags + (size_t)local * VH * SW;
         const unsigned int *meta = sc.meta + (size_t)local * VH * SW;
-        __syncthreads();                              // nobody reads the previous entry's anchors any more
-        // --- vertical (engine.py:11026-11083): floors and ceilings alike look downwards, within their own half
-        {
-            // what flat_tail_kernel found below the range for a column whose pixel in the range's last row is unresolved
-            const int below = sc.flat_tail[((size_t)local * 2 + half) * SW + x];
-            bool found = below >= 0;
-            int span_sector = found ? below : 0;
-            // eight rows at a time, their loads first: a column's rows are its own, so no store of the loop touches them
-            for (int y0 = hi; y0 >= lo; y0 -= 8) {
-                unsigned char row_flags[8]; unsigned short row_sector[8];
+        // what flat_tail_kernel found below the range for a column whose pixel in the range's last row is unresolved
+        const int4 tail = *reinterpret_cast<const int4 *>(sc.flat_tail + ((size_t)local * 2 + half) * SW + x0);
+        unsigned below[4] = {(unsigned)tail.x & 0xFFFFu, (unsigned)tail.y & 0xFFFFu, (unsigned)tail.z & 0xFFFFu, (unsigned)tail.w & 0xFFFFu};
+        for (int band_hi = hi; band_hi >= lo; band_hi -= FINISH_BAND) {
+            const int rows = min(band_hi - lo + 1, FINISH_BAND), band_lo = band_hi - rows + 1;
+            const int each = (rows + FINISH_CHUNKS - 1) / FINISH_CHUNKS, first = band_hi - chunk * each;   // a thread's rows, the lowest first
+            const int own = max(min(each, first - band_lo + 1), 0);
+            unsigned int flags_read[FINISH_ROWS]; uint2 sectors_read[FINISH_ROWS]; uint4 words[FINISH_ROWS];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int y = y0 - j < lo ? lo : y0 - j;
-                    row_flags[j] = flags[(size_t)y * SW + x]; row_sector[j] = sector[(size_t)y * SW + x];
+            for (int j = 0; j < FINISH_ROWS; ++j) {   // rows past the thread's own are read again and left out below
+                const size_t i = (size_t)max(first - min(j, each - 1), band_lo) * SW + x0;
+                flags_read[j] = *reinterpret_cast<const unsigned int *>(flags + i);
+                sectors_read[j] = *reinterpret_cast<const uint2 *>(sector + i);
+                words[j] = *reinterpret_cast<const uint4 *>(meta + i);
+            }
+            __syncthreads();                          // nobody reads the previous band's anchors and topmost pixels any more
+            u64 shown = 0;                            // a bit a pixel: does it show the flat pass's picture?
+#pragma unroll
+            for (int j = 0; j < FINISH_ROWS; ++j) {
+                row_flags[j][threadIdx.x] = flags_read[j]; row_sectors[j][threadIdx.x] = sectors_read[j];
+                const unsigned gap = (gap_pixel(words[j].x) ? 1u : 0u) | (gap_pixel(words[j].y) ? 2u : 0u) | (gap_pixel(words[j].z) ? 4u : 0u) | (gap_pixel(words[j].w) ? 8u : 0u);
+                shown |= (u64)gap << (4 * j);
+            }
+            for (int k = threadIdx.x; k < rows * (SW / 32); k += FINISH_THREADS) { (&anchors[0][0])[k] = 0u; (&open[0][0])[k] = 0u; }
+            unsigned span_sector[4] = {FINISH_NONE, FINISH_NONE, FINISH_NONE, FINISH_NONE};
+#pragma unroll 1
+            for (int j = 0; j < own; ++j) {
+                const unsigned int four = row_flags[j][threadIdx.x];
+                const uint2 sectors = row_sectors[j][threadIdx.x];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) span_sector[k] = (four >> (8 * k)) & 1u ? span_sector[k] : sector_of(sectors, k);
+            }
+            topmost[chunk][quad] = make_uint2(span_sector[0] | (span_sector[1] << 16), span_sector[2] | (span_sector[3] << 16));
+            __syncthreads();
+            // --- vertical (engine.py:11026-11083): floors and ceilings alike look downwards, within their own half
+#pragma unroll 1
+            for (int c = 0; c < FINISH_CHUNKS; ++c) {
+                const uint2 four = topmost[c][quad];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    span_sector[k] = c <= chunk ? below[k] : span_sector[k];   // what lies below the thread's own rows
+                    below[k] = sector_of(four, k) != FINISH_NONE ? sector_of(four, k) : below[k];
                 }
+            }
+#pragma unroll 1
+            for (int j = 0; j < own; ++j) {
+                const unsigned int four = row_flags[j][threadIdx.x];
+                const uint2 sectors = row_sectors[j][threadIdx.x];
+                unsigned int anchor = 0u, new_flags = four, pair[2] = {sectors.x, sectors.y};
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int y = y0 - j;
-                    if (y < lo) break;
-                    const size_t i = (size_t)y * SW + x;
-                    const bool resolved = !(row_flags[j] & 1);
-                    if (resolved) { found = true; span_sector = row_sector[j]; }
-                    const bool anchor = resolved || (found && span_sector != camera_sector);
+                for (int k = 0; k < 4; ++k) {
+                    const bool resolved = !((four >> (8 * k)) & 1u);
+                    if (resolved) span_sector[k] = sector_of(sectors, k);
+                    const bool found = span_sector[k] != FINISH_NONE, anchors_here = resolved || (found && span_sector[k] != camera_sector);
                     if (!resolved && found) {
-                        sector[i] = (unsigned short)span_sector;
+                        pair[k >> 1] = (pair[k >> 1] & ~(0xFFFFu << (16 * (k & 1)))) | (span_sector[k] << (16 * (k & 1)));
                         // bit1: vertical span; bit2: its sector differs from the camera's (anchor)
-                        flags[i] = (unsigned char)(1 | 2 | (anchor ? 4 : 0));
+                        new_flags |= (2u | (anchors_here ? 4u : 0u)) << (8 * k);
                     }
-                    const u64 row_anchors = __ballot(anchor);
-                    if (lane_id == 0) anchors[y][wave] = row_anchors;
+                    anchor |= anchors_here ? 1u << k : 0u;
                 }
+                if (new_flags != four) {
+                    const size_t i = (size_t)(first - j) * SW + x0;
+                    *reinterpret_cast<unsigned int *>(flags + i) = new_flags;
+                    *reinterpret_cast<uint2 *>(sector + i) = make_uint2(pair[0], pair[1]);
+                    row_flags[j][threadIdx.x] = new_flags; row_sectors[j][threadIdx.x] = make_uint2(pair[0], pair[1]);
+                }
+                const unsigned int wants = ~anchor & (unsigned)(shown >> (4 * j)) & 15u;
+                if (anchor) atomicOr(&anchors[first - j - band_lo][quad >> 3], anchor << (4 * (quad & 7)));
+                if (wants) atomicOr(&open[first - j - band_lo][quad >> 3], wants << (4 * (quad & 7)));
             }
-        }
-        __syncthreads();
-        // --- horizontal (engine.py:11085-11135): a shown pixel between a left and a right anchor of one sector.  (An anchor is
-        // its own on either side; what is not shown needs no repair.)
-        for (int y0 = lo; y0 <= hi; y0 += 8) {
-            unsigned int word[8]; unsigned char row_flags[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const size_t i = (size_t)min(y0 + j, hi) * SW + x;
-                word[j] = meta[i]; row_flags[j] = flags[i];
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int y = y0 + j;
-                if (y > hi || !(row_flags[j] & 1) || (row_flags[j] & 4)) continue;
-                if (!gap_pixel(word[j])) continue;
-                int left = -1, right = SW;            // this pixel is no anchor: the nearest ones on either side
-                for (int k = wave; k >= 0 && left < 0; --k) {
-                    const u64 bits = anchors[y][k] & (k == wave ? (1ULL << lane_id) - 1 : ~0ULL);
-                    if (bits) left = k * 64 + 63 - __clzll((long long)bits);
+            __syncthreads();
+            // --- horizontal (engine.py:11085-11135): a shown pixel between a left and a right anchor of one sector.  (An anchor is
+            // its own on either side; what is not shown needs no repair.)  A thread a word of 32 columns: the pixels are mostly one below the other.
+            for (int task = threadIdx.x; task < rows * (SW / 32); task += FINISH_THREADS) {
+                const int row = task / (SW / 32), word = task - row * (SW / 32), from_low = rows - 1 - row, holder = from_low / each, j = from_low - holder * each;
+                const unsigned int *row_anchors = anchors[row];
+                for (unsigned int rest = open[row][word]; rest; rest &= rest - 1u) {
+                    const int bit = __ffs((int)rest) - 1;
+                    int left = -1, right = SW;        // this pixel is no anchor: the nearest ones on either side
+                    for (int w = word; w >= 0 && left < 0; --w) {
+                        const unsigned int bits = row_anchors[w] & (w == word ? (1u << bit) - 1u : ~0u);
+                        if (bits) left = w * 32 + 31 - __clz((int)bits);
+                    }
+                    for (int w = word; w < SW / 32 && right >= SW; ++w) {
+                        const unsigned int bits = row_anchors[w] & (w == word ? ~0u << bit : ~0u);
+                        if (bits) right = w * 32 + __ffs((int)bits) - 1;
+                    }
+                    if (left < 0 || right >= SW) continue;
+                    const uint2 *held = &row_sectors[j][holder * FINISH_QUADS];      // anchors are not rewritten here
+                    const unsigned left_sector = sector_of(held[left >> 2], left & 3), right_sector = sector_of(held[right >> 2], right & 3);
+                    if (left_sector != right_sector) continue;
+                    const int x = word * 32 + bit;
+                    const size_t i = (size_t)(band_lo + row) * SW + x;
+                    sector[i] = (unsigned short)left_sector;
+                    flags[i] = (unsigned char)(((row_flags[j][holder * FINISH_QUADS + (x >> 2)] >> (8 * (x & 3))) & 0xFFu) | 8u);
                 }
-                for (int k = wave; k < SW / 64 && right >= SW; ++k) {
-                    const u64 bits = anchors[y][k] & (k == wave ? ~(((1ULL << lane_id) - 1) | (1ULL << lane_id)) : ~0ULL);
-                    if (bits) right = k * 64 + __ffsll((long long)bits) - 1;
-                }
-                if (left < 0 || right >= SW) continue;
-                // anchors are not rewritten here, so reading them while other threads write their own pixels is race free
-                const int left_sector = sector[(size_t)y * SW + left], right_sector = sector[(size_t)y * SW + right];
-                if (left_sector == right_sector) { sector[(size_t)y * SW + x] = (unsigned short)left_sector; flags[(size_t)y * SW + x] = (unsigned char)(row_flags[j] | 8); }
             }
         }
     }
@@ -6058,7 +6109,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     hipLaunchKernelGGL(level_masks ? flat_span_select_kernel<true> : flat_span_select_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, sc);
     mark();
     hipLaunchKernelGGL(level_masks ? flat_tail_kernel<true> : flat_tail_kernel<false>, flat_grid(4, 1024), dim3(64 * TAIL_ROWS), 0, stream, r->dm, *lanes, base, sc);
-    hipLaunchKernelGGL(flat_span_finish_kernel, flat_grid(2, 1024), dim3(SW), 0, stream, sc);
+    hipLaunchKernelGGL(flat_span_finish_kernel, flat_grid(2, 1024), dim3(FINISH_THREADS), 0, stream, sc);
     // Billboards that simply cover what lies under them need not wait for the flat pass's pixels: the lanes that hold no other
     // kind (lane_blends, decided on the device) have theirs painted right after the shading, on the side stream, where they
     // mark the gap pixels they take; the flat pass's pixels of those lanes are painted after the join, around the marks.  The
