@@ -273,15 +273,16 @@ struct Scratch {    // per-chunk working memory, sized at create
                            // show the flat pass's picture), of every lane, as one work list: lane << 9 | column, and the rows
                            // they lie in, first | one past the last << 8.  Listed by wall_raster_kernel.
     int *gap_column_count; // [1] its length (cleared by lane_tables_kernel)
-    int *flat_tail;        // [L,2,320] per screen half and column: the sector of the first resolved pixel below the
-                           // half's noted rows, -1 if the column was not looking for one or found none
+    unsigned int *flat_tail; // [L,2,320] per screen half and column: the first resolved pixel below the half's noted rows, row << 16 | sector,
+                           // all ones if the column was not looking for one or found none
     int *flat_span;        // [L,4] first / last row of the ceiling half, then of the floor half, that holds a shown
                            // pixel the flat pass could not resolve and whose repair reads its row (208, -1 = none):
                            // the rows the row repairs work on
     int *flat_spans;       // [L*2] the (lane << 1 | half) with such rows, as one work list
     int *flat_span_count;  // [1] its length (cleared by lane_tables_kernel)
-    int *flat_rows;        // [L*208] the noted rows of every lane as one work list, entry = lane << 8 | row
-    int *flat_row_count;   // [1] its length (cleared by lane_tables_kernel, filled by flat_rows_kernel)
+    int *flat_rows;        // [L*208] the noted rows of every lane as one work list, entry = lane << 8 | row, and from the end of the chunk's
+                           // lanes on backwards those below them, as far as their halves of the screen go
+    int *flat_row_count;   // [2] their lengths (cleared by lane_tables_kernel, filled by flat_rows_kernel)
     int pass_slots;        // passes a column can record in this chunk
     // where pass `pass` of a column lies in the three planes below: the passes that most columns make lie close together
     __device__ __forceinline__ size_t pass_at(int pass, int local, int x) const { return ((size_t)pass * (size_t)lane_stride + (size_t)local) * SW + (size_t)x; }
@@ -610,7 +611,7 @@ __global__ void __launch_bounds__(256) lane_tables_kernel(DeviceMap dm, gd_lanes
     else if (threadIdx.x == 64) {
         int *span = sc.flat_span + (size_t)local * 4;
         span[0] = VH; span[1] = -1; span[2] = VH; span[3] = -1;
-        if (local == 0) { *sc.flat_span_count = 0; *sc.flat_row_count = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
+        if (local == 0) { *sc.flat_span_count = 0; sc.flat_row_count[0] = 0; sc.flat_row_count[1] = 0; *sc.gap_column_count = 0; *sc.spill_count = 0; }
     }
     // the lane's per-column lists start empty
     for (int x = threadIdx.x; x < SW; x += blockDim.x) { sc.cand_count[(size_t)local * SW + x] = 0; sc.block_hit[(size_t)local * SW + x] = ~0ULL; sc.masked_hit[(size_t)local * SW + x] = CAND_KEY_NONE; }
@@ -1617,7 +1618,7 @@ __global__ void __launch_bounds__(64 * GAP_WAVES) flat_gap_kernel(DeviceMap dm, 
 }
 
 // The lanes' row ranges are final once every listed column is repaired: their rows join the work list that
-// flat_span_select_kernel deals out evenly, whichever lanes they come from.  One wavefront per lane.
+// flat_span_select_kernel deals out evenly, whichever lanes they come from, and those below them flat_tail_kernel's.  One wavefront per lane.
 __global__ void __launch_bounds__(64) flat_rows_kernel(int lane_count, Scratch sc) {
     const int local = blockIdx.x;
     if (local >= lane_count) return;
@@ -1625,11 +1626,17 @@ __global__ void __launch_bounds__(64) flat_rows_kernel(int lane_count, Scratch s
     const int lo0 = span[0], hi0 = span[1], lo1 = span[2], hi1 = span[3];
     const int rows0 = hi0 < lo0 ? 0 : hi0 - lo0 + 1, rows1 = hi1 < lo1 ? 0 : hi1 - lo1 + 1;
     if (rows0 + rows1 == 0) return;                  // the same in every thread
+    const int below0 = rows0 == 0 ? 0 : sc.ctx[local].last_ceiling_row - hi0, below1 = rows1 == 0 ? 0 : VH - 1 - hi1;
     int list_base = 0;
-    if (threadIdx.x == 0) list_base = atomicAdd(sc.flat_row_count, rows0 + rows1);
+    if (threadIdx.x < 2) list_base = atomicAdd(&sc.flat_row_count[threadIdx.x], threadIdx.x == 0 ? rows0 + rows1 : below0 + below1);
+    int *below = sc.flat_rows + (size_t)lane_count * VH - 1 - __shfl(list_base, 1);
     list_base = __shfl(list_base, 0);
     for (int r = threadIdx.x; r < rows0 + rows1; r += blockDim.x)
         sc.flat_rows[list_base + r] = (local << 8) | (r < rows0 ? lo0 + r : lo1 + (r - rows0));
+    for (int r = threadIdx.x; r < below0 + below1; r += blockDim.x)
+        below[-r] = (local << 8) | (r < below0 ? hi0 + 1 + r : hi1 + 1 + (r - below0));
+    for (int x = threadIdx.x; x < 2 * SW; x += blockDim.x)
+        if (x < SW ? rows0 > 0 : rows1 > 0) sc.flat_tail[(size_t)local * 2 * SW + x] = ~0u;
 }
 
 // Small per-sector / per-texture tables staged in LDS by the kernels whose inner loops chase
@@ -1844,38 +1851,25 @@ __global__ void __launch_bounds__(256) flat_span_select_kernel(DeviceMap dm, gd_
 }
 
 // A column whose pixel in the last noted row of a half is unresolved looks further down for a resolved one
-// (engine.py:11026-11083).  One block per 64 columns of a half with noted rows; its TAIL_ROWS wavefronts select that many rows
-// at a time, while any of the columns is still looking.
-#define TAIL_ROWS 16
+// (engine.py:11026-11083).  A wavefront takes 64 columns of a row at a time, like flat_span_select_kernel; the columns that look no
+// further, by what the rows above it have found so far, are left out.  (A work-group of sixteen wavefronts went down 64 columns
+// sixteen rows at a time, a step after the other and, for its LDS, one work-group a compute unit: 39 us at 256 lanes of 800
+// linedefs, 60 at 512 of 4000, 120 at 1024 of 2000; now 18, 35 and 61.)
 template <bool MASKS>
-__global__ void __launch_bounds__(64 * TAIL_ROWS) flat_tail_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, Scratch sc) {
-    __shared__ RowLds row_lds[TAIL_ROWS];
-    __shared__ int found_lds[TAIL_ROWS][64];
-    const int slot = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int total = *sc.flat_span_count * (SW / 64);
-    for (int task = blockIdx.x; task < total; task += gridDim.x) {
-        const int entry = task / (SW / 64), x = (task - entry * (SW / 64)) * 64 + slot;
-        const int packed = sc.flat_spans[entry], local = packed >> 1, half = packed & 1;
-        const int last = sc.flat_span[(size_t)local * 4 + 2 * half + 1];
-        const int half_end = half ? VH - 1 : sc.ctx[local].last_ceiling_row;
-        bool looking = sc.flat_flags[(size_t)local * VH * SW + (size_t)last * SW + x] & 1;
-        int found = -1;
-        for (int y0 = last + 1; y0 <= half_end; y0 += TAIL_ROWS) {
-            if (!__syncthreads_or(looking)) break;   // also keeps the rows of the previous step apart from this one's
-            const int y = y0 + wave;
-            int s = -1;
-            if (y <= half_end) s = flat_select_row<MASKS>(dm, sc, lanes, local, lane_base + local, x, y, looking, &row_lds[wave]);   // the same in a whole wavefront
-            found_lds[wave][slot] = s;
-            __syncthreads();
-            if (looking) {
-                for (int j = 0; j < TAIL_ROWS; ++j) {
-                    const int below = found_lds[j][slot];
-                    if (below >= 0) { looking = false; found = below; break; }
-                }
-            }
-        }
-        __syncthreads();
-        if (wave == 0) sc.flat_tail[((size_t)local * 2 + half) * SW + x] = found;
+__global__ void __launch_bounds__(256) flat_tail_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc) {
+    __shared__ RowLds row_lds[4];
+    const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63;
+    const int total = sc.flat_row_count[1] * (SW / 64);
+    for (int task = blockIdx.x * 4 + wave; task < total; task += gridDim.x * 4) {
+        const int entry = task / (SW / 64), x = (task - entry * (SW / 64)) * 64 + lane_id;
+        const int packed = sc.flat_rows[(size_t)lane_count * VH - 1 - entry], local = packed >> 8, y = packed & 255;
+        const int half = y > sc.ctx[local].last_ceiling_row ? 1 : 0, last = sc.flat_span[(size_t)local * 4 + 2 * half + 1];
+        unsigned int *found = sc.flat_tail + ((size_t)local * 2 + half) * SW + x;
+        const bool looking = (sc.flat_flags[(size_t)local * VH * SW + (size_t)last * SW + x] & 1) &&
+                             __hip_atomic_load(found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > ((unsigned)y << 16);
+        if (__ballot(looking) == 0) continue;
+        const int s = flat_select_row<MASKS>(dm, sc, lanes, local, lane_base + local, x, y, looking, &row_lds[wave]);
+        if (looking && s >= 0) atomicMin(found, ((unsigned)y << 16) | (unsigned)s);
     }
 }
 
@@ -1907,8 +1901,8 @@ __global__ void __launch_bounds__(FINISH_THREADS) flat_span_finish_kernel(Scratc
         unsigned char *flags = sc.flat_flags + (size_t)local * VH * SW;
         const unsigned int *meta = sc.meta + (size_t)local * VH * SW;
         // what flat_tail_kernel found below the range for a column whose pixel in the range's last row is unresolved
-        const int4 tail = *reinterpret_cast<const int4 *>(sc.flat_tail + ((size_t)local * 2 + half) * SW + x0);
-        unsigned below[4] = {(unsigned)tail.x & 0xFFFFu, (unsigned)tail.y & 0xFFFFu, (unsigned)tail.z & 0xFFFFu, (unsigned)tail.w & 0xFFFFu};
+        const uint4 tail = *reinterpret_cast<const uint4 *>(sc.flat_tail + ((size_t)local * 2 + half) * SW + x0);
+        unsigned below[4] = {tail.x & 0xFFFFu, tail.y & 0xFFFFu, tail.z & 0xFFFFu, tail.w & 0xFFFFu};
         for (int band_hi = hi; band_hi >= lo; band_hi -= FINISH_BAND) {
             const int rows = min(band_hi - lo + 1, FINISH_BAND), band_lo = band_hi - rows + 1;
             const int each = (rows + FINISH_CHUNKS - 1) / FINISH_CHUNKS, first = band_hi - chunk * each;   // a thread's rows, the lowest first
@@ -5822,7 +5816,7 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.flat_spans, L * 2);
     take(&sc.flat_span_count, 1);
     take(&sc.flat_rows, L * (size_t)VH);
-    take(&sc.flat_row_count, 1);
+    take(&sc.flat_row_count, 2);
     take(&sc.gap_columns, L * SW);
     take(&sc.gap_column_count, 1);
     sc.pass_slots = h.sector_count < 16 ? 16 : (h.sector_count > PASS_MAX ? PASS_MAX : h.sector_count);
@@ -6108,7 +6102,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     hipLaunchKernelGGL(flat_rows_kernel, dim3(count), dim3(64), 0, stream, count, sc);
     hipLaunchKernelGGL(level_masks ? flat_span_select_kernel<true> : flat_span_select_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, sc);
     mark();
-    hipLaunchKernelGGL(level_masks ? flat_tail_kernel<true> : flat_tail_kernel<false>, flat_grid(4, 1024), dim3(64 * TAIL_ROWS), 0, stream, r->dm, *lanes, base, sc);
+    hipLaunchKernelGGL(level_masks ? flat_tail_kernel<true> : flat_tail_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, count, sc);
     hipLaunchKernelGGL(flat_span_finish_kernel, flat_grid(2, 1024), dim3(FINISH_THREADS), 0, stream, sc);
     // Billboards that simply cover what lies under them need not wait for the flat pass's pixels: the lanes that hold no other
     // kind (lane_blends, decided on the device) have theirs painted right after the shading, on the side stream, where they
