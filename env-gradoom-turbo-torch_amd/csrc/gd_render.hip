@@ -3788,19 +3788,24 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     if (lane_of_column == 0) sc.pass_count[(size_t)local * SW + x] = (unsigned char)recorded;
 }
 
-// The strips from `first_slot` on in the order, as many as the grid has wavefronts for.  A strip of the longest that its lanes cannot hold is
-// drawn here too, not in a launch behind this one, which small batches paid 7 us for.  (16 lanes: 130 registers left to itself, 128 as told.)
+// The strips from `first` on in the order: `longest` of them with LANES wavefronts each, and as many more of one wavefront, a lane a column, as the
+// grid has wavefronts for.  The two kinds start by turns, eight wavefronts of each, so that both are dealt out over all eight dies and neither waits for
+// the other's to end.  A strip of the longest that its lanes cannot hold is drawn here too, not in a launch behind this one, which small batches
+// paid 7 us for.  (16 lanes: 130 registers left to itself, 128 as told.)
 template <bool SPLIT, int LANES>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES == 8 ? 3 : 4))) wall_select_kernel(DeviceMap dm, Scratch sc, int first_slot) {
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES == 8 ? 3 : 4))) wall_select_kernel(DeviceMap dm, Scratch sc, int first, int longest) {
     __shared__ LaneCtx lane_ctx;
-    const int segment = sc.strip_order[first_slot + (int)blockIdx.x / LANES], part = (int)blockIdx.x % LANES;
+    const int shares = longest * LANES, others = (int)gridDim.x - shares, mixed = min(shares, others) & ~7, b = (int)blockIdx.x;
+    const bool beyond = b < 2 * mixed ? (b & 8) != 0 : shares - mixed <= b - 2 * mixed;
+    const int at = b < 2 * mixed ? ((b >> 4) << 3) | (b & 7) : (beyond ? b - shares : b - mixed);
+    const int segment = sc.strip_order[first + (beyond ? longest + at : at / LANES)], part = beyond ? 0 : at % LANES;
     const int local = segment / SEGS_PER_LANE, strip_x = (segment - local * SEGS_PER_LANE) * SEG_COLS;
     if (threadIdx.x == 0) lane_ctx = sc.ctx[local];
     __syncthreads();
     if constexpr (LANES > 1) {
         // A strip with a column in the spill pool (more entries than its lanes hold) is the first of its wavefronts', a lane a column.
-        if (__ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + threadIdx.x] >> SPILL_SHIFT) != 0) != 0) {
-            if (part == 0) select_columns<SPLIT, 1>(dm, sc, lane_ctx, local, strip_x, 0);
+        if (beyond || __ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + threadIdx.x] >> SPILL_SHIFT) != 0) != 0) {
+            if (beyond || part == 0) select_columns<SPLIT, 1>(dm, sc, lane_ctx, local, strip_x, 0);
             return;
         }
     }
@@ -6023,31 +6028,26 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     {
         const int wavefronts = (count * SEGS_PER_LANE + 64 / SEG_COLS - 1) / (64 / SEG_COLS);
         const bool split = m.split_count > 0;
-        // The longest strips here, the others on the side stream, both at once.  This way round: the
-        // side stream starts a few microseconds behind, time enough for the longest strips' work-groups to be placed;
-        // started together, the other launch's 20,000 take every wavefront slot first and the strips that decide how long
-        // the pair lasts begin last.
+        // The longest strips' wavefronts and the others': in one launch, by turns, or the former here and the others on the side stream, both at
+        // once (select_together).  This way round: the side stream starts a few microseconds behind, time enough for the longest
+        // strips' work-groups to be placed; started together, the other launch's 20,000 take every wavefront slot first and the strips that
+        // decide how long the pair lasts begin last.
         const int strips = count * SEGS_PER_LANE;
         const int longest_wanted = select_strips(count, m.wall_count);
-        const int longest = r->side_ready ? (strips < longest_wanted ? strips : longest_wanted) : 0;
-        auto select_kernel = split ? wall_select_kernel<true, 1> : wall_select_kernel<false, 1>;
-        if (longest > 0) {
-            const bool alone = longest == strips;
-            if (!alone) {
-                HIP_TRY(hipEventRecord(r->fork_event, stream));
-                HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
-            }
-            const int column_lanes = select_lanes(count, m.wall_count);
-            auto pick = [&](auto lanes) { constexpr int L = decltype(lanes)::value; return split ? wall_select_kernel<true, L> : wall_select_kernel<false, L>; };
-            auto longest_kernel = column_lanes == 32 ? pick(std::integral_constant<int, 32>()) : (column_lanes == 16 ? pick(std::integral_constant<int, 16>()) : pick(std::integral_constant<int, 8>()));
-            hipLaunchKernelGGL(longest_kernel, dim3(longest * column_lanes), dim3(64), 0, stream, r->dm, sc, 0);
-            if (!alone) hipLaunchKernelGGL(select_kernel, dim3(strips - longest), dim3(64), 0, r->side_stream, r->dm, sc, longest);
-            if (!alone) {
-                HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
-                HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
-            }
+        const int longest = strips < longest_wanted ? strips : longest_wanted, others = strips - longest;
+        auto pick_select = [&](auto lanes) { constexpr int L = decltype(lanes)::value; return split ? wall_select_kernel<true, L> : wall_select_kernel<false, L>; };
+        const int column_lanes = longest > 0 ? select_lanes(count, m.wall_count) : 1;
+        auto longest_kernel = column_lanes == 32 ? pick_select(std::integral_constant<int, 32>())
+                              : (column_lanes == 16 ? pick_select(std::integral_constant<int, 16>()) : (column_lanes == 8 ? pick_select(std::integral_constant<int, 8>()) : pick_select(std::integral_constant<int, 1>())));
+        if (longest == 0 || others == 0 || select_together(count) || !r->side_ready) {
+            hipLaunchKernelGGL(longest_kernel, dim3(longest * column_lanes + others), dim3(64), 0, stream, r->dm, sc, 0, longest);
         } else {
-            hipLaunchKernelGGL(select_kernel, dim3(strips), dim3(64), 0, stream, r->dm, sc, 0);
+            HIP_TRY(hipEventRecord(r->fork_event, stream));
+            HIP_TRY(hipStreamWaitEvent(r->side_stream, r->fork_event, 0));
+            hipLaunchKernelGGL(longest_kernel, dim3(longest * column_lanes), dim3(64), 0, stream, r->dm, sc, 0, longest);
+            hipLaunchKernelGGL(pick_select(std::integral_constant<int, 1>()), dim3(others), dim3(64), 0, r->side_stream, r->dm, sc, longest, 0);
+            HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
+            HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
         }
         // the billboards' lists beside the walls' drawing, on the side stream (when stages are being timed, with the billboards)
         if (has_billboards && !fused && !timed) {

@@ -53,6 +53,18 @@ inline int select_lanes(int lanes, int linedefs) {
     return lanes <= 128 + w / 8 || (lanes >= 1536 && w >= 1024) ? 16 : 8;
 }
 
+// wall_select_kernel: the longest strips and the others in one launch?  A launch on the side stream and back costs 8 us and more.  In larger batches
+// the others' wavefronts are so many that they hold the longest strips' up, which the side stream's start a little later do not.  A frame in
+// us, one launch / two (32 billboards, two sets of poses):
+//   lanes        320             800             1400            2000            4000          701, bricks
+//    256     335 / 342       382 / 390       454 / 463       449 / 457       653 / 661       520 / 527
+//    384     420 / 423       464 / 474       575 / 582       547 / 554       780 / 787       586 / 587
+//    512     496 / 498       552 / 562       629 / 645       639 / 643       880 / 912       669 / 670
+//    640     570 / 572       617 / 627       747 / 761       716 / 720       978 / 994       724 / 726
+//    768     642 / 643       709 / 715       857 / 873       814 / 812      1130 /1136       838 / 839
+//   1024     737 / 742       817 / 805       956 / 952       973 / 962      1345 /1342       952 / 935
+inline bool select_together(int lanes) { return lanes <= 704; }
+
 // wall_geometry_kernel: wavefronts a lane for its linedefs (a power of two).  us with 4 / 8 / 16 of them: 16 lanes 13.6 / 10.7 / 8.3, 512 lanes
 // 63 / 48 / 46, 1024 lanes 48 / 41 / 42, 4096 lanes 263 / 242 / 247.
 inline int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
