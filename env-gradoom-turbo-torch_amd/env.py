@@ -323,6 +323,8 @@ class GraDoomVecEnv:
         self._words = torch.zeros(16, dtype=torch.int32, pin_memory=True) if self._native else None
         self._words_read = self._words.numpy() if self._native else None
         self._done_rows = torch.zeros(n, dtype=torch.int64, device=self.device) if self._native else None
+        # where a step's bookkeeping ends, and where its frames do: each is waited for by itself
+        self._listed_mark, self._drawn_mark = (torch.cuda.Event(), torch.cuda.Event()) if self._native else (None, None)
         self._rgb_staging = None        # pinned, at most RGB_STAGING_BYTES
         self._leave_frames = _FRAMES.join(self)
         self._seed_values = [None] * n
@@ -441,9 +443,14 @@ class GraDoomVecEnv:
         indices = self._require_device_tensor(actions, "actions", shape=(self.num_envs,), dtypes=INDEX_DTYPES).to(torch.int64)
         rewards, terminated, truncated = self._dynamics.step(indices)
         self._done_listed = self._after_step(terminated, truncated, list_done)
-        if not self._done_listed:
+        marks = self._done_listed and list_done
+        if marks:
+            self._listed_mark.record(torch.cuda.current_stream(self.device))
+        elif not self._done_listed:
             self.pending_reset.copy_(terminated | truncated)      # engine.py:9542
         self._renderer.render(self._dynamics.lane_state(), frames=self.frames, final_frames=final_frames, final_layout=final_layout)
+        if marks:
+            self._drawn_mark.record(torch.cuda.current_stream(self.device))
         if not self._done_listed:
             self._update_signals()
         return DeviceTransition(
@@ -459,21 +466,25 @@ class GraDoomVecEnv:
         final_signals = transition.signals.clone()
         final_info_histories = transition.info_histories.clone()
         listed = self._done_listed
-        if listed:   # how many lanes ended came with the step: one wait on the stream
-            self._wait()
+        if listed:   # how many lanes ended is known as soon as the step's bookkeeping is done, while its frames are being drawn
+            self._listed_mark.synchronize()
             done_count = int(self._words_read[0])
         else:
             done = transition.terminated | transition.truncated
             done_count = int(torch.count_nonzero(done))  # env.py:919: one host sync for the reference renderer
-        self.check_renderer_status()      # the stream has been waited for here anyway
+        alone = listed and 0 < done_count <= 65535 and self._resets_alone()
+        if alone:    # their reset is queued behind the step's frames: the device goes from one to the other without the host
+            observations, signals = self._reset_rows(self.pending_reset.clone(), reset_seeds, done_count)
+            self._drawn_mark.synchronize()
+            self._refuse_truncated(self._renderer.status_seen())
+        else:
+            self.check_renderer_status()
         if not done_count:
             return DeviceAutoResetTransition(
                 transition.observations, transition.rewards, transition.terminated, transition.truncated,
                 transition.signals, transition.info_histories, final_observations, final_signals, final_info_histories,
             )
-        if listed and done_count <= 65535 and self._resets_alone():
-            observations, signals = self._reset_rows(self.pending_reset.clone(), reset_seeds, done_count)
-        else:
+        if not alone:
             done = transition.terminated | transition.truncated
             observations, signals = self.reset_device(done, reset_seeds)
         return DeviceAutoResetTransition(
@@ -498,7 +509,9 @@ class GraDoomVecEnv:
             self._wait()
         elif status is None:
             status = getattr(self._renderer, "status", None)
-        flags = status() if status is not None else 0
+        self._refuse_truncated(status() if status is not None else 0)
+
+    def _refuse_truncated(self, flags: int) -> None:
         if flags & 1:
             raise RuntimeError(
                 "the renderer truncated a screen column's candidate list (more than 256 linedefs overlap one column of one "

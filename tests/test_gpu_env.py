@@ -143,6 +143,26 @@ def test_a_step_does_not_wait_for_other_streams():
     env.close()
 
 
+@pytest.mark.parametrize("timeout", [1, 50])
+def test_a_step_with_truncated_frames_is_refused_whether_lanes_end_or_not(monkeypatch, timeout):
+    """The lanes that end are reset behind the step's frames, before the host has waited for these: their check comes all the same."""
+
+    from gradoom_amd.env import GraDoomVecEnv
+
+    _meta, _data, smap, _tables = load_fixture("small_midtex_sprites")
+    lanes = 3
+    env = GraDoomVecEnv(smap, lanes, device="cuda:0", episode_timeout=timeout, sprites=4)
+    actions, seeds = torch.zeros(lanes, dtype=torch.int64, device="cuda:0"), torch.arange(lanes, device="cuda:0")
+    env.reset_device(torch.ones(lanes, dtype=torch.bool, device="cuda:0"), seeds)
+    assert bool(env.step_and_reset_device(actions, seeds).truncated.all()) == (timeout == 1)
+    monkeypatch.setattr(env._renderer, "status_seen", lambda: 1)
+    with pytest.raises(RuntimeError, match="candidate list"):
+        env.step_and_reset_device(actions, seeds)
+    monkeypatch.undo()
+    env.step_and_reset_device(actions, seeds)
+    env.close()
+
+
 def test_a_pose_pool_whose_lane_state_takes_no_lanes_resets_the_lanes_that_end():
     from gradoom_amd.env import GraDoomVecEnv, PosePoolDynamics
 
