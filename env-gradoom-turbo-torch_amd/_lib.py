@@ -37,6 +37,7 @@ SYMBOLS = (
     "gd_screen_blend",
     "gd_ray_tables",
     "gd_sprite_depth",
+    "gd_lane_floats",
     "gd_pose_lanes",
     "gd_pose_step",
     "gd_pose_reset",
@@ -111,6 +112,7 @@ def library() -> C.CDLL:
     lib.gd_sprite_depth.restype = C.c_int
     lib.gd_sprite_depth.argtypes = [C.c_void_p] * 5 + [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p]
     for name, arguments in (
+        ("gd_lane_floats", [C.c_void_p] * 6 + [C.c_int32, C.c_int32] + [C.c_void_p] * 4),
         ("gd_pack_actors_facing", [C.POINTER(_abi.ActorDesc), C.POINTER(_abi.FacingDesc), C.c_void_p]),
         ("gd_pack_weapon_narrow", [C.POINTER(_abi.WeaponDesc), C.c_uint32, C.c_void_p]),
         ("gd_pack_hud", [C.POINTER(_abi.HudDesc), C.c_void_p]),

@@ -105,6 +105,21 @@ def sprite_depth_kernel(x, y, angle, sprite_x, sprite_y) -> torch.Tensor:
     return depth
 
 
+def lane_floats_kernel(x, y, angle, offsets, sprite_x, sprite_y) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """``ray_tables_kernel`` and ``sprite_depth_kernel`` in one launch: (ray_cos, ray_sin, depth)."""
+
+    from . import _lib  # noqa: PLC0415
+
+    count, slots = sprite_x.shape
+    rays = count * SCREEN_WIDTH
+    floats = torch.empty(2 * rays + count * slots, dtype=torch.float32, device=angle.device)
+    ray_cos, ray_sin, depth = floats[:rays].view(count, SCREEN_WIDTH), floats[rays : 2 * rays].view(count, SCREEN_WIDTH), floats[2 * rays :].view(count, slots)
+    with torch.cuda.device(angle.device):
+        _lib.check(_lib.library().gd_lane_floats(x.data_ptr(), y.data_ptr(), angle.data_ptr(), offsets.data_ptr(), sprite_x.data_ptr(), sprite_y.data_ptr(), count, slots,
+                                                 ray_cos.data_ptr(), ray_sin.data_ptr(), depth.data_ptr(), torch.cuda.current_stream(angle.device).cuda_stream))
+    return ray_cos, ray_sin, depth
+
+
 def sprite_depth(x, y, angle, sprite_x, sprite_y) -> torch.Tensor:
     if _on_device(x, y, angle, sprite_x, sprite_y) and x.shape == y.shape == angle.shape == sprite_x.shape[:1] and sprite_x.shape == sprite_y.shape and sprite_x.dim() == 2:
         return sprite_depth_kernel(x, y, angle, sprite_x, sprite_y)

@@ -203,13 +203,10 @@ class HipRenderer:
             setattr(desc, name, _require(getattr(lanes, name), name, torch.float32, (count,), device).data_ptr())
         for name in ("x_fixed", "y_fixed", "angle_bam", "pitch_bam", "flash_light"):
             setattr(desc, name, _require(getattr(lanes, name), name, torch.int64, (count,), device).data_ptr())
-        if lanes.ray_cos is None or lanes.ray_sin is None:
-            ray_cos, ray_sin = hostmath.ray_tables_kernel(lanes.angle, _require(self.ray_offsets, "ray_offsets", torch.float32, (320,), device))
-        else:
-            ray_cos, ray_sin = lanes.ray_cos, lanes.ray_sin
-        keep += [ray_cos, ray_sin]
-        desc.ray_cos = _require(ray_cos, "ray_cos", torch.float32, (count, 320), device).data_ptr()
-        desc.ray_sin = _require(ray_sin, "ray_sin", torch.float32, (count, 320), device).data_ptr()
+        ray_cos, ray_sin, depth = lanes.ray_cos, lanes.ray_sin, lanes.sprite_depth
+        wants_rays = ray_cos is None or ray_sin is None
+        if wants_rays:
+            offsets = _require(self.ray_offsets, "ray_offsets", torch.float32, (320,), device)
         desc.sprite_slots = 0
         if lanes.sprite_x is not None and lanes.sprite_x.shape[1] > 0:
             slots = int(lanes.sprite_x.shape[1])
@@ -230,11 +227,18 @@ class HipRenderer:
                 desc.sprite_fullbright = _require(bright, "sprite_fullbright", torch.uint8, (count, slots), device).data_ptr()
             if lanes.sprite_style is not None:
                 desc.sprite_style = _require(lanes.sprite_style, "sprite_style", torch.int8, (count, slots), device).data_ptr()
-            depth = lanes.sprite_depth
-            if depth is None:
+            if depth is None and wants_rays:
+                ray_cos, ray_sin, depth = hostmath.lane_floats_kernel(lanes.x, lanes.y, lanes.angle, offsets, lanes.sprite_x, lanes.sprite_y)
+                wants_rays = False
+            elif depth is None:
                 depth = hostmath.sprite_depth_kernel(lanes.x, lanes.y, lanes.angle, lanes.sprite_x, lanes.sprite_y)
             keep.append(depth)
             desc.sprite_depth = _require(depth, "sprite_depth", torch.float32, (count, slots), device).data_ptr()
+        if wants_rays:
+            ray_cos, ray_sin = hostmath.ray_tables_kernel(lanes.angle, offsets)
+        keep += [ray_cos, ray_sin]
+        desc.ray_cos = _require(ray_cos, "ray_cos", torch.float32, (count, 320), device).data_ptr()
+        desc.ray_sin = _require(ray_sin, "ray_sin", torch.float32, (count, 320), device).data_ptr()
         if lanes.weapon_state is not None:
             desc.weapon_state = _require(lanes.weapon_state, "weapon_state", torch.int64, (count, 5), device).data_ptr()
         desc.decal_slots = 0

@@ -570,11 +570,14 @@ int gd_screen_blend(const int64_t *bonus_count, const int64_t *damage_count, con
  *   gd_ray_tables:    ray_cos / ray_sin [N,320] = cos / sin(angle[n] + ray_offsets[x])                 (engine.py:10966-10974)
  *   gd_sprite_depth:  depth [N,A] = max(|d|, 1) * cos(remainder(atan2(dy, dx) - angle + pi, 2 pi) - pi), d = sprite - camera
  *                     (engine.py:14684-14688)
+ *   gd_lane_floats:   both in one launch (without billboards, sprite_slots 0, the rays alone)
  * All pointers are device pointers to contiguous arrays.  Returns GD_E_ARG for a null pointer or a negative count.
  */
 int gd_ray_tables(const float *angle, const float *ray_offsets, int32_t lane_count, float *ray_cos, float *ray_sin, void *stream);
 int gd_sprite_depth(const float *x, const float *y, const float *angle, const float *sprite_x, const float *sprite_y,
                     int32_t lane_count, int32_t sprite_slots, float *depth, void *stream);
+int gd_lane_floats(const float *x, const float *y, const float *angle, const float *ray_offsets, const float *sprite_x, const float *sprite_y,
+                   int32_t lane_count, int32_t sprite_slots, float *ray_cos, float *ray_sin, float *depth, void *stream);
 
 /*
  * A vector environment's work around its frames (gradoom_amd/env.py), one kernel each on `stream`.  Pointers are device pointers, except

@@ -32,3 +32,5 @@ def test_ray_tables_and_sprite_depths_have_the_bits_of_the_torch_expressions(lan
     expected = torch.sqrt(dx * dx + dy * dy).clamp_min(1) * torch.cos(relative)
     depth = hostmath.sprite_depth(x, y, angle, sprite_x, sprite_y)
     assert torch.equal(depth.view(torch.int32), expected.view(torch.int32))
+    together = hostmath.lane_floats_kernel(x, y, angle, offsets, sprite_x, sprite_y)
+    assert all(torch.equal(one.view(torch.int32), other.view(torch.int32)) for one, other in zip(together, (ray_cos, ray_sin, depth)))
