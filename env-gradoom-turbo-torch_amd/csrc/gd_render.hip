@@ -6076,15 +6076,16 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         }
         mark();
         hipLaunchKernelGGL(split ? wall_geometry_kernel<true> : wall_geometry_kernel<false>, dim3(geometry_parts(count) + SW / 64, count), dim3(64), 0, stream, r->dm, count, sc, geometry_parts(count));
-        const dim3 grid((wavefronts * raster_parts(count) + WALL_STRIPS_PER_GROUP - 1) / WALL_STRIPS_PER_GROUP), block(64 * WALL_STRIPS_PER_GROUP);
+        const int parts = raster_sixteen(count) ? 16 : raster_parts(count);
+        const dim3 grid((wavefronts * parts + WALL_STRIPS_PER_GROUP - 1) / WALL_STRIPS_PER_GROUP), block(64 * WALL_STRIPS_PER_GROUP);
         const bool general = split || m.sector_count > LDS_SECTORS || m.texture_count > LDS_TEXTURES;
         auto pick = [&](auto parts) {
             constexpr int P = decltype(parts)::value;
             return decals ? (general ? wall_raster_kernel<true, true, P> : wall_raster_kernel<true, false, P>)
                           : (general ? wall_raster_kernel<false, true, P> : wall_raster_kernel<false, false, P>);
         };
-        const int parts = raster_parts(count);
-        auto kernel = parts == 8 ? pick(std::integral_constant<int, 8>()) : parts == 4 ? pick(std::integral_constant<int, 4>()) : parts == 2 ? pick(std::integral_constant<int, 2>()) : pick(std::integral_constant<int, 1>());
+        auto kernel = parts == 16 ? pick(std::integral_constant<int, 16>()) : parts == 8 ? pick(std::integral_constant<int, 8>()) : parts == 4 ? pick(std::integral_constant<int, 4>())
+                      : parts == 2 ? pick(std::integral_constant<int, 2>()) : pick(std::integral_constant<int, 1>());
         hipLaunchKernelGGL(kernel, grid, block, 0, stream, r->dm, count, sc, frame_base, frame_stride);
     }
     mark();

@@ -92,6 +92,18 @@ inline int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
 // issue 1.5 % fewer instructions and take as long: 686, 905, 1239, 975.)
 inline int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 2400 ? 2 : 1)); }
 
+// The smallest batches, whose strips leave most of the chip idle even so: sixteen wavefronts a strip, of four columns (as many as decide on a shared
+// group of rows together) with sixteen lanes each.  A frame in us, sixteen / eight (32 billboards, two sets of poses):
+//   lanes        320             800             1400            2000            4000          701, bricks
+//      1     123 / 124       127 / 130       186 / 190       153 / 157       209 / 213       202 / 214
+//     16     238 / 240       243 / 249       237 / 241       266 / 266       366 / 373       307 / 325
+//     64     264 / 267       276 / 287       302 / 301       335 / 343       525 / 544       386 / 408
+//     96     281 / 285       318 / 326       330 / 327       365 / 374       548 / 563       407 / 430
+//    128     289 / 292       330 / 334       364 / 349       389 / 403       573 / 586       414 / 438
+//    192     338 / 312       366 / 357       434 / 413       419 / 422       652 / 661       443 / 471
+//    256     389 / 333       419 / 378       509 / 450       481 / 444       662 / 649       495 / 518
+inline bool raster_sixteen(int lanes) { return lanes <= 96; }
+
 // flat_gap_kernel: wavefronts a half of a column.  The fewer the lanes, the fewer such halves and the longer the kernel lasts as its slowest one; the
 // more, the longer a large work-group waits for room beside the shading.  A frame in us with 2 / 4 / 8 / 16 wavefronts (32 billboards, two
 // sets of poses; in brackets with a column's halves one after the other, 16 wavefronts up to 1536 lanes, 8 beyond):

@@ -70,7 +70,7 @@ def test_batches_on_both_sides_of_a_sharing_rules_line_match_the_oracle(oracle, 
 
 # (those of the selection and of the drawing: test_gpu_shared_lists.py and test_gpu_shared_columns.py)
 @pytest.mark.parametrize("rule, billboards", [
-    ("setup_whole_lanes", True), ("select_together", True), ("geometry_parts", True), ("gap_waves", True), ("sprite_row_parts", True), ("side_stream_pays", True), ("side_stream_pays", False),
+    ("setup_whole_lanes", True), ("select_together", True), ("raster_sixteen", True), ("geometry_parts", True), ("gap_waves", True), ("sprite_row_parts", True), ("side_stream_pays", True), ("side_stream_pays", False),
 ])
 def test_batches_on_both_sides_of_a_rules_line_match_the_oracle(oracle, rule, billboards):
     import launch_rules
