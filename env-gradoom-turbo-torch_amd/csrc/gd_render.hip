@@ -297,7 +297,9 @@ struct Scratch {    // per-chunk working memory, sized at create
                            // slot in blocking_walls, all ones when no ray hits (engine.py:10534-10557)
     int *sprite_listed;    // [L] the lane's billboards that reach the view at all (sprite_list_kernel)
     int *lane_blends;      // [L] does some live billboard of the lane blend with the pixel below it (sprite_style other than -1)?
-                           // lane_tables_kernel says; launch_chunk's two billboard launches split the lanes by it
+                           // (lane_tables_kernel)
+    unsigned char *sprite_late; // [L, SW / SPRITE_COLUMNS, SPRITE_ROW_PARTS] did this work-group of the billboards' early launch leave pixels to the
+                           // late one? (written for lanes that blend)
     unsigned char *strip_key;  // [L*SEGS_PER_LANE] expected traversal length of each (lane, segment of SEG_COLS columns)
     int *strip_order;      // [L*SEGS_PER_LANE] segments, longest expected traversal first
     volatile unsigned char *status;   // [2] sticky flags in pinned host memory: a candidate list, a list of passes was cut short
@@ -317,10 +319,10 @@ struct Scratch {    // per-chunk working memory, sized at create
 #define META_FILLED 0x80000000u   // an opaque wall tier owns the pixel; its palette index sits in the low byte of the
                                   // plane sector field (plane shading, which writes every other view pixel, stores it)
 #define META_FLOOR 0x40000000u    // the owning plane is a floor
-// which lanes a billboard or flat-shading launch takes (launch_chunk splits them by Scratch::lane_blends)
-#define LANES_ALL 0
-#define LANES_PLAIN 1
-#define LANES_BLENDING 2
+// when a launch paints billboards: all of them at the end; those that need not wait for the flat pass's pixels; the others
+#define SPRITES_ALL 0
+#define SPRITES_EARLY 1
+#define SPRITES_LATE 2
 #define META_GAP_COVERED META_FLOOR   // in the word of a gap pixel (no tier, no plane, no masked texture: the bit above means nothing
                                   // there): a billboard was painted over it before the flat pass's pixels were, which flat_shade_kernel respects
 #define META_MASKED 0x20000000u   // a masked mid-texture was drawn over the pixel
@@ -4095,18 +4097,14 @@ __device__ void flat_shade_pixel(const DeviceMap &dm, const Scratch &sc, const L
     frame[pixel] = flat_pixel(tb, m->colormap, c, s, delta > 0, x, y);
 }
 
-// lane_pick: LANES_ALL, or one half of launch_chunk's split: LANES_PLAIN for the lanes whose billboards were painted first and
-// marked the gap pixels they took, LANES_BLENDING for the others, whose billboards come after this.
-__global__ void __launch_bounds__(64) flat_shade_kernel(DeviceMap dm, Scratch sc, unsigned char *frame_base, size_t frame_stride, int lane_pick) {
-    const bool after_billboards = lane_pick == LANES_PLAIN;
+__global__ void __launch_bounds__(64) flat_shade_kernel(DeviceMap dm, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const int total = *sc.gap_column_count;
     for (int entry = blockIdx.x; entry < total; entry += gridDim.x) {
         const int2 packed = sc.gap_columns[entry];
         const int local = packed.x >> 9, x = packed.x & 511, last = packed.y >> 8;
-        if (lane_pick != LANES_ALL && (sc.lane_blends[local] != 0) != (lane_pick == LANES_BLENDING)) continue;   // the same in the whole block
         for (int y = (packed.y & 255) + (int)threadIdx.x; y < last; y += 64) {
             const unsigned int word = sc.meta[(size_t)local * VH * SW + (size_t)y * SW + x];
-            if (gap_pixel(word) && !(after_billboards && (word & META_GAP_COVERED)))
+            if (gap_pixel(word) && !(word & META_GAP_COVERED))
                 flat_shade_pixel(dm, sc, sc.ctx[local], local, y * SW + x, frame_base + (size_t)local * frame_stride);
         }
     }
@@ -4404,7 +4402,9 @@ __global__ void __launch_bounds__(LIST_THREADS) sprite_list_kernel(DeviceMap dm,
 // A list longer than SPRITE_CHUNK, one word of bits, is painted in chunks of that many, the farthest first: the LDS a group
 // needs does not follow the slots a lane has.
 // Bound by the waits of pixels that show something: their clip, their texels (one word: three bytes each cost 3 % more), and the flat ray.
-// Five wavefronts a SIMD (seven registers spilled) are better than four by 4 %, six worse by 25 %.
+// BLENDS: frames with sprite_style.  The others have no use for what blending takes: five registers of the seven spilled (a frame of 4096 lanes
+// 3825 -> 3810 us without).  Five wavefronts a SIMD are better than four by 4 %, six worse by 25 %; four for the early launch that blends, which would
+// spill 17 (1024 lanes, a quarter of them blending, 1054 -> 1051 us).
 #define SPRITE_THREADS 256
 #define SPRITE_TILE_W 16      // columns of a wavefront's tile: 8 to 64 within 3 %
 #define SPRITE_TILE_H (64 / SPRITE_TILE_W)
@@ -4413,19 +4413,21 @@ __global__ void __launch_bounds__(LIST_THREADS) sprite_list_kernel(DeviceMap dm,
 #define SPRITE_COLUMNS 64     // a work-group for the whole lane: 0.95 ms instead of 0.70 (4 wavefronts), 0.86 (8)
 static_assert(SPRITE_COLUMNS == 64 && SW % SPRITE_COLUMNS == 0 && VH % (SPRITE_ROW_PARTS * SPRITE_TILE_H) == 0 && VH <= SPRITE_THREADS, "sprite_pixels_kernel: whole tiles");
 static_assert(SPRITE_CHUNK == 64 && SPRITE_CHUNK <= SPRITE_THREADS, "sprite_pixels_kernel: a bit an entry");
-__global__ void __launch_bounds__(SPRITE_THREADS, 5) sprite_pixels_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
-                                                                          unsigned char *frame_base, size_t frame_stride, int lane_pick) {
+template <int PHASE, bool BLENDS>
+__global__ void __launch_bounds__(SPRITE_THREADS, PHASE == SPRITES_EARLY && BLENDS ? 4 : 5) sprite_pixels_kernel(DeviceMap dm, gd_lanes_desc lanes, int lane_base, int lane_count, Scratch sc,
+                                                                          unsigned char *frame_base, size_t frame_stride) {
     __shared__ SpriteRec sp[SPRITE_CHUNK];         // the chunk's records, near to far
     __shared__ u64 cover[SPRITE_COLUMNS], in_row[VH];
     __shared__ unsigned short picked[SPRITE_SLOTS_MAX];   // the records of the billboards that reach the group's columns and rows, near to far
-    __shared__ int wave_picks[SPRITE_SLOTS_MAX / 64], next_tile;
+    __shared__ int wave_picks[SPRITE_SLOTS_MAX / 64], next_tile, left_over;
     const int local = blockIdx.y;
     if (local >= lane_count) return;
-    // lane_pick: LANES_ALL, or one half of launch_chunk's split: LANES_PLAIN (lanes whose billboards all simply cover what is
-    // under them: painted early, marking the gap pixels they take) or LANES_BLENDING (the others, after the flat pass)
-    const bool blends = sc.lane_blends[local] != 0;
-    if (lane_pick != LANES_ALL && blends != (lane_pick == LANES_BLENDING)) return;   // the same in the whole block
-    const bool mark_gaps = lane_pick == LANES_PLAIN;
+    // SPRITES_EARLY: all but gap pixels that show billboards which blend, and none that covers, since what is under them is not painted yet.
+    // SPRITES_LATE: those, in the groups that have any.
+    const bool blends = BLENDS && sc.lane_blends[local] != 0;
+    const auto late = [&]() -> unsigned char & { return sc.sprite_late[((size_t)local * (SW / SPRITE_COLUMNS) + blockIdx.x) * SPRITE_ROW_PARTS + blockIdx.z]; };
+    if (PHASE == SPRITES_LATE && (!blends || late() == 0)) return;     // the same in the whole block
+    if (PHASE == SPRITES_EARLY && blends && threadIdx.x == 0) { late() = 0; left_over = 0; }
     const gd_map_desc *m = &dm.d;
     const int n = lane_base + local, tid = threadIdx.x;
     const int rows = VH / gridDim.z;
@@ -4523,6 +4525,8 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 5) sprite_pixels_kernel(Device
                 const int t = t0 + j;
                 const int x = x_first + t % TILES_ACROSS * SPRITE_TILE_W + tile_x, y = row_first + t / TILES_ACROSS * SPRITE_TILE_H + tile_y;
                 const unsigned int pixel_word = pixel_words[j];
+                const bool open_gap = gap_pixel(pixel_word) && !(pixel_word & META_GAP_COVERED);
+                if (PHASE == SPRITES_LATE && !open_gap) continue;
                 PixelClip clip;
                 clip.set(dm, sc, local, L, pixel_word, y);
                 unsigned char *pixel = frame + (size_t)y * SW + x;
@@ -4569,6 +4573,7 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 5) sprite_pixels_kernel(Device
                         const SpriteRec &s = sp[bit];
                         const int lit = colour(s);
                         if (lit < 0) continue;
+                        if (!below_known && PHASE == SPRITES_EARLY && open_gap) { left_over = 1; break; }
                         if (!below_known) { value = *pixel; below_known = true; }
                         value = sprite_blend(m, (int)(signed char)(s.flags >> 8), (unsigned char)lit, (unsigned char)value);
                     }
@@ -4576,10 +4581,13 @@ __global__ void __launch_bounds__(SPRITE_THREADS, 5) sprite_pixels_kernel(Device
                 if (value < 0) continue;
                 *pixel = (unsigned char)value;
                 // painted ahead of the flat pass's pixels (launch_chunk): a gap pixel says that it is taken
-                if (mark_gaps && gap_pixel(pixel_word)) meta[(size_t)y * SW + x] = pixel_word | META_GAP_COVERED;
+                if (PHASE == SPRITES_EARLY && open_gap) meta[(size_t)y * SW + x] = pixel_word | META_GAP_COVERED;
             }
         }
     }
+    if (PHASE != SPRITES_EARLY || !blends) return;
+    __syncthreads();
+    if (tid == 0 && left_over) late() = 1;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -5857,6 +5865,7 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.block_hit, L * SW);
     take(&sc.sprite_listed, L);
     take(&sc.lane_blends, L);
+    take(&sc.sprite_late, L * (SW / SPRITE_COLUMNS) * SPRITE_ROW_PARTS);
     take(&sc.strip_key, L * SEGS_PER_LANE);
     take(&sc.strip_order, L * SEGS_PER_LANE);
     if (depth) take(&sc.scene_depth, L * PX);
@@ -6122,24 +6131,29 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     mark();
     hipLaunchKernelGGL(level_masks ? flat_tail_kernel<true> : flat_tail_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, count, sc);
     hipLaunchKernelGGL(flat_span_finish_kernel, flat_grid(2, 1024), dim3(FINISH_THREADS), 0, stream, sc);
-    // Billboards that simply cover what lies under them need not wait for the flat pass's pixels: the lanes that hold no other
-    // kind (lane_blends, decided on the device) have theirs painted right after the shading, on the side stream, where they
-    // mark the gap pixels they take; the flat pass's pixels of those lanes are painted after the join, around the marks.  The
-    // flat chain, which waits for memory most of its time, then has the billboards beside it as well as the shading.  Lanes
-    // with a billboard that blends with the pixel below (sprite_style) keep the order flat pass, then billboards; so do
-    // frames with decals, which go between the two.
+    // Billboards need not wait for the flat pass's pixels, but where one blends with such a pixel (sprite_style): they are painted right after the
+    // shading, on the side stream, and mark the gap pixels they take; the flat pass's pixels are painted after the join, around the marks, and the
+    // few that are blended with after these.  The flat chain, which waits for memory most of its time, then has the billboards beside it
+    // as well as the shading.  (When the lanes with any billboard that blends waited with all of theirs: 1024 lanes on the 2000-linedef map, a
+    // quarter of them so, 1094 us; now 1050.)  In frames with decals, which go between the flat pass and the billboards, all wait: to paint
+    // early what covers, and to mark it for the decals, leaves so much to the late launch that 2048 lanes take 2146 us instead of 2102.
     const bool billboards_split = beside && has_billboards && !decals;
-    const bool may_blend = lanes->sprite_style != nullptr;   // without styles no lane blends: the launches for such lanes are left out
-    auto paint_billboards = [&](hipStream_t on, int lane_pick) {
-        hipLaunchKernelGGL(sprite_pixels_kernel, dim3(SW / SPRITE_COLUMNS, count, sprite_row_parts(count)), dim3(SPRITE_THREADS), 0, on, r->dm, *lanes, base, count, sc, frame_base, frame_stride, lane_pick);
+    const bool left_over = billboards_split && lanes->sprite_style != nullptr;   // may the early launch leave pixels?
+    auto paint_billboards = [&](hipStream_t on, int phase) {
+        const bool blends = lanes->sprite_style != nullptr;
+        auto kernel = phase == SPRITES_LATE ? sprite_pixels_kernel<SPRITES_LATE, true>
+                      : phase == SPRITES_EARLY ? (blends ? sprite_pixels_kernel<SPRITES_EARLY, true> : sprite_pixels_kernel<SPRITES_EARLY, false>)
+                                               : (blends ? sprite_pixels_kernel<SPRITES_ALL, true> : sprite_pixels_kernel<SPRITES_ALL, false>);
+        hipLaunchKernelGGL(kernel, dim3(SW / SPRITE_COLUMNS, count, sprite_row_parts(count)), dim3(SPRITE_THREADS), 0, on, r->dm, *lanes, base, count, sc, frame_base, frame_stride);
     };
-    if (!fused && !(billboards_split && !may_blend)) hipLaunchKernelGGL(flat_shade_kernel, flat_grid(4, 4096), dim3(64), 0, stream, r->dm, sc, frame_base, frame_stride, billboards_split ? LANES_BLENDING : LANES_ALL);
+    auto shade_gaps = [&]() { hipLaunchKernelGGL(flat_shade_kernel, flat_grid(4, 4096), dim3(64), 0, stream, r->dm, sc, frame_base, frame_stride); };
+    if (!fused && !billboards_split) shade_gaps();
     if (beside) {
         shade_planes();
-        if (billboards_split) paint_billboards(r->side_stream, LANES_PLAIN);
+        if (billboards_split) paint_billboards(r->side_stream, SPRITES_EARLY);
         HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
         HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
-        if (billboards_split) hipLaunchKernelGGL(flat_shade_kernel, flat_grid(4, 4096), dim3(64), 0, stream, r->dm, sc, frame_base, frame_stride, LANES_PLAIN);
+        if (billboards_split) shade_gaps();
     }
     mark();
     const float *blend = lanes->screen_blend ? lanes->screen_blend + 2 * (size_t)base : nullptr;
@@ -6167,7 +6181,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     if (decals)
         hipLaunchKernelGGL(decal_kernel, dim3(count), dim3(SW), 0, stream, r->dm, r->overlays, *lanes, base, count, sc, frame_base, frame_stride);
     if (has_billboards && timed) list_billboards(stream);
-    if (has_billboards && !(billboards_split && !may_blend)) paint_billboards(stream, billboards_split ? LANES_BLENDING : LANES_ALL);
+    if (has_billboards && (!billboards_split || left_over)) paint_billboards(stream, billboards_split ? SPRITES_LATE : SPRITES_ALL);
     if (lanes->weapon_state && r->overlays.d.weapon_patch_count > 0)
         hipLaunchKernelGGL(weapon_overlay_kernel, dim3(WEAPON_PARTS, count), dim3(WEAPON_THREADS), 0, stream, r->overlays, lanes->weapon_state, base, count,
                            frame_base, frame_stride);

@@ -84,3 +84,42 @@ def test_eight_chunks_of_billboards_in_one_strip_match_the_oracle(oracle, copies
     assert renderer.status() == 0
     assert torch.equal(indexed.cpu(), expected.repeat(copies, 1, 1))
     renderer.close()
+
+
+@pytest.mark.parametrize("slots", [6, 100])
+@pytest.mark.parametrize("styles", [(0,), (-2, 1), (-1, 0, -2)])
+def test_billboards_that_blend_over_the_flat_passes_pixels_match_the_oracle(oracle, slots, styles):
+    """Cameras in the void look at billboards in front of the map: nothing is drawn below most of their pixels until the flat pass has been, which the
+    early launch leaves to the late one; more of them than a chunk holds, and opaque ones among them."""
+
+    from gradoom_amd import hostmath, mapbuild, synthmap
+    from gradoom_amd.renderer import HipRenderer, LaneState
+    from gradoom_amd.selfcheck import make_lane_arrays
+
+    lanes = 6
+    smap = synthmap.with_variant(synthmap.generate_map(81, grid=(6, 5), sectors=26, linedefs=180), 82, heights="uniform")
+    smap = synthmap.with_blend_tables(smap, 83)
+    poses = synthmap.generate_poses(smap, lanes, 84, margin=0.02)
+    segments = np.asarray(smap.wall_segments, dtype=np.float64)
+    rng = np.random.default_rng(85)
+    poses.x[:4], poses.y[:4], poses.angle_bam[:4] = segments[:, [0, 2]].min() - 160, segments[:, [1, 3]].mean() + 40 * np.arange(4), 0
+    sprites = synthmap.generate_sprites(smap, lanes, slots, 86)
+    sprites.x[:4] = poses.x[:4, None] + rng.integers(30, 130, (4, slots))
+    sprites.y[:4] = poses.y[:4, None] + rng.integers(-40, 41, (4, slots))
+    sprites.z[:4] = poses.view_z[:4, None] - rng.integers(0, 60, (4, slots))
+    arrays = make_lane_arrays(smap, poses, sprites)
+    arrays["sprite_style"] = rng.choice(np.asarray(styles, dtype=np.int8), size=(lanes, slots))
+    tables = mapbuild.build_map_tables(smap)
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    expected = oracle.render(tables, arrays, cosine)["indexed"]
+    opaque = oracle.render(tables, dict(arrays, sprite_style=np.full((lanes, slots), -1, dtype=np.int8)), cosine)["indexed"]
+    assert (expected[:4] != opaque[:4]).sum() > 1000     # blending shows
+    renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+    indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+    for _ in range(2):
+        renderer.scribble(0xA5)
+        renderer.render(LaneState.from_numpy(arrays, "cuda:0"), indexed=indexed)
+        torch.cuda.synchronize()
+        assert renderer.status() == 0
+        assert np.array_equal(indexed.cpu().numpy(), expected)
+    renderer.close()
