@@ -1779,14 +1779,21 @@ __device__ __forceinline__ size_t flat_sample_tabled(const Tables &tb, const Lan
 // flat_sample_tabled for neighbouring pixels of one row that show the same plane.  Of distance * (base + x * step) only bits 16..47 are
 // looked at, and distance * base + x * (distance * step) is the same number modulo 2^48: both products are worked out once
 // for the run, and a pixel costs two 24-bit multiply-adds an axis.
+// a * b + c of 24-bit factors, whatever lies above their 24 bits.  Written out: where only the sum's lower 24 bits are used the compiler
+// takes a 32-bit multiplication, which runs at a quarter of the rate.
+__device__ __forceinline__ unsigned mad24(unsigned a, unsigned b, unsigned c) {
+    unsigned sum;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(sum) : "v"(a), "v"(b), "v"(c));
+    return sum;
+}
 struct PlaneSpan {
     uint4 start;         // the fraction at the strip's first column, its lower and upper 24 bits: horizontal, then vertical
     uint4 step;          // what a column adds, likewise; the four upper bytes: 24 - log2 width, colormap row, 24 - log2 height, nothing
     unsigned texture;    // the texture's first texel in the atlas (which is below 4 GiB: checked at create)
     // the texel `column` (0..63) columns into the strip
     __device__ __forceinline__ unsigned texel(unsigned column, unsigned atlas_width) const {
-        const unsigned x = __umul24(step.y, column) + start.y + ((__umul24(step.x, column) + start.x) >> 24);
-        const unsigned y = __umul24(step.w, column) + start.w + ((__umul24(step.z, column) + start.z) >> 24);
+        const unsigned x = mad24(step.y, column, start.y) + (mad24(step.x, column, start.x) >> 24);
+        const unsigned y = mad24(step.w, column, start.w) + (mad24(step.z, column, start.z) >> 24);
         return texture + __umul24((y & 0xFFFFFFu) >> (step.z >> 24), atlas_width) + ((x & 0xFFFFFFu) >> (step.x >> 24));
     }
     __device__ __forceinline__ unsigned colormap_row() const { return step.y >> 24; }
@@ -3981,14 +3988,15 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
 // ---------------------------------------------------------------------------------------------
 // A wavefront takes a tile of 64 columns and SHADE_ROWS rows, a column a lane.  Everything but the texel is the same along a run of
 // pixels of a row that show one plane: each run's leftmost pixel is listed, a lane works out each listed run (PlaneSpan, one pass for
-// up to 64 of them: a tile has some forty), and its pixels read it back from LDS.  Bound by the per-pixel words in, gathers from the
-// textures and LDS; a work-group is four tiles (all of a lane's by two work-groups: 0.41 ms, five tiles 0.44, stores of four columns' words 0.54).
-// 4096 lanes on the 4000-linedef map: 0.69 ms with a run of four pixels a thread (three times the vector instructions, each plane of the
-// four worked out again), 0.38 now; 1024 lanes 0.202 -> 0.106, 16 lanes 0.043 -> 0.013.
+// up to 64 of them: a tile has some forty), and its pixels read it back from LDS.  Bound by the per-pixel words in and the pixels out (1.4 GB at 4096
+// lanes, 4.1 of the 5.2 TB/s of a copy), then by its vector instructions; a work-group is four tiles (all of a lane's by two work-groups: 0.41 ms,
+// five tiles 0.44, stores of four columns' words 0.54).  4096 lanes on the 4000-linedef map: 0.69 ms with a run of four pixels a thread (each plane
+// of the four worked out again), 0.374 at 717 vector instructions a tile, 0.342 now at 533 (the compiler's 32-bit multiplications as 24-bit ones,
+// no branch a pixel, a run's number that needs no range test); 16 lanes 0.043, 0.010, 0.009.
 #define SHADE_ROWS 16
 #define SHADE_BATCH 4        // rows whose texels are asked for together
 #define RUN_NONE 0x7FFu      // the number of a pixel's run, or that it has none (a tile has at most 1024)
-#define RUN_BEGINS 0x8000u
+#define RUN_ROUND 0x7C0u     // the first run of the round that works it out
 #define SHADE_THREADS 256
 #define SHADE_TILES ((SW / 64) * (VH / SHADE_ROWS))      // a lane's; a wavefront takes one
 static_assert(SW % 64 == 0 && VH % SHADE_ROWS == 0 && SHADE_ROWS <= 16, "plane_shade_kernel: whole tiles, of at most 1024 runs");
@@ -3997,12 +4005,13 @@ __global__ void __launch_bounds__(SHADE_THREADS) __attribute__((amdgpu_waves_per
     const gd_map_desc *m = &dm.d;
     constexpr int WAVES = SHADE_THREADS / 64;
     __shared__ __align__(16) unsigned char colormap_lds[32 * 256];
-    __shared__ uint4 start_lds[WAVES][64], step_lds[WAVES][64];
-    __shared__ unsigned int texture_lds[WAVES][64];     // a listed run, until its lane puts the run's texture there
+    struct Runs { uint4 start[64], step[64]; unsigned int texture[64]; };      // a listed run in `texture`, until its lane puts the run's texture there
+    __shared__ Runs runs_lds[WAVES];
     const int local = blockIdx.y;
     if (local >= lane_count) return;     // uniform over the block
     const LaneCtx &c = sc.ctx[local];
     const int lane_id = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    Runs &runs = runs_lds[wave];
     unsigned char *frame = frame_base + (size_t)local * frame_stride;
     // the lane's words and view pixels as buffers: a pixel that is not this kernel's is stored beyond the end, which the hardware drops
     // (with a branch around every store the rows' addresses and masks alone would fill the registers)
@@ -4025,52 +4034,59 @@ __global__ void __launch_bounds__(SHADE_THREADS) __attribute__((amdgpu_waves_per
         else for (int k = 0; k < 4; ++k) bar[k] = 0;
     }
     if (tile >= SHADE_TILES) return;     // the last work-group's spare wavefronts; their words lay beyond the buffer
-    // Each pixel's word becomes: what names its plane, the number of its run, whether it begins the run; or a tier's colour.
+    // Each pixel's word becomes: what names its plane and the number of its run; or a tier's colour and RUN_NONE.
     int total = 0;
 #pragma unroll
     for (int r = 0; r < SHADE_ROWS; ++r) {
         // no run where no plane shows (a wall tier, a masked texture, or neither tier nor plane: the flat pass's picture, which
         // flat_shade_kernel paints once that pass has run)
-        const unsigned int word = meta[r];
-        const bool plane = !(word & (META_FILLED | META_MASKED)) && (word & (META_SECTOR_MASK << META_SECTOR_SHIFT));
-        const unsigned int key = plane ? word & PLANE_KEY : 0u;
-        const unsigned int left = (unsigned)__builtin_amdgcn_update_dpp(0, (int)key, 0x138 /* wave_shr:1 */, 0xF, 0xF, false);
-        const u64 begins = __ballot(key != 0u && key != left), before = begins >> 1;
+        const unsigned int word = (meta[r] & META_MASKED) ? 0u : meta[r] & (META_FILLED | PLANE_KEY);
+        const unsigned int key = (unsigned)max((int)word, 0);      // a tier's word is negative, that of neither tier nor plane is zero
+        const unsigned int left = (unsigned)__builtin_amdgcn_update_dpp(0, (int)key, 0x138 /* wave_shr:1 */, 0xF, 0xF, true);
+        const bool plane = key != 0u;
+        const u64 begins = __builtin_amdgcn_ballot_w64(plane) & __builtin_amdgcn_ballot_w64(key != left), before = begins >> 1;
         const int run = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(before >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)before, 0u)) + (total + (int)(begins & 1) - 1);
-        const bool tier = (word & (META_FILLED | META_MASKED)) == META_FILLED;
-        meta[r] = plane ? key | (unsigned)run | (key != left ? RUN_BEGINS : 0u) : (tier ? (word & (META_FILLED | (META_SECTOR_MASK << META_SECTOR_SHIFT))) : 0u) | RUN_NONE;
-        if (key != 0u && key != left && run < 64) texture_lds[wave][run] = key | (unsigned)r;
+        meta[r] = word | (plane ? (unsigned)run : RUN_NONE);
+        if (__builtin_amdgcn_inverse_ballot_w64(begins) && run < 64) runs.texture[run] = key | (unsigned)r;
         total += __popcll(begins);
     }
     for (unsigned first = 0;;) {     // one round, but for the most varied tiles
         wave_lds_fence();
-        if (first + lane_id < (unsigned)total) {
-            const unsigned int listed = texture_lds[wave][lane_id];
-            const PlaneSpan span = plane_span(dm, sc, c, local, (int)((listed >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1, (listed & META_FLOOR) != 0, x_first, y_first + (int)(listed & 0xFFFFu));
-            start_lds[wave][lane_id] = span.start; step_lds[wave][lane_id] = span.step; texture_lds[wave][lane_id] = span.texture;
+        {
+            PlaneSpan span = {};                 // lanes without a run leave one whose texel is the atlas's first: pixels without one ask for it
+            if (first + lane_id < (unsigned)total) {
+                const unsigned int listed = runs.texture[lane_id];
+                span = plane_span(dm, sc, c, local, (int)((listed >> META_SECTOR_SHIFT) & META_SECTOR_MASK) - 1, (listed & META_FLOOR) != 0, x_first, y_first + (int)(listed & 0xFFFFu));
+            }
+            runs.start[lane_id] = span.start; runs.step[lane_id] = span.step; runs.texture[lane_id] = span.texture;
         }
         wave_lds_fence();
 #pragma unroll
         for (int r0 = 0; r0 < SHADE_ROWS; r0 += SHADE_BATCH) {
-            unsigned shade_at[SHADE_BATCH]; unsigned char texel[SHADE_BATCH];
-            bool any = false;
+            bool here[SHADE_BATCH], any = false;     // is the pixel's run one of this round's
 #pragma unroll
-            for (int j = 0; j < SHADE_BATCH; ++j) { any |= (meta[r0 + j] & RUN_NONE) - first < 64u; shade_at[j] = 0u; texel[j] = 0; }
+            for (int j = 0; j < SHADE_BATCH; ++j) { here[j] = (meta[r0 + j] & RUN_ROUND) == first; any |= here[j]; }
             if (__any(any)) {
+                unsigned shade_at[SHADE_BATCH]; unsigned char texel[SHADE_BATCH];
 #pragma unroll
                 for (int j = 0; j < SHADE_BATCH; ++j) {
-                    unsigned run = (meta[r0 + j] & RUN_NONE) - first;
-                    run = run < 64u ? run : 0u;        // a pixel without one asks for a texel of the first run's: in the atlas too
+                    const unsigned run = meta[r0 + j] & 63u;
                     PlaneSpan span;
-                    span.start = start_lds[wave][run]; span.step = step_lds[wave][run]; span.texture = texture_lds[wave][run];
+                    span.start = runs.start[run]; span.step = runs.step[run]; span.texture = runs.texture[run];
                     texel[j] = m->tex_atlas[span.texel((unsigned)lane_id, atlas_width)];
                     shade_at[j] = span.colormap_row() * 256;
                 }
-            }
+                __builtin_amdgcn_sched_barrier(0);   // all of the batch's texels are asked for before the first is looked at
 #pragma unroll
-            for (int j = 0; j < SHADE_BATCH; ++j) {
-                const bool tier = (meta[r0 + j] & META_FILLED) && first == 0;
-                put(tier || (meta[r0 + j] & RUN_NONE) - first < 64u, r0 + j, tier ? meta[r0 + j] >> META_SECTOR_SHIFT : colormap_lds[shade_at[j] + texel[j]]);
+                for (int j = 0; j < SHADE_BATCH; ++j) {
+                    unsigned colour = colormap_lds[shade_at[j] + texel[j]];
+                    asm volatile("" : "+v"(colour));   // looked up for all pixels: a branch around it costs more
+                    const bool tier = (int)meta[r0 + j] < 0;
+                    put(here[j] || (tier && first == 0), r0 + j, tier ? meta[r0 + j] >> META_SECTOR_SHIFT : colour);
+                }
+            } else if (first == 0) {
+#pragma unroll
+                for (int j = 0; j < SHADE_BATCH; ++j) put((int)meta[r0 + j] < 0, r0 + j, meta[r0 + j] >> META_SECTOR_SHIFT);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -4080,8 +4096,9 @@ __global__ void __launch_bounds__(SHADE_THREADS) __attribute__((amdgpu_waves_per
 #pragma unroll
         for (int r = 0; r < SHADE_ROWS; ++r) {
             asm volatile("" : "+v"(meta[r]));      // worked on afresh in every round: kept over the rounds, its derivatives would fill the registers
+            const unsigned int left = (unsigned)__builtin_amdgcn_update_dpp((int)RUN_NONE, (int)meta[r], 0x138 /* wave_shr:1 */, 0xF, 0xF, false);
             const unsigned run = (meta[r] & RUN_NONE) - first;
-            if ((meta[r] & RUN_BEGINS) && run < 64u) texture_lds[wave][run] = (meta[r] & PLANE_KEY) | (unsigned)r;
+            if (((left ^ meta[r]) & RUN_NONE) && run < 64u) runs.texture[run] = (meta[r] & PLANE_KEY) | (unsigned)r;
         }
     }
 }
