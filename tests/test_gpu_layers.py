@@ -128,3 +128,44 @@ def test_status_bars_of_every_kind_of_number_match_the_oracle(oracle, assembly, 
     torch.cuda.synchronize()
     assert np.array_equal(indexed.cpu().numpy(), expected)
     renderer.close()
+
+
+@pytest.mark.parametrize("slots, chips", [(1, 1), (63, 40), (64, 64), (65, 65), (200, 150)])
+def test_chips_in_any_number_of_slots_match_the_oracle(oracle, slots, chips):
+    """A chunk of decal_kernel is 64 slots; the chips of several chunks are painted in the order of their slots all the same."""
+    import sys
+    import types
+
+    from conftest import ROOT
+    from gradoom_amd import hostmath, overlay_inputs, synthmap
+    from gradoom_amd.renderer import HipRenderer, LaneState
+
+    sys.path.insert(0, f"{ROOT}/tests/golden")
+    import refdrive
+
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    overlays = synthmap.generate_overlays(34)
+    lanes = 4
+    smap, tables, arrays = closed_door_case(303, lanes)
+    engine = types.SimpleNamespace(num_envs=lanes, hitscan_decal_slots=slots, **{name: arrays[name] for name in ("x", "y", "angle", "view_z")})
+    for name, dtype, value in (("wall", torch.int64, 0), ("along", torch.float32, 0), ("z", torch.float32, 0), ("style", torch.int64, 0), ("serial", torch.int64, -1)):
+        setattr(engine, "hitscan_decal_" + name, torch.full((lanes, slots), value, dtype=dtype))
+    refdrive.set_decals(engine, smap, 35, per_lane=chips)
+    state, geometry = overlay_inputs.decal_inputs(
+        engine.hitscan_decal_serial, engine.hitscan_decal_wall, engine.hitscan_decal_along, engine.hitscan_decal_z, engine.hitscan_decal_style,
+        torch.as_tensor(np.asarray(tables["walls"], dtype=np.float32)), overlay_inputs.fine_sine_fixed(),
+    )
+    bare = oracle.render(tables, arrays, cosine)["indexed"]
+    arrays["decal_state"], arrays["decal_geom"] = state.numpy(), geometry.numpy()
+    oracle.set_overlays(overlays)
+    expected = oracle.render(tables, arrays, cosine)["indexed"]
+    oracle.set_overlays(None)
+    assert slots == 1 or (expected != bare).any()
+    renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+    renderer.set_overlays(overlays)
+    indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+    renderer.render(LaneState.from_numpy(arrays, "cuda:0"), indexed=indexed)
+    torch.cuda.synchronize()
+    assert renderer.status() == 0
+    assert np.array_equal(indexed.cpu().numpy(), expected)
+    renderer.close()
