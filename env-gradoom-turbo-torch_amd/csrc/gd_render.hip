@@ -1620,24 +1620,34 @@ __global__ void __launch_bounds__(64 * GAP_WAVES) flat_gap_kernel(DeviceMap dm, 
 }
 
 // The lanes' row ranges are final once every listed column is repaired: their rows join the work list that
-// flat_span_select_kernel deals out evenly, whichever lanes they come from, and those below them flat_tail_kernel's.  One wavefront per lane.
-__global__ void __launch_bounds__(64) flat_rows_kernel(int lane_count, Scratch sc) {
-    const int local = blockIdx.x;
-    if (local >= lane_count) return;
-    const int *span = sc.flat_span + (size_t)local * 4;
-    const int lo0 = span[0], hi0 = span[1], lo1 = span[2], hi1 = span[3];
+// flat_span_select_kernel deals out evenly, whichever lanes they come from, and those below them flat_tail_kernel's.  One wavefront per lane; a
+// work-group takes room in the lists for all of its lanes at once (each for itself: 18 us where half of 2048 lanes have rows, now 12; by sixteen lanes a
+// work-group 6, but at 4096 lanes such a one waits 0.2 ms for room beside the shading).
+#define ROWS_LANES 4
+__global__ void __launch_bounds__(64 * ROWS_LANES) flat_rows_kernel(int lane_count, Scratch sc) {
+    __shared__ int wanted[2][ROWS_LANES], base[2];
+    const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63, local = blockIdx.x * ROWS_LANES + wave;
+    int lo0 = VH, hi0 = -1, lo1 = VH, hi1 = -1, last_ceiling_row = 0;
+    if (local < lane_count) {
+        const int4 span = *reinterpret_cast<const int4 *>(sc.flat_span + (size_t)local * 4);
+        lo0 = span.x; hi0 = span.y; lo1 = span.z; hi1 = span.w;
+        last_ceiling_row = sc.ctx[local].last_ceiling_row;
+    }
     const int rows0 = hi0 < lo0 ? 0 : hi0 - lo0 + 1, rows1 = hi1 < lo1 ? 0 : hi1 - lo1 + 1;
-    if (rows0 + rows1 == 0) return;                  // the same in every thread
-    const int below0 = rows0 == 0 ? 0 : sc.ctx[local].last_ceiling_row - hi0, below1 = rows1 == 0 ? 0 : VH - 1 - hi1;
-    int list_base = 0;
-    if (threadIdx.x < 2) list_base = atomicAdd(&sc.flat_row_count[threadIdx.x], threadIdx.x == 0 ? rows0 + rows1 : below0 + below1);
-    int *below = sc.flat_rows + (size_t)lane_count * VH - 1 - __shfl(list_base, 1);
-    list_base = __shfl(list_base, 0);
-    for (int r = threadIdx.x; r < rows0 + rows1; r += blockDim.x)
-        sc.flat_rows[list_base + r] = (local << 8) | (r < rows0 ? lo0 + r : lo1 + (r - rows0));
-    for (int r = threadIdx.x; r < below0 + below1; r += blockDim.x)
-        below[-r] = (local << 8) | (r < below0 ? hi0 + 1 + r : hi1 + 1 + (r - below0));
-    for (int x = threadIdx.x; x < 2 * SW; x += blockDim.x)
+    const int below0 = rows0 == 0 ? 0 : last_ceiling_row - hi0, below1 = rows1 == 0 ? 0 : VH - 1 - hi1;
+    if (lane_id == 0) { wanted[0][wave] = rows0 + rows1; wanted[1][wave] = below0 + below1; }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        int total = 0;
+        for (int k = 0; k < ROWS_LANES; ++k) { const int own = wanted[threadIdx.x][k]; wanted[threadIdx.x][k] = total; total += own; }
+        base[threadIdx.x] = total ? atomicAdd(&sc.flat_row_count[threadIdx.x], total) : 0;
+    }
+    __syncthreads();
+    if (rows0 + rows1 == 0) return;                  // the same in the whole wavefront
+    int *rows = sc.flat_rows + base[0] + wanted[0][wave], *below = sc.flat_rows + (size_t)lane_count * VH - 1 - (base[1] + wanted[1][wave]);
+    for (int r = lane_id; r < rows0 + rows1; r += 64) rows[r] = (local << 8) | (r < rows0 ? lo0 + r : lo1 + (r - rows0));
+    for (int r = lane_id; r < below0 + below1; r += 64) below[-r] = (local << 8) | (r < below0 ? hi0 + 1 + r : hi1 + 1 + (r - below0));
+    for (int x = lane_id; x < 2 * SW; x += 64)
         if (x < SW ? rows0 > 0 : rows1 > 0) sc.flat_tail[(size_t)local * 2 * SW + x] = ~0u;
 }
 
@@ -6173,7 +6183,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     const int waves = gap_waves(count);
     hipLaunchKernelGGL(waves == 16 ? flat_gap_kernel<16> : (waves == 8 ? flat_gap_kernel<8> : flat_gap_kernel<4>), flat_grid(8, 16384 / waves), dim3(64 * waves), 0, stream,
                        r->dm, *lanes, base, sc);
-    hipLaunchKernelGGL(flat_rows_kernel, dim3(count), dim3(64), 0, stream, count, sc);
+    hipLaunchKernelGGL(flat_rows_kernel, dim3((count + ROWS_LANES - 1) / ROWS_LANES), dim3(64 * ROWS_LANES), 0, stream, count, sc);
     hipLaunchKernelGGL(level_masks ? flat_span_select_kernel<true> : flat_span_select_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, sc);
     mark();
     hipLaunchKernelGGL(level_masks ? flat_tail_kernel<true> : flat_tail_kernel<false>, flat_grid(16, 2048), dim3(256), 0, stream, r->dm, *lanes, base, count, sc);
