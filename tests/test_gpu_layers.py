@@ -130,7 +130,7 @@ def test_status_bars_of_every_kind_of_number_match_the_oracle(oracle, assembly, 
     renderer.close()
 
 
-@pytest.mark.parametrize("slots, chips", [(1, 1), (63, 40), (64, 64), (65, 65), (200, 150)])
+@pytest.mark.parametrize("slots, chips", [(3, 1), (63, 40), (64, 40), (65, 40), (200, 130)])
 def test_chips_in_any_number_of_slots_match_the_oracle(oracle, slots, chips):
     """A chunk of decal_kernel is 64 slots; the chips of several chunks are painted in the order of their slots all the same."""
     import sys
@@ -160,7 +160,7 @@ def test_chips_in_any_number_of_slots_match_the_oracle(oracle, slots, chips):
     oracle.set_overlays(overlays)
     expected = oracle.render(tables, arrays, cosine)["indexed"]
     oracle.set_overlays(None)
-    assert slots == 1 or (expected != bare).any()
+    assert chips == 1 or (expected != bare).any()
     renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
     renderer.set_overlays(overlays)
     indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
