@@ -1262,7 +1262,8 @@ __device__ __forceinline__ int flat_probe_group(const DeviceMap &dm, const Scrat
     const float delta = (float)y - flat_center(c);
     const bool is_floor = delta > 0;
     const float denom = fmaxf(fabsf(delta), 0.5f), cc = dm.cosine_correction[x];
-    const float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x];
+    float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x];
+    asm volatile("" : "+v"(rc), "+v"(rs));    // waited for here, not in every round behind its branches (flat_select_row)
     const LevelSide side = level_side(dm, sc, local, is_floor);
     const unsigned int *row = side.mask_words > 0 ? side.masks + level_bucket((192.0f / denom) / cc) * side.mask_words : nullptr;
     const u64 group_mask = ((1ULL << PROBE_LANES) - 1) << (group * PROBE_LANES), lower_lanes = (1ULL << lane_id) - 1;
@@ -1381,14 +1382,17 @@ __device__ __forceinline__ int flat_select_row(const DeviceMap &dm, const Scratc
     const float delta = (float)y - flat_center(c);
     const bool is_floor = __builtin_amdgcn_readfirstlane((int)(delta > 0)) != 0;   // the same in every lane, like the row
     const float denom = fmaxf(fabsf(delta), 0.5f);
-    const float cc = dm.cosine_correction[x];
-    const float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x];
+    float cc = dm.cosine_correction[x];
+    float rc = lanes.ray_cos[(size_t)n * SW + x], rs = lanes.ray_sin[(size_t)n * SW + x];
     const LevelSide side = level_side(dm, sc, local, is_floor);
     // cd = perpendicular / cc below is the hot division.  With y = RN(1 / cc), q = RN(p * y) is within
     // one ulp of p / cc, and RN(q + RN(p - cc * q) * y) is then the correctly rounded quotient
     // (Markstein's theorem; the inner product is exact in an FMA) as long as nothing over- or
     // underflows, which the range tests on both operands ensure.
-    const float inv_cc = dm.inverse_cosine[x];
+    float inv_cc = dm.inverse_cosine[x];
+    // Waited for here.  Where a probe first asks for one of them behind a branch, the compiler waits for all loads at every probe, the raster
+    // loads of the probes before among them, which then come one by one and not ROW_BATCH together.
+    asm volatile("" : "+v"(cc), "+v"(rc), "+v"(rs), "+v"(inv_cc));
     const bool cc_plain = cc >= 0.5f && cc <= 1.0f;
     const float inv_fine = dm.fine_inverse;       // a reciprocal is fine here: see fine_lookup_cells
     // the probe point camera + ray * cd in raster cell units, as one multiply-add per axis
