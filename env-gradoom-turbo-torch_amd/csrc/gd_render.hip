@@ -299,7 +299,7 @@ struct Scratch {    // per-chunk working memory, sized at create
     int *lane_blends;      // [L] does some live billboard of the lane blend with the pixel below it (sprite_style other than -1)?
                            // (lane_tables_kernel)
     unsigned char *sprite_late; // [L, SW / SPRITE_COLUMNS, SPRITE_ROW_PARTS] did this work-group of the billboards' early launch leave pixels to the
-                           // late one? (written for lanes that blend)
+                           // late one? (written for lanes that blend; in the memory of strip_order, which the walls are done with by then)
     unsigned char *strip_key;  // [L*SEGS_PER_LANE] expected traversal length of each (lane, segment of SEG_COLS columns)
     int *strip_order;      // [L*SEGS_PER_LANE] segments, longest expected traversal first
     volatile unsigned char *status;   // [2] sticky flags in pinned host memory: a candidate list, a list of passes was cut short
@@ -5926,9 +5926,10 @@ size_t carve_scratch(Scratch &sc, unsigned char *base, size_t L, const gd_map_de
     take(&sc.block_hit, L * SW);
     take(&sc.sprite_listed, L);
     take(&sc.lane_blends, L);
-    take(&sc.sprite_late, L * (SW / SPRITE_COLUMNS) * SPRITE_ROW_PARTS);
     take(&sc.strip_key, L * SEGS_PER_LANE);
     take(&sc.strip_order, L * SEGS_PER_LANE);
+    static_assert((SW / SPRITE_COLUMNS) * SPRITE_ROW_PARTS <= SEGS_PER_LANE * (int)sizeof(int), "Scratch::sprite_late: a byte a work-group");
+    sc.sprite_late = reinterpret_cast<unsigned char *>(sc.strip_order);
     if (depth) take(&sc.scene_depth, L * PX);
     take(&sc.frame, L * (size_t)GD_SCREEN_HEIGHT * SW);   // where a frame is put together kernel by kernel when the caller takes none
     return (used + 255) & ~(size_t)255;
