@@ -6185,7 +6185,7 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
     auto flat_grid = [count](int per_lane, int most) { return dim3((unsigned)(count >= most / per_lane ? most : (count * per_lane < 32 ? 32 : count * per_lane))); };
     const int plane_levels = m.floor_level_count + m.ceil_level_count;
     const bool level_masks = plane_levels > LEVEL_MASK_MIN_LEVELS && plane_levels <= 32 * LEVEL_MASK_WORDS_MAX;   // level_mask_words() > 0
-    const int waves = gap_waves(count);
+    const int waves = gap_waves(count, m.wall_count);
     hipLaunchKernelGGL(waves == 16 ? flat_gap_kernel<16> : (waves == 8 ? flat_gap_kernel<8> : flat_gap_kernel<4>), flat_grid(8, 16384 / waves), dim3(64 * waves), 0, stream,
                        r->dm, *lanes, base, sc);
     hipLaunchKernelGGL(flat_rows_kernel, dim3((count + ROWS_LANES - 1) / ROWS_LANES), dim3(64 * ROWS_LANES), 0, stream, count, sc);

@@ -114,7 +114,18 @@ inline bool raster_sixteen(int lanes) { return lanes <= 96; }
 //   1024   802 / 798 / 798 / 803 (815)  1025 /1004 /1010 /1026 (1031)   1532 /1520 /1491 /1531 (1512)    1049 /1061 /1125 /1144 (1172)
 //   2048  1260 /1260 /1266 /1285 (1278) 1624 /1632 /1639 /1696 (1659)   2347 /2338 /2346 /2404 (2371)    1721 /1737 /1833 /1888 (1870)
 //   4096  2188 /2199 /2201 /2241 (2248) 2864 /2881 /2939 /2955 (2965)   3851 /3856 /3922 /3985 (3870)    3001 /2995 /3166 /3264 (3205)
-inline int gap_waves(int lanes) { return lanes <= 384 ? 16 : (lanes <= 896 ? 8 : 4); }
+// Since the kernels behind it are shorter, a frame with 64 billboards with 4 / 8 / 16:
+//   lanes       320               800              1400             2000                4000
+//    400   432 / 431 / 427   466 / 470 / 469   526 / 548 / 577   560 / 545 / 544    823 / 799 / 786
+//    512   490 / 501 / 499   547 / 559 / 544   609 / 624 / 641   630 / 646 / 635    892 / 880 / 860
+//    640   573 / 581 / 581   616 / 625 / 609   717 / 746 / 755   714 / 725 / 713    985 / 978 / 968
+//    768   660 / 662 / 661   729 / 732 / 724   824 / 873 / 887   821 / 830 / 819   1156 /1148 /1154
+//   1024   765 / 765 / 758                     958 /1020 /1041   977 / 974 / 971   1340 /1310 /1341
+//   2048  1248 /1258 /1240                    1648 /1765 /1815  1606 /1610 /1640   2157 /2159 /2240
+inline int gap_waves(int lanes, int linedefs) {
+    if (linedefs >= 3000) return lanes <= 704 ? 16 : (lanes <= 1152 ? 8 : 4);
+    return lanes <= 384 ? 16 : (lanes <= 448 ? 8 : 4);
+}
 
 // sprite_pixels_kernel: work-groups that share the rows of a block of columns.  From 512 lanes on one takes them all: fewer listings, but the
 // last work-groups last longer.  Quarters and whole columns cost the same at 230 (4000 linedefs, 128 billboards) to 1100 lanes (320 linedefs,
