@@ -122,9 +122,11 @@ inline bool raster_sixteen(int lanes) { return lanes <= 96; }
 //    768   660 / 662 / 661   729 / 732 / 724   824 / 873 / 887   821 / 830 / 819   1156 /1148 /1154
 //   1024   765 / 765 / 758                     958 /1020 /1041   977 / 974 / 971   1340 /1310 /1341
 //   2048  1248 /1258 /1240                    1648 /1765 /1815  1606 /1610 /1640   2157 /2159 /2240
+// Asked of the lanes alone: what halves have while eight wavefronts or more of each still find room.
+inline int gap_waves(int lanes) { return lanes <= 384 ? 16 : 8; }
 inline int gap_waves(int lanes, int linedefs) {
     if (linedefs >= 3000) return lanes <= 704 ? 16 : (lanes <= 1152 ? 8 : 4);
-    return lanes <= 384 ? 16 : (lanes <= 448 ? 8 : 4);
+    return lanes <= 448 ? gap_waves(lanes) : 4;
 }
 
 // sprite_pixels_kernel: work-groups that share the rows of a block of columns.  From 512 lanes on one takes them all: fewer listings, but the

@@ -2,6 +2,10 @@
 
 from __future__ import annotations
 
+import os
+import subprocess
+import tempfile
+
 import pytest
 
 import launch_rules
@@ -24,3 +28,15 @@ def test_every_answer_is_one_the_launches_know(rule):
 
 def test_strips_of_a_screen_are_shared_in_whole_columns():
     assert all(64 % launch_rules.ask("raster_parts", lanes) == 0 for lanes in range(1, launch_rules.MOST_LANES + 1))
+
+
+def test_the_gap_columns_rule_can_be_asked_of_the_lanes_alone():
+    """Callers that know no map ask ``gap_waves(lanes)``: a kernel was built for every answer, and small maps' launches follow it as far as they share."""
+    source = '#include "gd_rules.h"\n#include <cstdio>\nint main() { for (int n = 1; n <= %d; ++n) printf("%%d ", gap_waves(n)); }\n' % launch_rules.MOST_LANES
+    with tempfile.TemporaryDirectory() as folder:
+        path = os.path.join(folder, "ask")
+        subprocess.run(["g++", "-std=c++17", "-x", "c++", "-I", launch_rules.CSRC, "-o", path, "-"], input=source, text=True, check=True)
+        answers = [int(word) for word in subprocess.run([path], capture_output=True, text=True, check=True).stdout.split()]
+    assert set(answers) == {8, 16}
+    for lanes, answer in enumerate(answers, start=1):
+        assert launch_rules.ask("gap_waves", lanes, 600) in (answer, 4)
