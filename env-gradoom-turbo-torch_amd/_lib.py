@@ -19,6 +19,8 @@ SYMBOLS = (
     "gd_renderer_destroy",
     "gd_renderer_status",
     "gd_renderer_status_seen",
+    "gd_renderer_mark_status",
+    "gd_renderer_wait_status",
     "gd_renderer_scribble",
     "gd_renderer_set_assembly",
     "gd_renderer_set_sector_lights",
@@ -79,6 +81,10 @@ def library() -> C.CDLL:
     lib.gd_renderer_status.argtypes = [C.c_void_p, C.POINTER(C.c_int32)]
     lib.gd_renderer_status_seen.restype = C.c_int
     lib.gd_renderer_status_seen.argtypes = [C.c_void_p, C.POINTER(C.c_int32)]
+    lib.gd_renderer_mark_status.restype = C.c_int
+    lib.gd_renderer_mark_status.argtypes = [C.c_void_p]
+    lib.gd_renderer_wait_status.restype = C.c_int
+    lib.gd_renderer_wait_status.argtypes = [C.c_void_p, C.c_void_p]
     lib.gd_renderer_set_assembly.restype = C.c_int
     lib.gd_renderer_set_assembly.argtypes = [C.c_void_p, C.c_int32]
     lib.gd_renderer_scribble.restype = C.c_int

@@ -5769,6 +5769,10 @@ struct gd_renderer {
     hipStream_t side_stream;
     hipEvent_t fork_event, join_event;
     bool side_ready;
+    // gd_renderer_mark_status: is the next gd_render call to say where its frames' status bits are final; did the last one, and on which stream?
+    hipEvent_t status_event;
+    bool status_wanted, status_marked;
+    hipStream_t status_stream;
     Overlays overlays;                       // device pointers, counts 0 until gd_renderer_set_overlays
     std::vector<void *> overlay_allocations;
 };
@@ -6073,7 +6077,7 @@ int validate_map(const gd_map_desc *h) {
 
 const int STAGE_COUNT = 9;
 
-int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_desc *lanes, const gd_frame_out *out, int base, int count, hipStream_t stream, bool timed) {
+int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_desc *lanes, const gd_frame_out *out, int base, int count, hipStream_t stream, bool timed, bool mark_status = false) {
     const gd_map_desc &m = r->dm.d;
     Scratch sc = chunk_scratch;
     if (out->final_frames && !out->frames) return fail(GD_E_ARG, "final_frames needs frames");
@@ -6136,6 +6140,15 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
             hipLaunchKernelGGL(pick_select(std::integral_constant<int, 1>()), dim3(others), dim3(64), 0, r->side_stream, r->dm, sc, longest, 0);
             HIP_TRY(hipEventRecord(r->join_event, r->side_stream));
             HIP_TRY(hipStreamWaitEvent(stream, r->join_event, 0));
+        }
+        // no kernel behind the selection sets a status bit
+        if (mark_status) {
+            hipStreamCaptureStatus capturing;
+            HIP_TRY(hipStreamIsCapturing(stream, &capturing));
+            if (capturing == hipStreamCaptureStatusNone) {      // an event of a capture cannot be waited for
+                HIP_TRY(hipEventRecord(r->status_event, stream));
+                r->status_marked = true; r->status_stream = stream;
+            }
         }
         // the billboards' lists beside the walls' drawing, on the side stream (when stages are being timed, with the billboards)
         if (has_billboards && !fused && !timed) {
@@ -6476,6 +6489,7 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
         else if (hipEventCreateWithFlags(&r->join_event, hipEventDisableTiming) != hipSuccess) {
             (void)hipEventDestroy(r->fork_event); (void)hipStreamDestroy(r->side_stream); rc = fail(GD_E_HIP, "hipEventCreateWithFlags");
         } else r->side_ready = true;
+        if (rc == GD_OK && hipEventCreateWithFlags(&r->status_event, hipEventDisableTiming) != hipSuccess) { r->status_event = nullptr; rc = fail(GD_E_HIP, "hipEventCreateWithFlags"); }
     }
     if (rc != GD_OK) { std::string keep = g_error; gd_renderer_destroy(r); g_error = keep; return rc; }
     *out = r;
@@ -6489,6 +6503,7 @@ void gd_renderer_destroy(gd_renderer *r) {
     if (r->sc.status) (void)hipHostFree(const_cast<unsigned char *>(r->sc.status));
     if (r->events_ready) for (int i = 0; i < 16; ++i) (void)hipEventDestroy(r->events[i]);
     if (r->side_ready) { (void)hipEventDestroy(r->fork_event); (void)hipEventDestroy(r->join_event); (void)hipStreamDestroy(r->side_stream); }
+    if (r->status_event) (void)hipEventDestroy(r->status_event);
     delete r;
 }
 
@@ -6519,9 +6534,11 @@ int gd_render(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_out *ou
     if (rc != GD_OK) return rc;
     if (r->chunk_lanes <= 0) return fail(GD_E_ARG, "this renderer was created for 0 lanes and holds no working memory: use gd_render_static");
     hipStream_t caller = static_cast<hipStream_t>(stream);
+    const bool mark_status = r->status_wanted;
+    r->status_wanted = r->status_marked = false;
     for (int base = 0; base < lanes->lane_count; base += r->chunk_lanes) {
         int count = lanes->lane_count - base < r->chunk_lanes ? lanes->lane_count - base : r->chunk_lanes;
-        rc = launch_chunk(r, r->sc, lanes, out, base, count, caller, false);
+        rc = launch_chunk(r, r->sc, lanes, out, base, count, caller, false, mark_status && base + count == lanes->lane_count);
         if (rc != GD_OK) return rc;
     }
     return GD_OK;
@@ -6588,6 +6605,20 @@ int gd_render_timed(gd_renderer *r, const gd_lanes_desc *lanes, const gd_frame_o
 int gd_renderer_status_seen(gd_renderer *r, int32_t *status) {
     if (!r || !status) return fail(GD_E_ARG, "null argument");
     *status = (r->sc.status[STATUS_CAND_OVERFLOW] ? 1 : 0) | (r->sc.status[STATUS_PASS_OVERFLOW] ? 2 : 0);
+    return GD_OK;
+}
+
+int gd_renderer_mark_status(gd_renderer *r) {
+    if (!r) return fail(GD_E_ARG, "null argument");
+    r->status_wanted = true;
+    return GD_OK;
+}
+
+int gd_renderer_wait_status(gd_renderer *r, void *stream) {
+    if (!r) return fail(GD_E_ARG, "null argument");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (r->status_marked && r->status_stream == st) HIP_TRY(hipEventSynchronize(r->status_event));
+    else HIP_TRY(hipStreamSynchronize(st));
     return GD_OK;
 }
 

@@ -323,8 +323,7 @@ class GraDoomVecEnv:
         self._words = torch.zeros(16, dtype=torch.int32, pin_memory=True) if self._native else None
         self._words_read = self._words.numpy() if self._native else None
         self._done_rows = torch.zeros(n, dtype=torch.int64, device=self.device) if self._native else None
-        # where a step's bookkeeping ends, and where its frames do: each is waited for by itself
-        self._listed_mark, self._drawn_mark = (torch.cuda.Event(), torch.cuda.Event()) if self._native else (None, None)
+        self._drawn_mark = torch.cuda.Event() if self._native else None     # where a step's frames end
         self._rgb_staging = None        # pinned, at most RGB_STAGING_BYTES
         self._leave_frames = _FRAMES.join(self)
         self._seed_values = [None] * n
@@ -443,12 +442,12 @@ class GraDoomVecEnv:
         indices = self._require_device_tensor(actions, "actions", shape=(self.num_envs,), dtypes=INDEX_DTYPES).to(torch.int64)
         rewards, terminated, truncated = self._dynamics.step(indices)
         self._done_listed = self._after_step(terminated, truncated, list_done)
-        marks = self._done_listed and list_done
-        if marks:
-            self._listed_mark.record(torch.cuda.current_stream(self.device))
-        elif not self._done_listed:
+        if not self._done_listed:
             self.pending_reset.copy_(terminated | truncated)      # engine.py:9542
-        self._renderer.render(self._dynamics.lane_state(), frames=self.frames, final_frames=final_frames, final_layout=final_layout)
+        lanes, marks = self._dynamics.lane_state(), self._done_listed and list_done
+        if marks and self._resets_alone():
+            self._renderer.mark_status()
+        self._renderer.render(lanes, frames=self.frames, final_frames=final_frames, final_layout=final_layout)
         if marks:
             self._drawn_mark.record(torch.cuda.current_stream(self.device))
         if not self._done_listed:
@@ -459,6 +458,12 @@ class GraDoomVecEnv:
         )
 
     def step_and_reset_device(self, actions: torch.Tensor, reset_seeds: torch.Tensor) -> DeviceAutoResetTransition:
+        """``step_device``, then ``reset_device`` of the lanes that ended (env.py:908-940).
+
+        Raises ``RuntimeError`` where the renderer truncated one of the step's frames: the step has been taken, no lane has been reset
+        (``pending_reset`` says which have ended) and the seeds have not been looked at.
+        """
+
         # the final-observation clone (env.py:915) is written by the observation kernel of the step
         final_frames = torch.empty_like(self.frames)
         transition = self._step(actions, final_frames, list_done=True)
@@ -466,17 +471,22 @@ class GraDoomVecEnv:
         final_signals = transition.signals.clone()
         final_info_histories = transition.info_histories.clone()
         listed = self._done_listed
-        if listed:   # how many lanes ended is known as soon as the step's bookkeeping is done, while its frames are being drawn
-            self._listed_mark.synchronize()
+        alone = listed and self._resets_alone()
+        if alone:    # how many lanes ended, and whether a frame was truncated, is known while the step's frames are still being put together
+            self._renderer.wait_status()
+            done_count = int(self._words_read[0])
+            alone = 0 < done_count <= 65535
+        elif listed:   # one wait on the stream
+            self._wait()
             done_count = int(self._words_read[0])
         else:
             done = transition.terminated | transition.truncated
             done_count = int(torch.count_nonzero(done))  # env.py:919: one host sync for the reference renderer
-        alone = listed and 0 < done_count <= 65535 and self._resets_alone()
-        if alone:    # their reset is queued behind the step's frames: the device goes from one to the other without the host
+        if alone:    # refused, a step leaves the lanes that ended as they are: none of the reset has begun
+            self._refuse_truncated(self._renderer.status_seen())
+            # the reset is queued behind the step's frames: the device goes from one to the other without the host
             observations, signals = self._reset_rows(self.pending_reset.clone(), reset_seeds, done_count)
             self._drawn_mark.synchronize()
-            self._refuse_truncated(self._renderer.status_seen())
         else:
             self.check_renderer_status()
         if not done_count:

@@ -154,6 +154,16 @@ class HipRenderer:
         _lib.check(self._lib.gd_renderer_status_seen(self._handle, C.byref(value)))
         return int(value.value)
 
+    def mark_status(self) -> None:
+        """The next ``render`` says where its frames' status bits are final: ``wait_status`` then waits no further."""
+
+        _lib.check(self._lib.gd_renderer_mark_status(self._handle))
+
+    def wait_status(self) -> None:
+        """Wait until ``status_seen`` is final for the frames last rendered on the current stream, which may still be under way."""
+
+        _lib.check(self._lib.gd_renderer_wait_status(self._handle, torch.cuda.current_stream(self.device).cuda_stream))
+
     def set_assembly(self, assembly: str) -> None:
         """``"separate"`` (kernel by kernel through a frame in device memory, the caller's or the working memory's own),
         ``"fused"`` (every frame is put together band by band in LDS and never reaches device memory unless asked for: a

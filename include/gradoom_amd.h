@@ -305,6 +305,15 @@ int gd_renderer_status(gd_renderer *r, int32_t *status);
 int gd_renderer_status_seen(gd_renderer *r, int32_t *status);
 
 /*
+ * For a caller that would know the bits while its frames are still being put together: they are set up to the selection of the walls, about half way.
+ * gd_renderer_mark_status: the next gd_render call says where on its stream the bits of its frames are final (which costs it 3 us).
+ * gd_renderer_wait_status: waits for that place of the last gd_render call, and for all that was queued on `stream` before it.  Where that call was
+ * not to say, was recorded into a graph, or went to another stream, it waits for all of `stream`.  Replace nothing in the reference.
+ */
+int gd_renderer_mark_status(gd_renderer *r);
+int gd_renderer_wait_status(gd_renderer *r, void *stream);
+
+/*
  * How a frame is put together once the walls are traversed.  GD_ASSEMBLY_SEPARATE: kernel by kernel through a
  * 320x240 frame in device memory, gd_frame_out.indexed or, when the caller takes none, a frame of the working memory's
  * own.  GD_ASSEMBLY_FUSED: band by band in LDS, where shading, billboards, overlays, PLAYPAL expansion, pooling and the

@@ -163,6 +163,64 @@ def test_a_step_with_truncated_frames_is_refused_whether_lanes_end_or_not(monkey
     env.close()
 
 
+@pytest.mark.parametrize("lanes", [3, 5, 113])     # frames that stay on one stream, that go to the side stream and back
+def test_a_refused_step_has_reset_no_lane(monkeypatch, lanes):
+    """Every lane ends with the step whose frames are truncated: the lanes, their stacks and seeds stay as the step left them, and bad seeds are not
+    what the step is refused for."""
+
+    from gradoom_amd.env import GraDoomVecEnv
+
+    _meta, _data, smap, _tables = load_fixture("small_midtex_sprites")
+    envs = [GraDoomVecEnv(smap, lanes, device="cuda:0", episode_timeout=2, sprites=4) for _ in range(2)]
+    actions, seeds = torch.zeros(lanes, dtype=torch.int64, device="cuda:0"), torch.arange(lanes, device="cuda:0") + 7
+    for env in envs:
+        env.reset_device(torch.ones(lanes, dtype=torch.bool, device="cuda:0"), seeds)
+        env.step_and_reset_device(actions, seeds + 1)
+    envs[1].step_device(actions)
+    monkeypatch.setattr(envs[0]._renderer, "status_seen", lambda: 1)
+    with pytest.raises(RuntimeError, match="candidate list"):
+        envs[0].step_and_reset_device(actions, seeds[:1].float())
+    monkeypatch.undo()
+    states = [(env.pending_reset, env._dynamics.episode_time, env._dynamics.phase, env._latest_reset_seeds, env.frames, env.signal_buffer) for env in envs]
+    assert bool(states[0][0].all()) and bool((states[0][1] == 2).all()) and torch.equal(states[0][3], seeds)
+    assert all(torch.equal(one, other) for one, other in zip(*states))
+    for env in envs:
+        env.reset_device(torch.ones(lanes, dtype=torch.bool, device="cuda:0"), seeds)
+        env.close()
+
+
+@pytest.mark.parametrize("lanes", [2, 24])     # frames that stay on one stream, that go to the side stream and back
+def test_the_status_is_final_where_the_frames_say_so(monkeypatch, lanes):
+    """More dividers in a column than its list holds; with and without a mark, asked on the frames' own stream and on another."""
+
+    from gradoom_amd import synthmap
+    from gradoom_amd.env import PosePoolDynamics
+    from gradoom_amd.renderer import HipRenderer
+
+    monkeypatch.setattr(synthmap, "CELL", 48)
+    smap = synthmap.generate_map(5, grid=(300, 1), sectors=300, linedefs=901)
+    dynamics = PosePoolDynamics(smap, lanes, "cuda:0", pool=4, sprites=4)
+    centre = smap.sector_quads[0].mean(axis=0)
+    for name, value in (("x", float(centre[0])), ("y", float(centre[1])), ("angle_bam", 0), ("pitch_bam", 0), ("view_z", float(smap.sector_heights[0, 0]) + 41.0)):
+        dynamics._pool[name].fill_(value)       # looking along +x, down the corridor
+    state, obs = dynamics.lane_state(), torch.empty((lanes, 84, 84), dtype=torch.uint8, device="cuda:0")
+    for marked, asked_elsewhere in ((True, False), (False, False), (True, True)):
+        renderer = HipRenderer(smap, lanes, "cuda:0")
+        torch.cuda.synchronize()
+        renderer.wait_status()
+        assert renderer.status_seen() == 0
+        if marked:
+            renderer.mark_status()
+        renderer.render(state, obs=obs)
+        stream = torch.cuda.Stream() if asked_elsewhere else torch.cuda.current_stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            renderer.wait_status()
+        assert renderer.status_seen() == 1
+        assert renderer.status() == 1
+        renderer.close()
+
+
 def test_a_pose_pool_whose_lane_state_takes_no_lanes_resets_the_lanes_that_end():
     from gradoom_amd.env import GraDoomVecEnv, PosePoolDynamics
 
