@@ -5044,14 +5044,19 @@ __device__ const __align__(16) PoolWeights POOL_WEIGHTS = pool_weights();
 // A work-group takes a run of the frames' blocks of rows, a wavefront OBS_TILE observation columns of each.  The next block's pixels are asked
 // for as soon as a tile's own are used up.
 // ALIGNED: the frames start on 16 bytes.
-template <bool ALIGNED>
-__global__ void __launch_bounds__(OBS_THREADS, 6) observe_kernel(const unsigned char *indexed, size_t lane_stride, int source_rows, const unsigned char *playpal,
+// FEW: a work-group takes half a block, the rows of one product down the columns (the three tiles that they lie in), and no more: twice the
+// work-groups, each with less to do one after the other, which asks for all it reads up front and looks colours up in the palette itself.
+// Few frames last as long as one work-group: 1 frame 5.4 us by blocks, 4.6 so; 16 frames 6.2, 4.7 (121 registers, four wavefronts a SIMD).
+template <bool ALIGNED, bool FEW>
+__global__ void __launch_bounds__(OBS_THREADS, FEW ? 3 : 6) observe_kernel(const unsigned char *indexed, size_t lane_stride, int source_rows, const unsigned char *playpal,
                                int lane_count, unsigned char *obs, unsigned char *frames, const unsigned char *reset_mask, int stack_mode,
                                unsigned char *final_frames, bool final_hwc, const float *blend) {
     __shared__ unsigned int pal[256];   // PLAYPAL after the lane's screen blend, one word per colour (red | green << 8 | blue << 16, each less 128)
-    __shared__ __align__(16) unsigned int copies[256 * OBS_COPIES];
-    __shared__ unsigned int gray_words[2][OBS_BLOCK_ROWS * GD_OBS_SIZE / 4];
-    const int tasks = lane_count * OBS_BLOCKS;
+    constexpr int COPIES = FEW ? 1 : OBS_COPIES, TILES = FEW ? 3 : OBS_ROW_TILES, AHEAD = FEW ? TILES : OBS_AHEAD;
+    constexpr int ROWS = FEW ? OBS_TILE : OBS_BLOCK_ROWS, PARTS = GD_OBS_SIZE / ROWS;      // observation rows of a task, tasks of a frame
+    __shared__ __align__(16) unsigned int copies[FEW ? 4 : 256 * OBS_COPIES];
+    __shared__ unsigned int gray_words[2][ROWS * GD_OBS_SIZE / 4];
+    const int tasks = lane_count * PARTS;
     const int first_task = (int)((long long)tasks * blockIdx.x / gridDim.x), end_task = (int)((long long)tasks * (blockIdx.x + 1) / gridDim.x);
     const int wave = threadIdx.x >> 6, lane_id = threadIdx.x & 63, group = lane_id >> 4, column = lane_id & 15;
     const size_t F = (size_t)GD_OBS_SIZE * GD_OBS_SIZE / 4;     // words per observation
@@ -5061,23 +5066,37 @@ __global__ void __launch_bounds__(OBS_THREADS, 6) observe_kernel(const unsigned 
         return (unsigned)p[0] | ((unsigned)p[1] << 8) | ((unsigned)p[2] << 16) | ((unsigned)p[3] << 24);
     };
     const unsigned int at = (unsigned)(obs_window(wave) + 16 * group + column * SW);      // lane strides are multiples of 16, like the window's start
+    auto tile_row = [](int part, int t) {      // a tile's first row: half a block's tiles are its first three, or its last
+        return (FEW ? part >> 1 : part) * OBS_SOURCE_ROWS + 16 * (t + (FEW && (part & 1) ? OBS_ROW_TILES - TILES : 0));
+    };
     auto load_tile = [&](int task, int t) -> uint4 {      // a lane's sixteen pixels of a tile; past the source, or the run, those of some row before
         task = min(task, end_task - 1);
-        const int n = task / OBS_BLOCKS, row = min((task - n * OBS_BLOCKS) * OBS_SOURCE_ROWS + 16 * t, source_rows - 16);
+        const int n = task / PARTS, row = min(tile_row(task - n * PARTS, t), source_rows - 16);
         const unsigned char *first = indexed + (size_t)n * lane_stride + (size_t)row * SW;
         if (ALIGNED) return *reinterpret_cast<const uint4 *>(first + at);
         const bool aligned = (reinterpret_cast<size_t>(indexed) & 3) == 0;
         return make_uint4(load_word(first + at, aligned), load_word(first + at + 4, aligned), load_word(first + at + 8, aligned), load_word(first + at + 12, aligned));
     };
-    uint4 pixels[OBS_ROW_TILES];
+    uint4 pixels[TILES];
 #pragma unroll
-    for (int t = 0; t < OBS_AHEAD; ++t) pixels[t] = load_tile(first_task, t);
+    for (int t = 0; t < AHEAD; ++t) pixels[t] = load_tile(first_task, t);
     const int4v along = *reinterpret_cast<const int4v *>(POOL_WEIGHTS.along[wave][lane_id]);
-    const int4v down[2] = {*reinterpret_cast<const int4v *>(POOL_WEIGHTS.down[0][lane_id]), *reinterpret_cast<const int4v *>(POOL_WEIGHTS.down[1][lane_id])};
+    const int4v down[2] = {*reinterpret_cast<const int4v *>(POOL_WEIGHTS.down[FEW ? first_task & 1 : 0][lane_id]), *reinterpret_cast<const int4v *>(POOL_WEIGHTS.down[1][lane_id])};
     const unsigned int bank = lane_id & (OBS_COPIES - 1);
-    auto colour_of = [&](unsigned int word, int k) { return copies[((word >> (8 * k)) & 255u) * OBS_COPIES + bank]; };
+    auto colour_of = [&](unsigned int word, int k) {
+        const unsigned int index = (word >> (8 * k)) & 255u;
+        return FEW ? pal[index] : copies[index * COPIES + bank];
+    };
     for (int task = first_task; task < end_task; ++task) {
-        const int n = task / OBS_BLOCKS, block = task - n * OBS_BLOCKS;
+        const int n = task / PARTS, block = task - n * PARTS;
+        unsigned int early[FEW ? GD_FRAME_STACK : 1];      // of few, the stack words that the roll keeps, asked for up front: nothing else goes on meanwhile
+        if constexpr (FEW) {
+            static_assert(ROWS * GD_OBS_SIZE / 4 <= OBS_THREADS, "observe_kernel: a word a thread");
+            const bool keeps = threadIdx.x < ROWS * GD_OBS_SIZE / 4 && frames && !(reset_mask && reset_mask[n]);
+#pragma unroll
+            for (int f = 0; f < GD_FRAME_STACK; ++f)
+                early[f] = keeps ? load_word(frames + ((size_t)n * GD_FRAME_STACK * F + f * F + (size_t)block * (ROWS * GD_OBS_SIZE / 4) + threadIdx.x) * 4, stack_aligned) : 0u;
+        }
         if (task == first_task || (blend && block == 0)) {      // nobody reads the last lane's copies any more: its last block has been put together
             if (threadIdx.x < 256) {
                 const int k = threadIdx.x;
@@ -5089,14 +5108,16 @@ __global__ void __launch_bounds__(OBS_THREADS, 6) observe_kernel(const unsigned 
                 pal[k] = (r | (g << 8) | (b << 16)) ^ 0x808080u;
             }
             __syncthreads();
-            for (int k = threadIdx.x; k < 256 * OBS_COPIES / 4; k += OBS_THREADS) {
-                const unsigned int colour = pal[k / (OBS_COPIES / 4)];
-                reinterpret_cast<uint4 *>(copies)[k] = make_uint4(colour, colour, colour, colour);
+            if constexpr (!FEW) {
+                for (int k = threadIdx.x; k < 256 * COPIES / 4; k += OBS_THREADS) {
+                    const unsigned int colour = pal[k / (COPIES / 4)];
+                    reinterpret_cast<uint4 *>(copies)[k] = make_uint4(colour, colour, colour, colour);
+                }
+                __syncthreads();
             }
-            __syncthreads();
         }
         const bool resets = reset_mask && reset_mask[n];
-        int low[OBS_ROW_TILES][3], high[OBS_ROW_TILES][3];      // the sums along the rows, a byte each of four rows a word
+        int low[TILES][3], high[TILES][3];      // the sums along the rows, a byte each of four rows a word
         const int4v start = {20 * 80 * 128 + 800, 20 * 80 * 128 + 800, 20 * 80 * 128 + 800, 20 * 80 * 128 + 800};      // the colours' 128, and half of 1600
         auto down_columns = [&](int half) __attribute__((always_inline)) {
             int4v total[3];
@@ -5117,8 +5138,8 @@ __global__ void __launch_bounds__(OBS_THREADS, 6) observe_kernel(const unsigned 
             }
         };
 #pragma unroll
-        for (int t = 0; t < OBS_ROW_TILES; ++t) {
-            pixels[(t + OBS_AHEAD) % OBS_ROW_TILES] = load_tile(task + (t + OBS_AHEAD) / OBS_ROW_TILES, (t + OBS_AHEAD) % OBS_ROW_TILES);
+        for (int t = 0; t < TILES; ++t) {
+            if constexpr (!FEW) pixels[(t + AHEAD) % TILES] = load_tile(task + (t + AHEAD) / TILES, (t + AHEAD) % TILES);
             const unsigned int word[4] = {pixels[t].x, pixels[t].y, pixels[t].z, pixels[t].w};
             int4v channel[3];
 #pragma unroll
@@ -5135,21 +5156,23 @@ __global__ void __launch_bounds__(OBS_THREADS, 6) observe_kernel(const unsigned 
                 const unsigned int front = __builtin_amdgcn_perm((unsigned)sums[1], (unsigned)sums[0], 0x05010400u), back = __builtin_amdgcn_perm((unsigned)sums[3], (unsigned)sums[2], 0x05010400u);
                 low[t][c] = (int)(__builtin_amdgcn_perm(back, front, 0x05040100u) ^ 0x80808080u);
                 high[t][c] = (int)__builtin_amdgcn_perm(back, front, 0x07060302u);
-                if (16 * t >= VH % OBS_SOURCE_ROWS && block * OBS_SOURCE_ROWS + 16 * t >= source_rows) { low[t][c] = 0; high[t][c] = (int)0xD8D8D8D8u; }   // black: 80 * -128 = 256 * -40
+                if ((FEW || 16 * t >= VH % OBS_SOURCE_ROWS) && tile_row(block, t) >= source_rows) { low[t][c] = 0; high[t][c] = (int)0xD8D8D8D8u; }   // black: 80 * -128 = 256 * -40
             }
             if (t == 2) down_columns(0);
-            if (t == 4) down_columns(1);
+            if (t == 4) down_columns(1);      // not reached by three tiles
         }
         // the stack words that the roll keeps
-        constexpr int WORDS = OBS_BLOCK_ROWS * GD_OBS_SIZE / 4, ROUNDS = (WORDS + OBS_THREADS - 1) / OBS_THREADS;
+        constexpr int WORDS = ROWS * GD_OBS_SIZE / 4, ROUNDS = (WORDS + OBS_THREADS - 1) / OBS_THREADS;
         const size_t first_word = (size_t)block * WORDS;
         unsigned int kept[ROUNDS][GD_FRAME_STACK];
 #pragma unroll
         for (int j = 0; j < ROUNDS; ++j) {
             const int k = threadIdx.x + j * OBS_THREADS;
 #pragma unroll
-            for (int f = 0; f < GD_FRAME_STACK; ++f)
-                kept[j][f] = k < WORDS && frames && !resets ? load_word(frames + ((size_t)n * GD_FRAME_STACK * F + f * F + first_word + k) * 4, stack_aligned) : 0u;
+            for (int f = 0; f < GD_FRAME_STACK; ++f) {
+                if constexpr (FEW) kept[j][f] = early[f];
+                else kept[j][f] = k < WORDS && frames && !resets ? load_word(frames + ((size_t)n * GD_FRAME_STACK * F + f * F + first_word + k) * 4, stack_aligned) : 0u;
+            }
         }
         __syncthreads();
         // the block's pixels are contiguous in the observation; they go out, and the stack is rolled, a word (four pixels) per thread
@@ -5171,8 +5194,13 @@ __global__ void __launch_bounds__(OBS_THREADS, 6) observe_kernel(const unsigned 
     }
 }
 
-decltype(&observe_kernel<true>) observe_kernel_for(const unsigned char *indexed) {
-    return (reinterpret_cast<size_t>(indexed) & 15) == 0 ? observe_kernel<true> : observe_kernel<false>;
+// `count` frames that lie `stride` bytes apart pooled to observations and stacks.
+void launch_observe(hipStream_t stream, const unsigned char *indexed, size_t stride, int source_rows, const unsigned char *playpal, int count, unsigned char *obs, unsigned char *frames,
+                    const unsigned char *reset_mask, int stack_mode, unsigned char *final_frames, bool final_hwc, const float *blend) {
+    const bool few = observe_few(count), aligned = (reinterpret_cast<size_t>(indexed) & 15) == 0;
+    auto kernel = few ? (aligned ? observe_kernel<true, true> : observe_kernel<false, true>) : (aligned ? observe_kernel<true, false> : observe_kernel<false, false>);
+    const int groups = few ? count * (GD_OBS_SIZE / OBS_TILE) : observe_groups(count * OBS_BLOCKS);
+    hipLaunchKernelGGL(kernel, dim3(groups), dim3(OBS_THREADS), 0, stream, indexed, stride, source_rows, playpal, count, obs, frames, reset_mask, stack_mode, final_frames, final_hwc, blend);
 }
 
 // engine.py:15381-15384: PLAYPAL expansion.  A thread takes sixteen pixels: one 16-byte load, sixteen palette words from LDS; the 48 bytes
@@ -6264,12 +6292,9 @@ int launch_chunk(gd_renderer *r, const Scratch &chunk_scratch, const gd_lanes_de
         hipLaunchKernelGGL(hud_kernel, dim3(HUD_TILES / (HUD_THREADS / 64), count), dim3(HUD_THREADS), 0, stream, r->overlays, lanes->hud_state, base, count, frame_base, frame_stride);
     mark();
     if (out->obs || out->frames) {
-        hipLaunchKernelGGL(observe_kernel_for(frame_base), dim3(observe_groups(count * OBS_BLOCKS)), dim3(OBS_THREADS), 0, stream,
-                           frame_base, frame_stride, source_rows, m.playpal, count, out->obs ? out->obs + (size_t)base * F : nullptr,
-                           out->frames ? out->frames + (size_t)base * GD_FRAME_STACK * F : nullptr,
-                           out->reset_mask ? out->reset_mask + base : nullptr, out->stack_mode,
-                           out->final_frames ? out->final_frames + (size_t)base * GD_FRAME_STACK * F : nullptr,
-                           out->final_frames_layout == GD_LAYOUT_HWC, blend);
+        launch_observe(stream, frame_base, frame_stride, source_rows, m.playpal, count, out->obs ? out->obs + (size_t)base * F : nullptr,
+                       out->frames ? out->frames + (size_t)base * GD_FRAME_STACK * F : nullptr, out->reset_mask ? out->reset_mask + base : nullptr, out->stack_mode,
+                       out->final_frames ? out->final_frames + (size_t)base * GD_FRAME_STACK * F : nullptr, out->final_frames_layout == GD_LAYOUT_HWC, blend);
     }
     if (out->rgb) {
         size_t pixels = (size_t)count * frame_stride;
@@ -6736,10 +6761,9 @@ int gd_observe(const uint8_t *indexed, int32_t source_rows, const uint8_t *playp
     for (int base = 0; base < lane_count; base += 32768) {
         int count = lane_count - base < 32768 ? lane_count - base : 32768;
         const size_t F = (size_t)GD_OBS_SIZE * GD_OBS_SIZE;
-        hipLaunchKernelGGL(observe_kernel_for(indexed), dim3(observe_groups(count * OBS_BLOCKS)), dim3(OBS_THREADS), 0, static_cast<hipStream_t>(stream),
-                           indexed + (size_t)base * source_rows * SW, (size_t)source_rows * SW, source_rows, playpal, count,
-                           obs ? obs + (size_t)base * F : nullptr, frames ? frames + (size_t)base * GD_FRAME_STACK * F : nullptr,
-                           reset_mask ? reset_mask + base : nullptr, stack_mode, nullptr, false, nullptr);
+        launch_observe(static_cast<hipStream_t>(stream), indexed + (size_t)base * source_rows * SW, (size_t)source_rows * SW, source_rows, playpal, count,
+                       obs ? obs + (size_t)base * F : nullptr, frames ? frames + (size_t)base * GD_FRAME_STACK * F : nullptr,
+                       reset_mask ? reset_mask + base : nullptr, stack_mode, nullptr, false, nullptr);
     }
     HIP_TRY(hipGetLastError());
     return GD_OK;

@@ -156,6 +156,11 @@ inline int sprite_row_parts(int lanes) { return lanes >= 512 ? 1 : SPRITE_ROW_PA
 //        96     16       251 / 293     232 / 234      376 / 408      283 / 315      274 / 277      374 / 403
 inline bool side_stream_pays(int lanes, bool billboards) { return lanes > 112 || (billboards && lanes >= 4); }
 
+// observe_kernel: few frames by half blocks of rows, a work-group each, or by blocks?  Up to 85 frames blocks leave compute units without any.  us,
+// halves / blocks, plain pooling of 208 rows and a stack with flashes: 1 frame 4.6 / 5.4, 5.1 / 6.5; 16 frames 4.7 / 6.2, 5.0 / 6.4; 42 frames 4.8 / 6.2,
+// 5.7 / 7.3; 64 frames 6.2 / 6.4, 6.9 / 7.5; 85 frames 6.5 / 6.5, 7.1 / 7.6; 128 frames 8.5 / 8.5, 9.9 / 9.6; 256 frames 15.6 / 11.0, 18.2 / 12.4.
+inline bool observe_few(int frames) { return frames <= 85; }
+
 // observe_kernel: work-groups, which share the frames' blocks of rows (three a frame).  Four of them are what a compute unit holds, and each pays once
 // for its copies of the palette.  4096 frames with 512 / 768 / 1024 / 2048 / 12288 work-groups: 115 / 105 / 105 / 110 / 118 us.
 inline int observe_groups(int blocks) { return blocks < 1024 ? blocks : 1024; }

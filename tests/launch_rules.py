@@ -14,7 +14,7 @@ MOST_LANES = 4096        # of one chunk: larger batches are rendered chunk by ch
 # what a rule is asked beside the lanes: the map's linedefs, or whether there are billboards
 LINEDEFS, BILLBOARDS, NOTHING = "linedefs", "billboards", None
 RULES = dict(setup_whole_lanes=LINEDEFS, select_strips=LINEDEFS, select_lanes=LINEDEFS, select_together=NOTHING, geometry_parts=NOTHING, raster_parts=NOTHING, raster_sixteen=NOTHING, gap_waves=LINEDEFS,
-             sprite_row_parts=NOTHING, side_stream_pays=BILLBOARDS)
+             sprite_row_parts=NOTHING, side_stream_pays=BILLBOARDS, observe_few=NOTHING)
 
 
 @functools.lru_cache(maxsize=1)

@@ -11,7 +11,7 @@ import pytest
 import launch_rules
 
 ANSWERS = dict(setup_whole_lanes={0, 1}, select_lanes={8, 16, 32}, select_together={0, 1}, geometry_parts={1, 2, 4, 8, 16, 32}, raster_parts={1, 2, 4, 8}, raster_sixteen={0, 1}, gap_waves={4, 8, 16}, sprite_row_parts={1, 4},
-               side_stream_pays={0, 1})
+               side_stream_pays={0, 1}, observe_few={0, 1})
 MAPS = (1, 2, 100, 160, 161, 320, 511, 512, 513, 899, 900, 1023, 1024, 2000, 4000, 4095, 4096, 4097, 65534)
 
 
