@@ -1740,6 +1740,7 @@ static void composite_weapon_patch(uint8_t *view, int64_t patch, int64_t horizon
 static void draw_hud_patch(uint8_t *canvas, int patch, int x, int y) {
     const gd_overlay_desc &o = g_overlays;
     const int rows = GD_SCREEN_HEIGHT - VH;
+    if (patch < 0 || patch >= o.hud_patch_count) return;
     x -= o.hud_left[patch];
     y -= o.hud_top[patch];
     const int width = o.hud_w[patch], height = o.hud_h[patch];
@@ -1765,8 +1766,7 @@ static void draw_hud_number(uint8_t *canvas, int value, int right, int y, bool s
     for (const char *c = text; *c; ++c) {
         if (*c == '-') { x += digit_width; continue; }
         const int patch = base + (*c - '0');
-        const int glyph_x = x - o.hud_left[patch], glyph_y = y - o.hud_top[patch];
-        draw_hud_patch(canvas, patch, glyph_x, glyph_y);
+        if (patch < o.hud_patch_count) draw_hud_patch(canvas, patch, x - o.hud_left[patch], y - o.hud_top[patch]);
         x += digit_width;
     }
 }

@@ -104,3 +104,33 @@ def test_decal_packing_keeps_every_slot_in_paint_order():
             # the direction goes through the 8192-entry fine-angle table: within one table step of the true cosine / sine
             assert abs(float(geom[lane, position, 2]) - np.cos(direction)) < 2e-3 and abs(float(geom[lane, position, 3]) - np.sin(direction)) < 2e-3
     assert overlay_inputs.decal_inputs(*(torch.as_tensor(v[:, :0]) for v in (serial, wall, along, impact_z, style)), torch.as_tensor(portal_walls), table) is None
+
+
+def test_the_oracle_leaves_out_status_bar_patches_that_do_not_exist(oracle):
+    """Past either end of the list lies memory of somebody else (here further patches, which must not show)."""
+    from conftest import lane_inputs
+    from gradoom_amd import synthmap
+
+    meta, data, _smap, tables = load_fixture("overlays")
+    arrays = lane_inputs(data)
+    every = dict(synthmap.generate_overlays(33))
+    kept = 45
+
+    def bars(faces, **hidden):
+        arrays["hud_state"] = np.array(arrays["hud_state"], copy=True)
+        arrays["hud_state"][:, 3] = faces
+        first, last = 1, kept
+        overlays = {name: np.ascontiguousarray(value)[first:last] if name.startswith("hud_") else value for name, value in every.items()}
+        overlays.update(hidden)
+        oracle.set_overlays(overlays)
+        try:
+            return oracle.render(tables, arrays, data["cosine_correction"], lane_range=(0, 1))["indexed"][0, 208:]
+        finally:
+            oracle.set_overlays(None)
+
+    blank = np.array(every["hud_w"][1:kept], copy=True)
+    blank[20] = 0
+    without = bars(20, hud_w=blank)
+    assert not np.array_equal(bars(20), without)
+    for face in (-1, kept - 1, kept + 1):
+        assert np.array_equal(bars(face), without)
