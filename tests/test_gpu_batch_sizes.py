@@ -99,3 +99,34 @@ def test_batches_on_both_sides_of_a_rules_line_match_the_oracle(oracle, rule, bi
         assert renderer.status() == 0
         assert torch.equal(indexed, expected[torch.as_tensor(which, device="cuda:0")])
         renderer.close()
+
+
+def test_batches_at_the_lines_of_large_maps_gap_columns_match_the_oracle(oracle):
+    """Maps of 3000 linedefs and more have lines of their own; a plane level per sector, and cameras off the map, whose frames are mostly gap pixels."""
+    import launch_rules
+    from gradoom_amd import hostmath, mapbuild, synthmap
+    from gradoom_amd.renderer import HipRenderer, LaneState
+    from gradoom_amd.selfcheck import make_lane_arrays
+
+    cosine = hostmath.cosine_correction("cpu").numpy()
+    smap = synthmap.with_variant(synthmap.generate_map(6007, grid=(19, 18), sectors=310, linedefs=3050, midtex=0.1), 6008, heights="uniform")
+    poses = synthmap.generate_poses(smap, CAMERAS, 6009, pitch=True, margin=0.02)
+    segments = np.asarray(smap.wall_segments, dtype=np.float64)
+    for camera in (1, 3):
+        poses.x[camera], poses.y[camera], poses.angle_bam[camera] = segments[:, [0, 2]].min() - 60 * camera, segments[:, [1, 3]].mean(), 0
+    arrays = make_lane_arrays(smap, poses, synthmap.generate_sprites(smap, CAMERAS, 32, 6010))
+    tables = mapbuild.build_map_tables(smap)
+    linedefs = len(tables["walls"])
+    lines = launch_rules.lines("gap_waves", linedefs)
+    assert linedefs >= 3000 and lines != launch_rules.lines("gap_waves", 600) and len(lines) == 2
+    expected = torch.as_tensor(oracle.render(tables, arrays, cosine)["indexed"]).to("cuda:0")
+    for lanes in sorted(set(lines) | {line - 1 for line in lines}):
+        print(f"{lanes} lanes", flush=True)
+        which = np.arange(lanes) % CAMERAS
+        renderer = HipRenderer(smap, lanes, "cuda:0", cosine_correction=cosine, tables=tables)
+        indexed = torch.zeros((lanes, 240, 320), dtype=torch.uint8, device="cuda:0")
+        renderer.render(LaneState.from_numpy({name: np.ascontiguousarray(value[which]) for name, value in arrays.items()}, "cuda:0"), indexed=indexed)
+        torch.cuda.synchronize()
+        assert renderer.status() == 0
+        assert torch.equal(indexed, expected[torch.as_tensor(which, device="cuda:0")])
+        renderer.close()

@@ -145,7 +145,7 @@ def test_a_step_does_not_wait_for_other_streams():
 
 @pytest.mark.parametrize("timeout", [1, 50])
 def test_a_step_with_truncated_frames_is_refused_whether_lanes_end_or_not(monkeypatch, timeout):
-    """The lanes that end are reset behind the step's frames, before the host has waited for these: their check comes all the same."""
+    """The reset of the lanes that end is queued behind the step's frames, which the host does not wait for: their check comes all the same."""
 
     from gradoom_amd.env import GraDoomVecEnv
 

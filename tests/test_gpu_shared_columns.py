@@ -1,4 +1,4 @@
-"""Columns that share a wavefront's lanes: on either side of the batch sizes at which a column has eight, four, two lanes or one, every
+"""Columns that share a wavefront's lanes: on either side of the batch sizes at which a column has sixteen lanes, eight, four, two or one, every
 lane's frame is the one the CPU oracle draws for its camera, wall depths (which chips are drawn against) among it."""
 
 from __future__ import annotations
@@ -47,8 +47,8 @@ def test_batches_at_the_lines_of_the_columns_shares_match_the_oracle(oracle, inv
     oracle.set_overlays(overlays)
     expected = torch.as_tensor(oracle.render(tables, arrays, cosine)["indexed"]).to("cuda:0")
     oracle.set_overlays(None)
-    lines = launch_rules.lines("raster_parts")
-    assert len(lines) == 3
+    lines = launch_rules.lines("raster_sixteen") + launch_rules.lines("raster_parts")
+    assert len(lines) == 4 and lines == sorted(lines)      # sixteen lanes a column go before what raster_parts says
     for lanes in sorted({1} | set(lines) | {line - 1 for line in lines}):
         print(f"{lanes} lanes", flush=True)
         which = np.arange(lanes) % CAMERAS
