@@ -299,7 +299,8 @@ struct Scratch {    // per-chunk working memory, sized at create
     int *lane_blends;      // [L] does some live billboard of the lane blend with the pixel below it (sprite_style other than -1)?
                            // (lane_tables_kernel)
     unsigned char *sprite_late; // [L, SW / SPRITE_COLUMNS, SPRITE_ROW_PARTS] did this work-group of the billboards' early launch leave pixels to the
-                           // late one? (written for lanes that blend; in the memory of strip_order, which the walls are done with by then)
+                           // late one? (Written for lanes that blend.  In the memory of strip_order, which nothing reads once the walls are drawn:
+                           // memory of its own would make a lane's share larger, and gd_render_static would refuse maps that it takes.)
     unsigned char *strip_key;  // [L*SEGS_PER_LANE] expected traversal length of each (lane, segment of SEG_COLS columns)
     int *strip_order;      // [L*SEGS_PER_LANE] segments, longest expected traversal first
     volatile unsigned char *status;   // [2] sticky flags in pinned host memory: a candidate list, a list of passes was cut short
@@ -1545,7 +1546,7 @@ __device__ __forceinline__ int flat_select_row(const DeviceMap &dm, const Scratc
 // where a sprite stands behind the plane with no sprite clip recorded, which the sprite pass finds out for
 // itself (flat_ray_resolves); the few pixels left (columns whose traversal left a gap) show the flat pass's
 // picture.  wall_raster_kernel lists their columns, of all lanes together: most lanes have none, some have hundreds.
-// flat_gap_kernel, a work-group per listed column, selects them.
+// flat_gap_kernel, a work-group per half of the screen of a listed column, selects them.
 //
 // Then, column by column, the vertical repair (engine.py:11026-11083).  An unresolved
 // pixel takes the sector of the next resolved pixel below it in its half of the screen; when that sector is not the camera's,
@@ -5877,8 +5878,8 @@ __global__ void __launch_bounds__(256) sprite_depth_kernel(const float *x, const
     const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < total) depth_of(x, y, angle, sprite_x, sprite_y, k, slots, depth);
 }
-// Both in one launch, the rays' work-groups first: a launch less in front of every frame with billboards (a view of one lane 257 -> 249 us, the
-// host's share of the descriptors 37 -> 29).
+// Both in one launch, the rays' work-groups first: a launch less in front of every frame with billboards.  (The host's share of the descriptors 37 -> 29 us;
+// a view of one lane, 285 us, and 48 RGB frames, 760 us, gain less than two runs of one side differ by.)
 __global__ void __launch_bounds__(256) lane_floats_kernel(const float *x, const float *y, const float *angle, const float *offsets, int rays, float *ray_cos, float *ray_sin,
                                                           const float *sprite_x, const float *sprite_y, long long billboards, int slots, float *depth) {
     const unsigned ray_blocks = ((unsigned)rays + 255u) / 256u;
