@@ -28,7 +28,7 @@ def needs_build() -> bool:
     if not os.path.exists(LIBRARY):
         return True
     built = os.path.getmtime(LIBRARY)
-    headers = [os.path.join(os.path.dirname(HERE), "include", "gradoom_amd.h"), *(os.path.join(HERE, "csrc", name) for name in ("gd_divide.h", "gd_internal.h", "gd_rules.h"))]
+    headers = [os.path.join(os.path.dirname(HERE), "include", "gradoom_amd.h"), *(os.path.join(HERE, "csrc", name) for name in ("gd_divide.h", "gd_internal.h", "gd_order.h", "gd_rules.h"))]
     return any(os.path.getmtime(path) > built for path in SOURCES + headers)
 
 

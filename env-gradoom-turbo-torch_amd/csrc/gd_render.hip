@@ -44,6 +44,7 @@
 
 #include "../../include/gradoom_amd.h"
 #include "gd_divide.h"
+#include "gd_order.h"
 #include "gd_internal.h"
 #include "gd_rules.h"
 
@@ -2029,7 +2030,6 @@ __global__ void __launch_bounds__(FINISH_THREADS) flat_span_finish_kernel(Scratc
 // ---------------------------------------------------------------------------------------------
 // walls: engine.py:11462-13745
 // ---------------------------------------------------------------------------------------------
-#define CAND_BATCH 8
 #define WALL_ROWS 8          // rows painted / clipped per step of the wall traversal
 struct ColumnCtx {
     const Tables *tb;
@@ -2064,23 +2064,6 @@ struct ColumnCtx {
         union { uint4 raw; Cand c; } u;
         u.raw = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(list) + (list_column + (unsigned)k * (SW * 16u)));   // one 16-byte load
         return u.c;
-    }
-    // Entries k0 .. k0+CAND_BATCH-1 of this column's list, loaded together so that their memory
-    // latencies overlap; slots past the end repeat the last entry (callers skip them).
-    __device__ __forceinline__ void cand_batch(int k0, Cand (&out)[CAND_BATCH]) const {
-#pragma unroll
-        for (int j = 0; j < CAND_BATCH; ++j) out[j] = cand(k0 + j < count ? k0 + j : count - 1);
-    }
-    // The next CAND_BATCH entries named by the bits of `rest` (list positions, ascending), loaded together;
-    // slot j is absent where at[j] < 0.
-    __device__ __forceinline__ void cand_batch_of(u64 &rest, Cand (&out)[CAND_BATCH], int (&at)[CAND_BATCH]) const {
-#pragma unroll
-        for (int j = 0; j < CAND_BATCH; ++j) {
-            at[j] = rest ? __ffsll((long long)rest) - 1 : -1;
-            rest &= rest - 1;
-        }
-#pragma unroll
-        for (int j = 0; j < CAND_BATCH; ++j) out[j] = cand(at[j] < 0 ? 0 : at[j]);
     }
     __device__ Eval eval(int w) const { return eval_wall(m, *c, spans + rec_base, x, w, rx, ry); }
 };
@@ -2142,17 +2125,95 @@ template <> struct NearestOf<1> {
     __device__ __forceinline__ int wall() const { return w; }
     __device__ __forceinline__ int flags() const { return f; }
 };
+// One lane alone reads the list where it is, nearest entries first: their places, sorted by distance when the column begins, lie in LDS.  The order is
+// that of the distances' bits but the lowest six, which hold the place, so that entries a few units in the last place apart may come in either order: a
+// scan takes the smallest of what it looks at, and looks on until what is left is farther than the answer by more than that.  A list in the spill pool is
+// looked at from end to end.  A pass looks at some eight entries so, of the thirty that a column of the 4000-linedef map lists: for 4096 lanes the launch
+// for the strips that are not among the longest issues 9,900 vector instructions and 370 loads a wavefront, 14,500 and 690 when every scan
+// went over the whole list, and takes 0.80 ms instead of 0.895 (0.20 for 0.23 at 1024 lanes of the 2000-linedef map): what is left waits for loads that
+// depend on one another.  The network for 64 needs more registers than there are (some forty words go to memory once a column), those for 32 and 48 do not.
+#define ORDER_ROWS (CAND_MAX / 4 + 1)      // words of four places, and one that is read and never asked about
 template <> struct ListShare<1> {
+    const unsigned *places;     // this lane's word of [ORDER_ROWS][64]
+    u64 ledges;                 // bit k: the entries k, k + 64, ... hold one whose projected span begins at this column (CF_PROJ and CF_LEDGE)
+    int from;                   // the entries before this one, in order, are no farther than `passed`
+    float passed;
+    bool sorted;
     static __device__ __forceinline__ u64 smallest(u64 v) { return v; }
     static __device__ __forceinline__ unsigned smallest(unsigned v) { return v; }
-    template <typename Look> __device__ __forceinline__ void each(const ColumnCtx &cc, Look look) const {
-        for (int k0 = 0; k0 < cc.count; k0 += CAND_BATCH) {
-            Cand batch[CAND_BATCH];
-            cc.cand_batch(k0, batch);
+
+    // A look at the whole list: ledges, whether some entry's span begins at this column, and the order.  COUNT: at least as many as any of the
+    // wavefront's sorted lists holds.
+    template <int COUNT> __device__ __forceinline__ void load(const ColumnCtx &cc, unsigned *words, bool &any_ledge) {
+        constexpr int BATCH = COUNT > 48 ? 4 : 8;       // as many loads at a time as there are registers for
+        unsigned keys[COUNT], own[2] = {0u, 0u}, flagged = 0u;
 #pragma unroll
-            for (int j = 0; j < CAND_BATCH; ++j)
-                if (k0 + j < cc.count) look(batch[j]);
+        for (int k0 = 0; k0 < COUNT; k0 += BATCH) {
+            Cand batch[BATCH];
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) batch[j] = cc.cand(max(min(k0 + j, cc.count - 1), 0));
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) {
+                const int k = k0 + j;
+                const bool there = k < cc.count;
+                const unsigned flags = there ? batch[j].flags : 0u;
+                flagged |= flags;
+                own[k / 32] |= (flags & (CF_LEDGE | CF_PROJ)) == (CF_LEDGE | CF_PROJ) ? 1u << (k & 31) : 0u;
+                keys[k] = there ? (__float_as_uint(batch[j].dist) & ~63u) | (unsigned)k : ~0u;
+            }
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) asm volatile("" : "+v"(keys[k0 + j]) : : "memory");
         }
+        any_ledge = flagged & CF_LEDGE;
+        ledges = own[0] | (u64)own[1] << 32;
+        order_up(keys);
+#pragma unroll
+        for (int k = 0; k < COUNT; k += 4) {
+            const unsigned low = __builtin_amdgcn_perm(keys[k + 1], keys[k], 0x0C0C0400u), high = __builtin_amdgcn_perm(keys[k + 3], keys[k + 2], 0x04000C0Cu);
+            words[(k / 4) * 64] = (low | high) & 0x3F3F3F3Fu;
+        }
+    }
+    __device__ __forceinline__ void start(const ColumnCtx &cc, unsigned *words, bool &any_ledge) {
+        places = words; ledges = 0; from = 0; passed = -1.0f;
+        sorted = cc.count <= CAND_MAX;
+        any_ledge = false;
+        const int most = wave_max(min(cc.count, CAND_MAX));
+        if (most <= 32) load<32>(cc, words, any_ledge);
+        else if (most <= 48) load<48>(cc, words, any_ledge);
+        else load<64>(cc, words, any_ledge);
+        for (int k = CAND_MAX; k < cc.count; ++k) {
+            const Cand q = cc.cand(k);
+            any_ledge |= (q.flags & CF_LEDGE) != 0;
+            ledges |= (q.flags & CF_LEDGE) && (q.flags & CF_PROJ) ? 1ULL << (k & 63) : 0ULL;
+        }
+    }
+    // A pass of the column begins: its scans ask for entries beyond `distance`.
+    __device__ __forceinline__ void begin(float distance) {
+        if (distance < passed) from = 0;
+        passed = distance;
+    }
+    // The entries beyond `passed` (and some that are not), nearest first, until those left are farther than enough().
+    template <bool ADVANCE, typename Look, typename Enough> __device__ __forceinline__ void walk(const ColumnCtx &cc, Look look, Enough enough) {
+        bool leading = sorted;
+        for (int k = from; k < cc.count;) {
+            const unsigned *row = places + (min(k, CAND_MAX - 1) >> 2) * 64;
+            const unsigned next = __builtin_amdgcn_alignbyte(row[64], row[0], (unsigned)k);
+            Cand batch[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) batch[j] = cc.cand(sorted ? (int)(next >> (8 * j) & 63u) : min(k + j, cc.count - 1));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool there = k + j < cc.count;
+                if (ADVANCE) { leading = leading && there && !(batch[j].dist > passed); from += leading ? 1 : 0; }
+                look(batch[j], there);
+            }
+            k += 4;
+            if (sorted && __uint_as_float(__float_as_uint(batch[3].dist) & ~63u) > enough()) break;
+        }
+    }
+    template <typename Look> __device__ __forceinline__ void each_ledge(const ColumnCtx &cc, Look look) const {
+        for (u64 rest = ledges; rest; rest &= rest - 1)
+            for (int k = __ffsll((long long)rest) - 1; k < cc.count; k += 64) look(cc.cand(k));
     }
 };
 
@@ -2584,7 +2645,7 @@ __device__ __forceinline__ PassRows clip_pass(const PassDraw &d, float ceiling_c
 
 // engine.py:11769-12239: selection of the pass's drawseg for one column
 template <bool SPLIT, int LANES>
-__device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ListShare<LANES> &list, const ColumnState &c, bool boundary_has_po, PassColumn &r) {
+__device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES> &list, const ColumnState &c, bool boundary_has_po, PassColumn &r) {
     const gd_map_desc *m = cc.m;
     const MapView &mv = cc.mv;
     const int x = cc.x;
@@ -2597,39 +2658,22 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ListShare
     // a. nearest incident linedef beyond previous_distance (engine.py:11769-11780)
     float distance = GD_INF; int wi = 0x7fffffff;
     Eval cwi;
-    // List positions of the candidates incident to the current sector and beyond previous_distance: the later
-    // scans of this pass ask for both (and more), so they only visit these.  Without a current sector: all.
-    // Bit b stands for the positions b, b + 64, b + 128, ... of a list longer than 64 (a spilled column's): the later
-    // scans test every candidate they visit again, so a bit that also names candidates outside the set costs a look.
-    u64 incident_beyond = cc.count >= 64 ? ~0ULL : ((1ULL << cc.count) - 1);
+    if constexpr (LANES == 1) list.begin(prev);
     if (cs >= 0) {
-        incident_beyond = 0;
         // b. equal-depth solid (engine.py:11784-11807): the nearest one-sided candidate replaces
         // the selection when it lies within 1e-3 of the nearest candidate, found in the same scan.
         u64 nearest = CAND_KEY_NONE, nearest_solid = CAND_KEY_NONE;
+        auto take = [&](const Cand &q, bool there) {
+            const u64 key = there && incident_c(q) && q.dist > prev ? cand_key(q) : CAND_KEY_NONE;
+            nearest = key < nearest ? key : nearest;
+            const u64 solid_key = q.s1 < 0 ? key : CAND_KEY_NONE;
+            nearest_solid = solid_key < nearest_solid ? solid_key : nearest_solid;
+        };
         if constexpr (LANES > 1) {
-            list.each(cc, [&](const Cand &q) {
-                const u64 key = incident_c(q) && q.dist > prev ? cand_key(q) : CAND_KEY_NONE;
-                nearest = key < nearest ? key : nearest;
-                const u64 solid_key = q.s1 < 0 ? key : CAND_KEY_NONE;
-                nearest_solid = solid_key < nearest_solid ? solid_key : nearest_solid;
-            });
+            list.each(cc, [&](const Cand &q) { take(q, true); });
             nearest = list.smallest(nearest); nearest_solid = list.smallest(nearest_solid);
-        } else for (int k0 = 0; k0 < cc.count; k0 += CAND_BATCH) {
-            Cand batch[CAND_BATCH];
-            cc.cand_batch(k0, batch);
-            unsigned batch_bits = 0u;
-#pragma unroll
-            for (int j = 0; j < CAND_BATCH; ++j) {
-                const Cand q = batch[j];
-                const bool hit = k0 + j < cc.count && incident_c(q) && q.dist > prev;
-                batch_bits |= hit ? 1u << j : 0u;
-                const u64 key = hit ? cand_key(q) : CAND_KEY_NONE;
-                nearest = key < nearest ? key : nearest;
-                const u64 solid_key = q.s1 < 0 ? key : CAND_KEY_NONE;
-                nearest_solid = solid_key < nearest_solid ? solid_key : nearest_solid;
-            }
-            incident_beyond |= (u64)batch_bits << (k0 & 63);
+        } else {
+            list.template walk<true>(cc, take, [&]() { return cand_key_distance(nearest) + 2e-3f; });
         }
         const float sd = cand_key_distance(nearest_solid);
         if (finitef(sd) && (fabsf(sd - cand_key_distance(nearest)) <= 1e-3f)) nearest = nearest_solid;
@@ -2656,8 +2700,8 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ListShare
     float ps_path_distance = distance; int ps_path_index = wi;
     bool ps_path_geo = cwi.flags & CF_GEO;
     float psd = GD_INF; int psi = 0x7fffffff; int psi_flags = 0;
-    // A later scan of the pass: over the positions `incident_beyond` names, or over all of a lane's own.  `look` says whether `ask`, of
-    // which there is one copy, has to be asked about the candidate as well.
+    // A later scan of the pass, over all of a lane's own.  `look` says whether `ask`, of which there is one copy, has to be asked about
+    // the candidate as well.
     auto look_beyond = [&](auto look, auto ask) {
         if constexpr (LANES > 1) {
             unsigned asked = 0;
@@ -2671,20 +2715,7 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ListShare
                 ask(q);
             }
         } else {
-            u64 asked = 0;
-            for (u64 rest = incident_beyond; rest;) {
-                Cand batch[CAND_BATCH]; int at[CAND_BATCH];
-                cc.cand_batch_of(rest, batch, at);
-#pragma unroll
-                for (int j = 0; j < CAND_BATCH; ++j)
-                    if (at[j] >= 0 && look(batch[j])) asked |= 1ULL << at[j];
-            }
-            for (; asked; asked &= asked - 1) ask(cc.cand(__ffsll((long long)asked) - 1));
-            for (int k = 64; k < cc.count; ++k)   // a spilled column's further entries
-                if ((incident_beyond >> (k & 63)) & 1ULL) {
-                    const Cand q = cc.cand(k);
-                    if (look(q)) ask(q);
-                }
+            list.each_ledge(cc, [&](const Cand &q) { if (look(q)) ask(q); });
         }
     };
     if (!sel_is_proj) {
@@ -2729,18 +2760,28 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, const ListShare
     const int so_s0 = mv.sec(wi, 0), so_s1 = mv.sec(wi, 1);
     if (!so_is_proj) {
         NearestOf<LANES> near;
-        look_beyond([&](const Cand &q) {
-            if (!(incident_c(q) && (q.s1 >= 0) && (q.flags & CF_PROJ) && (q.dist > prev_eps))) return false;
-            bool le = q.flags & CF_LEDGE;
-            bool same_pair = (q.s0 == so_s0 && q.s1 == so_s1) || (q.s0 == so_s1 && q.s1 == so_s0);
-            bool close = (same_pair || (le && so_excl_right && (so_narrow || (shares_sel_c(q) && so_short)))) &&
-                         (fabsf(q.dist - distance) <= tolerance_of(q.dist));
-            if (close) near.take(q);
-            return !close && le && so_excl_right && so_narrow;
-        }, [&](const Cand &q) {
-            int dummy;
-            if (mv.sector_bridge((q.flags & CF_ALONG_HI) ? 1 : 0, q.wall, no_path_index, &dummy)) near.take(q);
-        });
+        auto pairs_up = [&](const Cand &q) {
+            return ((q.s0 == so_s0 && q.s1 == so_s1) || (q.s0 == so_s1 && q.s1 == so_s0)) && (fabsf(q.dist - distance) <= tolerance_of(q.dist));
+        };
+        auto eligible = [&](const Cand &q) { return incident_c(q) && (q.s1 >= 0) && (q.flags & CF_PROJ) && (q.dist > prev_eps); };
+        // A lane alone looks for the linedefs of the same pair of sectors about `distance` (a distance that is not finite has none), and for the others, which all
+        // begin at this column, among those that do.
+        if constexpr (LANES == 1) {
+            if (finitef(distance))
+                list.template walk<false>(cc, [&](const Cand &q, bool there) { if (there && eligible(q) && pairs_up(q)) near.take(q); },
+                                          [&]() { return fmaxf(distance * 1.0080f, distance + 4.0f) + 0.25f; });
+        }
+        if (LANES > 1 || (so_excl_right && (so_narrow || so_short)))
+            look_beyond([&](const Cand &q) {
+                if (!eligible(q)) return false;
+                bool le = q.flags & CF_LEDGE;
+                bool close = pairs_up(q) || (le && so_excl_right && (so_narrow || (shares_sel_c(q) && so_short)) && (fabsf(q.dist - distance) <= tolerance_of(q.dist)));
+                if (close) near.take(q);
+                return !close && le && so_excl_right && so_narrow;
+            }, [&](const Cand &q) {
+                int dummy;
+                if (mv.sector_bridge((q.flags & CF_ALONG_HI) ? 1 : 0, q.wall, no_path_index, &dummy)) near.take(q);
+            });
         near.share();
         npd = near.distance(); npi = near.wall(); npi_flags = near.flags();
     }
@@ -3240,7 +3281,7 @@ __device__ __forceinline__ void advance_clips(const ColumnCtx &cc, ColumnState &
 
 // engine.py:13070-13371: where a pass takes its column's traversal: next sector, previous distance, pending boundaries
 template <bool SPLIT, int LANES>
-__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, const ListShare<LANES> &list, ColumnState &c, const PassColumn &r) {
+__device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ListShare<LANES> &list, ColumnState &c, const PassColumn &r) {
     const gd_map_desc *m = cc.m;
     const MapView &mv = cc.mv;
     const LaneCtx &L = *cc.c;
@@ -3268,8 +3309,9 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, const ListShar
         const unsigned none = __float_as_uint(GD_INF);
         unsigned current_solid = none, other_solid = none;      // distances: positive, so their bits order as they do
         const int v0 = mv.vert(wi, 0), v1 = mv.vert(wi, 1);
-        list.each(cc, [&](const Cand &q) {
+        auto look = [&](const Cand &q, bool there) {
             const float d = q.dist;
+            if (!there) return;
             bool os = q.s1 < 0;
             bool inc = (q.s0 == cur || q.s1 == cur), oinc = (q.s0 == other_sector || q.s1 == other_sector);
             bool future = ((q.flags & CF_GEO) || os) && (d > dist_eps);
@@ -3281,7 +3323,9 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, const ListShar
             if (shared_solid && oinc) other_solid = min(other_solid, __float_as_uint(d));
             bool sgp = (q.flags & CF_GEO) && inc && shares_endpoint && !os && (d > prior_eps) && (fabsf(d - distance) <= (1.0f / 16.0f));
             if (sgp) geometric.take(q);
-        });
+        };
+        if constexpr (LANES > 1) list.each(cc, [&](const Cand &q) { look(q, true); });
+        else list.template walk<false>(cc, look, [&]() { return fmaxf(fmaxf(current_next.distance(), other_next.distance()), distance + 0.07f); });
         current_next.share(); other_next.share(); geometric.share();
         current_solid = list.smallest(current_solid); other_solid = list.smallest(other_solid);
         const float cnd = current_next.distance(), ond = other_next.distance(), csd = __uint_as_float(current_solid), osd = __uint_as_float(other_solid);
@@ -3720,7 +3764,7 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int str
 static_assert(SEG_COLS == 64, "wall_select_kernel: a work-group is one wavefront, with columns of one strip");
 // The columns of one wavefront: 64 / LANES of a strip's, from the `part`-th such share on.
 template <bool SPLIT, int LANES>
-__device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratch &sc, const LaneCtx &lane_ctx, int local, int strip_x, int part) {
+__device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratch &sc, const LaneCtx &lane_ctx, unsigned (&order_lds)[ORDER_ROWS][64], int local, int strip_x, int part) {
     const gd_map_desc *m = &dm.d;
     constexpr bool SHARED = LANES > 1;
     constexpr int part_cols = 64 / LANES;
@@ -3749,14 +3793,7 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     st.previous_distance = 0.0f;
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
-    if (!SHARED) {
-        for (int k0 = 0; k0 < cc.count && !boundary_has_po; k0 += CAND_BATCH) {
-            Cand batch[CAND_BATCH];
-            cc.cand_batch(k0, batch);
-#pragma unroll
-            for (int j = 0; j < CAND_BATCH; ++j) boundary_has_po |= (batch[j].flags & CF_LEDGE) != 0;   // slots past the end repeat the last entry
-        }
-    }
+    if constexpr (!SHARED) list.start(cc, &order_lds[0][lane_id], boundary_has_po);
     PassRec *records = sc.pass_rec + sc.pass_at(0, local, x);
     float *path_distances = sc.pass_path_distance + sc.pass_at(0, local, x);
     const size_t pass_stride = (size_t)sc.lane_stride * SW;
@@ -3819,6 +3856,7 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
 template <bool SPLIT, int LANES>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES == 8 ? 3 : 4))) wall_select_kernel(DeviceMap dm, Scratch sc, int first, int longest) {
     __shared__ LaneCtx lane_ctx;
+    __shared__ unsigned order_lds[ORDER_ROWS][64];
     const int shares = longest * LANES, others = (int)gridDim.x - shares, mixed = min(shares, others) & ~7, b = (int)blockIdx.x;
     const bool beyond = b < 2 * mixed ? (b & 8) != 0 : shares - mixed <= b - 2 * mixed;
     const int at = b < 2 * mixed ? ((b >> 4) << 3) | (b & 7) : (beyond ? b - shares : b - mixed);
@@ -3829,11 +3867,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES =
     if constexpr (LANES > 1) {
         // A strip with a column in the spill pool (more entries than its lanes hold) is the first of its wavefronts', a lane a column.
         if (beyond || __ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + threadIdx.x] >> SPILL_SHIFT) != 0) != 0) {
-            if (beyond || part == 0) select_columns<SPLIT, 1>(dm, sc, lane_ctx, local, strip_x, 0);
+            if (beyond || part == 0) select_columns<SPLIT, 1>(dm, sc, lane_ctx, order_lds, local, strip_x, 0);
             return;
         }
     }
-    select_columns<SPLIT, LANES>(dm, sc, lane_ctx, local, strip_x, part);
+    select_columns<SPLIT, LANES>(dm, sc, lane_ctx, order_lds, local, strip_x, part);
 }
 
 // One wavefront per 64 / SEG_COLS segments.  Segments share nothing but read-only tables; a work-group of the drawing
