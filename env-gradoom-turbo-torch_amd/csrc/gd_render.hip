@@ -178,6 +178,22 @@ struct __align__(16) WallSide {
     i64 spare2;
 };
 
+// What the selection asks about a linedef it has come to, whatever the camera: in one place, so that it waits for memory once.  A pass is a chain of
+// loads that depend on one another, a trip to memory each: next to a table for sectors, one for vertices, one for neighbours, two for the bridges' ranges
+// (and the neighbours' ray tests asked for one after the other, a bridge's linedefs by number and then by sectors, linedef 0 again in every pass that finds
+// none) the launch for the longest strips takes 385 us instead of 433 at 4096 lanes of the 4000-linedef map, the other 788 instead of 800; 1024 lanes of the
+// 2000-linedef map 232 instead of 248 and 191 instead of 202.
+struct __align__(16) WallLinks {
+    unsigned sectors;        // front | back << 16 (0xFFFF: none)
+    unsigned vertices;       // start | end << 16
+    int neighbour[2];        // direct_neighbor_table's row
+    unsigned slots;
+    int solid[2];            // where its entries in the solid bridge lists start, by its start and by its end
+    unsigned solid_counts;   // how many they are, start | end << 16
+};
+// A vertex's linedefs with their sectors (vertex_wall_idx and wall_sectors in one place)
+struct VertexLink { int wall; unsigned sectors; };
+
 struct RecSpan {   // what a ray test of one linedef needs (eval_segment), kept for every linedef of the map; the full record
                    // above exists only for the linedefs the camera can see at all
     short pl, pr;
@@ -236,6 +252,8 @@ struct DeviceMap {  // device copy of gd_map_desc (device pointers) + fixed tabl
     const unsigned int *sprite_texels;   // [patches, spr_max_h, spr_max_w] texel | its post's first row << 8 | opaque << 16: one load instead of three
     const int *masked_slot;              // [W] number of the linedef among those with a mid-texture on a two-sided side, else -1
     int masked_count;                    // how many there are
+    const WallLinks *wall_links;         // [W]
+    const VertexLink *vertex_links;      // by vertex_wall_ofs
     const int *wall_facts;               // [W] WALL_*, and from bit WALL_BLOCKING_SHIFT on the linedef's position in blocking_walls plus one, 0 when it does not block
     const unsigned int *sector_level;    // [S] index of the floor in floor_levels | index of the ceiling in ceil_levels << 16;
                                          // null when some sector's height is missing from the level lists
@@ -391,59 +409,62 @@ __device__ __forceinline__ float tolerance_of(float d) { return fmaxf(fabsf(d) /
 // ---------------------------------------------------------------------------------------------
 // map relations (engine.py:399-484, 1578-1612), answered from vertex ids and the vertex CSR
 // ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ int link_sector(unsigned sectors, int side) { return (int)(short)(side ? sectors >> 16 : sectors & 0xFFFFu); }
+__device__ __forceinline__ int link_vertex(unsigned vertices, int slot) { return (int)(slot ? vertices >> 16 : vertices & 0xFFFFu); }
 struct MapView {
     const gd_map_desc *m;
-    __device__ int sec(int w, int side) const { return m->wall_sectors[2 * w + side]; }
-    __device__ int vert(int w, int slot) const { return m->wall_vertex[2 * w + slot]; }
-    __device__ bool one_sided(int w) const { return m->wall_sectors[2 * w + 1] < 0; }
-    __device__ bool two_sided_distinct(int w) const { return sec(w, 0) >= 0 && sec(w, 1) >= 0 && sec(w, 0) != sec(w, 1); }
-    __device__ bool same_pair(int a, int b) const {
-        int a0 = sec(a, 0), a1 = sec(a, 1), b0 = sec(b, 0), b1 = sec(b, 1);
-        return (a0 == b0 && a1 == b1) || (a0 == b1 && a1 == b0);
+    const WallLinks *walls;
+    const VertexLink *vertex_links;
+    // are a's and b's sectors the same two?
+    static __device__ __forceinline__ bool same_pair(unsigned a, unsigned b) { return a == b || a == (b >> 16 | b << 16); }
+    static __device__ __forceinline__ bool incident(unsigned sectors, int sector) { return link_sector(sectors, 0) == sector || link_sector(sectors, 1) == sector; }
+    static __device__ __forceinline__ bool has_vertex(unsigned vertices, int v) { return link_vertex(vertices, 0) == v || link_vertex(vertices, 1) == v; }
+    static __device__ __forceinline__ bool two_sided_distinct(unsigned sectors) {
+        const int front = link_sector(sectors, 0), back = link_sector(sectors, 1);
+        return front >= 0 && back >= 0 && front != back;
     }
-    __device__ bool shares_any_endpoint(int a, int b) const {
-        int a0 = vert(a, 0), a1 = vert(a, 1), b0 = vert(b, 0), b1 = vert(b, 1);
-        return a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1;
-    }
-    __device__ bool opposing(int a, int b) const {
-        if (!same_pair(a, b) || sec(a, 1) < 0 || sec(b, 1) < 0 || shares_any_endpoint(a, b)) return false;
-        const float *wa = m->walls + 4 * a, *wb = m->walls + 4 * b;
-        float ax = wa[2] - wa[0], ay = wa[3] - wa[1], bx = wb[2] - wb[0], by = wb[3] - wb[1];
+    __device__ __forceinline__ bool opposing(int a, unsigned a_sectors, unsigned a_vertices, int b, unsigned b_sectors, unsigned b_vertices) const {
+        if (!same_pair(a_sectors, b_sectors) || link_sector(a_sectors, 1) < 0 || link_sector(b_sectors, 1) < 0 ||
+            has_vertex(b_vertices, link_vertex(a_vertices, 0)) || has_vertex(b_vertices, link_vertex(a_vertices, 1))) return false;
+        const float4 wa = *reinterpret_cast<const float4 *>(m->walls + 4 * a), wb = *reinterpret_cast<const float4 *>(m->walls + 4 * b);
+        float ax = wa.z - wa.x, ay = wa.w - wa.y, bx = wb.z - wb.x, by = wb.w - wb.y;
         float dot = ax * bx + ay * by;
         float cross = ax * by - ay * bx;
         return dot < 0 && fabsf(cross) < 1e-6f;
     }
-    __device__ bool triangle_bridge(int vertex, int a, int b, int *index) const {
-        *index = 0;
-        if (!two_sided_distinct(a) || !two_sided_distinct(b)) return false;
-        int a0 = sec(a, 0), a1 = sec(a, 1), b0 = sec(b, 0), b1 = sec(b, 1);
+    // the one linedef at `vertex` between the two sectors that `a` and `b` do not share, and its sectors
+    __device__ bool triangle_bridge(int vertex, int a, unsigned a_sectors, int b, unsigned b_sectors, int *index, unsigned *sectors) const {
+        *index = 0; *sectors = 0;
+        if (!two_sided_distinct(a_sectors) || !two_sided_distinct(b_sectors)) return false;
+        int a0 = link_sector(a_sectors, 0), a1 = link_sector(a_sectors, 1), b0 = link_sector(b_sectors, 0), b1 = link_sector(b_sectors, 1);
         int shared_count = (a0 == b0 || a0 == b1) + (a1 == b0 || a1 == b1);
         if (shared_count != 1) return false;
         int shared = (a0 == b0 || a0 == b1) ? a0 : a1;
-        int pa = (a0 == shared) ? a1 : a0;
-        int pb = (b0 == shared) ? b1 : b0;
+        const unsigned between = (unsigned)((a0 == shared) ? a1 : a0) | (unsigned)((b0 == shared) ? b1 : b0) << 16;
         int found = -1, count = 0;
-        for (int k = m->vertex_wall_ofs[vertex]; k < m->vertex_wall_ofs[vertex + 1]; ++k) {
-            int w = m->vertex_wall_idx[k];
-            if (w == a || w == b) continue;
-            int s0 = sec(w, 0), s1 = sec(w, 1);
-            if ((s0 == pa && s1 == pb) || (s0 == pb && s1 == pa)) { found = w; ++count; }
+        const int first = m->vertex_wall_ofs[vertex], last = m->vertex_wall_ofs[vertex + 1];
+        for (int k = first; k < last; k += 4) {      // a vertex has four linedefs or so: all of them at once
+            VertexLink link[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) link[j] = vertex_links[min(k + j, last - 1)];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (k + j < last && link[j].wall != a && link[j].wall != b && same_pair(link[j].sectors, between)) { found = link[j].wall; *sectors = link[j].sectors; ++count; }
         }
         if (count != 1) return false;
         *index = found;
         return true;
     }
-    __device__ bool portal_bridge(int slot, int path, int owner, int *index) const {
+    __device__ bool portal_bridge(int slot, int path, unsigned path_sectors, unsigned path_vertices, int owner, unsigned owner_sectors, unsigned owner_vertices, int *index) const {
         *index = 0;
         if (owner == path) return false;
-        int v = vert(path, slot);
-        if (vert(owner, 0) != v && vert(owner, 1) != v) return false;
-        return triangle_bridge(v, path, owner, index);
+        const int v = link_vertex(path_vertices, slot);
+        unsigned sectors;
+        return has_vertex(owner_vertices, v) && triangle_bridge(v, path, path_sectors, owner, owner_sectors, index, &sectors);
     }
-    __device__ bool sector_bridge(int slot, int pending, int path, int *index) const {
-        *index = 0;
-        if (path == pending) return false;
-        return triangle_bridge(vert(pending, slot), pending, path, index);
+    __device__ bool sector_bridge(int vertex, int pending, unsigned pending_sectors, int path, unsigned path_sectors, int *index, unsigned *sectors) const {
+        *index = 0; *sectors = 0;
+        return path != pending && triangle_bridge(vertex, pending, pending_sectors, path, path_sectors, index, sectors);
     }
 };
 
@@ -2044,6 +2065,7 @@ struct ColumnCtx {
     int count;
     int x;
     float rx, ry;
+    Eval first;           // linedef 0 at this column, which stands in where a pass finds none
     __device__ __forceinline__ const WallRec &rec(int w) const { return recs[rec_base + (unsigned)w]; }
     // Where the list of column `x` of the chunk's lane `local` starts and how many entries it has: the column's own
     // slots, or its slot in the spill pool.
@@ -2359,31 +2381,32 @@ __device__ __forceinline__ i64 wall_shade(float light, i64 visibility) {
     return clampi((shade - min64(visibility, 24 * FIXED_UNIT)) >> 16, 0, 31);
 }
 
-// engine.py:11596-11730 for one (column, linedef)
-__device__ __forceinline__ void endpoint_owner(const ColumnCtx &cc, int w, const Eval &cw, int *owner_index, float *owner_distance) {
+// engine.py:11596-11730 for one (column, linedef): the owner and, if that is another linedef, what its ray test says
+__device__ __forceinline__ void endpoint_owner(const ColumnCtx &cc, int w, const Eval &cw, const WallLinks &links, int *owner_index, Eval *owner) {
     const gd_map_desc *m = cc.m;
     const int K = m->neighbor_slots;
     const bool subpixel = cw.flags & CF_SUBPIXEL;
     float tol_w = tolerance_of(cw.dist);
+    *owner_index = w; *owner = cw;
     // the owner only matters for a linedef that does not own this column itself (engine.py:11716)
-    if (cw.flags & CF_PROJ) { *owner_index = w; *owner_distance = cw.dist; return; }
+    if (cw.flags & CF_PROJ) return;
     bool uses_start = !(cw.flags & CF_ALONG_HI);
-    int index; float distance; bool valid;
+    int index; Eval found; bool valid;
     if (m->direct_neighbors) {
-        // {start neighbour, end neighbour, start slot | end slot << 8 | has start << 16 | has end << 17}
-        const int4 nb = *reinterpret_cast<const int4 *>(m->direct_neighbor_table + 4 * w);
-        int ss = nb.z & 0xFF, es = (nb.z >> 8) & 0xFF; bool hs = (nb.z >> 16) & 1, he = (nb.z >> 17) & 1;
+        // slots: start slot | end slot << 8 | has start << 16 | has end << 17
+        int ss = links.slots & 0xFF, es = (links.slots >> 8) & 0xFF; bool hs = (links.slots >> 16) & 1, he = (links.slots >> 17) & 1;
         int rslot = uses_start ? ss : es, oslot = uses_start ? es : ss;
         bool rexists = uses_start ? hs : he, oexists = uses_start ? he : hs;
-        int rn = uses_start ? nb.x : nb.y, on = uses_start ? nb.y : nb.x;
+        int rn = uses_start ? links.neighbour[0] : links.neighbour[1], on = uses_start ? links.neighbour[1] : links.neighbour[0];
         Eval r = cc.eval(rn);
         bool r_owns = rexists && (r.flags & CF_PROJ) && (r.flags & CF_LEDGE);
-        Eval o = (on == rn) ? r : cc.eval(on);
-        bool o_owns = subpixel && oexists && (o.flags & CF_PROJ) && (o.flags & CF_LEDGE) && (fabsf(o.dist - cw.dist) <= tol_w);
-        bool use_o = o_owns && (!r_owns || (o.dist < r.dist) || ((o.dist == r.dist) && (oslot < rslot)));
-        index = use_o ? on : rn;
-        distance = use_o ? o.dist : r.dist;
-        valid = r_owns || o_owns;
+        index = rn; found = r; valid = r_owns;
+        if (subpixel && oexists) {
+            Eval o = cc.eval(on);
+            bool o_owns = (o.flags & CF_PROJ) && (o.flags & CF_LEDGE) && (fabsf(o.dist - cw.dist) <= tol_w);
+            if (o_owns && (!r_owns || (o.dist < r.dist) || ((o.dist == r.dist) && (oslot < rslot)))) { index = on; found = o; }
+            valid = r_owns || o_owns;
+        }
     } else {
         float best = GD_INF; int best_slot = 0;
         for (int k = 0; k < K; ++k) {
@@ -2396,12 +2419,10 @@ __device__ __forceinline__ void endpoint_owner(const ColumnCtx &cc, int w, const
             if (v < best) { best = v; best_slot = k; }
         }
         index = m->endpoint_neighbors[w * K + best_slot];
-        distance = best;
         valid = finitef(best);
+        if (valid) found = cc.eval(index);
     }
-    bool has = !(cw.flags & CF_PROJ) && valid;
-    *owner_index = has ? index : w;
-    *owner_distance = has ? distance : cw.dist;
+    if (valid) { *owner_index = index; *owner = found; }
 }
 
 
@@ -2413,6 +2434,7 @@ struct ColumnState {   // engine.py:11561-11580, 11735-11762
     float previous_distance;
     int pend_po_vertex, pend_ep_vertex, pend_ep_wall, pend_eb_index, pend_pb_index, pend_pb_sector;
     float pend_pb_exit;
+    unsigned pend_ep_sectors, pend_ep_vertices;   // pend_ep_wall's
     int flags;  // bit0 pend_po_boundary, bit1 pend_ep_boundary, bit2 pend_eb_boundary, bit3 pend_pb
 };
 #define ST_PO 1
@@ -2435,6 +2457,7 @@ struct PassColumn {
     float distance;
     int ps_path_index, ps_other, no_path_other, sel_vertex, fb_idx;
     float ps_path_distance, no_path_distance;
+    unsigned sectors, vertices;   // wall's
     int bits, marks;       // PB_*, REC_*
 };
 #define PB_VALID 0x1
@@ -2653,7 +2676,6 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
     const int cur = cs < 0 ? 0 : cs;
     const float prev = c.previous_distance;
     const float prev_eps = prev + 1e-3f;
-    auto incident = [&](int w) { return mv.sec(w, 0) == cur || mv.sec(w, 1) == cur; };
     auto incident_c = [&](const Cand &q) { return q.s0 == cur || q.s1 == cur; };
     // a. nearest incident linedef beyond previous_distance (engine.py:11769-11780)
     float distance = GD_INF; int wi = 0x7fffffff;
@@ -2680,10 +2702,11 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
         distance = cand_key_distance(nearest); wi = cand_key_wall(nearest);
         cwi.dist = distance; cwi.flags = cand_key_flags(nearest);
     }
-    if (!finitef(distance)) { wi = 0; cwi = cc.eval(0); }
+    if (!finitef(distance)) { wi = 0; cwi = cc.first; }
+    WallLinks links = mv.walls[wi];
     // c. selected endpoint (engine.py:11815-11871)
     bool sel_start = !(cwi.flags & CF_ALONG_HI);
-    int sel_vertex = mv.vert(wi, sel_start ? 0 : 1);
+    int sel_vertex = link_vertex(links.vertices, sel_start ? 0 : 1);
     auto shares_sel_c = [&](const Cand &q) { return (int)q.v0 == sel_vertex || (int)q.v1 == sel_vertex; };
     bool continues_po_boundary = (c.flags & ST_PO) && (sel_vertex == c.pend_po_vertex);
     bool continues_ep_boundary = (c.flags & ST_EP) && (sel_vertex == c.pend_ep_vertex);
@@ -2691,13 +2714,14 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
     // the forward bridge only matters while an endpoint-projected boundary continues
     int fb_idx = 0;
     bool pend_ep_has_forward_bridge = false;
-    if (continues_ep_boundary && mv.portal_bridge(sel_slot, wi, c.pend_ep_wall, &fb_idx))
+    if (continues_ep_boundary && mv.portal_bridge(sel_slot, wi, links.sectors, links.vertices, c.pend_ep_wall, c.pend_ep_sectors, c.pend_ep_vertices, &fb_idx))
         pend_ep_has_forward_bridge = cc.eval(fb_idx).dist > distance + 1e-3f;
     bool completes_pending_endpoint_bridge = (c.flags & ST_EB) && (wi == c.pend_eb_index);
     bool sel_is_proj = cwi.flags & CF_PROJ;
     bool sel_excl_right = cwi.flags & CF_ENDS_HERE;
     // d. projected solid owner (engine.py:11872-11954)
     float ps_path_distance = distance; int ps_path_index = wi;
+    const unsigned ps_sectors = links.sectors;
     bool ps_path_geo = cwi.flags & CF_GEO;
     float psd = GD_INF; int psi = 0x7fffffff; int psi_flags = 0;
     // A later scan of the pass, over all of a lane's own.  `look` says whether `ask`, of which there is one copy, has to be asked about
@@ -2727,13 +2751,14 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
         solid.share();
         psd = solid.distance(); psi = solid.wall(); psi_flags = solid.flags();
         if (sel_excl_right) {
-            const int *ofs = sel_start ? m->solid_bridge_start_ofs : m->solid_bridge_end_ofs;
-            const int *idx = sel_start ? m->solid_bridge_start_idx : m->solid_bridge_end_idx;
+            const int *idx = (sel_start ? m->solid_bridge_start_idx : m->solid_bridge_end_idx) + links.solid[sel_start ? 0 : 1];
+            const int bridges = sel_start ? links.solid_counts & 0xFFFFu : links.solid_counts >> 16;
             float sbd = GD_INF; int sbi = 0; int sbi_flags = 0;
-            for (int k = ofs[wi]; k < ofs[wi + 1]; ++k) {
+            for (int k = 0; k < bridges; ++k) {
                 int b = idx[k];
-                if (!(incident(b) && mv.one_sided(b))) continue;
+                const unsigned bridge_sectors = mv.walls[b].sectors;
                 Eval q = cc.eval(b);
+                if (!(MapView::incident(bridge_sectors, cur) && link_sector(bridge_sectors, 1) < 0)) continue;
                 bool owner = (q.flags & CF_PROJ) && (q.flags & CF_LEDGE) && (q.dist > prev_eps);
                 float v = owner ? q.dist : GD_INF;
                 if (v < sbd) { sbd = v; sbi = b; sbi_flags = q.flags; }   // list is ascending: first slot wins ties
@@ -2742,22 +2767,24 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
         }
     }
     bool has_ps = finitef(psd);
-    if (has_ps) { distance = psd; wi = psi; cwi.dist = psd; cwi.flags = psi_flags; }
+    if (has_ps) { distance = psd; wi = psi; cwi.dist = psd; cwi.flags = psi_flags; links = mv.walls[wi]; }
     // e. endpoint owner (engine.py:11960-12001)
-    int eo_idx; float eo_dist;
-    endpoint_owner(cc, wi, cwi, &eo_idx, &eo_dist);
+    int eo_idx; Eval eo;
+    endpoint_owner(cc, wi, cwi, links, &eo_idx, &eo);
     bool eo_path_geo = cwi.flags & CF_GEO;
-    bool replace_eo = (eo_idx != wi) && (eo_dist > prev_eps);
-    if (replace_eo) { distance = eo_dist; wi = eo_idx; cwi = cc.eval(wi); }
+    bool replace_eo = (eo_idx != wi) && (eo.dist > prev_eps);
+    unsigned sectors = links.sectors, vertices = links.vertices;     // wi's
+    if (replace_eo) { distance = eo.dist; wi = eo_idx; cwi = eo; sectors = mv.walls[wi].sectors; vertices = mv.walls[wi].vertices; }
     int no_path_index = wi; float no_path_distance = distance;
+    const unsigned no_path_sectors = sectors;
     bool no_path_geo = replace_eo ? eo_path_geo : (bool)(cwi.flags & CF_GEO);
-    bool no_from_front = cs == mv.sec(no_path_index, 0);
-    int no_path_other = no_from_front ? mv.sec(no_path_index, 1) : mv.sec(no_path_index, 0);
+    bool no_from_front = cs == link_sector(no_path_sectors, 0);
+    int no_path_other = link_sector(no_path_sectors, no_from_front ? 1 : 0);
     // f. near projected owner (engine.py:12002-12179)
     bool so_is_proj = cwi.flags & CF_PROJ;
     const bool so_excl_right = cwi.flags & CF_ENDS_HERE, so_narrow = cwi.flags & CF_NARROW, so_short = cwi.flags & CF_SHORT;
     float npd = GD_INF; int npi = 0x7fffffff; int npi_flags = 0;
-    const int so_s0 = mv.sec(wi, 0), so_s1 = mv.sec(wi, 1);
+    const int so_s0 = link_sector(sectors, 0), so_s1 = link_sector(sectors, 1);
     if (!so_is_proj) {
         NearestOf<LANES> near;
         auto pairs_up = [&](const Cand &q) {
@@ -2779,24 +2806,26 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
                 if (close) near.take(q);
                 return !close && le && so_excl_right && so_narrow;
             }, [&](const Cand &q) {
-                int dummy;
-                if (mv.sector_bridge((q.flags & CF_ALONG_HI) ? 1 : 0, q.wall, no_path_index, &dummy)) near.take(q);
+                int bridge; unsigned bridge_sectors;
+                const unsigned pair = (unsigned)(unsigned short)q.s0 | (unsigned)(unsigned short)q.s1 << 16;
+                if (mv.sector_bridge((q.flags & CF_ALONG_HI) ? q.v1 : q.v0, q.wall, pair, no_path_index, no_path_sectors, &bridge, &bridge_sectors)) near.take(q);
             });
         near.share();
         npd = near.distance(); npi = near.wall(); npi_flags = near.flags();
     }
     int pe_wall = c.pend_ep_wall;
-    int pe_s0 = mv.sec(pe_wall, 0), pe_s1 = mv.sec(pe_wall, 1);
+    int pe_s0 = link_sector(c.pend_ep_sectors, 0), pe_s1 = link_sector(c.pend_ep_sectors, 1);
     bool pe_from_current = cs == pe_s0;
     bool pe_incident = pe_from_current || (cs == pe_s1);
     int pe_other = pe_from_current ? pe_s1 : pe_s0;
     bool use_psb = false; int psb_idx = 0;
     if ((c.flags & ST_EP) && pe_incident && (pe_other >= 0) && (no_path_other >= 0) && no_path_geo && !so_is_proj && so_excl_right &&
         (cc.rec(pe_wall).sr - cc.rec(pe_wall).sl <= 1)) {
-        int pe_slot = (c.pend_ep_vertex == mv.vert(pe_wall, 1)) ? 1 : 0;
-        bool psb_exists = mv.sector_bridge(pe_slot, pe_wall, no_path_index, &psb_idx);
+        int pe_slot = (c.pend_ep_vertex == link_vertex(c.pend_ep_vertices, 1)) ? 1 : 0;
+        unsigned psb_sectors;
+        bool psb_exists = mv.sector_bridge(link_vertex(c.pend_ep_vertices, pe_slot), pe_wall, c.pend_ep_sectors, no_path_index, no_path_sectors, &psb_idx, &psb_sectors);
         if (psb_exists) {
-            int b0 = mv.sec(psb_idx, 0), b1 = mv.sec(psb_idx, 1);
+            int b0 = link_sector(psb_sectors, 0), b1 = link_sector(psb_sectors, 1);
             bool matches = (b0 == pe_other && b1 == no_path_other) || (b1 == pe_other && b0 == no_path_other);
             Eval qb = cc.eval(psb_idx);
             float pe_tol = tolerance_of(cc.eval(pe_wall).dist);
@@ -2805,9 +2834,9 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
         }
     }
     bool replace_np = finitef(npd);
-    if (replace_np) { distance = npd; wi = npi; cwi.dist = npd; cwi.flags = npi_flags; }
+    if (replace_np) { distance = npd; wi = npi; cwi.dist = npd; cwi.flags = npi_flags; sectors = mv.walls[wi].sectors; vertices = mv.walls[wi].vertices; }
     bool final_proj = cwi.flags & CF_PROJ, final_geo = cwi.flags & CF_GEO;
-    bool completes_poab = (c.flags & ST_EP) && final_proj && !final_geo && mv.opposing(pe_wall, wi);
+    bool completes_poab = (c.flags & ST_EP) && final_proj && !final_geo && mv.opposing(pe_wall, c.pend_ep_sectors, c.pend_ep_vertices, wi, sectors, vertices);
     // g. validity (engine.py:12197-12239)
     bool valid = finitef(distance);
     bool excl_only = !so_is_proj && so_excl_right && !replace_np && so_narrow && !boundary_has_po;
@@ -2816,26 +2845,26 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
     bool geometric_intersection = replace_np ? no_path_geo : (replace_eo ? eo_path_geo : final_geo);
     bool no_keeps = replace_np && no_path_geo && (no_path_other >= 0);
     // h. sides (engine.py:12240-12292)
-    int front = mv.sec(wi, 0), back = mv.sec(wi, 1);
+    int front = link_sector(sectors, 0), back = link_sector(sectors, 1);
     bool from_front = cs == front;
     int other_sector = from_front ? back : front;
     int render_current = use_psb ? pe_other : (completes_poab ? other_sector : cur);
     bool render_from_front = render_current == front;
     int render_other = render_from_front ? back : front;
     int side = render_from_front ? 0 : 1;
-    bool ps_from_front = cs == mv.sec(ps_path_index, 0);
-    int ps_other = ps_from_front ? mv.sec(ps_path_index, 1) : mv.sec(ps_path_index, 0);
+    bool ps_from_front = cs == link_sector(ps_sectors, 0);
+    int ps_other = link_sector(ps_sectors, ps_from_front ? 1 : 0);
     bool ps_keeps = has_ps && ps_path_geo && (ps_other >= 0);
     bool one_sided = other_sector < 0;
 
     // Can the rows of the pass be read off its linedefs' lines (WallGeo)?  Not through BSP fragments, and only where the sector
     // drawn from is the one its side (and its portal path's side) faces.
     bool own_rows = render_current != (render_from_front ? front : back) || (!one_sided && back < 0) ||
-                    (ps_keeps && render_current != (ps_from_front ? cs : mv.sec(ps_path_index, 1)));
+                    (ps_keeps && render_current != (ps_from_front ? cs : link_sector(ps_sectors, 1)));
     if (SPLIT) own_rows = own_rows || m->wall_split_slot[wi] >= 0 || (ps_keeps && m->wall_split_slot[ps_path_index] >= 0);
     r.marks = (side ? REC_SIDE1 : 0) | (own_rows ? REC_OWN_ROWS : 0);
     r.wall = wi; r.side = side; r.render_current = render_current; r.other_sector = other_sector;
-    r.distance = distance;
+    r.distance = distance; r.sectors = sectors; r.vertices = vertices;
     r.ps_path_index = ps_path_index; r.ps_other = ps_other; r.no_path_other = no_path_other; r.sel_vertex = sel_vertex; r.fb_idx = fb_idx;
     r.ps_path_distance = ps_path_distance; r.no_path_distance = no_path_distance;
     r.bits = (valid ? PB_VALID : 0) | (raster_valid ? PB_RASTER : 0) | (one_sided ? PB_ONE_SIDED : 0) |
@@ -3292,7 +3321,6 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ListShare<LANE
     const int wi = r.wall;
     const float distance = r.distance;
     const bool valid = r.bits & PB_VALID, one_sided = r.bits & PB_ONE_SIDED;
-    auto incident = [&](int w) { return mv.sec(w, 0) == cur || mv.sec(w, 1) == cur; };
     // s. next sector (engine.py:13070-13241)
     const float prior = before.previous_distance;
     const float prior_eps = prior + 1e-3f;
@@ -3308,7 +3336,7 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ListShare<LANE
         NearestOf<LANES> current_next, other_next, geometric;
         const unsigned none = __float_as_uint(GD_INF);
         unsigned current_solid = none, other_solid = none;      // distances: positive, so their bits order as they do
-        const int v0 = mv.vert(wi, 0), v1 = mv.vert(wi, 1);
+        const int v0 = link_vertex(r.vertices, 0), v1 = link_vertex(r.vertices, 1);
         auto look = [&](const Cand &q, bool there) {
             const float d = q.dist;
             if (!there) return;
@@ -3335,17 +3363,19 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ListShare<LANE
         gpd = geometric.distance();
         if (!finitef(cnd)) cni = 0;
         if (!finitef(ond)) oni = 0;
-        bool enters_tied_strip = finitef(cnd) && (cni == oni) && mv.opposing(wi, cni);
+        bool enters_tied_strip = false;
+        if (finitef(cnd) && cni == oni) { const WallLinks &tied = mv.walls[cni]; enters_tied_strip = mv.opposing(wi, r.sectors, r.vertices, cni, tied.sectors, tied.vertices); }
         bool enters_other = (other_sector >= 0) && ((ond < cnd) || enters_tied_strip);
         bool enters_shared = (other_sector >= 0) && (osd < csd);
         bool uses_geometric_path = false;
         if (finitef(gpd)) {
-            bool gp_from_front = cs == mv.sec(gpi, 0);
-            gp_other = gp_from_front ? mv.sec(gpi, 1) : mv.sec(gpi, 0);
+            const unsigned gp_sectors = mv.walls[gpi].sectors, gp_vertices = mv.walls[gpi].vertices;
+            bool gp_from_front = cs == link_sector(gp_sectors, 0);
+            gp_other = link_sector(gp_sectors, gp_from_front ? 1 : 0);
             uses_geometric_path = gp_other >= 0;
             if (uses_geometric_path) {
                 int pb_slot = gp_along_hi ? 1 : 0;
-                bool ppb_exists = mv.portal_bridge(pb_slot, gpi, wi, &ppb_idx);
+                bool ppb_exists = mv.portal_bridge(pb_slot, gpi, gp_sectors, gp_vertices, wi, r.sectors, r.vertices, &ppb_idx);
                 if (ppb_exists) {
                     Eval qb = cc.eval(ppb_idx);
                     endpoint_portal_bridge = (qb.flags & CF_PROJ) && (qb.flags & CF_LEDGE) && (qb.dist > prior_eps) && (fabsf(qb.dist - gpd) <= tolerance_of(gpd));
@@ -3383,8 +3413,8 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ListShare<LANE
     if (starts_po) c.pend_po_vertex = r.sel_vertex;
     bool po = starts_po || ((before.flags & ST_PO) && (r.bits & PB_CONTINUES_PO));
     if (endpoint_only_portal) {
-        c.pend_ep_vertex = mv.vert(wi, (r.bits & PB_FINAL_ALONG_HI) ? 1 : 0);
-        c.pend_ep_wall = wi;
+        c.pend_ep_vertex = link_vertex(r.vertices, (r.bits & PB_FINAL_ALONG_HI) ? 1 : 0);
+        c.pend_ep_wall = wi; c.pend_ep_sectors = r.sectors; c.pend_ep_vertices = r.vertices;
     }
     if (r.bits & PB_FORWARD_BRIDGE) c.pend_eb_index = r.fb_idx;
     if (endpoint_portal_bridge) next_sector = other_sector;
@@ -3414,7 +3444,7 @@ __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const Col
     const MaskedGeo &masked = sc.masked_geo[(size_t)local * dm.masked_count + dm.masked_slot[mw]];
     const int texture_id = ws.tex[0];
     const Tables &tb = *cc.tb;
-    const int front_sector = cc.mv.sec(mw, 0), back_sector = cc.mv.sec(mw, 1);
+    const int front_sector = m->wall_sectors[2 * mw], back_sector = m->wall_sectors[2 * mw + 1];
     const int light_sector = mside == 0 ? front_sector : back_sector;
     const float world_top = fminf(tb.ceil_h(front_sector), tb.ceil_h(back_sector));
     const int th = m->tex_h[texture_id];   // the texture's own height, whatever its row mask (engine.py:13480-13483)
@@ -3771,13 +3801,14 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     const int lane_id = threadIdx.x & 63, lane_of_column = lane_id & (LANES - 1);
     const int x = strip_x + part * part_cols + lane_id / LANES;
     ColumnCtx cc;
-    cc.tb = nullptr; cc.m = m; cc.mv.m = m; cc.c = &lane_ctx;
+    cc.tb = nullptr; cc.m = m; cc.mv.m = m; cc.mv.walls = dm.wall_links; cc.mv.vertex_links = dm.vertex_links; cc.c = &lane_ctx;
     cc.recs = sc.rec; cc.spans = sc.span;
     cc.rec_base = (unsigned)local * (unsigned)m->wall_count;
     cc.frags = sc.frag_rec + (size_t)local * m->split_count * m->fragment_slots;
     cc.set_list(sc, local, x);
     cc.x = x;
     ray_direction(lane_ctx, x, &cc.rx, &cc.ry);
+    cc.first = cc.eval(0);
     bool boundary_has_po = false;   // does some entry's span begin at this column
     ListShare<LANES> list;
     if constexpr (SHARED) {
@@ -3791,7 +3822,7 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     st.ceiling_clip = 0.0f; st.floor_clip = (float)VH;
     st.masked_ceiling_clip = 0.0f; st.masked_floor_clip = (float)VH; st.masked_distance = GD_INF; st.masked_wall = -1;
     st.previous_distance = 0.0f;
-    st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_eb_index = 0;
+    st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_ep_sectors = 0; st.pend_ep_vertices = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
     if constexpr (!SHARED) list.start(cc, &order_lds[0][lane_id], boundary_has_po);
     PassRec *records = sc.pass_rec + sc.pass_at(0, local, x);
@@ -3933,7 +3964,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     bool window_dirty = false;
     GapRange gaps; gaps.reset();
     ColumnCtx cc;
-    cc.tb = &tb; cc.m = m; cc.mv.m = m; cc.c = &lane_ctx;
+    cc.tb = &tb; cc.m = m; cc.c = &lane_ctx;
     cc.recs = sc.rec; cc.spans = sc.span;
     cc.rec_base = (unsigned)local * (unsigned)m->wall_count;
     cc.frags = sc.frag_rec + (size_t)local * m->split_count * m->fragment_slots;
@@ -3955,7 +3986,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     st.ceiling_clip = 0.0f; st.floor_clip = (float)VH;
     st.masked_ceiling_clip = 0.0f; st.masked_floor_clip = (float)VH; st.masked_distance = GD_INF; st.masked_wall = -1;
     st.previous_distance = 0.0f;
-    st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_eb_index = 0;
+    st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_ep_sectors = 0; st.pend_ep_vertices = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
     SilhouetteBounds sb; sb.bot_row = VH; sb.top_row = 0; sb.bot_depth = -GD_INF; sb.top_depth = -GD_INF;
     const int passes = sc.pass_count[(size_t)local * SW + x];
@@ -6465,6 +6496,20 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
             if ((facts[w] >> WALL_BLOCKING_SHIFT) == 0) facts[w] |= (b + 1) << WALL_BLOCKING_SHIFT;   // the first slot wins ties, like the scan it replaces
         }
         if (rc == GD_OK) rc = upload(r, facts.data(), facts.size(), &r->dm.wall_facts);
+        std::vector<WallLinks> links(W);
+        for (size_t w = 0; w < W; ++w) {
+            WallLinks &link = links[w];
+            link.sectors = ((unsigned)h->wall_sectors[2 * w] & 0xFFFFu) | (unsigned)h->wall_sectors[2 * w + 1] << 16;
+            link.vertices = ((unsigned)h->wall_vertex[2 * w] & 0xFFFFu) | (unsigned)h->wall_vertex[2 * w + 1] << 16;
+            for (int k = 0; k < 2; ++k) link.neighbour[k] = h->direct_neighbor_table[4 * w + k];
+            link.slots = (unsigned)h->direct_neighbor_table[4 * w + 2];
+            link.solid[0] = h->solid_bridge_start_ofs[w]; link.solid[1] = h->solid_bridge_end_ofs[w];
+            link.solid_counts = (unsigned)(h->solid_bridge_start_ofs[w + 1] - link.solid[0]) | (unsigned)(h->solid_bridge_end_ofs[w + 1] - link.solid[1]) << 16;
+        }
+        if (rc == GD_OK) rc = upload(r, links.data(), links.size(), &r->dm.wall_links);
+        std::vector<VertexLink> vertex_links(h->vertex_wall_ofs[V]);
+        for (size_t k = 0; k < vertex_links.size(); ++k) vertex_links[k] = {h->vertex_wall_idx[k], links[h->vertex_wall_idx[k]].sectors};
+        if (rc == GD_OK) rc = upload(r, vertex_links.data(), vertex_links.size(), &r->dm.vertex_links);
         std::vector<WallSide> sides(W * 2);
         std::vector<int> masked_slot(W, -1);
         r->dm.masked_count = 0;
