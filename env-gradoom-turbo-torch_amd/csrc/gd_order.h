@@ -4,39 +4,56 @@
 #define GD_ORDER_H
 
 #ifdef __HIPCC__
-#define GD_ORDER_FN __host__ __device__ __attribute__((always_inline)) inline
+#define GD_ORDER_FN __device__ __attribute__((always_inline)) inline
 #else
 #define GD_ORDER_FN inline
 #endif
 
-// LOW .. LOW + SPAN (a power of two) of the first COUNT of `v`, STEP apart.  What lies beyond COUNT counts as larger than anything, so that no exchange
-// with it is ever made.
-template <int COUNT, int LOW, int SPAN, int STEP> GD_ORDER_FN void order_merge(unsigned (&v)[COUNT]) {
-    auto exchange = [&](int a, int b) {
-        const unsigned low = v[a] < v[b] ? v[a] : v[b], high = v[a] < v[b] ? v[b] : v[a];
-        v[a] = low; v[b] = high;
-    };
+// two numbers in order
+GD_ORDER_FN void order_two(double &low, double &high) {
+    const double a = low, b = high;
+#ifdef __HIPCC__
+    asm("v_min_f64 %0, %1, %2" : "=v"(low) : "v"(a), "v"(b));      // plain minima of numbers that are none of them NaN: fmin() would ask first
+    asm("v_max_f64 %0, %1, %2" : "=v"(high) : "v"(a), "v"(b));
+#else
+    low = a < b ? a : b; high = a < b ? b : a;
+#endif
+}
+// LOW .. LOW + SPAN (a power of two) of `v`, STEP apart
+template <int LOW, int SPAN, int STEP, int COUNT> GD_ORDER_FN void order_merge(double (&v)[COUNT]) {
     if constexpr (2 * STEP < SPAN) {
-        order_merge<COUNT, LOW, SPAN, 2 * STEP>(v);
-        order_merge<COUNT, LOW + STEP, SPAN, 2 * STEP>(v);
+        order_merge<LOW, SPAN, 2 * STEP>(v);
+        order_merge<LOW + STEP, SPAN, 2 * STEP>(v);
 #pragma unroll
-        for (int at = LOW + STEP; at + STEP < LOW + SPAN; at += 2 * STEP)
-            if (at + STEP < COUNT) exchange(at, at + STEP);
-    } else if constexpr (LOW + STEP < COUNT) {
-        exchange(LOW, LOW + STEP);
+        for (int at = LOW + STEP; at + STEP < LOW + SPAN; at += 2 * STEP) order_two(v[at], v[at + STEP]);
+    } else {
+        order_two(v[LOW], v[LOW + STEP]);
     }
 }
-template <int COUNT, int LOW, int SPAN> GD_ORDER_FN void order_part(unsigned (&v)[COUNT]) {
-    if constexpr (SPAN > 1 && LOW + 1 < COUNT) {
-        order_part<COUNT, LOW, SPAN / 2>(v);
-        order_part<COUNT, LOW + SPAN / 2, SPAN / 2>(v);
-        order_merge<COUNT, LOW, SPAN, 1>(v);
+template <int LOW, int SPAN, int COUNT> GD_ORDER_FN void order_part(double (&v)[COUNT]) {
+    if constexpr (SPAN > 1) {
+        order_part<LOW, SPAN / 2>(v);
+        order_part<LOW + SPAN / 2, SPAN / 2>(v);
+        order_merge<LOW, SPAN, 1>(v);
     }
 }
-// Up to 64 numbers, the smallest first.
-template <int COUNT> GD_ORDER_FN void order_up(unsigned (&v)[COUNT]) {
-    static_assert(COUNT <= 64, "order_up: a network for up to 64");
-    order_part<COUNT, 0, COUNT <= 32 ? 32 : 64>(v);
+// Numbers, a power of two of them, the smallest first.
+template <int COUNT> GD_ORDER_FN void order_up(double (&v)[COUNT]) {
+    static_assert((COUNT & (COUNT - 1)) == 0, "order_up: a power of two");
+    order_part<0, COUNT>(v);
+}
+// The smallest of two ordered runs, as many as each holds, in order, in `v`: the pairs from opposite ends hold them and rise, then fall.
+template <int COUNT> GD_ORDER_FN void order_merge_lowest(double (&v)[COUNT], const double (&other)[COUNT]) {
+#pragma unroll
+    for (int k = 0; k < COUNT; ++k) {
+        double most = other[COUNT - 1 - k];
+        order_two(v[k], most);
+    }
+#pragma unroll
+    for (int step = COUNT / 2; step > 0; step /= 2)
+#pragma unroll
+        for (int k = 0; k < COUNT; ++k)
+            if (!(k & step)) order_two(v[k], v[k + step]);
 }
 
 #endif

@@ -94,6 +94,7 @@ static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and it
 #define CF_NARROW 64    // its clipped span is at most two columns wide
 #define CF_SHORT 128    // at most 32 map units long
 #define CF_SUBPIXEL 256 // two-sided, and its clipped span at most one column wide
+#define CF_ONE_SIDED 512
 
 // wall record flags
 #define WF_HC 1        // owns at least one column after every span test
@@ -104,7 +105,8 @@ static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and it
 #define WF_NARROW CF_NARROW
 #define WF_SHORT CF_SHORT
 #define WF_SUBPIXEL CF_SUBPIXEL // two-sided and at most one column wide (engine.py:11589-11591)
-#define WF_SHOWN (WF_FF | WF_NARROW | WF_SHORT | WF_SUBPIXEL)
+#define WF_ONE_SIDED CF_ONE_SIDED
+#define WF_SHOWN (WF_FF | WF_NARROW | WF_SHORT | WF_SUBPIXEL | WF_ONE_SIDED)
 #define WF_END_SHIFT 16   // bits 16 and up: the column at which the clipped span ends, WF_END_NONE if that is not a column
 #define WF_END_NONE 1023
 
@@ -200,11 +202,8 @@ struct RecSpan {   // what a ray test of one linedef needs (eval_segment), kept 
     int flags;
 };
 
-struct __align__(16) Cand {      // one linedef with a finite ray distance at one column, with the static
-                   // linedef facts every scan needs packed in so that scans do no gathers
-    unsigned short flags, wall;   // in this order: the entry's first word under its last is the key below
-    short s0, s1;            // front / back sector (-1 = none)
-    unsigned short v0, v1;   // vertex ids of start / end
+struct __align__(8) Cand {      // one linedef with a finite ray distance at one column
+    unsigned short flags, wall;   // in this order: the entry's bits are the key below
     float dist;
 };
 // (distance, linedef, flags) of a candidate as one unsigned number.  Listed distances are positive, so their bit patterns
@@ -212,6 +211,7 @@ struct __align__(16) Cand {      // one linedef with a finite ray distance at on
 // traversal breaks them (no column lists a linedef twice).  CAND_KEY_NONE, greater than any entry's, stands for "none".
 #define CAND_KEY_NONE 0x7F800000FFFFFFFFULL
 __device__ __forceinline__ u64 cand_key(const Cand &q) { return ((u64)__float_as_uint(q.dist) << 32) | ((u64)q.wall << 16) | (u64)q.flags; }
+__device__ __forceinline__ Cand key_cand(u64 key) { Cand q; q.flags = (unsigned short)key; q.wall = (unsigned short)(key >> 16); q.dist = __uint_as_float((unsigned)(key >> 32)); return q; }
 __device__ __forceinline__ float cand_key_distance(u64 key) { return __uint_as_float((unsigned)(key >> 32)); }
 __device__ __forceinline__ int cand_key_wall(u64 key) { return key == CAND_KEY_NONE ? 0x7fffffff : (int)((unsigned)key >> 16); }
 __device__ __forceinline__ int cand_key_flags(u64 key) { return key == CAND_KEY_NONE ? 0 : (int)((unsigned)key & 0xFFFFu); }
@@ -279,7 +279,7 @@ struct Scratch {    // per-chunk working memory, sized at create
     WallRec *frag_rec;     // [L,split_count,fragment_slots] FWallCoords of the BSP fragments of split linedefs
     float *scene_depth;    // [L,208,320] depth of the wall tier or masked texture a pixel shows (engine.py:11553, 12700, 13740),
                            // kept only for frames that draw wall decals, else null; scene_depth_at() has the others
-    Cand *cand;            // [L,CAND_MAX,320], then the spill pool [spill_slots / 320, SPILL_DEPTH, 320]
+    Cand *cand;            // [L,CAND_MAX,320], eight bytes an entry (with sectors and vertices in it, sixteen, wall_setup_kernel took 455 us for 395), then the spill pool [spill_slots / 320, SPILL_DEPTH, 320]
     int *cand_count;       // [L,320] entries listed (beyond CAND_MAX: the column wanted more than its own slots hold), or for
                            // a column with a pool slot: entries in the pool | (slot + 1) << SPILL_SHIFT
     int *spill_columns;    // [spill_slots] the columns (lane * 320 + column) that were given pool slots, in slot order
@@ -718,7 +718,7 @@ __device__ __forceinline__ void ray_direction(const LaneCtx &c, int x, float *rx
 
 // distances / along / geometric / projected / left-edge of one linedef at one column
 // (engine.py:11317-11331, 11440-11460)
-__device__ __forceinline__ Eval eval_segment(const float4 wl, int rec_flags, int rec_pl, int rec_pr, bool os, const LaneCtx &c, int x, float rx, float ry) {
+__device__ __forceinline__ Eval eval_segment(const float4 wl, int rec_flags, int rec_pl, int rec_pr, const LaneCtx &c, int x, float rx, float ry) {
     float segx = wl.z - wl.x, segy = wl.w - wl.y;
     float offx = wl.x - c.x, offy = wl.y - c.y;
     float den = rx * segy - ry * segx;
@@ -729,7 +729,7 @@ __device__ __forceinline__ Eval eval_segment(const float4 wl, int rec_flags, int
     bool g = ok && (d > 0) && (a >= 0) && (a <= 1);
     bool screen_valid = (rec_flags & WF_HC) && (x >= rec_pl) && (x < rec_pr);
     bool p = ok && (d > 0) && screen_valid;
-    bool valid = os ? (p && (rec_flags & WF_FF)) : (g || p);
+    bool valid = (rec_flags & WF_ONE_SIDED) ? (p && (rec_flags & WF_FF)) : (g || p);
     Eval out;
     out.dist = valid ? d : GD_INF;
     out.flags = (g ? CF_GEO : 0) | (p ? CF_PROJ : 0) | ((x == rec_pl) ? CF_LEDGE : 0) | ((a > 0.5f) ? CF_ALONG_HI : 0) |
@@ -740,7 +740,7 @@ __device__ __forceinline__ Eval eval_segment(const float4 wl, int rec_flags, int
 __device__ __forceinline__ Eval eval_wall(const gd_map_desc *m, const LaneCtx &c, const RecSpan *spans, int x, int w, float rx, float ry) {
     const float4 wl = *reinterpret_cast<const float4 *>(m->walls + 4 * w);
     const RecSpan r = spans[w];
-    return eval_segment(wl, r.flags, r.pl, r.pr, m->wall_sectors[2 * w + 1] < 0, c, x, rx, ry);
+    return eval_segment(wl, r.flags, r.pl, r.pr, c, x, rx, ry);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -833,11 +833,10 @@ struct SetupWall {                // a linedef as the columns' look at it asks f
     int window;                   // first column | one past the last << 16
     int facts;                    // WF_* but for WF_HC and WF_ANYGEO, and SETUP_*
     int ends;                     // screen column of the left endpoint | of the right one << 9 | their visibility << 18, 19
-    int sectors, vertices, wall;
+    int wall;
     int blocking;                 // its position in blocking_walls, -1
 };
-#define SETUP_ONE_SIDED 0x200     // free bits of the WF_* word
-#define SETUP_MASKED 0x400        // a mid-texture on the side facing the camera
+#define SETUP_MASKED 0x400        // free bits of the WF_* word: a mid-texture on the side facing the camera
 #define SETUP_SPANS 0x800         // FWallCoords' span is not empty
 // The span a linedef owns (engine.py:11347-11427), within [0, 320]: first column | one past the last << 16, bit 31 when it owns any.
 __device__ __forceinline__ int setup_owned(int facts, int ends, bool any, int first, int last) {
@@ -896,7 +895,7 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
                 span.pl = 0; span.pr = 0;
                 // an unseen linedef has an empty span (sr == sl), so a two-sided one counts as at most one column wide
                 const int facts = dm.wall_facts[w];
-                span.flags = (ff ? WF_FF : 0) | ((facts & WALL_ONE_SIDED) ? 0 : WF_SUBPIXEL) | ((facts & WALL_SPLIT) ? WF_SPLIT : 0) |
+                span.flags = (ff ? WF_FF : 0) | ((facts & WALL_ONE_SIDED) ? WF_ONE_SIDED : WF_SUBPIXEL) | ((facts & WALL_SPLIT) ? WF_SPLIT : 0) |
                              WF_NARROW | ((facts & WALL_SHORT) ? WF_SHORT : 0) | (WF_END_NONE << WF_END_SHIFT);
                 sc.span[(size_t)local * m->wall_count + w] = span;
             }
@@ -963,21 +962,18 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
         int window0 = scans ? lo : SW, window1 = scans ? hi : 0;
         if (ends & (1 << 18)) window0 = min(window0, ends & 511);
         if (ends & (1 << 19)) window1 = max(window1, (ends >> 9) & 511);
-        const int s0 = m->wall_sectors[2 * w], s1 = m->wall_sectors[2 * w + 1];
-        const bool os = s1 < 0;
         const int known = dm.wall_facts[w];
+        const bool os = known & WALL_ONE_SIDED;
         const i64 span = r.sr - r.sl;
         const int facts = (ff ? WF_FF : 0) | ((span <= 1 && !os) ? WF_SUBPIXEL : 0) | ((known & WALL_SPLIT) ? WF_SPLIT : 0) | (span <= 2 ? WF_NARROW : 0) |
                           ((known & WALL_SHORT) ? WF_SHORT : 0) | ((r.sr >= 0 && r.sr < SW ? (int)r.sr : WF_END_NONE) << WF_END_SHIFT) |
-                          (os ? SETUP_ONE_SIDED : 0) | (!os && m->side_tex[(w * 2 + (ff ? 0 : 1)) * 3] >= 0 ? SETUP_MASKED : 0) | (span > 0 ? SETUP_SPANS : 0);
+                          (os ? WF_ONE_SIDED : 0) | (!os && m->side_tex[(w * 2 + (ff ? 0 : 1)) * 3] >= 0 ? SETUP_MASKED : 0) | (span > 0 ? SETUP_SPANS : 0);
         {
             SetupWall mine;
             mine.segx = segx; mine.segy = segy; mine.offx = offx; mine.offy = offy;
             mine.numer = offx * segy - offy * segx;
             mine.window = window0 | (window1 << 16);
             mine.facts = facts; mine.ends = ends;
-            mine.sectors = (s0 & 0xFFFF) | (s1 << 16);
-            mine.vertices = (int)(((unsigned)m->wall_vertex[2 * w] & 0xFFFFu) | ((unsigned)m->wall_vertex[2 * w + 1] << 16));
             mine.wall = w; mine.blocking = (known >> WALL_BLOCKING_SHIFT) - 1;
             walls_lds[wave][slot] = mine;
             hits_lds[wave][slot] = SW;                    // none: first 320, one past the last 0
@@ -997,14 +993,12 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
         auto enter = [&](const SetupWall &q, int x, bool ok, bool g, bool along_high, float d, int owned) {
             const int from = owned & 0xFFFF, to = (owned >> 16) & 0x7FFF;
             const bool p = ok && d > 0 && owned < 0 && x >= from && x < to;
-            const bool valid = (q.facts & SETUP_ONE_SIDED) ? p && (q.facts & WF_FF) : (g || p);
+            const bool valid = (q.facts & WF_ONE_SIDED) ? p && (q.facts & WF_FF) : (g || p);
             if (!valid || !finitef(d)) return;
             const int flags = (g ? CF_GEO : 0) | (p ? CF_PROJ : 0) | ((x == from) ? CF_LEDGE : 0) | (along_high ? CF_ALONG_HI : 0) |
                               (((q.facts >> WF_END_SHIFT) == x) ? CF_ENDS_HERE : 0) | (q.facts & WF_SHOWN);
             Cand entry;
             entry.flags = (unsigned short)flags; entry.wall = (unsigned short)q.wall;
-            entry.s0 = (short)(q.sectors & 0xFFFF); entry.s1 = (short)(q.sectors >> 16);
-            entry.v0 = (unsigned short)(q.vertices & 0xFFFF); entry.v1 = (unsigned short)((unsigned)q.vertices >> 16);
             entry.dist = d;
             if ((q.facts & SETUP_MASKED) && p) atomicMin(&masked_hits[x], cand_key(entry));
             const int at = atomicAdd(&counts[x], 1);
@@ -1076,7 +1070,7 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
             const int owned = setup_owned(facts, ends, any, any ? hits & 0xFFFF : 0, any ? (hits >> 16) - 1 : SW - 1);
             RecSpan shown;
             shown.pl = (short)(owned & 0xFFFF); shown.pr = (short)((owned >> 16) & 0x7FFF);
-            shown.flags = (facts & ~(SETUP_ONE_SIDED | SETUP_MASKED | SETUP_SPANS)) | (owned < 0 ? WF_HC : 0) | (any ? WF_ANYGEO : 0);
+            shown.flags = (facts & ~(SETUP_MASKED | SETUP_SPANS)) | (owned < 0 ? WF_HC : 0) | (any ? WF_ANYGEO : 0);
             r.pl = shown.pl; r.pr = shown.pr; r.flags = shown.flags;
             sc.rec[(size_t)local * m->wall_count + w] = r;
             sc.span[(size_t)local * m->wall_count + w] = shown;
@@ -1119,10 +1113,7 @@ __device__ __forceinline__ void list_spilled_columns(const DeviceMap &dm, const 
             if (w < walls) {
                 const Eval e = eval_wall(m, c, spans, x, w, rx, ry);
                 keep = finitef(e.dist);
-                const int s1 = m->wall_sectors[2 * w + 1];
                 entry.wall = (unsigned short)w;
-                entry.s0 = (short)m->wall_sectors[2 * w]; entry.s1 = (short)s1;
-                entry.v0 = (unsigned short)m->wall_vertex[2 * w]; entry.v1 = (unsigned short)m->wall_vertex[2 * w + 1];
                 entry.flags = (unsigned short)e.flags;
                 entry.dist = e.dist;
             }
@@ -2060,7 +2051,7 @@ struct ColumnCtx {
     const WallRec *recs;  // the chunk's [L,W] records, with rec_base = lane * W
     const RecSpan *spans; // the chunk's [L,W] ray-test facts of every linedef
     const WallRec *frags; // this lane's [split_count, fragment_slots] fragment records
-    const Cand *list;     // the chunk's candidate blocks; entry k of this column sits list_column + k * 320 * 16 bytes in
+    const Cand *list;     // the chunk's candidate blocks; entry k of this column sits list_column + k * 320 * 8 bytes in
     unsigned rec_base, list_column;
     int count;
     int x;
@@ -2075,33 +2066,44 @@ struct ColumnCtx {
         const unsigned spill = (unsigned)listed >> SPILL_SHIFT;
         if (spill) {
             const unsigned slot = spill - 1;
-            list_column = (sc.spill_base + (slot / SW) * (unsigned)(SPILL_DEPTH * SW) + slot % SW) * 16u;
+            list_column = (sc.spill_base + (slot / SW) * (unsigned)(SPILL_DEPTH * SW) + slot % SW) * 8u;
             count = listed & ((1 << SPILL_SHIFT) - 1);
         } else {
-            list_column = ((unsigned)local * (CAND_MAX * SW) + (unsigned)column) * 16u;
+            list_column = ((unsigned)local * (CAND_MAX * SW) + (unsigned)column) * 8u;
             count = listed < CAND_MAX ? listed : CAND_MAX;
         }
     }
-    __device__ __forceinline__ Cand cand(int k) const {
-        union { uint4 raw; Cand c; } u;
-        u.raw = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(list) + (list_column + (unsigned)k * (SW * 16u)));   // one 16-byte load
-        return u.c;
+    __device__ __forceinline__ u64 cand(int k) const {      // as its key
+        return *reinterpret_cast<const u64 *>(reinterpret_cast<const char *>(list) + (list_column + (unsigned)k * (SW * 8u)));
     }
     __device__ Eval eval(int w) const { return eval_wall(m, *c, spans + rec_base, x, w, rx, ry); }
 };
 
+// A candidate as a scan looks at it.
+struct ListEntry {
+    unsigned short flags, wall;
+    float dist;
+    unsigned sectors, vertices;    // as in WallLinks
+    __device__ __forceinline__ u64 key() const { return ((u64)__float_as_uint(dist) << 32) | ((u64)wall << 16) | (u64)flags; }
+};
 // A column's list as wall_select_kernel's LANES lanes of the column hold it between them: entry k in registers of lane k % LANES.  Each
-// looks at its own in a scan, and what the scan is after, the smallest of some keys, is exchanged.  One lane alone reads the list where it is.
+// looks at its own in a scan, and what the scan is after, the smallest of some keys, is exchanged.  One lane alone keeps what is near of it.
 template <int LANES> struct ListShare {
     static constexpr int ENTRIES = CAND_MAX / LANES;
-    Cand own[ENTRIES];
+    ListEntry own[ENTRIES];
     // an entry that is not there lies nearer than any distance a scan asks for: none takes it
     __device__ __forceinline__ void load(const ColumnCtx &cc, int lane) {
+        u64 keys[ENTRIES];
 #pragma unroll
-        for (int j = 0; j < ENTRIES; ++j) own[j] = cc.cand(max(min(j * LANES + lane, cc.count - 1), 0));
+        for (int j = 0; j < ENTRIES; ++j) keys[j] = cc.cand(max(min(j * LANES + lane, cc.count - 1), 0));
 #pragma unroll
-        for (int j = 0; j < ENTRIES; ++j)
-            if (j * LANES + lane >= cc.count) { own[j].dist = -GD_INF; own[j].flags = 0; }
+        for (int j = 0; j < ENTRIES; ++j) {
+            const bool there = j * LANES + lane < cc.count;
+            const Cand q = key_cand(keys[j]);
+            const WallLinks &links = cc.mv.walls[there ? q.wall : 0];
+            own[j].wall = q.wall; own[j].sectors = links.sectors; own[j].vertices = links.vertices;
+            own[j].dist = there ? q.dist : -GD_INF; own[j].flags = there ? q.flags : 0;
+        }
     }
     // the smallest of the column's lanes; all of them are executing
     template <int CONTROL> static __device__ __forceinline__ u64 moved(u64 v) {
@@ -2133,7 +2135,7 @@ template <int LANES> struct ListShare {
 // The nearest of the candidates a scan takes, the lowest linedef on ties, and its flags.
 template <int LANES> struct NearestOf {
     u64 key = CAND_KEY_NONE;
-    __device__ __forceinline__ void take(const Cand &q) { const u64 k = cand_key(q); key = k < key ? k : key; }
+    __device__ __forceinline__ void take(const ListEntry &q) { const u64 k = q.key(); key = k < key ? k : key; }
     __device__ __forceinline__ void share() { key = ListShare<LANES>::smallest(key); }     // what the column's lanes took
     __device__ __forceinline__ float distance() const { return cand_key_distance(key); }
     __device__ __forceinline__ int wall() const { return cand_key_wall(key); }
@@ -2141,101 +2143,136 @@ template <int LANES> struct NearestOf {
 };
 template <> struct NearestOf<1> {
     float d = GD_INF; int w = 0x7fffffff, f = 0;
-    __device__ __forceinline__ void take(const Cand &q) { if (q.dist < d || (q.dist == d && (int)q.wall < w)) { d = q.dist; w = q.wall; f = q.flags; } }
+    __device__ __forceinline__ void take(const ListEntry &q) { if (q.dist < d || (q.dist == d && (int)q.wall < w)) { d = q.dist; w = q.wall; f = q.flags; } }
     __device__ __forceinline__ void share() {}
     __device__ __forceinline__ float distance() const { return d; }
     __device__ __forceinline__ int wall() const { return w; }
     __device__ __forceinline__ int flags() const { return f; }
 };
-// One lane alone reads the list where it is, nearest entries first: their places, sorted by distance when the column begins, lie in LDS.  The order is
-// that of the distances' bits but the lowest six, which hold the place, so that entries a few units in the last place apart may come in either order: a
-// scan takes the smallest of what it looks at, and looks on until what is left is farther than the answer by more than that.  A list in the spill pool is
-// looked at from end to end.  A pass looks at some eight entries so, of the thirty that a column of the 4000-linedef map lists: for 4096 lanes the launch
-// for the strips that are not among the longest issues 9,900 vector instructions and 370 loads a wavefront, 14,500 and 690 when every scan
-// went over the whole list, and takes 0.80 ms instead of 0.895 (0.20 for 0.23 at 1024 lanes of the 2000-linedef map): what is left waits for loads that
-// depend on one another.  The network for 64 needs more registers than there are (some forty words go to memory once a column), those for 32 and 48 do not.
-#define ORDER_ROWS (CAND_MAX / 4 + 1)      // words of four places, and one that is read and never asked about
+// One lane alone keeps the nearest entries beyond the column's distance in LDS, in order, with their sectors: the window.  A scan goes through it until what is
+// left is too far to matter, and through the whole list in memory if the window ends before that.  When one of the wavefront's columns has passed
+// WINDOW_REFILL entries by, all of them fill theirs again: columns that did so one by one would have the wavefront fill in nearly every pass.
+// The launch for all but the longest strips waits for memory more than for anything else (60 % of its wavefronts' time), and the list is what it waited for: 30 KB a
+// wavefront at 16 bytes an entry, four times what L2 holds of it.  Read whole by every scan it takes 0.895 ms for 4096 lanes on the 4000-linedef map; only the
+// entries' order in LDS, nearest first, 0.79, with as many wavefronts a SIMD as one likes; this way 0.64 (11 million lines missed in L2, 15, 6).  1024 lanes on the
+// 2000-linedef map 231, 191, 156 us.  Filled again after 3 / 4 / 5 / 6 / 8 / 10 entries 645 / 646 / 642 / 710 / 730 / 770 us.  Twelve entries are what sixteen
+// wavefronts' LDS holds; with sixteen, and eight wavefronts, 1.0 ms.
+#define WINDOW 12
+#define WINDOW_REFILL 5
+#define WINDOW_BATCH 16        // entries ordered at a time
+#define WINDOW_PAD 3           // rows read with the last ones and not looked at
 template <> struct ListShare<1> {
-    const unsigned *places;     // this lane's word of [ORDER_ROWS][64]
-    u64 ledges;                 // bit k: the entries k, k + 64, ... hold one whose projected span begins at this column (CF_PROJ and CF_LEDGE)
-    int from;                   // the entries before this one, in order, are no farther than `passed`
-    float passed;
-    bool sorted;
+    static constexpr int WORDS = (WINDOW * 3 + WINDOW_PAD) * 64;
+    u64 *keys;                  // this lane's word of [WINDOW][64]
+    unsigned *sectors;          // the same of theirs, behind the keys
+    u64 solid_ledges, ledges;   // bit k: the entries k, k + 64, ... hold one whose projected span begins at this column (CF_PROJ and CF_LEDGE), one-sided, two-sided
+    int from, held;             // the window's entries before `from` are no farther than `passed`; it holds `held`
+    float passed, floor;        // floor: `passed` when it was filled
+    bool complete;              // nothing of the list lies beyond the window
     static __device__ __forceinline__ u64 smallest(u64 v) { return v; }
     static __device__ __forceinline__ unsigned smallest(unsigned v) { return v; }
 
-    // A look at the whole list: ledges, whether some entry's span begins at this column, and the order.  COUNT: at least as many as any of the
-    // wavefront's sorted lists holds.
-    template <int COUNT> __device__ __forceinline__ void load(const ColumnCtx &cc, unsigned *words, bool &any_ledge) {
-        constexpr int BATCH = COUNT > 48 ? 4 : 8;       // as many loads at a time as there are registers for
-        unsigned keys[COUNT], own[2] = {0u, 0u}, flagged = 0u;
+    __device__ __forceinline__ void start(const ColumnCtx &cc, unsigned *words, int lane_id, bool &any_ledge) {
+        keys = reinterpret_cast<u64 *>(words) + lane_id; sectors = words + WINDOW * 2 * 64 + lane_id;
+        solid_ledges = 0; ledges = 0; from = 0; held = 0; passed = 0.0f; floor = GD_INF; complete = false;
+        unsigned flagged = 0;
+        for (int k0 = 0; k0 < cc.count; k0 += 8) {
+            unsigned flags[8], solid = 0, portal = 0;
 #pragma unroll
-        for (int k0 = 0; k0 < COUNT; k0 += BATCH) {
-            Cand batch[BATCH];
+            for (int j = 0; j < 8; ++j) flags[j] = (unsigned)cc.cand(k0 + j);     // what lies behind the list's end is memory of the column's all the same
 #pragma unroll
-            for (int j = 0; j < BATCH; ++j) batch[j] = cc.cand(max(min(k0 + j, cc.count - 1), 0));
-#pragma unroll
-            for (int j = 0; j < BATCH; ++j) {
-                const int k = k0 + j;
-                const bool there = k < cc.count;
-                const unsigned flags = there ? batch[j].flags : 0u;
-                flagged |= flags;
-                own[k / 32] |= (flags & (CF_LEDGE | CF_PROJ)) == (CF_LEDGE | CF_PROJ) ? 1u << (k & 31) : 0u;
-                keys[k] = there ? (__float_as_uint(batch[j].dist) & ~63u) | (unsigned)k : ~0u;
+            for (int j = 0; j < 8; ++j) {
+                const unsigned f = k0 + j < cc.count ? flags[j] : 0u;
+                flagged |= f;
+                const bool ledge = (f & (CF_LEDGE | CF_PROJ)) == (CF_LEDGE | CF_PROJ);
+                solid |= ledge && (f & CF_ONE_SIDED) ? 1u << j : 0u;
+                portal |= ledge && !(f & CF_ONE_SIDED) ? 1u << j : 0u;
             }
-#pragma unroll
-            for (int j = 0; j < BATCH; ++j) asm volatile("" : "+v"(keys[k0 + j]) : : "memory");
+            solid_ledges |= (u64)solid << (k0 & 63);
+            ledges |= (u64)portal << (k0 & 63);
         }
         any_ledge = flagged & CF_LEDGE;
-        ledges = own[0] | (u64)own[1] << 32;
-        order_up(keys);
-#pragma unroll
-        for (int k = 0; k < COUNT; k += 4) {
-            const unsigned low = __builtin_amdgcn_perm(keys[k + 1], keys[k], 0x0C0C0400u), high = __builtin_amdgcn_perm(keys[k + 3], keys[k + 2], 0x04000C0Cu);
-            words[(k / 4) * 64] = (low | high) & 0x3F3F3F3Fu;
-        }
     }
-    __device__ __forceinline__ void start(const ColumnCtx &cc, unsigned *words, bool &any_ledge) {
-        places = words; ledges = 0; from = 0; passed = -1.0f;
-        sorted = cc.count <= CAND_MAX;
-        any_ledge = false;
-        const int most = wave_max(min(cc.count, CAND_MAX));
-        if (most <= 32) load<32>(cc, words, any_ledge);
-        else if (most <= 48) load<48>(cc, words, any_ledge);
-        else load<64>(cc, words, any_ledge);
-        for (int k = CAND_MAX; k < cc.count; ++k) {
-            const Cand q = cc.cand(k);
-            any_ledge |= (q.flags & CF_LEDGE) != 0;
-            ledges |= (q.flags & CF_LEDGE) && (q.flags & CF_PROJ) ? 1ULL << (k & 63) : 0ULL;
+    // The window: the nearest entries beyond `passed`.  Keys are positive float64 numbers (a float32's exponent of all ones is not one of float64's), whose
+    // order is theirs: an exchange is a minimum and a maximum.
+    __device__ __forceinline__ void fill(const ColumnCtx &cc) {
+        double best[WINDOW_BATCH];
+        const double none = __longlong_as_double((long long)CAND_KEY_NONE);
+        int beyond = 0;
+#pragma unroll
+        for (int j = 0; j < WINDOW_BATCH; ++j) best[j] = none;
+        for (int k0 = 0; k0 < cc.count; k0 += WINDOW_BATCH) {
+            u64 raw[WINDOW_BATCH];
+            double next[WINDOW_BATCH];
+#pragma unroll
+            for (int j = 0; j < WINDOW_BATCH; ++j) raw[j] = cc.cand(k0 + j);
+#pragma unroll
+            for (int j = 0; j < WINDOW_BATCH; ++j) {
+                const bool wanted = k0 + j < cc.count && cand_key_distance(raw[j]) > passed;
+                beyond += wanted ? 1 : 0;
+                next[j] = wanted ? __longlong_as_double((long long)raw[j]) : none;
+            }
+            order_up(next);
+            if (k0 == 0) {
+#pragma unroll
+                for (int j = 0; j < WINDOW_BATCH; ++j) best[j] = next[j];
+            } else {
+                order_merge_lowest(best, next);
+            }
         }
+        held = min(beyond, WINDOW); complete = beyond <= WINDOW;
+        from = 0; floor = passed;
+        unsigned pairs[WINDOW];
+#pragma unroll
+        for (int j = 0; j < WINDOW; ++j) {
+            const u64 key = (u64)__double_as_longlong(best[j]);
+            pairs[j] = cc.mv.walls[key == CAND_KEY_NONE ? 0 : (unsigned)key >> 16].sectors;
+            keys[j * 64] = key;
+        }
+#pragma unroll
+        for (int j = 0; j < WINDOW; ++j) sectors[j * 64] = pairs[j];
     }
     // A pass of the column begins: its scans ask for entries beyond `distance`.
-    __device__ __forceinline__ void begin(float distance) {
-        if (distance < passed) from = 0;
+    __device__ __forceinline__ void begin(const ColumnCtx &cc, float distance) {
         passed = distance;
+        if (__ballot(distance < floor || (from >= WINDOW_REFILL && !complete)) != 0 && !(complete && distance >= floor)) fill(cc);
     }
-    // The entries beyond `passed` (and some that are not), nearest first, until those left are farther than enough().
+    // The entries beyond `passed` (and some that are not, and some twice), nearest first as far as the window goes, until those left are
+    // farther than enough().
     template <bool ADVANCE, typename Look, typename Enough> __device__ __forceinline__ void walk(const ColumnCtx &cc, Look look, Enough enough) {
-        bool leading = sorted;
-        for (int k = from; k < cc.count;) {
-            const unsigned *row = places + (min(k, CAND_MAX - 1) >> 2) * 64;
-            const unsigned next = __builtin_amdgcn_alignbyte(row[64], row[0], (unsigned)k);
-            Cand batch[4];
+        bool leading = true, more = true;
+        for (int k = from; k < held && more;) {
+            u64 key[4]; unsigned pair[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) batch[j] = cc.cand(sorted ? (int)(next >> (8 * j) & 63u) : min(k + j, cc.count - 1));
+            for (int j = 0; j < 4; ++j) { key[j] = keys[(k + j) * 64]; pair[j] = sectors[(k + j) * 64]; }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const bool there = k + j < cc.count;
-                if (ADVANCE) { leading = leading && there && !(batch[j].dist > passed); from += leading ? 1 : 0; }
-                look(batch[j], there);
+                const Cand q = key_cand(key[j]);
+                const bool there = k + j < held;
+                if (ADVANCE) { leading = leading && there && !(q.dist > passed); from += leading ? 1 : 0; }
+                look(ListEntry{q.flags, q.wall, q.dist, pair[j], 0u}, there);
             }
             k += 4;
-            if (sorted && __uint_as_float(__float_as_uint(batch[3].dist) & ~63u) > enough()) break;
+            more = !(cand_key_distance(key[3]) > enough());
+        }
+        if (complete || !more) return;
+        for (int k0 = 0; k0 < cc.count; k0 += 4) {
+            u64 key[4]; unsigned pair[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) key[j] = cc.cand(k0 + j);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) pair[j] = cc.mv.walls[k0 + j < cc.count ? (unsigned)key[j] >> 16 : 0u].sectors;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { const Cand q = key_cand(key[j]); look(ListEntry{q.flags, q.wall, q.dist, pair[j], 0u}, k0 + j < cc.count); }
         }
     }
-    template <typename Look> __device__ __forceinline__ void each_ledge(const ColumnCtx &cc, Look look) const {
-        for (u64 rest = ledges; rest; rest &= rest - 1)
-            for (int k = __ffsll((long long)rest) - 1; k < cc.count; k += 64) look(cc.cand(k));
+    template <typename Look> __device__ __forceinline__ void each_of(const ColumnCtx &cc, u64 places, Look look) const {
+        for (u64 rest = places; rest; rest &= rest - 1)
+            for (int k = __ffsll((long long)rest) - 1; k < cc.count; k += 64) {
+                const Cand q = key_cand(cc.cand(k));
+                const WallLinks &links = cc.mv.walls[q.wall];
+                look(ListEntry{q.flags, q.wall, q.dist, links.sectors, links.vertices});
+            }
     }
 };
 
@@ -2676,23 +2713,24 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
     const int cur = cs < 0 ? 0 : cs;
     const float prev = c.previous_distance;
     const float prev_eps = prev + 1e-3f;
-    auto incident_c = [&](const Cand &q) { return q.s0 == cur || q.s1 == cur; };
+    auto incident_c = [&](const ListEntry &q) { return MapView::incident(q.sectors, cur); };
+    auto vertices_of = [&](const ListEntry &q) { return LANES > 1 ? q.vertices : mv.walls[q.wall].vertices; };
     // a. nearest incident linedef beyond previous_distance (engine.py:11769-11780)
     float distance = GD_INF; int wi = 0x7fffffff;
     Eval cwi;
-    if constexpr (LANES == 1) list.begin(prev);
+    if constexpr (LANES == 1) list.begin(cc, prev);
     if (cs >= 0) {
         // b. equal-depth solid (engine.py:11784-11807): the nearest one-sided candidate replaces
         // the selection when it lies within 1e-3 of the nearest candidate, found in the same scan.
         u64 nearest = CAND_KEY_NONE, nearest_solid = CAND_KEY_NONE;
-        auto take = [&](const Cand &q, bool there) {
-            const u64 key = there && incident_c(q) && q.dist > prev ? cand_key(q) : CAND_KEY_NONE;
+        auto take = [&](const ListEntry &q, bool there) {
+            const u64 key = there && incident_c(q) && q.dist > prev ? q.key() : CAND_KEY_NONE;
             nearest = key < nearest ? key : nearest;
-            const u64 solid_key = q.s1 < 0 ? key : CAND_KEY_NONE;
+            const u64 solid_key = (q.flags & CF_ONE_SIDED) ? key : CAND_KEY_NONE;
             nearest_solid = solid_key < nearest_solid ? solid_key : nearest_solid;
         };
         if constexpr (LANES > 1) {
-            list.each(cc, [&](const Cand &q) { take(q, true); });
+            list.each(cc, [&](const ListEntry &q) { take(q, true); });
             nearest = list.smallest(nearest); nearest_solid = list.smallest(nearest_solid);
         } else {
             list.template walk<true>(cc, take, [&]() { return cand_key_distance(nearest) + 2e-3f; });
@@ -2707,7 +2745,7 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
     // c. selected endpoint (engine.py:11815-11871)
     bool sel_start = !(cwi.flags & CF_ALONG_HI);
     int sel_vertex = link_vertex(links.vertices, sel_start ? 0 : 1);
-    auto shares_sel_c = [&](const Cand &q) { return (int)q.v0 == sel_vertex || (int)q.v1 == sel_vertex; };
+    auto shares_sel_c = [&](const ListEntry &q) { return MapView::has_vertex(vertices_of(q), sel_vertex); };
     bool continues_po_boundary = (c.flags & ST_PO) && (sel_vertex == c.pend_po_vertex);
     bool continues_ep_boundary = (c.flags & ST_EP) && (sel_vertex == c.pend_ep_vertex);
     int sel_slot = sel_start ? 0 : 1;
@@ -2724,30 +2762,32 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
     const unsigned ps_sectors = links.sectors;
     bool ps_path_geo = cwi.flags & CF_GEO;
     float psd = GD_INF; int psi = 0x7fffffff; int psi_flags = 0;
-    // A later scan of the pass, over all of a lane's own.  `look` says whether `ask`, of which there is one copy, has to be asked about
+    // A later scan of the pass, over all of a lane's own or, where a lane has the column alone, over `places` of the list.  `look` says whether `ask`, of which there is one copy, has to be asked about
     // the candidate as well.
-    auto look_beyond = [&](auto look, auto ask) {
+    auto look_beyond = [&](u64 places, auto look, auto ask) {
         if constexpr (LANES > 1) {
             unsigned asked = 0;
 #pragma unroll
             for (int j = 0; j < list.ENTRIES; ++j) asked |= look(list.own[j]) ? 1u << j : 0u;
             for (; asked; asked &= asked - 1) {
-                Cand q = list.own[0];
+                ListEntry q = list.own[0];
 #pragma unroll
                 for (int j = 1; j < list.ENTRIES; ++j)
                     if ((asked & ((2u << j) - 1u)) == 1u << j) q = list.own[j];
                 ask(q);
             }
         } else {
-            list.each_ledge(cc, [&](const Cand &q) { if (look(q)) ask(q); });
+            list.each_of(cc, places, [&](const ListEntry &q) { if (look(q)) ask(q); });
         }
     };
     if (!sel_is_proj) {
         NearestOf<LANES> solid;
-        look_beyond([&](const Cand &q) {
-            if (incident_c(q) && (q.s1 < 0) && (q.flags & CF_PROJ) && (q.flags & CF_LEDGE) && shares_sel_c(q) && (q.dist > prev_eps)) solid.take(q);
+        u64 places = 0;
+        if constexpr (LANES == 1) places = list.solid_ledges;
+        look_beyond(places, [&](const ListEntry &q) {
+            if (incident_c(q) && (q.flags & CF_ONE_SIDED) && (q.flags & CF_PROJ) && (q.flags & CF_LEDGE) && (q.dist > prev_eps) && shares_sel_c(q)) solid.take(q);
             return false;
-        }, [](const Cand &) {});
+        }, [](const ListEntry &) {});
         solid.share();
         psd = solid.distance(); psi = solid.wall(); psi_flags = solid.flags();
         if (sel_excl_right) {
@@ -2784,31 +2824,29 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
     bool so_is_proj = cwi.flags & CF_PROJ;
     const bool so_excl_right = cwi.flags & CF_ENDS_HERE, so_narrow = cwi.flags & CF_NARROW, so_short = cwi.flags & CF_SHORT;
     float npd = GD_INF; int npi = 0x7fffffff; int npi_flags = 0;
-    const int so_s0 = link_sector(sectors, 0), so_s1 = link_sector(sectors, 1);
     if (!so_is_proj) {
         NearestOf<LANES> near;
-        auto pairs_up = [&](const Cand &q) {
-            return ((q.s0 == so_s0 && q.s1 == so_s1) || (q.s0 == so_s1 && q.s1 == so_s0)) && (fabsf(q.dist - distance) <= tolerance_of(q.dist));
-        };
-        auto eligible = [&](const Cand &q) { return incident_c(q) && (q.s1 >= 0) && (q.flags & CF_PROJ) && (q.dist > prev_eps); };
+        auto pairs_up = [&](const ListEntry &q) { return MapView::same_pair(q.sectors, sectors) && (fabsf(q.dist - distance) <= tolerance_of(q.dist)); };
+        auto eligible = [&](const ListEntry &q) { return incident_c(q) && !(q.flags & CF_ONE_SIDED) && (q.flags & CF_PROJ) && (q.dist > prev_eps); };
         // A lane alone looks for the linedefs of the same pair of sectors about `distance` (a distance that is not finite has none), and for the others, which all
         // begin at this column, among those that do.
         if constexpr (LANES == 1) {
             if (finitef(distance))
-                list.template walk<false>(cc, [&](const Cand &q, bool there) { if (there && eligible(q) && pairs_up(q)) near.take(q); },
+                list.template walk<false>(cc, [&](const ListEntry &q, bool there) { if (there && eligible(q) && pairs_up(q)) near.take(q); },
                                           [&]() { return fmaxf(distance * 1.0080f, distance + 4.0f) + 0.25f; });
         }
-        if (LANES > 1 || (so_excl_right && (so_narrow || so_short)))
-            look_beyond([&](const Cand &q) {
+        u64 places = 0;
+        if constexpr (LANES == 1) places = so_excl_right && (so_narrow || so_short) ? list.ledges : 0;
+        if (LANES > 1 || places != 0)
+            look_beyond(places, [&](const ListEntry &q) {
                 if (!eligible(q)) return false;
                 bool le = q.flags & CF_LEDGE;
-                bool close = pairs_up(q) || (le && so_excl_right && (so_narrow || (shares_sel_c(q) && so_short)) && (fabsf(q.dist - distance) <= tolerance_of(q.dist)));
+                bool close = pairs_up(q) || (le && so_excl_right && (so_narrow || (so_short && shares_sel_c(q))) && (fabsf(q.dist - distance) <= tolerance_of(q.dist)));
                 if (close) near.take(q);
                 return !close && le && so_excl_right && so_narrow;
-            }, [&](const Cand &q) {
+            }, [&](const ListEntry &q) {
                 int bridge; unsigned bridge_sectors;
-                const unsigned pair = (unsigned)(unsigned short)q.s0 | (unsigned)(unsigned short)q.s1 << 16;
-                if (mv.sector_bridge((q.flags & CF_ALONG_HI) ? q.v1 : q.v0, q.wall, pair, no_path_index, no_path_sectors, &bridge, &bridge_sectors)) near.take(q);
+                if (mv.sector_bridge(link_vertex(vertices_of(q), (q.flags & CF_ALONG_HI) ? 1 : 0), q.wall, q.sectors, no_path_index, no_path_sectors, &bridge, &bridge_sectors)) near.take(q);
             });
         near.share();
         npd = near.distance(); npi = near.wall(); npi_flags = near.flags();
@@ -3337,23 +3375,34 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ListShare<LANE
         const unsigned none = __float_as_uint(GD_INF);
         unsigned current_solid = none, other_solid = none;      // distances: positive, so their bits order as they do
         const int v0 = link_vertex(r.vertices, 0), v1 = link_vertex(r.vertices, 1);
-        auto look = [&](const Cand &q, bool there) {
+        auto look = [&](const ListEntry &q, bool there) {
             const float d = q.dist;
             if (!there) return;
-            bool os = q.s1 < 0;
-            bool inc = (q.s0 == cur || q.s1 == cur), oinc = (q.s0 == other_sector || q.s1 == other_sector);
+            bool os = q.flags & CF_ONE_SIDED;
+            bool inc = MapView::incident(q.sectors, cur), oinc = MapView::incident(q.sectors, other_sector);
             bool future = ((q.flags & CF_GEO) || os) && (d > dist_eps);
             if (future && inc) current_next.take(q);
             if (future && oinc) other_next.take(q);
-            bool shares_endpoint = (int)q.v0 == v0 || (int)q.v0 == v1 || (int)q.v1 == v0 || (int)q.v1 == v1;
-            bool shared_solid = os && (shares_endpoint || (q.flags & CF_LEDGE)) && (d > prior_eps) && (d <= dist_eps);
+            bool shared_solid = os && (inc || oinc) && (d > prior_eps) && (d <= dist_eps);
+            bool sgp = (q.flags & CF_GEO) && inc && !os && (d > prior_eps) && (fabsf(d - distance) <= (1.0f / 16.0f));
+            if (sgp || (shared_solid && !(q.flags & CF_LEDGE))) {      // few of them: a lane alone asks memory for the vertices
+                const unsigned vertices = LANES > 1 ? q.vertices : mv.walls[q.wall].vertices;
+                const bool shares_endpoint = MapView::has_vertex(vertices, v0) || MapView::has_vertex(vertices, v1);
+                sgp = sgp && shares_endpoint; shared_solid = shared_solid && shares_endpoint;
+            }
             if (shared_solid && inc) current_solid = min(current_solid, __float_as_uint(d));
             if (shared_solid && oinc) other_solid = min(other_solid, __float_as_uint(d));
-            bool sgp = (q.flags & CF_GEO) && inc && shares_endpoint && !os && (d > prior_eps) && (fabsf(d - distance) <= (1.0f / 16.0f));
             if (sgp) geometric.take(q);
         };
-        if constexpr (LANES > 1) list.each(cc, [&](const Cand &q) { look(q, true); });
-        else list.template walk<false>(cc, look, [&]() { return fmaxf(fmaxf(current_next.distance(), other_next.distance()), distance + 0.07f); });
+        if constexpr (LANES > 1) list.each(cc, [&](const ListEntry &q) { look(q, true); });
+        else {
+            // Which of the two next ones is nearer is all that matters: with one of them found, what the other is beyond it does not.  (But for linedef 0 next
+            // in the current sector, which a search for the other's that finds none counts as tied with.)
+            list.template walk<false>(cc, look, [&]() {
+                const float cnd = current_next.distance(), ond = other_next.distance();
+                return fmaxf(cnd <= ond && current_next.wall() == 0 ? ond : fminf(cnd, ond), distance + 0.07f);
+            });
+        }
         current_next.share(); other_next.share(); geometric.share();
         current_solid = list.smallest(current_solid); other_solid = list.smallest(other_solid);
         const float cnd = current_next.distance(), ond = other_next.distance(), csd = __uint_as_float(current_solid), osd = __uint_as_float(other_solid);
@@ -3794,7 +3843,7 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int str
 static_assert(SEG_COLS == 64, "wall_select_kernel: a work-group is one wavefront, with columns of one strip");
 // The columns of one wavefront: 64 / LANES of a strip's, from the `part`-th such share on.
 template <bool SPLIT, int LANES>
-__device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratch &sc, const LaneCtx &lane_ctx, unsigned (&order_lds)[ORDER_ROWS][64], int local, int strip_x, int part) {
+__device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratch &sc, const LaneCtx &lane_ctx, unsigned *window_lds, int local, int strip_x, int part) {
     const gd_map_desc *m = &dm.d;
     constexpr bool SHARED = LANES > 1;
     constexpr int part_cols = 64 / LANES;
@@ -3814,7 +3863,7 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     if constexpr (SHARED) {
         list.load(cc, lane_of_column);
         unsigned first = 1u;
-        list.each(cc, [&](const Cand &q) { first = (q.flags & CF_LEDGE) ? 0u : first; });
+        list.each(cc, [&](const ListEntry &q) { first = (q.flags & CF_LEDGE) ? 0u : first; });
         boundary_has_po = list.smallest(first) == 0u;
     }
     ColumnState st;
@@ -3824,7 +3873,7 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     st.previous_distance = 0.0f;
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_ep_sectors = 0; st.pend_ep_vertices = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
-    if constexpr (!SHARED) list.start(cc, &order_lds[0][lane_id], boundary_has_po);
+    if constexpr (!SHARED) list.start(cc, window_lds, lane_id, boundary_has_po);
     PassRec *records = sc.pass_rec + sc.pass_at(0, local, x);
     float *path_distances = sc.pass_path_distance + sc.pass_at(0, local, x);
     const size_t pass_stride = (size_t)sc.lane_stride * SW;
@@ -3887,7 +3936,7 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
 template <bool SPLIT, int LANES>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES == 8 ? 3 : 4))) wall_select_kernel(DeviceMap dm, Scratch sc, int first, int longest) {
     __shared__ LaneCtx lane_ctx;
-    __shared__ unsigned order_lds[ORDER_ROWS][64];
+    __shared__ __align__(8) unsigned window_lds[ListShare<1>::WORDS];
     const int shares = longest * LANES, others = (int)gridDim.x - shares, mixed = min(shares, others) & ~7, b = (int)blockIdx.x;
     const bool beyond = b < 2 * mixed ? (b & 8) != 0 : shares - mixed <= b - 2 * mixed;
     const int at = b < 2 * mixed ? ((b >> 4) << 3) | (b & 7) : (beyond ? b - shares : b - mixed);
@@ -3898,11 +3947,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES =
     if constexpr (LANES > 1) {
         // A strip with a column in the spill pool (more entries than its lanes hold) is the first of its wavefronts', a lane a column.
         if (beyond || __ballot(((unsigned)sc.cand_count[(size_t)local * SW + strip_x + threadIdx.x] >> SPILL_SHIFT) != 0) != 0) {
-            if (beyond || part == 0) select_columns<SPLIT, 1>(dm, sc, lane_ctx, order_lds, local, strip_x, 0);
+            if (beyond || part == 0) select_columns<SPLIT, 1>(dm, sc, lane_ctx, window_lds, local, strip_x, 0);
             return;
         }
     }
-    select_columns<SPLIT, LANES>(dm, sc, lane_ctx, order_lds, local, strip_x, part);
+    select_columns<SPLIT, LANES>(dm, sc, lane_ctx, window_lds, local, strip_x, part);
 }
 
 // One wavefront per 64 / SEG_COLS segments.  Segments share nothing but read-only tables; a work-group of the drawing

@@ -1,5 +1,5 @@
-"""The sorting network that orders a column's list (``csrc/gd_order.h``), compiled for the host; and columns with lists of every length that the selection
-orders by a network of its own, drawn with a lane a column, against the CPU oracle."""
+"""The sorting networks that order the nearest entries of a column's list (``csrc/gd_order.h``), compiled for the host; and columns with lists of one to six
+such windows, drawn with a lane a column, against the CPU oracle."""
 
 from __future__ import annotations
 
@@ -15,32 +15,37 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 DRIVER = r"""
 #include "gd_order.h"
-template <int COUNT> static void order(unsigned *v) {
-    unsigned (&w)[COUNT] = *reinterpret_cast<unsigned (*)[COUNT]>(v);
-    order_up(w);
-}
-extern "C" void order_numbers(unsigned *v, int count) {
-    switch (count) { case 32: order<32>(v); break; case 48: order<48>(v); break; case 64: order<64>(v); break; }
+extern "C" void order_numbers(double *v) { order_up(*reinterpret_cast<double (*)[16]>(v)); }
+extern "C" void lowest_of(double *v, double *other) {
+    order_merge_lowest(*reinterpret_cast<double (*)[16]>(v), *reinterpret_cast<double (*)[16]>(other));
 }
 """
 
 
-@pytest.mark.parametrize("count", [32, 48, 64])
-def test_the_network_orders_numbers(tmp_path, count):
+def test_the_networks_order_numbers(tmp_path):
     path = str(tmp_path / "liborder.so")
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-Wno-unknown-pragmas", "-I", CSRC, "-x", "c++", "-o", path, "-"], input=DRIVER, text=True, check=True)
-    order = C.CDLL(path).order_numbers
-    rng = np.random.default_rng(count)
-    for share in np.linspace(0.0, 1.0, count + 1):          # zeros and ones (what a network orders of these it orders of all numbers), then any numbers
-        for numbers in (rng.random((40, count)) < share).astype(np.uint32), rng.integers(0, 1 << 32, (40, count), dtype=np.uint32):
-            for row in numbers:
-                ordered = row.copy()
-                order(ordered.ctypes.data_as(C.c_void_p), count)
-                assert np.array_equal(ordered, np.sort(row))
+    library = C.CDLL(path)
+    pointer = lambda values: values.ctypes.data_as(C.c_void_p)  # noqa: E731
+    for bits in range(1 << 16):              # zeros and ones: what a network orders of these it orders of all numbers
+        row = np.array([bits >> k & 1 for k in range(16)], dtype=np.float64)
+        library.order_numbers(pointer(row))
+        assert np.all(np.diff(row) >= 0.0)
+    for ones in np.ndindex(17, 17):          # all pairs of ordered runs of them
+        runs = [np.concatenate([np.zeros(16 - n), np.ones(n)]) for n in ones]
+        lowest = np.sort(np.concatenate(runs))[:16]
+        library.lowest_of(pointer(runs[0]), pointer(runs[1]))
+        assert np.array_equal(runs[0], lowest)
+    rng = np.random.default_rng(5)
+    for _ in range(200):
+        runs = [np.sort(rng.random(16)) for _ in range(2)]
+        lowest = np.sort(np.concatenate(runs))[:16]
+        library.lowest_of(pointer(runs[0]), pointer(runs[1]))
+        assert np.array_equal(runs[0], lowest)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("sectors", [10, 29, 41, 46, 60, 80])
+@pytest.mark.parametrize("sectors", [10, 14, 29, 41, 60, 80])
 def test_lists_of_every_length_match_the_oracle(oracle, sectors):
     """Corridors seen end on: the longest lists have about as many entries as there are sectors, on 80 more than a column's own slots hold."""
     import launch_rules
