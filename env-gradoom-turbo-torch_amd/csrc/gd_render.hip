@@ -95,6 +95,7 @@ static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and it
 #define CF_SHORT 128    // at most 32 map units long
 #define CF_SUBPIXEL 256 // two-sided, and its clipped span at most one column wide
 #define CF_ONE_SIDED 512
+#define CF_SECTOR0 4096   // one of its sides faces sector 0, which stands in where a column has none
 
 // wall record flags
 #define WF_HC 1        // owns at least one column after every span test
@@ -106,7 +107,8 @@ static_assert(SPILL_DEPTH < (1 << SPILL_SHIFT), "a spilled column's count and it
 #define WF_SHORT CF_SHORT
 #define WF_SUBPIXEL CF_SUBPIXEL // two-sided and at most one column wide (engine.py:11589-11591)
 #define WF_ONE_SIDED CF_ONE_SIDED
-#define WF_SHOWN (WF_FF | WF_NARROW | WF_SHORT | WF_SUBPIXEL | WF_ONE_SIDED)
+#define WF_SECTOR0 CF_SECTOR0
+#define WF_SHOWN (WF_FF | WF_NARROW | WF_SHORT | WF_SUBPIXEL | WF_ONE_SIDED | WF_SECTOR0)
 #define WF_END_SHIFT 16   // bits 16 and up: the column at which the clipped span ends, WF_END_NONE if that is not a column
 #define WF_END_NONE 1023
 
@@ -225,6 +227,7 @@ struct Eval {      // distances/along/geometric/projected/left-edge of one lined
 #define WALL_ONE_SIDED 1
 #define WALL_SPLIT 2
 #define WALL_SHORT 4     // at most 32 map units long
+#define WALL_SECTOR0 8   // one of its sides faces sector 0
 #define WALL_BLOCKING_SHIFT 4
 struct DeviceMap {  // device copy of gd_map_desc (device pointers) + fixed tables
     gd_map_desc d;
@@ -896,7 +899,7 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
                 // an unseen linedef has an empty span (sr == sl), so a two-sided one counts as at most one column wide
                 const int facts = dm.wall_facts[w];
                 span.flags = (ff ? WF_FF : 0) | ((facts & WALL_ONE_SIDED) ? WF_ONE_SIDED : WF_SUBPIXEL) | ((facts & WALL_SPLIT) ? WF_SPLIT : 0) |
-                             WF_NARROW | ((facts & WALL_SHORT) ? WF_SHORT : 0) | (WF_END_NONE << WF_END_SHIFT);
+                             WF_NARROW | ((facts & WALL_SHORT) ? WF_SHORT : 0) | ((facts & WALL_SECTOR0) ? WF_SECTOR0 : 0) | (WF_END_NONE << WF_END_SHIFT);
                 sc.span[(size_t)local * m->wall_count + w] = span;
             }
         }
@@ -967,7 +970,7 @@ __global__ void __launch_bounds__(WHOLE ? SETUP_WHOLE_THREADS : SETUP_THREADS) _
         const i64 span = r.sr - r.sl;
         const int facts = (ff ? WF_FF : 0) | ((span <= 1 && !os) ? WF_SUBPIXEL : 0) | ((known & WALL_SPLIT) ? WF_SPLIT : 0) | (span <= 2 ? WF_NARROW : 0) |
                           ((known & WALL_SHORT) ? WF_SHORT : 0) | ((r.sr >= 0 && r.sr < SW ? (int)r.sr : WF_END_NONE) << WF_END_SHIFT) |
-                          (os ? WF_ONE_SIDED : 0) | (!os && m->side_tex[(w * 2 + (ff ? 0 : 1)) * 3] >= 0 ? SETUP_MASKED : 0) | (span > 0 ? SETUP_SPANS : 0);
+                          (os ? WF_ONE_SIDED : 0) | ((known & WALL_SECTOR0) ? WF_SECTOR0 : 0) | (!os && m->side_tex[(w * 2 + (ff ? 0 : 1)) * 3] >= 0 ? SETUP_MASKED : 0) | (span > 0 ? SETUP_SPANS : 0);
         {
             SetupWall mine;
             mine.segx = segx; mine.segy = segy; mine.offx = offx; mine.offy = offy;
@@ -2079,6 +2082,7 @@ struct ColumnCtx {
     __device__ Eval eval(int w) const { return eval_wall(m, *c, spans + rec_base, x, w, rx, ry); }
 };
 
+#define STANDS_IN (CF_ONE_SIDED | CF_PROJ | CF_LEDGE | CF_SECTOR0)    // all of them: what a column without a sector may find (select_columns)
 // A candidate as a scan looks at it.
 struct ListEntry {
     unsigned short flags, wall;
@@ -2172,7 +2176,7 @@ template <> struct ListShare<1> {
     static __device__ __forceinline__ u64 smallest(u64 v) { return v; }
     static __device__ __forceinline__ unsigned smallest(unsigned v) { return v; }
 
-    __device__ __forceinline__ void start(const ColumnCtx &cc, unsigned *words, int lane_id, bool &any_ledge) {
+    __device__ __forceinline__ void start(const ColumnCtx &cc, unsigned *words, int lane_id, bool &any_ledge, bool &stand_in) {
         keys = reinterpret_cast<u64 *>(words) + lane_id; sectors = words + WINDOW * 2 * 64 + lane_id;
         solid_ledges = 0; ledges = 0; from = 0; held = 0; passed = 0.0f; floor = GD_INF; complete = false;
         unsigned flagged = 0;
@@ -2187,6 +2191,7 @@ template <> struct ListShare<1> {
                 const bool ledge = (f & (CF_LEDGE | CF_PROJ)) == (CF_LEDGE | CF_PROJ);
                 solid |= ledge && (f & CF_ONE_SIDED) ? 1u << j : 0u;
                 portal |= ledge && !(f & CF_ONE_SIDED) ? 1u << j : 0u;
+                stand_in |= (f & STANDS_IN) == STANDS_IN;
             }
             solid_ledges |= (u64)solid << (k0 & 63);
             ledges |= (u64)portal << (k0 & 63);
@@ -3859,12 +3864,13 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     ray_direction(lane_ctx, x, &cc.rx, &cc.ry);
     cc.first = cc.eval(0);
     bool boundary_has_po = false;   // does some entry's span begin at this column
+    bool stand_in = false;          // does some entry show all of STANDS_IN
     ListShare<LANES> list;
     if constexpr (SHARED) {
         list.load(cc, lane_of_column);
-        unsigned first = 1u;
-        list.each(cc, [&](const ListEntry &q) { first = (q.flags & CF_LEDGE) ? 0u : first; });
-        boundary_has_po = list.smallest(first) == 0u;
+        unsigned first = 3u;
+        list.each(cc, [&](const ListEntry &q) { first &= ~(((q.flags & CF_LEDGE) ? 1u : 0u) | ((q.flags & STANDS_IN) == STANDS_IN ? 2u : 0u)); });
+        boundary_has_po = list.smallest(first & 1u) == 0u; stand_in = list.smallest(first & 2u) == 0u;
     }
     ColumnState st;
     st.current_sector = lane_ctx.sector;
@@ -3873,7 +3879,16 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
     st.previous_distance = 0.0f;
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_ep_sectors = 0; st.pend_ep_vertices = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
-    if constexpr (!SHARED) list.start(cc, window_lds, lane_id, boundary_has_po);
+    if constexpr (!SHARED) list.start(cc, window_lds, lane_id, boundary_has_po, stand_in);
+    // A column that has come to the end of its way has no sector.  The passes that follow look at linedef 0 in place of a linedef and at sector 0 in place of
+    // a sector.  They find nothing, draw nothing and change nothing but flags that only matter where something is found, unless a solid linedef of sector 0 begins at
+    // the column, linedef 0's span ends at it, a neighbour of linedef 0 owns it, or an endpoint's boundary is still pending: but for these the column is done.
+    bool ends_quietly = !stand_in && !(cc.first.flags & CF_ENDS_HERE);
+    {
+        int owner; Eval of_owner;
+        endpoint_owner(cc, 0, cc.first, cc.mv.walls[0], &owner, &of_owner);
+        ends_quietly = ends_quietly && owner == 0;
+    }
     PassRec *records = sc.pass_rec + sc.pass_at(0, local, x);
     float *path_distances = sc.pass_path_distance + sc.pass_at(0, local, x);
     const size_t pass_stride = (size_t)sc.lane_stride * SW;
@@ -3923,6 +3938,7 @@ __device__ __forceinline__ void select_columns(const DeviceMap &dm, const Scratc
             const bool changed = pass_advance<SPLIT>(cc, list, st, pc);
             // A pass that found nothing and changed nothing repeats identically for ever.
             if (!(pc.bits & PB_VALID) && !changed) done = true;
+            if (ends_quietly && st.current_sector < 0 && !(st.flags & ST_EP)) done = true;
         }
         if (__ballot(!done) == 0) break;
     }
@@ -6538,7 +6554,8 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
         if (rc == GD_OK) rc = upload(r, around.data(), around.size(), &r->dm.level_box);
         std::vector<int> facts(W, 0);
         for (size_t w = 0; w < W; ++w)
-            facts[w] = (h->wall_sectors[2 * w + 1] < 0 ? WALL_ONE_SIDED : 0) | (h->wall_split_slot[w] >= 0 ? WALL_SPLIT : 0) | (h->wall_len[w] <= 32.0f ? WALL_SHORT : 0);
+            facts[w] = (h->wall_sectors[2 * w + 1] < 0 ? WALL_ONE_SIDED : 0) | (h->wall_split_slot[w] >= 0 ? WALL_SPLIT : 0) | (h->wall_len[w] <= 32.0f ? WALL_SHORT : 0) |
+                       (h->wall_sectors[2 * w] == 0 || h->wall_sectors[2 * w + 1] == 0 ? WALL_SECTOR0 : 0);
         for (int b = 0; b < h->blocking_count; ++b) {
             const int w = h->blocking_walls[b];
             if (w < 0 || (size_t)w >= W) { if (rc == GD_OK) rc = fail(GD_E_ARG, "blocking_walls holds a linedef index out of range"); continue; }
