@@ -2045,7 +2045,6 @@ __global__ void __launch_bounds__(FINISH_THREADS) flat_span_finish_kernel(Scratc
 // ---------------------------------------------------------------------------------------------
 // walls: engine.py:11462-13745
 // ---------------------------------------------------------------------------------------------
-#define WALL_ROWS 8          // rows painted / clipped per step of the wall traversal
 struct ColumnCtx {
     const Tables *tb;
     const gd_map_desc *m;
@@ -2927,33 +2926,37 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
 #define BUFFER_WORDS 0x00027000   // descriptor word 3: 32-bit elements
 #define BUFFER_NOWHERE 0x80000000u   // an offset beyond every plane: 4096 lanes are 1.1 GB
 template <int LANES> struct PixelBuffers {
-    unsigned char *frame;   // [L][240][320] or null
     unsigned int *meta;     // [L][208][320]
-    unsigned char *masked_texel;   // [L][208][320], used where there is no frame
     float *scene_depth;     // [L][208][320] or null
     __amdgpu_buffer_rsrc_t words, depths;   // meta and scene_depth once more, as buffers: see put()
+    __amdgpu_buffer_rsrc_t bytes;           // the frame [L][240][320] or, where there is none, masked_texel [L][208][320]
     unsigned word_column;   // byte offset of (lane, row 0, column) in the four-byte planes
-    unsigned frame_column;  // and in the frame
+    unsigned put_byte_column;  // and in `bytes`, `row_lane` rows further on
     // A column may have several lanes of its wavefront (wall_raster_kernel): all of them hold the same state, and of the rows of a run
     // the lane `row_lane` of them takes every row_lanes-th, from the run's `row_lane`-th on.
     static constexpr int row_lanes = LANES;
+    // a lane's rows per step of a walk over them.  Sixteen lanes take 64 rows a step: a run of 128 is rare, and a step costs what it has room for (16 lanes on
+    // the 320-linedef map with 2 x 64 rows 37.2 us, 64 rows 33.9; eight lanes of four rows and of eight take the same)
+    static constexpr int ROWS = LANES >= 16 ? 4 : 8;
     int row_lane;
     unsigned put_column;    // word_column, `row_lane` rows further on
     __device__ __forceinline__ unsigned int &m(int y) const { return *reinterpret_cast<unsigned int *>(reinterpret_cast<char *>(meta) + (word_column + (unsigned)y * (SW * 4u))); }
     // into row y + row_lane; `y` is the same in the whole wavefront
     __device__ __forceinline__ void put(bool active, int y, unsigned int word) const { __builtin_amdgcn_raw_buffer_store_b32(word, words, active ? put_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
+    // and out of it: zero for a lane that does not ask
+    __device__ __forceinline__ unsigned int get(bool active, int y) const { return __builtin_amdgcn_raw_buffer_load_b32(words, active ? put_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
     __device__ __forceinline__ void put_depth(bool active, int y, float depth) const { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(depth), depths, active ? put_column : BUFFER_NOWHERE, y * (SW * 4), 0); }
-    __device__ __forceinline__ unsigned char &t(int y) const { return masked_texel[(word_column >> 2) + (unsigned)y * (unsigned)SW]; }
+    __device__ __forceinline__ void put_byte(bool active, int y, unsigned char byte) const { __builtin_amdgcn_raw_buffer_store_b8(byte, bytes, active ? put_byte_column : BUFFER_NOWHERE, y * SW, 0); }
     __device__ __forceinline__ float &s(int y) const { return *reinterpret_cast<float *>(reinterpret_cast<char *>(scene_depth) + (word_column + (unsigned)y * (SW * 4u))); }
-    __device__ __forceinline__ unsigned char &f(int y) const { return frame[frame_column + (unsigned)y * (unsigned)SW]; }
 };
 
 // Silhouette bookkeeping: every row >= bot_row holds a clip depth <= bot_depth, every row
 // < top_row holds a clip depth <= top_depth.  Clip depths only ever decrease, so a silhouette
 // at a depth not below the bound cannot change those rows and they need not be visited.
+// No clip recorded so far is deeper than `deepest`.
 struct SilhouetteBounds {
     int bot_row, top_row;
-    float bot_depth, top_depth;
+    float bot_depth, top_depth, deepest;
 };
 
 // The ray distance of a linedef at this column: what the sprite clip of a row whose word names the linedef is at.  (Every clip is
@@ -2964,48 +2967,70 @@ __device__ __forceinline__ float clip_distance(const ColumnCtx &cc, int w) {
     return (offx * segy - offy * segx) / (cc.rx * segy - cc.ry * segx);
 }
 
-// Rows [first, last) of one column take `distance` / `wall` as their sprite clip where it is nearer
-// than what they hold.  WALL_ROWS rows at a time, loads first, so the rows' memory latencies overlap.
+// Rows that a silhouette may still change: they take its linedef as their sprite clip where it is nearer than what they hold.  `behind`: no clip of the column
+// is deeper, so that only rows without any change, and nobody has to be asked how far a clip is.
+struct ClipRun {
+    int first, last;
+    float distance;
+    int wall;
+    bool behind;
+};
+// The whole wavefront walks the rows together, as it does when it paints them (pass_paint): a few rows at a time, loads first, so that the rows' memory
+// latencies overlap and neighbouring columns ask for neighbouring words.  With a loop a column over rows of its own, which asked for the distance of every other
+// clip it met, silhouettes and masked mid-textures (masked_midtexture walks likewise) made wall_raster_kernel take 1013 us for 4096 lanes on the 4000-linedef map,
+// 980 now; 2048 lanes with depths 496, 475; 1024 on the 2000-linedef map 232, 224.  (Notes of the claims that a silhouette will reach, so that it
+// writes them anew without reading: 981 and 238, for the registers and the walks they take.)
 template <typename Pixels>
-__device__ __forceinline__ void clip_rows(const ColumnCtx &cc, Pixels &pb, int first, int last, float distance, int wall) {
+__device__ __forceinline__ void clip_rows(const ColumnCtx &cc, const Pixels &pb, const ClipRun &run) {
+    constexpr int ROWS = Pixels::ROWS;
+    const unsigned rows = (unsigned)max(run.last - run.first, 0);
+    if (!__any(rows != 0)) return;
+    const int step = pb.row_lanes, wave_last = wave_max(rows ? run.last : 0);
+    const bool asks = __any(rows != 0 && !run.behind);
     unsigned int held_wall = 0;           // linedef + 1 of the row before and its distance: rows of one clip are neighbours
-    float held = GD_INF;                  // no clip recorded yet: infinite
-    const int step = pb.row_lanes;
+    float held = GD_INF;
     wave_fence();                         // the column's other lanes may have written these rows
-    for (int y0 = first + pb.row_lane; y0 < last; y0 += WALL_ROWS * step) {
-        unsigned int meta[WALL_ROWS];
+    for (int y = wave_min(rows ? run.first : VH); y < wave_last; y += ROWS * step) {
+        unsigned int meta[ROWS]; bool takes[ROWS];
 #pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) meta[j] = pb.m(min(y0 + j * step, last - 1));
-#pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) {
-            const int y = y0 + j * step;
-            if (y >= last) break;
-            const unsigned int row_wall = meta[j] & META_WALL_MASK;
-            if (row_wall != held_wall) { held_wall = row_wall; held = row_wall ? clip_distance(cc, (int)row_wall - 1) : GD_INF; }
-            if (distance < held) pb.m(y) = (meta[j] & ~META_WALL_MASK) | (unsigned)(wall + 1);
+        for (int j = 0; j < ROWS; ++j) {
+            takes[j] = (unsigned)(y + j * step + pb.row_lane - run.first) < rows;
+            meta[j] = pb.get(takes[j], y + j * step);
         }
+        if (!asks) {
+#pragma unroll
+            for (int j = 0; j < ROWS; ++j) takes[j] = takes[j] && (meta[j] & META_WALL_MASK) == 0;
+        } else {
+#pragma unroll
+            for (int j = 0; j < ROWS; ++j) {
+                const unsigned int row_wall = meta[j] & META_WALL_MASK;
+                if (row_wall != held_wall && !run.behind) { held_wall = row_wall; held = row_wall ? clip_distance(cc, (int)row_wall - 1) : GD_INF; }
+                takes[j] = takes[j] && (row_wall == 0 || (!run.behind && run.distance < held));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) pb.put(takes[j], y + j * step, (meta[j] & ~META_WALL_MASK) | (unsigned)(run.wall + 1));
     }
 }
 
+// The rows that a bottom silhouette from `floor_clip` on and a top one up to `ceiling_clip` may change.
 // `done_from` / `done_to`: rows [done_from, done_to) already carry this silhouette (pass_paint wrote it with
 // the rows the pass took out of a window nothing had touched); an empty range otherwise.
-template <typename Pixels>
-__device__ __forceinline__ void apply_silhouette(const ColumnCtx &cc, Pixels &pb, SilhouetteBounds &sb, bool bottom, bool top, float floor_clip, float ceiling_clip, float distance, int wall,
-                                                 int done_from, int done_to) {
-    if (bottom) {
-        int first = floor_clip <= 0.0f ? 0 : (floor_clip >= (float)VH ? VH : (int)floor_clip);   // clips hold integers
-        int last = (distance >= sb.bot_depth) ? (sb.bot_row < VH ? sb.bot_row : VH) : VH;
-        clip_rows(cc, pb, (done_to > first && done_from <= first) ? done_to : first, last, distance, wall);
-        sb.bot_row = first < sb.bot_row ? first : sb.bot_row;
-        sb.bot_depth = fmaxf(sb.bot_depth, distance);
-    }
-    if (top) {
-        int end = ceiling_clip <= 0.0f ? 0 : (ceiling_clip >= (float)VH ? VH : (int)ceiling_clip);
-        int start = (distance >= sb.top_depth) ? (sb.top_row > 0 ? sb.top_row : 0) : 0;
-        clip_rows(cc, pb, start, (done_from < end && done_to >= end) ? done_from : end, distance, wall);
-        sb.top_row = end > sb.top_row ? end : sb.top_row;
-        sb.top_depth = fmaxf(sb.top_depth, distance);
-    }
+__device__ __forceinline__ ClipRun bottom_run(SilhouetteBounds &sb, float floor_clip, float distance, int wall, int done_from, int done_to) {
+    int first = floor_clip <= 0.0f ? 0 : (floor_clip >= (float)VH ? VH : (int)floor_clip);   // clips hold integers
+    int last = (distance >= sb.bot_depth) ? (sb.bot_row < VH ? sb.bot_row : VH) : VH;
+    const ClipRun run = {(done_to > first && done_from <= first) ? done_to : first, last, distance, wall, distance >= sb.deepest};
+    sb.bot_row = first < sb.bot_row ? first : sb.bot_row;
+    sb.bot_depth = fmaxf(sb.bot_depth, distance);
+    return run;
+}
+__device__ __forceinline__ ClipRun top_run(SilhouetteBounds &sb, float ceiling_clip, float distance, int wall, int done_from, int done_to) {
+    int end = ceiling_clip <= 0.0f ? 0 : (ceiling_clip >= (float)VH ? VH : (int)ceiling_clip);
+    int start = (distance >= sb.top_depth) ? (sb.top_row > 0 ? sb.top_row : 0) : 0;
+    const ClipRun run = {start, (done_from < end && done_to >= end) ? done_from : end, distance, wall, distance >= sb.deepest};
+    sb.top_row = end > sb.top_row ? end : sb.top_row;
+    sb.top_depth = fmaxf(sb.top_depth, distance);
+    return run;
 }
 
 // May pass_paint write a two-sided pass's sprite silhouettes along with the rows the pass takes out of an untouched
@@ -3053,6 +3078,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                            const bool group_valid[3], const float group_bottom[3], const unsigned char *colormap, bool &window_dirty, GapRange &gaps) {
     // The whole wavefront comes here together, columns with nothing to draw as well: they take part in the walks over the rows.
     const bool active = (d.flags & DRAW_RASTER) != 0;
+    constexpr int ROWS = Pixels::ROWS;
     const gd_map_desc *m = cc.m;
     const int x = cc.x, wi = (int)(d.wall_sector & 0xFFFFu);
     const unsigned sector = (d.wall_sector >> 16) & META_SECTOR_MASK;
@@ -3126,7 +3152,7 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
         {
             // The usual case: the rows of a tier are one run, [top, bottom) of a one-sided drawseg, or the upper tier
             // above the lower one.  Each run is painted by a loop that knows its texture, so a row costs an add, a
-            // shift, a texel, a colormap entry and the stores.  WALL_ROWS rows at a time, one batch ahead: the texels
+            // shift, a texel, a colormap entry and the stores.  ROWS rows at a time, one batch ahead: the texels
             // of the next batch are asked for before the rows of this one are stored, so that a step waits for memory
             // once, not for its stores and then for its loads.
             // The wavefront walks the rows together (as above): neighbouring columns then read neighbouring texels and store
@@ -3155,38 +3181,38 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                 // rows from tail_row on take the group's shade: (float)y >= tail_from, which no row meets if that is not a number
                 const int tail_row = !has_tail || !(tail_from < (float)VH) ? VH : (tail_from <= 0.0f ? 0 : (int)ceilf(tail_from));
                 const unsigned meta_word = META_FILLED | (unsigned)(wi + 1), rows = (unsigned)max(last - first, 0);
-                auto load_rows = [&](unsigned char (&texel)[WALL_ROWS]) {
+                auto load_rows = [&](unsigned char (&texel)[ROWS]) {
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) { texel[j] = m->tex_atlas[column + __umul24((frac >> shift) >> 1, atlas_w)]; frac += advance; }
+                    for (int j = 0; j < ROWS; ++j) { texel[j] = m->tex_atlas[column + __umul24((frac >> shift) >> 1, atlas_w)]; frac += advance; }
                 };
-                unsigned char texel[WALL_ROWS];
+                unsigned char texel[ROWS];
                 load_rows(texel);
-                for (int yb = wave_first; yb < wave_last; yb += WALL_ROWS * stride) {
+                for (int yb = wave_first; yb < wave_last; yb += ROWS * stride) {
                     const int y = yb + pb.row_lane;
-                    unsigned char next_texel[WALL_ROWS]; unsigned colour[WALL_ROWS];
+                    unsigned char next_texel[ROWS]; unsigned colour[ROWS];
                     load_rows(next_texel);
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) colour[j] = (y + j * stride >= tail_row ? group_shades : own_shades)[texel[j]];
+                    for (int j = 0; j < ROWS; ++j) colour[j] = (y + j * stride >= tail_row ? group_shades : own_shades)[texel[j]];
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) {
+                    for (int j = 0; j < ROWS; ++j) {
                         const bool own = (unsigned)(y + j * stride - first) < rows;
                         if (DEPTH) pb.put_depth(own, yb + j * stride, d.distance);
                         pb.put(own, yb + j * stride, meta_word | (colour[j] << META_SECTOR_SHIFT));
                     }
 #pragma unroll
-                    for (int j = 0; j < WALL_ROWS; ++j) texel[j] = next_texel[j];
+                    for (int j = 0; j < ROWS; ++j) texel[j] = next_texel[j];
                 }
             }
         }
         if (fresh && tiers_overlap) {
             // The lower and the upper tier share rows (a closed door, say): the lower tier has the say there, row by row.
             unsigned frac_a = d.frac_a + d.step_a * (unsigned)t0, frac_b = d.frac_b + d.step_b * (unsigned)t0;
-            // WALL_ROWS rows at a time, one batch ahead: the texels of the next batch are asked for before the rows of
+            // ROWS rows at a time, one batch ahead: the texels of the next batch are asked for before the rows of
             // this one are stored, so that a step waits for memory once, not for its stores and then for its loads
-            auto load_rows = [&](int yb, unsigned char (&texel)[WALL_ROWS], unsigned &draw, unsigned &tail) {
+            auto load_rows = [&](int yb, unsigned char (&texel)[ROWS], unsigned &draw, unsigned &tail) {
                 draw = 0; tail = 0;
 #pragma unroll
-                for (int j = 0; j < WALL_ROWS; ++j) {
+                for (int j = 0; j < ROWS; ++j) {
                     const int y = yb + j;
                     const float py = (float)y;
                     const bool lower_span = (py >= r.lower_top) && (py < r.bottom);
@@ -3203,22 +3229,22 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
                     frac_a += d.step_a; frac_b += d.step_b;
                 }
             };
-            unsigned char texel[WALL_ROWS]; unsigned draw = 0, tail = 0;
+            unsigned char texel[ROWS]; unsigned draw = 0, tail = 0;
             if (t0 < t1) load_rows(t0, texel, draw, tail);
-            for (int yb = t0; yb < t1; yb += WALL_ROWS) {
-                unsigned char next_texel[WALL_ROWS]; unsigned next_draw = 0, next_tail = 0;
+            for (int yb = t0; yb < t1; yb += ROWS) {
+                unsigned char next_texel[ROWS]; unsigned next_draw = 0, next_tail = 0;
 #pragma unroll
-                for (int j = 0; j < WALL_ROWS; ++j) next_texel[j] = 0;
-                if (yb + WALL_ROWS < t1) load_rows(yb + WALL_ROWS, next_texel, next_draw, next_tail);
+                for (int j = 0; j < ROWS; ++j) next_texel[j] = 0;
+                if (yb + ROWS < t1) load_rows(yb + ROWS, next_texel, next_draw, next_tail);
 #pragma unroll
-                for (int j = 0; j < WALL_ROWS; ++j) {
+                for (int j = 0; j < ROWS; ++j) {
                     if (!(draw & (1u << j))) continue;
                     const unsigned colour = ((tail & (1u << j)) ? group_shades : own_shades)[texel[j]];
                     if (DEPTH) pb.s(yb + j) = d.distance;
                     pb.m(yb + j) = META_FILLED | (colour << META_SECTOR_SHIFT) | (unsigned)(wi + 1);
                 }
 #pragma unroll
-                for (int j = 0; j < WALL_ROWS; ++j) texel[j] = next_texel[j];
+                for (int j = 0; j < ROWS; ++j) texel[j] = next_texel[j];
                 draw = next_draw; tail = next_tail;
             }
         }
@@ -3278,7 +3304,8 @@ __device__ __forceinline__ void pass_paint(const ColumnCtx &cc, const ColumnStat
     }
 }
 
-// engine.py:12885-13069: what a pass does to its column's clips, its masked drawseg snapshot and its sprite silhouettes
+// engine.py:12885-13069: what a pass does to its column's clips, its masked drawseg snapshot and its sprite silhouettes.  The whole wavefront comes here
+// together, columns whose pass does nothing as well (clip_rows).
 template <typename Pixels>
 __device__ __forceinline__ void advance_clips(const ColumnCtx &cc, ColumnState &c, const PassDraw &d, const PassRows &r, Pixels &pb, SilhouetteBounds &sb, bool window_untouched, GapRange &gaps,
                               const Scratch &sc, size_t at) {   // the pass's place in the chunk's planes
@@ -3288,6 +3315,8 @@ __device__ __forceinline__ void advance_clips(const ColumnCtx &cc, ColumnState &
     const int x = cc.x, wi = (int)(d.wall_sector & 0xFFFFu);
     const float distance = d.distance;
     auto row_of = [](float clip) { return clip <= 0.0f ? 0 : (clip >= (float)VH ? VH : (int)clip); };
+    const ClipRun nowhere = {VH, 0, 0.0f, 0, true};
+    ClipRun bottom = nowhere, top = nowhere;
     if ((d.flags & (DRAW_RASTER | DRAW_ONE_SIDED)) == DRAW_RASTER) {
         // o. clip updates (engine.py:12888-12913)
         const bool draws_upper = (d.flags & (DRAW_UPPER | DRAW_TEXTURE_B)) == (DRAW_UPPER | DRAW_TEXTURE_B), draws_lower = (d.flags & (DRAW_LOWER | DRAW_TEXTURE_A)) == (DRAW_LOWER | DRAW_TEXTURE_A);
@@ -3302,17 +3331,18 @@ __device__ __forceinline__ void advance_clips(const ColumnCtx &cc, ColumnState &
         // pass_paint, finding the window untouched, has written the silhouette into the rows that this pass took out
         // of it: [new floor clip, old floor clip) at the bottom, [old ceiling clip, new ceiling clip) at the top
         const int old_floor = row_of(before.floor_clip), old_ceiling = row_of(before.ceiling_clip);
-        if (window_untouched && silhouette_folds(d, r)) {
-            // one call per side: the rows already done differ.  pass_paint stays inside the old window, and a sector whose
-            // ceiling lies below its floor can carry a clip past the window's other end: then the rows beyond that end
-            // are not done, and the range is cut there (apply_silhouette then takes no short cut and visits them all).
-            apply_silhouette(cc, pb, sb, bottom_sil, false, c.floor_clip, c.ceiling_clip, distance, wi, max(row_of(c.floor_clip), old_ceiling), old_floor);
-            apply_silhouette(cc, pb, sb, false, top_sil, c.floor_clip, c.ceiling_clip, distance, wi, old_ceiling, min(row_of(c.ceiling_clip), old_floor));
-        } else {
-            apply_silhouette(cc, pb, sb, bottom_sil, top_sil, c.floor_clip, c.ceiling_clip, distance, wi, 0, 0);
-        }
+        // (pass_paint stays inside the old window, and a sector whose ceiling lies below its floor can carry a clip past the window's other end: then the
+        // rows beyond that end are not done, and the range is cut there: all of them are visited.)
+        const bool folded = window_untouched && silhouette_folds(d, r);
+        if (bottom_sil) bottom = bottom_run(sb, c.floor_clip, distance, wi, folded ? max(row_of(c.floor_clip), old_ceiling) : 0, folded ? old_floor : 0);
+        if (top_sil) top = top_run(sb, c.ceiling_clip, distance, wi, folded ? old_ceiling : 0, folded ? min(row_of(c.ceiling_clip), old_floor) : 0);
     }
+    clip_rows(cc, pb, bottom);
+    clip_rows(cc, pb, top);
+    if (d.flags & DRAW_RASTER) sb.deepest = fmaxf(sb.deepest, distance);     // what the pass painted shows its linedef
+    if (!__any(d.flags & DRAW_PS_KEEPS)) return;
     // r. clips of the geometric portal behind a projected solid (engine.py:12969-13069)
+    bottom = nowhere; top = nowhere;
     if (d.flags & DRAW_PS_KEEPS) {
         const PassRec rec = sc.pass_rec[at];
         const int path = rec.ps_path, current = rec.render_current;
@@ -3347,8 +3377,12 @@ __device__ __forceinline__ void advance_clips(const ColumnCtx &cc, ColumnState &
         bool pmasked = ptex[0] >= 0;
         bool pbottom = (view_floor > pof) || (L.view_z < pof) || pmasked;
         bool ptop = (view_ceiling < poc) || (L.view_z > poc) || pmasked;
-        apply_silhouette(cc, pb, sb, pbottom, ptop, c.floor_clip, c.ceiling_clip, path_distance, path, 0, 0);
+        if (pbottom) bottom = bottom_run(sb, c.floor_clip, path_distance, path, 0, 0);
+        if (ptop) top = top_run(sb, c.ceiling_clip, path_distance, path, 0, 0);
+        sb.deepest = fmaxf(sb.deepest, path_distance);
     }
+    clip_rows(cc, pb, bottom);
+    clip_rows(cc, pb, top);
 }
 
 // engine.py:13070-13371: where a pass takes its column's traversal: next sector, previous distance, pending boundaries
@@ -3479,103 +3513,105 @@ __device__ __forceinline__ bool pass_advance(const ColumnCtx &cc, ListShare<LANE
     return !same_state(before, c);
 }
 
-// engine.py:13424-13744 for one column
+// engine.py:13424-13744 for one column; the whole wavefront comes here
 template <bool DEPTH, bool GENERAL, typename Pixels>
 __device__ __forceinline__ void masked_midtexture(const DeviceMap &dm, const ColumnCtx &cc, const Scratch &sc, int local, const ColumnState &c, Pixels &pb, const unsigned char *colormap) {
+    constexpr int ROWS = Pixels::ROWS;
     const gd_map_desc *m = cc.m;
     const LaneCtx &L = *cc.c;
     const int x = cc.x;
     const u64 hit = sc.masked_hit[(size_t)local * SW + x];
-    if (hit == CAND_KEY_NONE) return;
     const int mw = cand_key_wall(hit), cand_flags = cand_key_flags(hit);
     const float md = cand_key_distance(hit);
     const int mside = (cand_flags & CF_FF) ? 0 : 1;   // engine.py:13436-13444, the float32 facing test
     bool left_edge = cand_flags & CF_LEDGE;
     bool has_saved = c.masked_wall == mw;
-    if (!(has_saved || left_edge)) return;
-    const WallSide &ws = dm.wall_side[2 * mw + mside];
-    const WallGeo &geo = sc.geo[sc.geo_slot[cc.rec_base + (unsigned)mw]];
-    const MaskedGeo &masked = sc.masked_geo[(size_t)local * dm.masked_count + dm.masked_slot[mw]];
-    const int texture_id = ws.tex[0];
-    const Tables &tb = *cc.tb;
-    const int front_sector = m->wall_sectors[2 * mw], back_sector = m->wall_sectors[2 * mw + 1];
-    const int light_sector = mside == 0 ? front_sector : back_sector;
-    const float world_top = fminf(tb.ceil_h(front_sector), tb.ceil_h(back_sector));
-    const int th = m->tex_h[texture_id];   // the texture's own height, whatever its row mask (engine.py:13480-13483)
-    float owall_top, owall_bottom;
-    i64 visibility = geo.visibility[mside].at(x);
-    bool split = false;
-    if (GENERAL) {
-        const WallRec &wr = cc.rec(mw);
-        split = (wr.flags & WF_SPLIT) != 0;
-        if (split) {
-            const FragmentChoice fragment = choose_fragment<true>(m, cc.frags, wr, mw, x);
+    const bool shows = hit != CAND_KEY_NONE && (has_saved || left_edge);
+    if (!__any(shows)) return;
+    // what a column walks over its rows with: none of them, and the first texel of the atlas
+    int y0 = VH, y1 = 0;
+    unsigned row_step = 0, row_base = 0, texel_base = 0, shift = 0, shades = 0;
+    if (shows) {
+        const WallSide &ws = dm.wall_side[2 * mw + mside];
+        const WallGeo &geo = sc.geo[sc.geo_slot[cc.rec_base + (unsigned)mw]];
+        const MaskedGeo &masked = sc.masked_geo[(size_t)local * dm.masked_count + dm.masked_slot[mw]];
+        const int texture_id = ws.tex[0];
+        const Tables &tb = *cc.tb;
+        const int front_sector = m->wall_sectors[2 * mw], back_sector = m->wall_sectors[2 * mw + 1];
+        const int light_sector = mside == 0 ? front_sector : back_sector;
+        const float world_top = fminf(tb.ceil_h(front_sector), tb.ceil_h(back_sector));
+        const int th = m->tex_h[texture_id];   // the texture's own height, whatever its row mask (engine.py:13480-13483)
+        float owall_top, owall_bottom;
+        i64 visibility = geo.visibility[mside].at(x);
+        bool split = false;
+        if (GENERAL) {
+            const WallRec &wr = cc.rec(mw);
+            split = (wr.flags & WF_SPLIT) != 0;
+            if (split) {
+                const FragmentChoice fragment = choose_fragment<true>(m, cc.frags, wr, mw, x);
 #pragma unroll 1
-            for (int k = 0; k < 2; ++k) {
-                float v = project(L, wr, fragment, k == 0 ? world_top : world_top - (float)th, x);
-                if (k == 0) owall_top = v; else owall_bottom = v;
+                for (int k = 0; k < 2; ++k) {
+                    float v = project(L, wr, fragment, k == 0 ? world_top : world_top - (float)th, x);
+                    if (k == 0) owall_top = v; else owall_bottom = v;
+                }
+                if (fragment.lights) visibility = wall_visibility(*fragment.rec, mside, x);
             }
-            if (fragment.lights) visibility = wall_visibility(*fragment.rec, mside, x);
         }
+        if (!split) {
+            const bool in_span = x >= geo.span0 && x < geo.span1;
+            const HeightBend top_bend = masked.bend[0], bottom_bend = masked.bend[1];
+            owall_top = !in_span && bends(top_bend) ? height_row(masked.outside[0], x) : bent_row(height_row(masked.line[0], x), top_bend, x);
+            owall_bottom = !in_span && bends(bottom_bend) ? height_row(masked.outside[1], x) : bent_row(height_row(masked.line[1], x), bottom_bend, x);
+        }
+        float mceil = fmaxf(owall_top, has_saved ? c.masked_ceiling_clip : 0.0f);
+        float mfloor = fminf(owall_bottom, has_saved ? c.masked_floor_clip : (float)VH);
+        i64 u_base, swall_cur;
+        texture_column(geo, geo.past_left != 0, ws, mside, x, &u_base, &swall_cur);
+        const i64 mu = tb.wrap_column(texture_id, u_base);
+        int height_bits = ilog2(th);
+        i64 vertical_step = mul64(swall_cur, shl64(1, 14 - height_bits));
+        i64 center_fixed = L.center_fixed;
+        i64 texture_mid = round_to_i64((world_top - L.view_z) * 65536.0f + ws.offset_y * 65536.0f);
+        const i64 sprite_scale = masked.scale.at(x);
+        i64 top_screen = center_fixed - (mul64(texture_mid, sprite_scale) >> 16);
+        i64 post_top = top_screen >> 16;
+        i64 post_bottom = ((top_screen + mul64(sprite_scale, th) - FIXED_UNIT) >> 16) + 1;
+        i64 clipped_top = max64(post_top, (i64)mceil);
+        i64 clipped_bottom = min64(post_bottom, (i64)mfloor);
+        i64 dc_iscale = mul64(swall_cur, FIXED_UNIT) >> 18;
+        bool initial_post = clipped_top < clipped_bottom;
+        i64 frac_start = texture_mid + mul64(clipped_top, dc_iscale) - (mul64(center_fixed - FIXED_UNIT, dc_iscale) >> 16);
+        i64 frac_end = frac_start + mul64(clipped_bottom - clipped_top - 1, dc_iscale);
+        bool extends = initial_post && ((float)clipped_bottom < mfloor) && (frac_end < (i64)th * FIXED_UNIT - dc_iscale);
+        clipped_bottom += extends ? 1 : 0;
+        float light = (tb.light(light_sector) + (float)(L.flash_light * 16)) + ws.contrast;
+        shades = (unsigned)wall_shade(light, visibility) * 256u;
+        y0 = (int)clampi(clipped_top, 0, VH); y1 = (int)clampi(clipped_bottom, 0, VH);
+        // as in pass_paint: only the low 32 bits of the row fraction matter, and they advance by the step's low 32 bits
+        row_step = (unsigned)vertical_step;
+        row_base = (unsigned)(shl64(texture_mid, 16 - height_bits) + (mul64(vertical_step, FIXED_UNIT - center_fixed) >> 16));
+        texel_base = (unsigned)texture_id * (unsigned)(m->tex_max_h * m->tex_max_w) + (unsigned)mu;    // the atlas is below 4 GiB
+        shift = 31u - (unsigned)height_bits;
     }
-    if (!split) {
-        const bool in_span = x >= geo.span0 && x < geo.span1;
-        const HeightBend top_bend = masked.bend[0], bottom_bend = masked.bend[1];
-        owall_top = !in_span && bends(top_bend) ? height_row(masked.outside[0], x) : bent_row(height_row(masked.line[0], x), top_bend, x);
-        owall_bottom = !in_span && bends(bottom_bend) ? height_row(masked.outside[1], x) : bent_row(height_row(masked.line[1], x), bottom_bend, x);
-    }
-    float mceil = fmaxf(owall_top, has_saved ? c.masked_ceiling_clip : 0.0f);
-    float mfloor = fminf(owall_bottom, has_saved ? c.masked_floor_clip : (float)VH);
-    i64 u_base, swall_cur;
-    texture_column(geo, geo.past_left != 0, ws, mside, x, &u_base, &swall_cur);
-    const i64 mu = tb.wrap_column(texture_id, u_base);
-    int height_bits = ilog2(th);
-    i64 vertical_step = mul64(swall_cur, shl64(1, 14 - height_bits));
-    i64 center_fixed = L.center_fixed;
-    i64 texture_mid = round_to_i64((world_top - L.view_z) * 65536.0f + ws.offset_y * 65536.0f);
-    const i64 sprite_scale = masked.scale.at(x);
-    i64 top_screen = center_fixed - (mul64(texture_mid, sprite_scale) >> 16);
-    i64 post_top = top_screen >> 16;
-    i64 post_bottom = ((top_screen + mul64(sprite_scale, th) - FIXED_UNIT) >> 16) + 1;
-    i64 clipped_top = max64(post_top, (i64)mceil);
-    i64 clipped_bottom = min64(post_bottom, (i64)mfloor);
-    i64 dc_iscale = mul64(swall_cur, FIXED_UNIT) >> 18;
-    bool initial_post = clipped_top < clipped_bottom;
-    i64 frac_start = texture_mid + mul64(clipped_top, dc_iscale) - (mul64(center_fixed - FIXED_UNIT, dc_iscale) >> 16);
-    i64 frac_end = frac_start + mul64(clipped_bottom - clipped_top - 1, dc_iscale);
-    bool extends = initial_post && ((float)clipped_bottom < mfloor) && (frac_end < (i64)th * FIXED_UNIT - dc_iscale);
-    clipped_bottom += extends ? 1 : 0;
-    float light = (tb.light(light_sector) + (float)(L.flash_light * 16)) + ws.contrast;
-    i64 shade = wall_shade(light, visibility);
-    int y0 = (int)clampi(clipped_top, 0, VH), y1 = (int)clampi(clipped_bottom, 0, VH);
-    // WALL_ROWS rows at a time: texels and meta words are asked for together, then the stores
-    // as in pass_paint: only the low 32 bits of the row fraction matter, and they advance by the step's low 32 bits
-    const unsigned row_step = (unsigned)vertical_step;
-    const unsigned row_base = (unsigned)(shl64(texture_mid, 16 - height_bits) + (mul64(vertical_step, FIXED_UNIT - center_fixed) >> 16));
-    const size_t texel_base = (size_t)texture_id * m->tex_max_h * m->tex_max_w + (size_t)mu;
-    const unsigned atlas_w = (unsigned)m->tex_max_w;
-    const int stride = pb.row_lanes;
+    // The wavefront walks the rows together (pass_paint).  The texel goes to the frame where there is one; otherwise it waits for the kernel that assembles
+    // the frame.
+    const unsigned atlas_w = (unsigned)m->tex_max_w, rows = (unsigned)max(y1 - y0, 0);
+    const int stride = pb.row_lanes, wave_last = wave_max(rows ? y1 : 0);
     wave_fence();                         // the column's other lanes may have written these rows
-    for (int yb = y0 + pb.row_lane; yb < y1; yb += WALL_ROWS * stride) {
-        unsigned char texel[WALL_ROWS]; unsigned int word[WALL_ROWS];
+    for (int yb = wave_min(rows ? y0 : VH); yb < wave_last; yb += ROWS * stride) {
+        unsigned char texel[ROWS]; unsigned int word[ROWS];
 #pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) {
-            const int y = min(yb + j * stride, y1 - 1);
-            const unsigned fraction = row_base + row_step * (unsigned)y;
-            const unsigned mv_ = (fraction >> (31 - height_bits)) >> 1;
-            texel[j] = m->tex_atlas[texel_base + __umul24(mv_, atlas_w)];
-            word[j] = pb.m(y);
+        for (int j = 0; j < ROWS; ++j) {
+            const int y = yb + j * stride + pb.row_lane;
+            texel[j] = m->tex_atlas[texel_base + __umul24(((row_base + row_step * (unsigned)y) >> shift) >> 1, atlas_w)];
+            word[j] = pb.get((unsigned)(y - y0) < rows, yb + j * stride);
         }
 #pragma unroll
-        for (int j = 0; j < WALL_ROWS; ++j) {
-            const int y = yb + j * stride;
-            if (y >= y1) continue;
-            // the texel goes to the frame where there is one; otherwise it waits for the kernel that assembles the frame
-            const unsigned char colour = colormap[shade * 256 + texel[j]];
-            if (pb.frame) pb.f(y) = colour;
-            else pb.t(y) = colour;
-            pb.m(y) = word[j] | META_MASKED;
-            if (DEPTH) pb.s(y) = md;
+        for (int j = 0; j < ROWS; ++j) {
+            const bool own = (unsigned)(yb + j * stride + pb.row_lane - y0) < rows;
+            pb.put_byte(own, yb + j * stride, colormap[shades + texel[j]]);
+            pb.put(own, yb + j * stride, word[j] | META_MASKED);
+            if (DEPTH) pb.put_depth(own, yb + j * stride, md);
         }
     }
 }
@@ -4036,14 +4072,15 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     cc.x = x;
     ray_direction(lane_ctx, x, &cc.rx, &cc.ry);
     PixelBuffers<PARTS> pb;
-    pb.frame = frame_base;
-    pb.meta = sc.meta; pb.masked_texel = sc.masked_texel;
+    pb.meta = sc.meta;
     pb.scene_depth = DEPTH ? sc.scene_depth : nullptr;
     pb.word_column = ((unsigned)local * (VH * SW) + (unsigned)x) * 4u;
     pb.words = __builtin_amdgcn_make_buffer_rsrc(sc.meta, 0, lane_count * (VH * SW * 4), BUFFER_WORDS);
     pb.depths = __builtin_amdgcn_make_buffer_rsrc(pb.scene_depth, 0, DEPTH ? lane_count * (VH * SW * 4) : 0, BUFFER_WORDS);
-    pb.frame_column = (unsigned)local * (unsigned)frame_stride + (unsigned)x;
     pb.row_lane = PARTS == 1 ? 0 : lane_id / part_cols;
+    const unsigned byte_stride = frame_base ? (unsigned)frame_stride : VH * SW;
+    pb.bytes = __builtin_amdgcn_make_buffer_rsrc(frame_base ? frame_base : sc.masked_texel, 0, (frame_base || sc.masked_texel) ? lane_count * (int)byte_stride : 0, BUFFER_WORDS);
+    pb.put_byte_column = (unsigned)local * byte_stride + (unsigned)pb.row_lane * SW + (unsigned)x;
     pb.put_column = pb.word_column + (unsigned)pb.row_lane * (SW * 4u);
     // the meta plane arrives with whatever the last frame left: see GapRange for how every row gets written
     ColumnState st;   // only the clips and the masked-drawseg snapshot live here; the traversal state stayed in wall_select_kernel
@@ -4053,7 +4090,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     st.previous_distance = 0.0f;
     st.pend_po_vertex = -1; st.pend_ep_vertex = -1; st.pend_ep_wall = 0; st.pend_ep_sectors = 0; st.pend_ep_vertices = 0; st.pend_eb_index = 0;
     st.pend_pb_index = 0; st.pend_pb_sector = -1; st.pend_pb_exit = 0.0f; st.flags = 0;
-    SilhouetteBounds sb; sb.bot_row = VH; sb.top_row = 0; sb.bot_depth = -GD_INF; sb.top_depth = -GD_INF;
+    SilhouetteBounds sb; sb.bot_row = VH; sb.top_row = 0; sb.bot_depth = -GD_INF; sb.top_depth = -GD_INF; sb.deepest = -GD_INF;
     const int passes = sc.pass_count[(size_t)local * SW + x];
     const size_t first_record = sc.pass_at(0, local, x), pass_stride = (size_t)sc.lane_stride * SW;
     const unsigned int *geo_slots = sc.geo_slot + cc.rec_base;
@@ -4108,7 +4145,7 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
             group_valid[1] = same_group && (agreed & 2) && (shared_lower_top < shared_bottom);
             group_valid[2] = same_group && (agreed & 4) && (shared_top < shared_upper_bottom);
             pass_paint<DEPTH>(cc, st, d, rows, pb, group_valid, common_bottom, colormap_lds, window_dirty, gaps);
-            if (d.flags & (DRAW_RASTER | DRAW_PS_KEEPS)) advance_clips(cc, st, d, rows, pb, sb, !window_dirty, gaps, sc, first_record + (size_t)(group + k) * pass_stride);
+            advance_clips(cc, st, d, rows, pb, sb, !window_dirty, gaps, sc, first_record + (size_t)(group + k) * pass_stride);
         }
     }
     // what is left of a window no one-sided drawseg closed shows the flat pass's picture
