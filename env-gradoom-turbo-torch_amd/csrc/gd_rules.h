@@ -11,59 +11,58 @@
 // 188 / 179, 4096 lanes 708 / 509.
 inline bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || linedefs <= 2 * SETUP_THREADS; }
 
-// wall_select_kernel's launch for the longest strips: how many of them, and how many lanes a column has there.  More strips and more lanes
-// shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a
-// large one's does.  Where the lists are short (they follow the map's linedefs) there is little to shorten: fewer strips in large batches, and none
-// where the lanes are as many as twelve times the linedefs beyond a hundred, in the largest batches of up to 900 linedefs, or on the
-// smallest maps.  Stage times in us of no such launch / 768 strips (1024 from 1024 linedefs on) of 8 / of 16 lanes
-// (of 32), in brackets what it took with the lists in LDS and 8 columns of one lane a wavefront:
-//   lanes       120              320                        800                         2000                          4000
-//      16    46 / 55 / 76     97 / 53 / 64 (61; [60])    168 / 74 / 62 (52)         339 / 120 / 89 (68; [151])     361 / 119 / 90 (69; [156])
-//     128    55 / 60 / 77     133 / 69 / 81 ([83])       181 / 83 / 71              436 / 153 / 113 (104; [203])   1003 / 236 / 172 (145; [430])
-//     256    59 / 73          137 / 84 / 96 ([102])      212 / 106 / 99             447 / 164 / 132 ([214])        999 / 247 / 197 ([420])
-//     512    63 / 81          140 / 107 / 119 ([111])    220 / 126 / 128            453 / 172 / 178 ([267])        1003 / 275 / 257 ([463])
-//    1024    69               149 / 146 ([138])          241 / 174 / 174            520 / 265 / 264 ([336])        1060 / 408 / 413 ([563])
-//    2048    80               166 / 180 ([171])          277 / 234 / 235            549 / 371 / 370 ([411])        1120 / 652 / 647 ([727])
-//    4096    130              230 / 288 ([279])          328 / 363                  667 / 604 / 576 ([600])        1249 / 945 / 887 ([966])
-// (the last two rows with 768 and with 512 strips.)  None / 256 / 512 / 768 strips of 8 lanes on maps below 1024 linedefs, in brackets as above:
-//   lanes         200 linedefs            240                   320                330, bricks               500                701, bricks               1000
-//     256    93/ 72/ 64/ 67 ( 67)   91/ 72/ 66/ 66 ( 72)  136/ 97/ 82/ 83 (104)  154/109/ 89/ 92 (105)  159/107/ 85/ 87 (116)  294/160/127/129 (166)
-//     512    97/ 84/ 80/ 85 ( 79)   95/ 92/ 83/ 80 ( 81)  138/121/109/105 (111)  176/131/120/112 (127)  198/131/123/115 (127)  303/188/176/151 (190)
-//     768   101/ 97/ 91/ 96 ( 90)   98/ 99/ 90/ 92 ( 89)  145/134/127/127 (128)  182/142/144/135 (145)  200/160/144/146 (148)  321/240/204/195 (210)  351/219/194/183 (215)
-//    1024   105/102/ 98/106 ( 97)  102/106/101/103 (100)  147/138/142/141 (138)  190/150/151/152 (150)  204/165/160/158 (160)  325/265/227/215 (231)  360/249/231/205 (235)
-//    1280   107/107/110/111 (108)  104/109/112/110 (110)  151/147/151/151 (146)  200/160/162/159 (162)  211/177/174/171 (173)  340/273/243/234 (250)  369/267/240/218 (248)
-//    1536   109/116/113/120 (113)  108/118/115/115 (115)  157/155/159/163 (157)  203/169/172/169 (171)  216/181/187/188 (186)  350/297/269/255 (280)  381/281/252/244 (263)
-//    2048   116/122/128/139 (124)  114/128/124/131 (125)  165/166/177/191 (170)  214/190/188/198 (184)  239/198/209/223 (206)  363/310/298/303 (312)  386/298/282/290 (296)
-//    2560   120/137/145/157 (137)  120/142/138/148 (132)  179/192/204/218 (194)  224/199/209/222 (200)  249/224/238/252 (228)  379/330/335/353 (344)  402/334/321/340 (326)
-//    3072   127/153/162/173 (153)  137/148/154/164 (146)  188/219/232/246 (220)  231/225/238/251 (225)  260/255/268/285 (259)  395/369/385/402 (372)  424/356/366/382 (358)
-//    4096   150/189/197/209 (189)  148/184/190/200 (182)  227/276/289/306 (279)  252/289/301/314 (288)  284/326/342/359 (332)  425/466/483/500 (472)  475/449/465/482 (458)
-// Over these and thirteen more maps of 60 to 800 linedefs, 16 to 4096 lanes, the rule's choice takes 1.2 % more in the mean than the best of the
-// four, 16 % at most.  Against the brackets' it is 7 % faster in the geometric mean; it is more than 5 % slower on maps of up to 240 linedefs
-// (by 4 to 12 us, mostly at 48 to 384 lanes) and at two places on 280.
+// wall_select_kernel: how many of the longest strips have their columns' lists shared out, and over how many lanes a column.  More strips and more lanes
+// shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a large one's does.
+// Since a lane alone keeps its column's nearest entries at hand, few strips are left to which sharing matters: none in large batches of all but the largest maps.
+// Stage times in us of strips:lanes a column, two sets of poses; "before" is what the line of up to 1024 strips took that lists read from memory asked for.
+//   lanes    240 linedefs                      320                              500                                        701, bricks
+//     96   0 68, 128:8 52, 256:16 74         84, 59, 72                       91, 128:16 55, 256:32 60                   152, 256:8 98, 256:16 78, 256:32 70
+//    256   80, 57, 68 (before 70)            86, 62, 66 (73)                  94, 256:8 65, 256:16 62 (68)               154, 103, 92, 512:16 94 (106)
+//    384   82, 60, 69 (85)                   90, 63, 68 (87)                  98, 72, 71, 384:16 70 (83)                 161, 104, 102, 384:16 96 (116)
+//    704   93, 73, 256:8 78 (113)            97, 81, 83 (112)                 111, 83, 89, 128:8 89 (112)                170, 119, 125, 128:8 125 (158)
+//   1024   98, 81, 84 (122)                  104, 87, 89 (124)                118, 94, 102, 128:8 95 (123)               178, 131, 138, 128:8 138 (185)
+//   1536   108, 97, 105 (127)                115, 99, 107 (130)               124, 109, 118, 128:8 112 (139)             191, 145, 156, 128:8 155 (206)
+//   2048   116, 122, 130 (117)               124, 122, 132 (151)              134, 134, 138, 128:8 124 (151)             206, 178, 189, 128:8 170 (232)
+//   4096   184, 216, 227 (184)               191, 224, 235 (191)              195, 240, 236 (195)                        263, 322, 314 (264)
+//   lanes    1000 linedefs                          2000                                             4000
+//     96                                          256:8 117, 256:16 85, 256:32 76 (81)             256:8 188, 256:16 132, 256:32 109 (115)
+//    160                                          512:16 93, 256:32 96 (96)                        512:16 139, 256:32 146 (152)
+//    256   256:8 95, 256:16 86 (98)               512:8 128, 512:16 95 (112)                       512:8 196, 512:16 144 (152)
+//    384   98, 102 (116)                          129, 113, 768:16 122 (133)                       199, 175, 768:16 160 (175)
+//    704   125, 134 (158)                         161, 151, 160 (182)                              240, 252, 222 (257)
+//   1024   143, 153 (181)                         200, 187, 196, 256:8 188 (223)                   290, 303, 275 (307)
+//   1536   158, 170 (209)                         233, 242, 258, 256:8 231 (260)                   383, 409, 373 (364)
+//   2048   192, 196, 128:8 180 (237)              269, 295, 316, 256:8 259 (284)                   439, 473, 469 (452)
+//   4096   0 276, 256:8 339, 256:16 323 (338)     0 436, 256:8 421, 256:16 403 (424)               0 842, 512:8 657, 512:16 670 (672)
+// 160 linedefs: 1280 lanes 0 67, 128:8 63, 1792 lanes 74, 79.  330, bricks: 2560 lanes 0 120, 128:8 116, 3072 lanes 130, 136.  700: 184, 166 and 192, 196.
+// 1400: 3072 lanes 0 237, 256:8 226, 4096 lanes 269, 291; 256 lanes 512:16 77, 512 lanes 512:8 105.  2800: 320 lanes 512:16 124, 900 lanes 206, 1792 lanes 256:8 294.
 inline int select_strips(int lanes, int linedefs) {
-    if (linedefs <= 128 || lanes >= 12 * (linedefs - 100) || (lanes >= 3584 && linedefs < 900)) return 0;
-    if (linedefs < 512) return lanes < 832 ? 768 : (lanes < 1152 ? 512 : 256);
-    if (linedefs < 1024) return lanes < 2304 ? 768 : (lanes < 2816 ? 512 : 256);
-    return lanes < 1792 ? 1024 : (lanes < 3584 ? 768 : 512);
+    if (linedefs <= 128 || (linedefs < 280 && lanes > 1536) || (linedefs < 1024 && lanes > 2816) || (linedefs < 1700 && lanes > 3072)) return 0;
+    if (linedefs < 400) return 128;
+    if (linedefs < 1024) return lanes <= 1792 ? 256 : 128;
+    if (linedefs < 3000) return lanes <= 1152 ? 512 : 256;
+    return lanes <= 1792 ? 768 : 512;
 }
 inline int select_lanes(int lanes, int linedefs) {
     const int w = linedefs < 4096 ? linedefs : 4096;      // no map of more was timed
-    if (w < 512) return 8;
-    if (lanes <= 64 + w / 24) return 32;
-    return lanes <= 128 + w / 8 || (lanes >= 1536 && w >= 1024) ? 16 : 8;
+    if (w < 400) return 8;
+    if (lanes <= 96 + w / 128) return 32;
+    if (w < 1024) return lanes <= 384 ? 16 : 8;
+    if (w < 3000) return lanes <= 1152 || lanes >= 3584 ? 16 : 8;
+    return lanes <= 1792 ? 16 : 8;
 }
 
-// wall_select_kernel: the longest strips and the others in one launch?  A launch on the side stream and back costs 8 us and more.  In larger batches
-// the others' wavefronts are so many that they hold the longest strips' up, which the side stream's start a little later do not.  A frame in
-// us, one launch / two (32 billboards, two sets of poses):
-//   lanes        320             800             1400            2000            4000          701, bricks
-//    256     335 / 342       382 / 390       454 / 463       449 / 457       653 / 661       520 / 527
-//    384     420 / 423       464 / 474       575 / 582       547 / 554       780 / 787       586 / 587
-//    512     496 / 498       552 / 562       629 / 645       639 / 643       880 / 912       669 / 670
-//    640     570 / 572       617 / 627       747 / 761       716 / 720       978 / 994       724 / 726
-//    768     642 / 643       709 / 715       857 / 873       814 / 812      1130 /1136       838 / 839
-//   1024     737 / 742       817 / 805       956 / 952       973 / 962      1345 /1342       952 / 935
-inline bool select_together(int lanes) { return lanes <= 704; }
+// wall_select_kernel: the longest strips and the others in one launch?  A launch on the side stream and back costs 20 us of the stage.  In larger batches
+// the others' wavefronts are so many that they hold the longest strips' up, which the side stream's start a little later do not.  Stage times in us, one
+// launch / two, of the strips and lanes above:
+//   lanes     320 linedefs    701, bricks    1400         2000         2800         4000
+//    768       82 / 109       124 / 151                 156 / 184                 231 / 260
+//   1536       99 / 128       145 / 179                 231 / 243                 373 / 385
+//   2048      122 / 145       170 / 206                 259 / 270                 439 / 479
+//   2560                                   204 / 241                 350 / 381    490 / 526
+//   3072                                   227 / 256                 395 / 406    577 / 571
+//   4096                                                407 / 403                 684 / 657
+inline bool select_together(int lanes) { return lanes <= 3072; }
 
 // wall_geometry_kernel: wavefronts a lane for its linedefs (a power of two).  us with 4 / 8 / 16 of them: 16 lanes 13.6 / 10.7 / 8.3, 512 lanes
 // 63 / 48 / 46, 1024 lanes 48 / 41 / 42, 4096 lanes 263 / 242 / 247.
