@@ -48,6 +48,7 @@ SYMBOLS = (
     "gd_env_check",
     "gd_fill_stacks",
     "gd_copy_pieces",
+    "gd_expand_rgb24_pieces",
 )
 
 _LIBRARY = None
@@ -130,6 +131,7 @@ def library() -> C.CDLL:
         ("gd_env_check", [C.c_void_p] * 3 + [C.c_int32, C.c_int32] + [C.c_void_p] * 2),
         ("gd_fill_stacks", [C.c_void_p] * 2 + [C.c_int32] + [C.c_void_p] * 2),
         ("gd_copy_pieces", [C.c_void_p] * 2 + [C.c_int32, C.c_int64]),
+        ("gd_expand_rgb24_pieces", [C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_int32] + [C.c_void_p] * 3),
     ):
         function = getattr(lib, name)
         function.restype, function.argtypes = C.c_int, arguments

@@ -5,11 +5,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <exception>
 #include <string>
 #include <thread>
+#include <vector>
 
 #include "../../include/gradoom_amd.h"
 #include "gd_internal.h"
@@ -226,6 +229,55 @@ int gd_copy_pieces(const void *source, void *const *targets, int32_t count, int6
     copy(0);
     for (std::thread &helper : helpers) if (helper.joinable()) helper.join();
     return GD_OK;
+}
+
+// The way of a frame over PCIe and its copy take 4.2 us each (four threads copying): one behind the other 48 frames are 0.4 ms, side by side little more than
+// half of that.  The threads are begun when the first part has come, so that they wait for the others' way only, each for the part it is at.
+int gd_expand_rgb24_pieces(const uint8_t *indexed, int32_t rows, const uint8_t *playpal, int32_t lane_count, int32_t part, uint8_t *staging, void *const *targets,
+                           void *stream) {
+    if (rows <= 0 || lane_count < 0 || part <= 0) return gd_fail(GD_E_ARG, "bad shape");
+    if (lane_count == 0) return GD_OK;
+    if (!indexed || !playpal || !staging || !targets) return gd_fail(GD_E_ARG, "null argument");
+    for (int32_t k = 0; k < lane_count; ++k) if (!targets[k]) return gd_fail(GD_E_ARG, "null target");
+    const size_t pixels = (size_t)rows * GD_SCREEN_WIDTH, bytes = pixels * 3;
+    struct Events {                       // given back whatever happens
+        std::vector<hipEvent_t> of;
+        ~Events() { for (hipEvent_t event : of) (void)hipEventDestroy(event); }
+    } events;
+    int device = 0;
+    GD_HIP_TRY(hipGetDevice(&device));
+    int status = GD_OK;
+    try {
+        events.of.reserve((size_t)(lane_count + part - 1) / (size_t)part);
+        for (int32_t first = 0; first < lane_count && status == GD_OK; first += part) {
+            const int32_t count = std::min(part, lane_count - first);
+            status = gd_expand_rgb24(indexed + (size_t)first * pixels, rows, playpal, count, staging + (size_t)first * bytes, stream);
+            hipEvent_t event = nullptr;
+            if (status == GD_OK && hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess) status = gd_fail(GD_E_HIP, "hipEventCreateWithFlags");
+            if (status == GD_OK) {
+                events.of.push_back(event);
+                if (hipEventRecord(event, static_cast<hipStream_t>(stream)) != hipSuccess) status = gd_fail(GD_E_HIP, "hipEventRecord");
+            }
+        }
+    } catch (const std::exception &) { status = gd_fail(GD_E_ARG, "out of host memory"); }
+    if (status != GD_OK) { (void)hipStreamSynchronize(static_cast<hipStream_t>(stream)); return status; }     // no frame is written into `staging` any more
+    std::atomic<bool> failed{hipEventSynchronize(events.of[0]) != hipSuccess};
+    constexpr int THREADS = 4;
+    auto copy = [&](int first) {
+        if (hipSetDevice(device) != hipSuccess) failed = true;
+        int32_t come = 0;                 // parts that have
+        for (int32_t k = first; k < lane_count; k += THREADS) {
+            for (; come <= k / part; ++come) if (hipEventSynchronize(events.of[come]) != hipSuccess) failed = true;
+            std::memcpy(targets[k], staging + (size_t)k * bytes, bytes);
+        }
+    };
+    std::thread helpers[THREADS - 1];
+    for (int t = 1; t < THREADS; ++t) {
+        try { helpers[t - 1] = std::thread(copy, t); } catch (const std::exception &) { copy(t); }   // no thread to be had
+    }
+    copy(0);
+    for (std::thread &helper : helpers) if (helper.joinable()) helper.join();
+    return failed ? gd_fail(GD_E_HIP, "hipEventSynchronize") : GD_OK;
 }
 
 }  // extern "C"

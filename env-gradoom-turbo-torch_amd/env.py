@@ -136,13 +136,20 @@ class _FramePool:
     def copies_of(self, frames: np.ndarray) -> list[np.ndarray]:
         """Every frame of a contiguous ``uint8 [N, 240, 320, 3]``, each in memory of its own."""
 
-        memories = [self._memory() for _ in range(len(frames))]
-        targets = (C.c_void_p * len(memories))(*[memory.address for memory in memories])
-        _lib.check(_lib.library().gd_copy_pieces(frames.ctypes.data, targets, len(memories), 240 * 320 * 3))
+        return self.filled_by(len(frames), lambda targets: _lib.check(_lib.library().gd_copy_pieces(frames.ctypes.data, targets, len(targets), 240 * 320 * 3)))
+
+    def filled_by(self, count: int, fill) -> list[np.ndarray]:
+        """``count`` frames in memory of their own, written by ``fill``, which is given their addresses."""
+
+        memories = [self._memory() for _ in range(count)]
+        fill((C.c_void_p * count)(*[memory.address for memory in memories]))
         return [np.asarray(self._Lent(self, memory)) for memory in memories]
 
 
 RGB_STAGING_BYTES = 64 << 20   # of frames on their way to the host: pinned, an environment; let go of, all of them together
+# Frames that are copied while others come.  get_images in us, all of them copied behind the last / 12 / 16 / 20 / 24 / 32 a part (two parts at least): 32 lanes
+# 623 / 560 / 565, 48 lanes 747 / 689 / 672 / 648 / 673, 64 lanes 888 / 779 / 771 / 787 / 737 / 780, 128 lanes 1451 / 1175 / 1168 / 1175 / 1173 / 1204.
+RGB_PART_FRAMES = 16
 _FRAMES = _FramePool(RGB_STAGING_BYTES // (240 * 320 * 3))
 
 
@@ -644,10 +651,21 @@ class GraDoomVecEnv:
         for base in range(0, count, room):
             part = min(room, count - base)
             staging = self._rgb_staging[:part]
-            render_to_host(state if part == count else state.select(slice(base, base + part)), staging)
-            self._wait()
-            frames += _FRAMES.copies_of(staging.numpy())
+            lanes = state if part == count else state.select(slice(base, base + part))
+            if part < 2 * RGB_PART_FRAMES or state.screen_blend is not None or not hasattr(self._renderer, "expand_rgb_to_pieces"):
+                render_to_host(lanes, staging)
+                self._wait()
+                frames += _FRAMES.copies_of(staging.numpy())
+            else:
+                frames += self._rgb_in_parts(lanes, staging)
         return frames
+
+    def _rgb_in_parts(self, lanes, staging: torch.Tensor) -> list[np.ndarray]:
+        """The frames of many lanes: while some are on their way over PCIe, those that have come are copied to memory of their own."""
+
+        indexed = torch.empty(tuple(staging.shape[:3]), dtype=torch.uint8, device=self.device)
+        self._renderer.render(lanes, indexed=indexed)
+        return _FRAMES.filled_by(len(staging), lambda targets: self._renderer.expand_rgb_to_pieces(indexed, staging, RGB_PART_FRAMES, targets))
 
     def render_lane(self, lane: int):  # env.py:1037-1053
         if self.closed:

@@ -335,6 +335,19 @@ class HipRenderer:
         _lib.check(self._lib.gd_render(self._handle, C.byref(desc), C.byref(out), C.c_void_p(stream)))
         del keep
 
+    def expand_rgb_to_pieces(self, indexed: torch.Tensor, rgb: torch.Tensor, part: int, targets) -> None:
+        """Frames as RGB by way of ``rgb``, a pinned host tensor ``[N, 240, 320, 3]``, to host memory of their own (``targets``, a ctypes array of
+        addresses), ``part`` of them at a time; there when the call returns."""
+
+        count = int(indexed.shape[0])
+        _require(indexed, "indexed", torch.uint8, (count, 240, 320), self.device)
+        if rgb.dtype != torch.uint8 or tuple(rgb.shape) != (count, 240, 320, 3) or not rgb.is_contiguous() or not rgb.is_pinned():
+            raise ValueError("rgb must be a contiguous pinned uint8 tensor of shape (frames, 240, 320, 3)")
+        stream = torch.cuda.current_stream(self.device).cuda_stream
+        if len(targets) != count:
+            raise ValueError("targets must hold an address per frame")
+        _lib.check(self._lib.gd_expand_rgb24_pieces(indexed.data_ptr(), 240, self.playpal.data_ptr(), count, part, rgb.data_ptr(), targets, C.c_void_p(stream)))
+
     def render_static(self, lanes: LaneState, *, indexed=None, obs=None, frames=None, reset_mask=None, rgb=None,
                       stack_only_masked: bool = False, final_frames=None, obs_source_rows: int = 208, final_layout: str = "chw") -> None:
         """``render`` through the entry point that allocates nothing (``gd_render_static``): the working memory is

@@ -654,6 +654,10 @@ int gd_fill_stacks(const uint8_t *obs, const int64_t *rows, int32_t count, uint8
 /* HOST memory: the `count` pieces of `bytes` bytes that follow each other from `source` on, each to an address of its own; done when the
    call returns.  A batch of RGB frames becomes arrays of their own this way (env.py:1058-1064 copies frame by frame). */
 int gd_copy_pieces(const void *source, void *const *targets, int32_t count, int64_t bytes);
+/* gd_expand_rgb24 of `lane_count` frames into pinned HOST memory `staging`, and every frame from there to an address of its own in HOST memory; done
+   when the call returns.  `part` frames at a time: those that have come are copied while others are on their way. */
+int gd_expand_rgb24_pieces(const uint8_t *indexed, int32_t rows, const uint8_t *playpal, int32_t lane_count, int32_t part, uint8_t *staging,
+                           void *const *targets, void *stream);
 
 /*
  * Time `launches` back-to-back gd_render launches with HIP events on `stream`

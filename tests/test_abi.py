@@ -198,3 +198,9 @@ def test_pieces_of_host_memory_each_land_at_their_own_address(count, size):
                 (source.ctypes.data, (ctypes.c_void_p * 1)(None), 1, size)):
         with pytest.raises(ValueError):
             _lib.check(_lib.library().gd_copy_pieces(*bad))
+    frame, pixels = source.ctypes.data, 16
+    for bad in ((frame, 0, frame, 1, 1, frame, addresses, None), (frame, pixels, frame, -1, 1, frame, addresses, None), (frame, pixels, frame, 1, 0, frame, addresses, None),
+                (None, pixels, frame, 1, 1, frame, addresses, None), (frame, pixels, None, 1, 1, frame, addresses, None), (frame, pixels, frame, 1, 1, None, addresses, None),
+                (frame, pixels, frame, 1, 1, frame, None, None), (frame, pixels, frame, 1, 1, frame, (ctypes.c_void_p * 1)(None), None)):
+        with pytest.raises(ValueError):
+            _lib.check(_lib.library().gd_expand_rgb24_pieces(*bad))

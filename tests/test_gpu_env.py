@@ -282,6 +282,24 @@ def test_a_reset_device_or_a_renderer_of_the_users_own_is_the_one_that_resets(ho
         each.close()
 
 
+@pytest.mark.parametrize("lanes, room", [(31, 64), (32, 64), (33, 64), (70, 48)])   # fewer than two parts, two, a part of one frame, memory for three parts
+def test_rgb_frames_of_many_lanes_come_in_parts(monkeypatch, lanes, room):
+    from gradoom_amd.env import GraDoomVecEnv, RGB_PART_FRAMES
+
+    assert RGB_PART_FRAMES == 16
+    monkeypatch.setattr(GraDoomVecEnv, "RGB_STAGING_BYTES", room * 240 * 320 * 3)
+    _meta, _data, smap, _tables = load_fixture("tiny_stages")
+    env = GraDoomVecEnv(smap, lanes, device="cuda:0", render_mode="rgb_array")
+    seeds = torch.arange(lanes, device="cuda:0")
+    for shift in (0, 7):       # the second time over what the first left
+        env.reset_device(torch.ones(lanes, dtype=torch.bool, device="cuda:0"), seeds + shift)
+        rgb = torch.zeros((lanes, 240, 320, 3), dtype=torch.uint8, device="cuda:0")
+        env._renderer.render(env._dynamics.lane_state(), rgb=rgb)
+        frames = env.get_images()
+        assert len(frames) == lanes and np.array_equal(np.stack(frames), rgb.cpu().numpy())
+    env.close()
+
+
 @pytest.mark.parametrize("room", [1, 2, 64])   # frames that the pinned staging memory holds
 def test_rgb_frames_are_arrays_of_their_own(monkeypatch, room):
     from gradoom_amd.env import GraDoomVecEnv
