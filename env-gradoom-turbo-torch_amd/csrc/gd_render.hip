@@ -1709,17 +1709,23 @@ struct TexLds { unsigned char bits[LDS_TEXTURES]; unsigned int odd[LDS_TEXTURES 
 __device__ __forceinline__ void stage_tables(const gd_map_desc *m, float4 *sector_lds, TexLds *tex_lds, Tables &tb) {
     int sectors = m->sector_count < LDS_SECTORS ? m->sector_count : LDS_SECTORS;
     int textures = m->texture_count < LDS_TEXTURES ? m->texture_count : LDS_TEXTURES;
+#pragma unroll 4
     for (int s = threadIdx.x; s < sectors; s += blockDim.x) {
         float4 v;
         v.x = m->sector_heights[2 * s]; v.y = m->sector_heights[2 * s + 1]; v.z = m->sector_lights[s];
         v.w = __uint_as_float(((unsigned)m->sector_floor_tex[s] & 0xFFFFu) | ((unsigned)m->sector_ceil_tex[s] << 16));
         sector_lds[s] = v;
     }
-    for (int t = threadIdx.x; t < textures; t += blockDim.x) tex_lds->bits[t] = (unsigned char)(ilog2(m->tex_w[t]) | (ilog2(m->tex_h[t]) << 4));
-    for (int k = threadIdx.x; k < LDS_TEXTURES / 32; k += blockDim.x) {
-        unsigned int odd = 0;
-        for (int t = 32 * k; t < 32 * k + 32 && t < textures; ++t) odd |= (m->tex_w[t] & (m->tex_w[t] - 1)) ? 1u << (t & 31) : 0u;
-        tex_lds->odd[k] = odd;
+    // Whole wavefronts, a texture a lane.  With a thread that went over a word's textures by itself every work-group of wall_raster_kernel began with 32 loads one
+    // after the other (and the colormap four bytes at a time); wall_geometry_kernel and it together, then / now: 16 lanes on the 2000-linedef map 80 / 75 us, 256
+    // 139 / 130, 2048 lanes on the 320-linedef map 354 / 291, 4096 on the 4000-linedef map 1208 / 1140.
+    for (int first = threadIdx.x & ~63; first < LDS_TEXTURES; first += blockDim.x) {
+        const int lane = threadIdx.x & 63, t = first + lane;
+        const bool there = t < textures;
+        const int width = there ? m->tex_w[t] : 1, height = there ? m->tex_h[t] : 1;
+        if (there) tex_lds->bits[t] = (unsigned char)(ilog2(width) | (ilog2(height) << 4));
+        const u64 odd = __ballot((width & (width - 1)) != 0);
+        if (lane < 2 && first / 32 + lane < LDS_TEXTURES / 32) tex_lds->odd[first / 32 + lane] = (unsigned int)(odd >> (32 * lane));
     }
     tb.m = m; tb.sector = sector_lds; tb.tex_bits = tex_lds->bits; tb.tex_odd = tex_lds->odd; tb.sector_cached = sectors; tb.tex_cached = textures;
 }
@@ -4015,6 +4021,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LANES =
 // those tables, 16.7 KB, are held once per group rather than once per wavefront (a CU has 160 KB of LDS and room for
 // sixteen of these wavefronts at 128 registers).  After the staging barrier the wavefronts never meet again.
 #define WALL_STRIPS_PER_GROUP 2
+static_assert(32 * 256 / 16 % (64 * WALL_STRIPS_PER_GROUP) == 0, "wall_raster_kernel: the colormap's rows in whole turns");
 #define RASTER_WAVES 4
 // The pass that the lane `k` of each column's PARTS lanes prepared, for all of them.
 template <int PARTS>
@@ -4043,7 +4050,7 @@ template <bool DEPTH, bool GENERAL, int PARTS>
 __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amdgpu_waves_per_eu(RASTER_WAVES, RASTER_WAVES))) wall_raster_kernel(DeviceMap dm, int lane_count, Scratch sc, unsigned char *frame_base, size_t frame_stride) {
     const gd_map_desc *m = &dm.d;
     __shared__ LaneCtx lane_ctxs[WALL_STRIPS_PER_GROUP][64 / SEG_COLS];
-    __shared__ unsigned char colormap_lds[32 * 256];   // shade rows 0..31 are the only ones indexed
+    __shared__ __align__(16) unsigned char colormap_lds[32 * 256];   // shade rows 0..31 are the only ones indexed
     __shared__ float4 sector_lds[LDS_SECTORS];
     __shared__ TexLds tex_lds;
     const int wave_in_group = threadIdx.x >> 6;
@@ -4059,7 +4066,8 @@ __global__ void __launch_bounds__(64 * WALL_STRIPS_PER_GROUP) __attribute__((amd
     stage_tables(m, sector_lds, &tex_lds, tb);
     tb.all_cached = !GENERAL;
     if ((lane_id & (SEG_COLS - 1)) == 0 && live) lane_ctxs[wave_in_group][segment_in_wave] = sc.ctx[local];
-    for (int k = threadIdx.x; k < 32 * 256 / 4; k += blockDim.x) reinterpret_cast<unsigned int *>(colormap_lds)[k] = reinterpret_cast<const unsigned int *>(m->colormap)[k];
+#pragma unroll
+    for (int k = 0; k < 32 * 256 / 16; k += 64 * WALL_STRIPS_PER_GROUP) reinterpret_cast<uint4 *>(colormap_lds)[k + threadIdx.x] = reinterpret_cast<const uint4 *>(m->colormap)[k + threadIdx.x];
     __syncthreads();
     if (!live) return;   // whole segments: the groups of four columns that exchange values below live or leave together
     const LaneCtx &lane_ctx = lane_ctxs[wave_in_group][segment_in_wave];
