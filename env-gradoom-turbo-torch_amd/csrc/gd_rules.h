@@ -72,24 +72,25 @@ inline int geometry_parts(int lanes) { return lanes >= 1024 ? 8 : 16; }
 // long as its longest strips, shares a strip out over eight wavefronts, a larger one over four, over two.  The wavefront's columns then have
 // eight, four or two lanes each: these prepare as many passes at once and share every run of rows out, so that both the chain of waits and
 // the vector instructions of a column shrink with them (when the spare lanes stood idle, eight wavefronts never paid).  What a strip more
-// wavefronts costs is room on the SIMDs.  Stage times in us (wall_geometry_kernel among them) for 1 / 2 / 4 / 8 wavefronts a
-// strip, in brackets with idle lanes and the lines of then (four up to 560 lanes, two up to 1344):
-//   lanes           320 linedefs                     2000                             4000                             701, bricks
-//      16         / 90 / 72 / 65 (106)            / 136 / 110 / 97 (155)           / 184 / 149 / 139 (196)          / 263 / 218 / 188 (285)
-//     256        / 142 / 119 / 113 (155)         / 198 / 161 / 145 (212)          / 328 / 259 / 229 (327)          / 291 / 238 / 208 (310)
-//     384        / 148 / 121 / 136 (174)         / 206 / 175 / 170 (229)          / 349 / 276 / 274 (345)          / 298 / 247 / 219 (322)
-//     512        / 156 / 126 / 175 (202)         / 219 / 189 / 222 (250)          / 425 / 401 / 367 (480)          / 313 / 256 / 249 (318)
-//     640        / 165 / 156 / 222 (202)         / 233 / 204 / 279 (277)          / 432 / 416 / 394 (498)          / 346 / 273 / 309 (408)
-//     768     235 / 173 / 187 / 270 (214)     328 / 239 / 236 / 333 (282)      527 / 445 / 422 / 457 (513)      430 / 345 / 283 / 371 (415)
-//    1024     253 / 204 / 233 / 351 (249)     385 / 270 / 303 / 437 (330)      555 / 466 / 445 / 598 (539)      449 / 354 / 334 / 487 (431)
-//    1536     294 / 287 / 342 (298)           438 / 383 / 440 (448)            597 / 528 / 630 (619)            479 / 392 / 490 (501)
-//    2048     365 / 357 / 450 (364)           492 / 478 / 583 (487)            701 / 674 / 835 (695)            524 / 509 / 643 (536)
-//    2560     439 / 425 (440)                 596 / 589 (583)                  831 / 845 (820)                  639 / 625 (649)
-//    3072     519 / 542 (514)                 700 / 722 (683)                  930 / 969 (918)                  751 / 744 (753)
-// With one lane a column nothing is shared, and the stage takes up to 1.7 % longer than before columns could share: on one card at 4096 lanes 679 -> 684,
-// 886 -> 901, 1229 -> 1238 and 971 -> 974 us.  (A prepared pass's flags and rows kept in registers of their own there, not packed into words,
-// issue 1.5 % fewer instructions and take as long: 686, 905, 1239, 975.)
-inline int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 2400 ? 2 : 1)); }
+// wavefronts costs is room on the SIMDs.  Stage times in us (wall_geometry_kernel among them) for 1 / 2 / 4 / 8 wavefronts a strip:
+//   lanes           320 linedefs              701, bricks                 2000                      4000
+//     256           / 103 / 93                / 231 / 199               / 142 / 130               / 225 / 219
+//     336           / 104 / 99                / 242 / 202               / 162 / 155               / 255 / 244
+//     384           / 105 / 111               / 243 / 207               / 163 / 160               / 260 / 258
+//     512       143 / 111 / 142           283 / 251 / 229           208 / 177 / 189           309 / 271 / 289
+//     704       150 / 139 / 194           293 / 261 / 280           220 / 191 / 257           345 / 316 / 370
+//     768       152 / 151 / 213           293 / 265 / 306           223 / 204 / 277           353 / 324 / 394
+//    1024       170 / 193                 308 / 290                 246 / 264                 409 / 400
+//    1536  263 / 243 / 280           455 / 364 / 417           399 / 338 / 385           569 / 494 / 563
+//    2048  336 / 317                 493 / 462                 462 / 438                 647 / 630
+//    3072  482 / 467                 692 / 683                 647 / 635                 888 / 887
+//    4096  636 / 619                 904 / 902                 842 / 831                1162 /1169
+// Between 704 and 1024 lanes four and two change places at 600 lanes (200 linedefs) to 1024 (4000), between 336 and 512 eight and four at 336 (200) to 512
+// (701 bricks); from 3328 lanes on one is as good as two on the 1400-linedef map and 1 % better on the 4000-linedef map, the headline's.  (Before a
+// work-group staged its tables with all of its lanes one was the better from 2400 lanes on: 2 / 1 took 761 / 735 us on the 4000-linedef map, 716 / 731 now.)
+// With one lane a column nothing is shared.  (A prepared pass's flags and rows kept in registers of their own there, not packed into words,
+// issue 1.5 % fewer instructions and take as long.)
+inline int raster_parts(int lanes) { return lanes <= 336 ? 8 : (lanes <= 704 ? 4 : (lanes <= 3328 ? 2 : 1)); }
 
 // The smallest batches, whose strips leave most of the chip idle even so: sixteen wavefronts a strip, of four columns (as many as decide on a shared
 // group of rows together) with sixteen lanes each.  A frame in us, sixteen / eight (32 billboards, two sets of poses):
