@@ -187,6 +187,9 @@ struct __align__(16) WallSide {
 // (and the neighbours' ray tests asked for one after the other, a bridge's linedefs by number and then by sectors, linedef 0 again in every pass that finds
 // none) the launch for the longest strips takes 385 us instead of 433 at 4096 lanes of the 4000-linedef map, the other 788 instead of 800; 1024 lanes of the
 // 2000-linedef map 232 instead of 248 and 191 instead of 202.
+// A choice between two of its members is made between their values: written between the members themselves it is one between addresses, which kept the record in
+// private memory, written and read back in every pass.  The stage at 4096 lanes of the 4000-linedef map 643 us that way, 577 now; 2048 lanes 445, 422; 256 lanes 147, 125;
+// 1024 of the 2000-linedef map 192, 175.
 struct __align__(16) WallLinks {
     unsigned sectors;        // front | back << 16 (0xFFFF: none)
     unsigned vertices;       // start | end << 16
@@ -2448,7 +2451,8 @@ __device__ __forceinline__ void endpoint_owner(const ColumnCtx &cc, int w, const
         int ss = links.slots & 0xFF, es = (links.slots >> 8) & 0xFF; bool hs = (links.slots >> 16) & 1, he = (links.slots >> 17) & 1;
         int rslot = uses_start ? ss : es, oslot = uses_start ? es : ss;
         bool rexists = uses_start ? hs : he, oexists = uses_start ? he : hs;
-        int rn = uses_start ? links.neighbour[0] : links.neighbour[1], on = uses_start ? links.neighbour[1] : links.neighbour[0];
+        const int at_start = links.neighbour[0], at_end = links.neighbour[1];      // values: see WallLinks
+        int rn = uses_start ? at_start : at_end, on = uses_start ? at_end : at_start;
         Eval r = cc.eval(rn);
         bool r_owns = rexists && (r.flags & CF_PROJ) && (r.flags & CF_LEDGE);
         index = rn; found = r; valid = r_owns;
@@ -2805,7 +2809,8 @@ __device__ __forceinline__ void pass_select(const ColumnCtx &cc, ListShare<LANES
         solid.share();
         psd = solid.distance(); psi = solid.wall(); psi_flags = solid.flags();
         if (sel_excl_right) {
-            const int *idx = (sel_start ? m->solid_bridge_start_idx : m->solid_bridge_end_idx) + links.solid[sel_start ? 0 : 1];
+            const int by_start = links.solid[0], by_end = links.solid[1];      // values: see WallLinks
+            const int *idx = (sel_start ? m->solid_bridge_start_idx : m->solid_bridge_end_idx) + (sel_start ? by_start : by_end);
             const int bridges = sel_start ? links.solid_counts & 0xFFFFu : links.solid_counts >> 16;
             float sbd = GD_INF; int sbi = 0; int sbi_flags = 0;
             for (int k = 0; k < bridges; ++k) {
