@@ -1,5 +1,5 @@
-// A sorting network for a thread's registers: K. E. Batcher, "Sorting networks and their applications" (1968), the merge of odd and even places.
-// Host code as well, which the tests compile.
+// A sorting network for a thread's registers: K. E. Batcher, "Sorting networks and their applications" (1968), the merge of odd and even places; and the walk
+// over what it ordered.  Host code as well, which the tests compile.
 #ifndef GD_ORDER_H
 #define GD_ORDER_H
 
@@ -54,6 +54,31 @@ template <int COUNT> GD_ORDER_FN void order_merge_lowest(double (&v)[COUNT], con
 #pragma unroll
         for (int k = 0; k < COUNT; ++k)
             if (!(k & step)) order_two(v[k], v[k + step]);
+}
+
+// Rows `from` .. `held` of an ordered window, some at a time, until the last of them is farther than enough(): true if it came to that, so that what lies beyond
+// the window is farther still.  row(k) gives a row, which has a distance; look() is asked about every one and told whether it is there.  Rows from `held` on are
+// read with the last ones and hold anything: they neither end a walk nor keep it from ending.  ADVANCE: `from` moves past those leading ones that are no
+// farther than `passed`.
+#define WINDOW_WALK_ROWS 4
+template <bool ADVANCE, typename Row, typename Look, typename Enough>
+GD_ORDER_FN bool window_walk(int &from, int held, float passed, Row row, Look look, Enough enough) {
+    bool leading = true, more = true;
+    for (int k = from; k < held && more; k += WINDOW_WALK_ROWS) {
+        decltype(row(0)) rows[WINDOW_WALK_ROWS];
+#pragma unroll
+        for (int j = 0; j < WINDOW_WALK_ROWS; ++j) rows[j] = row(k + j);
+        float last = rows[0].dist;
+#pragma unroll
+        for (int j = 0; j < WINDOW_WALK_ROWS; ++j) {
+            const bool there = k + j < held;
+            if (ADVANCE) { leading = leading && there && !(rows[j].dist > passed); from += leading ? 1 : 0; }
+            last = there ? rows[j].dist : last;
+            look(rows[j], there);
+        }
+        more = !(last > enough());
+    }
+    return !more;
 }
 
 #endif

@@ -2176,7 +2176,7 @@ template <> struct NearestOf<1> {
 #define WINDOW 12
 #define WINDOW_REFILL 5
 #define WINDOW_BATCH 16        // entries ordered at a time
-#define WINDOW_PAD 3           // rows read with the last ones and not looked at
+#define WINDOW_PAD (WINDOW_WALK_ROWS - 1)   // rows read with the last ones: words of other lanes, which window_walk says are not there
 template <> struct ListShare<1> {
     static constexpr int WORDS = (WINDOW * 3 + WINDOW_PAD) * 64;
     u64 *keys;                  // this lane's word of [WINDOW][64]
@@ -2257,22 +2257,9 @@ template <> struct ListShare<1> {
     // The entries beyond `passed` (and some that are not, and some twice), nearest first as far as the window goes, until those left are
     // farther than enough().
     template <bool ADVANCE, typename Look, typename Enough> __device__ __forceinline__ void walk(const ColumnCtx &cc, Look look, Enough enough) {
-        bool leading = true, more = true;
-        for (int k = from; k < held && more;) {
-            u64 key[4]; unsigned pair[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) { key[j] = keys[(k + j) * 64]; pair[j] = sectors[(k + j) * 64]; }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const Cand q = key_cand(key[j]);
-                const bool there = k + j < held;
-                if (ADVANCE) { leading = leading && there && !(q.dist > passed); from += leading ? 1 : 0; }
-                look(ListEntry{q.flags, q.wall, q.dist, pair[j], 0u}, there);
-            }
-            k += 4;
-            more = !(cand_key_distance(key[3]) > enough());
-        }
-        if (complete || !more) return;
+        auto row = [&](int k) { const Cand q = key_cand(keys[k * 64]); return ListEntry{q.flags, q.wall, q.dist, sectors[k * 64], 0u}; };
+        const bool ended = window_walk<ADVANCE>(from, held, passed, row, look, enough);
+        if (complete || ended) return;
         for (int k0 = 0; k0 < cc.count; k0 += 4) {
             u64 key[4]; unsigned pair[4];
 #pragma unroll

@@ -1,5 +1,5 @@
-"""The sorting networks that order the nearest entries of a column's list (``csrc/gd_order.h``), compiled for the host; and columns with lists of one to six
-such windows, drawn with a lane a column, against the CPU oracle."""
+"""The sorting networks that order the nearest entries of a column's list and the walk over them (``csrc/gd_order.h``), compiled for the host; and columns with
+lists of one to six such windows, drawn with a lane a column, against the CPU oracle."""
 
 from __future__ import annotations
 
@@ -19,13 +19,25 @@ extern "C" void order_numbers(double *v) { order_up(*reinterpret_cast<double (*)
 extern "C" void lowest_of(double *v, double *other) {
     order_merge_lowest(*reinterpret_cast<double (*)[16]>(v), *reinterpret_cast<double (*)[16]>(other));
 }
+// a walk over distances: which rows were looked at as there, where `from` went, whether it ended
+struct Entry { float dist; int at; };
+extern "C" int walk(const float *rows, int count, int *from, int held, float passed, float limit, int advance, int *looked) {
+    auto row = [&](int k) { if (k >= count) __builtin_trap(); return Entry{rows[k], k}; };
+    auto look = [&](const Entry &e, bool there) { looked[e.at] += there ? 1 : 0; };
+    auto enough = [&]() { return limit; };
+    return advance ? window_walk<true>(*from, held, passed, row, look, enough) : window_walk<false>(*from, held, passed, row, look, enough);
+}
 """
 
 
-def test_the_networks_order_numbers(tmp_path):
-    path = str(tmp_path / "liborder.so")
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("order") / "liborder.so")
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-Wno-unknown-pragmas", "-I", CSRC, "-x", "c++", "-o", path, "-"], input=DRIVER, text=True, check=True)
-    library = C.CDLL(path)
+    return C.CDLL(path)
+
+
+def test_the_networks_order_numbers(library):
     pointer = lambda values: values.ctypes.data_as(C.c_void_p)  # noqa: E731
     for bits in range(1 << 16):              # zeros and ones: what a network orders of these it orders of all numbers
         row = np.array([bits >> k & 1 for k in range(16)], dtype=np.float64)
@@ -42,6 +54,28 @@ def test_the_networks_order_numbers(tmp_path):
         lowest = np.sort(np.concatenate(runs))[:16]
         library.lowest_of(pointer(runs[0]), pointer(runs[1]))
         assert np.array_equal(runs[0], lowest)
+
+
+@pytest.mark.parametrize("stray", [np.float32(np.inf), np.float32(1e30), np.float32(1e-38), np.float32(np.nan), np.float32(0.0)])
+@pytest.mark.parametrize("advance", [0, 1])
+def test_a_walk_ends_by_the_windows_entries_alone(library, advance, stray):
+    """Twelve rows hold distances 1, 2, ..; the three behind them, words of other lanes, hold ``stray``."""
+    library.walk.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_float, C.c_float, C.c_int, C.c_void_p]
+    for held in range(13):
+        rows = np.full(15, stray, dtype=np.float32)
+        rows[:held] = np.arange(1, held + 1)
+        for first in range(held + 1):
+            for passed in range(first, held + 1):        # entries before `first` are no farther than `passed`
+                for limit in np.arange(first, held + 1.5, 0.5):
+                    at, looked = np.array([first], dtype=np.int32), np.zeros(15, dtype=np.int32)
+                    ended = library.walk(rows.ctypes.data, 15, at.ctypes.data, held, float(passed), float(limit), advance, looked.ctypes.data)
+                    # what is left beyond a walk that ended is farther than the limit, and it ends wherever the window's last entry is
+                    assert ended == (first < held and held > limit), (held, first, passed, limit)
+                    assert np.all(looked <= 1) and not looked[held:].any() and not looked[:first].any()
+                    assert looked[first:held].all() if not ended else looked[first:min(held, int(limit))].all()
+                    assert first <= at[0] <= passed and (at[0] == first or advance)
+                    if advance and not ended:
+                        assert at[0] == passed
 
 
 @pytest.mark.gpu
