@@ -83,6 +83,12 @@ def _kernel_ready(tensor, dtype, count: int, device) -> bool:
     return isinstance(tensor, torch.Tensor) and tensor.dtype is dtype and tensor.shape == (count,) and tensor.device == device and tensor.is_contiguous()
 
 
+def _own(method, function) -> bool:
+    """Is this bound method the package's ``function``, and no other put in its place?"""
+
+    return getattr(method, "__func__", None) is function
+
+
 class _FramePool:
     """Host memory of RGB frames that their holders have let go of, for the next frames: at most ``limit`` frames of it.
 
@@ -403,8 +409,7 @@ class GraDoomVecEnv:
         is asked for the frames of all lanes with a reset mask, as its interface has it.
         """
 
-        own = lambda method, function: getattr(method, "__func__", None) is function  # noqa: E731
-        return own(self.reset_device, GraDoomVecEnv.reset_device) and own(getattr(self._renderer, "render", None), HipRenderer.render)
+        return _own(self.reset_device, GraDoomVecEnv.reset_device) and _own(getattr(self._renderer, "render", None), HipRenderer.render)
 
     def _lane_rows(self, rows: torch.Tensor) -> LaneState:
         """The lane state of some lanes.  A dynamics object owes ``lane_state()`` and no more; the pool's own also takes the lanes."""
@@ -647,17 +652,19 @@ class GraDoomVecEnv:
         room = max(1, min(count, self.RGB_STAGING_BYTES // frame_bytes))
         if self._rgb_staging is None or self._rgb_staging.shape[0] < room:
             self._rgb_staging = torch.empty((room, 240, 320, 3), dtype=torch.uint8, pin_memory=True)
+        # By parts only where `render_rgb_to_host`, which is asked otherwise, and `render` are this package's.
+        by_parts = state.screen_blend is None and _own(render_to_host, HipRenderer.render_rgb_to_host) and _own(getattr(self._renderer, "render", None), HipRenderer.render)
         frames = []
         for base in range(0, count, room):
             part = min(room, count - base)
             staging = self._rgb_staging[:part]
             lanes = state if part == count else state.select(slice(base, base + part))
-            if part < 2 * RGB_PART_FRAMES or state.screen_blend is not None or not hasattr(self._renderer, "expand_rgb_to_pieces"):
+            if by_parts and part >= 2 * RGB_PART_FRAMES:
+                frames += self._rgb_in_parts(lanes, staging)
+            else:
                 render_to_host(lanes, staging)
                 self._wait()
                 frames += _FRAMES.copies_of(staging.numpy())
-            else:
-                frames += self._rgb_in_parts(lanes, staging)
         return frames
 
     def _rgb_in_parts(self, lanes, staging: torch.Tensor) -> list[np.ndarray]:

@@ -300,6 +300,41 @@ def test_rgb_frames_of_many_lanes_come_in_parts(monkeypatch, lanes, room):
     env.close()
 
 
+@pytest.mark.parametrize("where", ["class", "object"])
+@pytest.mark.parametrize("lanes", [31, 32])   # fewer than two parts, two
+def test_a_renderer_that_writes_rgb_frames_in_its_own_way_is_asked_for_them(lanes, where):
+    from gradoom_amd.env import GraDoomVecEnv
+    from gradoom_amd.renderer import HipRenderer
+
+    class Marking(HipRenderer):
+        def render_rgb_to_host(self, state, rgb):
+            HipRenderer.render_rgb_to_host(self, state, rgb)
+            torch.cuda.current_stream(self.device).synchronize()
+            rgb[:, :8, :8] = 255
+
+    class Refusing(HipRenderer):    # RGB frames never were a matter of render()
+        def render(self, state, **out):
+            assert "indexed" not in out
+            HipRenderer.render(self, state, **out)
+
+    _meta, _data, smap, _tables = load_fixture("tiny_stages")
+    reset = torch.ones(lanes, dtype=torch.bool, device="cuda:0"), torch.arange(lanes, device="cuda:0")
+    taken = []
+    for kind in (HipRenderer, Marking, Refusing):
+        renderer = (kind if where == "class" else HipRenderer)(smap, lanes, "cuda:0")
+        if where == "object" and kind is not HipRenderer:
+            name = "render_rgb_to_host" if kind is Marking else "render"
+            setattr(renderer, name, getattr(kind, name).__get__(renderer))
+        env = GraDoomVecEnv(smap, lanes, device="cuda:0", render_mode="rgb_array", renderer=renderer)
+        env.reset_device(*reset)
+        taken.append(np.stack(env.get_images()))
+        env.close()
+    plain, marked, refused = taken
+    assert np.array_equal(plain, refused)
+    plain[:, :8, :8] = 255
+    assert np.array_equal(plain, marked)
+
+
 @pytest.mark.parametrize("room", [1, 2, 64])   # frames that the pinned staging memory holds
 def test_rgb_frames_are_arrays_of_their_own(monkeypatch, room):
     from gradoom_amd.env import GraDoomVecEnv
