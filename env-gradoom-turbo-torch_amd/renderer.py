@@ -339,6 +339,8 @@ class HipRenderer:
         """Frames as RGB by way of ``rgb``, a pinned host tensor ``[N, 240, 320, 3]``, to host memory of their own (``targets``, a ctypes array of
         addresses), ``part`` of them at a time; there when the call returns."""
 
+        if self._handle is None:
+            raise RuntimeError("renderer is closed")
         count = int(indexed.shape[0])
         _require(indexed, "indexed", torch.uint8, (count, 240, 320), self.device)
         if rgb.dtype != torch.uint8 or tuple(rgb.shape) != (count, 240, 320, 3) or not rgb.is_contiguous() or not rgb.is_pinned():
@@ -346,7 +348,8 @@ class HipRenderer:
         stream = torch.cuda.current_stream(self.device).cuda_stream
         if len(targets) != count:
             raise ValueError("targets must hold an address per frame")
-        _lib.check(self._lib.gd_expand_rgb24_pieces(indexed.data_ptr(), 240, self.playpal.data_ptr(), count, part, rgb.data_ptr(), targets, C.c_void_p(stream)))
+        with torch.cuda.device(self.device):    # its events are the current device's, and recorded on this renderer's stream
+            _lib.check(self._lib.gd_expand_rgb24_pieces(indexed.data_ptr(), 240, self.playpal.data_ptr(), count, part, rgb.data_ptr(), targets, C.c_void_p(stream)))
 
     def render_static(self, lanes: LaneState, *, indexed=None, obs=None, frames=None, reset_mask=None, rgb=None,
                       stack_only_masked: bool = False, final_frames=None, obs_source_rows: int = 208, final_layout: str = "chw") -> None:

@@ -418,3 +418,42 @@ def test_an_environment_that_is_closed_leaves_the_frame_pool(env):
     assert module._FRAMES._users == users - 1
     env.close()
     assert module._FRAMES._users == users - 1
+
+
+def test_frames_by_parts_are_expanded_under_the_renderers_device(monkeypatch):
+    """With stand-ins for the library and the devices: the call is made with the renderer's device current, and not at all once the renderer is closed."""
+
+    import ctypes
+    from types import SimpleNamespace
+
+    from gradoom_amd.renderer import HipRenderer
+
+    current, calls = [], []
+
+    class Device:
+        def __init__(self, device):
+            self.device = device
+
+        def __enter__(self):
+            current.append(self.device)
+
+        def __exit__(self, *_):
+            current.pop()
+
+    class Pinned:
+        dtype, shape = torch.uint8, (2, 240, 320, 3)
+        is_contiguous = is_pinned = lambda self: True  # noqa: E731
+        data_ptr = lambda self: 1  # noqa: E731
+
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=7))
+    renderer = HipRenderer.__new__(HipRenderer)
+    renderer.device, renderer.playpal, renderer._handle = torch.device("cpu"), torch.zeros(768, dtype=torch.uint8), 1
+    renderer._lib = SimpleNamespace(gd_expand_rgb24_pieces=lambda *_: calls.append(list(current)) or 0)
+    frames, targets = torch.zeros((2, 240, 320), dtype=torch.uint8), (ctypes.c_void_p * 2)(1, 1)
+    renderer.expand_rgb_to_pieces(frames, Pinned(), 1, targets)
+    assert calls == [[torch.device("cpu")]] and current == []
+    renderer._handle = None
+    with pytest.raises(RuntimeError, match="renderer is closed"):
+        renderer.expand_rgb_to_pieces(frames, Pinned(), 1, targets)
+    assert len(calls) == 1
