@@ -239,6 +239,7 @@ int gd_expand_rgb24_pieces(const uint8_t *indexed, int32_t rows, const uint8_t *
     if (lane_count == 0) return GD_OK;
     if (!indexed || !playpal || !staging || !targets) return gd_fail(GD_E_ARG, "null argument");
     for (int32_t k = 0; k < lane_count; ++k) if (!targets[k]) return gd_fail(GD_E_ARG, "null target");
+    part = std::min(part, lane_count);    // any number above stands for all of them
     const size_t pixels = (size_t)rows * GD_SCREEN_WIDTH, bytes = pixels * 3;
     struct Events {                       // given back whatever happens
         std::vector<hipEvent_t> of;
@@ -248,7 +249,7 @@ int gd_expand_rgb24_pieces(const uint8_t *indexed, int32_t rows, const uint8_t *
     GD_HIP_TRY(hipGetDevice(&device));
     int status = GD_OK;
     try {
-        events.of.reserve((size_t)(lane_count + part - 1) / (size_t)part);
+        events.of.reserve((size_t)((lane_count - 1) / part + 1));
         for (int32_t first = 0; first < lane_count && status == GD_OK; first += part) {
             const int32_t count = std::min(part, lane_count - first);
             status = gd_expand_rgb24(indexed + (size_t)first * pixels, rows, playpal, count, staging + (size_t)first * bytes, stream);

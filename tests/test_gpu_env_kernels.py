@@ -78,6 +78,22 @@ def test_rgb_expansion_in_device_and_pinned_memory(lanes, rows):
     renderer.close()
 
 
+@pytest.mark.parametrize("part", [1, 2, 4, 5, 6, 2**31 - 1])   # five frames; the last stands for any number beyond them
+def test_rgb_frames_by_parts_of_any_size(part):
+    import ctypes
+
+    from gradoom_amd.renderer import HipRenderer
+
+    _meta, _data, smap, tables = load_fixture("tiny_stages")
+    renderer = HipRenderer(smap, 1, "cuda:0", tables=tables)
+    indexed = torch.randint(0, 256, (5, 240, 320), generator=torch.Generator(device="cuda:0").manual_seed(part), device="cuda:0", dtype=torch.uint8)
+    staging, frames = torch.zeros((5, 240, 320, 3), dtype=torch.uint8, pin_memory=True), np.zeros((5, 240, 320, 3), dtype=np.uint8)
+    print(f"parts of {part}", flush=True)
+    renderer.expand_rgb_to_pieces(indexed, staging, part, (ctypes.c_void_p * 5)(*[frame.ctypes.data for frame in frames]))
+    assert np.array_equal(frames, np.asarray(tables["playpal"])[indexed.cpu().numpy()])
+    renderer.close()
+
+
 @pytest.mark.parametrize("form", ["int64", "int32", "strided", "two_dimensions", "list", "negative", "none"])
 def test_the_lanes_asked_of_a_pose_pool_may_come_in_any_form(form):
     """A kernel reads int64 rows of one contiguous piece; whatever else is handed in goes the way of the Torch expressions."""
