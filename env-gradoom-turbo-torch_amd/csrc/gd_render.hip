@@ -6529,8 +6529,6 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
     UP(side_tex, W * 6); UP(side_off, W * 4); UP(wall_len, W);
     UP(endpoint_neighbors, W * K); UP(endpoint_neighbor_starts, W * K); UP(endpoint_neighbor_ends, W * K);
     UP(direct_neighbor_table, W * 4);
-    UP(solid_bridge_start_ofs, W + 1); UP(solid_bridge_start_idx, h->solid_bridge_start_ofs[W]);
-    UP(solid_bridge_end_ofs, W + 1); UP(solid_bridge_end_idx, h->solid_bridge_end_ofs[W]);
     UP(vertex_wall_ofs, V + 1); UP(vertex_wall_idx, h->vertex_wall_ofs[V]);
     UP(sector_wall_ofs, S + 1); UP(sector_wall_idx, h->sector_wall_ofs[S]);
     UP(sector_edge_ofs, S + 1); UP(sector_edge_idx, h->sector_edge_ofs[S]);
@@ -6603,15 +6601,35 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
             if ((facts[w] >> WALL_BLOCKING_SHIFT) == 0) facts[w] |= (b + 1) << WALL_BLOCKING_SHIFT;   // the first slot wins ties, like the scan it replaces
         }
         if (rc == GD_OK) rc = upload(r, facts.data(), facts.size(), &r->dm.wall_facts);
+        // The solid bridges by the first time each linedef comes in its row, which is all that is asked of it: a row then has fewer than 65536 (WallLinks).
+        const int *const bridge_ofs[2] = {h->solid_bridge_start_ofs, h->solid_bridge_end_ofs}, *const bridge_idx[2] = {h->solid_bridge_start_idx, h->solid_bridge_end_idx};
+        std::vector<int> bridge_first[2], bridges[2];
+        for (int end = 0; end < 2; ++end) {
+            std::vector<size_t> seen(W, W);
+            for (size_t w = 0; w < W; ++w) {
+                bridge_first[end].push_back((int)bridges[end].size());
+                for (int k = bridge_ofs[end][w]; k < bridge_ofs[end][w + 1]; ++k) {
+                    const int b = bridge_idx[end][k];
+                    if (seen[b] != w) bridges[end].push_back(b);
+                    seen[b] = w;
+                }
+            }
+            bridge_first[end].push_back((int)bridges[end].size());
+        }
+        d.solid_bridge_start_ofs = d.solid_bridge_end_ofs = nullptr;      // WallLinks has them
+        if (rc == GD_OK) rc = upload(r, bridges[0].data(), bridges[0].size(), &d.solid_bridge_start_idx);
+        if (rc == GD_OK) rc = upload(r, bridges[1].data(), bridges[1].size(), &d.solid_bridge_end_idx);
         std::vector<WallLinks> links(W);
         for (size_t w = 0; w < W; ++w) {
-            WallLinks &link = links[w];
+            WallLinks &link = links[w];      // all zero
             link.sectors = ((unsigned)h->wall_sectors[2 * w] & 0xFFFFu) | (unsigned)h->wall_sectors[2 * w + 1] << 16;
             link.vertices = ((unsigned)h->wall_vertex[2 * w] & 0xFFFFu) | (unsigned)h->wall_vertex[2 * w + 1] << 16;
             for (int k = 0; k < 2; ++k) link.neighbour[k] = h->direct_neighbor_table[4 * w + k];
             link.slots = (unsigned)h->direct_neighbor_table[4 * w + 2];
-            link.solid[0] = h->solid_bridge_start_ofs[w]; link.solid[1] = h->solid_bridge_end_ofs[w];
-            link.solid_counts = (unsigned)(h->solid_bridge_start_ofs[w + 1] - link.solid[0]) | (unsigned)(h->solid_bridge_end_ofs[w + 1] - link.solid[1]) << 16;
+            for (int end = 0; end < 2; ++end) {
+                link.solid[end] = bridge_first[end][w];
+                link.solid_counts |= (unsigned)(bridge_first[end][w + 1] - link.solid[end]) << (16 * end);
+            }
         }
         if (rc == GD_OK) rc = upload(r, links.data(), links.size(), &r->dm.wall_links);
         std::vector<VertexLink> vertex_links(h->vertex_wall_ofs[V]);

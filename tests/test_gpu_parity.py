@@ -23,6 +23,26 @@ def _renderer(name):
     return meta, data, tables, renderer, lanes
 
 
+@pytest.mark.parametrize("copies", [2, 32768, 65536])
+def test_solid_bridges_listed_more_than_once_are_the_same_bridges(copies):
+    """A row may name a linedef again and again, and then hold more entries than a map has linedefs.  The frame needs its bridges: without them 33 pixels differ."""
+    from gradoom_amd.renderer import HipRenderer, LaneState
+
+    meta, data, smap, tables = load_fixture("rare_rules_brick26")
+    tables = dict(tables)
+    for end in ("start", "end"):
+        ofs, idx = tables[f"solid_bridge_{end}_ofs"], tables[f"solid_bridge_{end}_idx"]
+        tables[f"solid_bridge_{end}_ofs"] = (ofs.astype(np.int64) * copies).astype(ofs.dtype)
+        tables[f"solid_bridge_{end}_idx"] = np.concatenate([np.tile(idx[a:b], copies) for a, b in zip(ofs[:-1], ofs[1:])]).astype(idx.dtype)
+    renderer = HipRenderer(smap, meta["lanes"], "cuda:0", cosine_correction=data["cosine_correction"], tables=tables)
+    indexed = torch.zeros((meta["lanes"], 240, 320), dtype=torch.uint8, device="cuda:0")
+    renderer.render(LaneState.from_numpy(lane_inputs(data), "cuda:0"), indexed=indexed)
+    torch.cuda.synchronize()
+    assert renderer.status() == 0
+    assert np.array_equal(indexed.cpu().numpy(), data["indexed"])
+    renderer.close()
+
+
 @pytest.mark.parametrize("name", fixture_names())
 def test_indexed_frame_bit_exact_vs_reference_golden(name):
     print(f"case {name}", flush=True)
