@@ -14,55 +14,77 @@ inline bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || 
 // wall_select_kernel: how many of the longest strips have their columns' lists shared out, and over how many lanes a column.  More strips and more lanes
 // shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a large one's does.
 // Since a lane alone keeps its column's nearest entries at hand, few strips are left to which sharing matters: none in large batches of all but the largest maps.
-// Stage times in us of strips:lanes a column, two sets of poses; "before" is what the line of up to 1024 strips took that lists read from memory asked for.
-//   lanes    240 linedefs                      320                              500                                        701, bricks
-//     96   0 68, 128:8 52, 256:16 74         84, 59, 72                       91, 128:16 55, 256:32 60                   152, 256:8 98, 256:16 78, 256:32 70
-//    256   80, 57, 68 (before 70)            86, 62, 66 (73)                  94, 256:8 65, 256:16 62 (68)               154, 103, 92, 512:16 94 (106)
-//    384   82, 60, 69 (85)                   90, 63, 68 (87)                  98, 72, 71, 384:16 70 (83)                 161, 104, 102, 384:16 96 (116)
-//    704   93, 73, 256:8 78 (113)            97, 81, 83 (112)                 111, 83, 89, 128:8 89 (112)                170, 119, 125, 128:8 125 (158)
-//   1024   98, 81, 84 (122)                  104, 87, 89 (124)                118, 94, 102, 128:8 95 (123)               178, 131, 138, 128:8 138 (185)
-//   1536   108, 97, 105 (127)                115, 99, 107 (130)               124, 109, 118, 128:8 112 (139)             191, 145, 156, 128:8 155 (206)
-//   2048   116, 122, 130 (117)               124, 122, 132 (151)              134, 134, 138, 128:8 124 (151)             206, 178, 189, 128:8 170 (232)
-//   4096   184, 216, 227 (184)               191, 224, 235 (191)              195, 240, 236 (195)                        263, 322, 314 (264)
-//   lanes    1000 linedefs                          2000                                             4000
-//     96                                          256:8 117, 256:16 85, 256:32 76 (81)             256:8 188, 256:16 132, 256:32 109 (115)
-//    160                                          512:16 93, 256:32 96 (96)                        512:16 139, 256:32 146 (152)
-//    256   256:8 95, 256:16 86 (98)               512:8 128, 512:16 95 (112)                       512:8 196, 512:16 144 (152)
-//    384   98, 102 (116)                          129, 113, 768:16 122 (133)                       199, 175, 768:16 160 (175)
-//    704   125, 134 (158)                         161, 151, 160 (182)                              240, 252, 222 (257)
-//   1024   143, 153 (181)                         200, 187, 196, 256:8 188 (223)                   290, 303, 275 (307)
-//   1536   158, 170 (209)                         233, 242, 258, 256:8 231 (260)                   383, 409, 373 (364)
-//   2048   192, 196, 128:8 180 (237)              269, 295, 316, 256:8 259 (284)                   439, 473, 469 (452)
-//   4096   0 276, 256:8 339, 256:16 323 (338)     0 436, 256:8 421, 256:16 403 (424)               0 842, 512:8 657, 512:16 670 (672)
-// 160 linedefs: 1280 lanes 0 67, 128:8 63, 1792 lanes 74, 79.  330, bricks: 2560 lanes 0 120, 128:8 116, 3072 lanes 130, 136.  700: 184, 166 and 192, 196.
-// 1400: 3072 lanes 0 237, 256:8 226, 4096 lanes 269, 291; 256 lanes 512:16 77, 512 lanes 512:8 105.  2800: 320 lanes 512:16 124, 900 lanes 206, 1792 lanes 256:8 294.
+// Stage times in us of strips:lanes a column, on the one draw of each map and two sets of poses: the rule's choice and the fastest two of the others (none, 128, 256,
+// 512 or 768 strips of 8 or 16 lanes, up to 160 lanes of 32; + on two streams, see select_together).  Runs differ by 1 to 3 us, by 5 from 2048 lanes on.
+//   lanes  240 linedefs                    320                             500
+//      96  128:8 46, 256:8 51, 128:32 52   128:8 57, 128:16 59, 128:32 59  256:32 60, 128:32 57, 128:16 57
+//     160  128:8 47, 256:8 51, 768:8 55    128:8 56, 128:32 57, 256:8 57   256:16 62, 128:16 60, 128:32 61
+//     256  128:8 49, 256:8 49, 512:8 54    128:8 57, 256:8 56, 512:8 58    256:16 62, 512:8 61, 256:8 62
+//     512  128:8 57, 256:8 58, 128:16 60   256:8 65, 256:16 65, 128:8 65   256:8 73, 256:16 73, 512:16 80
+//     704  128:8 62, 256:8 62, 128:16 63   256:8 72, 256:16 75, 128:8 75   256:8 79, 256:16 80, 128:8 87
+//    1024  128:8 69, 256:8 69, 128:16 73   256:8 80, 256:16 84, 128:8 86   256:8 89, 256:16 92, 128:8 93
+//    1536  128:8 78, 128:16 79, 256:8 84   256:8 97, 128:8 91, 128:16 94   256:8 106, 128:8 105, 256:16 106
+//    2048  0 94, 128:16 94, 128:8 97       128:8 112, 128:16 107, 0 111    128:8 118, 128:16 118, 256:16 125
+//    2560  0 103, 128:16 109, 128:8 114    0 114, 128:16 123, 128:8 131    0 138, 128:16 131, 128:8 139
+//    3072  0 105, 128:16 125, 128:8 132    0 123, 128:16 142, 128:16+ 150  0 144, 128:16 151, 128:16+ 159
+//    4096  0 138, 128:16 158, 128:16+ 164  0 157, 128:16 181, 128:16+ 186  0 168, 128:16 194, 128:16+ 195
+//   lanes  701, bricks                        1000, bricks                       1400
+//      96  256:32 59, 128:32 63, 128:16 65    256:32 62, 256:16 75, 128:16 77    256:32 56, 256:16 60, 128:16 74
+//     160  256:16 63, 512:16 65, 256:32 65    256:16 75, 256:32 75, 512:16 76    512:16 62, 256:32 63, 768:16 63
+//     256  512:16 74, 256:16 80, 768:16 83    512:16 81, 768:16 87, 256:16 95    512:16 69, 768:16 76, 512:8 85
+//     512  512:16 90, 256:8 92, 256:16 93     512:16 108, 512:8 118, 768:16 120  512:16 104, 768:16 95, 768:8 100
+//     704  512:16 103, 256:8 110, 256:16 113  512:16 125, 768:16 135, 512:8 139  512:16 112, 768:16 112, 512:8 115
+//    1024  256:8 135, 512:16 126, 128:8 132   256:8 155, 512:16 150, 256:16 160  512:16 127, 768:16 133, 512:8 139
+//    1536  256:8 145, 128:8 146, 128:16 150   256:8 174, 128:8 175, 128:16 180   256:8 165, 512:8 151, 512:16 160
+//    2048  128:8 152, 256:8 157, 128:16 158   128:8 190, 256:8 185, 256:16 190   256:8 167, 128:8 169, 512:8 174
+//    2560  128:16 174, 128:8 170, 0 179       128:16 217, 128:8 208, 256:16 210  256:8 194, 128:8 193, 128:16 201
+//    3072  0 189, 128:16 188, 128:8 197       0 245, 128:16 228, 128:8 238       256:8+ 221, 128:8 202, 128:16 207
+//    4096  0 208, 128:16+ 235, 128:16 236     0 266, 128:16+ 273, 256:16+ 283    256:8+ 258, 128:16 244, 128:16+ 255
+//   lanes  2000                                 2800                                 4000
+//      96  256:32 63, 256:16 79, 128:32 84      256:32 76, 256:16 88, 128:16 108     256:32 90, 256:16 108, 128:16 143
+//     160  512:16 82, 256:16 82, 256:32 82      512:16 96, 768:16 97, 512:32 98      512:16 132, 512:32 119, 768:16 133
+//     256  512:16 83, 768:16 91, 256:16 107     768:16 102, 512:16 102, 256:16 135   768:16 137, 512:16 135, 256:16 168
+//     512  512:16 125, 768:16 125, 512:8 129    768:16 133, 512:16 146, 512:8 165    768:16 175, 768:8 196, 512:16 197
+//     704  512:16 149, 768:16 146, 512:8 151    768:16 158, 768:8 177, 512:8 179     768:16 196, 768:8 220, 512:8 222
+//    1024  512:16 176, 256:8 178, 768:16 179    768:16 198, 512:16 206, 512:8 216    768:16 256, 512:8 272, 768:8 278
+//    1536  256:8 212, 256:16 220, 512:8 224     768:16 266, 512:8 261, 512:16 262    768:16 337, 512:8 339, 512:16 360
+//    2048  256:8 254, 512:8 251, 768:8+ 254     512:8 299, 768:8+ 292, 768:16+ 292   512:8 472, 256:8 483, 768:8 485
+//    2560  256:8 268, 128:8 266, 512:16+ 270    256:8 340, 768:8+ 336, 768:16+ 336   512:8 449, 768:8+ 449, 768:16+ 449
+//    3072  512:16+ 290, 128:8 293, 512:8+ 297   768:16+ 356, 768:8+ 369, 128:8 370   768:16+ 490, 768:8+ 490, 512:16+ 526
+//    4096  512:16+ 355, 128:16 357, 256:8+ 363  768:16+ 431, 256:8+ 440, 512:8+ 445  768:16+ 566, 768:8+ 588, 512:8+ 592
+// The lines lie where the choices change places over four draws of eighteen maps, 160 to 4000 linedefs, in grids and in bricks: over these the choice takes 0.9 %
+// longer than the fastest in the mean, 17 % at worst (16 lanes on 160 linedefs; with the lines that the selection's kernels had before a linedef's record lay in
+// registers 2.5 and 22 %).  Maps alike in their linedefs differ by as much in where their lines would be.
 inline int select_strips(int lanes, int linedefs) {
-    if (linedefs <= 128 || (linedefs < 280 && lanes > 1536) || (linedefs < 1024 && lanes > 2816) || (linedefs < 1700 && lanes > 3072)) return 0;
-    if (linedefs < 400) return 128;
-    if (linedefs < 1024) return lanes <= 1792 ? 256 : 128;
-    if (linedefs < 3000) return lanes <= 1152 ? 512 : 256;
-    return lanes <= 1792 ? 768 : 512;
+    if (linedefs <= 128 || (linedefs < 280 && lanes > 1536) || (linedefs < 512 && lanes > 2304) || (linedefs < 1024 && lanes > 2688)) return 0;
+    if (linedefs < 400) return linedefs >= 280 && lanes > 288 && lanes <= 1600 ? 256 : 128;
+    if (linedefs < 1024) return lanes > 1792 ? 128 : (linedefs >= 660 && lanes > 192 && lanes <= 736 ? 512 : 256);
+    if (lanes <= 112) return 256;
+    if (linedefs < 2300) return lanes <= 1408 || (lanes > 2688 && linedefs >= 1700) ? 512 : 256;
+    if (lanes <= 192) return 512;
+    return lanes <= 1600 || lanes > 2688 ? 768 : (linedefs < 3000 && lanes > 2304 ? 256 : 512);
 }
 inline int select_lanes(int lanes, int linedefs) {
-    const int w = linedefs < 4096 ? linedefs : 4096;      // no map of more was timed
-    if (w < 400) return 8;
-    if (lanes <= 96 + w / 128) return 32;
-    if (w < 1024) return lanes <= 384 ? 16 : 8;
-    if (w < 3000) return lanes <= 1152 || lanes >= 3584 ? 16 : 8;
-    return lanes <= 1792 ? 16 : 8;
+    if (linedefs < 400) return 8;
+    if (lanes <= (linedefs < 2300 ? 112 : 144)) return 32;
+    if (linedefs < 512) return lanes <= 384 ? 16 : 8;
+    if (linedefs < 1024) return (lanes <= (linedefs < 660 ? 600 : 736)) || lanes > 2304 ? 16 : 8;
+    if (linedefs < 2300) return lanes <= 1408 || (lanes > 2688 && linedefs >= 1700) ? 16 : 8;
+    return lanes <= 1600 || lanes > 2688 ? 16 : 8;
 }
 
 // wall_select_kernel: the longest strips and the others in one launch?  A launch on the side stream and back costs 20 us of the stage.  In larger batches
 // the others' wavefronts are so many that they hold the longest strips' up, which the side stream's start a little later do not.  Stage times in us, one
-// launch / two, of the strips and lanes above:
-//   lanes     320 linedefs    701, bricks    1400         2000         2800         4000
-//    768       82 / 109       124 / 151                 156 / 184                 231 / 260
-//   1536       99 / 128       145 / 179                 231 / 243                 373 / 385
-//   2048      122 / 145       170 / 206                 259 / 270                 439 / 479
-//   2560                                   204 / 241                 350 / 381    490 / 526
-//   3072                                   227 / 256                 395 / 406    577 / 571
-//   4096                                                407 / 403                 684 / 657
-inline bool select_together(int lanes) { return lanes <= 3072; }
+// launch / two, of the same strips and lanes up to 1536 lanes, then of the fastest that either has:
+//   lanes     701, bricks    1400         2000         2800         4000
+//     768      123 / 147    128 / 152    158 / 187    188 / 212    220 / 250
+//    1536      154 / 182    165 / 187    223 / 248    276 / 301    349 / 361
+//    2048      152 / 178    167 / 182    251 / 254    299 / 292    472 / 491
+//    2560      170 / 191    193 / 203    266 / 270    340 / 336    449 / 449
+//    3072      188 / 207    202 / 218    293 / 290    370 / 356    528 / 490
+//    4096      236 / 235    244 / 255    357 / 355    458 / 431    628 / 566
+// (Maps of fewer than 1024 linedefs have none among the longest from 2689 lanes on.)
+inline bool select_together(int lanes) { return lanes <= 2688; }
 
 // wall_geometry_kernel: wavefronts a lane for its linedefs (a power of two).  us with 4 / 8 / 16 of them: 16 lanes 13.6 / 10.7 / 8.3, 512 lanes
 // 63 / 48 / 46, 1024 lanes 48 / 41 / 42, 4096 lanes 263 / 242 / 247.
