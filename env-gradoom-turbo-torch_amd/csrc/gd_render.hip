@@ -2514,11 +2514,6 @@ struct PassColumn {
 #define PB_FORWARD_BRIDGE 0x4000
 #define PB_FINAL_ALONG_HI 0x8000
 
-// (distance, linedef) lexicographic minimum: what torch.min(dim) returns on ascending indices
-__device__ __forceinline__ void take_min(float v, int w, float &best, int &best_w) {
-    if (v < best || (v == best && w < best_w && finitef(v))) { best = v; best_w = w; }
-}
-
 __device__ __forceinline__ float height_row(const ColumnLine &line, int x) { return (float)(int)clampi(line.at(x) >> 16, 0, VH); }
 __device__ __forceinline__ float bent_row(float row, const HeightBend &b, int x) {
     const int top0 = b.top & 1023u, top1 = (b.top >> 10) & 1023u, collapsed = (int)(b.top >> 20) - 1;
@@ -6525,14 +6520,15 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
     const size_t W = h->wall_count, S = h->sector_count, V = h->vertex_count, K = h->neighbor_slots;
     int rc = hipGetDevice(&r->device) == hipSuccess ? GD_OK : fail(GD_E_HIP, "hipGetDevice");
 #define UP(field, count) if (rc == GD_OK) rc = upload(r, h->field, (size_t)(count), &d.field)
-    UP(walls, W * 4); UP(walls_fixed, W * 4); UP(wall_sectors, W * 2); UP(wall_vertex, W * 2);
-    UP(side_tex, W * 6); UP(side_off, W * 4); UP(wall_len, W);
+    UP(walls, W * 4); UP(walls_fixed, W * 4); UP(wall_sectors, W * 2);
+    UP(side_tex, W * 6);
     UP(endpoint_neighbors, W * K); UP(endpoint_neighbor_starts, W * K); UP(endpoint_neighbor_ends, W * K);
-    UP(direct_neighbor_table, W * 4);
-    UP(vertex_wall_ofs, V + 1); UP(vertex_wall_idx, h->vertex_wall_ofs[V]);
-    UP(sector_wall_ofs, S + 1); UP(sector_wall_idx, h->sector_wall_ofs[S]);
-    UP(sector_edge_ofs, S + 1); UP(sector_edge_idx, h->sector_edge_ofs[S]);
+    UP(vertex_wall_ofs, V + 1);
     UP(blocking_walls, h->blocking_count);
+    // what only the tables made of them below ask for: no kernel
+    d.wall_vertex = d.direct_neighbor_table = d.vertex_wall_idx = d.solid_bridge_start_ofs = d.solid_bridge_end_ofs = nullptr;
+    d.sector_wall_ofs = d.sector_wall_idx = d.sector_edge_ofs = d.sector_edge_idx = nullptr;
+    d.side_off = d.wall_len = nullptr;
     {
         const size_t fragments = (size_t)(h->split_count > 0 ? h->split_count : 1) * h->fragment_slots;
         UP(wall_split_slot, W);
@@ -6616,7 +6612,6 @@ int gd_renderer_create(const gd_map_desc *h, const float *cosine_correction, int
             }
             bridge_first[end].push_back((int)bridges[end].size());
         }
-        d.solid_bridge_start_ofs = d.solid_bridge_end_ofs = nullptr;      // WallLinks has them
         if (rc == GD_OK) rc = upload(r, bridges[0].data(), bridges[0].size(), &d.solid_bridge_start_idx);
         if (rc == GD_OK) rc = upload(r, bridges[1].data(), bridges[1].size(), &d.solid_bridge_end_idx);
         std::vector<WallLinks> links(W);
