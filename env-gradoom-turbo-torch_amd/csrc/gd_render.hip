@@ -2172,7 +2172,7 @@ template <> struct NearestOf<1> {
 // wavefront at 16 bytes an entry, four times what L2 holds of it.  Read whole by every scan it takes 0.895 ms for 4096 lanes on the 4000-linedef map; only the
 // entries' order in LDS, nearest first, 0.79, with as many wavefronts a SIMD as one likes; this way 0.64 (11 million lines missed in L2, 15, 6).  1024 lanes on the
 // 2000-linedef map 231, 191, 156 us.  Filled again after 3 / 4 / 5 / 6 / 8 / 10 entries 645 / 646 / 642 / 710 / 730 / 770 us.  Twelve entries are what sixteen
-// wavefronts' LDS holds; with sixteen, and eight wavefronts, 1.0 ms.
+// wavefronts' LDS holds; with sixteen, and eight wavefronts, 1.0 ms.  (All of it before a linedef's record lay in registers, see WallLinks, which made 0.64 ms 0.54.)
 #define WINDOW 12
 #define WINDOW_REFILL 5
 #define WINDOW_BATCH 16        // entries ordered at a time
@@ -3868,14 +3868,12 @@ __global__ void __launch_bounds__(1024) strip_order_kernel(DeviceMap dm, int str
 // runs the other half over the records (pass_draw, clip_pass, pass_paint, advance_clips, the masked mid-texture).
 // Each half is lighter in registers and in code than the two together, so more of its wavefronts share a SIMD and
 // its pass loop fits the instruction cache.  Same segment order and one wavefront per segment in both.
-// The kernel lasts as long as its longest strips: on the 4000-linedef map the 256 longest of 20,480 take 0.94 ms with the
-// chip to themselves, all of them together 1.22 ms, all but the 4096 longest 0.53 ms.  Such a strip's wavefront is held
-// up by its candidate scans (the longest lists, read from device memory beside 20,000 other wavefronts) and by running,
-// pass after pass, every rule that any of its 64 columns takes.  So the longest strips (they lead the order; select_strips) go to a launch of
-// their own, beside the launch for all other strips, in which a column has LANES lanes: a strip is LANES wavefronts, the lanes of a
+// The kernel lasts as long as its longest strips.  Such a strip's wavefront is held up by its candidate scans (the longest lists) and by running,
+// pass after pass, every rule that any of its 64 columns takes.  So in the longest strips (they lead the order; select_strips) a column has LANES
+// lanes: a strip is LANES wavefronts, the lanes of a
 // column hold its list between them in registers, each scans its own entries, and what a scan is after is the smallest of the lanes' keys, three to
-// five lane moves away.  All else they do alike, and the first of them writes the records.  Next to eight wavefronts of 8 columns with one lane
-// each, their lists copied to LDS: 16 lanes on the 2000-linedef map 151 -> 68 us, 512 on the 4000-linedef map 463 -> 257, 4096 of them 0.97 -> 0.89 ms.  What the
+// five lane moves away.  All else they do alike, and the first of them writes the records.  The stage with a lane a column in all strips, and with these shared out:
+// 64 lanes on the 2000-linedef map 216, 66 us, 512 lanes of it 256, 125; on the 4000-linedef map 64 lanes 372, 89, 512 lanes 470, 173, 4096 lanes 782, 564.  What the
 // rules ask beyond the list (a sector bridge) they ask behind the scan, once for each entry concerned: a copy of that code for every entry made the
 // kernels larger than the instruction cache.
 static_assert(SEG_COLS == 64, "wall_select_kernel: a work-group is one wavefront, with columns of one strip");
@@ -5991,7 +5989,7 @@ struct OnDevice {
 };
 
 // Working memory of callers that may not allocate (gd_render_static): one array per device, held until the
-// process ends; about twenty lanes of a 4000-linedef map.  (A batch lasts as long as its longest strips, so a chunk more costs the
+// process ends; 23 lanes of a 4000-linedef map of 400 sectors.  (A batch lasts as long as its longest strips, so a chunk more costs the
 // time of a small batch: 16 such lanes 0.55 ms in one chunk, 0.97 ms in the two that 64 MiB make of them.)  In host code the array's name only stands for the symbol; its address on the current
 // device comes from hipGetSymbolAddress, once per device.
 #define STATIC_SCRATCH_BYTES ((size_t)GD_STATIC_SCRATCH_MIB << 20)
@@ -6066,8 +6064,8 @@ __global__ void fill_words_kernel(unsigned int *words, size_t count, unsigned in
     for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < count; k += (size_t)gridDim.x * blockDim.x) words[k] = value;
 }
 
-// Blocks of the spill pool (320 columns each, 1.25 MiB) for a chunk of `lanes` lanes: every column of up to eight
-// lanes, one column in 32 of a large chunk (160 MiB at 4096 lanes).  The static working memory has room for one.
+// Blocks of the spill pool (320 columns each, 641 KiB) for a chunk of `lanes` lanes: every column of up to eight
+// lanes, one column in 32 of a large chunk (80 MiB at 4096 lanes).  The static working memory has room for one.
 size_t spill_pool_blocks(int lanes) {
     const int share = lanes / 32 > 8 ? lanes / 32 : 8;
     return (size_t)(lanes < share ? lanes : share);
