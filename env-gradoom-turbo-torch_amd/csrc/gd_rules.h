@@ -14,7 +14,7 @@ inline bool setup_whole_lanes(int lanes, int linedefs) { return lanes >= 800 || 
 // wall_select_kernel: how many of the longest strips have their columns' lists shared out, and over how many lanes a column.  More strips and more lanes
 // shorten the longest strips' time, which is all that a small batch's lasts, and add to what all of them take together, which a large one's does.
 // Since a lane alone keeps its column's nearest entries at hand, few strips are left to which sharing matters: none in large batches of all but the largest maps.
-// Stage times in us of strips:lanes a column, on the one draw of each map and two sets of poses: the rule's choice and the fastest two of the others (none, 128, 256,
+// Stage times in us of strips:lanes a column, on one draw of each map and two sets of poses: the rule's choice and the fastest two of the others (none, 128, 256,
 // 512 or 768 strips of 8 or 16 lanes, up to 160 lanes of 32; + on two streams, see select_together).  Runs differ by 1 to 3 us, by 5 from 2048 lanes on.
 //   lanes  240 linedefs                    320                             500
 //      96  128:8 46, 256:8 51, 128:32 52   128:8 57, 128:16 59, 128:32 59  256:32 60, 128:32 57, 128:16 57
